@@ -5,7 +5,7 @@
 // model.py:60-66 via nn.Linear); gemm_generic.hip remains for operands of mixed types and for a K
 // that is no multiple of 4.
 //
-// gemm_f32_stream (M <= 64, decoding): the product is a stream of the weight matrix from HBM.  A
+// gemm_f32_stream (M <= 32, decoding): the product is a stream of the weight matrix from HBM.  A
 // workgroup owns 16 weight rows and its waves split K between them; lane (r, g) keeps groups of four
 // 16-byte loads of weight row r in flight, k = 16 s + 4 g .. + 3 of every 16-wide step s.  An MFMA
 // takes a 16 x 4 piece of the weights as its A operand (lane (r, g) gives A[r][g]) and 4 x 16 of x^T as
@@ -13,10 +13,17 @@
 // takes element j of each lane's load: k = 16 s + 4 g + j.  The waves' partial tiles are added through
 // LDS in wave order, so a row's bits depend on the shape of the weight only, never on the batch.
 //
-// gemm_f32_tiled (any M, prompt portions): 128 weight rows x 128 rows of x a workgroup, four waves as
-// 2 x 2, each 2 x 2 tiles of v_mfma_f32_32x32x2_f32; K in steps of 16 through two LDS buffers, the next
-// step's 16-byte pieces requested from global memory before the current step is multiplied.  A staged
-// row is 16 floats padded to 20, so that the 16-byte reads of an operand spread over all banks.
+// gemm_f32_tiled (more rows, prompt portions): a tile of weight rows by rows of x a workgroup of four waves, each
+// one to four tiles of v_mfma_f32_32x32x2_f32; K in steps of 16 (of 32 or 64 where two or four waves share a tile
+// and take 16 each) through two LDS buffers.  A staged row is padded by 4 floats, so that the 16-byte reads of an
+// operand spread over all banks.  The matrix cores' float32 rate bounds it (a 64 x 64 tile over K 1,536 is 20 us of
+// it); what kept the kernel from it was one tile size, 128 x 128: 129 rows cost what 256 do, and a product of few
+// tiles left most CUs idle (2,048 x 1,536 weights at 192 rows: 32 workgroups of 122 us each).  So there are five
+// tiles, and `pick_tile` takes the one that the sizes are done with first; and the 16-byte pieces are asked for four
+// steps ahead, in registers (one step, 512 clocks, is less than a trip to memory: 128 x 128 tiles 120 -> 118 us, 32 x
+// 32 ones 18 -> 17).  Us before -> now, a captured chain over different weights: N 17,920 K 1,536 gated: 65 rows
+// 130 -> 67, 129 rows 217 -> 99, 192 rows 219 -> 114, 512 rows 319 -> 247; N 1,536 K 8,960 in parts: 65 rows 91 -> 37, 192
+// rows 94 -> 58, 2,048 rows 462 -> 453; N 2,048 K 1,536: 65 rows 120 -> 17, 192 rows 122 -> 23, 2,048 rows 127 -> 113.
 //
 // With `gated`, weight rows alternate gate_j, up_j and the epilogue writes silu(gate) * up (reference
 // model.py:188) to out[M, N / 2].  With `splits` > 1, K is cut over workgroups and `out` is
@@ -143,8 +150,7 @@ template <int WAVES, bool GATED>
 static int pick_tiles(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, int splits,
                       int k_split, hipStream_t stream) {
   if (M <= 16) return launch_stream<WAVES, 1, GATED>(x, w, bias, out, M, N, K, splits, k_split, stream);
-  if (M <= 32) return launch_stream<WAVES, 2, GATED>(x, w, bias, out, M, N, K, splits, k_split, stream);
-  return launch_stream<WAVES, 4, GATED>(x, w, bias, out, M, N, K, splits, k_split, stream);
+  return launch_stream<WAVES, 2, GATED>(x, w, bias, out, M, N, K, splits, k_split, stream);
 }
 
 template <bool GATED>
@@ -164,9 +170,7 @@ static int pick_stream(const float* x, const float* w, const float* bias, float*
 
 // ---------------------------------------------------------------------------- many rows
 
-#define TILE 128      // weight rows and rows of x a workgroup
-#define TILE_K 16     // k a step
-#define ROW_PAD 20    // floats a staged row takes: 16 and 4 of padding
+#define TILE_K 16  // k a wave multiplies a step
 
 // The tile (n, m) that a workgroup takes.  The chip hands workgroups to its eight chiplets in turn
 // (workgroup i to chiplet i % 8), each with an L2 of its own: where the tiles divide by eight, chiplet c
@@ -176,102 +180,131 @@ __device__ __forceinline__ int tile_of_workgroup(int id, int total) {
   return total % 8 == 0 ? (id % 8) * (total / 8) + id / 8 : id;
 }
 
-template <bool GATED>
+// WN x WM waves, each TN x TM tiles of 32 x 32, and WK of them to a tile, which take 16 k of a step each.
+template <int WN, int WM, int WK, int TN, int TM, int AHEAD, bool GATED>
 __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                              const float* __restrict__ bias, float* __restrict__ out,
                                                              int M, int N, int K, int k_split, int tiles_m,
                                                              int tiles_n) {
-  __shared__ __attribute__((aligned(16))) float ws[2][TILE * ROW_PAD];
-  __shared__ __attribute__((aligned(16))) float xs[2][TILE * ROW_PAD];
+  static_assert(WN * WM * WK == 4, "four waves");
+  constexpr int TILE_N = WN * TN * 32, TILE_M = WM * TM * 32, ROWS = TILE_N + TILE_M;
+  constexpr int STEP_K = TILE_K * WK, ROW_PIECES = STEP_K / 4, ROW_PAD = STEP_K + 4;  // floats a staged row takes, 4 of them padding
+  constexpr int PIECES = ROWS * ROW_PIECES, MINE = (PIECES + 255) / 256;                // 16-byte pieces of a step; of one thread
+  constexpr int SUMS = (WK - 1) * WN * WM * 64 * 16 * TN * TM;                          // floats that meet at the end
+  constexpr int FLOATS = 2 * ROWS * ROW_PAD > SUMS ? 2 * ROWS * ROW_PAD : SUMS;
+  __shared__ __attribute__((aligned(16))) float staged[FLOATS];
   const int tile = tile_of_workgroup(blockIdx.x, tiles_m * tiles_n);
   const int tile_m = tile % tiles_m, tile_n = tile / tiles_m;
-  const int n0 = tile_n * TILE, m0 = tile_m * TILE;
+  const int n0 = tile_n * TILE_N, m0 = tile_m * TILE_M;
   const int k_first = blockIdx.y * k_split;
   const int k_end = min(K, k_first + k_split);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int n_wave = (wave & 1) * 64, m_wave = (wave >> 1) * 64;
+  const int wave_k = wave / (WN * WM);
+  const int n_wave = (wave % WN) * TN * 32, m_wave = (wave / WN % WM) * TM * 32;
   const int i = lane & 31, half = lane >> 5;
 
-  // what this thread brings of a step: piece `piece` (4 k) of rows `row` and `row + 64` of each operand
-  const int row = threadIdx.x >> 2, piece = threadIdx.x & 3;
-  const float* w_from[2];
-  const float* x_from[2];
+  // what this thread brings of a step: pieces threadIdx.x + 256 h, the weights' rows before x's
+  const float* from[MINE];
+  int k_mine[MINE], to[MINE];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    w_from[h] = w + (size_t)min(n0 + row + 64 * h, N - 1) * K + piece * 4;
-    x_from[h] = x + (size_t)min(m0 + row + 64 * h, M - 1) * K + piece * 4;
+  for (int h = 0; h < MINE; ++h) {
+    const int place = threadIdx.x + 256 * h, row = place / ROW_PIECES;
+    k_mine[h] = place % ROW_PIECES * 4;
+    to[h] = row * ROW_PAD + k_mine[h];
+    from[h] = (row < TILE_N ? w + (size_t)min(n0 + row, N - 1) * K : x + (size_t)min(m0 + row - TILE_N, M - 1) * K) + k_mine[h];
   }
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  f32x16 acc[2][2];
+  f32x16 acc[TN][TM];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < TN; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < TM; ++b)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[a][b][e] = 0.f;
 
-  f32x4 w_in[2], x_in[2];
-  auto fetch = [&](int k0) {
-    const bool inside = k0 + piece * 4 < k_end;
+  f32x4 in[AHEAD][MINE];
+  auto fetch = [&](f32x4 (&to_here)[MINE], int k0) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      w_in[h] = inside ? load4(w_from[h] + k0) : zero;
-      x_in[h] = inside ? load4(x_from[h] + k0) : zero;
-    }
+    for (int h = 0; h < MINE; ++h) to_here[h] = k0 + k_mine[h] < k_end ? load4(from[h] + k0) : zero;
   };
-  auto stage = [&](int buffer) {
+  auto stage = [&](const f32x4 (&here)[MINE], int buffer) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      *(f32x4*)(ws[buffer] + (row + 64 * h) * ROW_PAD + piece * 4) = w_in[h];
-      *(f32x4*)(xs[buffer] + (row + 64 * h) * ROW_PAD + piece * 4) = x_in[h];
-    }
+    for (int h = 0; h < MINE; ++h)
+      if (PIECES % 256 == 0 || threadIdx.x + 256 * h < PIECES) *(f32x4*)(staged + buffer * ROWS * ROW_PAD + to[h]) = here[h];
   };
-
-  fetch(k_first);
-  stage(0);
-  __syncthreads();
-  int buffer = 0;
-  for (int k0 = k_first; k0 < k_end; k0 += TILE_K) {
-    const bool more = k0 + TILE_K < k_end;
-    if (more) fetch(k0 + TILE_K);
-    // lane (i, half) holds k = 8 half .. + 7 of row i of each of its tiles; instruction s takes element s
-    f32x4 a_low[2], a_high[2], b_low[2], b_high[2];
+  auto multiply = [&](int buffer) {
+    // lane (i, half) holds k = 8 half .. + 7 of its wave's 16 of row i of each of its tiles; instruction s takes element s
+    const float* at = staged + buffer * ROWS * ROW_PAD + wave_k * TILE_K + 8 * half;
+    f32x4 a_low[TN], a_high[TN], b_low[TM], b_high[TM];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const float* a_at = ws[buffer] + (n_wave + 32 * t + i) * ROW_PAD + 8 * half;
-      const float* b_at = xs[buffer] + (m_wave + 32 * t + i) * ROW_PAD + 8 * half;
-      a_low[t] = *(const f32x4*)a_at;
-      a_high[t] = *(const f32x4*)(a_at + 4);
-      b_low[t] = *(const f32x4*)b_at;
-      b_high[t] = *(const f32x4*)(b_at + 4);
+    for (int t = 0; t < TN; ++t) {
+      a_low[t] = *(const f32x4*)(at + (n_wave + 32 * t + i) * ROW_PAD);
+      a_high[t] = *(const f32x4*)(at + (n_wave + 32 * t + i) * ROW_PAD + 4);
+    }
+#pragma unroll
+    for (int t = 0; t < TM; ++t) {
+      b_low[t] = *(const f32x4*)(at + (TILE_N + m_wave + 32 * t + i) * ROW_PAD);
+      b_high[t] = *(const f32x4*)(at + (TILE_N + m_wave + 32 * t + i) * ROW_PAD + 4);
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
+      for (int a = 0; a < TN; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < TM; ++b)
           acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(a_low[a][s], b_low[b][s], acc[a][b], 0, 0, 0);
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
+      for (int a = 0; a < TN; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < TM; ++b)
           acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(a_high[a][s], b_high[b][s], acc[a][b], 0, 0, 0);
-    if (more) stage(buffer ^ 1);
+  };
+
+  // AHEAD steps are asked for before they are multiplied (beyond the end: zeros, nothing is read), two are staged
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) fetch(in[u], k_first + u * STEP_K);
+  stage(in[0], 0);
+  __syncthreads();
+  for (int k0 = k_first; k0 < k_end; k0 += AHEAD * STEP_K) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      if (k0 + u * STEP_K < k_end) {
+        fetch(in[u], k0 + (u + AHEAD) * STEP_K);
+        multiply(u & 1);
+        stage(in[(u + 1) % AHEAD], (u + 1) & 1);
+        __syncthreads();
+      }
+    }
+  }
+  if (WK > 1) {  // the waves of one tile add their sums, in the order of their k
+    float* sums = staged + (size_t)((wave % (WN * WM)) * 64 + lane) * 16 * TN * TM;
+    constexpr int OF_A_WAVE_K = WN * WM * 64 * 16 * TN * TM;
+    if (wave_k > 0) {
+#pragma unroll
+      for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int b = 0; b < TM; ++b) *(f32x16*)(sums + (size_t)(wave_k - 1) * OF_A_WAVE_K + (a * TM + b) * 16) = acc[a][b];
+    }
     __syncthreads();
-    buffer ^= 1;
+    if (wave_k > 0) return;
+#pragma unroll
+    for (int v = 0; v < WK - 1; ++v)
+#pragma unroll
+      for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int b = 0; b < TM; ++b) acc[a][b] += *(const f32x16*)(sums + (size_t)v * OF_A_WAVE_K + (a * TM + b) * 16);
   }
 
   // D[n][m] of a 32 x 32 tile: the lane holds column m = i and rows n = 8 q + 4 half + e, q = 0 .. 3, e = 0 .. 3
   const bool with_bias = bias && blockIdx.y == 0;
 #pragma unroll
-  for (int b = 0; b < 2; ++b) {
+  for (int b = 0; b < TM; ++b) {
     const int m = m0 + m_wave + 32 * b + i;
     if (m >= M) continue;
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
+    for (int a = 0; a < TN; ++a) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int n = n0 + n_wave + 32 * a + 8 * q + 4 * half;
@@ -301,25 +334,79 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
   }
 }
 
+template <int WN, int WM, int WK, int TN, int TM, int AHEAD, bool GATED>
+static int launch_tiles(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, int splits,
+                        hipStream_t stream) {
+  constexpr int TILE_N = WN * TN * 32, TILE_M = WM * TM * 32;
+  const int k_split = splits == 1 ? K : ((K + splits - 1) / splits + TILE_K - 1) / TILE_K * TILE_K;
+  if ((size_t)k_split * (splits - 1) >= (size_t)K) return ERR_BAD_ARGUMENT;
+  const int tiles_m = (M + TILE_M - 1) / TILE_M, tiles_n = (N + TILE_N - 1) / TILE_N;
+  hipLaunchKernelGGL((gemm_f32_tiled_kernel<WN, WM, WK, TN, TM, AHEAD, GATED>), dim3(tiles_m * tiles_n, splits), dim3(256), 0, stream, x, w,
+                     bias, out, M, N, K, k_split, tiles_m, tiles_n);
+  return LAUNCH_STATUS();
+}
+
+// The tiles, and what a workgroup of each takes over K = 1,536, us: the first on a CU, and every further one there
+// (measured at 65 to 2,048 rows of the four weights named above; larger tiles read less from L2 a product, smaller
+// ones leave fewer rows and fewer CUs idle).
+struct TileCost {
+  int n, m;
+  float first, further;
+};
+static const TileCost TILE_COSTS[] = {{128, 128, 118.f, 100.f}, {128, 64, 68.f, 51.f}, {64, 64, 39.5f, 27.f},
+                                      {64, 32, 27.f, 14.7f},    {32, 32, 17.f, 8.3f}};
+
+// Us that the product takes with tile `t`: workgroups are spread over 256 CUs, and a part of K costs its partial
+// sums' way to memory and back besides.
+static float tiled_us(const TileCost& t, int M, int N, int K, int splits) {
+  const long groups = (long)((N + t.n - 1) / t.n) * ((M + t.m - 1) / t.m) * splits;
+  const float rounds = (float)((groups + 255) / 256);
+  return (t.first + (rounds - 1.f) * t.further) * (float)K / (float)splits / 1536.f +
+         (splits > 1 ? (float)splits * M * N * 8e-6f / 4.5f : 0.f);
+}
+
+static int pick_tile(int M, int N, int K, int splits) {
+  int best = 0;
+  for (int t = 1; t < 5; ++t)
+    if (tiled_us(TILE_COSTS[t], M, N, K, splits) < tiled_us(TILE_COSTS[best], M, N, K, splits)) best = t;
+  return best;
+}
+
+// Into how many parts of K (at most 8, each at least 256 long) the tiled product of these sizes is best cut where its
+// result may stay in parts.
+extern "C" int llmserve_gemm_f32_parts(int M, int N, int K) {
+  int best = 1;
+  float best_us = 0.f;
+  for (int splits = 1; splits <= 8; ++splits) {
+    if (splits > 1 && K / splits < 256) break;
+    const float us = tiled_us(TILE_COSTS[pick_tile(M, N, K, splits)], M, N, K, splits);
+    if (splits == 1 || us < best_us) best = splits, best_us = us;
+  }
+  return best;
+}
+
 template <bool GATED>
 static int launch_tiled(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, int splits,
                         hipStream_t stream) {
-  const int k_split = splits == 1 ? K : ((K + splits - 1) / splits + TILE_K - 1) / TILE_K * TILE_K;
-  if ((size_t)k_split * (splits - 1) >= (size_t)K) return ERR_BAD_ARGUMENT;
-  const int tiles_m = (M + TILE - 1) / TILE, tiles_n = (N + TILE - 1) / TILE;
-  hipLaunchKernelGGL((gemm_f32_tiled_kernel<GATED>), dim3(tiles_m * tiles_n, splits), dim3(256), 0, stream, x, w, bias,
-                     out, M, N, K, k_split, tiles_m, tiles_n);
-  return LAUNCH_STATUS();
+  switch (pick_tile(M, N, K, splits)) {
+    case 0: return launch_tiles<2, 2, 1, 2, 2, 4, GATED>(x, w, bias, out, M, N, K, splits, stream);
+    case 1: return launch_tiles<4, 1, 1, 1, 2, 4, GATED>(x, w, bias, out, M, N, K, splits, stream);
+    case 2: return launch_tiles<2, 2, 1, 1, 1, 4, GATED>(x, w, bias, out, M, N, K, splits, stream);
+    case 3: return launch_tiles<2, 1, 2, 1, 1, 4, GATED>(x, w, bias, out, M, N, K, splits, stream);
+    default: return launch_tiles<1, 1, 4, 1, 1, 4, GATED>(x, w, bias, out, M, N, K, splits, stream);
+  }
 }
 
 // out [M, N] (or [splits, M, N] partial sums) = x [M, K] . w [N, K]^T (+ bias [N]); all float32, K a multiple
 // of 4.  gated: w's rows alternate gate and up (N even), out is [M, N / 2] = silu(gate) * up, no splits.
-// Up to 64 rows of x go to the weight-streaming kernel, more to the tiled one.
+// Up to 32 rows of x go to the weight-streaming kernel, more to the tiled one (64 rows, us, streaming against tiled: N
+// 17,920 K 1,536 gated 74 and 53, N 1,536 K 8,960 in parts 38 and 26, N 2,048 K 1,536 22 and 17; 32 rows: 47 and 36, 24 and 20,
+// but 13 and 17 for the small weight, and 17 rows 38 and 35, 19 and 20, 11 and 17).
 extern "C" int llmserve_gemm_f32(const float* x, const float* w, const float* bias, float* out, int gated, int M, int N,
                                  int K, int splits, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || K % 4 || splits < 1 || (gated && (splits != 1 || N % 2))) return ERR_BAD_ARGUMENT;
-  if (M <= 64)
+  if (M <= 32)
     return gated ? pick_stream<true>(x, w, bias, out, M, N, K, splits, stream)
                  : pick_stream<false>(x, w, bias, out, M, N, K, splits, stream);
   return gated ? launch_tiled<true>(x, w, bias, out, M, N, K, splits, stream)

@@ -61,6 +61,7 @@ _SIGNATURES = {
     "llmserve_gather_rows": "ppiippiip",
     "llmserve_gemm_generic": "pipipipiiiip",
     "llmserve_gemm_f32": "ppppiiiiip",
+    "llmserve_gemm_f32_parts": "iii",
     "llmserve_gemm_skinny": "pppipiiiiiip",
     "llmserve_gemm_skinny_tail": "pppipipiiiip",
     "llmserve_gemm_stream": "pppipiiiiiip",
@@ -673,18 +674,15 @@ class HipKernels:
             and weights.in_features % 4 == 0
         )
 
-    @staticmethod
-    def _float32_splits(rows: int, out_features: int, in_features: int) -> int:
-        """Into how many parts of K a float32 product is cut when its result may stay in parts: up to 64
+    def _float32_splits(self, rows: int, out_features: int, in_features: int) -> int:
+        """Into how many parts of K a float32 product is cut when its result may stay in parts: up to 32
         rows (the weight-streaming kernel, workgroups of 16 weight rows) until about a thousand workgroups
-        run, a part at least 512 long; more rows (128 x 128 tiles) until there is one tile for every CU."""
-        if rows <= 64:
-            tiles, least, goal = -(-out_features // 16), 512, 1024
-        else:
-            tiles, least, goal = -(-rows // 128) * -(-out_features // 128), 256, 256
-        best = 1
+        run, a part at least 512 long; more rows (the tiled kernel) as its own estimate has it."""
+        if rows > 32:
+            return self._gemm_f32.llmserve_gemm_f32_parts(rows, out_features, in_features)
+        tiles, best = -(-out_features // 16), 1
         for splits in range(2, 9):
-            if in_features // splits >= least and tiles * splits <= goal:
+            if in_features // splits >= 512 and tiles * splits <= 1024:
                 best = splits
         return best
 

@@ -422,6 +422,20 @@ def test_float32_products_in_parts_and_at_odd_sizes(kernels, rows, inner, outer)
     torch.testing.assert_close(gated.cpu().double(), want, **bound)
 
 
+@pytest.mark.parametrize("rows,inner,outer", [(33, 1540, 96), (64, 260, 2050), (97, 516, 7003), (129, 1028, 9001), (230, 260, 37890),
+                                              (1000, 300, 8197)])
+def test_float32_tiles(kernels, rows, inner, outer):
+    """The tiled 32-bit product with each of its five tiles, at rows, weight rows and K that leave remainders (the bound as above)."""
+    k = kernels[torch.float32]
+    x, w = torch.randn(rows, inner), torch.randn(outer, inner) / math.sqrt(inner)
+    expected = x.double() @ w.double().T
+    bound = dict(atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5)
+    handle = k.prepare_linear([on_gpu(w)], None)
+    torch.testing.assert_close(k.linear(on_gpu(x), handle).cpu().double(), expected, **bound)
+    parts = k.linear(on_gpu(x), handle, out_dtype=torch.float32, partial=True)
+    torch.testing.assert_close((parts if parts.ndim == 2 else parts.double().sum(0)).cpu().double(), expected, **bound)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("pairing", ["adjacent", "half", "none"])
 @pytest.mark.parametrize("heads,kv_heads,dim,page", [(6, 2, 32, 8), (5, 1, 48, 16), (2, 2, 128, 4)])
