@@ -69,7 +69,8 @@ _SIGNATURES = {
     "llmserve_gemm_medium": "pppipiiiiiip",
     "llmserve_gemm_ring": "pppipiiiiiiip",
     "llmserve_gemm_merged": "ppippipiiiip",
-    "llmserve_gemm_tiled": "pppipiiiiiip",
+    "llmserve_gemm_blocks": "pppipiiiiiip",
+    "llmserve_gemm_blocks_parts": "iii",
     "llmserve_attention_generic": "pipiipppippiiiiifipfpiiipip",
     "llmserve_attention_f32": "pipipppppippiiiiiifiipfpiiipip",
     "llmserve_attention_tiles": "pipipppppippiiiiiifiiipippfpiipiiifffpiip",
@@ -184,10 +185,8 @@ class HipKernels:
         shared_portions: str = "auto",
     ) -> None:
         """`library_products=False` keeps every product on the hand-written kernels (the command line's and
-        bench.py's --own-products): the weight-streaming ones up to 64 rows, the LDS-tiled ones above, with
-        their fused epilogues.  Inside a whole step the library is ahead for many rows (at 2,048 rows of the
-        1.5B sizes gate/up with its fused SiLU * up takes 150 us against the library's 120 + 18 for SiLU * up),
-        so it is the default there.
+        bench.py's --own-products): the weight-streaming ones up to 64 rows, the LDS-tiled one above, with
+        their fused epilogues.  For many rows the library takes what it is ahead with (`_tiled_ahead`).
         `shared_portions`:
         whether prompt portions at head size 128 go to the attention kernel whose waves share K and V
         through LDS: "auto" (when the step's walks, taken together, are long beside the longest), "always", "never"."""
@@ -210,6 +209,7 @@ class HipKernels:
         self._gemm_f32 = _declared(load_module("gemm_f32")) if dtype == torch.float32 else None
         self._attention_generic = _declared(load_module("attention_generic"))
         self._gemm_bf16 = _declared(load_module("gemm_bf16")) if dtype == torch.bfloat16 else None
+        self._gemm_blocks = _declared(load_module("gemm_blocks")) if dtype == torch.bfloat16 else None
         self._pinned_stream: int | None = None
         self.ring_products = True  # 17 to 64 rows of a large weight go to the kernel that streams it through a ring in LDS
         self.ring_rows_from = 4     # (and from this many rows on where K may be cut or the weight is very large)
@@ -420,16 +420,16 @@ class HipKernels:
             # workgroups: the 32B sizes' gate/up 100-110 us at the library, 98-106 here, 113-177 in several rounds; the 1.5B
             # sizes' head, 9,496 tiles, 108-120 against 101-165)
             return "ring"
+        if rows > 64 and HipKernels._tiled_ahead(rows, weights.out_features, inner, gated, may_split):
+            return "tiled"
         if self.ring_products and 64 < rows <= 128 and inner % 128 == 0 and (
             (may_split and (1 << 20) < size <= 150_000_000) or (gated and (1 << 22) < size <= 150_000_000)
         ):
-            # 65 to 128 rows, where the step from the kernel above to the library was a cliff (a decode step of the 1.5B
-            # sizes 2.01 ms at 64 rows and 2.76 at 65): the same kernel with eight tiles of x for the products whose K
-            # may be cut and the smaller gated ones.  Us at 65 / 128 rows in a captured chain over different weights,
-            # the library against it: 1.5B sizes gate/up with its activation 25.8 / 26.5 -> 21.9 / 22.3, down 21.8 / 23.2 ->
-            # 13.4 / 14.7, o 7.5 -> 5.8 / 6.3; 7B sizes down 40.1 / 52.4 -> 44.3 / 45.1, o 18.6 / 22.6 -> 13.2 / 14.3; the
-            # gate/up with ten weight tiles a workgroup, 237 workgroups, 67.1 / 72.1 -> 59.1 / 61.3 (80-82 with five, which
-            # make 474); the library keeps qkv (7.5 against 10.2; 19-23 against 21-23).
+            # 65 to 128 rows of gate/up, and of what may be cut where K is no multiple of 256: the same kernel with eight
+            # tiles of x.  Us at 65 / 128 rows in a captured chain over different weights, the library against it: 1.5B sizes
+            # gate/up with its activation 25.8 / 26.5 -> 21.9 / 22.3; the 7B sizes' with ten weight tiles a workgroup, 237
+            # workgroups, 67.1 / 72.1 -> 59.1 / 61.3 (80-82 with five, which make 474); the library keeps qkv (7.5 against 10.2;
+            # 19-23 against 21-23).
             return "ring"
         if self.library_products and (rows > 64 or self._for_replay or weights.out_features * inner > 150_000_000):
             # On the device the library is ahead of "medium" as it stands, so a captured step (which
@@ -450,6 +450,25 @@ class HipKernels:
         if rows > 64 and inner % 32 == 0:
             return "tiled"
         return None
+
+    @staticmethod
+    def _tiled_ahead(rows: int, out_features: int, in_features: int, gated: bool, may_split: bool) -> bool:
+        """Whether a product of more than 64 rows is faster on the LDS-tiled kernel than at the library.  A captured chain
+        over different weights, us, the library (its best of one piece and two to eight slices of K; a gated product with the kernel
+        for silu(gate) * up behind it) against the tiled kernel.  Where the result may stay partial sums, a result of few tiles:
+        N 1,536 K 8,960: 96 rows 17.7 and 11.5 (the kernel through a ring 13.4), 384 rows 25.3 and 20.1, 1,024 rows 37.8 and 35.8,
+        1,536 rows 53.7 and 50.4, 2,048 rows 55.1 and 60.2; N 3,584 K 18,944: 128 rows 50.5 and 34.0 (the ring 45), 512 rows 84.5 and 79.6, 768
+        rows 109 and 124; N = K = 1,536: 192 rows 8.1 and 6.4, 1,024 rows 13.3 and 12.4; N = K = 3,584: 512 rows 22.6 and 20.3, 768 rows 26.4
+        and 28.5.  Gated: N 17,920 K 1,536: 256 rows 35 and 29, 384 rows 37 and 30, 512 rows 45 and 44, 1,024 rows 80 and 74, 2,048
+        rows 133 and 111; N 37,888 K 3,584: 192 rows 84 and 96, 512 rows 149 and 164, 1,024 rows 315 and 274, 2,048 rows 546 and 474;
+        up to 128 rows the ring's 22.5 and 61 are as good or better.  The rest (the qkv products: 384 rows of N 2,048 K 1,536 9.4 and
+        10.1, of N 4,608 K 3,584 25.2 and 27.7) stays with the library."""
+        if in_features % 64:
+            return False
+        if gated:
+            return rows > 128 and (out_features * in_features <= 40_000_000 or rows >= 1024)
+        # (a K of 256s divides into two and four parts of whole stages; else the library's slices may be the only way to cut it)
+        return may_split and in_features % 256 == 0 and (rows <= 128 or rows * out_features <= 2_400_000)
 
     def _library(self, x: torch.Tensor, weights: LinearWeights) -> bool:
         """Whether the product goes to the BLAS library (hipBLASLt through torch), as the
@@ -553,18 +572,6 @@ class HipKernels:
             wanted //= 2
         return wanted
 
-    @staticmethod
-    def _tiled_splits(rows: int, out_features: int, in_features: int) -> int:
-        """Into how many parts of K the tiled product is cut when its float32 result may stay in
-        parts: as many (at most 8, K / parts a multiple of 256) as it takes for the 256 x 256 tiles
-        to number about 256, one for every CU."""
-        tiles = -(-rows // 256) * -(-out_features // 256)
-        best = 1
-        for splits in range(2, 9):
-            if in_features % (splits * 256) == 0 and tiles * (splits - 1) < 256:
-                best = splits
-        return best
-
     def linear(
         self, x: torch.Tensor, weights: LinearWeights, out_dtype: torch.dtype | None = None, *, partial: bool = False
     ) -> torch.Tensor:
@@ -623,7 +630,7 @@ class HipKernels:
                 return out
             if partial and out_dtype == torch.float32:
                 if streaming == "tiled":
-                    splits = self._tiled_splits(rows, weights.out_features, inner)
+                    splits = self._gemm_blocks.llmserve_gemm_blocks_parts(rows, weights.out_features, inner)
                 elif streaming == "medium":
                     splits = self._medium_splits(weights.out_features, inner)
                 elif rows > 16 and weights.out_features * inner <= (1 << 22) and inner % 256 == 0:
@@ -633,7 +640,7 @@ class HipKernels:
             shape = (rows, weights.out_features) if splits == 1 else (splits, rows, weights.out_features)
             out = self._empty(shape, out_dtype or self.dtype)
             if streaming == "tiled":
-                status = self._gemm_bf16.llmserve_gemm_tiled(
+                status = self._gemm_blocks.llmserve_gemm_blocks(
                     _pointer(x), _pointer(weights.weight), _pointer(bias), bias_is_float, _pointer(out),
                     _is_float(out), 0, rows, weights.out_features, inner, splits, self._stream,
                 )
@@ -727,7 +734,7 @@ class HipKernels:
             return out
         if streaming is not None:
             if streaming == "tiled":
-                status = self._gemm_bf16.llmserve_gemm_tiled(
+                status = self._gemm_blocks.llmserve_gemm_blocks(
                     _pointer(x), _pointer(weights.both.weight), None, 0, _pointer(out), _is_float(out), 1,
                     x.shape[0], 2 * weights.width, x.shape[1], 1, self._stream,
                 )

@@ -9,6 +9,7 @@ DEFAULT_VARIANTS: dict[str, list[dict[str, object]]] = {
     "gemm_generic": [{}],
     "gemm_f32": [{}],
     "gemm_bf16": [{}],
+    "gemm_blocks": [{}],
     "attention_generic": [{}],
     "sampling": [{}],
     "columns": [{}],

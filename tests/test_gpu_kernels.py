@@ -125,6 +125,32 @@ def test_products_without_the_library(own_kernels, rows, inner, outer):
     torch.testing.assert_close(gated.cpu().double(), want, **TOLERANCE[dtype])
 
 
+@pytest.mark.parametrize("rows,inner,outer", [(65, 64, 1536), (96, 1536, 17920), (129, 128, 2050), (200, 192, 40), (257, 1024, 4100), (384, 8960, 1536),
+                                              (511, 640, 9000), (640, 320, 20000), (1100, 1536, 6400), (2048, 256, 17920)])
+def test_tiles_of_many_rows(own_kernels, rows, inner, outer):
+    """The LDS-tiled product with each of its tiles, from one stage of K on (fewer stages than it has, as many, more), at rows and weight
+    rows that leave remainders: plain, gated, and in every number of parts that K allows.  Partial sums are float32 sums of
+    `inner` products of bfloat16 values: a few times sqrt(K) * 2^-24 of a result of size 1."""
+    k, dtype = own_kernels, torch.bfloat16
+    generator = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, inner, generator=generator, device="cuda").to(dtype)
+    w, up = (torch.randn(outer, inner, generator=generator, device="cuda").div_(math.sqrt(inner)).to(dtype) for _ in range(2))
+    b = torch.randn(outer, generator=generator, device="cuda").to(dtype)
+    expected = x.double() @ w.double().T + b.double()
+    torch.testing.assert_close(k.linear(x, k.prepare_linear([w], [b])).double(), expected, **TOLERANCE[dtype])
+    want = F.silu(x.double() @ w.double().T) * (x.double() @ up.double().T)
+    torch.testing.assert_close(k.gated_linear(x, k.prepare_gated_linear(w, up)).double(), want, **TOLERANCE[dtype])
+    bound = dict(atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5)
+    for splits in range(1, 13):
+        if inner % (32 * splits):
+            continue
+        parts = torch.full((splits, rows, outer), float("nan"), device="cuda")
+        status = k._gemm_blocks.llmserve_gemm_blocks(x.data_ptr(), w.data_ptr(), b.data_ptr(), 0, parts.data_ptr(), 1, 0, rows, outer, inner, splits,
+                                                     torch.cuda.current_stream().cuda_stream)
+        assert status == 0
+        torch.testing.assert_close(parts.double().sum(0), expected, **bound)
+
+
 def key_pieces(rows):
     """Key pages written as rows [pages, kv, offset, dim] -> as the cache keeps them, in pieces of eight
     elements, the same piece of all the keys of a page side by side: [pages, kv, dim / w, offset, w]
