@@ -42,11 +42,20 @@ __device__ __forceinline__ void block_argmax(const float* row, int n, float* bes
                                              float* shared_v, int* shared_i) {
   float value = -INFINITY;
   int index = 0x7fffffff;  // no entry seen yet
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    const float v = row[i];
-    if (v > value || index == 0x7fffffff) {  // strided indices ascend, so ties keep the first
-      value = v;
-      index = i;
+  for (int first = threadIdx.x; first < n; first += 4 * blockDim.x) {  // four loads under way together
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = first + u * blockDim.x;
+      v[u] = i < n ? row[i] : -INFINITY;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = first + u * blockDim.x;
+      if (i < n && (v[u] > value || index == 0x7fffffff)) {  // strided indices ascend, so ties keep the first
+        value = v[u];
+        index = i;
+      }
     }
   }
 #pragma unroll
@@ -225,16 +234,19 @@ extern "C" int llmserve_argmax_static(const float* logits, int* out, int rows, i
 // kept as that integer.  Integer sums do not depend on their order, so the blocks of a row add into
 // one histogram with atomic additions and the result is the same on every run.
 
-#define SAMPLE_BLOCK 256  // threads of a block that works on a piece of a row
+#define SAMPLE_BLOCK 512  // threads of a block that works on a piece of a row
 #define SAMPLE_BINS 1024
 #define SAMPLE_BINS_EACH (SAMPLE_BINS / SAMPLE_BLOCK)  // bins that a thread of the head looks at
 #define SAMPLE_LEVEL_BITS 10
 #define SAMPLE_PIECES_MAX 64  // a wave looks at a row's pieces, a lane at each
 #define SAMPLE_HISTOGRAMS 5   // the cut search's three levels, then levels 1 and 2 of the chosen search
 
-static int sample_pieces(int rows) {
+// About 512 blocks of 512 threads in all for top-p, where every piece adds its bins to the row's with atomic additions of
+// its own (64 rows: 98 us, 110 with twice as many; 16 rows 61 and 81; 256 threads and 2,048 blocks 121 and 69), and twice as
+// many without, where more blocks only hide more of the trips to memory (64 rows: 38 us and 43).
+static int sample_pieces(int rows, bool with_top_p) {
   int pieces = SAMPLE_PIECES_MAX;
-  while (pieces > 4 && rows * pieces > 2048) pieces /= 2;
+  while (pieces > 4 && rows * pieces > (with_top_p ? 512 : 1024)) pieces /= 2;
   return pieces;
 }
 
@@ -348,23 +360,38 @@ __device__ __forceinline__ void clear_histogram(unsigned long long* lds_sums, un
   }
 }
 
-// Adds this piece's entries inside the bucket `base` of `level` into the row's histogram.  The block
-// has cleared lds_sums and lds_counts and passed a barrier since.
-__device__ __forceinline__ void add_histogram(const float* __restrict__ p, int begin, int end, unsigned base, int level,
-                                              unsigned long long* lds_sums, unsigned* lds_counts,
-                                              unsigned long long* __restrict__ sums, unsigned* __restrict__ counts,
-                                              unsigned* __restrict__ piece_counts) {
-  const int shift = level_shift(level);
-  const unsigned bucket = base >> (shift + SAMPLE_LEVEL_BITS);
-  for (int i = begin + threadIdx.x; i < end; i += blockDim.x) {
-    const unsigned pattern = __float_as_uint(p[i]);
-    if ((pattern >> (shift + SAMPLE_LEVEL_BITS)) == bucket) {
-      const unsigned bin = (pattern >> shift) & (SAMPLE_BINS - 1);
-      atomicAdd(lds_sums + bin, significand_of(pattern));
-      atomicAdd(lds_counts + bin, 1u);
-    }
+// A piece's entries are taken in batches, all loads of a batch under way together: a thread of 256 had ten entries of a row of
+// 151,936 in 64 pieces, and a loop that asks for one, waits, and adds it paid ten trips to memory one after the other; and
+// the first batch of a search's stage is asked for before its head (1 / 8 / 16 / 32 / 64 rows of 151,936 with top-p: 51.6 / 55.1 /
+// 71.4 / 96.9 / 126 -> 42.8 / 53.7 / 60.6 / 72.6 / 97.7 us with the blocks of `sample_pieces`).
+#define SAMPLE_BATCH 6
+struct Batch {
+  float v[SAMPLE_BATCH];
+};
+// entries first, first + SAMPLE_BLOCK, ... below end; beyond it zeros, which nobody uses
+__device__ __forceinline__ Batch load_batch(const float* __restrict__ p, int first, int end) {
+  Batch batch;
+#pragma unroll
+  for (int u = 0; u < SAMPLE_BATCH; ++u) {
+    const int i = first + u * SAMPLE_BLOCK;
+    batch.v[u] = i < end ? p[i] : 0.f;
   }
-  __syncthreads();
+  return batch;
+}
+
+__device__ __forceinline__ void add_entry(float value, unsigned bucket, int shift, unsigned long long* lds_sums, unsigned* lds_counts) {
+  const unsigned pattern = __float_as_uint(value);
+  if ((pattern >> (shift + SAMPLE_LEVEL_BITS)) == bucket) {
+    const unsigned bin = (pattern >> shift) & (SAMPLE_BINS - 1);
+    atomicAdd(lds_sums + bin, significand_of(pattern));
+    atomicAdd(lds_counts + bin, 1u);
+  }
+}
+
+// Adds what the block has gathered of its piece to the row's histogram (a barrier before).
+__device__ __forceinline__ void give_histogram(const unsigned long long* lds_sums, const unsigned* lds_counts,
+                                               unsigned long long* __restrict__ sums, unsigned* __restrict__ counts,
+                                               unsigned* __restrict__ piece_counts) {
   for (int bin = threadIdx.x; bin < SAMPLE_BINS; bin += blockDim.x) {
     const unsigned count = lds_counts[bin];
     if (count != 0u) {
@@ -416,18 +443,25 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_exp_kernel(const float* _
   float* p = buffers.p + (size_t)r * vocab;
   const int per = (vocab + pieces - 1) / pieces;
   const int begin = min(vocab, piece * per), end = min(vocab, begin + per);
+  const bool with_histogram = with_top_p && top_ps[r] < 1.f;
   const float top_logit = row[best_index] / temperature;
   double partial = 0.0;
-  for (int i = begin + threadIdx.x; i < end; i += blockDim.x) {
-    const float v = expf(row[i] / temperature - top_logit);
-    p[i] = v;
-    partial += (double)v;
+  for (int first = begin + threadIdx.x; first < end; first += SAMPLE_BATCH * SAMPLE_BLOCK) {
+    const Batch batch = load_batch(row, first, end);
+#pragma unroll
+    for (int u = 0; u < SAMPLE_BATCH; ++u) {
+      const int i = first + u * SAMPLE_BLOCK;
+      if (i >= end) break;
+      const float v = expf(batch.v[u] / temperature - top_logit);
+      p[i] = v;
+      partial += (double)v;
+      if (with_histogram) add_entry(v, 0u, level_shift(0), lds_sums, lds_counts);
+    }
   }
-  const double sum = block_sum_f64(partial, sd);
+  const double sum = block_sum_f64(partial, sd);  // (its barriers stand between the additions and what reads them)
   if (threadIdx.x == 0) buffers.piece_sums[r * pieces + piece] = sum;
-  if (!with_top_p || top_ps[r] >= 1.f) return;
-  add_histogram(p, begin, end, 0u, 0, lds_sums, lds_counts, buffers.sums + (size_t)r * SAMPLE_BINS,
-                buffers.counts + (size_t)r * SAMPLE_BINS, nullptr);
+  if (!with_histogram) return;
+  give_histogram(lds_sums, lds_counts, buffers.sums + (size_t)r * SAMPLE_BINS, buffers.counts + (size_t)r * SAMPLE_BINS, nullptr);
 }
 
 // One stage of the two searches of the rows with top-p.  stage 1, 2: levels 1, 2 of the cut search;
@@ -450,13 +484,20 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_level_kernel(const float*
   const float top_p = top_ps[r];
   if (temperatures[r] <= 0.f || top_p >= 1.f) return;
   clear_histogram(lds_sums, lds_counts);  // the head's barriers lie between this and the additions
+  const int per = (vocab + pieces - 1) / pieces;
+  const int begin = min(vocab, piece * per), end = min(vocab, begin + per);
+  const float* p = buffers.p + (size_t)r * vocab;
+  Batch batch = load_batch(p, begin + threadIdx.x, end);  // under way while the head works
   const size_t per_histogram = (size_t)rows * SAMPLE_BINS, of_row = (size_t)r * SAMPLE_BINS;
   const int search = stage <= 2 ? 0 : 1, level = stage <= 2 ? stage : stage - 2;
 
   SampleState st;
   if (stage == 1) {
+    __shared__ double sums_here[SAMPLE_PIECES_MAX];  // a thread a piece asks, then everybody adds them in order
+    if ((int)threadIdx.x < pieces) sums_here[threadIdx.x] = buffers.piece_sums[r * pieces + threadIdx.x];
+    __syncthreads();
     double total = 0.0;
-    for (int q = 0; q < pieces; ++q) total += buffers.piece_sums[r * pieces + q];
+    for (int q = 0; q < pieces; ++q) total += sums_here[q];
     // the bound is strict, so a bound of 0 would be met nowhere: the least positive one keeps the maximum alone
     st.limit = fmax((double)top_p * total, 2.2250738585072014e-308);
     st.target = st.above_cut = st.kept_at_cut = st.above[0] = st.above[1] = 0.0;
@@ -498,13 +539,19 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_level_kernel(const float*
   }
   if (piece == 0 && threadIdx.x == 0) buffers.states[(size_t)stage * rows + r] = st;
 
-  const int per = (vocab + pieces - 1) / pieces;
-  const int begin = min(vocab, piece * per), end = min(vocab, begin + per);
   unsigned* piece_counts = nullptr;  // the last level: the final stage asks which piece holds the entry
   if (level == 2) piece_counts = buffers.piece_counts + (((size_t)search * rows + r) * pieces + piece) * SAMPLE_BINS;
   const size_t to = (size_t)stage * per_histogram + of_row;
-  add_histogram(buffers.p + (size_t)r * vocab, begin, end, st.base[search], level, lds_sums, lds_counts,
-                buffers.sums + to, buffers.counts + to, piece_counts);
+  const int shift = level_shift(level);
+  const unsigned bucket = st.base[search] >> (shift + SAMPLE_LEVEL_BITS);
+  for (int first = begin + threadIdx.x; first < end; first += SAMPLE_BATCH * SAMPLE_BLOCK) {
+    if (first != begin + (int)threadIdx.x) batch = load_batch(p, first, end);
+#pragma unroll
+    for (int u = 0; u < SAMPLE_BATCH; ++u)
+      if (first + u * SAMPLE_BLOCK < end) add_entry(batch.v[u], bucket, shift, lds_sums, lds_counts);
+  }
+  __syncthreads();
+  give_histogram(lds_sums, lds_counts, buffers.sums + to, buffers.counts + to, piece_counts);
 }
 
 // Sums of v over the threads before this one, in thread order.  shared: at least 16 of its kind.
@@ -679,7 +726,7 @@ struct SampleWorkspace {
 };
 
 static SampleWorkspace sample_workspace(int rows, int vocab) {
-  const size_t pieces = sample_pieces(rows), bins = (size_t)SAMPLE_HISTOGRAMS * rows * SAMPLE_BINS;
+  const size_t pieces = sample_pieces(rows, false), bins = (size_t)SAMPLE_HISTOGRAMS * rows * SAMPLE_BINS;
   SampleWorkspace w;
   size_t at = 0;
   w.sums = at, at += rounded(bins * sizeof(unsigned long long));
@@ -723,7 +770,7 @@ extern "C" int llmserve_sample(const float* logits, const float* temperatures, c
   buffers.states = (SampleState*)(base + w.states);
   buffers.piece_values = piece_values;
   buffers.piece_indices = piece_indices;
-  const int first_pieces = argmax_pieces(rows), pieces = sample_pieces(rows);
+  const int first_pieces = argmax_pieces(rows), pieces = sample_pieces(rows, with_top_p != 0);
   hipLaunchKernelGGL(argmax_pieces_kernel, dim3(rows, first_pieces), dim3(SAMPLE_THREADS), 0, stream, logits,
                      piece_values, piece_indices, vocab, first_pieces, with_top_p ? (unsigned*)base : (unsigned*)nullptr,
                      with_top_p ? w.cleared_words : (size_t)0);
