@@ -55,6 +55,79 @@ __device__ __forceinline__ float gate_value(float gate) {
   return GATED == 2 ? fmaxf(gate, 0.f) : gate / (1.f + expf(-gate));
 }
 
+// Two products with a norm between them, without a kernel for the norm (steps of up to 64 single tokens).  The first one
+// (INTO_NORM) holds whole sums over K, adds them to the residual stream in its epilogue, and writes what the second reads:
+// x * weight in bfloat16, not yet divided by the row's root mean square, and each tile's sum of squares of x a row.  The second
+// one (SCALED) multiplies its float32 results by rsqrt(mean of squares + eps), which is the same for all of a row's
+// products: rounding x * weight loses what rounding the normed row loses.  A norm's kernel is a launch, two trips to
+// memory and a sum over a workgroup: 4.4 us of a layer's 46 at the 1.5B sizes, whatever the rows.  Against that the first product
+// needs whole sums over K (with key splits to merge 6.6 -> 8.2 us: 96 workgroups read what 288 did; 7B sizes 7.3 -> 7.7) and the second one
+// brings the sums of squares (gate/up 11.7 -> 12.8 us at one row, 13.4 -> 13.9 at eight; 7B sizes 47.5 -> 48.7).  A decode step, ms, before -> after: 1.5B
+// sizes 1 row 1.320 -> 1.301, 8 rows 1.430 -> 1.409 (contexts of 8,192: 1.822 -> 1.765), 64 rows 2.045 -> 2.030; 7B sizes 8 rows 3.303 -> 3.206.
+enum { NO_LINK = 0, INTO_NORM = 1, SCALED = 2 };
+struct Link {
+  float* hidden;             // INTO_NORM: [M, N], added to in place
+  const void* weight;        // INTO_NORM: the norm's [N]
+  int weight_is_float;
+  bf16_t* rows;              // INTO_NORM: [M, N]
+  float* sums;               // [tiles, stride]: of 16 columns of x each, row by row
+  int stride, tiles;
+  float inverse_width, eps;  // SCALED
+};
+
+// The end of a product into a norm: `total` four neighbouring columns from n_first of row m, of 16 (tile) that the lanes
+// r, r + 16, r + 32, r + 48 share; they are in the branch together.  N is a multiple of 16.
+struct LinkedColumns {
+  f32x4 hidden;
+  uint2 low, high;  // of the weight: four bfloat16 (twice) or the halves of four float32
+};
+// (asked for at the start and used at the end; without a branch, at whose end the loads inside would be waited for: that cost
+// the 1.5B sizes' output projection 1.5 us)
+__device__ __forceinline__ LinkedColumns linked_columns(const Link& link, int m, int n_first, int M, int N) {
+  LinkedColumns columns;
+  columns.hidden = *(const f32x4*)(link.hidden + (size_t)min(m, M - 1) * N + n_first);
+  const char* weight = (const char*)link.weight + (size_t)n_first * (link.weight_is_float ? 4 : 2);
+  columns.low = *(const uint2*)weight;
+  columns.high = *(const uint2*)(weight + (link.weight_is_float ? 8 : 0));
+  asm volatile("" ::: "memory");  // (asked for here)
+  return columns;
+}
+__device__ __forceinline__ void store_into_norm(const Link& link, const LinkedColumns& columns, f32x4 total, int m, int n_first, int N) {
+  const f32x4 x = columns.hidden + total;
+  *(f32x4*)(link.hidden + (size_t)m * N + n_first) = x;
+  const unsigned halves[4] = {columns.low.x << 16, columns.low.x & 0xffff0000u, columns.low.y << 16, columns.low.y & 0xffff0000u};
+  const unsigned words[4] = {columns.low.x, columns.low.y, columns.high.x, columns.high.y};
+  bf16_t row[4];
+  float squares = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    row[i] = (bf16_t)(x[i] * __uint_as_float(link.weight_is_float ? words[i] : halves[i]));
+    squares = fmaf(x[i], x[i], squares);
+  }
+  *(uint2*)(link.rows + (size_t)m * N + n_first) = *(const uint2*)row;
+  squares += __shfl_xor(squares, 16, WAVE);
+  squares += __shfl_xor(squares, 32, WAVE);
+  if (n_first % 16 == 0) link.sums[(size_t)(n_first / 16) * link.stride + m] = squares;
+}
+
+// This thread's share of the sums of squares of row threadIdx.x % ROWS: the tiles threadIdx.x / ROWS, + THREADS / ROWS, ...
+template <int THREADS, int ROWS>
+__device__ __forceinline__ float squares_share(const Link& link, int M) {
+  const float* of_row = link.sums + min((int)threadIdx.x % ROWS, M - 1);
+  float share = 0.f;
+#pragma unroll 8
+  for (int tile = threadIdx.x / ROWS; tile < link.tiles; tile += THREADS / ROWS) share += of_row[(size_t)tile * link.stride];
+  return share;
+}
+// The factor of row m, once every thread's share is in LDS (`shares`, a thread after the other) and a barrier has passed.
+template <int THREADS, int ROWS>
+__device__ __forceinline__ float row_factor(const Link& link, const float* shares, int m) {
+  float squares = 0.f;
+#pragma unroll
+  for (int part = 0; part < THREADS / ROWS; ++part) squares += shares[part * ROWS + m];
+  return rsqrtf(squares * link.inverse_width + link.eps);
+}
+
 template <int WAVES, int MT, typename TO, int GATED>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* __restrict__ x,
                                                                  const bf16_t* __restrict__ w,
@@ -344,12 +417,12 @@ __device__ __forceinline__ void stream_wait_loads() {
 
 // MT: 16-row tiles of x (up to 16 MT rows).  A stage then holds MT chunks of x beside the NT of the
 // weights for every step, and each weight operand meets MT operands of x.
-template <int WAVES, int NT, int MT, int G, typename TO, int GATED>
+template <int WAVES, int NT, int MT, int G, typename TO, int GATED, int LINK = NO_LINK>
 __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* __restrict__ x,
                                                                  const bf16_t* __restrict__ w,
                                                                  const void* __restrict__ bias, int bias_is_float,
                                                                  TO* __restrict__ out, int M, int N, int K,
-                                                                 int k_split, Tail tail) {
+                                                                 int k_split, Tail tail, Link link) {
   extern __shared__ __attribute__((aligned(16))) unsigned char stream_lds[];
   constexpr int OPERANDS = (NT + MT) * G;                // of one group: the weight tiles' steps, then x's
   constexpr int STAGE_BYTES = OPERANDS * STREAM_CHUNK;
@@ -382,7 +455,19 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
       bias_here[i] =
           load_as_float(bias, bias_is_float, min(((int)blockIdx.x * NT + wave / MT) * 16 + g * 4 + i, N - 1));
   }
+  static_assert(LINK != INTO_NORM || (TILES <= WAVES && sizeof(TO) == 4), "a wave finishes one tile of whole sums");
+  static_assert(LINK != SCALED || MT == 1, "up to 16 rows");
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // so that the counts below count the stream alone
+  LinkedColumns columns;  // (ahead of the stream, whose first wait covers them)
+  if (LINK == INTO_NORM) columns = linked_columns(link, (wave % MT) * 16 + r, ((int)blockIdx.x * NT + min(wave, TILES - 1) / MT) * 16 + g * 4, M, N);
+  // The sums of squares [tiles, 16 rows] go into LDS ahead of the stream, whose first wait covers them: a workgroup that waited
+  // for them by themselves lost a trip to memory, and there are several rounds of workgroups (gate/up 11.7 -> 15.6 us).
+  float* raw_sums = (float*)(stream_lds + (WAVES * WAVE_BYTES > WAVES * TILES * 1024 ? WAVES * WAVE_BYTES : WAVES * TILES * 1024));
+  float* shares = raw_sums + (size_t)(link.tiles + 15) / 16 * 256;  // [WAVES][16 rows]
+  if (LINK == SCALED)
+    for (int chunk = wave; chunk * 16 < link.tiles; chunk += WAVES)
+      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(link.sums + chunk * 256 + lane * 4),
+                                       (void __attribute__((address_space(3)))*)(raw_sums + chunk * 256), 16, 0, 0);
 
   auto request = [&](int group, int stage) {
     unsigned char* to = mine + (size_t)stage * STAGE_BYTES;
@@ -437,6 +522,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
   for (int s = 0; s < NT; ++s)
 #pragma unroll
     for (int t = 0; t < MT; ++t) *(f32x4*)(partial + ((wave * TILES + s * MT + t) * 64 + lane) * 4) = acc[s][t];
+  if (LINK == SCALED) {  // every wave adds up its share of the tiles' sums
+    float squares = 0.f;
+    for (int tile = wave * 4 + g; tile < link.tiles; tile += WAVES * 4) squares += raw_sums[tile * 16 + r];
+    squares += __shfl_xor(squares, 16, WAVE);
+    squares += __shfl_xor(squares, 32, WAVE);
+    if (g == 0) shares[wave * 16 + r] = squares;
+  }
   __syncthreads();
   for (int tile = wave; tile < TILES; tile += WAVES) {
     const int s = tile / MT;
@@ -452,7 +544,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
 #pragma unroll
       for (int i = 0; i < 4; ++i) total[i] += load_as_float(bias, bias_is_float, min(n_first + i, N - 1));
     }
-    if (GATED == 3) {
+    if (LINK == SCALED) {
+      const float factor = row_factor<WAVES * 16, 16>(link, shares, m);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) total[i] *= factor;  // (such a product has no bias)
+    }
+    if (LINK == INTO_NORM) {
+      store_into_norm(link, columns, total, m, n_first, N);
+    } else if (GATED == 3) {
       store_with_tail(out, tail, m, n_first, N, total);
     } else if (GATED) {
       TO* dst = out + (size_t)m * (N / 2) + n_first / 2;
@@ -472,25 +571,32 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
   }
 }
 
-template <int WAVES, int NT, int MT, int G, typename TO, int GATED>
+template <int WAVES, int NT, int MT, int G, typename TO, int GATED, int LINK = NO_LINK>
 static int launch_stream(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N,
-                         int K, int splits, hipStream_t stream, Tail tail = {}) {
+                         int K, int splits, hipStream_t stream, Tail tail = {}, Link link = {}) {
   const size_t stages = (size_t)WAVES * STREAM_STAGES * (NT + MT) * G * STREAM_CHUNK;
   const size_t sums = (size_t)WAVES * NT * MT * 64 * 4 * sizeof(float);
-  const size_t lds = stages > sums ? stages : sums;
+  const size_t lds = (stages > sums ? stages : sums) + (LINK == SCALED ? ((size_t)(link.tiles + 15) / 16 * 256 + WAVES * 16) * sizeof(float) : 0);
   if (lds > 64 * 1024) {
     static bool asked = false;
     if (!asked) {
-      if (hipFuncSetAttribute((const void*)gemm_stream_kernel<WAVES, NT, MT, G, TO, GATED>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+      if (hipFuncSetAttribute((const void*)gemm_stream_kernel<WAVES, NT, MT, G, TO, GATED, LINK>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, LINK == SCALED ? 80 * 1024 : (int)lds) != hipSuccess)
         return ERR_BAD_ARGUMENT;
       asked = true;
     }
   }
-  hipLaunchKernelGGL((gemm_stream_kernel<WAVES, NT, MT, G, TO, GATED>), dim3((N + 16 * NT - 1) / (16 * NT), splits),
+  hipLaunchKernelGGL((gemm_stream_kernel<WAVES, NT, MT, G, TO, GATED, LINK>), dim3((N + 16 * NT - 1) / (16 * NT), splits),
                      dim3(WAVES * 64), lds, stream, (const bf16_t*)x, (const bf16_t*)w, bias, bias_is_float, (TO*)out, M,
-                     N, K, K / splits, tail);
+                     N, K, K / splits, tail, link);
   return LAUNCH_STATUS();
+}
+
+// two tiles a wave for a middling number of weight rows over a K that is not cut (the qkv products of the
+// 7B and 32B sizes: 11.6 -> 10.6 and 20.0 -> 17.5 us); with K cut over workgroups one tile is as good or
+// better (the 32B sizes' o in two parts: 13.5 us against 16.9)
+static bool streams_by_two(long tiles, int K, int splits) {
+  return splits == 1 && tiles >= 256 && tiles < 1024 && tiles * K >= 1000000L;
 }
 
 // One tile a wave in groups of four steps, or two tiles in groups of two.  Measured at 8 rows against
@@ -524,10 +630,7 @@ static int pick_stream(const void* x, const void* w, const void* bias, int bias_
 #undef ROWS_CASE
     return ERR_BAD_ARGUMENT;
   }
-  // two tiles a wave for a middling number of weight rows over a K that is not cut (the qkv products of the
-  // 7B and 32B sizes: 11.6 -> 10.6 and 20.0 -> 17.5 us); with K cut over workgroups one tile is as good or
-  // better (the 32B sizes' o in two parts: 13.5 us against 16.9)
-  if (splits == 1 && tiles >= 256 && tiles < 1024 && tiles * K >= 1000000L)
+  if (streams_by_two(tiles, K, splits))
     return launch_stream<4, 2, 1, 2, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, tail);
   return launch_stream<4, 1, 1, 4, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, tail);
 }
@@ -569,13 +672,13 @@ extern "C" int llmserve_gemm_stream_shaped(const void* x, const void* w, const v
 // A kernel of its own that merges costs a decode step as much as the attention itself (a launch and two
 // trips to memory); here the lanes that load x for the MFMA's B operand merge as they load.  Heads are
 // 128 wide, a group of K (128 k), so a wave's group is one head and its S coefficients are made once.
-template <int WAVES, int S>
+template <int WAVES, int S, int LINK>
 __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* __restrict__ split_x,
                                                                  const float* __restrict__ split_ml,
                                                                  const bf16_t* __restrict__ w,
                                                                  const void* __restrict__ bias, int bias_is_float,
                                                                  float* __restrict__ out, int M, int N, int K,
-                                                                 int k_split) {
+                                                                 int k_split, Link link) {
   extern __shared__ float partial[];  // [WAVES][64 lanes][4]
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
@@ -593,6 +696,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* _
     for (int i = 0; i < 4; ++i)
       bias_here[i] = load_as_float(bias, bias_is_float, min((int)blockIdx.x * 16 + g * 4 + i, N - 1));
   }
+  LinkedColumns columns;  // (asked for now and used at the end, by the first wave)
+  if (LINK == INTO_NORM) columns = linked_columns(link, row, (int)blockIdx.x * 16 + g * 4, M, N);
   const int groups = k_split / (STEP * GROUP);
   for (int group = wave; group < groups; group += WAVES) {
     bf16x8 a[GROUP];
@@ -642,42 +747,74 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* _
   for (int v = 0; v < WAVES; ++v) total_tile += *(const f32x4*)(partial + (v * 64 + lane) * 4);
   const int n_first = blockIdx.x * 16 + g * 4;
   if (r >= M) return;
+  if (LINK == INTO_NORM) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) total_tile[i] += bias_here[i];
+    store_into_norm(link, columns, total_tile, r, n_first, N);
+    return;
+  }
   float* dst = out + ((size_t)blockIdx.y * M + r) * N + n_first;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     if (n_first + i < N) dst[i] = total_tile[i] + bias_here[i];
 }
 
-template <int S>
+template <int S, int LINK>
 static int launch_merged(const void* split_x, const float* split_ml, const void* w, const void* bias, int bias_is_float,
-                         float* out, int M, int N, int K, int k_splits, hipStream_t stream) {
+                         float* out, int M, int N, int K, int k_splits, hipStream_t stream, Link link) {
   const int groups = K / k_splits / (STEP * GROUP);
   const dim3 grid((N + 15) / 16, k_splits);
-  if (groups <= 4)
-    hipLaunchKernelGGL((gemm_merged_kernel<4, S>), grid, dim3(256), 4 * 64 * 4 * sizeof(float), stream,
-                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits);
+  if (LINK == INTO_NORM && groups > 8)  // whole sums: a head a wave, or two
+    hipLaunchKernelGGL((gemm_merged_kernel<12, S, LINK>), grid, dim3(768), 12 * 64 * 4 * sizeof(float), stream,
+                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link);
+  else if (groups <= 4)
+    hipLaunchKernelGGL((gemm_merged_kernel<4, S, LINK>), grid, dim3(256), 4 * 64 * 4 * sizeof(float), stream,
+                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link);
   else
-    hipLaunchKernelGGL((gemm_merged_kernel<8, S>), grid, dim3(512), 8 * 64 * 4 * sizeof(float), stream,
-                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits);
+    hipLaunchKernelGGL((gemm_merged_kernel<8, S, LINK>), grid, dim3(512), 8 * 64 * 4 * sizeof(float), stream,
+                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link);
   return LAUNCH_STATUS();
 }
 
 // out [k_splits, M, N] float32 partial sums of x . w^T (+ bias in the first), x [M, K] being the merge of
 // split_x bfloat16 [K / 128, splits, 16, 16 rows, 8] with split_ml float32 [K / 128, splits, 16 rows, 2] as above.
 // M <= 16; K a multiple of 128 * k_splits; splits 2, 3, 4, 6 or 8.
+template <int LINK>
+static int pick_merged(const void* split_x, const float* split_ml, int splits, const void* w, const void* bias, int bias_is_float,
+                       float* out, int M, int N, int K, int k_splits, hipStream_t stream, Link link) {
+  switch (splits) {
+    case 2: return launch_merged<2, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link);
+    case 3: return launch_merged<3, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link);
+    case 4: return launch_merged<4, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link);
+    case 6: return launch_merged<6, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link);
+    case 8: return launch_merged<8, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link);
+    default: return ERR_BAD_ARGUMENT;
+  }
+}
+
 extern "C" int llmserve_gemm_merged(const void* split_x, const float* split_ml, int splits, const void* w,
                                     const void* bias, int bias_is_float, float* out, int M, int N, int K,
                                     int k_splits, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 16 || K <= 0 || k_splits < 1 || K % (STEP * GROUP * k_splits)) return ERR_BAD_ARGUMENT;
-  switch (splits) {
-    case 2: return launch_merged<2>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream);
-    case 3: return launch_merged<3>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream);
-    case 4: return launch_merged<4>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream);
-    case 6: return launch_merged<6>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream);
-    case 8: return launch_merged<8>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream);
-    default: return ERR_BAD_ARGUMENT;
-  }
+  return pick_merged<NO_LINK>(split_x, split_ml, splits, w, bias, bias_is_float, out, M, N, K, k_splits, stream, Link{});
+}
+
+static int sums_stride(int M) { return M <= 16 ? 16 : M <= 32 ? 32 : 64; }
+
+// The product (split_x null: of x; else of the merge of its key splits, as above, M <= 16) into a norm: hidden [M, N] float32 +=
+// x . w^T (+ bias); rows [M, N] bfloat16 = hidden * weight; sums float32 [N / 16, 16 rows, or 32 or 64: as many as hold M].
+// M <= 64, N a multiple of 16, K of 128.
+extern "C" int llmserve_gemm_into_norm(const void* x, const void* split_x, const float* split_ml, int splits, const void* w, const void* bias,
+                                       int bias_is_float, float* hidden, const void* weight, int weight_is_float, void* rows, float* sums,
+                                       int M, int N, int K, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (M > 64 || N % 16 || K <= 0 || K % (STEP * GROUP) || (split_x && M > 16) || (!x && !split_x)) return ERR_BAD_ARGUMENT;
+  const Link link{hidden, weight, weight_is_float, (bf16_t*)rows, sums, sums_stride(M), N / 16, 0.f, 0.f};
+  if (split_x) return pick_merged<INTO_NORM>(split_x, split_ml, splits, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, link);
+  if (M <= 16) return launch_stream<4, 1, 1, 4, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
+  if (M <= 32) return launch_stream<4, 1, 2, 2, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
+  return launch_stream<4, 1, 4, 1, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
 }
 
 // ---------------------------------------------------------------------------- 16 < M <= 64
@@ -880,10 +1017,10 @@ __device__ __forceinline__ void ring_wait(int younger) {
   }
 }
 
-template <int NT, int MT, int KSTEPS, int DEPTH, typename TO, bool GATED>
+template <int NT, int MT, int KSTEPS, int DEPTH, typename TO, bool GATED, int LINK = NO_LINK>
 __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                         const void* __restrict__ bias, int bias_is_float,
-                                                        TO* __restrict__ out, int M, int N, int K, int k_split) {
+                                                        TO* __restrict__ out, int M, int N, int K, int k_split, Link link) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
   constexpr int XPW = MT > 4 ? MT / 4 : 1;   // tiles of x a wave multiplies
   constexpr int XGROUPS = MT / XPW;          // groups of waves by their tiles of x
@@ -955,7 +1092,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
 #pragma unroll
   for (int s = 0; s < DEPTH - 1; ++s)
     if (s < stages) request(s);
-  for (int stage = 0; stage < stages; ++stage) {
+  auto one_stage = [&](int stage) {
     // this wave's loads of the stage have landed once only the younger stages' are under way
     ring_wait<PER_WAVE, DEPTH - 2>(stages - 1 - stage);
     // everyone's have, and everyone has read the stage before this one: it may be filled again
@@ -983,6 +1120,22 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
 #pragma unroll
         for (int j = 0; j < XPW; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(from_w[i][u], from_x[j][u], acc[i][j], 0, 0, 0);
+  };
+  int stage = 0;
+  float* shares = (float*)(ring + (size_t)DEPTH * STAGE_BYTES);
+  if constexpr (LINK == SCALED) {
+    // the rows' factors are asked for behind the last stages' loads, and come back while those are multiplied
+    for (; stage < stages - 2; ++stage) one_stage(stage);
+    shares[threadIdx.x] = squares_share<256, 16 * MT>(link, M);
+  }
+  for (; stage < stages; ++stage) one_stage(stage);
+  float factor[XPW];
+#pragma unroll
+  for (int t = 0; t < XPW; ++t) factor[t] = 1.f;
+  if constexpr (LINK == SCALED) {
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < XPW; ++t) factor[t] = row_factor<256, 16 * MT>(link, shares, (x_tile + t) * 16 + r);
   }
 
   // The results leave through LDS as whole rows of the workgroup's tile, 16 bytes a lane, where the sizes allow it
@@ -1006,7 +1159,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
       for (int i = 0; i < MINE; ++i) {
         f32x4 total = acc[i][t];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) total[j] += bias_here[i][j];
+        for (int j = 0; j < 4; ++j) total[j] = LINK == SCALED ? total[j] * factor[t] : total[j] + bias_here[i][j];
         const int c_first = (first_tile + WAYS * i) * 16 + g * 4;  // column of the tile before gating
         if (GATED) {
           TO* dst = tile + m * COLUMNS + c_first / 2;
@@ -1040,7 +1193,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
       const int n_first = ((int)blockIdx.x * NT + first_tile + WAYS * i) * 16 + g * 4;
       f32x4 total = acc[i][t];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) total[j] += bias_here[i][j];
+      for (int j = 0; j < 4; ++j) total[j] = LINK == SCALED ? total[j] * factor[t] : total[j] + bias_here[i][j];
       if (GATED) {
         TO* dst = out + (size_t)m * (N / 2) + n_first / 2;
 #pragma unroll
@@ -1060,23 +1213,23 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
   }
 }
 
-template <int NT, int MT, int KSTEPS, int DEPTH, typename TO, bool GATED>
+template <int NT, int MT, int KSTEPS, int DEPTH, typename TO, bool GATED, int LINK = NO_LINK>
 static int launch_ring(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
-                       int splits, hipStream_t stream) {
-  const size_t lds = (size_t)DEPTH * (NT + MT) * KSTEPS * STREAM_CHUNK;
+                       int splits, hipStream_t stream, Link link = {}) {
+  const size_t lds = (size_t)DEPTH * (NT + MT) * KSTEPS * STREAM_CHUNK + (LINK == SCALED ? 256 * sizeof(float) : 0);
   if ((K / splits) % (KSTEPS * STEP)) return ERR_BAD_ARGUMENT;
   if (lds > 64 * 1024) {
     static bool asked = false;
     if (!asked) {
-      if (hipFuncSetAttribute((const void*)gemm_ring_kernel<NT, MT, KSTEPS, DEPTH, TO, GATED>,
+      if (hipFuncSetAttribute((const void*)gemm_ring_kernel<NT, MT, KSTEPS, DEPTH, TO, GATED, LINK>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return ERR_BAD_ARGUMENT;
       asked = true;
     }
   }
-  hipLaunchKernelGGL((gemm_ring_kernel<NT, MT, KSTEPS, DEPTH, TO, GATED>), dim3((N + 16 * NT - 1) / (16 * NT), splits),
+  hipLaunchKernelGGL((gemm_ring_kernel<NT, MT, KSTEPS, DEPTH, TO, GATED, LINK>), dim3((N + 16 * NT - 1) / (16 * NT), splits),
                      dim3(256), lds, stream, (const bf16_t*)x, (const bf16_t*)w, bias, bias_is_float, (TO*)out, M, N, K,
-                     K / splits);
+                     K / splits, link);
   return LAUNCH_STATUS();
 }
 
@@ -1130,6 +1283,55 @@ extern "C" int llmserve_gemm_ring(const void* x, const void* w, const void* bias
                       : pick_ring<bf16_t, false>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, nt);
 }
 
+// Weight tiles a wave of the kernels for up to 16 rows shares its x between: several where a wave has many groups of K to
+// walk (or x is all 16 rows) and enough workgroups are left (measured at the 1.5B and 7B sizes).
+static int skinny_share(int M, int N, int K, int splits) {
+  const int per_wave = K / splits / (STEP * GROUP) / 4;
+  const long tiles = (N + 15) / 16;
+  const long by_four = (tiles + 3) / 4 * splits, by_two = (tiles + 1) / 2 * splits;  // workgroups
+  return (per_wave >= 8 && by_four >= 128 && (M > 2 || tiles <= 1024)) || (tiles >= 4096 && M >= 4) ? 4
+         : (per_wave >= 4 || M > 8 || (tiles >= 4096 && M >= 4)) && by_two * 4 >= TARGET_WAVES ? 2
+                                                                                                 : 1;
+}
+// Whether such a product goes through LDS (gemm_stream): with one or two tiles, unless many rows of x meet a long walk over K.
+static bool skinny_streams(int M, int N, int K, int splits) {
+  const int share = skinny_share(M, N, K, splits);
+  return share != 4 && !(share == 2 && M > 8 && K / splits / (STEP * GROUP) / 4 >= 4);
+}
+
+#define SCALED_STREAM_K 3840  // the sums of so long a row leave room for two workgroups of gemm_stream in a CU's LDS
+
+// silu(gate) * up, bfloat16 [M, N / 2], of rows that a product into a norm has left (`rows` [M, K], `sums` as there, in a
+// buffer of whole KB): every result
+// times rsqrt(sum of the row's sums / K + eps).  tiles 0: through gemm_stream, M <= 16; else through gemm_ring with so many
+// weight tiles a workgroup.
+extern "C" int llmserve_gemm_scaled(const void* rows, float* sums, float eps, const void* w, void* out, int tiles, int M, int N, int K,
+                                    hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (M > 64 || K <= 0 || K % (STEP * GROUP) || N % 2 || (tiles == 0 && (M > 16 || K > SCALED_STREAM_K))) return ERR_BAD_ARGUMENT;
+  const Link link{nullptr, nullptr, 0, nullptr, sums, sums_stride(M), K / 16, 1.f / (float)K, eps};
+  if (tiles == 0) return launch_stream<4, 1, 1, 4, bf16_t, 1, SCALED>(rows, w, nullptr, 0, out, M, N, K, 1, stream, {}, link);
+#define SCALED_CASE(NT_, KSTEPS_)                                                                                      \
+  if (tiles == NT_)                                                                                                    \
+    return M <= 32 ? launch_ring<NT_, 2, KSTEPS_, 4, bf16_t, true, SCALED>(rows, w, nullptr, 0, out, M, N, K, 1, stream, link) \
+                   : launch_ring<NT_, 4, KSTEPS_, 4, bf16_t, true, SCALED>(rows, w, nullptr, 0, out, M, N, K, 1, stream, link);
+  SCALED_CASE(2, 4)
+  SCALED_CASE(4, 4)
+  SCALED_CASE(6, 4)
+  SCALED_CASE(8, 2)
+  SCALED_CASE(10, 2)
+  SCALED_CASE(12, 2)
+  SCALED_CASE(14, 2)
+#undef SCALED_CASE
+  if (tiles == 5 && M > 32) return launch_ring<5, 4, 4, 4, bf16_t, true, SCALED>(rows, w, nullptr, 0, out, M, N, K, 1, stream, link);
+  return ERR_BAD_ARGUMENT;
+}
+
+// Whether the kernel and shape of llmserve_gemm_scaled with tiles 0 is what a gated product of these sizes takes without the norm.
+extern "C" int llmserve_gemm_scaled_streams(int M, int N, int K) {
+  return M > 0 && M <= 16 && K > 0 && K <= SCALED_STREAM_K && K % (STEP * GROUP) == 0 && skinny_streams(M, N, K, 1) && !streams_by_two((N + 15) / 16, K, 1);
+}
+
 // x, w bfloat16; out bfloat16 or float32.  Needs 1 <= M <= 64, K a multiple of 32, and with
 // `gated` (1: silu(gate) * up, 2: relu(gate) * up) an even N.  Any N.  With splits > 1 (float32 out, not gated, K / splits a multiple of
 // 32) `out` is [splits, M, N]: slice s holds the sums over the s-th part of K (the bias in slice 0),
@@ -1138,16 +1340,8 @@ static int skinny_entry(const void* x, const void* w, const void* bias, int bias
                         int M, int N, int K, int splits, hipStream_t stream, Tail tail) {
   if (splits > 1 && (gated || !out_is_float || K % splits || (K / splits) % STEP)) return ERR_BAD_ARGUMENT;
   if (M <= 16 && (K / splits) % (STEP * GROUP) == 0) {
-    // several weight tiles a wave where a wave has many groups of K to walk (or x is all 16 rows) and
-    // enough workgroups are left (measured at the 1.5B and 7B sizes)
-    const int per_wave = K / splits / (STEP * GROUP) / 4;
-    const long tiles = (N + 15) / 16;
-    const long by_four = (tiles + 3) / 4 * splits, by_two = (tiles + 1) / 2 * splits;  // workgroups
-    const int share = (per_wave >= 8 && by_four >= 128 && (M > 2 || tiles <= 1024)) || (tiles >= 4096 && M >= 4) ? 4
-                      : (per_wave >= 4 || M > 8 || (tiles >= 4096 && M >= 4)) && by_two * 4 >= TARGET_WAVES ? 2
-                                                                                                            : 1;
-    // Two tiles or one: through LDS (gemm_stream), unless many rows of x meet a long walk over K.
-    if (share != 4 && !(share == 2 && M > 8 && per_wave >= 4)) {
+    const int share = skinny_share(M, N, K, splits);
+    if (skinny_streams(M, N, K, splits)) {
       if (gated == 3) return pick_stream<bf16_t, 3>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, 0, 0, tail);
       if (gated == 2)
         return out_is_float ? pick_stream<float, 2>(x, w, bias, bias_is_float, out, M, N, K, 1, stream)

@@ -69,6 +69,9 @@ _SIGNATURES = {
     "llmserve_gemm_medium": "pppipiiiiiip",
     "llmserve_gemm_ring": "pppipiiiiiiip",
     "llmserve_gemm_merged": "ppippipiiiip",
+    "llmserve_gemm_into_norm": "pppippippippiiip",
+    "llmserve_gemm_scaled": "ppfppiiiip",
+    "llmserve_gemm_scaled_streams": "iii",
     "llmserve_gemm_blocks": "pppipiiiiiip",
     "llmserve_gemm_blocks_parts": "iii",
     "llmserve_attention_generic": "pipiipppippiiiiifipfpiiipip",
@@ -177,6 +180,27 @@ class GatedLinearWeights:
     width: int
     activation: str = "silu"
     limit: float = 0.0  # of "limited_swish"
+
+
+@dataclass
+class NormInto:
+    """What a product is told when the norm behind it may be made by it and the product that reads the normed rows
+    (`HipKernels.norm_into`): the stream it adds into, the norm, and that reader."""
+
+    hidden: torch.Tensor
+    weight: torch.Tensor
+    eps: float
+    reader: GatedLinearWeights
+
+
+@dataclass
+class ScaledRows:
+    """Rows times a norm's weight that are not yet divided by their root mean square: `sums` [width / 16, rows] are the sums of
+    squares, of 16 columns each, that their reader divides by."""
+
+    rows: torch.Tensor
+    sums: torch.Tensor
+    eps: float
 
 
 class HipKernels:
@@ -693,8 +717,62 @@ class HipKernels:
                 best = splits
         return best
 
-    def gated_linear(self, x: torch.Tensor, weights: GatedLinearWeights) -> torch.Tensor:
+    def norm_into(self, hidden: torch.Tensor, weight: torch.Tensor, eps: float, reader: GatedLinearWeights) -> NormInto:
+        return NormInto(hidden, weight, eps, reader)
+
+    def _linear_into_norm(self, x, split: tuple | None, project: LinearWeights, into: NormInto) -> ScaledRows | None:
+        """`into.hidden += linear(x, project)` (or of the merge of key splits: `split` is what the attention left) and the rows that
+        `into.reader` reads, where both products are of the kernels that do a norm between them; else None, and nothing done.
+        Up to 64 rows: those of the kernels for a few rows, the first with whole sums over K (the 1.5B sizes' output projection
+        costs 1.6 us more than in three parts, at 64 rows 2.7; the norm's kernel 4.4 and 4.7)."""
+        hidden, reader = into.hidden, into.reader
+        rows, width = hidden.shape
+        weight = reader.both.weight
+        if (
+            self.dtype != torch.bfloat16 or not 0 < rows <= 64 or width % 128 or project.out_features != width or project.in_features % 128
+            or project.weight.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or reader.activation != "silu"
+            or reader.both.in_features != width or into.weight.dtype not in (torch.bfloat16, torch.float32)
+            or (rows > 16 and project.out_features * project.in_features > (1 << 22))
+        ):
+            return None
+        like_rows = x if x is not None and x.shape[1] == width else torch.empty((rows, width), dtype=torch.bfloat16, device="meta")
+        route = self._streaming(like_rows, reader.both, gated=True)
+        if route == "ring":
+            tiles = self._ring_shape(rows, 2 * reader.width, width, False)[0]
+        elif route == "skinny" and rows <= 16 and self._gemm_bf16.llmserve_gemm_scaled_streams(rows, 2 * reader.width, width):
+            tiles = 0
+        else:
+            return None
+        stride = 16 if rows <= 16 else 32 if rows <= 32 else 64
+        scaled = self._empty((rows, width), torch.bfloat16)
+        sums = self._empty((-(-width // 256) * 16, stride), torch.float32)  # (whole KB: the reader brings them to LDS by the KB)
+        split_x, split_ml, splits = split if split is not None else (None, None, 0)
+        bias = project.bias
+        status = self._gemm_bf16.llmserve_gemm_into_norm(
+            _pointer(x) if split is None else None, _pointer(split_x), _pointer(split_ml), splits, _pointer(project.weight), _pointer(bias),
+            _is_float(bias) if bias is not None else 0, _pointer(hidden), _pointer(into.weight), _is_float(into.weight), _pointer(scaled),
+            _pointer(sums), rows, width, project.in_features, self._stream,
+        )
+        _check(status, "linear into a norm")
+        return ScaledRows(scaled, sums, into.eps)
+
+    def _scaled_gated_linear(self, x: ScaledRows, weights: GatedLinearWeights) -> torch.Tensor:
+        rows, width = x.rows.shape
+        out = self._empty((rows, weights.width), self.dtype)
+        tiles = 0
+        if self._streaming(x.rows, weights.both, gated=True) == "ring":
+            tiles = self._ring_shape(rows, 2 * weights.width, width, False)[0]
+        status = self._gemm_bf16.llmserve_gemm_scaled(
+            _pointer(x.rows), _pointer(x.sums), x.eps, _pointer(weights.both.weight), _pointer(out), tiles, rows, 2 * weights.width, width,
+            self._stream,
+        )
+        _check(status, "gated_linear of scaled rows")
+        return out
+
+    def gated_linear(self, x: torch.Tensor | ScaledRows, weights: GatedLinearWeights) -> torch.Tensor:
         """silu (or another activation) of the even rows' products times the odd rows'."""
+        if isinstance(x, ScaledRows):
+            return self._scaled_gated_linear(x, weights)
         out = self._empty((x.shape[0], weights.width), self.dtype)
         if (
             weights.activation == "relu"
@@ -1233,19 +1311,25 @@ class HipKernels:
     def rotate_store_attend(
         self, qkv, layout, batch, cell, inverse_frequencies, pairing: str, scale: float, window: int | None,
         project: LinearWeights | None = None, *, sinks: torch.Tensor | None = None, chunk: int | None = None, out: torch.Tensor | None = None,
-    ) -> torch.Tensor:
+        into: NormInto | None = None,
+    ) -> torch.Tensor | ScaledRows:
         """`rotate_and_store` followed by `paged_attention`; one kernel when every request of
         the step brings a single token and the MFMA kernel takes the sizes.  With `project`, the result
         is `linear(that, project, float32, partial=True)`: for up to 16 single tokens at head size 128
-        the attention leaves its key splits unmerged and the product merges them as it loads its x."""
+        the attention leaves its key splits unmerged and the product merges them as it loads its x.  With `into`
+        too, the product may add to the stream itself and leave rows for the norm's reader (`ScaledRows`)."""
         if project is not None and out is not None:
             raise KernelError("rotate_store_attend: the result goes to given rows or through a product")
-        out, projected = self._rotate_store_attend(qkv, layout, batch, cell, inverse_frequencies, pairing, scale, window, project, sinks, chunk, out)
+        out, projected = self._rotate_store_attend(qkv, layout, batch, cell, inverse_frequencies, pairing, scale, window, project, sinks, chunk, out, into)
         if project is None or projected:
             return out
+        if into is not None and batch.max_query_length == 1:
+            scaled = self._linear_into_norm(out, None, project, into)
+            if scaled is not None:
+                return scaled
         return self.linear(out, project, out_dtype=torch.float32, partial=True)
 
-    def _rotate_store_attend(self, qkv, layout, batch, cell, inverse_frequencies, pairing, scale, window, project, sinks, chunk, out):
+    def _rotate_store_attend(self, qkv, layout, batch, cell, inverse_frequencies, pairing, scale, window, project, sinks, chunk, out, into):
         """(the attention's output, False) or, where the key splits were left to the product, (the product's, True)."""
         group = batch.groups[cell.group]
         dim = layout.head_dim
@@ -1290,6 +1374,10 @@ class HipKernels:
             if left is None:
                 return out, False
             split_x, split_ml, splits = left
+            if into is not None:
+                scaled = self._linear_into_norm(None, left, project, into)
+                if scaled is not None:
+                    return scaled, True
             k_splits = self._partial_splits(project.out_features, project.in_features)
             shape = (rows, project.out_features) if k_splits == 1 else (k_splits, rows, project.out_features)
             result = self._empty(shape, torch.float32)

@@ -97,10 +97,15 @@ class Attention(Mixer):
         self.position = POSITIONS.build(spec.position, own, kernels)
         self.replayable = self.position.replayable
 
-    def forward(self, x: torch.Tensor, batch, cell) -> torch.Tensor:
+    @property
+    def takes_into(self) -> bool:
+        """Whether `forward` can be told of the norm behind it (`into`)."""
+        return getattr(self.position, "takes_into", False)
+
+    def forward(self, x: torch.Tensor, batch, cell, **into) -> torch.Tensor:
         qkv = self.kernels.linear(x, self.qkv)
         # the output projection goes with the attention: a kernel library may fuse the two (key splits of
         # a decode step merged by the product that reads them)
         return self.position.encode_store_attend(
-            qkv, self.layout, batch, cell, self.spec.scale, self.spec.window, project=self.out
+            qkv, self.layout, batch, cell, self.spec.scale, self.spec.window, project=self.out, **into
         )

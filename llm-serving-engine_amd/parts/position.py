@@ -88,9 +88,11 @@ class Rotary(PositionEncoding):
             qkv, layout, batch, cell, self.inverse_frequencies, self.spec.pairing
         )
 
-    def encode_store_attend(self, qkv, layout: HeadLayout, batch, cell, scale: float, window, project=None):
+    takes_into = True
+
+    def encode_store_attend(self, qkv, layout: HeadLayout, batch, cell, scale: float, window, project=None, **into):
         return self.kernels.rotate_store_attend(
-            qkv, layout, batch, cell, self.inverse_frequencies, self.spec.pairing, scale, window, project=project
+            qkv, layout, batch, cell, self.inverse_frequencies, self.spec.pairing, scale, window, project=project, **into
         )
 
 
