@@ -458,7 +458,10 @@ class ModelRunner:
 
     @staticmethod
     def _token_bucket(tokens: int) -> int:
-        for size in (16, 32, 64, 96, 128, 192, 256, 384, 512, 768, 1024):
+        """The tokens of the graph that a step of so many replays: few shapes, and no more than a quarter of padding from 129 on,
+        where a step's time goes by its rows (287 tokens of the 1.5B sizes in a graph of 384 rows 3.09 ms, of 320 2.93; 129
+        in float32 6.97 in 192 rows, 6.52 in 160)."""
+        for size in (16, 32, 64, 96, 128, 160, 192, 224, 256, 320, 384, 448, 512, 768, 1024):
             if tokens <= size:
                 return size
         return -(-tokens // 512) * 512
