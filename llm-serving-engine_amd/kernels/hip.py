@@ -1294,6 +1294,17 @@ class HipKernels:
                     held = 16 if unmerged else tokens  # the product that merges wants 16 rows side by side
                     partial_acc = self._empty((held * heads * maps * splits * layout.head_dim,), qkv.dtype if unmerged else torch.float32)
                     partial_ml = self._empty((held * heads * maps * splits * 2,), torch.float32)
+            elif column_tiles == 2 and changed is None and finish is None:
+                # A portion beside decoded tokens whose contexts are long: few items, and the longest walked by one workgroup.
+                # Cut into runs of at least 32 steps of 32 keys, up to about 512 workgroups in all, and merged.  Us a layer,
+                # whole (four waves) against runs with their merging: 8 tokens over 4,000 keys beside a portion of 64 at the 1.5B
+                # sizes 72.7 and 22.4 (whole with eight waves 58.7), 24 over 2,500 beside 200 48.3 and 29.1; 6 over 2,500
+                # beside 100 at the 7B sizes 47.0 and 31.4.
+                blocks = items * kv_heads * head_tiles
+                splits = max(1, min(-(-self._walked_keys(batch, window, keep_first, chunk) // 32) // 32, 512 // blocks, 8))
+                if splits > 1:
+                    partial_acc = self._empty((tokens * heads * splits * layout.head_dim,), torch.float32)
+                    partial_ml = self._empty((tokens * heads * splits * 2,), torch.float32)
             table, pairing = fuse if fuse is not None else (None, "none")
             status = library.llmserve_attention_tiles(
                 _pointer(qkv), layout.stride, _pointer(out), out.shape[1], _pointer(partial_acc), _pointer(partial_ml),

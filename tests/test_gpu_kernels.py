@@ -912,6 +912,24 @@ def test_rotation_store_and_attention_of_prompt_portions(kernels, dtype, pairing
     torch.testing.assert_close(stored_v, want_v, atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,window", [(6, 2, 64, None), (6, 1, 128, None), (8, 4, 128, 2048), (5, 1, 32, None), (4, 2, 160, None)])
+@pytest.mark.parametrize("lengths,counts", [([3000, 20, 2100, 700, 1], [1, 20, 60, 1, 1]), ([520, 9, 300], [200, 9, 1]), ([4200, 2050], [1, 33])])
+def test_portions_beside_long_contexts(kernels, heads, kv_heads, dim, window, lengths, counts):
+    """A step of portions and decoded tokens whose longest walks are cut into runs that a second kernel merges (short requests
+    in it have no key in the later runs), and whose tiles are walked by eight waves; against the plain attention."""
+    dtype, page = torch.bfloat16, 16
+    batch, cell, per_request, layout = paged_case(lengths, counts, heads, kv_heads, dim, page, dtype, shuffle_seed=dim)
+    out = kernels[dtype].paged_attention(on_gpu(step_rows(per_request, counts, heads, kv_heads, dim), dtype), layout, batch, cell, dim ** -0.5, window)
+    expected = []
+    for (q, k, v), count in zip(per_request, counts):
+        q, k, v = (rounded(rows, dtype).double() for rows in (q[-count:], k, v))
+        k, v = (rows.repeat_interleave(heads // kv_heads, 1).transpose(0, 1) for rows in (k, v))
+        distance = torch.arange(k.shape[1] - count, k.shape[1])[:, None] - torch.arange(k.shape[1])[None]
+        scores = (q.transpose(0, 1) @ k.transpose(1, 2) * dim ** -0.5).masked_fill((distance < 0) | (distance >= (window or 1 << 30)), -math.inf)
+        expected.append((scores.softmax(-1) @ v).transpose(0, 1).flatten(1))
+    torch.testing.assert_close(out.cpu().double(), torch.cat(expected), **TOLERANCE[dtype])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("activation", ["silu", "gelu", "gelu_tanh", "relu"])
 @pytest.mark.parametrize("rows,inner,outer", [(5, 96, 200), (16, 512, 520), (40, 128, 264), (70, 64, 333), (300, 128, 1000)])
