@@ -485,12 +485,17 @@ class HipKernels:
         rows 109 and 124; N = K = 1,536: 192 rows 8.1 and 6.4, 1,024 rows 13.3 and 12.4; N = K = 3,584: 512 rows 22.6 and 20.3, 768 rows 26.4
         and 28.5.  Gated: N 17,920 K 1,536: 256 rows 35 and 29, 384 rows 37 and 30, 512 rows 45 and 44, 1,024 rows 80 and 74, 2,048
         rows 133 and 111; N 37,888 K 3,584: 192 rows 84 and 96, 512 rows 149 and 164, 1,024 rows 315 and 274, 2,048 rows 546 and 474;
-        up to 128 rows the ring's 22.5 and 61 are as good or better.  The rest (the qkv products: 384 rows of N 2,048 K 1,536 9.4 and
-        10.1, of N 4,608 K 3,584 25.2 and 27.7) stays with the library."""
+        up to 128 rows the ring's 22.5 and 61 are as good or better.  Plain ones and results of more tiles: small weights over more than
+        512 rows, up to a result of four million (N 2,048 K 1,536: 384 rows 9.4 and 10.1, 768 rows 12.8 and 11.7, 1,024 rows 13.8 and
+        12.1, 2,048 rows 17.2 and 17.0; whole prompts of the 1.5B sizes with their qkv and output projections here: 520 tokens
+        3.99 -> 3.92 ms, 1,024 5.60 -> 5.51, 1,500 7.19 -> 7.13, 2,048 8.01 -> 7.94).  The rest (384 rows of N 4,608 K 3,584 25.2
+        and 27.7) stays with the library."""
         if in_features % 64:
             return False
         if gated:
             return rows > 128 and (out_features * in_features <= 40_000_000 or rows >= 1024)
+        if rows > 512 and out_features >= 1024 and out_features * in_features <= (1 << 22) and rows * out_features <= (1 << 22):
+            return True
         # (a K of 256s divides into two and four parts of whole stages; else the library's slices may be the only way to cut it)
         return may_split and in_features % 256 == 0 and (rows <= 128 or rows * out_features <= 2_400_000)
 

@@ -151,6 +151,24 @@ def test_tiles_of_many_rows(own_kernels, rows, inner, outer):
         torch.testing.assert_close(parts.double().sum(0), expected, **bound)
 
 
+@pytest.mark.parametrize("rows,inner,outer", [(512, 1536, 2048), (513, 1536, 2048), (2048, 1536, 2048), (2049, 1536, 2048), (513, 64, 1024), (777, 320, 1030), (600, 1536, 1536)])
+def test_small_weights_over_many_rows(kernels, rows, inner, outer):
+    """Both sides of the line from which small plain products are the tiled kernel's, with and without leave to split: a route that takes
+    one and not the other would leave a product to the generic kernel.  Float32 results as in `test_tiles_of_many_rows`."""
+    k, dtype = kernels[torch.bfloat16], torch.bfloat16
+    generator = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, inner, generator=generator, device="cuda").to(dtype)
+    w = torch.randn(outer, inner, generator=generator, device="cuda").div_(math.sqrt(inner)).to(dtype)
+    b = torch.randn(outer, generator=generator, device="cuda").to(dtype)
+    expected, handle = x.double() @ w.double().T + b.double(), k.prepare_linear([w], [b])
+    taken = 512 < rows and rows * outer <= 1 << 22
+    assert (k._streaming(x, handle) == "tiled") == taken and (not taken or k._streaming(x, handle, may_split=True) == "tiled")
+    torch.testing.assert_close(k.linear(x, handle).double(), expected, **TOLERANCE[dtype])
+    parts = k.linear(x, handle, out_dtype=torch.float32, partial=True)
+    summed = parts.double() if parts.ndim == 2 else parts.double().sum(0)
+    torch.testing.assert_close(summed, expected, atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5)
+
+
 def key_pieces(rows):
     """Key pages written as rows [pages, kv, offset, dim] -> as the cache keeps them, in pieces of eight
     elements, the same piece of all the keys of a page side by side: [pages, kv, dim / w, offset, w]
