@@ -1122,20 +1122,27 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(from_w[i][u], from_x[j][u], acc[i][j], 0, 0, 0);
   };
   int stage = 0;
-  float* shares = (float*)(ring + (size_t)DEPTH * STAGE_BYTES);
+  float share = 0.f;
   if constexpr (LINK == SCALED) {
-    // the rows' factors are asked for behind the last stages' loads, and come back while those are multiplied
+    // The sums of squares are asked for two stages before the end, when the last stage has been asked for too: a thread waits
+    // for its own here, and as loads come back in order for those stages with them.
     for (; stage < stages - 2; ++stage) one_stage(stage);
-    shares[threadIdx.x] = squares_share<256, 16 * MT>(link, M);
+    share = squares_share<256, 16 * MT>(link, M);
   }
   for (; stage < stages; ++stage) one_stage(stage);
   float factor[XPW];
 #pragma unroll
   for (int t = 0; t < XPW; ++t) factor[t] = 1.f;
   if constexpr (LINK == SCALED) {
+    // The shares meet in the ring itself (six weight tiles beside four of x leave no byte of a CU's LDS, and eight beside two
+    // no byte of half of it): everyone has read the last stage, and everyone has its factors before results go there.
+    float* shares = (float*)ring;
+    __syncthreads();
+    shares[threadIdx.x] = share;
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < XPW; ++t) factor[t] = row_factor<256, 16 * MT>(link, shares, (x_tile + t) * 16 + r);
+    __syncthreads();
   }
 
   // The results leave through LDS as whole rows of the workgroup's tile, 16 bytes a lane, where the sizes allow it
@@ -1216,7 +1223,8 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
 template <int NT, int MT, int KSTEPS, int DEPTH, typename TO, bool GATED, int LINK = NO_LINK>
 static int launch_ring(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
                        int splits, hipStream_t stream, Link link = {}) {
-  const size_t lds = (size_t)DEPTH * (NT + MT) * KSTEPS * STREAM_CHUNK + (LINK == SCALED ? 256 * sizeof(float) : 0);
+  constexpr size_t lds = (size_t)DEPTH * (NT + MT) * KSTEPS * STREAM_CHUNK;
+  static_assert(lds <= 160 * 1024, "a CU's LDS");
   if ((K / splits) % (KSTEPS * STEP)) return ERR_BAD_ARGUMENT;
   if (lds > 64 * 1024) {
     static bool asked = false;

@@ -16,14 +16,8 @@ def kernels():
     return HipKernels(torch.bfloat16)
 
 
-# rows at the edges of the kernels' tiles; widths whose tiles of 16 columns divide evenly over the threads and not; gated products for
-# the kernel for few rows (short and long K), and for the ring with four, five and ten tiles a workgroup
-@pytest.mark.parametrize("rows", [1, 3, 8, 15, 16, 17, 31, 33, 64])
-@pytest.mark.parametrize("width,inner,gated,bias,norm", [
-    (128, 128, 96, True, torch.float32), (384, 256, 200, False, torch.bfloat16), (1536, 1536, 8960, False, torch.bfloat16),
-    (1664, 896, 9000, True, torch.bfloat16), (3584, 3584, 18944, False, torch.bfloat16),
-])
-def test_linked_products(kernels, rows, width, inner, gated, bias, norm):
+def check_linked(kernels, rows, width, inner, gated, bias=False, norm=torch.float32):
+    """The two linked products against the three steps apart in 64 bits; False where they are of other kernels (and nothing has been done)."""
     generator = torch.Generator(device="cuda").manual_seed(rows + width)
 
     def some(*shape, scale=1.0):
@@ -37,9 +31,9 @@ def test_linked_products(kernels, rows, width, inner, gated, bias, norm):
     reader = kernels.prepare_gated_linear(gate, up)
     stream = hidden.clone()
     scaled = kernels._linear_into_norm(x, None, project, kernels.norm_into(stream, weight, 1e-6, reader))
-    if scaled is None:  # the products are of other kernels at these sizes, and nothing has been done
-        assert torch.equal(stream, hidden) and (rows > 16 or gated > 10000 or width == 3584)
-        return
+    if scaled is None:
+        assert torch.equal(stream, hidden)
+        return False
     got = kernels.gated_linear(scaled, reader).double()
     after = hidden.double() + x.double() @ w.double().T + (b.double() if bias else 0.0)
     # float32 sums of `inner` products of values of size 1
@@ -50,6 +44,27 @@ def test_linked_products(kernels, rows, width, inner, gated, bias, norm):
     # the result; in norm no more than their sum
     assert (got - want).norm() < 3 * 2.0 ** -9 * want.norm()
     torch.testing.assert_close(got, want, atol=3e-2, rtol=3e-2)
+    return True
+
+
+# rows at the edges of the kernels' tiles; widths whose tiles of 16 columns divide evenly over the threads and not; gated products for
+# the kernel for few rows (short and long K), and for the ring with four, five and ten tiles a workgroup
+@pytest.mark.parametrize("rows", [1, 3, 8, 15, 16, 17, 31, 33, 64])
+@pytest.mark.parametrize("width,inner,gated,bias,norm", [
+    (128, 128, 96, True, torch.float32), (384, 256, 200, False, torch.bfloat16), (1536, 1536, 8960, False, torch.bfloat16),
+    (1664, 896, 9000, True, torch.bfloat16), (3584, 3584, 18944, False, torch.bfloat16),
+])
+def test_linked_products(kernels, rows, width, inner, gated, bias, norm):
+    taken = check_linked(kernels, rows, width, inner, gated, bias, norm)
+    assert taken or rows > 16 or gated > 10000 or width == 3584
+
+
+@pytest.mark.parametrize("rows", [33, 48, 64])
+@pytest.mark.parametrize("width,inner,gated", [(256, 128, 10336), (2048, 2048, 11008)])
+def test_six_weight_tiles_beside_four_of_x(kernels, rows, width, inner, gated):
+    """The ring whose stages fill a CU's LDS to the last byte: the second product has no more of it than without a norm."""
+    assert kernels._ring_shape(rows, 2 * gated, width, False)[0] == 6
+    assert check_linked(kernels, rows, width, inner, gated)
 
 
 def test_what_is_not_linked(kernels):
