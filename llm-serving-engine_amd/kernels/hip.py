@@ -196,11 +196,13 @@ class NormInto:
 @dataclass
 class ScaledRows:
     """Rows times a norm's weight that are not yet divided by their root mean square: `sums` [width / 16, rows] are the sums of
-    squares, of 16 columns each, that their reader divides by."""
+    squares, of 16 columns each, that their `reader` divides by; `tiles`: how its kernel is shaped (`llmserve_gemm_scaled`)."""
 
     rows: torch.Tensor
     sums: torch.Tensor
     eps: float
+    reader: GatedLinearWeights
+    tiles: int
 
 
 class HipKernels:
@@ -736,12 +738,15 @@ class HipKernels:
         if (
             self.dtype != torch.bfloat16 or not 0 < rows <= 64 or width % 128 or project.out_features != width or project.in_features % 128
             or project.weight.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or reader.activation != "silu"
-            or reader.both.in_features != width or into.weight.dtype not in (torch.bfloat16, torch.float32)
+            or reader.both.in_features != width or into.weight.dtype not in (torch.bfloat16, torch.float32) or into.weight.shape != (width,)
             or (rows > 16 and project.out_features * project.in_features > (1 << 22))
         ):
             return None
-        like_rows = x if x is not None and x.shape[1] == width else torch.empty((rows, width), dtype=torch.bfloat16, device="meta")
-        route = self._streaming(like_rows, reader.both, gated=True)
+        # (what `linear` and `add_rms_norm` refuse goes on to them)
+        if hidden.dtype != torch.float32 or (split is None and (x.dtype != torch.bfloat16 or x.shape != (rows, project.in_features))):
+            return None
+        scaled = self._empty((rows, width), torch.bfloat16)
+        route = self._streaming(scaled, reader.both, gated=True)
         if route == "ring":
             tiles = self._ring_shape(rows, 2 * reader.width, width, False)[0]
         elif route == "skinny" and rows <= 16 and self._gemm_bf16.llmserve_gemm_scaled_streams(rows, 2 * reader.width, width):
@@ -749,7 +754,6 @@ class HipKernels:
         else:
             return None
         stride = 16 if rows <= 16 else 32 if rows <= 32 else 64
-        scaled = self._empty((rows, width), torch.bfloat16)
         sums = self._empty((-(-width // 256) * 16, stride), torch.float32)  # (whole KB: the reader brings them to LDS by the KB)
         split_x, split_ml, splits = split if split is not None else (None, None, 0)
         bias = project.bias
@@ -759,16 +763,15 @@ class HipKernels:
             _pointer(sums), rows, width, project.in_features, self._stream,
         )
         _check(status, "linear into a norm")
-        return ScaledRows(scaled, sums, into.eps)
+        return ScaledRows(scaled, sums, into.eps, reader, tiles)
 
     def _scaled_gated_linear(self, x: ScaledRows, weights: GatedLinearWeights) -> torch.Tensor:
+        if weights is not x.reader:
+            raise KernelError("gated_linear: the rows were left for another product")
         rows, width = x.rows.shape
         out = self._empty((rows, weights.width), self.dtype)
-        tiles = 0
-        if self._streaming(x.rows, weights.both, gated=True) == "ring":
-            tiles = self._ring_shape(rows, 2 * weights.width, width, False)[0]
         status = self._gemm_bf16.llmserve_gemm_scaled(
-            _pointer(x.rows), _pointer(x.sums), x.eps, _pointer(weights.both.weight), _pointer(out), tiles, rows, 2 * weights.width, width,
+            _pointer(x.rows), _pointer(x.sums), x.eps, _pointer(weights.both.weight), _pointer(out), x.tiles, rows, 2 * weights.width, width,
             self._stream,
         )
         _check(status, "gated_linear of scaled rows")

@@ -15,7 +15,7 @@ from types import SimpleNamespace
 import pytest
 import torch
 
-from llmserve_amd.kernels.hip import HipKernels, LinearWeights
+from llmserve_amd.kernels.hip import HipKernels, KernelError, LinearWeights
 
 ROOT = Path(__file__).resolve().parents[1]
 LDS_KB = 160
@@ -178,3 +178,53 @@ def test_attention_work_lists_cover_every_column_once_and_fit_the_padded_shape()
         assert steps >= 0
         padded_tokens = sum(counts) + draw.randint(0, 64)
         assert len(work) <= HipKernels._work_capacity((padded_tokens, requests + draw.randint(0, 3)), group, column_tiles, packed)
+
+
+class Launches:
+    """Takes the place of a kernel library: counts the launches of the product into a norm."""
+
+    def __init__(self) -> None:
+        self.count = 0
+
+    def llmserve_gemm_scaled_streams(self, rows, out_features, in_features):
+        return 1
+
+    def llmserve_gemm_into_norm(self, *arguments):
+        self.count += 1
+        return 0
+
+
+def on_the_host(**changes):
+    """`HipKernels` without a GPU: its rules and checks, on CPU tensors, with `Launches` for the kernels."""
+    kernels = object.__new__(HipKernels)
+    settings = dict(dtype=torch.bfloat16, device=torch.device("cpu"), ring_products=True, ring_rows_from=4, library_products=True,
+                    _for_replay=True, _pinned_stream=0, _gemm_bf16=Launches())
+    kernels.__dict__.update(settings | changes)
+    return kernels
+
+
+@pytest.mark.parametrize("rows", [4, 33])
+def test_a_product_into_a_norm_takes_no_form_that_the_steps_apart_refuse(rows):
+    """`linear` refuses an x that is not as wide as the weight, `add_rms_norm` a stream that is not float32: where the two are one
+    product the same forms are left to them, and nothing is launched."""
+    width, inner = 1536, 1280
+    kernels = on_the_host()
+    project = LinearWeights(torch.zeros(width, inner, dtype=torch.bfloat16), None)
+    reader = kernels.prepare_gated_linear(*(torch.zeros(1400, width, dtype=torch.bfloat16) for _ in range(2)))
+
+    def linked(x, hidden, weight=torch.ones(width)):
+        before = kernels._gemm_bf16.count
+        result = kernels._linear_into_norm(x, None, project, kernels.norm_into(hidden, weight, 1e-6, reader))
+        assert kernels._gemm_bf16.count - before == (result is not None)
+        return result
+
+    x, hidden = torch.zeros(rows, inner, dtype=torch.bfloat16), torch.zeros(rows, width)
+    assert linked(x, hidden) is not None
+    assert linked(x[:, :1152].contiguous(), hidden) is None
+    assert linked(torch.zeros(rows, width, dtype=torch.bfloat16), hidden) is None  # as wide as the stream
+    assert linked(x[:-1], hidden) is None
+    assert linked(x.float(), hidden) is None
+    assert linked(x, hidden.bfloat16()) is None
+    assert linked(x, hidden, torch.ones(width + 16)) is None
+    with pytest.raises(KernelError):
+        kernels.gated_linear(linked(x, hidden), kernels.prepare_gated_linear(*(torch.zeros(1400, width, dtype=torch.bfloat16) for _ in range(2))))
