@@ -99,8 +99,8 @@ class Attention(Mixer):
 
     @property
     def takes_into(self) -> bool:
-        """Whether `forward` can be told of the norm behind it (`into`)."""
-        return getattr(self.position, "takes_into", False)
+        """Whether `forward` can be told of the norm behind it (`into`); a mixer with a `forward` of its own says so itself."""
+        return type(self).forward is Attention.forward and getattr(self.position, "takes_into", False)
 
     def forward(self, x: torch.Tensor, batch, cell, **into) -> torch.Tensor:
         qkv = self.kernels.linear(x, self.qkv)

@@ -9,6 +9,7 @@ from typing import Any
 import torch
 
 from .base import BLOCKS, FEED_FORWARDS, MIXERS, NORMS, CacheNeed, Part, TensorSpec, prefixed, side_by_side, under
+from .feed_forward import GatedMLP
 from .norm import RMSNorm
 
 
@@ -72,17 +73,19 @@ class PreNormBlock(Block):
         self.feed_forward_norm, self.feed_forward = built[2:] if len(built) > 2 else (None, None)
         self.replayable = all(part.replayable for part in built)
         # the mixer's last product and the feed-forward's first one may do the norm between them themselves (a kernel library with
-        # `norm_into`): where it takes the step's sizes the mixer returns what the feed-forward's product reads, no delta
+        # `norm_into`): where it takes the step's sizes the mixer returns what the feed-forward's product reads, no delta.
+        # (Parts derived from these that do one of the three steps in a way of their own are asked for it, as ever.)
         self._norm_into = None
         norm, feed_forward = self.feed_forward_norm, self.feed_forward
-        if getattr(self.mixer, "takes_into", False) and getattr(feed_forward, "reader", None) is not None and isinstance(norm, RMSNorm):
+        as_they_stand = getattr(type(norm), "forward", None) is RMSNorm.forward and getattr(type(feed_forward), "forward", None) is GatedMLP.forward
+        if getattr(self.mixer, "takes_into", False) and as_they_stand:
             self._norm_into = getattr(kernels, "norm_into", None)
 
     def forward(self, hidden, delta, batch, cell) -> torch.Tensor:
         normed = self.mixer_norm.forward(hidden, delta)
         if self._norm_into is not None:
             norm = self.feed_forward_norm
-            mixed = self.mixer.forward(normed, batch, cell, into=self._norm_into(hidden, norm.weight, norm.spec.eps, self.feed_forward.reader))
+            mixed = self.mixer.forward(normed, batch, cell, into=self._norm_into(hidden, norm.weight, norm.spec.eps, self.feed_forward.gate_up))
         else:
             mixed = self.mixer.forward(normed, batch, cell)
         if self.feed_forward is None:

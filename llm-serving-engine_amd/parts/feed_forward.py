@@ -53,7 +53,6 @@ class GatedMLP(FeedForward):
         else:
             self.gate_up = kernels.prepare_gated_linear(tensors[gate], tensors[up], spec.activation, limit=spec.limit)
         self.down = kernels.prepare_linear([tensors[down]], None)
-        self.reader = self.gate_up  # the one product that reads the normed rows
 
     def forward(self, x: torch.Tensor, batch) -> torch.Tensor:
         activated = self.kernels.gated_linear(x, self.gate_up)

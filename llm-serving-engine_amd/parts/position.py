@@ -88,7 +88,10 @@ class Rotary(PositionEncoding):
             qkv, layout, batch, cell, self.inverse_frequencies, self.spec.pairing
         )
 
-    takes_into = True
+    @property
+    def takes_into(self) -> bool:
+        """Whether `encode_store_attend` can be told of a norm behind the product (`into`); an encoding with one of its own says so itself."""
+        return type(self).encode_store_attend is Rotary.encode_store_attend
 
     def encode_store_attend(self, qkv, layout: HeadLayout, batch, cell, scale: float, window, project=None, **into):
         return self.kernels.rotate_store_attend(

@@ -4,11 +4,16 @@ for the kernels; tests/test_gpu_parts.py does the same on the GPU)."""
 
 from __future__ import annotations
 
+from dataclasses import replace
+
 import pytest
 import torch
 
 from llmserve_amd import CacheConfig, ModelRunner, StepEntry
-from llmserve_amd.parts import FixedState, PagedKeyValue
+from llmserve_amd.parts import (
+    FEED_FORWARDS, MIXERS, NORMS, POSITIONS, Attention, AttentionSpec, FixedState, GatedMLP, GatedMLPSpec, PagedKeyValue, PreNormBlock,
+    PreNormBlockSpec, RMSNorm, RMSNormSpec, Rotary, RotarySpec,
+)
 from llmserve_amd.weights import load_model_folder
 from tests import toy
 from tests.tiny import random_tokens
@@ -174,3 +179,63 @@ def test_a_gate_activation_without_a_kernel_is_refused_by_name():
     tensors = {name: torch.zeros(shape.shape) for name, shape in FEED_FORWARDS.tensors(spec).items()}
     with pytest.raises(ValueError, match="swish7"):
         FEED_FORWARDS.build(spec, tensors, TorchKernels(torch.float32))
+
+
+class StubAttention(TorchKernels):
+    def rotate_store_attend(self, qkv, layout, batch, cell, inverse_frequencies, pairing, scale, window, project=None):
+        return self.linear(qkv[:, : project.weight.shape[1]], project, out_dtype=torch.float32)
+
+
+class LinkingKernels(StubAttention):
+    """A kernel library that may do the norm between two products: it is told of one, and leaves it to the steps apart."""
+
+    told = 0
+
+    def norm_into(self, hidden, weight, eps, reader):
+        return hidden, weight, eps, reader
+
+    def rotate_store_attend(self, *arguments, into=None, **options):
+        self.told += into is not None
+        return super().rotate_store_attend(*arguments, **options)
+
+
+class SomeMixer(Attention):
+    def forward(self, x, batch, cell):
+        return 2.0 * super().forward(x, batch, cell)
+
+
+class SomePosition(Rotary):
+    def encode_store_attend(self, qkv, layout, batch, cell, scale, window, project=None):
+        return super().encode_store_attend(3.0 * qkv, layout, batch, cell, scale, window, project)
+
+
+class SomeNorm(RMSNorm):
+    def forward(self, hidden, delta):
+        return 1.0 + super().forward(hidden, delta)
+
+
+class SomeFeedForward(GatedMLP):
+    def forward(self, x, batch):
+        return super().forward(-x, batch)
+
+
+@pytest.mark.parametrize("derived", [None, SomeMixer, SomePosition, SomeNorm, SomeFeedForward])
+def test_parts_derived_from_those_that_a_library_links_are_asked_as_ever(derived, monkeypatch):
+    """A part that derives from one of the library's and does its step in a way of its own: the block asks it for that step, whether
+    or not the kernel library could have done it together with its neighbours."""
+    width = 16
+    for registry, cls in ((MIXERS, SomeMixer), (POSITIONS, SomePosition), (NORMS, SomeNorm), (FEED_FORWARDS, SomeFeedForward)):
+        monkeypatch.setitem(registry._classes, cls.__name__, cls)
+
+    def of(spec, cls):
+        return replace(spec, kind=cls.__name__) if derived is cls else spec
+
+    attention = AttentionSpec(width, 2, 1, 8, 0.3, of(RotarySpec(8, 100.0), SomePosition), qkv_bias=False)
+    norm = RMSNormSpec(width, 1e-6)
+    spec = PreNormBlockSpec(norm, of(attention, SomeMixer), of(norm, SomeNorm), of(GatedMLPSpec(width, 24), SomeFeedForward))
+    generator = torch.Generator().manual_seed(2)
+    tensors = {name: torch.randn(tensor.shape, generator=generator) for name, tensor in PreNormBlock.tensors(spec).items()}
+    hidden = torch.randn((3, width), generator=generator)
+    linking = LinkingKernels()
+    apart, linked = (PreNormBlock(spec, tensors, kernels).forward(hidden.clone(), None, None, None) for kernels in (StubAttention(), linking))
+    assert torch.equal(apart, linked) and linking.told == (derived is None)
