@@ -45,6 +45,11 @@ def _pointer(tensor: torch.Tensor | None) -> int | None:
     return tensor.data_ptr()
 
 
+def _in_pieces(*tensors: torch.Tensor) -> bool:
+    """Whether rows can be read in 16-byte pieces: contiguous tensors that begin at one (rows of a whole number of pieces)."""
+    return all(tensor.is_contiguous() and tensor.data_ptr() % 16 == 0 for tensor in tensors)
+
+
 # Argument types of every entry point: p pointer, i int, f float.  Declared once, so that a call
 # costs no guessing: a decode step is replayed from a graph, but every other step pays per launch.
 _SIGNATURES = {
@@ -446,7 +451,7 @@ class HipKernels:
             # workgroups: the 32B sizes' gate/up 100-110 us at the library, 98-106 here, 113-177 in several rounds; the 1.5B
             # sizes' head, 9,496 tiles, 108-120 against 101-165)
             return "ring"
-        if rows > 64 and HipKernels._tiled_ahead(rows, weights.out_features, inner, gated, may_split):
+        if rows > 64 and HipKernels._tiled_ahead(rows, weights.out_features, inner, gated, may_split) and _in_pieces(x, weights.weight):
             return "tiled"
         if self.ring_products and 64 < rows <= 128 and inner % 128 == 0 and (
             (may_split and (1 << 20) < size <= 150_000_000) or (gated and (1 << 22) < size <= 150_000_000)

@@ -228,3 +228,27 @@ def test_a_product_into_a_norm_takes_no_form_that_the_steps_apart_refuse(rows):
     assert linked(x, hidden, torch.ones(width + 16)) is None
     with pytest.raises(KernelError):
         kernels.gated_linear(linked(x, hidden), kernels.prepare_gated_linear(*(torch.zeros(1400, width, dtype=torch.bfloat16) for _ in range(2))))
+
+
+@pytest.mark.parametrize("rows,out_features,in_features,gated,may_split", [(96, 1536, 8960, False, True), (384, 1536, 8960, False, True),
+                                                                            (600, 2048, 1536, False, False), (300, 9728, 896, True, False)])
+def test_rows_that_are_views_go_to_the_library(rows, out_features, in_features, gated, may_split):
+    """The library takes rows of any stride and at any address; the tiled kernel brings 16-byte pieces of whole rows, so such rows stay
+    with the library (up to 128 rows with the kernel before it in line, which has always refused strides)."""
+    kernels = stand_in()
+    flat = torch.empty(rows * in_features + 8, dtype=torch.bfloat16)
+    weight = torch.empty(out_features * in_features + 8, dtype=torch.bfloat16)
+    forms = {
+        "rows": flat[:-8].view(rows, in_features),
+        "every second row": torch.empty((2 * rows, in_features), dtype=torch.bfloat16)[::2],
+        "columns of wider rows": torch.empty((rows, in_features + 64), dtype=torch.bfloat16)[:, 64:],
+        "rows that begin inside a piece": flat[1:-7].view(rows, in_features),
+    }
+
+    def way(x, w):
+        return HipKernels._streaming(kernels, x, LinearWeights(w.view(out_features, in_features), None), gated=gated, may_split=may_split)
+
+    assert way(forms["rows"], weight[:-8]) == "tiled"
+    other = "ring" if rows <= 128 else None
+    assert all(way(x, weight[:-8]) == other for name, x in forms.items() if name != "rows")
+    assert way(forms["rows"], weight[1:-7]) == other
