@@ -484,27 +484,44 @@ class HipKernels:
 
     @staticmethod
     def _tiled_ahead(rows: int, out_features: int, in_features: int, gated: bool, may_split: bool) -> bool:
-        """Whether a product of more than 64 rows is faster on the LDS-tiled kernel than at the library.  A captured chain
-        over different weights, us, the library (its best of one piece and two to eight slices of K; a gated product with the kernel
-        for silu(gate) * up behind it) against the tiled kernel.  Where the result may stay partial sums, a result of few tiles:
-        N 1,536 K 8,960: 96 rows 17.7 and 11.5 (the kernel through a ring 13.4), 384 rows 25.3 and 20.1, 1,024 rows 37.8 and 35.8,
-        1,536 rows 53.7 and 50.4, 2,048 rows 55.1 and 60.2; N 3,584 K 18,944: 128 rows 50.5 and 34.0 (the ring 45), 512 rows 84.5 and 79.6, 768
-        rows 109 and 124; N = K = 1,536: 192 rows 8.1 and 6.4, 1,024 rows 13.3 and 12.4; N = K = 3,584: 512 rows 22.6 and 20.3, 768 rows 26.4
-        and 28.5.  Gated: N 17,920 K 1,536: 256 rows 35 and 29, 384 rows 37 and 30, 512 rows 45 and 44, 1,024 rows 80 and 74, 2,048
-        rows 133 and 111; N 37,888 K 3,584: 192 rows 84 and 96, 512 rows 149 and 164, 1,024 rows 315 and 274, 2,048 rows 546 and 474;
-        up to 128 rows the ring's 22.5 and 61 are as good or better.  Plain ones and results of more tiles: small weights over more than
-        512 rows, up to a result of four million (N 2,048 K 1,536: 384 rows 9.4 and 10.1, 768 rows 12.8 and 11.7, 1,024 rows 13.8 and
-        12.1, 2,048 rows 17.2 and 17.0; whole prompts of the 1.5B sizes with their qkv and output projections here: 520 tokens
-        3.99 -> 3.92 ms, 1,024 5.60 -> 5.51, 1,500 7.19 -> 7.13, 2,048 8.01 -> 7.94).  The rest (384 rows of N 4,608 K 3,584 25.2
-        and 27.7) stays with the library."""
+        """Whether a product of more than 64 rows is faster on the LDS-tiled kernel than where it goes otherwise (up to 128 rows partly
+        the ring, else the library; a gated product there has the kernel for silu(gate) * up behind it).  Both sides measured in turn on the
+        same buffers, a captured chain over different weights with what adds up the parts, at 62 weights (K of 768 to 27,648) and
+        up to 29 numbers of rows each; below, the kernel's time over the other's.  The library's times jump by a third between
+        neighbouring sizes, so single points lie on the wrong side of every line: the lines follow the means.
+
+        Gated, up to weights of 40 million: ahead while one round of 256 x 128 tiles holds the result (K 896 0.59-0.76, N 17,920 K 1,536
+        0.79-0.90, K 2,048 0.70-0.97), behind where it takes a second one that is half empty (N 17,920 at 416-576 rows 1.00-1.14, N 16,384 K
+        2,048 at 520-600 1.28, N 11,264-16,384 K 2,048 at 700-900 1.05-1.30), ahead again for K up to 1,536 from about 160 tiles of 256 x 256
+        on (N 17,920 at 640-896 0.79-0.98).  From 1,024 rows on the activation's own pass decides, which is a share of
+        the library's time that falls with K: K up to 1,536 0.57-1.08, mean 0.87; beyond, only where the tiles make many rounds (N 37,888 K
+        3,584 0.85-0.99, N 55,296 K 5,120 0.89-0.98, N 34,816 K 5,120 0.95 and N 44,032 K 4,096 0.99 in the mean; but N 18,432 K 2,304 1.03,
+        N 19,456 K 2,560 0.83-1.18, N 24,576 and 28,672 K 4,096 1.16 and 1.03, N 59,136 K 8,192 1.06-1.13).
+
+        In parts: up to 128 rows 0.57-1.01 at every size.  More rows: weights of up to 100 million (N 5,120 K 13,824 0.54-0.92 and N 3,584 K
+        22,528 0.67-0.98; N 5,120 K 27,648 at 160-256 rows 1.07-1.14), results of up to two million (K 8,960 to 14,336: 0.45-1.04; beyond,
+        N 4,096 K 14,336 at 576 rows 1.33, N 1,536 K 10,496 at 1,536 1.07, N 2,560 K 9,728 at 896 1.07), and where K is no
+        long one up to 512 rows (N = K = 3,584 0.69-0.99, at 513-576 rows 1.14; N = K = 4,096 1.06 there).
+
+        Plain, and in parts with any number of rows: small weights over more than 512 rows, up to a result of four million.  On the device
+        the two are alike (N 2,048 K 1,536 0.90-1.18, N = K = 1,536 0.96-1.05), but so long a step is launched kernel by kernel, and
+        a launch of ours costs the host less than a call of the library: whole prompts of the 1.5B sizes, gate/up at the library in both, these
+        at the library and here, 513 tokens 4.43 and 3.80 ms, 640 4.15 and 4.07, 1,024 5.90 and 5.70, 2,048 9.20 and 9.08."""
         if in_features % 64:
             return False
+        size, results = out_features * in_features, rows * out_features
         if gated:
-            return rows > 128 and (out_features * in_features <= 40_000_000 or rows >= 1024)
-        if rows > 512 and out_features >= 1024 and out_features * in_features <= (1 << 22) and rows * out_features <= (1 << 22):
+            if rows <= 128:
+                return False
+            if rows < 1024:
+                one_round = -(-out_features // 256) * -(-rows // 128) <= 256
+                return size <= 40_000_000 and (one_round or (in_features <= 1536 and results >= 160 * 256 * 256))
+            return in_features <= 1536 or (out_features >= 32768 and in_features <= 5120)
+        if rows > 512 and out_features >= 1024 and size <= (1 << 22) and results <= (1 << 22):
             return True
-        # (a K of 256s divides into two and four parts of whole stages; else the library's slices may be the only way to cut it)
-        return may_split and in_features % 256 == 0 and (rows <= 128 or rows * out_features <= 2_400_000)
+        if not may_split or in_features % 256:  # (a K of 256s divides into two and four parts of whole stages; else the library's slices may be the only way to cut it)
+            return False
+        return rows <= 128 or (size <= 100_000_000 and results <= (1 << 21) and (rows <= 512 or in_features >= 2 * out_features))
 
     def _library(self, x: torch.Tensor, weights: LinearWeights) -> bool:
         """Whether the product goes to the BLAS library (hipBLASLt through torch), as the

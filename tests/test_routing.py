@@ -252,3 +252,21 @@ def test_rows_that_are_views_go_to_the_library(rows, out_features, in_features, 
     other = "ring" if rows <= 128 else None
     assert all(way(x, weight[:-8]) == other for name, x in forms.items() if name != "rows")
     assert way(forms["rows"], weight[1:-7]) == other
+
+
+@pytest.mark.parametrize("rows,out_features,in_features,gated,may_split,tiled", [
+    # gated: a round of tiles, a second one half empty, long K
+    (384, 17920, 1536, True, False, True), (416, 17920, 1536, True, False, False), (576, 17920, 1536, True, False, False),
+    (704, 17920, 1536, True, False, True), (600, 11264, 2048, True, False, True), (900, 12288, 2048, True, False, False),
+    (520, 16384, 2048, True, False, False), (2048, 17920, 1536, True, False, True), (1536, 19456, 2560, True, False, False),
+    (2048, 37888, 3584, True, False, True), (1024, 24576, 4096, True, False, False), (2048, 59136, 8192, True, False, False),
+    # in parts: few rows, very large weights, large results, a K as long as the result is wide
+    (128, 5120, 27648, False, True, True), (160, 5120, 27648, False, True, False), (320, 5120, 13824, False, True, True),
+    (512, 4096, 14336, False, True, True), (576, 4096, 14336, False, True, False), (1280, 1536, 8960, False, True, True),
+    (1536, 1536, 10496, False, True, False), (512, 3584, 3584, False, True, True), (576, 3584, 3584, False, True, False),
+    # plain, small weights
+    (512, 2048, 1536, False, False, False), (513, 2048, 1536, False, False, True), (2048, 2048, 1536, False, False, True),
+])
+def test_products_of_many_rows_go_where_they_were_measured_ahead(rows, out_features, in_features, gated, may_split, tiled):
+    """Both sides of the lines that `_tiled_ahead` draws, at sizes that were measured there."""
+    assert (route(stand_in(), rows, out_features, in_features, gated, may_split) == "tiled") == tiled
