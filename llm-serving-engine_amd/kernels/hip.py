@@ -1146,6 +1146,20 @@ class HipKernels:
         reach = window + keep_first if window else chunk
         return min(batch.max_context_length, reach) if reach else batch.max_context_length
 
+    @staticmethod
+    def _portion_runs(keys: int, blocks: int) -> int:
+        """Into how many runs the walks of a step with portions are cut, which a second kernel merges, when `blocks` workgroups
+        walk up to `keys` keys (in a captured step what its tables have room for, mostly a quarter more than the longest context): runs of
+        at least 32 steps of 32 keys, up to about 512 workgroups in all.  Us a layer, whole (four waves) against runs with their
+        merging: 8 tokens over 4,000 keys beside a portion of 64 at the 1.5B sizes 72.7 and 22.4 (whole with eight waves 58.7), 24 over
+        2,500 beside 200 48.3 and 29.1; 6 over 2,500 beside 100 at the 7B sizes 47.0 and 31.4.  Two runs that leave the range of eight waves
+        a walk (256 workgroups) gain less than the merging costs, but for the longest walks.  Whole steps, cut over whole, 1.5B sizes, tables of 2,048
+        keys: 1 to 16 requests over 800 to 1,700 beside 16 to 120 tokens 0.93-0.98, beside 200 in two runs on 200 workgroups 0.97-0.99, on 296 0.99-1.01,
+        beside 300 and 400 on 272 to 464 1.00-1.04, 31 requests 0.99-1.03; of 4,096 in three runs or more 0.78-0.98, in two on 290 to 460
+        0.98-1.02; of 8,192 in two on 368 0.95; 7B sizes, tables of 2,048 in two on 250 0.98-1.00, on 290 to 460 1.01-1.02."""
+        runs = max(1, min(-(-keys // 32) // 32, 512 // blocks, 8))
+        return runs if blocks * runs <= 256 or runs >= 3 or keys >= 8192 else 1
+
     def _attention_float32(self, qkv, out, layout, batch, cell, group, scale: float, window: int, score_slopes=None, soft_cap=None, sinks=None,
                            keep_first: int = 0, chunk: int = 0, maps: int = 1, bias=None, reach: int = 0) -> None:
         """The 32-bit path's attention on the matrix cores: an item is 16 (decoding) or 32 columns of one
@@ -1326,12 +1340,7 @@ class HipKernels:
                     partial_ml = self._empty((held * heads * maps * splits * 2,), torch.float32)
             elif column_tiles == 2 and changed is None and finish is None:
                 # A portion beside decoded tokens whose contexts are long: few items, and the longest walked by one workgroup.
-                # Cut into runs of at least 32 steps of 32 keys, up to about 512 workgroups in all, and merged.  Us a layer,
-                # whole (four waves) against runs with their merging: 8 tokens over 4,000 keys beside a portion of 64 at the 1.5B
-                # sizes 72.7 and 22.4 (whole with eight waves 58.7), 24 over 2,500 beside 200 48.3 and 29.1; 6 over 2,500
-                # beside 100 at the 7B sizes 47.0 and 31.4.
-                blocks = items * kv_heads * head_tiles
-                splits = max(1, min(-(-self._walked_keys(batch, window, keep_first, chunk) // 32) // 32, 512 // blocks, 8))
+                splits = self._portion_runs(self._walked_keys(batch, window, keep_first, chunk), items * kv_heads * head_tiles)
                 if splits > 1:
                     partial_acc = self._empty((tokens * heads * splits * layout.head_dim,), torch.float32)
                     partial_ml = self._empty((tokens * heads * splits * 2,), torch.float32)

@@ -270,3 +270,12 @@ def test_rows_that_are_views_go_to_the_library(rows, out_features, in_features, 
 def test_products_of_many_rows_go_where_they_were_measured_ahead(rows, out_features, in_features, gated, may_split, tiled):
     """Both sides of the lines that `_tiled_ahead` draws, at sizes that were measured there."""
     assert (route(stand_in(), rows, out_features, in_features, gated, may_split) == "tiled") == tiled
+
+
+@pytest.mark.parametrize("keys,blocks,runs", [
+    (1024, 20, 1), (2048, 28, 2), (2048, 100, 2), (2048, 128, 2), (2048, 148, 1), (2048, 184, 1), (2048, 232, 1), (2048, 296, 1),
+    (4096, 28, 4), (4096, 148, 3), (4096, 184, 1), (8192, 184, 2), (8192, 28, 8), (8192, 300, 1), (65536, 10, 8),
+])
+def test_walks_of_portions_are_cut_where_it_was_measured_to_pay(keys, blocks, runs):
+    """Two runs for more workgroups than eight waves walk for cost a short context more than they save."""
+    assert HipKernels._portion_runs(keys, blocks) == runs
