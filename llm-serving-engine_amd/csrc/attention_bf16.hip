@@ -1274,12 +1274,6 @@ extern "C" int llmserve_attention_portions(const void*, int, void*, int, float*,
 #ifndef FUSED_WAVES
 #define FUSED_WAVES (HEAD_DIM > 128 ? 4 : 8)
 #endif
-// Two column tiles a wave: eight waves walk a tile's keys where the launch has about a workgroup a CU and walks of some
-// length (us, four waves -> eight; 1.5B sizes: 31 decoded tokens over 500 keys beside a portion of 256, 248 workgroups, 15.9 -> 14.2; 30 over
-// 300 beside 400 16.9 -> 14.5; a portion of 512 of a 2,000-token prompt, 196 workgroups, 18.4 -> 15.2; a 500-token prompt 11.0 -> 10.3; 7B
-// sizes, 260 workgroups, 18.4 -> 15.1; but 376 workgroups, a 1,000-token prompt, 16.8 -> 19.5).
-#define FEW_TILES 288
-#define LONG_WALK 512  // keys
 #define EIGHT_WAVES (HEAD_DIM > 128 ? 4 : 8)  // (of the kinds that write finished results, in a step of single tokens)
 template <int COLUMN_TILES, bool FUSED, int WAVES, int CHANGED = CHANGED_NOT>
 static int launch_tiles(const void* qkv, int row_width, void* out, int out_stride, float* partial_acc, float* partial_ml,
@@ -1341,7 +1335,8 @@ extern "C" int llmserve_attention_can_fuse(int pairing) {
 // `maps` 2: differential attention, column_tiles 2 with work items made for one column tile, or, in a step of single tokens with up
 // to eight query heads a kv head, column_tiles 1 with work items of both maps of a token; partial results twice as many
 // ([rows * heads * 2 * splits ..]); `fuse` 8 says that they are for a step of single tokens, whose keys eight waves a workgroup
-// walk; each of the three writes heads of `vdim` side by side, and goes with no other change.
+// walk; each of the three writes heads of `vdim` side by side, and goes with no other change.  `fuse` 16: eight waves a workgroup
+// walk a tile's keys, where two column tiles and no change of the scores leave the choice.
 // A row of `out` begins every `out_stride` elements (a multiple of 4 from heads * D, or heads * vdim, on).
 extern "C" int llmserve_attention_tiles(const void* qkv, int row_width, void* out, int out_stride, float* partial_acc,
                                         float* partial_ml, void* keys, void* values,
@@ -1353,6 +1348,8 @@ extern "C" int llmserve_attention_tiles(const void* qkv, int row_width, void* ou
                                         int maps, int vdim, float factor, float eps, float out_scale, const void* gates,
                                         int gate_stride, int gate_first, hipStream_t stream) {
   if (tiles <= 0) return 0;
+  const bool wide = (fuse & 16) != 0;  // eight waves a workgroup, with two column tiles and no change of the scores
+  fuse &= ~16;
   if (keep_first < 0 || chunk < 0 || (chunk > 0 && window > 0)) return ERR_BAD_ARGUMENT;
   const bool finished = vdim > 0;
   if (out_stride < heads * (finished ? vdim : D) || (out_stride % 4 && (!finished || vdim % 4 == 0))) return ERR_BAD_ARGUMENT;
@@ -1412,10 +1409,9 @@ extern "C" int llmserve_attention_tiles(const void* qkv, int row_width, void* ou
              : edges ? LAUNCH_TILES(1, false, 4, CHANGED_EDGES)
                      : LAUNCH_TILES(1, false, 4, CHANGED_NOT);
   } else if (column_tiles == 2) {
-    const bool few = (long)tiles * kv_heads * ((heads / kv_heads + 15) / 16) * splits <= FEW_TILES && (long)table_width * page_size >= LONG_WALK;
     status = scores  ? LAUNCH_TILES(2, false, 4, CHANGED_SCORES)
              : edges ? LAUNCH_TILES(2, false, 4, CHANGED_EDGES)
-             : few   ? LAUNCH_TILES(2, false, EIGHT_WAVES, CHANGED_NOT)
+             : wide  ? LAUNCH_TILES(2, false, EIGHT_WAVES, CHANGED_NOT)
                      : LAUNCH_TILES(2, false, 4, CHANGED_NOT);
   } else {
     return ERR_BAD_ARGUMENT;

@@ -1160,6 +1160,17 @@ class HipKernels:
         runs = max(1, min(-(-keys // 32) // 32, 512 // blocks, 8))
         return runs if blocks * runs <= 256 or runs >= 3 or keys >= 8192 else 1
 
+    @staticmethod
+    def _portion_eight_waves(blocks: int, keys: int, padded: bool) -> bool:
+        """Whether eight waves, not four, walk the keys of a tile in a step with portions: where the launch has at most a workgroup a CU
+        and tables of some length (one more, and a second workgroup of as many waves waits for a CU).  Us, four waves -> eight: 1.5B sizes,
+        a portion of 640 tokens, 240 workgroups, 11.1 -> 10.0, behind 600 keys 16.6 -> 14.1; of 680, 256 workgroups, 12.0 -> 11.0 and 16.6 ->
+        14.2; of 720, 270, 12.3 -> 13.3 and 18.2 -> 19.6; 31 decoded tokens over 500 to 800 keys beside 500, 250, 12.2 -> 10.8, beside 600, 288, 13.1
+        -> 14.2; 7B sizes, 280 behind 300, 248, 11.2 -> 10.2, 300 behind 300, 264, 11.9 -> 16.8; 32B sizes, 70 behind 900, 88, 14.3 ->
+        13.0.  A captured step's launch has room for the most items of its padded shape, and the empty ones end at once: of 288 at
+        most 256 do work as a rule (7B sizes, 12 requests beside 240 tokens, 260 of 288, a step 6.88 -> 6.80 ms)."""
+        return blocks <= (288 if padded else 256) and keys >= 512
+
     def _attention_float32(self, qkv, out, layout, batch, cell, group, scale: float, window: int, score_slopes=None, soft_cap=None, sinks=None,
                            keep_first: int = 0, chunk: int = 0, maps: int = 1, bias=None, reach: int = 0) -> None:
         """The 32-bit path's attention on the matrix cores: an item is 16 (decoding) or 32 columns of one
@@ -1280,7 +1291,7 @@ class HipKernels:
             if items == 0:
                 continue
             splits, partial_acc, partial_ml = 1, None, None
-            by_item = False
+            by_item = eight_waves = False
             if shared:
                 # The few short requests (decoded tokens) of a step whose portions went to the other kernel: alone
                 # in this launch, so a long context is walked by one workgroup a kv head (30,000 keys: 237 us) unless
@@ -1340,7 +1351,9 @@ class HipKernels:
                     partial_ml = self._empty((held * heads * maps * splits * 2,), torch.float32)
             elif column_tiles == 2 and changed is None and finish is None:
                 # A portion beside decoded tokens whose contexts are long: few items, and the longest walked by one workgroup.
-                splits = self._portion_runs(self._walked_keys(batch, window, keep_first, chunk), items * kv_heads * head_tiles)
+                blocks = items * kv_heads * head_tiles
+                splits = self._portion_runs(self._walked_keys(batch, window, keep_first, chunk), blocks)
+                eight_waves = self._portion_eight_waves(blocks * splits, group.width * group.page_size, padded)
                 if splits > 1:
                     partial_acc = self._empty((tokens * heads * splits * layout.head_dim,), torch.float32)
                     partial_ml = self._empty((tokens * heads * splits * 2,), torch.float32)
@@ -1348,7 +1361,7 @@ class HipKernels:
             status = library.llmserve_attention_tiles(
                 _pointer(qkv), layout.stride, _pointer(out), out.shape[1], _pointer(partial_acc), _pointer(partial_ml),
                 _pointer(cell.keys), _pointer(cell.values), _pointer(group.block_tables), group.width, _pointer(batch.positions), _pointer(work), items,
-                column_tiles if maps == 1 or paired else 2, tokens, heads, kv_heads, group.page_size, scale, window, splits, (1 if fuse is not None else 0) + (2 if unmerged else 0) + (4 if by_item else 0) + (8 if finish is not None and batch.max_query_length == 1 else 0),
+                column_tiles if maps == 1 or paired else 2, tokens, heads, kv_heads, group.page_size, scale, window, splits, (1 if fuse is not None else 0) + (2 if unmerged else 0) + (4 if by_item else 0) + (8 if finish is not None and batch.max_query_length == 1 else 0) + (16 if eight_waves else 0),
                 _pointer(table), _PAIRINGS[pairing], _pointer(group.slot_mapping), _pointer(slopes), soft_cap, _pointer(sinks), keep_first, chunk,
                 _pointer(bias), reach, maps, vdim, float(factor), float(eps), float(out_scale), _pointer(gates),
                 gates.shape[1] if gates is not None else 0, gate_first, self._stream,

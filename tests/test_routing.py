@@ -279,3 +279,11 @@ def test_products_of_many_rows_go_where_they_were_measured_ahead(rows, out_featu
 def test_walks_of_portions_are_cut_where_it_was_measured_to_pay(keys, blocks, runs):
     """Two runs for more workgroups than eight waves walk for cost a short context more than they save."""
     assert HipKernels._portion_runs(keys, blocks) == runs
+
+
+@pytest.mark.parametrize("blocks,keys,padded,eight", [
+    (88, 1024, False, True), (256, 704, False, True), (264, 608, False, False), (288, 2000, False, False), (100, 256, False, False),
+    (288, 1024, True, True), (296, 1024, True, False),
+])
+def test_eight_waves_walk_where_a_workgroup_has_a_cu(blocks, keys, padded, eight):
+    assert HipKernels._portion_eight_waves(blocks, keys, padded) == eight
