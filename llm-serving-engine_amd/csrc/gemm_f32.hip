@@ -5,13 +5,14 @@
 // model.py:60-66 via nn.Linear); gemm_generic.hip remains for operands of mixed types and for a K
 // that is no multiple of 4.
 //
-// gemm_f32_stream (M <= 32, decoding): the product is a stream of the weight matrix from HBM.  A
-// workgroup owns 16 weight rows and its waves split K between them; lane (r, g) keeps groups of four
+// gemm_f32_stream (M <= 64, decoding): the product is a stream of the weight matrix from HBM.  A
+// workgroup owns 16 weight rows (from 33 rows of x on 32) and its waves split K between them; lane (r, g) keeps groups of four
 // 16-byte loads of weight row r in flight, k = 16 s + 4 g .. + 3 of every 16-wide step s.  An MFMA
 // takes a 16 x 4 piece of the weights as its A operand (lane (r, g) gives A[r][g]) and 4 x 16 of x^T as
 // B; which four k an instruction covers is free as long as A and B agree, so instruction j of a step
 // takes element j of each lane's load: k = 16 s + 4 g + j.  The waves' partial tiles are added through
-// LDS in wave order, so a row's bits depend on the shape of the weight only, never on the batch.
+// LDS in wave order, so a row's bits depend on the shape of the weight only, never on the batch (the tiled kernel's, for
+// larger ones, on the number of rows too).
 //
 // gemm_f32_tiled (more rows, prompt portions): a tile of weight rows by rows of x a workgroup of four waves, each
 // one to four tiles of v_mfma_f32_32x32x2_f32; K in steps of 16 (of 32 or 64 where two or four waves share a tile
@@ -39,21 +40,22 @@ __device__ __forceinline__ f32x4 load4(const float* p) { return *(const f32x4*)p
 
 __device__ __forceinline__ float silu(float gate) { return gate / (1.f + expf(-gate)); }
 
-// MT: 16-row tiles of x (up to 16 MT rows): every weight operand meets MT operands of x, which each wave
-// reads for itself (M / 16 of what it reads of the weights, from L2).
-template <int WAVES, int MT, bool GATED>
+// NT: 16-row tiles of weights a workgroup, MT: 16-row tiles of x (up to 16 MT rows).  Every weight operand meets MT operands of
+// x, which each wave reads for itself (M / (16 NT) of what it reads of the weights, from L2).
+template <int WAVES, int NT, int MT, bool GATED>
 __global__ __launch_bounds__(WAVES * 64) void gemm_f32_stream_kernel(const float* __restrict__ x,
                                                                      const float* __restrict__ w,
                                                                      const float* __restrict__ bias,
                                                                      float* __restrict__ out, int M, int N, int K,
                                                                      int k_split) {
-  extern __shared__ float partial[];  // [WAVES][MT][64 lanes][4]
+  extern __shared__ float partial[];  // [WAVES][NT MT tiles][64 lanes][4]
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
-  const int n = min((int)blockIdx.x * 16 + r, N - 1);
   const int k_first = blockIdx.y * k_split;
   const int k_count = min(k_split, K - k_first);  // the last slice may be shorter
-  const float* w_row = w + (size_t)n * K + k_first + g * 4;
+  const float* w_row[NT];
+#pragma unroll
+  for (int s = 0; s < NT; ++s) w_row[s] = w + (size_t)min(((int)blockIdx.x * NT + s) * 16 + r, N - 1) * K + k_first + g * 4;
   bool x_live[MT];
   const float* x_row[MT];
 #pragma unroll
@@ -62,16 +64,20 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_stream_kernel(const float
     x_row[t] = x + (size_t)min(t * 16 + r, M - 1) * K + k_first + g * 4;
   }
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4 acc[MT];
+  f32x4 acc[NT][MT];
 #pragma unroll
-  for (int t = 0; t < MT; ++t) acc[t] = zero;
+  for (int s = 0; s < NT; ++s)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[s][t] = zero;
 
   const int groups = k_count / (16 * STREAM_GROUP);
-  f32x4 a[STREAM_GROUP], a_next[STREAM_GROUP];
+  f32x4 a[NT][STREAM_GROUP], a_next[NT][STREAM_GROUP];
   int group = wave;
   if (group < groups) {
 #pragma unroll
-    for (int u = 0; u < STREAM_GROUP; ++u) a[u] = load4(w_row + (group * STREAM_GROUP + u) * 16);
+    for (int s = 0; s < NT; ++s)
+#pragma unroll
+      for (int u = 0; u < STREAM_GROUP; ++u) a[s][u] = load4(w_row[s] + (group * STREAM_GROUP + u) * 16);
   }
   while (group < groups) {
     const int next = group + WAVES;
@@ -85,63 +91,79 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_stream_kernel(const float
     asm volatile("" ::: "memory");
     if (next < groups) {
 #pragma unroll
-      for (int u = 0; u < STREAM_GROUP; ++u) a_next[u] = load4(w_row + (next * STREAM_GROUP + u) * 16);
+      for (int s = 0; s < NT; ++s)
+#pragma unroll
+        for (int u = 0; u < STREAM_GROUP; ++u) a_next[s][u] = load4(w_row[s] + (next * STREAM_GROUP + u) * 16);
     }
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
       for (int u = 0; u < STREAM_GROUP; ++u)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][j], b[t][u][j], acc[t], 0, 0, 0);
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int u = 0; u < STREAM_GROUP; ++u) a[u] = a_next[u];
+          for (int s = 0; s < NT; ++s)
+            acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][u][j], b[t][u][j], acc[s][t], 0, 0, 0);
+#pragma unroll
+    for (int s = 0; s < NT; ++s)
+#pragma unroll
+      for (int u = 0; u < STREAM_GROUP; ++u) a[s][u] = a_next[s][u];
     group = next;
   }
   // the steps left over when the slice is no multiple of 64; the last may be cut (K is a multiple of 4)
   for (int step = groups * STREAM_GROUP + wave; step * 16 < k_count; step += WAVES) {
     const bool inside = step * 16 + g * 4 < k_count;
-    const f32x4 a_tail = inside ? load4(w_row + step * 16) : zero;
+    f32x4 a_tail[NT];
+#pragma unroll
+    for (int s = 0; s < NT; ++s) a_tail[s] = inside ? load4(w_row[s] + step * 16) : zero;
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       const f32x4 b_tail = inside && x_live[t] ? load4(x_row[t] + step * 16) : zero;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a_tail[j], b_tail[j], acc[t], 0, 0, 0);
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int s = 0; s < NT; ++s)
+          acc[s][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a_tail[s][j], b_tail[j], acc[s][t], 0, 0, 0);
     }
   }
 
+  constexpr int TILES = NT * MT;
 #pragma unroll
-  for (int t = 0; t < MT; ++t) *(f32x4*)(partial + ((wave * MT + t) * 64 + lane) * 4) = acc[t];
+  for (int s = 0; s < NT; ++s)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) *(f32x4*)(partial + ((wave * TILES + s * MT + t) * 64 + lane) * 4) = acc[s][t];
   __syncthreads();
-  if (wave >= MT) return;
-  // wave t finishes tile t of x.  D[n][m]: the lane holds token m = 16 t + r and rows n0 + 4 g .. + 3
-  const int t = wave;
-  f32x4 total = zero;
-  for (int v = 0; v < WAVES; ++v) total += *(const f32x4*)(partial + ((v * MT + t) * 64 + lane) * 4);
-  const int m = t * 16 + r;
-  const int n_first = blockIdx.x * 16 + g * 4;
-  if (m >= M) return;
-  if (bias && blockIdx.y == 0) {
+  // a wave finishes tiles wave, wave + WAVES, ...  D[n][m]: the lane holds token m = 16 t + r and rows n0 + 4 g .. + 3
+  for (int tile = wave; tile < TILES; tile += WAVES) {
+    f32x4 total = zero;
+    for (int v = 0; v < WAVES; ++v) total += *(const f32x4*)(partial + ((v * TILES + tile) * 64 + lane) * 4);
+    const int m = tile % MT * 16 + r;
+    const int n_first = ((int)blockIdx.x * NT + tile / MT) * 16 + g * 4;
+    if (m >= M) continue;
+    if (bias && blockIdx.y == 0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) total[i] += bias[min(n_first + i, N - 1)];
-  }
-  if (GATED) {
-    float* dst = out + (size_t)m * (N / 2) + n_first / 2;
+      for (int i = 0; i < 4; ++i) total[i] += bias[min(n_first + i, N - 1)];
+    }
+    if (GATED) {
+      float* dst = out + (size_t)m * (N / 2) + n_first / 2;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-      if (n_first + 2 * i + 1 < N) dst[i] = silu(total[2 * i]) * total[2 * i + 1];
-  } else {
-    float* dst = out + ((size_t)blockIdx.y * M + m) * N + n_first;
+      for (int i = 0; i < 2; ++i)
+        if (n_first + 2 * i + 1 < N) dst[i] = silu(total[2 * i]) * total[2 * i + 1];
+    } else {
+      float* dst = out + ((size_t)blockIdx.y * M + m) * N + n_first;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (n_first + i < N) dst[i] = total[i];
+      for (int i = 0; i < 4; ++i)
+        if (n_first + i < N) dst[i] = total[i];
+    }
   }
 }
 
-template <int WAVES, int MT, bool GATED>
+template <int WAVES, int NT, int MT, bool GATED>
 static int launch_stream(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, int splits,
                          int k_split, hipStream_t stream) {
-  const size_t lds = (size_t)WAVES * MT * 64 * 4 * sizeof(float);
-  hipLaunchKernelGGL((gemm_f32_stream_kernel<WAVES, MT, GATED>), dim3((N + 15) / 16, splits), dim3(WAVES * 64), lds,
+  constexpr size_t lds = (size_t)WAVES * NT * MT * 64 * 4 * sizeof(float);
+  static_assert(lds <= 64 * 1024, "what a launch has without asking");
+  hipLaunchKernelGGL((gemm_f32_stream_kernel<WAVES, NT, MT, GATED>), dim3((N + 16 * NT - 1) / (16 * NT), splits), dim3(WAVES * 64), lds,
                      stream, x, w, bias, out, M, N, K, k_split);
   return LAUNCH_STATUS();
 }
@@ -149,8 +171,13 @@ static int launch_stream(const float* x, const float* w, const float* bias, floa
 template <int WAVES, bool GATED>
 static int pick_tiles(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, int splits,
                       int k_split, hipStream_t stream) {
-  if (M <= 16) return launch_stream<WAVES, 1, GATED>(x, w, bias, out, M, N, K, splits, k_split, stream);
-  return launch_stream<WAVES, 2, GATED>(x, w, bias, out, M, N, K, splits, k_split, stream);
+  if (M <= 16) return launch_stream<WAVES, 1, 1, GATED>(x, w, bias, out, M, N, K, splits, k_split, stream);
+  if (M <= 32) return launch_stream<WAVES, 1, 2, GATED>(x, w, bias, out, M, N, K, splits, k_split, stream);
+  // From 33 rows on x costs the caches more than the weights cost memory, so two tiles of weights share it (a wave's walk and the order
+  // of its sums stay as they are; sixteen waves, of a small weight, leave no room for that).
+  constexpr int NT = WAVES <= 8 ? 2 : 1;
+  if (M <= 48) return launch_stream<WAVES, NT, 3, GATED>(x, w, bias, out, M, N, K, splits, k_split, stream);
+  return launch_stream<WAVES, NT, 4, GATED>(x, w, bias, out, M, N, K, splits, k_split, stream);
 }
 
 template <bool GATED>
@@ -399,14 +426,15 @@ static int launch_tiled(const float* x, const float* w, const float* bias, float
 
 // out [M, N] (or [splits, M, N] partial sums) = x [M, K] . w [N, K]^T (+ bias [N]); all float32, K a multiple
 // of 4.  gated: w's rows alternate gate and up (N even), out is [M, N / 2] = silu(gate) * up, no splits.
-// Up to 32 rows of x go to the weight-streaming kernel, more to the tiled one (64 rows, us, streaming against tiled: N
-// 17,920 K 1,536 gated 74 and 53, N 1,536 K 8,960 in parts 38 and 26, N 2,048 K 1,536 22 and 17; 32 rows: 47 and 36, 24 and 20,
-// but 13 and 17 for the small weight, and 17 rows 38 and 35, 19 and 20, 11 and 17).
+// Up to 64 rows of x go to the weight-streaming kernel, more to the tiled one.  (Us at 33 / 48 / 64 rows, in parts with what adds them
+// up, one tile of weights against the tiled kernel against this: N 17,920 K 1,536 gated 56 / 61 / 74, 53 / 54 / 54, 52 / 55 / 63; N 1,536 K 8,960
+// in parts 32 / 36 / 42, 30 / 30 / 31, 33 / 35 / 42; N 2,048 K 1,536 17 / 18 / 21, 18 / 18 / 18, 14 / 16 / 21; N 37,888 K 3,584 gated
+// 221 / 266 / 316, 202 / 206 / 205, 175 / 189 / 211; N 3,584 K 18,944 in parts 138 / 148 / 176, 109 / 110 / 110, 94 / 100 / 119.)
 extern "C" int llmserve_gemm_f32(const float* x, const float* w, const float* bias, float* out, int gated, int M, int N,
                                  int K, int splits, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || K % 4 || splits < 1 || (gated && (splits != 1 || N % 2))) return ERR_BAD_ARGUMENT;
-  if (M <= 32)
+  if (M <= 64)
     return gated ? pick_stream<true>(x, w, bias, out, M, N, K, splits, stream)
                  : pick_stream<false>(x, w, bias, out, M, N, K, splits, stream);
   return gated ? launch_tiled<true>(x, w, bias, out, M, N, K, splits, stream)

@@ -735,10 +735,10 @@ class HipKernels:
         )
 
     def _float32_splits(self, rows: int, out_features: int, in_features: int) -> int:
-        """Into how many parts of K a float32 product is cut when its result may stay in parts: up to 32
+        """Into how many parts of K a float32 product is cut when its result may stay in parts: up to 64
         rows (the weight-streaming kernel, workgroups of 16 weight rows) until about a thousand workgroups
         run, a part at least 512 long; more rows (the tiled kernel) as its own estimate has it."""
-        if rows > 32:
+        if rows > 64:
             return self._gemm_f32.llmserve_gemm_f32_parts(rows, out_features, in_features)
         tiles, best = -(-out_features // 16), 1
         for splits in range(2, 9):

@@ -466,6 +466,22 @@ def test_float32_products_in_parts_and_at_odd_sizes(kernels, rows, inner, outer)
     torch.testing.assert_close(gated.cpu().double(), want, **bound)
 
 
+@pytest.mark.parametrize("inner,outer", [(1536, 2048), (1540, 4098), (260, 9002), (4100, 1030)])
+def test_a_float32_row_has_the_same_bits_in_every_batch_of_few_rows(kernels, inner, outer):
+    """Up to 64 rows the waves' walks and the order of their sums follow the weight alone: with four, eight and sixteen waves a
+    workgroup, a K and weight rows that leave remainders, whole, in parts and gated."""
+    k = kernels[torch.float32]
+    x, w = on_gpu(torch.randn(64, inner)), on_gpu(torch.randn(outer, inner) / math.sqrt(inner))
+    handle, gated = k.prepare_linear([w], [on_gpu(torch.randn(outer))]), k.prepare_gated_linear(w[: outer // 2], w[outer // 2 : outer // 2 * 2])
+    forms = [lambda rows: k.linear(rows, handle), lambda rows: k.linear(rows, handle, out_dtype=torch.float32, partial=True), lambda rows: k.gated_linear(rows, gated)]
+    for form in forms:
+        alone = form(x[:7])
+        for rows in (1, 16, 17, 32, 33, 48, 49, 64):
+            assert torch.equal(form(x[:rows])[..., : min(rows, 7), :], alone[..., : min(rows, 7), :]), rows
+    expected = x.double() @ w.double().T + handle.bias.double()
+    torch.testing.assert_close(k.linear(x, handle).double(), expected, atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5)
+
+
 @pytest.mark.parametrize("rows,inner,outer", [(33, 1540, 96), (64, 260, 2050), (97, 516, 7003), (129, 1028, 9001), (230, 260, 37890),
                                               (1000, 300, 8197)])
 def test_float32_tiles(kernels, rows, inner, outer):
