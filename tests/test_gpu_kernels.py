@@ -482,8 +482,8 @@ def test_a_float32_row_has_the_same_bits_in_every_batch_of_few_rows(kernels, inn
     torch.testing.assert_close(k.linear(x, handle).double(), expected, atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5)
 
 
-@pytest.mark.parametrize("rows,inner,outer", [(33, 1540, 96), (64, 260, 2050), (97, 516, 7003), (129, 1028, 9001), (230, 260, 37890),
-                                              (1000, 300, 8197)])
+@pytest.mark.parametrize("rows,inner,outer", [(33, 1540, 96), (64, 260, 2050), (65, 1540, 98), (67, 260, 2050), (97, 516, 7003), (129, 1028, 9001), (230, 260, 37890),
+                                              (509, 300, 16001), (1000, 300, 8197)])
 def test_float32_tiles(kernels, rows, inner, outer):
     """The tiled 32-bit product with each of its five tiles, at rows, weight rows and K that leave remainders (the bound as above)."""
     k = kernels[torch.float32]
