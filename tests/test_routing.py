@@ -287,3 +287,45 @@ def test_walks_of_portions_are_cut_where_it_was_measured_to_pay(keys, blocks, ru
 ])
 def test_eight_waves_walk_where_a_workgroup_has_a_cu(blocks, keys, padded, eight):
     assert HipKernels._portion_eight_waves(blocks, keys, padded) == eight
+
+
+def steps_with_portions(requests: int, chunk: int, longest: int, seed: int, steps: int):
+    """(tokens, requests, longest context) of the steps with a portion in a run of ragged prompts beside decoded tokens."""
+    rng = random.Random(seed)
+    running, left, done = [], 0, 0
+    for _ in range(steps):
+        if not left and len(running) < requests and rng.random() < 0.15:
+            left, done = int(2 ** rng.uniform(4, longest)), 0
+        portion = min(chunk, left)
+        context = max([length for length, _ in running] + [done + portion])
+        if portion:
+            yield len(running) + portion, len(running) + 1, context, bool(running) or portion == left
+        running = [(length + 1, more - 1) for length, more in running if more > 1]
+        if portion:
+            left, done = left - portion, done + portion
+            if not left:
+                running.append((done, int(2 ** rng.uniform(3, 9))))
+
+
+@pytest.mark.parametrize("requests,chunk,longest", [(8, 512, 11), (32, 256, 11), (64, 256, 12), (64, 480, 12), (32, 512, 13)])
+def test_ragged_steps_seldom_capture_a_shape_again(requests, chunk, longest):
+    """A captured step's shape is dropped when too many others have come since.  The graphs kept have to go with the shapes that
+    the buckets make: a shape that is captured anew costs as much as many steps."""
+    from llmserve_amd.engine.runner import ModelRunner
+
+    seen, kept, captured = {}, {}, 0
+    for tokens, present, context, wanted in steps_with_portions(requests, chunk, longest, 1, 20_000):
+        if tokens > 512:  # (launched kernel by kernel)
+            continue
+        padded = ModelRunner._bucket(present + 1)
+        key = (ModelRunner._token_bucket(tokens), padded, ModelRunner._bucket(-(-context // 16)), padded if wanted else 0)
+        seen[key] = seen.get(key, 0) + 1
+        if kept.pop(key, None) is None:
+            if seen[key] < 2:
+                continue
+            captured += 1
+            if len(kept) >= ModelRunner.max_step_graphs:
+                kept.pop(next(iter(kept)))
+        kept[key] = True
+    again = captured - sum(1 for times in seen.values() if times >= 2)
+    assert again <= captured // 4, f"{again} of {captured} captures were of shapes captured before"
