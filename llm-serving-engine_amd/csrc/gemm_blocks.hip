@@ -54,6 +54,7 @@ template <int TN, int TM, bool INSIDE, typename TO, bool GATED>
 __device__ __forceinline__ void store_tiles(const f32x16 (&acc)[TN][TM], float* mine, TO* __restrict__ out,
                                             const void* __restrict__ bias, int bias_is_float, int slice, int M, int N,
                                             int n_wave, int m_wave, int lane) {
+  static_assert(!GATED || sizeof(TO) == 2, "a gated result is bfloat16");
   constexpr int ROW = 32 * TN + 4;  // floats of a transposed row, padded
   constexpr int LANES_A_ROW = 4 * TN, ROWS_A_PASS = 64 / LANES_A_ROW;
   const int r32 = lane & 31, half = lane >> 5;
@@ -83,18 +84,17 @@ __device__ __forceinline__ void store_tiles(const f32x16 (&acc)[TN][TM], float* 
 #pragma unroll
       for (int e = 0; e < 8; ++e) value[e] += bias_here[e];
       if (!INSIDE && m >= M) continue;
-      if (GATED) {
+      if constexpr (GATED) {
         TO* dst = out + (size_t)m * (N / 2) + n_piece / 2;
         float gated[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          // a bfloat16 result takes the hardware's 2^x and 1/x (a tile has 128 of these a lane; the
+          // the hardware's 2^x and 1/x, as the result is bfloat16 (a tile has 128 of these a lane; the
           // library routines are some forty instructions each and took most of a tile's way out)
           const float gate = value[2 * e], up = value[2 * e + 1];
-          gated[e] = sizeof(TO) == 2 ? gate * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gate * -1.44269504088896f)) * up
-                                     : gate / (1.f + expf(-gate)) * up;
+          gated[e] = gate * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gate * -1.44269504088896f)) * up;
         }
-        if (sizeof(TO) == 2 && (INSIDE || (n_piece + 8 <= N && (N / 2) % 4 == 0))) {
+        if (INSIDE || (n_piece + 8 <= N && (N / 2) % 4 == 0)) {
           bf16_t packed[4] = {(bf16_t)gated[0], (bf16_t)gated[1], (bf16_t)gated[2], (bf16_t)gated[3]};
           *(uint2*)dst = *(const uint2*)packed;
         } else {
@@ -358,17 +358,15 @@ static int launch_shape(const void* x, const void* w, const void* bias, int bias
 #undef BLOCK
 }
 
-// x, w bfloat16; out bfloat16 or float32; any M and N, K a multiple of 32, an even N with `gated` (silu).
+// x, w bfloat16; out bfloat16 or float32; any M and N, K a multiple of 32, an even N and a bfloat16 result with `gated` (silu).
 // With splits > 1 (float32 out, not gated, K / splits a multiple of 32) `out` is [splits, M, N]
 // partial sums, the bias in the first.
 extern "C" int llmserve_gemm_blocks(const void* x, const void* w, const void* bias, int bias_is_float, void* out,
                                     int out_is_float, int gated, int M, int N, int K, int splits, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (K <= 0 || K % 32 || (gated && N % 2) || splits < 1 || gated > 1) return ERR_BAD_ARGUMENT;  // (this epilogue knows silu alone)
+  if (K <= 0 || K % 32 || (gated && N % 2) || splits < 1 || gated > 1 || (gated && out_is_float)) return ERR_BAD_ARGUMENT;  // (this epilogue knows silu alone)
   if (splits > 1 && (gated || !out_is_float || K % splits || (K / splits) % 32)) return ERR_BAD_ARGUMENT;
-  if (gated)
-    return out_is_float ? launch_shape<float, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream)
-                        : launch_shape<bf16_t, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
+  if (gated) return launch_shape<bf16_t, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
   return out_is_float ? launch_shape<float, false>(x, w, bias, bias_is_float, out, M, N, K, splits, stream)
                       : launch_shape<bf16_t, false>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
 }
