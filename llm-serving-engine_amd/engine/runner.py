@@ -408,7 +408,7 @@ class ModelRunner:
     def _request_bucket(cls, requests: int) -> int:
         """The rows of the graph that a step of so many single tokens replays: a power of two up to 128, where the
         kernels' cost goes by tiles of 16 to 128 rows and padding costs little (65 requests of the 1.5B sizes 2.37 ms a
-        step, 128 requests 2.55), and multiples of 64 beyond, where every product is the library's and goes by its rows
+        step, 128 requests 2.55), and multiples of 64 beyond, where the products' tiles go by its rows
         (192 requests take 3.80 ms a step in a graph of 256 rows and 3.66 in one of 192)."""
         return cls._bucket(requests) if requests <= 128 else -(-requests // 64) * 64
 
@@ -462,8 +462,8 @@ class ModelRunner:
 
     @staticmethod
     def _token_bucket(tokens: int) -> int:
-        """The tokens of the graph that a step of so many replays: few shapes, and no more than a quarter of padding from 129 on,
-        where a step's time goes by its rows (287 tokens of the 1.5B sizes in a graph of 384 rows 3.09 ms, of 320 2.93; 129
+        """The tokens of the graph that a step of so many replays: few shapes, and between 129 and 512, where a step's time goes by its
+        rows, at most a quarter more rows than tokens (287 tokens of the 1.5B sizes in a graph of 384 rows 3.09 ms, of 320 2.93; 129
         in float32 6.97 in 192 rows, 6.52 in 160)."""
         for size in (16, 32, 64, 96, 128, 160, 192, 224, 256, 320, 384, 448, 512, 768, 1024):
             if tokens <= size:

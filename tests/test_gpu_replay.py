@@ -172,7 +172,7 @@ def test_captured_steps_of_many_rows_at_benchmark_layer_sizes(wide_models, sizes
     """Decode steps of 17 rows and more are replayed from a graph in which the products go other ways than
     in every other step (up to 64 rows the kernel that streams a weight through a ring in LDS, the BLAS
     library or the weight-streaming kernel for small weights; 65 to 128 rows the ring kernel with eight tiles
-    of x; beyond that the library, in a graph of a multiple of 64 rows).
+    of x or, where K may be cut, the tiled kernel; beyond that the tiled kernel or the library, in a graph of a multiple of 64 rows).
     So many requests decode side by side through the step function; every step's logits are
     compared with the plain forward over each request's whole sequence."""
     from llmserve_amd import CacheConfig, ModelRunner, StepEntry
