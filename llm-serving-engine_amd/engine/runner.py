@@ -172,7 +172,8 @@ class ModelRunner:
 
     # Graphs kept of steps with portions.  Eight of the thirteen sizes of `_token_bucket` up to `graph_token_limit` lie beyond 128 tokens;
     # ragged prompts beside up to 64 decoded tokens meet 70 to 90 shapes in 5,000 such steps.  With 48 graphs kept they drop and
-    # capture shapes again (184 captures), with 72 hardly ever (76 captures; with 96 as many).
+    # capture shapes again (184 captures), with 72 hardly ever (76 captures; with 96 as many).  A graph holds 60 MB at the 1.5B sizes,
+    # 95 MB at the 7B sizes.
     max_step_graphs = 72
 
     def __init__(
