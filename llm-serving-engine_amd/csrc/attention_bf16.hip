@@ -325,7 +325,7 @@ __global__ __launch_bounds__(WAVES * 64, (COLUMN_TILES > 2 || HEAD_DIM > 192 || 
     float* __restrict__ partial_ml, bf16_t* __restrict__ keys,
     bf16_t* __restrict__ values, const int* __restrict__ block_tables, int table_width,
     const int* __restrict__ positions, const int* __restrict__ work, int heads, int kv_heads, int tokens_per_tile,
-    int page_size, int page_shift, float scale, int window, int splits, FusedDecode fused, ScoreChange change, Finish finish) {
+    int page_size, int page_shift, float scale, int window, int splits, FusedDecode fused, ScoreChange change, Finish finish, Ahead ahead) {
   static_assert(!FUSED || CHANGED == CHANGED_NOT || CHANGED == CHANGED_EDGES, "the fused decode form leaves the scores as they are");
   constexpr bool PAIRED = CHANGED == CHANGED_MAPS && COLUMN_TILES == 1;  // a head's two maps are neighbouring columns
   constexpr bool TILE_A_MAP = CHANGED == CHANGED_MAPS && COLUMN_TILES == 2;
@@ -333,6 +333,11 @@ __global__ __launch_bounds__(WAVES * 64, (COLUMN_TILES > 2 || HEAD_DIM > 192 || 
   if (FUSED)  // a short kernel: fetch all arguments in one go rather than each before its first use
     asm volatile("" ::"s"(row_width), "s"(table_width), "s"(heads), "s"(kv_heads), "s"(page_size), "s"(page_shift),
                  "s"(scale), "s"(window), "s"(splits), "s"(fused.pairing));
+  if (FUSED && (int)blockIdx.z >= splits) {  // (behind the workgroups that attend)
+    const unsigned plane = gridDim.x * gridDim.y;
+    bring_ahead(ahead, blockIdx.z * plane + blockIdx.y * gridDim.x + blockIdx.x, splits * plane, gridDim.z * plane);
+    return;
+  }
   const int group = heads / kv_heads;
   const int kv_head = blockIdx.y % kv_heads, head_tile = blockIdx.y / kv_heads;
   const int heads_here = min(group - head_tile * 16, 16);
@@ -1280,7 +1285,7 @@ static int launch_tiles(const void* qkv, int row_width, void* out, int out_strid
                         void* keys, void* values, const int* block_tables, int table_width,
                         const int* positions, const int* work, int tiles, int heads, int kv_heads,
                         int tokens_per_tile, int page_size, float scale, int window, int splits, FusedDecode fused,
-                        hipStream_t stream, ScoreChange change, Finish finish) {
+                        hipStream_t stream, ScoreChange change, Finish finish, int helpers, Ahead ahead) {
   const int group = heads / kv_heads;
   const int page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
   const int head_tiles = (group + 15) / 16;
@@ -1294,10 +1299,11 @@ static int launch_tiles(const void* qkv, int row_width, void* out, int out_strid
       asked = true;
     }
   }
-  hipLaunchKernelGGL((attention_tiles_kernel<COLUMN_TILES, FUSED, WAVES, CHANGED>), dim3(tiles, kv_heads * head_tiles, splits),
+  const int plane = tiles * kv_heads * head_tiles, planes = FUSED ? splits + (helpers + plane - 1) / plane : splits;
+  hipLaunchKernelGGL((attention_tiles_kernel<COLUMN_TILES, FUSED, WAVES, CHANGED>), dim3(tiles, kv_heads * head_tiles, planes),
                      dim3(WAVES * 64), shared, stream, (const bf16_t*)qkv, row_width, (bf16_t*)out, out_stride, partial_acc,
                      partial_ml, (bf16_t*)keys, (bf16_t*)values, block_tables, table_width, positions, work,
-                     heads, kv_heads, tokens_per_tile, page_size, page_shift, scale, window, splits, fused, change, finish);
+                     heads, kv_heads, tokens_per_tile, page_size, page_shift, scale, window, splits, fused, change, finish, ahead);
   return LAUNCH_STATUS();
 }
 
@@ -1330,6 +1336,7 @@ extern "C" int llmserve_attention_can_fuse(int pairing) {
 // this file), `sinks` (float32 [heads], or null) add exp(sink) to a head's denominator, `keep_first` keeps a sequence's first
 // keys visible behind a window, `chunk` (0 for none; not together with a window) shows a query the keys of its own chunk of
 // positions; slopes, cap and kept keys not together with `fuse` & 1, sinks not with `fuse` & 2.
+// `helpers` further workgroups, with `fuse` & 1, bring the runs of `ahead` into the caches (common.h: Ahead).
 // `bias` (float32 [heads][reach + BIAS_SPARE], common.h: bias_element, or null) adds a bias by distance to the scores, `gates`
 // (bfloat16 rows of `gate_stride`, or null) multiplies a result's element with the sigmoid of column gate_first + its own;
 // `maps` 2: differential attention, column_tiles 2 with work items made for one column tile, or, in a step of single tokens with up
@@ -1346,8 +1353,11 @@ extern "C" int llmserve_attention_tiles(const void* qkv, int row_width, void* ou
                                         const float* table, int pairing, const int* slots, const float* slopes,
                                         float soft_cap, const float* sinks, int keep_first, int chunk, const float* bias, int reach,
                                         int maps, int vdim, float factor, float eps, float out_scale, const void* gates,
-                                        int gate_stride, int gate_first, hipStream_t stream) {
+                                        int gate_stride, int gate_first, int helpers, const void* ahead, int stripe, int stripes,
+                                        hipStream_t stream) {
   if (tiles <= 0) return 0;
+  if (!ahead_fits(helpers, ahead, stripe, stripes)) return ERR_BAD_ARGUMENT;
+  const Ahead next = {(const unsigned char*)ahead, (unsigned)stripe, (unsigned)stripes};
   const bool wide = (fuse & 16) != 0;  // eight waves a workgroup, with two column tiles and no change of the scores
   fuse &= ~16;
   if (keep_first < 0 || chunk < 0 || (chunk > 0 && window > 0)) return ERR_BAD_ARGUMENT;
@@ -1383,7 +1393,7 @@ extern "C" int llmserve_attention_tiles(const void* qkv, int row_width, void* ou
 #define LAUNCH_TILES(COLUMN_TILES, FUSED, WAVES, CHANGED)                                                                 \
   launch_tiles<COLUMN_TILES, FUSED, WAVES, CHANGED>(qkv, row_width, out, out_stride, partial_acc, partial_ml, keys, values, \
                                                     block_tables, table_width, positions, work, tiles, heads, kv_heads,     \
-                                                    tokens_per_tile, page_size, scale, window, splits, fused, stream, change, finish)
+                                                    tokens_per_tile, page_size, scale, window, splits, fused, stream, change, finish, helpers, next)
     status = edges ? LAUNCH_TILES(1, true, FUSED_WAVES, CHANGED_EDGES) : LAUNCH_TILES(1, true, FUSED_WAVES, CHANGED_NOT);
   } else if (finished) {
 #if HEAD_DIM % 32 == 0

@@ -104,3 +104,36 @@ __device__ __forceinline__ size_t value_element(int d, int offset, int page_size
 // below 0 (keys that are masked) nothing.
 #define BIAS_SPARE 24
 __device__ __forceinline__ int bias_element(int distance, int reach) { return reach + 7 - max(min(distance, reach + 7), -8); }
+
+// Memory that the next kernel reads, brought into the caches by workgroups of a kernel that leaves the path to memory idle: a
+// weight as `stripes` runs of `stripe` bytes (a multiple of 16; the rows that one workgroup of the next kernel takes), of
+// which that kernel's workgroup i reads run i.  The chip hands the workgroups of a launch to its eight chiplets in turn and each has an
+// L2 of its own, so the runs i, i + 8, ... are brought by workgroups of the chiplet that will read them.
+struct Ahead {
+  const unsigned char* from;  // null: nothing
+  unsigned stripe, stripes;
+};
+// What an entry point takes: `helpers` workgroups for it (0: none, and the rest is not looked at), 16-byte pieces counted in 32 bits.
+static inline bool ahead_fits(int helpers, const void* from, int stripe, int stripes) {
+  if (helpers == 0) return true;
+  return helpers > 0 && from && (size_t)from % 16 == 0 && stripe >= 16 && stripe % 16 == 0 && stripes >= 1 && (long)stripe * stripes < (1L << 31);
+}
+// For a workgroup that does nothing else: number `index` of the launch's `all`, of which those from `first` on are such ones.
+__device__ __forceinline__ void bring_ahead(const Ahead& ahead, unsigned index, unsigned first, unsigned all) {
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  const unsigned chiplet = index % 8, lowest = first + (chiplet + 8 - first % 8) % 8;
+  const unsigned rank = (index - lowest) / 8, helpers = (all - 1 - lowest) / 8 + 1;
+  if (!ahead.from || chiplet >= ahead.stripes) return;
+  const unsigned a_stripe = ahead.stripe / 16, pieces = (ahead.stripes - chiplet + 7) / 8 * a_stripe;
+  constexpr unsigned TOGETHER = 4;  // loads of a thread under way
+  for (unsigned at = rank * TOGETHER * blockDim.x + threadIdx.x; at < pieces; at += helpers * TOGETHER * blockDim.x) {
+    u32x4 piece[TOGETHER];
+#pragma unroll
+    for (unsigned u = 0; u < TOGETHER; ++u) {
+      const unsigned i = min(at + u * blockDim.x, pieces - 1), stripe = i / a_stripe;
+      piece[u] = *(const u32x4*)(ahead.from + (size_t)(chiplet + 8 * stripe) * ahead.stripe + (size_t)(i - stripe * a_stripe) * 16);
+    }
+#pragma unroll
+    for (unsigned u = 0; u < TOGETHER; ++u) asm volatile("" ::"v"(piece[u]));
+  }
+}

@@ -144,8 +144,12 @@ __global__ __launch_bounds__(1024) void add_rms_norm_vector_kernel(float* __rest
                                                                    size_t part_stride,
                                                                    const void* __restrict__ weight,
                                                                    int weight_is_float, TO* __restrict__ out,
-                                                                   int width, float eps) {
+                                                                   int width, float eps, int rows, Ahead ahead) {
   __shared__ float shared[17];
+  if ((int)blockIdx.x >= rows) {  // (a few rows wait for their trips to memory; the path to it is free for the next product's weight)
+    bring_ahead(ahead, blockIdx.x, rows, gridDim.x);
+    return;
+  }
   const int quads = width / 4;
   float4* row = (float4*)(hidden + (size_t)blockIdx.x * width);
   const float* add = delta ? delta + (size_t)blockIdx.x * width : nullptr;
@@ -195,35 +199,37 @@ __global__ __launch_bounds__(1024) void add_rms_norm_vector_kernel(float* __rest
 template <typename TO>
 static void launch_add_rms_norm_vector(float* hidden, const float* delta, int parts, size_t part_stride,
                                        const void* weight, int weight_is_float, TO* out, int rows, int width,
-                                       float eps, hipStream_t stream) {
+                                       float eps, int helpers, Ahead ahead, hipStream_t stream) {
   // a thread for every four floats of the row, in whole waves: the block size depends on the width alone
   const int quads = width / 4;
   const int pieces = quads <= 1024 ? 1 : quads <= 2048 ? 2 : 4;
   const int threads = ((quads + pieces - 1) / pieces + WAVE - 1) / WAVE * WAVE;
   if (pieces == 1)
-    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 1>), dim3(rows), dim3(threads), 0, stream, hidden, delta, parts,
-                       part_stride, weight, weight_is_float, out, width, eps);
+    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 1>), dim3(rows + helpers), dim3(threads), 0, stream, hidden, delta, parts,
+                       part_stride, weight, weight_is_float, out, width, eps, rows, ahead);
   else if (pieces == 2)
-    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 2>), dim3(rows), dim3(threads), 0, stream, hidden, delta, parts,
-                       part_stride, weight, weight_is_float, out, width, eps);
+    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 2>), dim3(rows + helpers), dim3(threads), 0, stream, hidden, delta, parts,
+                       part_stride, weight, weight_is_float, out, width, eps, rows, ahead);
   else
-    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 4>), dim3(rows), dim3(threads), 0, stream, hidden, delta, parts,
-                       part_stride, weight, weight_is_float, out, width, eps);
+    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 4>), dim3(rows + helpers), dim3(threads), 0, stream, hidden, delta, parts,
+                       part_stride, weight, weight_is_float, out, width, eps, rows, ahead);
 }
 
 extern "C" int llmserve_add_rms_norm(float* hidden, const float* delta, int parts, const void* weight,
                                      int weight_is_float, void* out, int out_is_float, int rows, int width, float eps,
-                                     hipStream_t stream) {
+                                     int helpers, const void* ahead, int stripe, int stripes, hipStream_t stream) {
   if (rows <= 0) return 0;
   if (delta && parts < 1) return ERR_BAD_ARGUMENT;
+  if (!ahead_fits(helpers, ahead, stripe, stripes)) return ERR_BAD_ARGUMENT;
+  const Ahead next = {(const unsigned char*)ahead, (unsigned)stripe, (unsigned)stripes};
   const size_t part_stride = (size_t)rows * width;
   if (width % 4 == 0 && width <= 1024 * 4 * 4) {
     if (out_is_float)
       launch_add_rms_norm_vector<float>(hidden, delta, parts, part_stride, weight, weight_is_float, (float*)out, rows,
-                                        width, eps, stream);
+                                        width, eps, helpers, next, stream);
     else
       launch_add_rms_norm_vector<bf16_t>(hidden, delta, parts, part_stride, weight, weight_is_float, (bf16_t*)out,
-                                         rows, width, eps, stream);
+                                         rows, width, eps, helpers, next, stream);
     return LAUNCH_STATUS();
   }
   const int threads = width >= 2048 ? 512 : 256;

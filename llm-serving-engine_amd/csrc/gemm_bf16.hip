@@ -422,8 +422,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
                                                                  const bf16_t* __restrict__ w,
                                                                  const void* __restrict__ bias, int bias_is_float,
                                                                  TO* __restrict__ out, int M, int N, int K,
-                                                                 int k_split, Tail tail, Link link) {
+                                                                 int k_split, Tail tail, Link link, int tiles, Ahead ahead) {
   extern __shared__ __attribute__((aligned(16))) unsigned char stream_lds[];
+  if (LINK == INTO_NORM && (int)blockIdx.x >= tiles) {
+    bring_ahead(ahead, blockIdx.x, tiles, gridDim.x);
+    return;
+  }
   constexpr int OPERANDS = (NT + MT) * G;                // of one group: the weight tiles' steps, then x's
   constexpr int STAGE_BYTES = OPERANDS * STREAM_CHUNK;
   constexpr int WAVE_BYTES = STREAM_STAGES * STAGE_BYTES;
@@ -573,7 +577,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
 
 template <int WAVES, int NT, int MT, int G, typename TO, int GATED, int LINK = NO_LINK>
 static int launch_stream(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N,
-                         int K, int splits, hipStream_t stream, Tail tail = {}, Link link = {}) {
+                         int K, int splits, hipStream_t stream, Tail tail = {}, Link link = {}, int helpers = 0,
+                         Ahead ahead = {}) {
   const size_t stages = (size_t)WAVES * STREAM_STAGES * (NT + MT) * G * STREAM_CHUNK;
   const size_t sums = (size_t)WAVES * NT * MT * 64 * 4 * sizeof(float);
   const size_t lds = (stages > sums ? stages : sums) + (LINK == SCALED ? ((size_t)(link.tiles + 15) / 16 * 256 + WAVES * 16) * sizeof(float) : 0);
@@ -586,9 +591,10 @@ static int launch_stream(const void* x, const void* w, const void* bias, int bia
       asked = true;
     }
   }
-  hipLaunchKernelGGL((gemm_stream_kernel<WAVES, NT, MT, G, TO, GATED, LINK>), dim3((N + 16 * NT - 1) / (16 * NT), splits),
+  const int tiles = (N + 16 * NT - 1) / (16 * NT);
+  hipLaunchKernelGGL((gemm_stream_kernel<WAVES, NT, MT, G, TO, GATED, LINK>), dim3(tiles + helpers, splits),
                      dim3(WAVES * 64), lds, stream, (const bf16_t*)x, (const bf16_t*)w, bias, bias_is_float, (TO*)out, M,
-                     N, K, K / splits, tail, link);
+                     N, K, K / splits, tail, link, tiles, ahead);
   return LAUNCH_STATUS();
 }
 
@@ -678,8 +684,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* _
                                                                  const bf16_t* __restrict__ w,
                                                                  const void* __restrict__ bias, int bias_is_float,
                                                                  float* __restrict__ out, int M, int N, int K,
-                                                                 int k_split, Link link) {
+                                                                 int k_split, Link link, int tiles, Ahead ahead) {
   extern __shared__ float partial[];  // [WAVES][64 lanes][4]
+  if (LINK == INTO_NORM && (int)blockIdx.x >= tiles) {
+    bring_ahead(ahead, blockIdx.x, tiles, gridDim.x);
+    return;
+  }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
   const int n = min((int)blockIdx.x * 16 + r, N - 1);
@@ -761,18 +771,19 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* _
 
 template <int S, int LINK>
 static int launch_merged(const void* split_x, const float* split_ml, const void* w, const void* bias, int bias_is_float,
-                         float* out, int M, int N, int K, int k_splits, hipStream_t stream, Link link) {
+                         float* out, int M, int N, int K, int k_splits, hipStream_t stream, Link link, int helpers, Ahead ahead) {
   const int groups = K / k_splits / (STEP * GROUP);
-  const dim3 grid((N + 15) / 16, k_splits);
+  const int tiles = (N + 15) / 16;
+  const dim3 grid(tiles + helpers, k_splits);
   if (LINK == INTO_NORM && groups > 8)  // whole sums: a head a wave, or two
     hipLaunchKernelGGL((gemm_merged_kernel<12, S, LINK>), grid, dim3(768), 12 * 64 * 4 * sizeof(float), stream,
-                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link);
+                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link, tiles, ahead);
   else if (groups <= 4)
     hipLaunchKernelGGL((gemm_merged_kernel<4, S, LINK>), grid, dim3(256), 4 * 64 * 4 * sizeof(float), stream,
-                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link);
+                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link, tiles, ahead);
   else
     hipLaunchKernelGGL((gemm_merged_kernel<8, S, LINK>), grid, dim3(512), 8 * 64 * 4 * sizeof(float), stream,
-                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link);
+                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link, tiles, ahead);
   return LAUNCH_STATUS();
 }
 
@@ -781,13 +792,13 @@ static int launch_merged(const void* split_x, const float* split_ml, const void*
 // M <= 16; K a multiple of 128 * k_splits; splits 2, 3, 4, 6 or 8.
 template <int LINK>
 static int pick_merged(const void* split_x, const float* split_ml, int splits, const void* w, const void* bias, int bias_is_float,
-                       float* out, int M, int N, int K, int k_splits, hipStream_t stream, Link link) {
+                       float* out, int M, int N, int K, int k_splits, hipStream_t stream, Link link, int helpers = 0, Ahead ahead = {}) {
   switch (splits) {
-    case 2: return launch_merged<2, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link);
-    case 3: return launch_merged<3, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link);
-    case 4: return launch_merged<4, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link);
-    case 6: return launch_merged<6, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link);
-    case 8: return launch_merged<8, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link);
+    case 2: return launch_merged<2, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link, helpers, ahead);
+    case 3: return launch_merged<3, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link, helpers, ahead);
+    case 4: return launch_merged<4, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link, helpers, ahead);
+    case 6: return launch_merged<6, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link, helpers, ahead);
+    case 8: return launch_merged<8, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link, helpers, ahead);
     default: return ERR_BAD_ARGUMENT;
   }
 }
@@ -804,17 +815,20 @@ static int sums_stride(int M) { return M <= 16 ? 16 : M <= 32 ? 32 : 64; }
 
 // The product (split_x null: of x; else of the merge of its key splits, as above, M <= 16) into a norm: hidden [M, N] float32 +=
 // x . w^T (+ bias); rows [M, N] bfloat16 = hidden * weight; sums float32 [N / 16, 16 rows, or 32 or 64: as many as hold M].
-// M <= 64, N a multiple of 16, K of 128.
+// M <= 64, N a multiple of 16, K of 128.  `helpers` further workgroups bring the runs of `ahead` into the caches (common.h: Ahead).
 extern "C" int llmserve_gemm_into_norm(const void* x, const void* split_x, const float* split_ml, int splits, const void* w, const void* bias,
                                        int bias_is_float, float* hidden, const void* weight, int weight_is_float, void* rows, float* sums,
-                                       int M, int N, int K, hipStream_t stream) {
+                                       int M, int N, int K, int helpers, const void* ahead, int stripe, int stripes,
+                                       hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 64 || N % 16 || K <= 0 || K % (STEP * GROUP) || (split_x && M > 16) || (!x && !split_x)) return ERR_BAD_ARGUMENT;
+  if (!ahead_fits(helpers, ahead, stripe, stripes)) return ERR_BAD_ARGUMENT;
+  const Ahead next = {(const unsigned char*)ahead, (unsigned)stripe, (unsigned)stripes};
   const Link link{hidden, weight, weight_is_float, (bf16_t*)rows, sums, sums_stride(M), N / 16, 0.f, 0.f};
-  if (split_x) return pick_merged<INTO_NORM>(split_x, split_ml, splits, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, link);
-  if (M <= 16) return launch_stream<4, 1, 1, 4, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
-  if (M <= 32) return launch_stream<4, 1, 2, 2, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
-  return launch_stream<4, 1, 4, 1, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
+  if (split_x) return pick_merged<INTO_NORM>(split_x, split_ml, splits, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, link, helpers, next);
+  if (M <= 16) return launch_stream<4, 1, 1, 4, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link, helpers, next);
+  if (M <= 32) return launch_stream<4, 1, 2, 2, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link, helpers, next);
+  return launch_stream<4, 1, 4, 1, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link, helpers, next);
 }
 
 // ---------------------------------------------------------------------------- 16 < M <= 64

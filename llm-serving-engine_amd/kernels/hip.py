@@ -54,7 +54,7 @@ def _in_pieces(*tensors: torch.Tensor) -> bool:
 # costs no guessing: a decode step is replayed from a graph, but every other step pays per launch.
 _SIGNATURES = {
     "llmserve_embedding": "pippiifppip",
-    "llmserve_add_rms_norm": "ppipipiiifp",
+    "llmserve_add_rms_norm": "ppipipiiifipiip",
     "llmserve_rotary_table": "pppiip",
     "llmserve_rotate_and_store": "piipiiiiipppip",
     "llmserve_silu_mul": "pipiiip",
@@ -74,14 +74,14 @@ _SIGNATURES = {
     "llmserve_gemm_medium": "pppipiiiiiip",
     "llmserve_gemm_ring": "pppipiiiiiiip",
     "llmserve_gemm_merged": "ppippipiiiip",
-    "llmserve_gemm_into_norm": "pppippippippiiip",
+    "llmserve_gemm_into_norm": "pppippippippiiiipiip",
     "llmserve_gemm_scaled": "ppfppiiiip",
     "llmserve_gemm_scaled_streams": "iii",
     "llmserve_gemm_blocks": "pppipiiiiiip",
     "llmserve_gemm_blocks_parts": "iii",
     "llmserve_attention_generic": "pipiipppippiiiiifipfpiiipip",
     "llmserve_attention_f32": "pipipppppippiiiiiifiipfpiiipip",
-    "llmserve_attention_tiles": "pipipppppippiiiiiifiiipippfpiipiiifffpiip",
+    "llmserve_attention_tiles": "pipipppppippiiiiiifiiipippfpiipiiifffpiiipiip",
     "llmserve_attention_portions": "pipipppppippiiiiiifiip",
     "llmserve_attention_can_fuse": "i",
     "llmserve_argmax": "ppppiip",
@@ -211,6 +211,8 @@ class ScaledRows:
 
 
 class HipKernels:
+    brings_ahead = True  # `add_rms_norm` takes the weight of its reader along (`_whole_ahead`)
+
     def __init__(
         self, dtype: torch.dtype = torch.bfloat16, device: str | torch.device = "cuda:0", *, library_products: bool = True,
         shared_portions: str = "auto",
@@ -330,7 +332,34 @@ class HipKernels:
         _check(status, "embedding")
         return out
 
-    def add_rms_norm(self, hidden, delta, weight, eps: float) -> torch.Tensor:
+    @staticmethod
+    def _ahead(weights: LinearWeights | None, busy: int, up_to: int, tiles: int = 1) -> tuple:
+        """What a kernel of `busy` workgroups is told of the weight that the next product reads (csrc/common.h: Ahead), which takes
+        `tiles` tiles of 16 weight rows a workgroup: (workgroups that bring it into the caches, its address, bytes a run, runs).  As
+        many workgroups as fill the CUs that the others leave idle; the weight's first `up_to` bytes, (0, ...) for nothing."""
+        if weights is None or weights.weight.dtype != torch.bfloat16 or not _in_pieces(weights.weight) or weights.in_features % 8 or busy >= 256:
+            return 0, None, 0, 0
+        stripe = 32 * tiles * weights.in_features
+        stripes = min(weights.out_features // (16 * tiles), up_to // stripe)
+        return (256 - busy, _pointer(weights.weight), stripe, stripes) if stripes > 0 else (0, None, 0, 0)
+
+    # The bytes of a weight that are brought ahead of a step of up to 64 single tokens: whole weights that a chiplet's L2 (4 MB) holds an eighth of beside
+    # what passes through it.  At the 1.5B sizes qkv is 6.3 MB and o 4.7: out of the L2 a product takes 2.6 us, out of memory 4.3.  A step, ms, before ->
+    # after, by the norm and by the attention: 1 row 1.308 -> 1.292, 8 rows 1.424 -> 1.382, 64 rows 2.067 -> 1.944, 8 rows over 8,192 keys
+    # 1.783 -> 1.737.  The 7B sizes' qkv and o (33 and 26 MB) gain nothing from their first 8 MB.
+    _WHOLE_AHEAD = 8 << 20
+
+    # Of gate and up, beside an output projection that merges key splits, whose 96 workgroups wait more than they read (8 us for 4.7 MB): as much as
+    # they leave time for.  A step at 1 and 8 rows, ms, with nothing, 8, 16, 24, 30 and 38 MB: 1.271 1.259 1.253 1.255 1.244 1.298, 1.382 1.374 1.366 1.364
+    # 1.353 1.385.  Beside the projection that has no splits to merge (4.8 us) 8 MB gain nothing and 16 lose 3 %.
+    _MERGING_AHEAD = 30 << 20
+
+    def _whole_ahead(self, weights: LinearWeights | None, rows: int, busy: int) -> tuple:
+        if weights is None or rows > 64 or weights.weight.numel() * weights.weight.element_size() > self._WHOLE_AHEAD:
+            return 0, None, 0, 0
+        return self._ahead(weights, busy, self._WHOLE_AHEAD)
+
+    def add_rms_norm(self, hidden, delta, weight, eps: float, ahead=None) -> torch.Tensor:
         rows, width = hidden.shape
         if hidden.dtype != torch.float32 or (delta is not None and delta.dtype != torch.float32):
             raise KernelError("add_rms_norm: the residual stream and what is added to it are float32")
@@ -338,7 +367,7 @@ class HipKernels:
         parts = 1 if delta is None or delta.ndim == 2 else delta.shape[0]  # [parts, rows, width]: partial sums
         status = self._elementwise.llmserve_add_rms_norm(
             _pointer(hidden), _pointer(delta), parts, _pointer(weight), _is_float(weight), _pointer(out),
-            _is_float(out), rows, width, eps, self._stream,
+            _is_float(out), rows, width, eps, *self._whole_ahead(ahead, rows, rows), self._stream,
         )
         _check(status, "add_rms_norm")
         return out
@@ -782,7 +811,8 @@ class HipKernels:
         status = self._gemm_bf16.llmserve_gemm_into_norm(
             _pointer(x) if split is None else None, _pointer(split_x), _pointer(split_ml), splits, _pointer(project.weight), _pointer(bias),
             _is_float(bias) if bias is not None else 0, _pointer(hidden), _pointer(into.weight), _is_float(into.weight), _pointer(scaled),
-            _pointer(sums), rows, width, project.in_features, self._stream,
+            _pointer(sums), rows, width, project.in_features, *self._ahead(reader.both if split is not None else None, width // 16, self._MERGING_AHEAD, max(1, tiles)),
+            self._stream,
         )
         _check(status, "linear into a norm")
         return ScaledRows(scaled, sums, into.eps, reader, tiles)
@@ -1204,7 +1234,7 @@ class HipKernels:
         )
         _check(status, "paged_attention")
 
-    def _attention_tiles(self, qkv, out, layout, batch, cell, group, scale: float, window: int, fuse=None, unmerged=False, changed=None, finish=None):
+    def _attention_tiles(self, qkv, out, layout, batch, cell, group, scale: float, window: int, fuse=None, unmerged=False, changed=None, finish=None, ahead=None):
         """The MFMA kernel: requests that bring a few tokens (decoding) one column tile per
         wave, split over the keys when there are few of them; longer portions two tiles
         per wave.  `fuse` = (rotary table, pairing) lets a step of single tokens rotate and
@@ -1364,7 +1394,7 @@ class HipKernels:
                 column_tiles if maps == 1 or paired else 2, tokens, heads, kv_heads, group.page_size, scale, window, splits, (1 if fuse is not None else 0) + (2 if unmerged else 0) + (4 if by_item else 0) + (8 if finish is not None and batch.max_query_length == 1 else 0) + (16 if eight_waves else 0),
                 _pointer(table), _PAIRINGS[pairing], _pointer(group.slot_mapping), _pointer(slopes), soft_cap, _pointer(sinks), keep_first, chunk,
                 _pointer(bias), reach, maps, vdim, float(factor), float(eps), float(out_scale), _pointer(gates),
-                gates.shape[1] if gates is not None else 0, gate_first, self._stream,
+                gates.shape[1] if gates is not None else 0, gate_first, *self._whole_ahead(ahead if fuse is not None else None, tokens, items * kv_heads * head_tiles * splits), self._stream,
             )
             _check(status, "paged_attention")
             if unmerged and splits > 1:
@@ -1432,7 +1462,7 @@ class HipKernels:
                 # 3.29 / 3.67 with the merging kernel): what decides is the weight, so the gate is its size.
                 and project.weight.numel() * project.weight.element_size() <= self.merge_weight_bytes
             )
-            left = self._attention_tiles(qkv, out, layout, batch, cell, group, scale, int(window or 0), fuse=(table, pairing), unmerged=merging,
+            left = self._attention_tiles(qkv, out, layout, batch, cell, group, scale, int(window or 0), fuse=(table, pairing), unmerged=merging, ahead=project,
                                          changed=(None, 0.0, sinks, 0, int(chunk or 0)) if sinks is not None or chunk else None)
             if left is None:
                 return out, False

@@ -80,9 +80,13 @@ class PreNormBlock(Block):
         as_they_stand = getattr(type(norm), "forward", None) is RMSNorm.forward and getattr(type(feed_forward), "forward", None) is GatedMLP.forward
         if getattr(self.mixer, "takes_into", False) and as_they_stand:
             self._norm_into = getattr(kernels, "norm_into", None)
+        # (a library's norm may take the weight of the product behind it along, to bring it into the caches meanwhile)
+        self._ahead = {}
+        if getattr(kernels, "brings_ahead", False) and getattr(type(self.mixer_norm), "forward", None) is RMSNorm.forward:
+            self._ahead = {"ahead": getattr(self.mixer, "qkv", None)}
 
     def forward(self, hidden, delta, batch, cell) -> torch.Tensor:
-        normed = self.mixer_norm.forward(hidden, delta)
+        normed = self.mixer_norm.forward(hidden, delta, **self._ahead)
         if self._norm_into is not None:
             norm = self.feed_forward_norm
             mixed = self.mixer.forward(normed, batch, cell, into=self._norm_into(hidden, norm.weight, norm.spec.eps, self.feed_forward.gate_up))

@@ -40,9 +40,10 @@ class RMSNorm(Part):
         if spec.weight_scale != 1.0 or spec.weight_offset != 0.0:
             self.weight = ((self.weight.float() + float(spec.weight_offset)) * float(spec.weight_scale)).contiguous()
 
-    def forward(self, hidden: torch.Tensor, delta: torch.Tensor | None) -> torch.Tensor:
-        """Adds `delta` into `hidden` (in place) and returns the normed rows in the run dtype."""
-        return self.kernels.add_rms_norm(hidden, delta, self.weight, self.spec.eps)
+    def forward(self, hidden: torch.Tensor, delta: torch.Tensor | None, **ahead) -> torch.Tensor:
+        """Adds `delta` into `hidden` (in place) and returns the normed rows in the run dtype.  `ahead`: the prepared weight that
+        their reader multiplies them with, for a kernel library that can bring it into the caches meanwhile."""
+        return self.kernels.add_rms_norm(hidden, delta, self.weight, self.spec.eps, **ahead)
 
     def add_normed(self, hidden: torch.Tensor, update: torch.Tensor) -> torch.Tensor:
         """The norm on a sublayer's output instead of its input: `hidden += update * rsqrt(mean(update^2) + eps) *
