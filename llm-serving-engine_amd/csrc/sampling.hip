@@ -216,30 +216,36 @@ extern "C" int llmserve_argmax_static(const float* logits, int* out, int rows, i
 // ---------------------------------------------------------------------------------------------
 // Sampling with a temperature and top-p.
 //
-// A row is cut into `pieces` contiguous pieces and every stage runs one block per (row, piece), so
-// that a few rows of a large vocabulary use the whole chip; what a stage needs of the whole row it
-// takes from what the stages before it wrote, every block for itself and all alike.
+// Every launch but the last cuts a row into `pieces` contiguous pieces, a block a (row, piece), so that a few rows of a large
+// vocabulary use the whole chip: the row's argmax; p and its sums; with top-p, the entries that the choice is among.  In the last one
+// a block a row chooses the token.
 //
 // Top-p needs, twice, the smallest float t with mass_above(t) below a bound, where mass_above(t) is the
 // sum of the entries of p greater than t: first the value at which the kept set ends (bound top_p * Z,
 // strict), then the value in which u falls (bound u * kept mass).  p >= 0, so float order is the order
 // of the bit patterns, and p <= 1 = exp(0), so a pattern has 30 bits.  A search fixes them ten at a
-// time: a stage adds up the mass and the number of the entries in each of the 1,024 bins that the next
-// ten bits cut the present bucket into, and the head of the next stage takes the lowest bin at whose
-// end the bound is met and goes on inside it.  After three levels the bucket is one value.  Both
-// searches start from the same first histogram, so the second has two stages of its own.
+// time: it adds up the mass and the number of the entries in each of the 1,024 bins that the next
+// ten bits cut the present bucket into, takes the lowest bin at whose end the bound is met and goes on inside it.
+// After three levels the bucket is one value.  Both searches start from the same first histogram, which the
+// blocks of the second launch make together.  What the later levels look at are the entries of a few of its bins, an eighth
+// of an octave each: the one in which the kept set ends, and those in which u can fall, as the kept mass lies between the
+// first bound and the end of that bin beyond it.  The third launch lists those entries (of a row of 151,936 some
+// thousands), the row's block has them in registers and does all levels by itself.  A launch a level, of many blocks a row, took 8.6 us for
+// each of the four levels behind the first, most of it launch, trips to memory and atomic additions: 1 / 8 / 16 / 32 / 64
+// rows of 151,936 with top-p 45.1 / 54.4 / 62.0 / 71.7 / 97.6 -> 30.1 / 38.1 / 45.0 / 48.6 / 64.4 us; logits of a third of the spread at
+// temperature 1.5, which list some twenty thousand, 46.8 / 55.2 / 63.7 / 76.4 / 102.8 -> 46.3 / 53.6 / 63.1 / 68.3 / 83.2; rows of
+// nothing but equal entries, which list all, 63 / 87 / 131 / 215 / 381 -> 130 / 141 / 143 / 159 / 220.  What is left is four launches that wait for one another.
 //
 // The entries of a bin share their exponent (it lies in the ten bits that are fixed first), so their
 // sum is 2^exponent times the sum of their 24-bit significands, an integer below 2^42: a bin's mass is
-// kept as that integer.  Integer sums do not depend on their order, so the blocks of a row add into
+// kept as that integer.  Integer sums do not depend on their order, so threads and blocks add into
 // one histogram with atomic additions and the result is the same on every run.
 
 #define SAMPLE_BLOCK 512  // threads of a block that works on a piece of a row
 #define SAMPLE_BINS 1024
-#define SAMPLE_BINS_EACH (SAMPLE_BINS / SAMPLE_BLOCK)  // bins that a thread of the head looks at
 #define SAMPLE_LEVEL_BITS 10
 #define SAMPLE_PIECES_MAX 64  // a wave looks at a row's pieces, a lane at each
-#define SAMPLE_HISTOGRAMS 5   // the cut search's three levels, then levels 1 and 2 of the chosen search
+#define SAMPLE_KEPT 8         // listed entries that a thread of the row's block keeps in registers; further ones are read again at every level
 
 // About 512 blocks of 512 threads in all for top-p, where every piece adds its bins to the row's with atomic additions of
 // its own (64 rows: 98 us, 110 with twice as many; 16 rows 61 and 81; 256 threads and 2,048 blocks 121 and 69), and twice as
@@ -261,97 +267,64 @@ __device__ __forceinline__ int binary_exponent_of(unsigned pattern) {
   return (exponent != 0 ? exponent : 1) - 150;
 }
 
-// What the searches of one row have found so far.  A stage reads what the stage before wrote and
-// writes its own (so that no block reads what another block of the same launch writes).
-struct SampleState {
-  double limit;        // top_p * Z: the bound of the cut search
-  double target;       // u * (kept mass): the bound of the chosen search
-  double above_cut;    // mass above the cut value
-  double kept_at_cut;  // how many of the entries equal to the cut value are kept
-  double above[2];     // per search: mass above the bucket it is in
-  unsigned base[2];    // per search: first pattern of that bucket
-  unsigned cut;        // pattern of the cut value
-  unsigned unused;
-};
-
-struct Picked {
-  int bin;
-  double above;    // mass above the end of that bin
-  unsigned count;  // entries in it
-};
-
-// The lowest of the bins of one level at whose end the mass above (that of the bucket, `above`, and
-// of the bins after it) meets the bound: < limit if strict, else <= limit.  `sums`, `counts`: the
-// row's histogram; `base`: the bucket's first pattern; `level`: which ten bits the bins are.  Every
-// thread of the block calls it (blockDim.x >= SAMPLE_BLOCK); after: SAMPLE_BLOCK / WAVE doubles of LDS.
-__device__ Picked pick_bin(const unsigned long long* __restrict__ sums, const unsigned* __restrict__ counts,
-                           unsigned base, int level, double above, double limit, bool strict, double* after,
-                           int* lowest, double* lowest_above, unsigned* lowest_count) {
-  const int t = threadIdx.x;
-  double mass[SAMPLE_BINS_EACH];
-  unsigned count[SAMPLE_BINS_EACH];
-  double mine = 0.0;
-  __syncthreads();  // whoever read the LDS arrays before is done
-  if (t < SAMPLE_BLOCK) {
+// The mass above the end of each of the 1,024 bins of one level, to `above` (LDS): that of the bucket, `start`, and of the bins
+// after it.  `sums`: the histogram; `base`: the bucket's first pattern.  THREADS threads, a run of bins each; waves: a double of LDS a wave.
+template <int THREADS>
+__device__ void masses_above(const unsigned long long* sums, unsigned base, int level, double start, double* above, double* waves) {
+  constexpr int EACH = SAMPLE_BINS / THREADS;
+  const int t = threadIdx.x, lane = t % WAVE, wave = t / WAVE;
+  double mass[EACH], inclusive = 0.0;
 #pragma unroll
-    for (int j = SAMPLE_BINS_EACH - 1; j >= 0; --j) {
-      const int bin = t * SAMPLE_BINS_EACH + j;
-      const unsigned first = base + ((unsigned)bin << level_shift(level));  // the bin's first pattern
-      mass[j] = ldexp((double)sums[bin], binary_exponent_of(first));
-      count[j] = counts[bin];
-      mine += mass[j];
-    }
+  for (int j = EACH - 1; j >= 0; --j) {
+    const int bin = t * EACH + j;
+    mass[j] = ldexp((double)sums[bin], binary_exponent_of(base + ((unsigned)bin << level_shift(level))));
+    inclusive += mass[j];
   }
-  // the sum of the threads after this one: inside a wave by shuffles, then the waves after it
-  const int lane = t % WAVE, wave = t / WAVE;
-  double inclusive = mine;
 #pragma unroll
   for (int offset = 1; offset < WAVE; offset <<= 1) {
     const double other = __shfl_down(inclusive, offset, WAVE);
     if (lane + offset < WAVE) inclusive += other;
   }
   const double after_in_wave = __shfl_down(inclusive, 1, WAVE);
-  if (t < SAMPLE_BLOCK && lane == 0) after[wave] = inclusive;
-  if (t == 0) *lowest = SAMPLE_BINS;
+  __syncthreads();  // whoever read the LDS arrays before is done
+  if (lane == 0) waves[wave] = inclusive;
   __syncthreads();
-  double after_mine = lane == WAVE - 1 ? 0.0 : after_in_wave;
-  if (t < SAMPLE_BLOCK)
-    for (int w = SAMPLE_BLOCK / WAVE - 1; w > wave; --w) after_mine += after[w];
-  int my_bin = SAMPLE_BINS;
-  double my_above = 0.0;
-  unsigned my_count = 0;
-  if (t < SAMPLE_BLOCK) {
-    double later = after_mine;  // mass of the bins after the one looked at
+  double later = lane == WAVE - 1 ? 0.0 : after_in_wave;
+  for (int w = THREADS / WAVE - 1; w > wave; --w) later += waves[w];
 #pragma unroll
-    for (int j = SAMPLE_BINS_EACH - 1; j >= 0; --j) {
-      const double m = above + later;
-      if (strict ? m < limit : m <= limit) {
-        my_bin = t * SAMPLE_BINS_EACH + j;
-        my_above = m;
-        my_count = count[j];
-      }
-      later += mass[j];
-    }
-    if (my_bin < SAMPLE_BINS) atomicMin(lowest, my_bin);
+  for (int j = EACH - 1; j >= 0; --j) {
+    above[t * EACH + j] = start + later;
+    later += mass[j];
   }
-  __syncthreads();
-  if (my_bin < SAMPLE_BINS && my_bin == *lowest) {
-    *lowest_above = my_above;
-    *lowest_count = my_count;
-  }
-  __syncthreads();
-  Picked picked;
-  picked.bin = *lowest;
-  if (picked.bin == SAMPLE_BINS) {  // the bound is met nowhere (it cannot be: nothing lies above the maximum)
-    picked.bin = SAMPLE_BINS - 1;
-    picked.above = above;
-    picked.count = 0;
-    return picked;
-  }
-  picked.above = *lowest_above;
-  picked.count = *lowest_count;
-  return picked;
 }
+
+// The lowest bin at whose end the bound is met (mass above < limit if strict, else <= limit); the last one if it is nowhere (it
+// cannot be: nothing lies above the maximum).  Every thread asks for its own run of `above`; *lowest is LDS, and nobody reads it any more.
+template <int THREADS>
+__device__ __forceinline__ int lowest_bin(const double* above, double limit, bool strict, int* lowest) {
+  constexpr int EACH = SAMPLE_BINS / THREADS;
+  if (threadIdx.x == 0) *lowest = SAMPLE_BINS - 1;
+  __syncthreads();
+  int mine = SAMPLE_BINS;
+#pragma unroll
+  for (int j = EACH - 1; j >= 0; --j) {
+    const double m = above[threadIdx.x * EACH + j];
+    if (strict ? m < limit : m <= limit) mine = (int)threadIdx.x * EACH + j;
+  }
+  const unsigned long long met = __ballot(mine < SAMPLE_BINS);  // (the first lane of a wave that meets it has the wave's lowest bin)
+  if (met != 0ull && (int)threadIdx.x % WAVE == __ffsll((long long)met) - 1) atomicMin(lowest, mine);
+  __syncthreads();
+  return *lowest;
+}
+
+// Which bins of the first histogram a row's choice is among, and the bound at which its kept set ends.
+struct Candidates {
+  double limit;                     // top_p * Z
+  int cut_bin, first_bin, last_bin;  // the kept set ends in the first of them, u falls in one of the run between the others
+  __device__ __forceinline__ bool has(unsigned bin) const {
+    return bin == (unsigned)cut_bin || (bin >= (unsigned)first_bin && bin <= (unsigned)last_bin);
+  }
+};
 
 __device__ __forceinline__ void clear_histogram(unsigned long long* lds_sums, unsigned* lds_counts) {
   for (int i = threadIdx.x; i < SAMPLE_BINS; i += blockDim.x) {
@@ -361,9 +334,7 @@ __device__ __forceinline__ void clear_histogram(unsigned long long* lds_sums, un
 }
 
 // A piece's entries are taken in batches, all loads of a batch under way together: a thread of 256 had ten entries of a row of
-// 151,936 in 64 pieces, and a loop that asks for one, waits, and adds it paid ten trips to memory one after the other; and
-// the first batch of a search's stage is asked for before its head (1 / 8 / 16 / 32 / 64 rows of 151,936 with top-p: 51.6 / 55.1 /
-// 71.4 / 96.9 / 126 -> 42.8 / 53.7 / 60.6 / 72.6 / 97.7 us with the blocks of `sample_pieces`).
+// 151,936 in 64 pieces, and a loop that asks for one, waits, and adds it paid ten trips to memory one after the other.
 #define SAMPLE_BATCH 6
 struct Batch {
   float v[SAMPLE_BATCH];
@@ -390,27 +361,25 @@ __device__ __forceinline__ void add_entry(float value, unsigned bucket, int shif
 
 // Adds what the block has gathered of its piece to the row's histogram (a barrier before).
 __device__ __forceinline__ void give_histogram(const unsigned long long* lds_sums, const unsigned* lds_counts,
-                                               unsigned long long* __restrict__ sums, unsigned* __restrict__ counts,
-                                               unsigned* __restrict__ piece_counts) {
+                                               unsigned long long* __restrict__ sums, unsigned* __restrict__ counts) {
   for (int bin = threadIdx.x; bin < SAMPLE_BINS; bin += blockDim.x) {
     const unsigned count = lds_counts[bin];
     if (count != 0u) {
       atomicAdd(sums + bin, lds_sums[bin]);
       atomicAdd(counts + bin, count);
     }
-    if (piece_counts != nullptr) piece_counts[bin] = count;
   }
 }
 
-// The layout of what the stages share, per row: SAMPLE_HISTOGRAMS histograms (cleared by the first
-// launch), the entries of each piece in every bin of the two last levels, the states.
+// The layout of what the launches share, per row: the first histogram (cleared by the first launch), p and its pieces' sums.
 struct SampleBuffers {
   float* p;                     // [rows, vocab]
   double* piece_sums;           // [rows, pieces]
-  unsigned long long* sums;     // [SAMPLE_HISTOGRAMS, rows, SAMPLE_BINS]
-  unsigned* counts;             // [SAMPLE_HISTOGRAMS, rows, SAMPLE_BINS]
-  unsigned* piece_counts;       // [2, rows, pieces, SAMPLE_BINS]: of the last level of the cut search, of the chosen search
-  SampleState* states;          // [SAMPLE_HISTOGRAMS, rows]
+  unsigned long long* sums;     // [rows, SAMPLE_BINS]
+  unsigned* counts;             // [rows, SAMPLE_BINS]
+  unsigned* listed;             // [rows]: how many entries are listed (cleared by the first launch)
+  uint2* list;                  // [rows, vocab]: pattern and index of each, in no order
+  Candidates* candidates;       // [rows]
   const float* piece_values;    // [rows, argmax_pieces]
   const int* piece_indices;
 };
@@ -461,97 +430,7 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_exp_kernel(const float* _
   const double sum = block_sum_f64(partial, sd);  // (its barriers stand between the additions and what reads them)
   if (threadIdx.x == 0) buffers.piece_sums[r * pieces + piece] = sum;
   if (!with_histogram) return;
-  give_histogram(lds_sums, lds_counts, buffers.sums + (size_t)r * SAMPLE_BINS, buffers.counts + (size_t)r * SAMPLE_BINS, nullptr);
-}
-
-// One stage of the two searches of the rows with top-p.  stage 1, 2: levels 1, 2 of the cut search;
-// 3, 4: levels 1, 2 of the chosen search.  The head takes from the histogram of the stage before the
-// bucket to go on in (stage 3: the cut value from the histogram of stage 2, what is kept, and the
-// chosen search's first bucket from the first histogram); the body adds up this piece's entries
-// inside that bucket into histogram `stage`.
-__global__ __launch_bounds__(SAMPLE_BLOCK) void sample_level_kernel(const float* __restrict__ temperatures,
-                                                                    const float* __restrict__ top_ps,
-                                                                    const float* __restrict__ uniforms,
-                                                                    SampleBuffers buffers, int rows, int vocab,
-                                                                    int pieces, int stage) {
-  __shared__ double after[SAMPLE_BLOCK / WAVE];
-  __shared__ int lowest;
-  __shared__ double lowest_above;
-  __shared__ unsigned lowest_count;
-  __shared__ unsigned long long lds_sums[SAMPLE_BINS];
-  __shared__ unsigned lds_counts[SAMPLE_BINS];
-  const int r = blockIdx.x, piece = blockIdx.y;
-  const float top_p = top_ps[r];
-  if (temperatures[r] <= 0.f || top_p >= 1.f) return;
-  clear_histogram(lds_sums, lds_counts);  // the head's barriers lie between this and the additions
-  const int per = (vocab + pieces - 1) / pieces;
-  const int begin = min(vocab, piece * per), end = min(vocab, begin + per);
-  const float* p = buffers.p + (size_t)r * vocab;
-  Batch batch = load_batch(p, begin + threadIdx.x, end);  // under way while the head works
-  const size_t per_histogram = (size_t)rows * SAMPLE_BINS, of_row = (size_t)r * SAMPLE_BINS;
-  const int search = stage <= 2 ? 0 : 1, level = stage <= 2 ? stage : stage - 2;
-
-  SampleState st;
-  if (stage == 1) {
-    __shared__ double sums_here[SAMPLE_PIECES_MAX];  // a thread a piece asks, then everybody adds them in order
-    if ((int)threadIdx.x < pieces) sums_here[threadIdx.x] = buffers.piece_sums[r * pieces + threadIdx.x];
-    __syncthreads();
-    double total = 0.0;
-    for (int q = 0; q < pieces; ++q) total += sums_here[q];
-    // the bound is strict, so a bound of 0 would be met nowhere: the least positive one keeps the maximum alone
-    st.limit = fmax((double)top_p * total, 2.2250738585072014e-308);
-    st.target = st.above_cut = st.kept_at_cut = st.above[0] = st.above[1] = 0.0;
-    st.base[0] = st.base[1] = st.cut = st.unused = 0u;
-  } else {
-    st = buffers.states[(size_t)(stage - 1) * rows + r];
-  }
-  if (stage <= 2) {  // one more level of the cut search
-    const size_t at = (size_t)(stage - 1) * per_histogram + of_row;
-    const Picked got = pick_bin(buffers.sums + at, buffers.counts + at, st.base[0], stage - 1, st.above[0], st.limit,
-                                true, after, &lowest, &lowest_above, &lowest_count);
-    st.base[0] += (unsigned)got.bin << level_shift(stage - 1);
-    st.above[0] = got.above;
-  } else if (stage == 3) {
-    // the cut value: everything above it is kept, and of the entries equal to it as many as still
-    // start below the bound (engine.py:34-37)
-    size_t at = (size_t)2 * per_histogram + of_row;
-    Picked got = pick_bin(buffers.sums + at, buffers.counts + at, st.base[0], 2, st.above[0], st.limit, true, after,
-                          &lowest, &lowest_above, &lowest_count);
-    st.cut = st.base[0] + (unsigned)got.bin;
-    st.above_cut = got.above;
-    const double cut_value = (double)__uint_as_float(st.cut), count_at_cut = (double)got.count;
-    double kept_at_cut = count_at_cut;
-    if (cut_value > 0.0) kept_at_cut = fmin(count_at_cut, ceil((st.limit - st.above_cut) / cut_value));
-    if (kept_at_cut < 1.0) kept_at_cut = 1.0;
-    st.kept_at_cut = kept_at_cut;
-    st.target = (double)uniforms[r] * (st.above_cut + kept_at_cut * cut_value);
-    // the chosen value: the smallest one whose preceding mass is <= target
-    got = pick_bin(buffers.sums + of_row, buffers.counts + of_row, 0u, 0, 0.0, st.target, false, after, &lowest,
-                   &lowest_above, &lowest_count);
-    st.base[1] = (unsigned)got.bin << level_shift(0);
-    st.above[1] = got.above;
-  } else {
-    const size_t at = (size_t)3 * per_histogram + of_row;
-    const Picked got = pick_bin(buffers.sums + at, buffers.counts + at, st.base[1], 1, st.above[1], st.target, false,
-                                after, &lowest, &lowest_above, &lowest_count);
-    st.base[1] += (unsigned)got.bin << level_shift(1);
-    st.above[1] = got.above;
-  }
-  if (piece == 0 && threadIdx.x == 0) buffers.states[(size_t)stage * rows + r] = st;
-
-  unsigned* piece_counts = nullptr;  // the last level: the final stage asks which piece holds the entry
-  if (level == 2) piece_counts = buffers.piece_counts + (((size_t)search * rows + r) * pieces + piece) * SAMPLE_BINS;
-  const size_t to = (size_t)stage * per_histogram + of_row;
-  const int shift = level_shift(level);
-  const unsigned bucket = st.base[search] >> (shift + SAMPLE_LEVEL_BITS);
-  for (int first = begin + threadIdx.x; first < end; first += SAMPLE_BATCH * SAMPLE_BLOCK) {
-    if (first != begin + (int)threadIdx.x) batch = load_batch(p, first, end);
-#pragma unroll
-    for (int u = 0; u < SAMPLE_BATCH; ++u)
-      if (first + u * SAMPLE_BLOCK < end) add_entry(batch.v[u], bucket, shift, lds_sums, lds_counts);
-  }
-  __syncthreads();
-  give_histogram(lds_sums, lds_counts, buffers.sums + to, buffers.counts + to, piece_counts);
+  give_histogram(lds_sums, lds_counts, buffers.sums + (size_t)r * SAMPLE_BINS, buffers.counts + (size_t)r * SAMPLE_BINS);
 }
 
 // Sums of v over the threads before this one, in thread order.  shared: at least 16 of its kind.
@@ -588,21 +467,222 @@ __device__ __forceinline__ int block_sum_before_int(int v, int* shared) {
   return before + inclusive - v;
 }
 
-// The token of every row with a temperature: one block per row.  `out` holds the argmax already.
+// Lists the entries that the choice of a row with top-p is among: a block takes its piece's.
+__global__ __launch_bounds__(SAMPLE_BLOCK) void sample_list_kernel(const float* __restrict__ temperatures, const float* __restrict__ top_ps,
+                                                                   const float* __restrict__ uniforms, SampleBuffers buffers, int vocab,
+                                                                   int pieces) {
+  __shared__ double above[SAMPLE_BINS], waves[SAMPLE_BLOCK / WAVE], sums_here[SAMPLE_PIECES_MAX];
+  __shared__ int lowest;
+  __shared__ unsigned found, place;
+  const int r = blockIdx.x, piece = blockIdx.y, t = threadIdx.x;
+  const float top_p = top_ps[r];
+  if (temperatures[r] <= 0.f || top_p >= 1.f) return;
+  const int per = (vocab + pieces - 1) / pieces;
+  const int begin = min(vocab, piece * per), end = min(vocab, begin + per);
+  const float* p = buffers.p + (size_t)r * vocab;
+  Batch batch = load_batch(p, begin + t, end);  // under way while the histogram is looked at
+  if (t < pieces) sums_here[t] = buffers.piece_sums[r * pieces + t];  // a thread a piece asks, then everybody adds them in order
+  if (t == 0) found = 0u;
+  masses_above<SAMPLE_BLOCK>(buffers.sums + (size_t)r * SAMPLE_BINS, 0u, 0, 0.0, above, waves);
+  double total = 0.0;
+  for (int q = 0; q < pieces; ++q) total += sums_here[q];
+  Candidates c;
+  // the bound is strict, so a bound of 0 would be met nowhere: the least positive one keeps the maximum alone
+  c.limit = fmax((double)top_p * total, 2.2250738585072014e-308);
+  c.cut_bin = lowest_bin<SAMPLE_BLOCK>(above, c.limit, true, &lowest);
+  // the kept mass is at least the bound, and beyond it by less than a value of that bin (up to rounding, which the row's block sees to)
+  const double end_of_bin = (double)__uint_as_float((unsigned)(c.cut_bin + 1) << level_shift(0)), u = (double)uniforms[r];
+  __syncthreads();
+  c.first_bin = lowest_bin<SAMPLE_BLOCK>(above, u * (c.limit + end_of_bin), false, &lowest);
+  __syncthreads();
+  c.last_bin = lowest_bin<SAMPLE_BLOCK>(above, u * c.limit, false, &lowest);
+  if (piece == 0 && t == 0) buffers.candidates[r] = c;
+  // count them, ask for a place in the row's list, and write them there
+  auto taken = [&](int i, float v) { return i < end && c.has(__float_as_uint(v) >> level_shift(0)); };
+  unsigned mine = 0u;
+  for (int first = begin + t; first < end; first += SAMPLE_BATCH * SAMPLE_BLOCK) {
+    if (first != begin + t) batch = load_batch(p, first, end);
+#pragma unroll
+    for (int k = 0; k < SAMPLE_BATCH; ++k) mine += taken(first + k * SAMPLE_BLOCK, batch.v[k]) ? 1u : 0u;
+  }
+  if (mine != 0u) mine = atomicAdd(&found, mine);  // (where this thread's begin)
+  __syncthreads();
+  if (found == 0u) return;
+  if (t == 0) place = atomicAdd(buffers.listed + r, found);
+  __syncthreads();
+  uint2* list = buffers.list + (size_t)r * vocab + place;
+  const bool again = begin + SAMPLE_BATCH * SAMPLE_BLOCK < end;  // more than one batch: the first is not here any more
+  for (int first = begin + t; first < end; first += SAMPLE_BATCH * SAMPLE_BLOCK) {
+    if (again) batch = load_batch(p, first, end);
+#pragma unroll
+    for (int k = 0; k < SAMPLE_BATCH; ++k) {
+      const int i = first + k * SAMPLE_BLOCK;
+      if (taken(i, batch.v[k])) list[mine++] = make_uint2(__float_as_uint(batch.v[k]), (unsigned)i);
+    }
+  }
+}
+
+// The token of a row with top-p (out holds the argmax already), by the row's block; see the head of this section.
+__device__ void sample_top_p(const SampleBuffers& buffers, int r, float uniform, int vocab, int* __restrict__ out) {
+  __shared__ double above[SAMPLE_BINS], first_above[SAMPLE_BINS], waves[SAMPLE_THREADS / WAVE];
+  __shared__ unsigned long long sums[SAMPLE_BINS];
+  __shared__ unsigned counts[SAMPLE_BINS];
+  __shared__ int lowest, before_lowest, scan[17];
+  const int t = threadIdx.x, lane = t % WAVE;
+  const float* p = buffers.p + (size_t)r * vocab;
+  const uint2* list = buffers.list + (size_t)r * vocab;
+  const int n = (int)buffers.listed[r];
+  const Candidates c = buffers.candidates[r];
+  uint2 kept[SAMPLE_KEPT];
+#pragma unroll
+  for (int k = 0; k < SAMPLE_KEPT; ++k) kept[k] = t + k * SAMPLE_THREADS < n ? list[t + k * SAMPLE_THREADS] : make_uint2(~0u, 0u);
+  masses_above<SAMPLE_THREADS>(buffers.sums + (size_t)r * SAMPLE_BINS, 0u, 0, 0.0, first_above, waves);
+  bool listed = true;  // whether the entries that a search looks at are in the list
+  // calls f(pattern, index) for every entry, of the list (and for none, whose pattern is no entry's) or of the row
+  auto each = [&](auto f) {
+    if (listed) {
+#pragma unroll
+      for (int k = 0; k < SAMPLE_KEPT; ++k) f(kept[k].x, (int)kept[k].y);
+      for (int first = t + SAMPLE_KEPT * SAMPLE_THREADS; first < n; first += SAMPLE_KEPT * SAMPLE_THREADS) {
+        uint2 more[SAMPLE_KEPT];
+#pragma unroll
+        for (int k = 0; k < SAMPLE_KEPT; ++k) more[k] = list[min(first + k * SAMPLE_THREADS, n - 1)];
+#pragma unroll
+        for (int k = 0; k < SAMPLE_KEPT; ++k) f(first + k * SAMPLE_THREADS < n ? more[k].x : ~0u, (int)more[k].y);
+      }
+    } else {
+      for (int first = t; first < vocab; first += SAMPLE_KEPT * SAMPLE_THREADS) {
+        float more[SAMPLE_KEPT];
+#pragma unroll
+        for (int k = 0; k < SAMPLE_KEPT; ++k) more[k] = p[min(first + k * SAMPLE_THREADS, vocab - 1)];
+#pragma unroll
+        for (int k = 0; k < SAMPLE_KEPT; ++k)
+          f(first + k * SAMPLE_THREADS < vocab ? __float_as_uint(more[k]) : ~0u, first + k * SAMPLE_THREADS);
+      }
+    }
+  };
+  // levels 1 and 2 of a search, inside the bucket of the first level that begins at `base`, `mass` above it: the value's pattern, and the mass above it
+  auto searched = [&](unsigned base, double& mass, double bound, bool strict) {
+    for (int level = 1; level <= 2; ++level) {
+      __syncthreads();
+      sums[t] = 0ull;
+      counts[t] = 0u;
+      __syncthreads();
+      const int shift = level_shift(level);
+      const unsigned bucket = base >> (shift + SAMPLE_LEVEL_BITS);
+      each([&](unsigned pattern, int) {
+        if ((pattern >> (shift + SAMPLE_LEVEL_BITS)) != bucket) return;
+        const unsigned bin = (pattern >> shift) & (SAMPLE_BINS - 1);
+        // (equal entries of a wave go together: additions to one place wait for one another)
+        const unsigned long long here = __ballot(1), same = __ballot(pattern == (unsigned)__builtin_amdgcn_readfirstlane((int)pattern));
+        if (same == here) {
+          if (lane == __ffsll((long long)here) - 1) {
+            atomicAdd(sums + bin, significand_of(pattern) * (unsigned long long)__popcll(here));
+            atomicAdd(counts + bin, (unsigned)__popcll(here));
+          }
+          return;
+        }
+        atomicAdd(sums + bin, significand_of(pattern));
+        atomicAdd(counts + bin, 1u);
+      });
+      __syncthreads();
+      masses_above<SAMPLE_THREADS>(sums, base, level, mass, above, waves);
+      const int bin = lowest_bin<SAMPLE_THREADS>(above, bound, strict, &lowest);
+      mass = above[bin];
+      base += (unsigned)bin << shift;
+    }
+    return base;
+  };
+  // the cut value: everything above it is kept, and of the entries equal to it as many as still
+  // start below the bound (engine.py:34-37)
+  __syncthreads();
+  double above_cut = first_above[c.cut_bin];
+  // (a long list may be of one value over and over, as of a row of equal entries: nothing is left to search then)
+  bool one_value = n > SAMPLE_KEPT * SAMPLE_THREADS;
+  if (one_value) {
+    unsigned least = ~0u, most = 0u;
+    each([&](unsigned pattern, int) {
+      least = min(least, pattern);
+      most = max(most, pattern == ~0u ? 0u : pattern);
+    });
+    if (t < 2) counts[t] = t == 0 ? ~0u : 0u;
+    __syncthreads();
+    atomicMin(counts, least);
+    atomicMax(counts + 1, most);
+    __syncthreads();
+    one_value = counts[0] == counts[1] && (counts[0] >> level_shift(0)) == (unsigned)c.cut_bin;
+  }
+  const unsigned cut = one_value ? counts[0] : searched((unsigned)c.cut_bin << level_shift(0), above_cut, c.limit, true);
+  const unsigned equal_at_cut = one_value ? (unsigned)n : counts[cut & (SAMPLE_BINS - 1)];
+  const double cut_value = (double)__uint_as_float(cut), count_at_cut = (double)equal_at_cut;
+  double kept_at_cut = count_at_cut;
+  if (cut_value > 0.0) kept_at_cut = fmin(count_at_cut, ceil((c.limit - above_cut) / cut_value));
+  if (kept_at_cut < 1.0) kept_at_cut = 1.0;
+  const double target = (double)uniform * (above_cut + kept_at_cut * cut_value);
+  // the chosen value: the smallest one whose preceding mass is <= target
+  __syncthreads();
+  const int chosen_bin = lowest_bin<SAMPLE_THREADS>(first_above, target, false, &lowest);
+  listed = c.has((unsigned)chosen_bin);
+  double above_chosen = first_above[chosen_bin];
+  const bool at_cut = one_value && chosen_bin == c.cut_bin;
+  unsigned chosen = at_cut ? cut : searched((unsigned)chosen_bin << level_shift(0), above_chosen, target, false);
+  unsigned equal = at_cut ? equal_at_cut : counts[chosen & (SAMPLE_BINS - 1)];
+  if (chosen < cut) {  // never below the cut
+    chosen = cut;
+    above_chosen = above_cut;
+    equal = equal_at_cut;
+    listed = true;
+  }
+  if (equal == 0u) return;  // no entry has the chosen value: the argmax stands
+  const double chosen_value = (double)__uint_as_float(chosen);
+  double which = chosen_value > 0.0 ? floor((target - above_chosen) / chosen_value) : 0.0;
+  if (which < 0.0) which = 0.0;
+  if (chosen == cut && which > kept_at_cut - 1.0) which = kept_at_cut - 1.0;
+  // rounding may put the target past the last equal entry: then that one
+  int rank = which > (double)(equal - 1) ? (int)equal - 1 : (int)which;
+  if (equal == 1u) {
+    each([&](unsigned pattern, int index) {
+      if (pattern == chosen) *out = index;
+    });
+    return;
+  }
+  // the entry of that rank among the equal ones in index order: their indices ten bits at a time, from the highest
+  int shift = 0, prefix = 0;
+  while (shift + SAMPLE_LEVEL_BITS < 31 && (vocab - 1) >> (shift + SAMPLE_LEVEL_BITS) != 0) shift += SAMPLE_LEVEL_BITS;
+  for (; shift >= 0; shift -= SAMPLE_LEVEL_BITS) {
+    __syncthreads();
+    counts[t] = 0u;
+    __syncthreads();
+    each([&](unsigned pattern, int index) {
+      if (pattern != chosen || (shift + SAMPLE_LEVEL_BITS < 31 && index >> (shift + SAMPLE_LEVEL_BITS) != prefix)) return;
+      const int bin = (index >> shift) & (SAMPLE_BINS - 1);
+      const unsigned long long here = __ballot(1), same = __ballot(bin == __builtin_amdgcn_readfirstlane(bin));
+      if (same != here) atomicAdd(counts + bin, 1u);
+      else if (lane == __ffsll((long long)here) - 1) atomicAdd(counts + bin, (unsigned)__popcll(here));
+    });
+    __syncthreads();
+    const int here = (int)counts[t], before = block_sum_before_int(here, scan);
+    if (before <= rank && rank < before + here) {  // one thread
+      lowest = t;
+      before_lowest = before;
+    }
+    __syncthreads();
+    prefix = (prefix << SAMPLE_LEVEL_BITS) | lowest;
+    rank -= before_lowest;
+  }
+  if (t == 0) *out = prefix;
+}
+
+// The token of every row with a temperature: one block per row.  `out` holds the argmax already.  WITH_TOP_P: rows may have top_p < 1.
+template <bool WITH_TOP_P>
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(const float* __restrict__ temperatures,
                                                                      const float* __restrict__ top_ps,
                                                                      const float* __restrict__ uniforms,
                                                                      SampleBuffers buffers, int* __restrict__ out,
-                                                                     int rows, int vocab, int pieces, int with_top_p) {
-  __shared__ double after[SAMPLE_BLOCK / WAVE];
-  __shared__ int lowest;
-  __shared__ double lowest_above;
-  __shared__ unsigned lowest_count;
+                                                                     int vocab, int pieces) {
   __shared__ double sd[17];
-  __shared__ int si[17];
   __shared__ int owner_piece, owner_thread;
   __shared__ double before_piece, shared_target;
-  __shared__ int wanted;  // which of the entries equal to the chosen value, counted inside the owner piece
   const int r = blockIdx.x;
   if (temperatures[r] <= 0.f) return;  // engine.py:30-31
   const float* p = buffers.p + (size_t)r * vocab;
@@ -610,132 +690,78 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(const float
   const int per_piece = (vocab + pieces - 1) / pieces;
   const int lane = threadIdx.x % WAVE;
 
-  if (top_p >= 1.f || !with_top_p) {
-    // inverse CDF in index order: the piece first, from the pieces' sums, then inside it
-    if (threadIdx.x == 0) owner_thread = 0x7fffffff;
-    if (threadIdx.x < WAVE) {  // a lane per piece
-      const double sum = lane < pieces ? buffers.piece_sums[r * pieces + lane] : 0.0;
-      double inclusive = sum;
-#pragma unroll
-      for (int offset = 1; offset < WAVE; offset <<= 1) {
-        const double other = __shfl_up(inclusive, offset, WAVE);
-        if (lane >= offset) inclusive += other;
-      }
-      const double total = __shfl(inclusive, WAVE - 1, WAVE);
-      const double target = (double)uniforms[r] * total;
-      const double from_below = __shfl_up(inclusive, 1, WAVE);  // every lane takes part in it
-      const double before = lane == 0 ? 0.0 : from_below;
-      const unsigned long long holds = __ballot(lane < pieces && before + sum > target);
-      const int owner = holds != 0ull ? __ffsll((long long)holds) - 1 : -1;
-      if (lane == (owner < 0 ? 0 : owner)) {
-        owner_piece = owner;
-        before_piece = before;
-        shared_target = target;
-      }
-    }
-    __syncthreads();
-    if (owner_piece < 0) {
-      if (threadIdx.x == 0) out[r] = vocab - 1;
-      return;
-    }
-    const double target = shared_target;
-    const int begin = min(vocab, owner_piece * per_piece), end = min(vocab, begin + per_piece);
-    const int per = (end - begin + blockDim.x - 1) / blockDim.x;  // each thread owns a contiguous run
-    const int b = min(end, begin + (int)threadIdx.x * per), e = min(end, b + per);
-    double mine = 0.0;
-    for (int i = b; i < e; ++i) mine += (double)p[i];
-    const double before = before_piece + block_sum_before_f64(mine, sd);
-    if (before + mine > target) atomicMin(&owner_thread, (int)threadIdx.x);
-    __syncthreads();
-    if (owner_thread == 0x7fffffff) {  // rounding put the target past the piece's end
-      if (threadIdx.x == 0) out[r] = end - 1;
-    } else if ((int)threadIdx.x == owner_thread) {
-      double running = before;
-      int found = e - 1;
-      for (int i = b; i < e; ++i) {
-        running += (double)p[i];
-        if (running > target) { found = i; break; }
-      }
-      out[r] = found;
-    }
+  if (WITH_TOP_P && !(top_p >= 1.f)) {
+    sample_top_p(buffers, r, uniforms[r], vocab, out + r);
     return;
   }
-
-  // top-p: the chosen search's last level, then the entry among the equal ones, in index order
-  const size_t per_histogram = (size_t)rows * SAMPLE_BINS, of_row = (size_t)r * SAMPLE_BINS;
-  const SampleState st = buffers.states[(size_t)(SAMPLE_HISTOGRAMS - 1) * rows + r];
-  const size_t at = (size_t)(SAMPLE_HISTOGRAMS - 1) * per_histogram + of_row;
-  const Picked got = pick_bin(buffers.sums + at, buffers.counts + at, st.base[1], 2, st.above[1], st.target, false,
-                              after, &lowest, &lowest_above, &lowest_count);
-  unsigned chosen = st.base[1] + (unsigned)got.bin;
-  double above_chosen = got.above;
-  int search = 1;
-  if (chosen < st.cut) {  // never below the cut
-    chosen = st.cut;
-    above_chosen = st.above_cut;
-    search = 0;
-  }
-  // how many entries of each piece equal the chosen value: the last level of that search has counted them
-  const unsigned* equal_in = buffers.piece_counts + ((size_t)search * rows + r) * pieces * SAMPLE_BINS + (chosen & (SAMPLE_BINS - 1));
+  // inverse CDF in index order: the piece first, from the pieces' sums, then inside it
+  if (threadIdx.x == 0) owner_thread = 0x7fffffff;
   if (threadIdx.x < WAVE) {  // a lane per piece
-    const int here = lane < pieces ? (int)equal_in[(size_t)lane * SAMPLE_BINS] : 0;
-    int inclusive = here;
+    const double sum = lane < pieces ? buffers.piece_sums[r * pieces + lane] : 0.0;
+    double inclusive = sum;
 #pragma unroll
     for (int offset = 1; offset < WAVE; offset <<= 1) {
-      const int other = __shfl_up(inclusive, offset, WAVE);
+      const double other = __shfl_up(inclusive, offset, WAVE);
       if (lane >= offset) inclusive += other;
     }
-    const int equal = __shfl(inclusive, WAVE - 1, WAVE);
-    const double chosen_value = (double)__uint_as_float(chosen);
-    double which = chosen_value > 0.0 ? floor((st.target - above_chosen) / chosen_value) : 0.0;
-    if (which < 0.0) which = 0.0;
-    if (chosen == st.cut && which > st.kept_at_cut - 1.0) which = st.kept_at_cut - 1.0;
-    // rounding may put the target past the last equal entry: then that one
-    const int index = which > (double)(equal - 1) ? equal - 1 : (int)which;
-    const int before = inclusive - here;
-    const unsigned long long holds = __ballot(equal > 0 && before <= index && index < inclusive);
+    const double total = __shfl(inclusive, WAVE - 1, WAVE);
+    const double target = (double)uniforms[r] * total;
+    const double from_below = __shfl_up(inclusive, 1, WAVE);  // every lane takes part in it
+    const double before = lane == 0 ? 0.0 : from_below;
+    const unsigned long long holds = __ballot(lane < pieces && before + sum > target);
     const int owner = holds != 0ull ? __ffsll((long long)holds) - 1 : -1;
     if (lane == (owner < 0 ? 0 : owner)) {
       owner_piece = owner;
-      wanted = index - before;
+      before_piece = before;
+      shared_target = target;
     }
   }
   __syncthreads();
-  if (owner_piece < 0) return;  // no entry has the chosen value: the argmax stands
+  if (owner_piece < 0) {
+    if (threadIdx.x == 0) out[r] = vocab - 1;
+    return;
+  }
+  const double target = shared_target;
   const int begin = min(vocab, owner_piece * per_piece), end = min(vocab, begin + per_piece);
-  const int per = (end - begin + blockDim.x - 1) / blockDim.x;
+  const int per = (end - begin + blockDim.x - 1) / blockDim.x;  // each thread owns a contiguous run
   const int b = min(end, begin + (int)threadIdx.x * per), e = min(end, b + per);
-  int mine = 0;
-  for (int i = b; i < e; ++i) mine += __float_as_uint(p[i]) == chosen ? 1 : 0;
-  const int before = block_sum_before_int(mine, si);
-  if (before <= wanted && wanted < before + mine) {
-    int seen = before;
-    for (int i = b; i < e; ++i)
-      if (__float_as_uint(p[i]) == chosen) {
-        if (seen == wanted) { out[r] = i; break; }
-        ++seen;
-      }
+  double mine = 0.0;
+  for (int i = b; i < e; ++i) mine += (double)p[i];
+  const double before = before_piece + block_sum_before_f64(mine, sd);
+  if (before + mine > target) atomicMin(&owner_thread, (int)threadIdx.x);
+  __syncthreads();
+  if (owner_thread == 0x7fffffff) {  // rounding put the target past the piece's end
+    if (threadIdx.x == 0) out[r] = end - 1;
+  } else if ((int)threadIdx.x == owner_thread) {
+    double running = before;
+    int found = e - 1;
+    for (int i = b; i < e; ++i) {
+      running += (double)p[i];
+      if (running > target) { found = i; break; }
+    }
+    out[r] = found;
   }
 }
 
 static size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
 struct SampleWorkspace {
-  size_t sums, counts, cleared_words;  // the histograms come first: the first launch clears them
-  size_t p, piece_sums, piece_counts, states, piece_values, piece_indices, bytes;
+  size_t sums, counts, listed, cleared_words;  // these come first: the first launch clears them
+  size_t p, piece_sums, list, candidates, piece_values, piece_indices, bytes;
 };
 
 static SampleWorkspace sample_workspace(int rows, int vocab) {
-  const size_t pieces = sample_pieces(rows, false), bins = (size_t)SAMPLE_HISTOGRAMS * rows * SAMPLE_BINS;
+  const size_t pieces = sample_pieces(rows, false), bins = (size_t)rows * SAMPLE_BINS;
   SampleWorkspace w;
   size_t at = 0;
   w.sums = at, at += rounded(bins * sizeof(unsigned long long));
   w.counts = at, at += rounded(bins * sizeof(unsigned));
+  w.listed = at, at += rounded((size_t)rows * sizeof(unsigned));
   w.cleared_words = at / sizeof(unsigned);
   w.p = at, at += rounded((size_t)rows * vocab * sizeof(float));
   w.piece_sums = at, at += rounded((size_t)rows * pieces * sizeof(double));
-  w.piece_counts = at, at += rounded((size_t)2 * rows * pieces * SAMPLE_BINS * sizeof(unsigned));
-  w.states = at, at += rounded((size_t)SAMPLE_HISTOGRAMS * rows * sizeof(SampleState));
+  w.list = at, at += rounded((size_t)rows * vocab * sizeof(uint2));
+  w.candidates = at, at += rounded((size_t)rows * sizeof(Candidates));
   w.piece_values = at, at += rounded((size_t)rows * ARGMAX_PIECES * sizeof(float));
   w.piece_indices = at, at += rounded((size_t)rows * ARGMAX_PIECES * sizeof(int));
   w.bytes = at;
@@ -766,8 +792,9 @@ extern "C" int llmserve_sample(const float* logits, const float* temperatures, c
   buffers.piece_sums = (double*)(base + w.piece_sums);
   buffers.sums = (unsigned long long*)(base + w.sums);
   buffers.counts = (unsigned*)(base + w.counts);
-  buffers.piece_counts = (unsigned*)(base + w.piece_counts);
-  buffers.states = (SampleState*)(base + w.states);
+  buffers.listed = (unsigned*)(base + w.listed);
+  buffers.list = (uint2*)(base + w.list);
+  buffers.candidates = (Candidates*)(base + w.candidates);
   buffers.piece_values = piece_values;
   buffers.piece_indices = piece_indices;
   const int first_pieces = argmax_pieces(rows), pieces = sample_pieces(rows, with_top_p != 0);
@@ -776,11 +803,13 @@ extern "C" int llmserve_sample(const float* logits, const float* temperatures, c
                      with_top_p ? w.cleared_words : (size_t)0);
   hipLaunchKernelGGL(sample_exp_kernel, dim3(rows, pieces), dim3(SAMPLE_BLOCK), 0, stream, logits, temperatures, top_ps,
                      buffers, out, rows, vocab, pieces, first_pieces, with_top_p);
-  if (with_top_p)
-    for (int stage = 1; stage < SAMPLE_HISTOGRAMS; ++stage)
-      hipLaunchKernelGGL(sample_level_kernel, dim3(rows, pieces), dim3(SAMPLE_BLOCK), 0, stream, temperatures, top_ps,
-                         uniforms, buffers, rows, vocab, pieces, stage);
-  hipLaunchKernelGGL(sample_pick_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, temperatures, top_ps, uniforms,
-                     buffers, out, rows, vocab, pieces, with_top_p);
+  if (with_top_p) {
+    hipLaunchKernelGGL(sample_list_kernel, dim3(rows, pieces), dim3(SAMPLE_BLOCK), 0, stream, temperatures, top_ps, uniforms, buffers, vocab, pieces);
+    hipLaunchKernelGGL(sample_pick_kernel<true>, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, temperatures, top_ps, uniforms, buffers, out, vocab,
+                       pieces);
+  } else {
+    hipLaunchKernelGGL(sample_pick_kernel<false>, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, temperatures, top_ps, uniforms, buffers, out, vocab,
+                       pieces);
+  }
   return LAUNCH_STATUS();
 }

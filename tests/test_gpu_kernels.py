@@ -1233,3 +1233,30 @@ def test_product_through_the_ring(kernels, tiles, rows, inner, outer, parts):
     gated = torch.empty(rows, outer, dtype=dtype, device="cuda")
     _check(run(both, None, gated, True, 1), "ring")
     torch.testing.assert_close(gated.cpu().double(), F.silu(want) * (rounded(x, dtype) @ rounded(up, dtype).T), **TOLERANCE[dtype])
+
+
+@pytest.mark.parametrize("vocab", [9000, 8193, 40961])
+def test_top_p_over_more_entries_than_a_block_keeps(kernels, vocab):
+    """The row's block keeps 8,192 listed entries in registers: rows that list as many or more (a spread so small that all lie in two bins of
+    the first level, nothing but one value, two values side by side, many ties) against the rule in 64 bits."""
+    k = kernels[torch.float32]
+    generator = torch.Generator().manual_seed(vocab)
+    logits = torch.stack([
+        0.01 * torch.randn(vocab, generator=generator), torch.full((vocab,), 2.5), torch.randint(0, 2, (vocab,), generator=generator) * 0.03,
+        torch.randint(0, 9, (vocab,), generator=generator) * 0.005, torch.cat([torch.full((8192,), 1.0), torch.full((vocab - 8192,), -9.0)]),
+    ])
+    rows = logits.shape[0]
+    p = torch.exp(logits - logits.amax(1, keepdim=True))  # float32, as the rule has it
+    for draw, top_p in enumerate((0.1, 0.5, 0.93)):
+        uniforms = [plain.uniform_for(draw, row) for row in range(rows)]
+        got = k.sample(on_gpu(logits), on_gpu(torch.ones(rows)), on_gpu(torch.full((rows,), top_p)), on_gpu(torch.tensor(uniforms))).cpu().tolist()
+        for row in range(rows):
+            order = torch.argsort(p[row], descending=True, stable=True)
+            mass = p[row].double()[order].cumsum(0)
+            limit = float(torch.tensor(top_p)) * float(mass[-1])
+            kept = int((mass - p[row].double()[order] < limit).sum())
+            target = float(torch.tensor(uniforms[row])) * float(mass[kept - 1])
+            # the kernel's exp may be off torch's in the last place: the place of the token in the order is right to as much of the mass
+            place = int((order == got[row]).nonzero())
+            slack = 4 * 2.0 ** -23 * float(mass[-1])
+            assert place < kept + 1 and mass[place] > target - slack and (place == 0 or mass[place - 1] <= target + slack), (row, top_p)
