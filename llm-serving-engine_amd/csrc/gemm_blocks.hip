@@ -44,17 +44,105 @@ __device__ __forceinline__ void tile_of_workgroup(int index, int tiles_n, int ti
   tile_n = within / rows;
 }
 
+// What the way out does with the sums (and the bias).
+#define OUT_PLAIN 0
+#define OUT_GATED 1    // silu(gate) * up of columns that alternate gate_j, up_j
+#define OUT_ROTATED 2  // rows of q, k and v heads: q and k rotated in neighbouring pairs, k and v stored in their pages too
+
+// What OUT_ROTATED needs: cos and sin of [token][dim / 2], the layer's pages and each token's place there (negative: none; the
+// layout of a page is common.h's).  `dim` is a multiple of 16.
+struct Rotated {
+  const float2* table;
+  bf16_t *keys, *values;
+  const int* slots;
+  int heads, kv_heads, dim, page_size;
+};
+
+// What a wave of OUT_ROTATED asks for before its products, as their way from memory would be waited for at the end: lane l
+// holds where row l % 32 of its row tile j goes (the place of a negative slot is not used), the bias of the columns that it will write, and,
+// where one tile leaves the registers, their angles.
+template <int TN, int TM>
+struct Early {
+  static constexpr int PASSES = TN * TM == 1 ? 32 / (64 / (4 * TN)) : 0;
+  int slot[TM], page[TM], offset[TM], value_row[TM];
+  float bias[8];
+  f32x4 angles[PASSES ? PASSES : 1][2];
+};
+
+__device__ __forceinline__ const f32x4* angles_of(const Rotated& to, int m, int d) { return (const f32x4*)(to.table + ((size_t)m * to.dim + d) / 2); }
+
+template <int TN, int TM>
+__device__ __forceinline__ void ask_early(Early<TN, TM>& early, const Rotated& to, const void* bias, int bias_is_float, int M, int N,
+                                          int n_wave, int m_wave, int lane) {
+  constexpr int LANES_A_ROW = 4 * TN, ROWS_A_PASS = 64 / LANES_A_ROW;
+  const int n = min(n_wave + lane % LANES_A_ROW * 8, N - 8), width = value_piece_width(to.page_size);
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    const int m = m_wave + j * 32 + (lane & 31), slot = m < M ? to.slots[m] : -1;
+    early.slot[j] = slot;
+    early.page[j] = slot / to.page_size;
+    early.offset[j] = slot % to.page_size;
+    early.value_row[j] = early.offset[j] / width * width * to.dim + early.offset[j] % width;
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) early.bias[e] = bias ? load_as_float(bias, bias_is_float, n + e) : 0.f;
+#pragma unroll
+  for (int pass = 0; pass < Early<TN, TM>::PASSES; ++pass) {
+    const f32x4* angles = angles_of(to, min(m_wave + pass * ROWS_A_PASS + lane / LANES_A_ROW, M - 1), n % to.dim);
+    early.angles[pass][0] = angles[0], early.angles[pass][1] = angles[1];
+  }
+}
+
+// The values of 32 rows, which lie in `mine` with their bias (rows of `ROW` floats, a column each of the wave's 32 TN): a page keeps
+// them transposed in pieces of eight keys, so a lane takes one column of eight rows, and where the rows are one piece (a prompt's
+// portion) 64 lanes store 1 KB in a row.
+template <int TN, int TM, int ROW>
+__device__ __forceinline__ void store_values(const Rotated& to, const float* mine, const Early<TN, TM>& early, int j, int N, int n_wave, int lane) {
+  const int v_first = (to.heads + to.kv_heads) * to.dim, width = value_piece_width(to.page_size);
+  if (n_wave + 32 * TN <= v_first) return;
+#pragma unroll 1
+  for (int unit = 0; unit < 2 * TN; ++unit) {
+    const int column = (unit * 64 + lane) % (32 * TN), octet = (unit * 64 + lane) / (32 * TN);
+    const int n = n_wave + column;
+    const bool mine_to_store = n >= v_first && n < N;
+    const int head = (n - v_first) / to.dim, d = (n - v_first) % to.dim;
+    const size_t a_page = (size_t)to.page_size * to.dim;
+    bf16x8 run;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) run[i] = (bf16_t)mine[(size_t)(octet * 8 + i) * ROW + column];
+    const int slot = __shfl(early.slot[j], octet * 8);
+    bool together = width == 8 && slot >= 0 && slot % 8 == 0;
+#pragma unroll
+    for (int i = 1; i < 8; ++i) {
+      const int place = __shfl(early.slot[j], octet * 8 + i);
+      together = together & (place == slot + i);
+    }
+    if (__all(together)) {
+      const int page = __shfl(early.page[j], octet * 8), row = __shfl(early.value_row[j], octet * 8);
+      if (mine_to_store) *(bf16x8*)(to.values + ((size_t)page * to.kv_heads + head) * a_page + row + d * 8) = run;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        // (asked of other lanes by all lanes, before any is left out)
+        const int place = __shfl(early.slot[j], octet * 8 + i), page = __shfl(early.page[j], octet * 8 + i);
+        const int row = __shfl(early.value_row[j], octet * 8 + i);
+        if (mine_to_store && place >= 0) to.values[((size_t)page * to.kv_heads + head) * a_page + row + d * width] = run[i];
+      }
+    }
+  }
+}
+
 // The way out.  D[n][m] of a 32 x 32 tile: a lane holds column m = lane % 32 and rows n = 8 * (e / 4) +
 // 4 * (lane / 32) + e % 4, so its values lie in 32 different rows of `out`.  They go through LDS (`mine`: 32 x
 // (32 TN + 4) floats of this wave's own), 32 rows of x at a time, and leave as whole rows: 4 TN lanes write the
 // 32 TN columns of a row, eight columns (16 bytes of bfloat16) a lane.  n_wave, m_wave: where the wave's tiles begin;
 // `slice` the part of K (its own copy of `out`).  INSIDE: all of it lies inside the result, rows of which are a multiple of
 // eight long, so nothing is asked row by row (such questions kept the reads of one row from running beside the next).
-template <int TN, int TM, bool INSIDE, typename TO, bool GATED>
+template <int TN, int TM, bool INSIDE, typename TO, int OUT>
 __device__ __forceinline__ void store_tiles(const f32x16 (&acc)[TN][TM], float* mine, TO* __restrict__ out,
                                             const void* __restrict__ bias, int bias_is_float, int slice, int M, int N,
-                                            int n_wave, int m_wave, int lane) {
-  static_assert(!GATED || sizeof(TO) == 2, "a gated result is bfloat16");
+                                            int n_wave, int m_wave, int lane, const Rotated& rotated, const Early<TN, TM>& early) {
+  static_assert(OUT == OUT_PLAIN || sizeof(TO) == 2, "a gated or rotated result is bfloat16");
   constexpr int ROW = 32 * TN + 4;  // floats of a transposed row, padded
   constexpr int LANES_A_ROW = 4 * TN, ROWS_A_PASS = 64 / LANES_A_ROW;
   const int r32 = lane & 31, half = lane >> 5;
@@ -64,7 +152,8 @@ __device__ __forceinline__ void store_tiles(const f32x16 (&acc)[TN][TM], float* 
   float bias_here[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e)
-    bias_here[e] = with_bias && (INSIDE || n_piece + e < N) ? load_as_float(bias, bias_is_float, n_piece + e) : 0.f;
+    bias_here[e] = OUT == OUT_ROTATED ? early.bias[e] : with_bias && (INSIDE || n_piece + e < N) ? load_as_float(bias, bias_is_float, n_piece + e) : 0.f;
+  const int head = OUT == OUT_ROTATED ? n_piece / rotated.dim : 0, d = OUT == OUT_ROTATED ? n_piece % rotated.dim : 0;
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
 #pragma unroll
@@ -83,8 +172,36 @@ __device__ __forceinline__ void store_tiles(const f32x16 (&acc)[TN][TM], float* 
       float value[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 #pragma unroll
       for (int e = 0; e < 8; ++e) value[e] += bias_here[e];
+      int slot = 0, page = 0, offset = 0;
+      if constexpr (OUT == OUT_ROTATED) slot = __shfl(early.slot[j], row), page = __shfl(early.page[j], row), offset = __shfl(early.offset[j], row);
       if (!INSIDE && m >= M) continue;
-      if constexpr (GATED) {
+      if constexpr (OUT == OUT_ROTATED) {
+        if (!INSIDE && n_piece >= N) continue;  // (N is a multiple of 16)
+        // rounded before they are rotated, as where a kernel of its own reads them from memory
+        bf16_t packed[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) packed[e] = (bf16_t)value[e];
+        if (head < rotated.heads + rotated.kv_heads) {
+          constexpr bool HERE = Early<TN, TM>::PASSES > 0;
+          const f32x4* angles = angles_of(rotated, m, d);
+          const f32x4 first = HERE ? early.angles[HERE ? pass : 0][0] : angles[0], second = HERE ? early.angles[HERE ? pass : 0][1] : angles[1];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float c = e < 2 ? first[2 * e] : second[2 * e - 4], s = e < 2 ? first[2 * e + 1] : second[2 * e - 3];
+            const float a = (float)packed[2 * e], b = (float)packed[2 * e + 1];
+            packed[2 * e] = (bf16_t)(a * c - b * s);
+            packed[2 * e + 1] = (bf16_t)(b * c + a * s);
+          }
+        }
+        *(uint4*)(out + (size_t)m * N + n_piece) = *(const uint4*)packed;
+        if (head >= rotated.heads + rotated.kv_heads) {
+          *(f32x4*)(mine + (size_t)row * ROW + piece * 8) = (f32x4){value[0], value[1], value[2], value[3]};  // (for store_values)
+          *(f32x4*)(mine + (size_t)row * ROW + piece * 8 + 4) = (f32x4){value[4], value[5], value[6], value[7]};
+        } else if (head >= rotated.heads && slot >= 0) {
+          bf16_t* keys = rotated.keys + ((size_t)page * rotated.kv_heads + head - rotated.heads) * rotated.page_size * rotated.dim;
+          *(uint4*)(keys + ((size_t)(d / KEY_PIECE) * rotated.page_size + offset) * KEY_PIECE) = *(const uint4*)packed;
+        }
+      } else if constexpr (OUT == OUT_GATED) {
         TO* dst = out + (size_t)m * (N / 2) + n_piece / 2;
         float gated[4];
 #pragma unroll
@@ -121,6 +238,7 @@ __device__ __forceinline__ void store_tiles(const f32x16 (&acc)[TN][TM], float* 
         }
       }
     }
+    if constexpr (OUT == OUT_ROTATED) store_values<TN, TM, ROW>(rotated, mine, early, j, N, n_wave, lane);
   }
 }
 
@@ -145,10 +263,10 @@ __device__ __forceinline__ void wait_stages(int younger) {
 }
 
 // WN x WM waves of TN x TM tiles; stages of BK k; A_SIMD: the waves a SIMD is to hold.
-template <int WN, int WM, int TN, int TM, int BK, int STAGES, int A_SIMD, typename TO, bool GATED>
+template <int WN, int WM, int TN, int TM, int BK, int STAGES, int A_SIMD, typename TO, int OUT>
 __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                           const void* __restrict__ bias, int bias_is_float,
-                                                                          TO* __restrict__ out, int M, int N, int K, int k_split) {
+                                                                          TO* __restrict__ out, int M, int N, int K, int k_split, Rotated rotated) {
   constexpr int THREADS = WN * WM * 64, BN = WN * TN * 32, BM = WM * TM * 32, SLOTS = BK / 8, HALVES = BK / 16;
   constexpr int ROW_BYTES = BK * 2, W_BYTES = BN * ROW_BYTES, STAGE_BYTES = W_BYTES + BM * ROW_BYTES;
   constexpr int PER_W = BN * SLOTS / THREADS, PER = PER_W + BM * SLOTS / THREADS;  // 16-byte pieces of a stage a lane asks for
@@ -182,6 +300,10 @@ __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const 
   const int turned = swizzle(r32);
   const unsigned row_w = base + (unsigned)(wave_n * TN * 32 + r32) * ROW_BYTES;
   const unsigned row_x = base + W_BYTES + (unsigned)(wave_m * TM * 32 + r32) * ROW_BYTES;
+
+  Early<TN, TM> early;
+  if constexpr (OUT == OUT_ROTATED)
+    ask_early(early, rotated, bias, bias_is_float, M, N, n0 + wave_n * TN * 32, m0 + wave_m * TM * 32, lane);
 
   f32x16 acc[TN][TM];  // [tile of weight rows][tile of x rows]
 #pragma unroll
@@ -269,28 +391,28 @@ __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const 
   float* mine = (float*)lds + (size_t)wave * 32 * (32 * TN + 4);
   if (m_wave >= M || n_wave >= N) return;
   if (m_wave + 32 * TM <= M && n_wave + 32 * TN <= N && N % 8 == 0)
-    store_tiles<TN, TM, true, TO, GATED>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane);
+    store_tiles<TN, TM, true, TO, OUT>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane, rotated, early);
   else
-    store_tiles<TN, TM, false, TO, GATED>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane);
+    store_tiles<TN, TM, false, TO, OUT>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane, rotated, early);
 }
 
-template <int WN, int WM, int TN, int TM, int BK, int STAGES, int A_SIMD, typename TO, bool GATED>
+template <int WN, int WM, int TN, int TM, int BK, int STAGES, int A_SIMD, typename TO, int OUT>
 static int launch_block(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
-                        int splits, hipStream_t stream) {
+                        int splits, hipStream_t stream, const Rotated& rotated) {
   constexpr int BN = WN * TN * 32, BM = WM * TM * 32;
   constexpr size_t stages = (size_t)STAGES * (BN + BM) * BK * 2, way_out = (size_t)WN * WM * 32 * (32 * TN + 4) * sizeof(float);
   constexpr size_t bytes = stages > way_out ? stages : way_out;
   static_assert(bytes <= 160 * 1024, "a CU's LDS");
   static bool asked = false;
   if (!asked) {
-    if (hipFuncSetAttribute((const void*)gemm_block_kernel<WN, WM, TN, TM, BK, STAGES, A_SIMD, TO, GATED>,
+    if (hipFuncSetAttribute((const void*)gemm_block_kernel<WN, WM, TN, TM, BK, STAGES, A_SIMD, TO, OUT>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
       return ERR_BAD_ARGUMENT;
     asked = true;
   }
-  hipLaunchKernelGGL((gemm_block_kernel<WN, WM, TN, TM, BK, STAGES, A_SIMD, TO, GATED>),
+  hipLaunchKernelGGL((gemm_block_kernel<WN, WM, TN, TM, BK, STAGES, A_SIMD, TO, OUT>),
                      dim3(((N + BN - 1) / BN) * ((M + BM - 1) / BM), 1, splits), dim3(WN * WM * 64), bytes, stream, (const bf16_t*)x,
-                     (const bf16_t*)w, bias, bias_is_float, (TO*)out, M, N, K, K / splits);
+                     (const bf16_t*)w, bias, bias_is_float, (TO*)out, M, N, K, K / splits, rotated);
   return LAUNCH_STATUS();
 }
 
@@ -338,10 +460,10 @@ extern "C" int llmserve_gemm_blocks_parts(int M, int N, int K) {
   return best;
 }
 
-template <typename TO, bool GATED>
+template <typename TO, int OUT>
 static int launch_shape(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
                         int splits, hipStream_t stream) {
-#define BLOCK(...) return launch_block<__VA_ARGS__, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream)
+#define BLOCK(...) return launch_block<__VA_ARGS__, TO, OUT>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, {})
   const int shape = pick_shape(M, N, K, splits);
   if ((K / splits) % 64) {  // a K that ends in half a stage: stages of 32
     if (shape < 3) BLOCK(2, 4, 4, 2, 32, 5, 2);
@@ -366,7 +488,37 @@ extern "C" int llmserve_gemm_blocks(const void* x, const void* w, const void* bi
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || K % 32 || (gated && N % 2) || splits < 1 || gated > 1 || (gated && out_is_float)) return ERR_BAD_ARGUMENT;  // (this epilogue knows silu alone)
   if (splits > 1 && (gated || !out_is_float || K % splits || (K / splits) % 32)) return ERR_BAD_ARGUMENT;
-  if (gated) return launch_shape<bf16_t, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
-  return out_is_float ? launch_shape<float, false>(x, w, bias, bias_is_float, out, M, N, K, splits, stream)
-                      : launch_shape<bf16_t, false>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
+  if (gated) return launch_shape<bf16_t, OUT_GATED>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
+  return out_is_float ? launch_shape<float, OUT_PLAIN>(x, w, bias, bias_is_float, out, M, N, K, splits, stream)
+                      : launch_shape<bf16_t, OUT_PLAIN>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
+}
+
+// A product whose heads are rotated on the way out, in the smallest tile of which one round of 256 workgroups holds the result, as
+// more CUs then bring the operands.  Us at N 2,048 K 1,536, tiles of 64 x 32, 64 x 64, 128 x 64 and 128 x 128 (without the values' way to
+// their pages): 96 rows 10.4 10.9 16.1 21.1, 256 rows 10.6 11.4 16.4 22.8, 512 rows 13.7 11.7 16.4 22.4, 1,024 rows 26.8 16.6 16.9 23.8,
+// 2,048 rows 48.5 31.2 25.3 24.8; at N 4,608 K 3,584: 96 rows 19.2 19.9 30.0 37.6, 192 rows 26.6 21.3 30.7 36.0.  What it saves is a launch and
+// the rows' way to memory and back: with the kernel that rotates and stores behind the library's product 15.5 us at 96 rows of N 2,048 K 1,536, here
+// 11.6; 16.1 -> 11.7 at 256, 27.3 -> 26.0 at 2,048.  (Places, bias and angles asked for only on the way out: 13.4 at 96 rows.)
+static int launch_rotated(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
+                          hipStream_t stream, const Rotated& rotated) {
+#define BLOCK(...) return launch_block<__VA_ARGS__, bf16_t, OUT_ROTATED>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, rotated)
+  auto one_round = [&](int n, int m) { return (long)((N + n - 1) / n) * ((M + m - 1) / m) <= 256; };
+  if (K % 64) BLOCK(2, 2, 2, 2, 32, 4, 2);
+  if (one_round(64, 32)) BLOCK(2, 1, 1, 1, 64, 5, 2);
+  if (one_round(64, 64)) BLOCK(2, 2, 1, 1, 64, 5, 2);
+  if (one_round(128, 64)) BLOCK(2, 2, 2, 1, 64, 3, 2);
+  BLOCK(2, 2, 2, 2, 64, 5, 1);
+#undef BLOCK
+}
+
+// Rows of q, k and v heads: out [M, (heads + 2 kv_heads) dim] bfloat16 = x . w^T (+ bias), of which the q and k heads are rotated in
+// neighbouring pairs by `table` (cos, sin of [M][dim / 2]), and k and v also stored in the pages.  `dim` a multiple of 16, K of 32.
+extern "C" int llmserve_gemm_rotated(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int K,
+                                     const float* table, int heads, int kv_heads, int dim, void* keys, void* values, const int* slots,
+                                     int page_size, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (K <= 0 || K % 32 || heads < 1 || kv_heads < 1 || dim < 16 || dim % 16 || page_size < 1 || !table || !keys || !values || !slots) return ERR_BAD_ARGUMENT;
+  if ((size_t)table % 16 || (size_t)keys % 16 || (size_t)values % 16) return ERR_BAD_ARGUMENT;
+  return launch_rotated(x, w, bias, bias_is_float, out, M, (heads + 2 * kv_heads) * dim, K, stream,
+                        {(const float2*)table, (bf16_t*)keys, (bf16_t*)values, slots, heads, kv_heads, dim, page_size});
 }

@@ -77,6 +77,7 @@ _SIGNATURES = {
     "llmserve_gemm_into_norm": "pppippippippiiiipiip",
     "llmserve_gemm_scaled": "ppfppiiiip",
     "llmserve_gemm_scaled_streams": "iii",
+    "llmserve_gemm_rotated": "pppipiipiiipppip",
     "llmserve_gemm_blocks": "pppipiiiiiip",
     "llmserve_gemm_blocks_parts": "iii",
     "llmserve_attention_generic": "pipiipppippiiiiifipfpiiipip",
@@ -408,6 +409,50 @@ class HipKernels:
             group.page_size if store else 1, self._stream,
         )
         _check(status, "rotate_and_store")
+
+    def linear_rotated(self, x, weights: LinearWeights, layout, batch, cell, inverse_frequencies, pairing: str) -> torch.Tensor | None:
+        """`linear(x, weights)` and `rotate_and_store` of its rows in one kernel, where it takes them and is ahead; else None, and nothing done."""
+        rows, inner = x.shape
+        dim, store = layout.head_dim, cell is not None and cell.writable
+        if (
+            pairing != "adjacent" or not store or batch.max_query_length == 1 or rows <= 64 or dim % 16 or weights.out_features != layout.width
+            or layout.stride != layout.width or inner != weights.in_features or inverse_frequencies.shape != (dim // 2,)
+            or any(tensor.dtype != torch.bfloat16 for tensor in (x, weights.weight, cell.keys, cell.values))
+            or not _in_pieces(x, weights.weight, cell.keys, cell.values) or not HipKernels._rotated_ahead(rows, weights.out_features, inner)
+        ):
+            return None
+        # (a library derived from this one that does a step in a way of its own is asked for it)
+        kind = type(self)
+        if any(getattr(kind, step) is not getattr(HipKernels, step) for step in ("linear", "rotate_and_store", "rotate_store_attend", "_rotate_store_attend")):
+            return None
+        group = batch.groups[cell.group]
+        if cell.values.shape[1:] != cell.need.page_fields(group.page_size)["values"] or batch.positions.shape[0] != rows or group.slot_mapping.shape[0] != rows:
+            return None
+        table, bias = self.rotary_table(batch, inverse_frequencies), weights.bias
+        out = self._empty((rows, weights.out_features), torch.bfloat16)
+        status = self._gemm_blocks.llmserve_gemm_rotated(
+            _pointer(x), _pointer(weights.weight), _pointer(bias), _is_float(bias) if bias is not None else 0, _pointer(out), rows, inner,
+            _pointer(table), layout.num_heads, layout.num_kv_heads, dim, _pointer(cell.keys), _pointer(cell.values),
+            _pointer(group.slot_mapping), group.page_size, self._stream,
+        )
+        _check(status, "linear_rotated")
+        return out
+
+    @staticmethod
+    def _rotated_ahead(rows: int, out_features: int, in_features: int) -> bool:
+        """Where `linear_rotated` is ahead of the product (the library's up to 512 rows) and the kernel that rotates and stores: while one
+        round of 64 x 64 tiles holds the result, for K up to 2,048 one of 128 x 64, and where the product alone is the tiled kernel's too.
+        Us, both in a captured chain over different weights, before -> now: N 2,048 K 1,536: 96 rows 15.5 -> 11.6, 256 16.1 -> 11.7, 512 17.4
+        -> 12.9, 1,024 23.9 -> 18.5, 2,048 27.3 -> 26.0; N 1,152 K 896: 96 rows 14.6 -> 8.9, 1,024 17.3 -> 13.1; N 2,560 K 2,048: 96 rows 17.5 -> 13.4,
+        448 21.1 -> 21.5, 768 23.5 -> 21.5; N 4,608 K 3,584: 96 rows 26.0 -> 19.9, 192 36.2 -> 22.3, 320 30.3 -> 32.9, 1,024 52.2 -> 58.7; N 7,168 K
+        5,120: 96 rows 35.6 -> 30.2, 320 54.2 -> 55.4, 2,048 142 -> 168."""
+        if in_features % 64:
+            return False
+        by_rows = -(-rows // 64)
+        return (
+            -(-out_features // 64) * by_rows <= 256 or (in_features <= 2048 and -(-out_features // 128) * by_rows <= 256)
+            or HipKernels._tiled_ahead(rows, out_features, in_features, False, False)
+        )
 
     def gather_rows(self, hidden, delta, rows) -> torch.Tensor:
         count, width = rows.shape[0], hidden.shape[1]

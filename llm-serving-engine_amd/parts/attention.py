@@ -8,7 +8,7 @@ from typing import Any, ClassVar
 import torch
 
 from .base import MIXERS, POSITIONS, PagedKeyValue, Part, TensorSpec
-from .position import HeadLayout
+from .position import HeadLayout, Rotary
 
 
 class Mixer(Part):
@@ -103,6 +103,11 @@ class Attention(Mixer):
         return type(self).forward is Attention.forward and getattr(self.position, "takes_into", False)
 
     def forward(self, x: torch.Tensor, batch, cell, **into) -> torch.Tensor:
+        if isinstance(self.position, Rotary):
+            qkv = self.position.project_and_store(x, self.qkv, self.layout, batch, cell)
+            if qkv is not None:
+                mixed = self.kernels.paged_attention(qkv, self.layout, batch, cell, self.spec.scale, self.spec.window)
+                return self.kernels.linear(mixed, self.out, out_dtype=torch.float32, partial=True)
         qkv = self.kernels.linear(x, self.qkv)
         # the output projection goes with the attention: a kernel library may fuse the two (key splits of
         # a decode step merged by the product that reads them)

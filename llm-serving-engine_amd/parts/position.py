@@ -88,6 +88,15 @@ class Rotary(PositionEncoding):
             qkv, layout, batch, cell, self.inverse_frequencies, self.spec.pairing
         )
 
+    def project_and_store(self, x, weights, layout: HeadLayout, batch, cell):
+        """The rows that `encode_and_store` leaves of `linear(x, weights)`, k and v stored, by one kernel of a library that has one for
+        these sizes; else None, and nothing done.  (An encoding derived from this one is asked for its own steps.)"""
+        fused = getattr(self.kernels, "linear_rotated", None)
+        kind = type(self)
+        if fused is None or kind.encode_and_store is not Rotary.encode_and_store or kind.encode_store_attend is not Rotary.encode_store_attend:
+            return None
+        return fused(x, weights, layout, batch, cell, self.inverse_frequencies, self.spec.pairing)
+
     @property
     def takes_into(self) -> bool:
         """Whether `encode_store_attend` can be told of a norm behind the product (`into`); an encoding with one of its own says so itself."""

@@ -946,6 +946,71 @@ def test_rotation_store_and_attention_of_prompt_portions(kernels, dtype, pairing
     torch.testing.assert_close(stored_v, want_v, atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("with_bias", [torch.bfloat16, torch.float32, None])
+@pytest.mark.parametrize("heads,kv_heads,dim,page,inner,counts", [
+    (12, 2, 128, 16, 1536, [65]),              # tiles of 64 x 32, the last of one row
+    (12, 2, 128, 16, 256, [33, 1, 223]),       # nine of them down, then too many: 64 x 64
+    (2, 1, 16, 8, 64, [90, 7]),                # fewer columns than a tile, one stage
+    (5, 3, 48, 24, 128, [70, 50]),             # heads across the tiles' edges, a page that is no power of two
+    (4, 2, 80, 4, 192, [66, 3]),               # pages of less than a piece of values
+    (14, 2, 64, 16, 896, [40, 9, 980]),        # 128 x 64
+    (12, 2, 128, 16, 128, [7, 1026]),          # 128 x 128
+    (12, 2, 128, 16, 96, [130, 30]),           # half a stage at the end of K
+])
+def test_product_rotated_and_stored_in_one_kernel(kernels, monkeypatch, heads, kv_heads, dim, page, inner, counts, with_bias):
+    """`linear_rotated` against the product in 64 bits, rounded to bfloat16, rotated.  The sums are float32, so what is rotated may be the
+    neighbouring bfloat16 (2^-7 of it), which a rotation keeps within 2^-7 of the pair's length, and the result is rounded once more (2^-8):
+    together below 2^-6.  Values are rounded once.  Pages hold the rows' keys and values bit for bit; slots of no token stay as they were."""
+    dtype = torch.bfloat16
+    lengths = [count + 5 * index for index, count in enumerate(counts)]
+    batch, cell, _, layout = paged_case(lengths, counts, heads, kv_heads, dim, page, dtype, shuffle_seed=dim + heads)
+    rows, generator = sum(counts), torch.Generator().manual_seed(inner)
+    x = torch.randn(rows, inner, generator=generator).to(dtype)
+    weight = (torch.randn(layout.width, inner, generator=generator) * inner ** -0.5).to(dtype)
+    bias = None if with_bias is None else torch.randn(layout.width, generator=generator).to(with_bias)
+    batch.groups[0].slot_mapping[3] = -1  # (a row that is not stored)
+    slots = batch.groups[0].slot_mapping.cpu().long()
+    before_k, before_v = key_rows(cell.keys.cpu().float()).clone(), value_rows(cell.values.cpu().float()).clone()
+    library = kernels[dtype]
+    prepared = library.prepare_linear([on_gpu(weight, dtype)], [on_gpu(bias, with_bias)] if bias is not None else None)
+    inverse = 1.0 / (3000.0 ** (torch.arange(0, dim, 2).float() / dim))
+    monkeypatch.setattr(type(library), "_rotated_ahead", staticmethod(lambda *sizes: True))  # every size, not only where it is ahead
+    got = library.linear_rotated(x.cuda(), prepared, layout, batch, cell, on_gpu(inverse), "adjacent")
+    assert got is not None
+    got = got.cpu().double()
+    exact = x.double() @ weight.double().T + (bias.double() if bias is not None else 0)
+    split = (heads + kv_heads) * dim
+    turned = exact.to(dtype).double()[:, :split].unflatten(1, (-1, dim))
+    angles = plain.rope_angles(dim, 3000.0, batch.positions.cpu().long())
+    turned = plain.rope_adjacent(turned, angles)
+    lengths_of_pairs = turned.unflatten(2, (-1, 2)).norm(dim=-1, keepdim=True).expand(-1, -1, -1, 2).flatten(2)
+    assert ((got[:, :split].unflatten(1, (-1, dim)) - turned).abs() <= lengths_of_pairs * 2.0 ** -6 + 1e-4).all()
+    assert ((got[:, split:] - exact[:, split:]).abs() <= exact[:, split:].abs() * 2.0 ** -8 + 1e-4).all()
+    stored = slots >= 0
+    k, v = got[:, heads * dim : split].unflatten(1, (-1, dim)), got[:, split:].unflatten(1, (-1, dim))
+    now_k, now_v = key_rows(cell.keys.cpu().float()), value_rows(cell.values.cpu().float())
+    before_k[slots[stored] // page, :, slots[stored] % page] = k[stored].float()
+    before_v[slots[stored] // page, :, :, slots[stored] % page] = v[stored].float()
+    assert torch.equal(now_k.nan_to_num(7e7), before_k.nan_to_num(7e7)) and torch.equal(now_v.nan_to_num(7e7), before_v.nan_to_num(7e7))
+
+
+def test_product_rotated_and_stored_refuses_bad_sizes(kernels):
+    from llmserve_amd.kernels.hip import _pointer
+
+    k = kernels[torch.bfloat16]
+    x, w, out, table, pages = (torch.zeros(4096, device="cuda") for _ in range(5))
+    slots = torch.zeros(4, dtype=torch.int32, device="cuda")
+
+    def status(inner=64, heads=1, kv_heads=1, dim=16, page=16, keys=pages.data_ptr(), angles=table.data_ptr()):
+        return k._gemm_blocks.llmserve_gemm_rotated(_pointer(x), _pointer(w), None, 0, _pointer(out), 1, inner, angles, heads, kv_heads, dim,
+                                                    keys, pages.data_ptr(), _pointer(slots), page, k._stream)
+
+    for wrong in (dict(inner=48), dict(inner=0), dict(heads=0), dict(kv_heads=0), dict(dim=24), dict(dim=0), dict(page=0), dict(keys=None),
+                  dict(angles=None), dict(keys=pages.data_ptr() + 8)):
+        assert status(**wrong) == 1001
+    assert status() == 0
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,window", [(6, 2, 64, None), (6, 1, 128, None), (8, 4, 128, 2048), (5, 1, 32, None), (4, 2, 160, None)])
 @pytest.mark.parametrize("lengths,counts", [([3000, 20, 2100, 700, 1], [1, 20, 60, 1, 1]), ([520, 9, 300], [200, 9, 1]), ([4200, 2050], [1, 33])])
 def test_portions_beside_long_contexts(kernels, heads, kv_heads, dim, window, lengths, counts):

@@ -272,6 +272,15 @@ def test_products_of_many_rows_go_where_they_were_measured_ahead(rows, out_featu
     assert (route(stand_in(), rows, out_features, in_features, gated, may_split) == "tiled") == tiled
 
 
+@pytest.mark.parametrize("rows,out_features,in_features,ahead", [
+    (65, 2048, 1536, True), (2048, 2048, 1536, True), (2112, 2048, 1536, False), (1024, 1152, 896, True), (192, 4608, 3584, True),
+    (256, 4608, 3584, False), (128, 7168, 5120, True), (192, 7168, 5120, False), (768, 2560, 2048, True), (1024, 2560, 2048, False), (96, 2048, 96, False),
+])
+def test_rotated_products_are_fused_where_it_was_measured_ahead(rows, out_features, in_features, ahead):
+    """Both sides of the lines that `_rotated_ahead` draws."""
+    assert HipKernels._rotated_ahead(rows, out_features, in_features) == ahead
+
+
 @pytest.mark.parametrize("keys,blocks,runs", [
     (1024, 20, 1), (2048, 28, 2), (2048, 100, 2), (2048, 128, 2), (2048, 148, 1), (2048, 184, 1), (2048, 232, 1), (2048, 296, 1),
     (4096, 28, 4), (4096, 148, 3), (4096, 184, 1), (8192, 184, 2), (8192, 28, 8), (8192, 300, 1), (65536, 10, 8),
