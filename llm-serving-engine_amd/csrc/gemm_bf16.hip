@@ -1010,7 +1010,7 @@ extern "C" int llmserve_gemm_medium(const void* x, const void* w, const void* bi
 // many stages of weights whatever the compiler does with the registers, and a weight row is read from memory
 // once for all rows of x.  The waves divide a stage's chunks between them; one barrier a stage says that
 // everyone's loads have landed and that the stage before may be filled again.  A wave multiplies one tile of x
-// (two, with eight tiles of x: up to 128 rows) with its share of the weight tiles, so no sums meet at the end.
+// (two, with six or eight tiles of x: up to 96 and 128 rows) with its share of the weight tiles, so no sums meet at the end.
 __device__ __forceinline__ void ring_load(const bf16_t* from, unsigned to) {
   // (M0 names the place in LDS; it is put back, the compiler keeps other things there)
   unsigned kept;
@@ -1036,15 +1036,15 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
                                                         const void* __restrict__ bias, int bias_is_float,
                                                         TO* __restrict__ out, int M, int N, int K, int k_split, Link link) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
-  constexpr int XPW = MT > 4 ? MT / 4 : 1;   // tiles of x a wave multiplies
-  constexpr int XGROUPS = MT / XPW;          // groups of waves by their tiles of x
+  constexpr int XPW = MT > 4 ? 2 : 1;        // tiles of x a wave multiplies
+  constexpr int XGROUPS = MT > 4 ? 4 : MT;   // groups of waves by their tiles of x
   constexpr int WAYS = 4 / XGROUPS;          // groups of waves that divide the weight tiles between them
   constexpr int MINE = NT / WAYS;            // weight tiles a wave multiplies
   constexpr int TILES = NT + MT;        // of a stage, each KSTEPS chunks of 1 KB
   constexpr int STAGE_BYTES = TILES * KSTEPS * STREAM_CHUNK;
   constexpr int PER_WAVE = TILES * KSTEPS / 4;  // chunks a wave brings per stage
   constexpr int APART = 4 / KSTEPS;             // tiles between two chunks of a wave
-  static_assert(MT == 2 || MT == 4 || MT == 8, "two, four or eight tiles of x");
+  static_assert(MT == 2 || MT == 4 || MT == 6 || MT == 8, "two, four, six or eight tiles of x");
   static_assert(KSTEPS == 2 || KSTEPS == 4, "stages of 64 or 128 k");
   static_assert(NT % WAYS == 0, "the waves divide the weight tiles evenly");
   static_assert(TILES * KSTEPS % 4 == 0, "the waves divide a stage's chunks evenly");
@@ -1065,7 +1065,8 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
     src[j] = row + k_first + my_step * STEP + load_piece * 8;
   }
   const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)ring;
-  const int x_tile = (wave % XGROUPS) * XPW, first_tile = wave / XGROUPS;  // the wave's first tile of x, of weights
+  // the wave's first tile of x, of weights (of six tiles of x the fourth wave multiplies what the third does: the same sums to the same places)
+  const int x_tile = min((wave % XGROUPS) * XPW, MT - XPW), first_tile = wave / XGROUPS;
   const unsigned read_at = base + (unsigned)(4 * r + (g ^ ((r >> 1) & 3))) * 16;
   const unsigned read_w = read_at + (unsigned)first_tile * KSTEPS * STREAM_CHUNK;
   const unsigned read_x = read_at + (unsigned)(NT + x_tile) * KSTEPS * STREAM_CHUNK;
@@ -1255,7 +1256,7 @@ static int launch_ring(const void* x, const void* w, const void* bias, int bias_
   return LAUNCH_STATUS();
 }
 
-// nt tiles of 16 weight rows a workgroup, stages of 128 k; four stages, or three with eight tiles of x (65 to 128
+// nt tiles of 16 weight rows a workgroup, stages of 128 k; four stages, or three with six or eight tiles of x (65 to 128
 // rows), which fill the LDS with five weight tiles beside them
 template <typename TO, bool GATED>
 static int pick_ring(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
@@ -1269,6 +1270,10 @@ static int pick_ring(const void* x, const void* w, const void* bias, int bias_is
   RING_CASE(6)
 #undef RING_CASE
   if (nt == 5 && M > 32 && M <= 64) return launch_ring<5, 4, 4, 4, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream);
+  // Up to 96 rows six tiles of x, where eight would bring and multiply rows that are not there: a third of x's bytes a stage and of the products.
+  // (gated, 65 / 80 / 96 rows, us, eight -> six: N 17,920 K 1,536 22.2 21.7 21.6 -> 19.1 18.4 18.5; N 9,728 K 896 11.9 12.2 12.2 -> 11.0 11.2 11.2;
+  // N 12,288 K 2,048 25.5 24.9 25.1 -> 21.5 21.0 21.1; the same bits)
+  if (nt == 5 && M > 64 && M <= 96) return launch_ring<5, 6, 4, 3, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream);
 #define ROWS_CASE(NT_)                                                                                                  \
   if (nt == NT_ && M > 64) return launch_ring<NT_, 8, 4, 3, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream);
   ROWS_CASE(2)

@@ -1325,3 +1325,26 @@ def test_top_p_over_more_entries_than_a_block_keeps(kernels, vocab):
             place = int((order == got[row]).nonzero())
             slack = 4 * 2.0 ** -23 * float(mass[-1])
             assert place < kept + 1 and mass[place] > target - slack and (place == 0 or mass[place - 1] <= target + slack), (row, top_p)
+
+
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("rows", [65, 79, 80, 81, 95, 96, 97])
+def test_ring_of_six_tiles_of_rows_has_the_bits_of_eight(kernels, rows, gated):
+    """Up to 96 rows the ring has six tiles of x, beyond eight: a row's sums are the same products in the same order.  A last workgroup of
+    weight rows that are not all there, rows that end inside a tile, and nothing written behind the last row."""
+    from llmserve_amd.kernels.hip import _pointer
+
+    k, inner, outer = kernels[torch.bfloat16], 640, 5 * 16 * 7 + 48
+    generator = torch.Generator(device="cuda").manual_seed(rows)
+    x, w = (torch.randn(shape, generator=generator, device="cuda").bfloat16() for shape in ((128, inner), (outer, inner)))
+    results = []
+    for count in (rows, 128):
+        out = torch.full((130, outer // 2 if gated else outer), 7.0, device="cuda", dtype=torch.bfloat16)
+        assert k._gemm_bf16.llmserve_gemm_ring(_pointer(x), _pointer(w), None, 0, _pointer(out), 0, int(gated), count, outer, inner, 1, 5, k._stream) == 0
+        assert (out[count:] == 7.0).all()
+        results.append(out[:rows])
+    assert torch.equal(*results)
+    exact = x[:rows].double() @ w.double().T
+    if gated:
+        exact = torch.nn.functional.silu(exact[:, ::2]) * exact[:, 1::2]
+    torch.testing.assert_close(results[0].double(), exact, **TOLERANCE[torch.bfloat16])
