@@ -105,6 +105,14 @@ __device__ __forceinline__ size_t value_element(int d, int offset, int page_size
 #define BIAS_SPARE 24
 __device__ __forceinline__ int bias_element(int distance, int reach) { return reach + 7 - max(min(distance, reach + 7), -8); }
 
+// The pair (x, y) of a head turned by an angle of cosine c and sine s: x c - y s and y c + x s.  Which product of the difference is rounded
+// before the other is subtracted from it is said here and not left to the compiler, as every kernel that turns bfloat16 rows has to
+// give the same bits: x c in the first of eight pairs (`first`), y s in the others.
+__device__ __forceinline__ void turn_pair(float x, float y, float c, float s, bool first, float* turned_x, float* turned_y) {
+  *turned_x = first ? __builtin_fmaf(-y, s, x * c) : __builtin_fmaf(x, c, -(y * s));
+  *turned_y = __builtin_fmaf(y, c, x * s);
+}
+
 // Memory that the next kernel reads, brought into the caches by workgroups of a kernel that leaves the path to memory idle: a
 // weight as `stripes` runs of `stripe` bytes (a multiple of 16; the rows that one workgroup of the next kernel takes), of
 // which that kernel's workgroup i reads run i.  The chip hands the workgroups of a launch to its eight chiplets in turn and each has an

@@ -525,22 +525,19 @@ __global__ __launch_bounds__(256) void rotate_and_store_vector_kernel(
     const float2* angles = table + (size_t)token * half + 8 * p;
 #pragma unroll
     for (int i = 0; i < 8; ++i) cs[i] = angles[i];
+    auto turn = [&](auto& here, int x, auto& there, int y, int pair) {
+      float first, second;
+      turn_pair((float)here[x], (float)there[y], cs[pair].x, cs[pair].y, pair == 0, &first, &second);
+      here[x] = (bf16_t)first, there[y] = (bf16_t)second;
+    };
     if (pairing == 2) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float x = (float)a[i], y = (float)b[i];
-        a[i] = (bf16_t)(x * cs[i].x - y * cs[i].y);
-        b[i] = (bf16_t)(y * cs[i].x + x * cs[i].y);
-      }
+      for (int i = 0; i < 8; ++i) turn(a, i, b, i, i);
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float x = (float)a[2 * i], y = (float)a[2 * i + 1];
-        a[2 * i] = (bf16_t)(x * cs[i].x - y * cs[i].y);
-        a[2 * i + 1] = (bf16_t)(y * cs[i].x + x * cs[i].y);
-        const float u = (float)b[2 * i], v = (float)b[2 * i + 1];
-        b[2 * i] = (bf16_t)(u * cs[4 + i].x - v * cs[4 + i].y);
-        b[2 * i + 1] = (bf16_t)(v * cs[4 + i].x + u * cs[4 + i].y);
+        turn(a, 2 * i, a, 2 * i + 1, i);
+        turn(b, 2 * i, b, 2 * i + 1, 4 + i);
       }
     }
     *(bf16x8*)(h + ia) = a;

@@ -188,9 +188,9 @@ __device__ __forceinline__ void store_tiles(const f32x16 (&acc)[TN][TM], float* 
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float c = e < 2 ? first[2 * e] : second[2 * e - 4], s = e < 2 ? first[2 * e + 1] : second[2 * e - 3];
-            const float a = (float)packed[2 * e], b = (float)packed[2 * e + 1];
-            packed[2 * e] = (bf16_t)(a * c - b * s);
-            packed[2 * e + 1] = (bf16_t)(b * c + a * s);
+            float x, y;
+            turn_pair((float)packed[2 * e], (float)packed[2 * e + 1], c, s, e == 0 && d % 16 == 0, &x, &y);
+            packed[2 * e] = (bf16_t)x, packed[2 * e + 1] = (bf16_t)y;
           }
         }
         *(uint4*)(out + (size_t)m * N + n_piece) = *(const uint4*)packed;

@@ -994,6 +994,37 @@ def test_product_rotated_and_stored_in_one_kernel(kernels, monkeypatch, heads, k
     assert torch.equal(now_k.nan_to_num(7e7), before_k.nan_to_num(7e7)) and torch.equal(now_v.nan_to_num(7e7), before_v.nan_to_num(7e7))
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,inner,counts", [
+    (12, 2, 128, 256, [65, 448]),      # 64 x 64
+    (12, 2, 128, 128, [7, 1026]),      # 128 x 128
+    (5, 3, 48, 128, [700]),            # heads across the tiles' edges
+    (14, 2, 64, 896, [40, 9, 980]),    # 128 x 64
+])
+def test_product_rotated_and_stored_has_the_bits_of_its_two_kernels(kernels, monkeypatch, heads, kv_heads, dim, inner, counts):
+    """The tiled product's sums are the same in every tile, and a rotation rounds in the same places in either kernel, so that rows and pages
+    are those of the product and of the kernel behind it, bit for bit."""
+    dtype, page = torch.bfloat16, 16
+    library, rows, generator = kernels[dtype], sum(counts), torch.Generator().manual_seed(rows_seed := inner + dim)
+    x = torch.randn(rows, inner, generator=generator).to(dtype).cuda()
+    monkeypatch.setattr(type(library), "_rotated_ahead", staticmethod(lambda *sizes: True))
+    inverse = on_gpu(1.0 / (3000.0 ** (torch.arange(0, dim, 2).float() / dim)))
+    found = []
+    for fused in (False, True):
+        batch, cell, _, layout = paged_case([count + 5 for count in counts], counts, heads, kv_heads, dim, page, dtype, shuffle_seed=rows_seed)
+        generator.manual_seed(rows_seed)
+        weight = (torch.randn(layout.width, inner, generator=generator) * inner ** -0.5).to(dtype)
+        prepared = library.prepare_linear([on_gpu(weight, dtype)], [on_gpu(torch.randn(layout.width, generator=generator), dtype)])
+        if fused:
+            qkv = library.linear_rotated(x, prepared, layout, batch, cell, inverse, "adjacent")
+        else:
+            qkv = torch.empty(rows, layout.width, dtype=dtype, device="cuda")
+            assert library._gemm_blocks.llmserve_gemm_blocks(
+                x.data_ptr(), prepared.weight.data_ptr(), prepared.bias.data_ptr(), 0, qkv.data_ptr(), 0, 0, rows, layout.width, inner, 1, library._stream) == 0
+            library.rotate_and_store(qkv, layout, batch, cell, inverse, "adjacent")
+        found.append((qkv, cell.keys.float().nan_to_num(7e7), cell.values.float().nan_to_num(7e7)))
+    assert all(torch.equal(apart, together) for apart, together in zip(*found))
+
+
 def test_product_rotated_and_stored_refuses_bad_sizes(kernels):
     from llmserve_amd.kernels.hip import _pointer
 
