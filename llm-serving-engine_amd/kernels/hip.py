@@ -212,8 +212,6 @@ class ScaledRows:
 
 
 class HipKernels:
-    brings_ahead = True  # `add_rms_norm` takes the weight of its reader along (`_whole_ahead`)
-
     def __init__(
         self, dtype: torch.dtype = torch.bfloat16, device: str | torch.device = "cuda:0", *, library_products: bool = True,
         shared_portions: str = "auto",
@@ -372,6 +370,8 @@ class HipKernels:
         )
         _check(status, "add_rms_norm")
         return out
+
+    add_rms_norm.takes_ahead = True  # (of this very method: one that a derived library has in its place is called without)
 
     def rotary_table(self, batch, inverse_frequencies: torch.Tensor, magnitude: float = 1.0) -> torch.Tensor:
         """(cos, sin) [T, D/2, 2] float32 of position * frequency for the step's tokens, times `magnitude`.  Every

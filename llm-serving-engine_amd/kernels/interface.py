@@ -32,7 +32,9 @@ class Kernels(Protocol):
     def add_rms_norm(
         self, hidden: torch.Tensor, delta: torch.Tensor | None, weight: torch.Tensor, eps: float
     ) -> torch.Tensor:
-        """`hidden += delta` in place (float32), then rows * rsqrt(mean(rows^2) + eps) * weight in the run dtype."""
+        """`hidden += delta` in place (float32), then rows * rsqrt(mean(rows^2) + eps) * weight in the run dtype.  A method that
+        has the attribute `takes_ahead` set is also called with `ahead` = what `prepare_linear` returned for the product that reads
+        the rows (or None): it may bring that weight into the caches meanwhile; the result is the same."""
 
     def prepare_linear(self, weights: list[torch.Tensor], biases: list[torch.Tensor] | None) -> Any:
         """Concatenates [N_i, K] weights (and biases) along N into whatever layout `linear` wants."""

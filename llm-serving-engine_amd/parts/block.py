@@ -82,7 +82,7 @@ class PreNormBlock(Block):
             self._norm_into = getattr(kernels, "norm_into", None)
         # (a library's norm may take the weight of the product behind it along, to bring it into the caches meanwhile)
         self._ahead = {}
-        if getattr(kernels, "brings_ahead", False) and getattr(type(self.mixer_norm), "forward", None) is RMSNorm.forward:
+        if getattr(type(self.mixer_norm), "forward", None) is RMSNorm.forward:
             self._ahead = {"ahead": getattr(self.mixer, "qkv", None)}
 
     def forward(self, hidden, delta, batch, cell) -> torch.Tensor:

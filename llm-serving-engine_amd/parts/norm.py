@@ -40,10 +40,13 @@ class RMSNorm(Part):
         if spec.weight_scale != 1.0 or spec.weight_offset != 0.0:
             self.weight = ((self.weight.float() + float(spec.weight_offset)) * float(spec.weight_scale)).contiguous()
 
-    def forward(self, hidden: torch.Tensor, delta: torch.Tensor | None, **ahead) -> torch.Tensor:
+    def forward(self, hidden: torch.Tensor, delta: torch.Tensor | None, ahead=None) -> torch.Tensor:
         """Adds `delta` into `hidden` (in place) and returns the normed rows in the run dtype.  `ahead`: the prepared weight that
-        their reader multiplies them with, for a kernel library that can bring it into the caches meanwhile."""
-        return self.kernels.add_rms_norm(hidden, delta, self.weight, self.spec.eps, **ahead)
+        their reader multiplies them with, for a library whose `add_rms_norm` takes it along (`Kernels.add_rms_norm`)."""
+        step = self.kernels.add_rms_norm
+        if ahead is not None and getattr(step, "takes_ahead", False):
+            return step(hidden, delta, self.weight, self.spec.eps, ahead=ahead)
+        return step(hidden, delta, self.weight, self.spec.eps)
 
     def add_normed(self, hidden: torch.Tensor, update: torch.Tensor) -> torch.Tensor:
         """The norm on a sublayer's output instead of its input: `hidden += update * rsqrt(mean(update^2) + eps) *

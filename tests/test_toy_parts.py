@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from llmserve_amd import CacheConfig, ModelRunner, StepEntry
+from llmserve_amd.kernels.hip import HipKernels
 from llmserve_amd.parts import (
     FEED_FORWARDS, MIXERS, NORMS, POSITIONS, Attention, AttentionSpec, FixedState, GatedMLP, GatedMLPSpec, PagedKeyValue, PreNormBlock,
     PreNormBlockSpec, RMSNorm, RMSNormSpec, Rotary, RotarySpec,
@@ -239,3 +240,23 @@ def test_parts_derived_from_those_that_a_library_links_are_asked_as_ever(derived
     linking = LinkingKernels()
     apart, linked = (PreNormBlock(spec, tensors, kernels).forward(hidden.clone(), None, None, None) for kernels in (StubAttention(), linking))
     assert torch.equal(apart, linked) and linking.told == (derived is None)
+
+
+class FourParameters(LinkingKernels, HipKernels):
+    """A library derived from the one for the GPU that has its own steps, as the interface declares them."""
+
+    def __init__(self):
+        LinkingKernels.__init__(self)
+
+
+def one_block(kernels, mixer=None, hidden=None, generator_seed=3):
+    width = 16
+    attention = AttentionSpec(width, 2, 1, 8, 0.3, RotarySpec(8, 100.0), qkv_bias=False)
+    spec = PreNormBlockSpec(RMSNormSpec(width, 1e-6), mixer or attention, RMSNormSpec(width, 1e-6), GatedMLPSpec(width, 24))
+    generator = torch.Generator().manual_seed(generator_seed)
+    tensors = {name: torch.randn(tensor.shape, generator=generator) for name, tensor in PreNormBlock.tensors(spec).items()}
+    return PreNormBlock(spec, tensors, kernels).forward(torch.randn((3, width), generator=generator), None, None, None)
+
+
+def test_a_derived_library_with_a_norm_of_its_own_is_called_as_the_interface_has_it():
+    assert torch.equal(one_block(FourParameters()), one_block(StubAttention()))
