@@ -331,12 +331,20 @@ class HipKernels:
         _check(status, "embedding")
         return out
 
-    @staticmethod
-    def _ahead(weights: LinearWeights | None, busy: int, up_to: int, tiles: int = 1) -> tuple:
+    def _here(self, tensor: torch.Tensor) -> bool:
+        """Whether the tensor lies in the memory of this library's device."""
+        index = self.device.index if self.device.index is not None else torch.cuda.current_device()
+        return tensor.device.type == "cuda" and tensor.device.index == index
+
+    def _ahead(self, weights: Any, busy: int, up_to: int, tiles: int = 1) -> tuple:
         """What a kernel of `busy` workgroups is told of the weight that the next product reads (csrc/common.h: Ahead), which takes
         `tiles` tiles of 16 weight rows a workgroup: (workgroups that bring it into the caches, its address, bytes a run, runs).  As
-        many workgroups as fill the CUs that the others leave idle; the weight's first `up_to` bytes, (0, ...) for nothing."""
-        if weights is None or weights.weight.dtype != torch.bfloat16 or not _in_pieces(weights.weight) or weights.in_features % 8 or busy >= 256:
+        many workgroups as fill the CUs that the others leave idle; the weight's first `up_to` bytes, (0, ...) for nothing.  Nothing of what
+        another library prepared, and of weights that lie elsewhere (a library derived from this one may bring them when it multiplies)."""
+        if (
+            not isinstance(weights, LinearWeights) or weights.weight.dtype != torch.bfloat16 or not self._here(weights.weight)
+            or not _in_pieces(weights.weight) or weights.in_features % 8 or busy >= 256
+        ):
             return 0, None, 0, 0
         stripe = 32 * tiles * weights.in_features
         stripes = min(weights.out_features // (16 * tiles), up_to // stripe)
@@ -353,8 +361,8 @@ class HipKernels:
     # 1.353 1.385.  Beside the projection that has no splits to merge (4.8 us) 8 MB gain nothing and 16 lose 3 %.
     _MERGING_AHEAD = 30 << 20
 
-    def _whole_ahead(self, weights: LinearWeights | None, rows: int, busy: int) -> tuple:
-        if weights is None or rows > 64 or weights.weight.numel() * weights.weight.element_size() > self._WHOLE_AHEAD:
+    def _whole_ahead(self, weights: Any, rows: int, busy: int) -> tuple:
+        if not isinstance(weights, LinearWeights) or rows > 64 or weights.weight.numel() * weights.weight.element_size() > self._WHOLE_AHEAD:
             return 0, None, 0, 0
         return self._ahead(weights, busy, self._WHOLE_AHEAD)
 

@@ -27,6 +27,12 @@ class Mixer(Part):
 
     joins: ClassVar[bool] = False
 
+    @property
+    def first_product(self) -> Any:
+        """What `prepare_linear` returned for the product that `forward` begins with, if it begins with one, for whoever may bring that
+        weight into the caches before; None: nothing is said of it."""
+        return None
+
     def forward(self, x: torch.Tensor, batch, cell) -> torch.Tensor:
         raise NotImplementedError
 
@@ -96,6 +102,10 @@ class Attention(Mixer):
         own = {name[len("position."):]: tensor for name, tensor in tensors.items() if name.startswith("position.")}
         self.position = POSITIONS.build(spec.position, own, kernels)
         self.replayable = self.position.replayable
+
+    @property
+    def first_product(self) -> Any:
+        return self.qkv if type(self).forward is Attention.forward else None
 
     @property
     def takes_into(self) -> bool:

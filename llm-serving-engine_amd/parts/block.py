@@ -8,6 +8,7 @@ from typing import Any
 
 import torch
 
+from .attention import Mixer
 from .base import BLOCKS, FEED_FORWARDS, MIXERS, NORMS, CacheNeed, Part, TensorSpec, prefixed, side_by_side, under
 from .feed_forward import GatedMLP
 from .norm import RMSNorm
@@ -81,12 +82,11 @@ class PreNormBlock(Block):
         if getattr(self.mixer, "takes_into", False) and as_they_stand:
             self._norm_into = getattr(kernels, "norm_into", None)
         # (a library's norm may take the weight of the product behind it along, to bring it into the caches meanwhile)
-        self._ahead = {}
-        if getattr(type(self.mixer_norm), "forward", None) is RMSNorm.forward:
-            self._ahead = {"ahead": getattr(self.mixer, "qkv", None)}
+        self._tells_ahead = getattr(type(self.mixer_norm), "forward", None) is RMSNorm.forward and isinstance(self.mixer, Mixer)
 
     def forward(self, hidden, delta, batch, cell) -> torch.Tensor:
-        normed = self.mixer_norm.forward(hidden, delta, **self._ahead)
+        ahead = {"ahead": self.mixer.first_product} if self._tells_ahead else {}
+        normed = self.mixer_norm.forward(hidden, delta, **ahead)
         if self._norm_into is not None:
             norm = self.feed_forward_norm
             mixed = self.mixer.forward(normed, batch, cell, into=self._norm_into(hidden, norm.weight, norm.spec.eps, self.feed_forward.gate_up))

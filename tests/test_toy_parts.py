@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from llmserve_amd import CacheConfig, ModelRunner, StepEntry
-from llmserve_amd.kernels.hip import HipKernels
+from llmserve_amd.kernels.hip import HipKernels, LinearWeights
 from llmserve_amd.parts import (
     FEED_FORWARDS, MIXERS, NORMS, POSITIONS, Attention, AttentionSpec, FixedState, GatedMLP, GatedMLPSpec, PagedKeyValue, PreNormBlock,
     PreNormBlockSpec, RMSNorm, RMSNormSpec, Rotary, RotarySpec,
@@ -260,3 +260,44 @@ def one_block(kernels, mixer=None, hidden=None, generator_seed=3):
 
 def test_a_derived_library_with_a_norm_of_its_own_is_called_as_the_interface_has_it():
     assert torch.equal(one_block(FourParameters()), one_block(StubAttention()))
+
+
+class AskingKernels(FourParameters):
+    """Asks for a weight ahead of its reader as the library for the GPU does, which on this machine has none to bring."""
+
+    asked = ()
+
+    def add_rms_norm(self, hidden, delta, weight, eps, ahead=None):
+        self.asked += (ahead,)
+        assert self._whole_ahead(ahead, hidden.shape[0], hidden.shape[0]) == (0, None, 0, 0)
+        return super().add_rms_norm(hidden, delta, weight, eps)
+
+    add_rms_norm.takes_ahead = True
+
+
+class ForeignMixer(Attention):
+    """A mixer that calls something else `qkv`."""
+
+    def __init__(self, spec, tensors, kernels):
+        super().__init__(spec, tensors, kernels)
+        self.rows, self.qkv = self.qkv, "which heads are queries, keys and values"
+
+    def forward(self, x, batch, cell):
+        return self.kernels.linear(self.kernels.linear(x, self.rows)[:, : x.shape[1]].contiguous(), self.out, torch.float32)
+
+
+def test_a_library_is_told_of_the_product_that_a_mixer_names(monkeypatch):
+    monkeypatch.setitem(MIXERS._classes, "ForeignMixer", ForeignMixer)
+    foreign = AttentionSpec(16, 2, 1, 8, 0.3, RotarySpec(8, 100.0), qkv_bias=False, kind="ForeignMixer")
+    for mixer, named in ((None, True), (foreign, False)):
+        kernels = AskingKernels()
+        assert torch.equal(one_block(kernels, mixer), one_block(StubAttention(), mixer))
+        assert [ahead is not None for ahead in kernels.asked] == [named, False]  # (the second norm's reader is told of otherwise)
+
+
+def test_nothing_is_brought_of_what_lies_elsewhere_or_is_none_of_the_librarys():
+    library = object.__new__(HipKernels)
+    library.device = torch.device("cuda:0")
+    here = LinearWeights(torch.empty((2048, 1536), dtype=torch.bfloat16), None)
+    for weights in (here, LinearWeights(here.weight.to("meta"), None), None, "qkv", object(), here.weight):
+        assert library._whole_ahead(weights, 1, 1) == (0, None, 0, 0) and library._ahead(weights, 1, 1 << 24, 4) == (0, None, 0, 0)
