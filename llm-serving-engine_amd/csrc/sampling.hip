@@ -92,17 +92,17 @@ __device__ __forceinline__ void block_argmax(const float* row, int n, float* bes
 
 // Two stages, so that a few rows still fill the chip: each row is cut into `pieces` pieces,
 // a block finds the first maximum of its piece, and one more block per row picks among them.
-// `zero` (may be null): `zero_words` words that the launch clears, for whoever runs after it.
+// `zero` (may be null): for every row, `zero_words` words that the launch clears, `zero_stride` apart, for whoever runs after it.
 __global__ __launch_bounds__(SAMPLE_THREADS) void argmax_pieces_kernel(const float* __restrict__ logits,
                                                                        float* __restrict__ piece_values,
                                                                        int* __restrict__ piece_indices, int vocab,
                                                                        int pieces, unsigned* __restrict__ zero,
-                                                                       size_t zero_words) {
+                                                                       size_t zero_stride, int zero_words) {
   __shared__ float sv[17];
   __shared__ int si[17];
   if (zero != nullptr) {
-    const size_t block = (size_t)blockIdx.y * gridDim.x + blockIdx.x, blocks = (size_t)gridDim.x * gridDim.y;
-    for (size_t i = block * blockDim.x + threadIdx.x; i < zero_words; i += blocks * blockDim.x) zero[i] = 0u;
+    unsigned* mine = zero + blockIdx.x * zero_stride;
+    for (int i = blockIdx.y * blockDim.x + threadIdx.x; i < zero_words; i += gridDim.y * blockDim.x) mine[i] = 0u;
   }
   const int per = (vocab + pieces - 1) / pieces;
   const int begin = min(vocab, (int)blockIdx.y * per), count = min(vocab, begin + per) - begin;
@@ -166,7 +166,7 @@ extern "C" int llmserve_argmax(const float* logits, float* piece_values, int* pi
   if (vocab <= 0) return ERR_BAD_ARGUMENT;
   const int pieces = argmax_pieces(rows);
   hipLaunchKernelGGL(argmax_pieces_kernel, dim3(rows, pieces), dim3(SAMPLE_THREADS), 0, stream, logits,
-                     piece_values, piece_indices, vocab, pieces, (unsigned*)nullptr, (size_t)0);
+                     piece_values, piece_indices, vocab, pieces, (unsigned*)nullptr, (size_t)0, 0);
   hipLaunchKernelGGL(argmax_pick_kernel, dim3(rows), dim3(WAVE), 0, stream, piece_values, piece_indices, out, pieces);
   return LAUNCH_STATUS();
 }
@@ -208,7 +208,7 @@ extern "C" int llmserve_argmax_static(const float* logits, int* out, int rows, i
   int* piece_indices = (int*)((unsigned char*)base + ARGMAX_STATIC_SLOTS * sizeof(float));
   const int pieces = argmax_pieces(rows);
   hipLaunchKernelGGL(argmax_pieces_kernel, dim3(rows, pieces), dim3(SAMPLE_THREADS), 0, stream, logits,
-                     piece_values, piece_indices, vocab, pieces, (unsigned*)nullptr, (size_t)0);
+                     piece_values, piece_indices, vocab, pieces, (unsigned*)nullptr, (size_t)0, 0);
   hipLaunchKernelGGL(argmax_pick_kernel, dim3(rows), dim3(WAVE), 0, stream, piece_values, piece_indices, out, pieces);
   return LAUNCH_STATUS();
 }
@@ -218,7 +218,7 @@ extern "C" int llmserve_argmax_static(const float* logits, int* out, int rows, i
 //
 // Every launch but the last cuts a row into `pieces` contiguous pieces, a block a (row, piece), so that a few rows of a large
 // vocabulary use the whole chip: the row's argmax; p and its sums; with top-p, the entries that the choice is among.  In the last one
-// a block a row chooses the token.
+// a block a row chooses the token, or a few blocks where a row leaves many to choose among.
 //
 // Top-p needs, twice, the smallest float t with mass_above(t) below a bound, where mass_above(t) is the
 // sum of the entries of p greater than t: first the value at which the kept set ends (bound top_p * Z,
@@ -229,12 +229,19 @@ extern "C" int llmserve_argmax_static(const float* logits, int* out, int rows, i
 // After three levels the bucket is one value.  Both searches start from the same first histogram, which the
 // blocks of the second launch make together.  What the later levels look at are the entries of a few of its bins, an eighth
 // of an octave each: the one in which the kept set ends, and those in which u can fall, as the kept mass lies between the
-// first bound and the end of that bin beyond it.  The third launch lists those entries (of a row of 151,936 some
-// thousands), the row's block has them in registers and does all levels by itself.  A launch a level, of many blocks a row, took 8.6 us for
-// each of the four levels behind the first, most of it launch, trips to memory and atomic additions: 1 / 8 / 16 / 32 / 64
-// rows of 151,936 with top-p 45.1 / 54.4 / 62.0 / 71.7 / 97.6 -> 30.1 / 38.1 / 45.0 / 48.6 / 64.4 us; logits of a third of the spread at
-// temperature 1.5, which list some twenty thousand, 46.8 / 55.2 / 63.7 / 76.4 / 102.8 -> 46.3 / 53.6 / 63.1 / 68.3 / 83.2; rows of
-// nothing but equal entries, which list all, 63 / 87 / 131 / 215 / 381 -> 130 / 141 / 143 / 159 / 220.  What is left is four launches that wait for one another.
+// first bound and the end of that bin beyond it.  The third launch lists those entries (of a row of 151,936 whose logits have a spread of three
+// some hundreds) and the row's block has them in registers and does all levels by itself.  Where they are more than 8,192 (small spreads,
+// high temperatures, equal entries), the third launch adds up their second level instead, of up to three bins, and of the last launch up to
+// sixteen blocks a row gather what lies in the one or two of its 1,024 runs that are left and add up the third level; the one that is done last
+// goes on with the block's part.  So one block never goes through all of a row but for the place of one among a thousand equal entries.
+// Us a call in a captured chain, 1 / 8 / 16 / 32 / 64 / 256 rows of 151,936: a launch a level, of many blocks a row | lists of any length,
+// searched by one block | this:
+//   spread 3, temperature 0.8, top-p 0.9   43 54 61 73 99 317   | 30 38 45 50 65 376     | 31 38 42 48 60 156
+//   spread 1, temperature 1.5 (20,000)     44 54 63 77 104      | 46 59 66 70 89         | 40 47 57 68 87
+//   spread 0.01 (nearly all)               49 62 76 104 155 523 | 162 195 218 263 324 977 | 43 57 69 93 137 394
+//   equal entries                          62 86 130 215 383    | 129 141 144 160 221    | 61 66 81 111 170
+//   two values                             52 65 90 137 229     | 244 254 262 300 353    | 62 65 77 104 152
+// What is left is four launches that wait for one another.
 //
 // The entries of a bin share their exponent (it lies in the ten bits that are fixed first), so their
 // sum is 2^exponent times the sum of their 24-bit significands, an integer below 2^42: a bin's mass is
@@ -245,7 +252,8 @@ extern "C" int llmserve_argmax_static(const float* logits, int* out, int rows, i
 #define SAMPLE_BINS 1024
 #define SAMPLE_LEVEL_BITS 10
 #define SAMPLE_PIECES_MAX 64  // a wave looks at a row's pieces, a lane at each
-#define SAMPLE_KEPT 8         // listed entries that a thread of the row's block keeps in registers; further ones are read again at every level
+#define SAMPLE_KEPT 8         // listed entries that a thread of the row's block keeps in registers
+#define SAMPLE_LIST (SAMPLE_KEPT * SAMPLE_THREADS)
 
 // About 512 blocks of 512 threads in all for top-p, where every piece adds its bins to the row's with atomic additions of
 // its own (64 rows: 98 us, 110 with twice as many; 16 rows 61 and 81; 256 threads and 2,048 blocks 121 and 69), and twice as
@@ -255,6 +263,10 @@ static int sample_pieces(int rows, bool with_top_p) {
   while (pieces > 4 && rows * pieces > (with_top_p ? 512 : 1024)) pieces /= 2;
   return pieces;
 }
+
+// How many blocks of the last launch a row with many candidates has: what fills the chip once, as further ones only wait (spread 0.01, 16 / 64
+// rows: 256 blocks in all 69.4 / 137 us, one a row 77.5 / 138; two values 77 / 153 and 165 / 219).  A row with few leaves all but the first at once.
+static int pick_parts(int rows) { return rows >= 256 ? 1 : rows > 16 ? 256 / rows : 16; }
 
 __device__ __forceinline__ int level_shift(int level) { return (2 - level) * SAMPLE_LEVEL_BITS; }
 
@@ -270,7 +282,7 @@ __device__ __forceinline__ int binary_exponent_of(unsigned pattern) {
 // The mass above the end of each of the 1,024 bins of one level, to `above` (LDS): that of the bucket, `start`, and of the bins
 // after it.  `sums`: the histogram; `base`: the bucket's first pattern.  THREADS threads, a run of bins each; waves: a double of LDS a wave.
 template <int THREADS>
-__device__ void masses_above(const unsigned long long* sums, unsigned base, int level, double start, double* above, double* waves) {
+__device__ __forceinline__ void masses_above(const unsigned long long* sums, unsigned base, int level, double start, double* above, double* waves) {
   constexpr int EACH = SAMPLE_BINS / THREADS;
   const int t = threadIdx.x, lane = t % WAVE, wave = t / WAVE;
   double mass[EACH], inclusive = 0.0;
@@ -320,11 +332,40 @@ __device__ __forceinline__ int lowest_bin(const double* above, double limit, boo
 // Which bins of the first histogram a row's choice is among, and the bound at which its kept set ends.
 struct Candidates {
   double limit;                     // top_p * Z
+  double above_cut;                 // the mass above `cut_bin`, as it met the bound: a search inside the bin begins from it
   int cut_bin, first_bin, last_bin;  // the kept set ends in the first of them, u falls in one of the run between the others
+  int many;                         // whether they hold more entries than a list: then their second level is made instead
   __device__ __forceinline__ bool has(unsigned bin) const {
     return bin == (unsigned)cut_bin || (bin >= (unsigned)first_bin && bin <= (unsigned)last_bin);
   }
+  // which second-level histogram is the bin's; -1 for the bins inside the run, which hold an entry at most: they begin above the cut, and u's
+  // two bounds lie less than a value of the cut bin apart
+  __device__ __forceinline__ int slot(int bin) const { return bin == cut_bin ? 0 : bin == first_bin ? 1 : bin == last_bin ? 2 : -1; }
 };
+
+// What the launches share of a row with top-p.  The first launch clears it up to the list, the second the second level, the third, where it
+// makes that one, the third level.
+#define SAMPLE_SLOTS 3
+#define SAMPLE_FEW 1024
+struct SampleRow {
+  unsigned listed;  // how many entries are listed
+  unsigned found, done;  // of a row with many candidates: how many entries are in `few` or would be, parts of the row that are done
+  unsigned unused[61];
+  unsigned long long sums[SAMPLE_BINS];  // the first histogram
+  unsigned counts[SAMPLE_BINS];
+  union {
+    uint2 list[SAMPLE_LIST];  // pattern and index of the candidates, in no order
+    struct {
+      unsigned long long fine_sums[SAMPLE_SLOTS][SAMPLE_BINS];  // or the second level of their bins,
+      unsigned fine_counts[SAMPLE_SLOTS][SAMPLE_BINS];
+      unsigned long long run_sums[2][SAMPLE_BINS];  // the third of one or two runs of a second one,
+      unsigned run_counts[2][SAMPLE_BINS];
+      uint2 few[SAMPLE_FEW];  // and the entries of those runs
+    };
+  };
+  Candidates candidates;
+};
+#define SAMPLE_CLEARED offsetof(SampleRow, list)
 
 __device__ __forceinline__ void clear_histogram(unsigned long long* lds_sums, unsigned* lds_counts) {
   for (int i = threadIdx.x; i < SAMPLE_BINS; i += blockDim.x) {
@@ -359,10 +400,34 @@ __device__ __forceinline__ void add_entry(float value, unsigned bucket, int shif
   }
 }
 
-// Adds what the block has gathered of its piece to the row's histogram (a barrier before).
-__device__ __forceinline__ void give_histogram(const unsigned long long* lds_sums, const unsigned* lds_counts,
+// Adds a lane's entry to a histogram in LDS, where `mine`; all lanes of the wave that are here together.  Additions to one place wait for one
+// another, so entries that are equal in many lanes (a row of equal entries, or of a few values) go together, two values a time.
+__device__ __forceinline__ void add_equal_together(bool mine, unsigned pattern, unsigned bin, unsigned long long* sums, unsigned* counts) {
+  const int lane = threadIdx.x % WAVE;
+#pragma unroll
+  for (int turn = 0; turn < 2; ++turn) {
+    const unsigned long long left = __ballot(mine);
+    if (left == 0ull) return;
+    const int leader = __ffsll((long long)left) - 1;
+    const unsigned long long same = __ballot(mine && pattern == (unsigned)__builtin_amdgcn_readlane((int)pattern, leader));
+    const int equal = __popcll(same);
+    if (equal < 4) break;
+    if (lane == leader) {
+      atomicAdd(sums + bin, significand_of(pattern) * (unsigned long long)equal);
+      atomicAdd(counts + bin, (unsigned)equal);
+    }
+    if ((same >> lane) & 1ull) mine = false;
+  }
+  if (mine) {
+    atomicAdd(sums + bin, significand_of(pattern));
+    atomicAdd(counts + bin, 1u);
+  }
+}
+
+// Adds what the block has gathered of its piece to the row's histogram of `bins` bins (a barrier before).
+__device__ __forceinline__ void give_histogram(const unsigned long long* lds_sums, const unsigned* lds_counts, int bins,
                                                unsigned long long* __restrict__ sums, unsigned* __restrict__ counts) {
-  for (int bin = threadIdx.x; bin < SAMPLE_BINS; bin += blockDim.x) {
+  for (int bin = threadIdx.x; bin < bins; bin += blockDim.x) {
     const unsigned count = lds_counts[bin];
     if (count != 0u) {
       atomicAdd(sums + bin, lds_sums[bin]);
@@ -371,16 +436,13 @@ __device__ __forceinline__ void give_histogram(const unsigned long long* lds_sum
   }
 }
 
-// The layout of what the launches share, per row: the first histogram (cleared by the first launch), p and its pieces' sums.
+// What the launches share: p, whose rows begin `stride` entries apart (a multiple of four), its pieces' sums, and what rows with top-p need.
 struct SampleBuffers {
-  float* p;                     // [rows, vocab]
-  double* piece_sums;           // [rows, pieces]
-  unsigned long long* sums;     // [rows, SAMPLE_BINS]
-  unsigned* counts;             // [rows, SAMPLE_BINS]
-  unsigned* listed;             // [rows]: how many entries are listed (cleared by the first launch)
-  uint2* list;                  // [rows, vocab]: pattern and index of each, in no order
-  Candidates* candidates;       // [rows]
-  const float* piece_values;    // [rows, argmax_pieces]
+  float* p;
+  size_t stride;
+  double* piece_sums;         // [rows, pieces]
+  SampleRow* rows;            // null where no row has top-p
+  const float* piece_values;  // [rows, argmax_pieces]
   const int* piece_indices;
 };
 
@@ -409,12 +471,16 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_exp_kernel(const float* _
   const float temperature = temperatures[r];
   if (temperature <= 0.f) return;  // engine.py:30-31: the argmax stands
   const float* row = logits + (size_t)r * vocab;
-  float* p = buffers.p + (size_t)r * vocab;
+  float* p = buffers.p + r * buffers.stride;
   const int per = (vocab + pieces - 1) / pieces;
   const int begin = min(vocab, piece * per), end = min(vocab, begin + per);
   const bool with_histogram = with_top_p && top_ps[r] < 1.f;
   const float top_logit = row[best_index] / temperature;
   double partial = 0.0;
+  if (with_histogram) {
+    unsigned* fine = (unsigned*)buffers.rows[r].fine_sums;
+    for (int i = piece * SAMPLE_BLOCK + threadIdx.x; i < SAMPLE_SLOTS * SAMPLE_BINS * 3; i += pieces * SAMPLE_BLOCK) fine[i] = 0u;
+  }
   for (int first = begin + threadIdx.x; first < end; first += SAMPLE_BATCH * SAMPLE_BLOCK) {
     const Batch batch = load_batch(row, first, end);
 #pragma unroll
@@ -430,7 +496,7 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_exp_kernel(const float* _
   const double sum = block_sum_f64(partial, sd);  // (its barriers stand between the additions and what reads them)
   if (threadIdx.x == 0) buffers.piece_sums[r * pieces + piece] = sum;
   if (!with_histogram) return;
-  give_histogram(lds_sums, lds_counts, buffers.sums + (size_t)r * SAMPLE_BINS, buffers.counts + (size_t)r * SAMPLE_BINS);
+  give_histogram(lds_sums, lds_counts, SAMPLE_BINS, buffers.rows[r].sums, buffers.rows[r].counts);
 }
 
 // Sums of v over the threads before this one, in thread order.  shared: at least 16 of its kind.
@@ -467,171 +533,326 @@ __device__ __forceinline__ int block_sum_before_int(int v, int* shared) {
   return before + inclusive - v;
 }
 
-// Lists the entries that the choice of a row with top-p is among: a block takes its piece's.
+// Lists the entries that the choice of a row with top-p is among, or, where they are more than a list holds, adds them up by the second
+// ten bits: a block takes its piece's.
 __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_list_kernel(const float* __restrict__ temperatures, const float* __restrict__ top_ps,
                                                                    const float* __restrict__ uniforms, SampleBuffers buffers, int vocab,
                                                                    int pieces) {
   __shared__ double above[SAMPLE_BINS], waves[SAMPLE_BLOCK / WAVE], sums_here[SAMPLE_PIECES_MAX];
+  __shared__ unsigned long long fine_sums[SAMPLE_SLOTS * SAMPLE_BINS];
+  __shared__ unsigned fine_counts[SAMPLE_SLOTS * SAMPLE_BINS];
   __shared__ int lowest;
-  __shared__ unsigned found, place;
+  __shared__ unsigned candidates, found, place;
+  constexpr unsigned STAGE = SAMPLE_SLOTS * SAMPLE_BINS;
+  uint2* stage = (uint2*)fine_sums;  // (a row has a list or the second level)
   const int r = blockIdx.x, piece = blockIdx.y, t = threadIdx.x;
   const float top_p = top_ps[r];
   if (temperatures[r] <= 0.f || top_p >= 1.f) return;
+  SampleRow& row = buffers.rows[r];
   const int per = (vocab + pieces - 1) / pieces;
   const int begin = min(vocab, piece * per), end = min(vocab, begin + per);
-  const float* p = buffers.p + (size_t)r * vocab;
+  const float* p = buffers.p + r * buffers.stride;
   Batch batch = load_batch(p, begin + t, end);  // under way while the histogram is looked at
   if (t < pieces) sums_here[t] = buffers.piece_sums[r * pieces + t];  // a thread a piece asks, then everybody adds them in order
-  if (t == 0) found = 0u;
-  masses_above<SAMPLE_BLOCK>(buffers.sums + (size_t)r * SAMPLE_BINS, 0u, 0, 0.0, above, waves);
+  if (t == 0) candidates = found = 0u;
+  unsigned in_bin[SAMPLE_BINS / SAMPLE_BLOCK];
+#pragma unroll
+  for (int j = 0; j < SAMPLE_BINS / SAMPLE_BLOCK; ++j) in_bin[j] = row.counts[t + j * SAMPLE_BLOCK];
+  masses_above<SAMPLE_BLOCK>(row.sums, 0u, 0, 0.0, above, waves);
   double total = 0.0;
   for (int q = 0; q < pieces; ++q) total += sums_here[q];
   Candidates c;
   // the bound is strict, so a bound of 0 would be met nowhere: the least positive one keeps the maximum alone
   c.limit = fmax((double)top_p * total, 2.2250738585072014e-308);
   c.cut_bin = lowest_bin<SAMPLE_BLOCK>(above, c.limit, true, &lowest);
-  // the kept mass is at least the bound, and beyond it by less than a value of that bin (up to rounding, which the row's block sees to)
+  c.above_cut = above[c.cut_bin];
+  // the kept mass is at least the bound, and beyond it by less than a value of that bin (up to rounding, which the row's block sees to);
+  // and what is chosen is not below the cut
   const double end_of_bin = (double)__uint_as_float((unsigned)(c.cut_bin + 1) << level_shift(0)), u = (double)uniforms[r];
   __syncthreads();
-  c.first_bin = lowest_bin<SAMPLE_BLOCK>(above, u * (c.limit + end_of_bin), false, &lowest);
+  c.first_bin = max(c.cut_bin, lowest_bin<SAMPLE_BLOCK>(above, u * (c.limit + end_of_bin), false, &lowest));
   __syncthreads();
-  c.last_bin = lowest_bin<SAMPLE_BLOCK>(above, u * c.limit, false, &lowest);
-  if (piece == 0 && t == 0) buffers.candidates[r] = c;
-  // count them, ask for a place in the row's list, and write them there
-  auto taken = [&](int i, float v) { return i < end && c.has(__float_as_uint(v) >> level_shift(0)); };
-  unsigned mine = 0u;
-  for (int first = begin + t; first < end; first += SAMPLE_BATCH * SAMPLE_BLOCK) {
-    if (first != begin + t) batch = load_batch(p, first, end);
+  c.last_bin = max(c.cut_bin, lowest_bin<SAMPLE_BLOCK>(above, u * c.limit, false, &lowest));
 #pragma unroll
-    for (int k = 0; k < SAMPLE_BATCH; ++k) mine += taken(first + k * SAMPLE_BLOCK, batch.v[k]) ? 1u : 0u;
-  }
-  if (mine != 0u) mine = atomicAdd(&found, mine);  // (where this thread's begin)
+  for (int j = 0; j < SAMPLE_BINS / SAMPLE_BLOCK; ++j)
+    if (c.has(t + j * SAMPLE_BLOCK) && in_bin[j] != 0u) atomicAdd(&candidates, in_bin[j]);
   __syncthreads();
-  if (found == 0u) return;
-  if (t == 0) place = atomicAdd(buffers.listed + r, found);
-  __syncthreads();
-  uint2* list = buffers.list + (size_t)r * vocab + place;
-  const bool again = begin + SAMPLE_BATCH * SAMPLE_BLOCK < end;  // more than one batch: the first is not here any more
-  for (int first = begin + t; first < end; first += SAMPLE_BATCH * SAMPLE_BLOCK) {
-    if (again) batch = load_batch(p, first, end);
+  c.many = candidates > SAMPLE_LIST ? 1 : 0;
+  if (piece == 0 && t == 0) row.candidates = c;
+
+  if (c.many) {
+    for (int i = t; i < SAMPLE_SLOTS * SAMPLE_BINS; i += SAMPLE_BLOCK) fine_sums[i] = 0ull, fine_counts[i] = 0u;
+    unsigned* runs = (unsigned*)row.run_sums;
+    for (int i = piece * SAMPLE_BLOCK + t; i < 2 * SAMPLE_BINS * 3; i += pieces * SAMPLE_BLOCK) runs[i] = 0u;
+    __syncthreads();
+    for (int first = begin + t; first < end; first += SAMPLE_BATCH * SAMPLE_BLOCK) {
+      if (first != begin + t) batch = load_batch(p, first, end);
 #pragma unroll
-    for (int k = 0; k < SAMPLE_BATCH; ++k) {
-      const int i = first + k * SAMPLE_BLOCK;
-      if (taken(i, batch.v[k])) list[mine++] = make_uint2(__float_as_uint(batch.v[k]), (unsigned)i);
+      for (int k = 0; k < SAMPLE_BATCH; ++k) {
+        const unsigned pattern = __float_as_uint(batch.v[k]);
+        const int slot = first + k * SAMPLE_BLOCK < end ? c.slot((int)(pattern >> level_shift(0))) : -1;
+        const int bin = max(slot, 0) * SAMPLE_BINS + (int)((pattern >> level_shift(1)) & (SAMPLE_BINS - 1));
+        add_equal_together(slot >= 0, pattern, bin, fine_sums, fine_counts);
+      }
     }
+    __syncthreads();
+    give_histogram(fine_sums, fine_counts, SAMPLE_SLOTS * SAMPLE_BINS, row.fine_sums[0], row.fine_counts[0]);
+    return;
   }
+  // They are gathered here, and go to a run of the row's list together; what does not fit here (a piece that holds most of them) is gone through
+  // again.  The list holds them all, as the first histogram has counted them.
+  auto gather = [&](auto f) {
+    for (int first = begin + t; first < end; first += SAMPLE_BATCH * SAMPLE_BLOCK) {
+#pragma unroll
+      for (int k = 0; k < SAMPLE_BATCH; ++k) {
+        const int i = first + k * SAMPLE_BLOCK;
+        if (i < end && c.has(__float_as_uint(batch.v[k]) >> level_shift(0))) f(atomicAdd(&found, 1u), make_uint2(__float_as_uint(batch.v[k]), (unsigned)i));
+      }
+      batch = load_batch(p, first + SAMPLE_BATCH * SAMPLE_BLOCK, end);
+    }
+  };
+  gather([&](unsigned at, uint2 entry) {
+    if (at < STAGE) stage[at] = entry;
+  });
+  __syncthreads();
+  const unsigned here = found;
+  if (here == 0u) return;
+  if (t == 0) place = atomicAdd(&row.listed, here);
+  __syncthreads();
+  if (here <= STAGE) {
+    for (unsigned i = t; i < here; i += SAMPLE_BLOCK)
+      if (place + i < SAMPLE_LIST) row.list[place + i] = stage[i];
+    return;
+  }
+  if (t == 0) found = 0u;
+  batch = load_batch(p, begin + t, end);
+  __syncthreads();
+  gather([&](unsigned at, uint2 entry) {
+    if (place + at < SAMPLE_LIST) row.list[place + at] = entry;
+  });
 }
 
-// The token of a row with top-p (out holds the argmax already), by the row's block; see the head of this section.
-__device__ void sample_top_p(const SampleBuffers& buffers, int r, float uniform, int vocab, int* __restrict__ out) {
-  __shared__ double above[SAMPLE_BINS], first_above[SAMPLE_BINS], waves[SAMPLE_THREADS / WAVE];
-  __shared__ unsigned long long sums[SAMPLE_BINS];
-  __shared__ unsigned counts[SAMPLE_BINS];
+// The token of a row with top-p (out holds the argmax already), by the row's block or blocks; see the head of this section.  Bound by trips to memory, barriers
+// and code that is fetched for the first time, one after the other: a row of 151,936 with a short list 14 us, with a long one 24.
+__device__ __forceinline__ void sample_top_p(const SampleBuffers& buffers, int r, float uniform, int vocab, int* __restrict__ out) {
+  constexpr int T = SAMPLE_THREADS;
+  __shared__ double above[SAMPLE_BINS], first_above[SAMPLE_BINS], fine_above[SAMPLE_BINS], waves[T / WAVE];
+  __shared__ unsigned long long sums[2 * SAMPLE_BINS];
+  __shared__ unsigned counts[2 * SAMPLE_BINS];
+  __shared__ uint2 stage[SAMPLE_FEW];
+  __shared__ unsigned found, place;
   __shared__ int lowest, before_lowest, scan[17];
   const int t = threadIdx.x, lane = t % WAVE;
-  const float* p = buffers.p + (size_t)r * vocab;
-  const uint2* list = buffers.list + (size_t)r * vocab;
-  const int n = (int)buffers.listed[r];
-  const Candidates c = buffers.candidates[r];
-  uint2 kept[SAMPLE_KEPT];
+  const float* p = buffers.p + r * buffers.stride;
+  SampleRow& row = buffers.rows[r];
+  const Candidates c = row.candidates;
+  const unsigned listed = row.listed;
+  const double u = (double)uniform;
+  uint2 kept[SAMPLE_KEPT];  // (the pattern ~0u: no entry)
+  int n = 0;  // how many of the block's
+  auto keep = [&](const uint2* list, int entries) __attribute__((always_inline)) {
+    n = entries;
 #pragma unroll
-  for (int k = 0; k < SAMPLE_KEPT; ++k) kept[k] = t + k * SAMPLE_THREADS < n ? list[t + k * SAMPLE_THREADS] : make_uint2(~0u, 0u);
-  masses_above<SAMPLE_THREADS>(buffers.sums + (size_t)r * SAMPLE_BINS, 0u, 0, 0.0, first_above, waves);
-  bool listed = true;  // whether the entries that a search looks at are in the list
-  // calls f(pattern, index) for every entry, of the list (and for none, whose pattern is no entry's) or of the row
-  auto each = [&](auto f) {
-    if (listed) {
-#pragma unroll
-      for (int k = 0; k < SAMPLE_KEPT; ++k) f(kept[k].x, (int)kept[k].y);
-      for (int first = t + SAMPLE_KEPT * SAMPLE_THREADS; first < n; first += SAMPLE_KEPT * SAMPLE_THREADS) {
-        uint2 more[SAMPLE_KEPT];
-#pragma unroll
-        for (int k = 0; k < SAMPLE_KEPT; ++k) more[k] = list[min(first + k * SAMPLE_THREADS, n - 1)];
-#pragma unroll
-        for (int k = 0; k < SAMPLE_KEPT; ++k) f(first + k * SAMPLE_THREADS < n ? more[k].x : ~0u, (int)more[k].y);
-      }
-    } else {
-      for (int first = t; first < vocab; first += SAMPLE_KEPT * SAMPLE_THREADS) {
-        float more[SAMPLE_KEPT];
-#pragma unroll
-        for (int k = 0; k < SAMPLE_KEPT; ++k) more[k] = p[min(first + k * SAMPLE_THREADS, vocab - 1)];
+    for (int k = 0; k < SAMPLE_KEPT; ++k) kept[k] = t + k * T < n ? list[t + k * T] : make_uint2(~0u, 0u);
+  };
+  keep(row.list, (int)min(listed, (unsigned)SAMPLE_LIST));  // (none of a row with many candidates)
+  if (blockIdx.y > 0 && !c.many) return;
+  masses_above<T>(row.sums, 0u, 0, 0.0, first_above, waves);
+  // calls f(pattern, index) for the entries that are kept or, where what is looked for may be none of them, for the whole row, a part at a time
+  bool from_row = false;
+  auto each = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll 1
+    for (unsigned first = t; first < (unsigned)(from_row ? vocab : T); first += SAMPLE_KEPT * T) {
+      if (from_row) {
 #pragma unroll
         for (int k = 0; k < SAMPLE_KEPT; ++k)
-          f(first + k * SAMPLE_THREADS < vocab ? __float_as_uint(more[k]) : ~0u, first + k * SAMPLE_THREADS);
+          kept[k] = first + k * T < (unsigned)vocab ? make_uint2(__float_as_uint(p[first + k * T]), first + k * T) : make_uint2(~0u, 0u);
+      }
+      const int here = from_row ? SAMPLE_KEPT * T : n;
+#pragma unroll
+      for (int k = 0; k < SAMPLE_KEPT; ++k) {
+        if (k * T >= here) break;  // (most lists are short, and code that is not reached is not waited for)
+        f(kept[k].x, (int)kept[k].y);
       }
     }
   };
-  // levels 1 and 2 of a search, inside the bucket of the first level that begins at `base`, `mass` above it: the value's pattern, and the mass above it
-  auto searched = [&](unsigned base, double& mass, double bound, bool strict) {
-    for (int level = 1; level <= 2; ++level) {
+  // one level of a search: the bin of a histogram at whose end the bound is met, inside the bucket that begins at `base`, `mass` above it
+  auto level_of = [&](const unsigned long long* of, unsigned& base, int level, double& mass, double bound, bool strict) __attribute__((always_inline)) {
+    masses_above<T>(of, base, level, mass, above, waves);
+    const int bin = lowest_bin<T>(above, bound, strict, &lowest);
+    mass = above[bin];
+    base += (unsigned)bin << level_shift(level);
+    __syncthreads();
+  };
+  // the levels from `level` on: the value's pattern to `base`, and the mass above it
+  auto searched = [&](unsigned& base, int level, double& mass, double bound, bool strict) __attribute__((always_inline)) {
+#pragma unroll 1
+    for (; level <= 2; ++level) {
       __syncthreads();
-      sums[t] = 0ull;
-      counts[t] = 0u;
+      sums[t] = 0ull, counts[t] = 0u;
       __syncthreads();
       const int shift = level_shift(level);
       const unsigned bucket = base >> (shift + SAMPLE_LEVEL_BITS);
       each([&](unsigned pattern, int) {
-        if ((pattern >> (shift + SAMPLE_LEVEL_BITS)) != bucket) return;
-        const unsigned bin = (pattern >> shift) & (SAMPLE_BINS - 1);
-        // (equal entries of a wave go together: additions to one place wait for one another)
-        const unsigned long long here = __ballot(1), same = __ballot(pattern == (unsigned)__builtin_amdgcn_readfirstlane((int)pattern));
-        if (same == here) {
-          if (lane == __ffsll((long long)here) - 1) {
-            atomicAdd(sums + bin, significand_of(pattern) * (unsigned long long)__popcll(here));
-            atomicAdd(counts + bin, (unsigned)__popcll(here));
-          }
-          return;
-        }
-        atomicAdd(sums + bin, significand_of(pattern));
-        atomicAdd(counts + bin, 1u);
+        add_equal_together((pattern >> (shift + SAMPLE_LEVEL_BITS)) == bucket, pattern, (pattern >> shift) & (SAMPLE_BINS - 1), sums, counts);
       });
       __syncthreads();
-      masses_above<SAMPLE_THREADS>(sums, base, level, mass, above, waves);
-      const int bin = lowest_bin<SAMPLE_THREADS>(above, bound, strict, &lowest);
-      mass = above[bin];
-      base += (unsigned)bin << shift;
+      level_of(sums, base, level, mass, bound, strict);
     }
-    return base;
   };
-  // the cut value: everything above it is kept, and of the entries equal to it as many as still
-  // start below the bound (engine.py:34-37)
+  // of a row with many candidates: the run of 1,024 patterns of a bin at whose end the bound is met, and the mass above it
+  int held = -1;  // whose masses fine_above holds
+  auto fine_run = [&](int bin, int slot, double bound, double& mass) __attribute__((always_inline)) -> unsigned {
+    if (held != slot) masses_above<T>(row.fine_sums[slot], (unsigned)bin << level_shift(0), 1, first_above[bin], fine_above, waves);
+    held = slot;
+    const int run = lowest_bin<T>(fine_above, bound, false, &lowest);
+    mass = fine_above[run];
+    __syncthreads();
+    return ((unsigned)bin << SAMPLE_LEVEL_BITS) + (unsigned)run;
+  };
+  unsigned cut_run = 0u, first_run = 0u, last_run = 0u;  // of 1,024 patterns: the one of the cut, those in one of which u falls
+  double above_run = c.above_cut;
   __syncthreads();
-  double above_cut = first_above[c.cut_bin];
-  // (a long list may be of one value over and over, as of a row of equal entries: nothing is left to search then)
-  bool one_value = n > SAMPLE_KEPT * SAMPLE_THREADS;
-  if (one_value) {
-    unsigned least = ~0u, most = 0u;
-    each([&](unsigned pattern, int) {
-      least = min(least, pattern);
-      most = max(most, pattern == ~0u ? 0u : pattern);
+  if (c.many) {
+    cut_run = (unsigned)c.cut_bin << level_shift(0);
+    level_of(row.fine_sums[0], cut_run, 1, above_run, c.limit, true);
+    cut_run >>= level_shift(1);
+    auto run_of = [&](double bound, unsigned whole) __attribute__((always_inline)) -> unsigned {
+      const int bin = lowest_bin<T>(first_above, bound, false, &lowest), slot = c.slot(bin);
+      __syncthreads();
+      if (bin < c.cut_bin) return cut_run;
+      if (slot < 0) return ((unsigned)bin << SAMPLE_LEVEL_BITS) | whole;
+      double mass;
+      const unsigned run = fine_run(bin, slot, bound, mass);
+      return run > cut_run ? run : cut_run;
+    };
+    first_run = run_of(u * (c.limit + (double)__uint_as_float((cut_run + 1u) << level_shift(1))), 0u);
+    last_run = run_of(u * c.limit, SAMPLE_BINS - 1);
+    // Every part of the row gathers the entries of those runs and adds up the third level of the cut's and, if it is one alone, u's.  (One block
+    // for the whole row is bound by its instructions, about a microsecond for each that it spends on an entry of 151,936.)
+    const bool second = first_run == last_run && first_run != cut_run;
+    const unsigned from_cut = cut_run << level_shift(1), from_u = first_run << level_shift(1), span_u = (last_run - first_run + 1u) << level_shift(1);
+    const int quads = (vocab + 3) / 4, a_part = (quads + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int begin = min(quads, (int)blockIdx.y * a_part), end = min(quads, begin + a_part);
+    auto of_part = [&](auto f) __attribute__((always_inline)) {  // f(quad, its number, whether it is there), a quad a lane; all lanes
+      constexpr int TOGETHER = 4;
+#pragma unroll 1
+      for (int first = begin; first < end; first += TOGETHER * T) {
+        float4 v[TOGETHER];
+#pragma unroll
+        for (int k = 0; k < TOGETHER; ++k) v[k] = ((const float4*)p)[min(first + k * T + t, end - 1)];
+#pragma unroll
+        for (int k = 0; k < TOGETHER; ++k) f(v[k], first + k * T + t, first + k * T + t < end);
+      }
+    };
+    auto at_cut = [&](unsigned pattern) { return pattern - from_cut < (unsigned)SAMPLE_BINS; };
+    auto at_u = [&](unsigned pattern) { return pattern - from_u < span_u; };
+    auto patterns_of = [&](const float4& v, unsigned* patterns) __attribute__((always_inline)) {
+      patterns[0] = __float_as_uint(v.x), patterns[1] = __float_as_uint(v.y), patterns[2] = __float_as_uint(v.z), patterns[3] = __float_as_uint(v.w);
+    };
+    auto add = [&](bool there, unsigned pattern) __attribute__((always_inline)) {
+      const bool cuts = at_cut(pattern);
+      add_equal_together(there && (cuts || (second && at_u(pattern))), pattern, (cuts ? 0u : SAMPLE_BINS) + (pattern & (SAMPLE_BINS - 1)), sums, counts);
+    };
+    for (int i = t; i < 2 * SAMPLE_BINS; i += T) sums[i] = 0ull, counts[i] = 0u;
+    if (t == 0) found = 0u;
+    __syncthreads();
+    of_part([&](const float4& v, int quad, bool there) __attribute__((always_inline)) {
+      unsigned patterns[4];
+      patterns_of(v, patterns);
+      bool any = false;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) any |= at_cut(patterns[j]) || at_u(patterns[j]);
+      if (__ballot(there && any) == 0ull || !there) return;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (quad * 4 + j >= vocab || !(at_cut(patterns[j]) || at_u(patterns[j]))) continue;
+        const unsigned at = atomicAdd(&found, 1u);
+        if (at < SAMPLE_FEW) stage[at] = make_uint2(patterns[j], (unsigned)(quad * 4 + j));
+      }
     });
-    if (t < 2) counts[t] = t == 0 ? ~0u : 0u;
     __syncthreads();
-    atomicMin(counts, least);
-    atomicMax(counts + 1, most);
+    const unsigned here = found;
+    if (here <= SAMPLE_FEW) {
+      for (unsigned i = t; i < SAMPLE_FEW; i += T) add(i < here, i < here ? stage[i].x : 0u);
+    } else {  // (equal entries, a thousand of them)
+      of_part([&](const float4& v, int quad, bool there) __attribute__((always_inline)) {
+        unsigned patterns[4];
+        patterns_of(v, patterns);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) add(there && quad * 4 + j < vocab, patterns[j]);
+      });
+    }
+    unsigned all = here;
+    const uint2* few = stage;
+    if (gridDim.y > 1) {
+      if (t == 0 && here > 0u) place = atomicAdd(&row.found, min(here, SAMPLE_FEW + 1u));
+      __syncthreads();
+      if (here <= SAMPLE_FEW)
+        for (unsigned i = t; i < here; i += T)
+          if (place + i < SAMPLE_FEW) row.few[place + i] = stage[i];
+      give_histogram(sums, counts, 2 * SAMPLE_BINS, row.run_sums[0], row.run_counts[0]);
+      // The part that is done last goes on, with what all have left: every wave's writes have ended and are out of its chiplet's cache before the
+      // part counts itself done, and nothing of it is read before the last one is.  Nobody waits for another part.
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (t == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        place = atomicAdd(&row.done, 1u);
+      }
+      __syncthreads();
+      if (place != gridDim.y - 1) return;
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      for (int i = t; i < 2 * SAMPLE_BINS; i += T) sums[i] = row.run_sums[0][i], counts[i] = row.run_counts[0][i];
+      all = row.found;
+      few = row.few;
+    }
+    from_row = all > SAMPLE_FEW;
     __syncthreads();
-    one_value = counts[0] == counts[1] && (counts[0] >> level_shift(0)) == (unsigned)c.cut_bin;
+    keep(few, from_row ? 0 : (int)all);
   }
-  const unsigned cut = one_value ? counts[0] : searched((unsigned)c.cut_bin << level_shift(0), above_cut, c.limit, true);
-  const unsigned equal_at_cut = one_value ? (unsigned)n : counts[cut & (SAMPLE_BINS - 1)];
-  const double cut_value = (double)__uint_as_float(cut), count_at_cut = (double)equal_at_cut;
-  double kept_at_cut = count_at_cut;
-  if (cut_value > 0.0) kept_at_cut = fmin(count_at_cut, ceil((c.limit - above_cut) / cut_value));
-  if (kept_at_cut < 1.0) kept_at_cut = 1.0;
-  const double target = (double)uniform * (above_cut + kept_at_cut * cut_value);
-  // the chosen value: the smallest one whose preceding mass is <= target
-  __syncthreads();
-  const int chosen_bin = lowest_bin<SAMPLE_THREADS>(first_above, target, false, &lowest);
-  listed = c.has((unsigned)chosen_bin);
-  double above_chosen = first_above[chosen_bin];
-  const bool at_cut = one_value && chosen_bin == c.cut_bin;
-  unsigned chosen = at_cut ? cut : searched((unsigned)chosen_bin << level_shift(0), above_chosen, target, false);
-  unsigned equal = at_cut ? equal_at_cut : counts[chosen & (SAMPLE_BINS - 1)];
+  // The cut value: everything above it is kept, and of the entries equal to it as many as still
+  // start below the bound (engine.py:34-37).  Then the chosen value: the smallest one whose preceding mass is <= target.
+  // (one copy of the searches' code for both, which the second finds in the instruction cache)
+  unsigned cut = 0u, equal_at_cut = 0u, chosen = 0u, equal = 0u;
+  double above_cut = 0.0, above_chosen = 0.0, kept_at_cut = 0.0, target = 0.0;
+#pragma unroll 1
+  for (int search = 0; search < 2; ++search) {
+    int level = 1, made = -1;  // where the last level is made already
+    if (search == 0) {
+      chosen = (unsigned)c.cut_bin << level_shift(0), above_chosen = c.above_cut;
+      if (c.many) chosen = cut_run << level_shift(1), above_chosen = above_run, made = 0;
+    } else {
+      const int bin = lowest_bin<T>(first_above, target, false, &lowest);
+      __syncthreads();
+      if (bin < c.cut_bin) break;
+      chosen = (unsigned)bin << level_shift(0), above_chosen = first_above[bin];
+      const int slot = c.many ? c.slot(bin) : -1;
+      if (slot >= 0) {
+        const unsigned run = fine_run(bin, slot, target, above_chosen);
+        chosen = run << level_shift(1), level = 2;
+        made = run == cut_run ? 0 : run == first_run && run == last_run ? SAMPLE_BINS : -1;
+      }
+      // (rounding may put the target outside what was listed)
+      const unsigned run = chosen >> level_shift(1);
+      if (c.many ? made < 0 && (run < first_run || (slot >= 0 ? run : run | (SAMPLE_BINS - 1)) > last_run) : !c.has((unsigned)bin)) from_row = true;
+    }
+    if (made >= 0) level_of(sums + made, chosen, 2, above_chosen, search == 0 ? c.limit : target, search == 0);
+    else searched(chosen, level, above_chosen, search == 0 ? c.limit : target, search == 0);
+    equal = counts[max(made, 0) + (int)(chosen & (SAMPLE_BINS - 1))];
+    if (search == 0) {
+      cut = chosen, above_cut = above_chosen, equal_at_cut = equal;
+      const double cut_value = (double)__uint_as_float(cut), count_at_cut = (double)equal_at_cut;
+      kept_at_cut = count_at_cut;
+      if (cut_value > 0.0) kept_at_cut = fmin(count_at_cut, ceil((c.limit - above_cut) / cut_value));
+      if (kept_at_cut < 1.0) kept_at_cut = 1.0;
+      target = u * (above_cut + kept_at_cut * cut_value);
+    }
+  }
   if (chosen < cut) {  // never below the cut
     chosen = cut;
     above_chosen = above_cut;
     equal = equal_at_cut;
-    listed = true;
   }
   if (equal == 0u) return;  // no entry has the chosen value: the argmax stands
   const double chosen_value = (double)__uint_as_float(chosen);
@@ -646,9 +867,44 @@ __device__ void sample_top_p(const SampleBuffers& buffers, int r, float uniform,
     });
     return;
   }
-  // the entry of that rank among the equal ones in index order: their indices ten bits at a time, from the highest
+  // the entry of that rank among the equal ones in index order
+  if (from_row) {
+    // thousands of them: how many a wave's contiguous share of the row holds, then in the share of the one with the entry how many a thread's
+    const int wave = t / WAVE, quads = (vocab + 3) / 4, a_wave = (quads + T / WAVE - 1) / (T / WAVE);
+    int begin = min(quads, wave * a_wave), end = min(quads, begin + a_wave), mine = 0;
+#pragma unroll 1
+    for (int first = begin; first < end; first += 8 * WAVE) {
+      float4 v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = ((const float4*)p)[min(first + k * WAVE + lane, end - 1)];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int quad = first + k * WAVE + lane;
+        const int equal_here = (__float_as_uint(v[k].x) == chosen) + (quad * 4 + 1 < vocab && __float_as_uint(v[k].y) == chosen) +
+                               (quad * 4 + 2 < vocab && __float_as_uint(v[k].z) == chosen) + (quad * 4 + 3 < vocab && __float_as_uint(v[k].w) == chosen);
+        mine += quad < end ? equal_here : 0;
+      }
+    }
+    int before = block_sum_before_int(mine, scan);  // (of all lanes of the waves before, and of this wave's lanes before)
+    before = __shfl(before, 0, WAVE);
+#pragma unroll
+    for (int offset = WAVE / 2; offset > 0; offset >>= 1) mine += __shfl_xor(mine, offset, WAVE);
+    if (lane == 0 && before <= rank && rank < before + mine) lowest = wave, before_lowest = before;
+    __syncthreads();
+    begin = (int)min((long)vocab, (long)lowest * a_wave * 4), end = (int)min((long)vocab, (long)begin + (long)a_wave * 4), rank -= before_lowest;
+    const int a_thread = (end - begin + T - 1) / T, from = min(end, begin + t * a_thread), to = min(end, from + a_thread);
+    mine = 0;
+    for (int i = from; i < to; ++i) mine += __float_as_uint(p[i]) == chosen ? 1 : 0;
+    before = block_sum_before_int(mine, scan);
+    if (before <= rank && rank < before + mine)
+      for (int i = from, seen = before; i < to; ++i)
+        if (__float_as_uint(p[i]) == chosen && seen++ == rank) *out = i;
+    return;
+  }
+  // their indices ten bits at a time, from the highest
   int shift = 0, prefix = 0;
   while (shift + SAMPLE_LEVEL_BITS < 31 && (vocab - 1) >> (shift + SAMPLE_LEVEL_BITS) != 0) shift += SAMPLE_LEVEL_BITS;
+#pragma unroll 1
   for (; shift >= 0; shift -= SAMPLE_LEVEL_BITS) {
     __syncthreads();
     counts[t] = 0u;
@@ -673,7 +929,8 @@ __device__ void sample_top_p(const SampleBuffers& buffers, int r, float uniform,
   if (t == 0) *out = prefix;
 }
 
-// The token of every row with a temperature: one block per row.  `out` holds the argmax already.  WITH_TOP_P: rows may have top_p < 1.
+// The token of every row with a temperature.  `out` holds the argmax already.  A block a row, and WITH_TOP_P (rows may have top_p < 1) as many
+// parts of a row as the grid has, of which a row with many candidates needs more than the first.
 template <bool WITH_TOP_P>
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(const float* __restrict__ temperatures,
                                                                      const float* __restrict__ top_ps,
@@ -685,7 +942,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(const float
   __shared__ double before_piece, shared_target;
   const int r = blockIdx.x;
   if (temperatures[r] <= 0.f) return;  // engine.py:30-31
-  const float* p = buffers.p + (size_t)r * vocab;
+  const float* p = buffers.p + r * buffers.stride;
   const float top_p = top_ps[r];
   const int per_piece = (vocab + pieces - 1) / pieces;
   const int lane = threadIdx.x % WAVE;
@@ -694,6 +951,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(const float
     sample_top_p(buffers, r, uniforms[r], vocab, out + r);
     return;
   }
+  if (blockIdx.y > 0) return;
   // inverse CDF in index order: the piece first, from the pieces' sums, then inside it
   if (threadIdx.x == 0) owner_thread = 0x7fffffff;
   if (threadIdx.x < WAVE) {  // a lane per piece
@@ -746,24 +1004,19 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(const float
 static size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
 struct SampleWorkspace {
-  size_t sums, counts, listed, cleared_words;  // these come first: the first launch clears them
-  size_t p, piece_sums, list, candidates, piece_values, piece_indices, bytes;
+  size_t stride, p, piece_sums, piece_values, piece_indices, rows, bytes;
 };
 
 static SampleWorkspace sample_workspace(int rows, int vocab) {
-  const size_t pieces = sample_pieces(rows, false), bins = (size_t)rows * SAMPLE_BINS;
+  const size_t pieces = sample_pieces(rows, false);
   SampleWorkspace w;
   size_t at = 0;
-  w.sums = at, at += rounded(bins * sizeof(unsigned long long));
-  w.counts = at, at += rounded(bins * sizeof(unsigned));
-  w.listed = at, at += rounded((size_t)rows * sizeof(unsigned));
-  w.cleared_words = at / sizeof(unsigned);
-  w.p = at, at += rounded((size_t)rows * vocab * sizeof(float));
+  w.stride = ((size_t)vocab + 3) / 4 * 4;
+  w.p = at, at += rounded((size_t)rows * w.stride * sizeof(float));
   w.piece_sums = at, at += rounded((size_t)rows * pieces * sizeof(double));
-  w.list = at, at += rounded((size_t)rows * vocab * sizeof(uint2));
-  w.candidates = at, at += rounded((size_t)rows * sizeof(Candidates));
   w.piece_values = at, at += rounded((size_t)rows * ARGMAX_PIECES * sizeof(float));
   w.piece_indices = at, at += rounded((size_t)rows * ARGMAX_PIECES * sizeof(int));
+  w.rows = at, at += rounded((size_t)rows * sizeof(SampleRow));
   w.bytes = at;
   return w;
 }
@@ -787,26 +1040,19 @@ extern "C" int llmserve_sample(const float* logits, const float* temperatures, c
   unsigned char* base = (unsigned char*)workspace;
   float* piece_values = (float*)(base + w.piece_values);
   int* piece_indices = (int*)(base + w.piece_indices);
-  SampleBuffers buffers;
-  buffers.p = (float*)(base + w.p);
-  buffers.piece_sums = (double*)(base + w.piece_sums);
-  buffers.sums = (unsigned long long*)(base + w.sums);
-  buffers.counts = (unsigned*)(base + w.counts);
-  buffers.listed = (unsigned*)(base + w.listed);
-  buffers.list = (uint2*)(base + w.list);
-  buffers.candidates = (Candidates*)(base + w.candidates);
-  buffers.piece_values = piece_values;
-  buffers.piece_indices = piece_indices;
+  SampleRow* of_rows = with_top_p ? (SampleRow*)(base + w.rows) : nullptr;
+  const SampleBuffers buffers = {(float*)(base + w.p), w.stride, (double*)(base + w.piece_sums), of_rows, piece_values, piece_indices};
   const int first_pieces = argmax_pieces(rows), pieces = sample_pieces(rows, with_top_p != 0);
+  static_assert(sizeof(SampleRow) % 8 == 0 && SAMPLE_CLEARED % sizeof(unsigned) == 0, "rows lie side by side");
   hipLaunchKernelGGL(argmax_pieces_kernel, dim3(rows, first_pieces), dim3(SAMPLE_THREADS), 0, stream, logits,
-                     piece_values, piece_indices, vocab, first_pieces, with_top_p ? (unsigned*)base : (unsigned*)nullptr,
-                     with_top_p ? w.cleared_words : (size_t)0);
+                     piece_values, piece_indices, vocab, first_pieces, (unsigned*)of_rows, sizeof(SampleRow) / sizeof(unsigned),
+                     (int)(SAMPLE_CLEARED / sizeof(unsigned)));
   hipLaunchKernelGGL(sample_exp_kernel, dim3(rows, pieces), dim3(SAMPLE_BLOCK), 0, stream, logits, temperatures, top_ps,
                      buffers, out, rows, vocab, pieces, first_pieces, with_top_p);
   if (with_top_p) {
     hipLaunchKernelGGL(sample_list_kernel, dim3(rows, pieces), dim3(SAMPLE_BLOCK), 0, stream, temperatures, top_ps, uniforms, buffers, vocab, pieces);
-    hipLaunchKernelGGL(sample_pick_kernel<true>, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, temperatures, top_ps, uniforms, buffers, out, vocab,
-                       pieces);
+    hipLaunchKernelGGL(sample_pick_kernel<true>, dim3(rows, pick_parts(rows)), dim3(SAMPLE_THREADS), 0, stream, temperatures, top_ps, uniforms,
+                       buffers, out, vocab, pieces);
   } else {
     hipLaunchKernelGGL(sample_pick_kernel<false>, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, temperatures, top_ps, uniforms, buffers, out, vocab,
                        pieces);

@@ -1379,3 +1379,45 @@ def test_ring_of_six_tiles_of_rows_has_the_bits_of_eight(kernels, rows, gated):
     if gated:
         exact = torch.nn.functional.silu(exact[:, ::2]) * exact[:, 1::2]
     torch.testing.assert_close(results[0].double(), exact, **TOLERANCE[torch.bfloat16])
+
+
+@pytest.mark.parametrize("rows", [1, 33, 257])
+@pytest.mark.parametrize("vocab", [8191, 8193, 20003])
+def test_top_p_of_rows_with_more_candidates_than_a_list_holds(kernels, rows, vocab):
+    """Around 8,192 candidates, and far more; rows of a length that is no multiple of four, in sixteen parts, in seven and in one; more equal
+    entries of one value and of several than what is gathered of a row holds.  Against the rule in 64 bits: the kernel's exp may be off by two
+    units in the last place (2^-22 of the value), which moves every mass by as much of the whole, and logits that lie so close may tie in p."""
+    k = kernels[torch.float32]
+    generator = torch.Generator().manual_seed(vocab + rows)
+    kinds = [lambda: torch.full((vocab,), 2.5), lambda: torch.randint(0, 3, (vocab,), generator=generator) * 0.003,
+             lambda: 0.3 * torch.randn(vocab, generator=generator).bfloat16().float(), lambda: 0.01 * torch.randn(vocab, generator=generator),
+             lambda: 4.0 * torch.randn(vocab, generator=generator)]
+    logits = torch.stack([kinds[(row + vocab) % 5]() for row in range(rows)])
+    p = torch.exp(logits.double() - logits.amax(1, keepdim=True).double())
+    ranked, order = torch.sort(p, dim=1, descending=True, stable=True)
+    mass = ranked.cumsum(1)
+    for draw, top_p in enumerate((0.2, 0.95, 0.9999)):
+        uniforms = torch.tensor([plain.uniform_for(draw, row) for row in range(rows)], dtype=torch.float32)
+        if rows > 1:
+            uniforms[0], uniforms[-1] = 0.0, 1.0 - 2.0 ** -24
+        got = k.sample(on_gpu(logits), on_gpu(torch.ones(rows)), on_gpu(torch.full((rows,), top_p)), on_gpu(uniforms)).cpu().long()
+        limit = float(torch.tensor(top_p)) * mass[:, -1]
+        kept = (mass - ranked < limit[:, None]).sum(1)
+        target = uniforms.double() * mass.gather(1, kept[:, None] - 1)[:, 0]
+        place, value = (order == got[:, None]).int().argmax(1), p.gather(1, got[:, None])
+        slack = 2.0 ** -21 * mass[:, -1]
+        above = torch.where(p > value * (1 + 2.0 ** -21), p, 0.0).sum(1)  # certainly ranked before, and perhaps
+        not_below = torch.where(p >= value * (1 - 2.0 ** -21), p, 0.0).sum(1)
+        right = (above < limit + slack) & (above <= target + slack) & (not_below > target - slack)
+        # values far apart, and equal ones in the order of their indices: the very entry, where the end of the kept set is not in question
+        after, before = mass.gather(1, place[:, None])[:, 0], (mass - ranked).gather(1, place[:, None])[:, 0]
+        exact = torch.tensor([(row + vocab) % 5 < 3 for row in range(rows)])
+        right &= ~exact | ((after > target - slack) & (before <= target + slack) & (before < limit + slack + 1))
+        assert not (wrong := (~right).nonzero()[:, 0].tolist()), (top_p, wrong[:9], got[wrong[:9]].tolist())
+
+
+def test_the_samplers_memory(kernels):
+    """A list holds 8,192 entries of a row and no longer the whole row: not beyond what a row's histograms and counts of its pieces took before."""
+    library = kernels[torch.float32]._sampling_library()
+    for rows in (1, 8, 64, 512):
+        assert library.llmserve_sample_workspace_kib(rows, 151936) * 1024 < rows * (151936 * 4 + 96 * 1024) + 4096
