@@ -1004,7 +1004,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_pick_kernel(const float
 static size_t rounded(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
 struct SampleWorkspace {
-  size_t stride, p, piece_sums, piece_values, piece_indices, rows, bytes;
+  size_t stride, p, piece_sums, piece_values, piece_indices, plain_bytes, rows, bytes;  // (what only rows with top-p need comes last)
 };
 
 static SampleWorkspace sample_workspace(int rows, int vocab) {
@@ -1016,6 +1016,7 @@ static SampleWorkspace sample_workspace(int rows, int vocab) {
   w.piece_sums = at, at += rounded((size_t)rows * pieces * sizeof(double));
   w.piece_values = at, at += rounded((size_t)rows * ARGMAX_PIECES * sizeof(float));
   w.piece_indices = at, at += rounded((size_t)rows * ARGMAX_PIECES * sizeof(int));
+  w.plain_bytes = at;
   w.rows = at, at += rounded((size_t)rows * sizeof(SampleRow));
   w.bytes = at;
   return w;
@@ -1027,16 +1028,22 @@ extern "C" int llmserve_sample_workspace_kib(int rows, int vocab) {
   return (int)((sample_workspace(rows, vocab).bytes + 1023) / 1024);
 }
 
+// The same with with_top_p = 0: 0.6 MB a row of 151,936, with top-p 0.08 more.
+extern "C" int llmserve_sample_plain_workspace_kib(int rows, int vocab) {
+  if (rows <= 0 || vocab <= 0) return -1;
+  return (int)((sample_workspace(rows, vocab).plain_bytes + 1023) / 1024);
+}
+
 // out[r]: the token of row r.  workspace: 256-byte aligned device memory of llmserve_sample_workspace_kib
-// KiB, overwritten.  with_top_p = 0 promises that no row with a temperature has top_p < 1, and leaves the
-// searches out.
+// KiB, overwritten.  with_top_p = 0 promises that no row with a temperature has top_p < 1, leaves the
+// searches out, and needs llmserve_sample_plain_workspace_kib KiB alone.
 extern "C" int llmserve_sample(const float* logits, const float* temperatures, const float* top_ps,
                                const float* uniforms, void* workspace, int workspace_kib, int* out, int rows,
                                int vocab, int with_top_p, hipStream_t stream) {
   if (rows <= 0) return 0;
   if (vocab <= 0 || workspace == nullptr || ((size_t)workspace & 255) != 0) return ERR_BAD_ARGUMENT;
   const SampleWorkspace w = sample_workspace(rows, vocab);
-  if ((size_t)workspace_kib * 1024 < w.bytes) return ERR_BAD_ARGUMENT;
+  if ((size_t)workspace_kib * 1024 < (with_top_p ? w.bytes : w.plain_bytes)) return ERR_BAD_ARGUMENT;
   unsigned char* base = (unsigned char*)workspace;
   float* piece_values = (float*)(base + w.piece_values);
   int* piece_indices = (int*)(base + w.piece_indices);

@@ -88,6 +88,7 @@ _SIGNATURES = {
     "llmserve_argmax": "ppppiip",
     "llmserve_argmax_static": "ppiip",
     "llmserve_sample_workspace_kib": "ii",
+    "llmserve_sample_plain_workspace_kib": "ii",
     "llmserve_sample": "pppppipiiip",
     "llmserve_add_layer_norm": "ppippipiiifp",
     "llmserve_rms_norm_columns": "piiiiipifpiiiip",
@@ -2128,7 +2129,7 @@ class HipKernels:
         rows, vocab = logits.shape
         out = self._empty((rows,), torch.int32)
         library = self._sampling_library()
-        kib = library.llmserve_sample_workspace_kib(rows, vocab)
+        kib = library.llmserve_sample_workspace_kib(rows, vocab) if with_top_p else library.llmserve_sample_plain_workspace_kib(rows, vocab)
         if kib <= 0:
             raise KernelError(f"sample: no workspace for {rows} rows of {vocab}")
         workspace = self._empty((kib * 1024,), torch.uint8)

@@ -1421,3 +1421,26 @@ def test_the_samplers_memory(kernels):
     library = kernels[torch.float32]._sampling_library()
     for rows in (1, 8, 64, 512):
         assert library.llmserve_sample_workspace_kib(rows, 151936) * 1024 < rows * (151936 * 4 + 96 * 1024) + 4096
+
+
+def test_sampling_without_top_p_needs_no_memory_for_it(kernels):
+    """The workspace of a call whose rows have no top-p is p and little else, one smaller is refused, and tokens are those with the rest around it."""
+    from llmserve_amd.kernels.hip import _pointer
+
+    k = kernels[torch.float32]
+    library = k._sampling_library()
+    rows, vocab = 9, 20001
+    kib = library.llmserve_sample_plain_workspace_kib(rows, vocab)
+    assert rows * vocab * 4 // 1024 < kib < rows * vocab * 4 // 1024 + 32 and library.llmserve_sample_plain_workspace_kib(0, vocab) < 0
+    assert library.llmserve_sample_workspace_kib(rows, vocab) > kib
+    generator = torch.Generator().manual_seed(3)
+    logits, ones, uniforms = on_gpu(torch.randn(rows, vocab, generator=generator)), on_gpu(torch.ones(rows)), on_gpu(torch.rand(rows, generator=generator))
+    workspace, out = torch.full((kib * 1024 + 256,), 7, dtype=torch.uint8, device="cuda"), torch.zeros(rows, dtype=torch.int32, device="cuda")
+
+    def status(size, with_top_p):
+        return library.llmserve_sample(_pointer(logits), _pointer(ones), _pointer(ones), _pointer(uniforms), _pointer(workspace), size, _pointer(out),
+                                       rows, vocab, with_top_p, k._stream)
+
+    assert status(kib - 1, 0) == 1001 and status(kib, 1) == 1001 and status(kib, 0) == 0
+    assert (workspace[kib * 1024 :] == 7).all()
+    assert torch.equal(out, k.sample(logits, ones, ones, uniforms)) and torch.equal(out, k.sample(logits, ones, ones, uniforms, with_top_p=False))
