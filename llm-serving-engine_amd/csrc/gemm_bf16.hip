@@ -1001,8 +1001,8 @@ extern "C" int llmserve_gemm_medium(const void* x, const void* w, const void* bi
                       : pick_medium<bf16_t, false>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
 }
 
-// ---------------------------------------------------------------------------- 17 to 64 rows through a ring
-// gemm_ring: the product for 17 to 64 rows of x, bound by how fast the weights come from memory.  A
+// ---------------------------------------------------------------------------- 17 to 128 rows through a ring
+// gemm_ring: the product for 17 to 128 rows of x (and few of a large weight), bound by how fast the weights come from memory.  A
 // workgroup of four waves owns NT tiles of 16 weight rows over its whole K range and MT tiles of x; both
 // go through a ring of DEPTH stages of KSTEPS * 32 k in LDS that the waves share, filled straight from
 // memory (global_load_lds_dwordx4, a chunk of 16 rows x 32 k in lane order, laid out and swizzled as in
@@ -1257,7 +1257,13 @@ static int launch_ring(const void* x, const void* w, const void* bias, int bias_
 }
 
 // nt tiles of 16 weight rows a workgroup, stages of 128 k; four stages, or three with six or eight tiles of x (65 to 128
-// rows), which fill the LDS with five weight tiles beside them
+// rows), which fill the LDS with five weight tiles beside them.
+// Up to 96 rows six tiles of x, where eight would bring rows that are not there: a quarter less of x a stage.  (The instructions are as many: the fourth
+// wave repeats the third's tiles.)  The same bits.  Us at 65 / 96 rows, eight -> six, in the shape that the products get: gated, two weight tiles N 4,864
+// K 896 7.3 / 7.5 -> 7.0 / 7.1, N 7,168 K 1,024 8.3 / 8.4 -> 7.6 / 7.6; four N 9,728 K 896 10.9 / 11.0 -> 9.9 / 10.0, N 12,288 K 2,048 21.0 / 21.2 -> 19.9 /
+// 20.2, N 13,824 K 2,304 25.0 / 25.0 -> 23.0 / 22.3; five N 17,920 K 1,536 22.8 / 22.8 -> 20.2 / 20.1, N 18,944 K 3,584 44.5 / 44.5 -> 39.2 / 38.9;
+// eight N 24,576 K 3,072 44.2 / 46.5 -> 43.0 / 45.4, N 28,672 K 4,096 58.7 / 59.5 -> 58.1 / 58.3; ten N 37,888 K 3,584 63.0 / 63.2 -> 60.2 / 61.6; in
+// parts, two N 2,048 K 1,408 9.4 / 9.6 -> 8.5 / 8.7, N 2,560 K 1,920 6.8 / 7.1 -> 6.5 / 6.6.
 template <typename TO, bool GATED>
 static int pick_ring(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
                      int splits, hipStream_t stream, int nt) {
@@ -1270,15 +1276,15 @@ static int pick_ring(const void* x, const void* w, const void* bias, int bias_is
   RING_CASE(6)
 #undef RING_CASE
   if (nt == 5 && M > 32 && M <= 64) return launch_ring<5, 4, 4, 4, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream);
-  // Up to 96 rows six tiles of x, where eight would bring and multiply rows that are not there: a third of x's bytes a stage and of the products.
-  // (gated, 65 / 80 / 96 rows, us, eight -> six: N 17,920 K 1,536 22.2 21.7 21.6 -> 19.1 18.4 18.5; N 9,728 K 896 11.9 12.2 12.2 -> 11.0 11.2 11.2;
-  // N 12,288 K 2,048 25.5 24.9 25.1 -> 21.5 21.0 21.1; the same bits)
-  if (nt == 5 && M > 64 && M <= 96) return launch_ring<5, 6, 4, 3, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream);
-#define ROWS_CASE(NT_)                                                                                                  \
-  if (nt == NT_ && M > 64) return launch_ring<NT_, 8, 4, 3, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream);
-  ROWS_CASE(2)
-  ROWS_CASE(4)
-  ROWS_CASE(5)
+#define ROWS_CASE(NT_, KSTEPS_, DEPTH_)                                                                                  \
+  if (nt == NT_ && M > 64)                                                                                               \
+    return M <= 96 ? launch_ring<NT_, 6, KSTEPS_, DEPTH_, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream) \
+                   : launch_ring<NT_, 8, KSTEPS_, DEPTH_, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream);
+  ROWS_CASE(2, 4, 3)
+  ROWS_CASE(4, 4, 3)
+  ROWS_CASE(5, 4, 3)
+  ROWS_CASE(8, 2, 4)
+  ROWS_CASE(10, 2, 4)
 #undef ROWS_CASE
   // many weight tiles a workgroup, in stages of 64 k: for a weight of so many rows that fewer tiles make several rounds
 #define MANY_CASE(NT_)                                                                                                  \
@@ -1290,8 +1296,6 @@ static int pick_ring(const void* x, const void* w, const void* bias, int bias_is
   MANY_CASE(12)
   MANY_CASE(14)
 #undef MANY_CASE
-  if (nt == 8 && M > 64) return launch_ring<8, 8, 2, 4, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream);
-  if (nt == 10 && M > 64) return launch_ring<10, 8, 2, 4, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream);
   return ERR_BAD_ARGUMENT;
 }
 

@@ -539,10 +539,10 @@ class HipKernels:
         if self.ring_products and 64 < rows <= 128 and inner % 128 == 0 and (
             (may_split and (1 << 20) < size <= 150_000_000) or (gated and (1 << 22) < size <= 150_000_000)
         ):
-            # 65 to 128 rows of gate/up, and of what may be cut where K is no multiple of 256: the same kernel with eight
-            # tiles of x.  Us at 65 / 128 rows in a captured chain over different weights, the library against it: 1.5B sizes
-            # gate/up with its activation 25.8 / 26.5 -> 21.9 / 22.3; the 7B sizes' with ten weight tiles a workgroup, 237
-            # workgroups, 67.1 / 72.1 -> 59.1 / 61.3 (80-82 with five, which make 474); the library keeps qkv (7.5 against 10.2;
+            # 65 to 128 rows of gate/up, and of what may be cut where K is no multiple of 256: the same kernel with six (up to 96 rows) or
+            # eight tiles of x.  Us at 65 / 128 rows in a captured chain over different weights, the library against it: 1.5B sizes
+            # gate/up with its activation 25.8 / 26.5 -> 19.9 / 23.0; the 7B sizes' with ten weight tiles a workgroup, 237
+            # workgroups, 67.1 / 72.1 -> 60.2 / 60.4 (80-82 with five, which make 474); the library keeps qkv (7.5 against 10.2;
             # 19-23 against 21-23).
             return "ring"
         if self.library_products and (rows > 64 or self._for_replay or weights.out_features * inner > 150_000_000):
@@ -651,6 +651,8 @@ class HipKernels:
         103.4 / 114.8 -> 101.5 / 108.8, down 91.1 / 58.8 -> 52.1 / 59.1, o 20.2 / 22.3 -> 14.6 / 16.8, qkv 19.8 / 25.6 ->
         18.8 / 27.7)."""
         tiles = -(-out_features // 16)
+        # (up to 96 rows the kernel brings six tiles of x.  Told of six the estimate picks other shapes for gated weights of 41,216 to 49,152 rows alone,
+        # four weight tiles for eight: N 41,216 K 1,536 43-45 us and 44-45, N 45,056 K 2,048 55 and 57-58, N 49,152 K 2,560 72-74 and 70-72, K 1,024 34 and 33)
         x_tiles = 2 if rows <= 32 else 4 if rows <= 64 else 8
         stages = in_features // 128
         best = None

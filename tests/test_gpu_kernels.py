@@ -1381,6 +1381,29 @@ def test_ring_of_six_tiles_of_rows_has_the_bits_of_eight(kernels, rows, gated):
     torch.testing.assert_close(results[0].double(), exact, **TOLERANCE[torch.bfloat16])
 
 
+@pytest.mark.parametrize("tiles,inner", [(2, 384), (4, 640), (8, 640), (8, 192), (10, 320)])
+@pytest.mark.parametrize("rows", [65, 81, 96, 97])
+def test_ring_of_six_tiles_of_rows_beside_any_weight_tiles(kernels, rows, tiles, inner):
+    """As above beside two, four, eight and ten weight tiles (five: above), gated, whole and in parts."""
+    from llmserve_amd.kernels.hip import _pointer
+
+    k, outer = kernels[torch.bfloat16], tiles * 16 * 3 + 16
+    generator = torch.Generator(device="cuda").manual_seed(rows + tiles)
+    x, w = (torch.randn(shape, generator=generator, device="cuda").bfloat16() for shape in ((128, inner), (outer, inner)))
+    exact = x.double() @ w.double().T
+    for gated, parts in ((1, 1), (0, 1), (0, inner // 128 if inner % 128 == 0 else 1)):
+        results, split = [], parts > 1
+        for count in (rows, 128):
+            out = torch.full((parts, 130, outer // 2 if gated else outer), 7.0, device="cuda", dtype=torch.float32 if split else torch.bfloat16)
+            flat = out.view(-1)[: parts * count * out.shape[2]].view(parts, count, out.shape[2])
+            assert k._gemm_bf16.llmserve_gemm_ring(_pointer(x), _pointer(w), None, 0, _pointer(out), int(split), gated, count, outer, inner, parts, tiles, k._stream) == 0
+            assert (out.view(-1)[flat.numel() :] == 7.0).all()
+            results.append(flat[:, :rows])
+        assert torch.equal(*results)
+        want = torch.nn.functional.silu(exact[:, ::2]) * exact[:, 1::2] if gated else exact
+        torch.testing.assert_close(results[0].double().sum(0), want[:rows], **TOLERANCE[torch.bfloat16])
+
+
 @pytest.mark.parametrize("rows", [1, 33, 257])
 @pytest.mark.parametrize("vocab", [8191, 8193, 20003])
 def test_top_p_of_rows_with_more_candidates_than_a_list_holds(kernels, rows, vocab):
