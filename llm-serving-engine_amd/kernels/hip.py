@@ -357,10 +357,14 @@ class HipKernels:
     # 1.783 -> 1.737.  The 7B sizes' qkv and o (33 and 26 MB) gain nothing from their first 8 MB.
     _WHOLE_AHEAD = 8 << 20
 
-    # Of gate and up, beside an output projection that merges key splits, whose 96 workgroups wait more than they read (8 us for 4.7 MB): as much as
-    # they leave time for.  A step at 1 and 8 rows, ms, with nothing, 8, 16, 24, 30 and 38 MB: 1.271 1.259 1.253 1.255 1.244 1.298, 1.382 1.374 1.366 1.364
-    # 1.353 1.385.  Beside the projection that has no splits to merge (4.8 us) 8 MB gain nothing and 16 lose 3 %.
-    _MERGING_AHEAD = 30 << 20
+    # Of gate and up, beside an output projection that merges key splits, whose workgroups wait more than they read: as much as it leaves time for,
+    # for each workgroup that brings (they are what the projection's leave idle).  A layer of a step over 640 keys, us, with nothing and with 8, 16, 24,
+    # 30 and 38 MB, at 1 and 8 rows: width 1,536 of 12 heads, gate and up 52 MB (160 workgroups bring 30 MB) 43.6 42.9 42.7 42.7 42.1 44.2, 47.3 46.8 46.5 46.5 45.9
+    # 47.0; width 2,048 of 16, 66 MB (128: 24) 53.2 51.9 51.6 51.4 51.4 51.7, 58.0 56.6 56.8 56.2 56.3 56.2; width 2,560 of 12, 95 MB (96: 18) 58.5 57.6 57.2
+    # 57.8 58.7 60.5, 65.2 64.4 63.8 64.4 65.0 66.5; width 1,152 of 9, 30 MB (184: all) 36.5 36.1 35.1 35.1 34.7, 39.3 39.0 38.4 38.1 37.7; width 1,024 of 8, 22 MB
+    # 33.4 32.5 32.4 31.5, 34.9 34.8 34.7 33.9.  16 rows gain 0.3-1.5 us.  Beside the projection that has no splits to merge (4.8 us) 8 MB gain nothing
+    # and 16 lose 3 %.
+    _MERGING_AHEAD_EACH = 192 << 10
 
     def _whole_ahead(self, weights: Any, rows: int, busy: int) -> tuple:
         if not isinstance(weights, LinearWeights) or rows > 64 or weights.weight.numel() * weights.weight.element_size() > self._WHOLE_AHEAD:
@@ -867,7 +871,7 @@ class HipKernels:
         status = self._gemm_bf16.llmserve_gemm_into_norm(
             _pointer(x) if split is None else None, _pointer(split_x), _pointer(split_ml), splits, _pointer(project.weight), _pointer(bias),
             _is_float(bias) if bias is not None else 0, _pointer(hidden), _pointer(into.weight), _is_float(into.weight), _pointer(scaled),
-            _pointer(sums), rows, width, project.in_features, *self._ahead(reader.both if split is not None else None, width // 16, self._MERGING_AHEAD, max(1, tiles)),
+            _pointer(sums), rows, width, project.in_features, *self._ahead(reader.both if split is not None else None, width // 16, self._MERGING_AHEAD_EACH * max(0, 256 - width // 16), max(1, tiles)),
             self._stream,
         )
         _check(status, "linear into a norm")
