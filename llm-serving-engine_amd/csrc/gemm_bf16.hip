@@ -422,12 +422,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
                                                                  const bf16_t* __restrict__ w,
                                                                  const void* __restrict__ bias, int bias_is_float,
                                                                  TO* __restrict__ out, int M, int N, int K,
-                                                                 int k_split, Tail tail, Link link, int tiles, Ahead ahead) {
+                                                                 int k_split, Tail tail, Link link) {
   extern __shared__ __attribute__((aligned(16))) unsigned char stream_lds[];
-  if (LINK == INTO_NORM && (int)blockIdx.x >= tiles) {
-    bring_ahead(ahead, blockIdx.x, tiles, gridDim.x);
-    return;
-  }
   constexpr int OPERANDS = (NT + MT) * G;                // of one group: the weight tiles' steps, then x's
   constexpr int STAGE_BYTES = OPERANDS * STREAM_CHUNK;
   constexpr int WAVE_BYTES = STREAM_STAGES * STAGE_BYTES;
@@ -577,8 +573,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
 
 template <int WAVES, int NT, int MT, int G, typename TO, int GATED, int LINK = NO_LINK>
 static int launch_stream(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N,
-                         int K, int splits, hipStream_t stream, Tail tail = {}, Link link = {}, int helpers = 0,
-                         Ahead ahead = {}) {
+                         int K, int splits, hipStream_t stream, Tail tail = {}, Link link = {}) {
   const size_t stages = (size_t)WAVES * STREAM_STAGES * (NT + MT) * G * STREAM_CHUNK;
   const size_t sums = (size_t)WAVES * NT * MT * 64 * 4 * sizeof(float);
   const size_t lds = (stages > sums ? stages : sums) + (LINK == SCALED ? ((size_t)(link.tiles + 15) / 16 * 256 + WAVES * 16) * sizeof(float) : 0);
@@ -591,10 +586,9 @@ static int launch_stream(const void* x, const void* w, const void* bias, int bia
       asked = true;
     }
   }
-  const int tiles = (N + 16 * NT - 1) / (16 * NT);
-  hipLaunchKernelGGL((gemm_stream_kernel<WAVES, NT, MT, G, TO, GATED, LINK>), dim3(tiles + helpers, splits),
+  hipLaunchKernelGGL((gemm_stream_kernel<WAVES, NT, MT, G, TO, GATED, LINK>), dim3((N + 16 * NT - 1) / (16 * NT), splits),
                      dim3(WAVES * 64), lds, stream, (const bf16_t*)x, (const bf16_t*)w, bias, bias_is_float, (TO*)out, M,
-                     N, K, K / splits, tail, link, tiles, ahead);
+                     N, K, K / splits, tail, link);
   return LAUNCH_STATUS();
 }
 
@@ -815,20 +809,20 @@ static int sums_stride(int M) { return M <= 16 ? 16 : M <= 32 ? 32 : 64; }
 
 // The product (split_x null: of x; else of the merge of its key splits, as above, M <= 16) into a norm: hidden [M, N] float32 +=
 // x . w^T (+ bias); rows [M, N] bfloat16 = hidden * weight; sums float32 [N / 16, 16 rows, or 32 or 64: as many as hold M].
-// M <= 64, N a multiple of 16, K of 128.  `helpers` further workgroups bring the runs of `ahead` into the caches (common.h: Ahead).
+// M <= 64, N a multiple of 16, K of 128.  With split_x `helpers` further workgroups bring the runs of `ahead` into the caches (common.h: Ahead).
 extern "C" int llmserve_gemm_into_norm(const void* x, const void* split_x, const float* split_ml, int splits, const void* w, const void* bias,
                                        int bias_is_float, float* hidden, const void* weight, int weight_is_float, void* rows, float* sums,
                                        int M, int N, int K, int helpers, const void* ahead, int stripe, int stripes,
                                        hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 64 || N % 16 || K <= 0 || K % (STEP * GROUP) || (split_x && M > 16) || (!x && !split_x)) return ERR_BAD_ARGUMENT;
-  if (!ahead_fits(helpers, ahead, stripe, stripes)) return ERR_BAD_ARGUMENT;
+  if (!ahead_fits(helpers, ahead, stripe, stripes) || (helpers && !split_x)) return ERR_BAD_ARGUMENT;
   const Ahead next = {(const unsigned char*)ahead, (unsigned)stripe, (unsigned)stripes};
   const Link link{hidden, weight, weight_is_float, (bf16_t*)rows, sums, sums_stride(M), N / 16, 0.f, 0.f};
   if (split_x) return pick_merged<INTO_NORM>(split_x, split_ml, splits, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, link, helpers, next);
-  if (M <= 16) return launch_stream<4, 1, 1, 4, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link, helpers, next);
-  if (M <= 32) return launch_stream<4, 1, 2, 2, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link, helpers, next);
-  return launch_stream<4, 1, 4, 1, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link, helpers, next);
+  if (M <= 16) return launch_stream<4, 1, 1, 4, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
+  if (M <= 32) return launch_stream<4, 1, 2, 2, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
+  return launch_stream<4, 1, 4, 1, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
 }
 
 // ---------------------------------------------------------------------------- 16 < M <= 64
