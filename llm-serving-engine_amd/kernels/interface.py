@@ -15,6 +15,16 @@ import torch
 
 
 class Kernels(Protocol):
+    """What every library has.  Two more the parts ask for where a library has them:
+
+    `linear_rotated(x, weights, layout, batch, cell, inverse_frequencies, pairing)`: the rows that `linear(x, weights)` and `rotate_and_store`
+    leave, k and v stored, or None, and nothing done, where it doesn't take the sizes.  A library that derives from one with it and has
+    `linear`, `rotate_and_store` or `rotate_store_attend` of its own is asked for those.
+
+    `norm_into(hidden, weight, eps, reader)`: what `rotate_store_attend` may be handed as `into`: the stream, the norm behind the product
+    `project`, and the gated product that reads the normed rows.  It may then add to the stream itself and return what that `reader` alone
+    takes, instead of rows to add."""
+
     device: torch.device
     dtype: torch.dtype
 

@@ -5,14 +5,16 @@ for the kernels; tests/test_gpu_parts.py does the same on the GPU)."""
 from __future__ import annotations
 
 from dataclasses import replace
+from types import SimpleNamespace
 
 import pytest
 import torch
 
 from llmserve_amd import CacheConfig, ModelRunner, StepEntry
+from llmserve_amd.cache import CacheCell
 from llmserve_amd.kernels.hip import HipKernels, LinearWeights
 from llmserve_amd.parts import (
-    FEED_FORWARDS, MIXERS, NORMS, POSITIONS, Attention, AttentionSpec, FixedState, GatedMLP, GatedMLPSpec, PagedKeyValue, PreNormBlock,
+    FEED_FORWARDS, MIXERS, NORMS, POSITIONS, Attention, AttentionSpec, FixedState, GatedMLP, GatedMLPSpec, HeadLayout, PagedKeyValue, PreNormBlock,
     PreNormBlockSpec, RMSNorm, RMSNormSpec, Rotary, RotarySpec,
 )
 from llmserve_amd.weights import load_model_folder
@@ -301,3 +303,56 @@ def test_nothing_is_brought_of_what_lies_elsewhere_or_is_none_of_the_librarys():
     here = LinearWeights(torch.empty((2048, 1536), dtype=torch.bfloat16), None)
     for weights in (here, LinearWeights(here.weight.to("meta"), None), None, "qkv", object(), here.weight):
         assert library._whole_ahead(weights, 1, 1) == (0, None, 0, 0) and library._ahead(weights, 1, 1 << 24, 4) == (0, None, 0, 0)
+
+
+class Asked(Exception):
+    pass
+
+
+class AskedForTheTable(HipKernels):
+    """Goes as far as the first thing that the fused product, rotation and store ask a library for."""
+
+    def __init__(self):
+        self.device, self.dtype = torch.device("cpu"), torch.bfloat16
+
+    def rotary_table(self, batch, inverse_frequencies, magnitude=1.0):
+        raise Asked
+
+
+def test_rows_are_rotated_by_their_product_only_where_nobody_has_these_steps_of_their_own():
+    """`linear_rotated` does `linear` and `rotate_and_store`, and stands before `rotate_store_attend`: a library that has one of them of its own is
+    asked for it, and so is an encoding derived from the rotary one; what the fused form does not take is left to the two as well."""
+    rows, heads, kv_heads, dim, page, inner = 96, 2, 1, 32, 8, 64
+    layout = HeadLayout(heads, kv_heads, dim)
+    x = torch.zeros(rows, inner, dtype=torch.bfloat16)
+    weights = LinearWeights(torch.zeros(layout.width, inner, dtype=torch.bfloat16), None)
+    cell = CacheCell(PagedKeyValue(kv_heads, dim), True, 0, torch.zeros(13, kv_heads, dim // 8, page, 8, dtype=torch.bfloat16),
+                     torch.zeros(13, *PagedKeyValue(kv_heads, dim).page_fields(page)["values"], dtype=torch.bfloat16))
+    batch = SimpleNamespace(max_query_length=rows, positions=torch.zeros(rows, dtype=torch.int32),
+                            groups=[SimpleNamespace(page_size=page, slot_mapping=torch.zeros(rows, dtype=torch.int32))])
+    inverse = torch.ones(dim // 2)
+
+    def asked(library, pairing="adjacent", x=x, weights=weights):
+        try:
+            return library.linear_rotated(x, weights, layout, batch, cell, inverse, pairing)
+        except Asked:
+            return "asked"
+
+    assert asked(AskedForTheTable()) == "asked"
+    for step in ("linear", "rotate_and_store", "rotate_store_attend", "_rotate_store_attend"):
+        own = type("Own", (AskedForTheTable,), {step: lambda self, *arguments, **options: None})
+        assert asked(own()) is None
+    assert asked(AskedForTheTable(), "half") is None and asked(AskedForTheTable(), x=x.float()) is None
+    assert asked(AskedForTheTable(), x=torch.zeros(inner, rows, dtype=torch.bfloat16).T) is None
+    batch.max_query_length = 1
+    assert asked(AskedForTheTable()) is None
+    batch.max_query_length = rows
+
+    for derived, expected in ((Rotary, "asked"), (SomePosition, None),
+                              (type("Stores", (Rotary,), {"encode_and_store": lambda self, *arguments: None}), None)):
+        encoding = derived(RotarySpec(dim, 100.0, "adjacent"), {}, TorchKernels(torch.bfloat16))
+        encoding.kernels = AskedForTheTable()
+        try:
+            assert encoding.project_and_store(x, weights, layout, batch, cell) is expected
+        except Asked:
+            assert expected == "asked"
