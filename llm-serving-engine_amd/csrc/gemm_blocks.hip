@@ -503,7 +503,7 @@ static int launch_rotated(const void* x, const void* w, const void* bias, int bi
                           hipStream_t stream, const Rotated& rotated) {
 #define BLOCK(...) return launch_block<__VA_ARGS__, bf16_t, OUT_ROTATED>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, rotated)
   auto one_round = [&](int n, int m) { return (long)((N + n - 1) / n) * ((M + m - 1) / m) <= 256; };
-  if (K % 64) BLOCK(2, 2, 2, 2, 32, 4, 2);
+  if (K % 64) BLOCK(2, 2, 2, 2, 32, 4, 2);  // (a K that ends in half a stage, which the entry point takes; `_rotated_ahead` leaves it to the two kernels)
   if (one_round(64, 32)) BLOCK(2, 1, 1, 1, 64, 5, 2);
   if (one_round(64, 64)) BLOCK(2, 2, 1, 1, 64, 5, 2);
   if (one_round(128, 64)) BLOCK(2, 2, 2, 1, 64, 3, 2);

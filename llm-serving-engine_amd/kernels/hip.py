@@ -424,7 +424,8 @@ class HipKernels:
         _check(status, "rotate_and_store")
 
     def linear_rotated(self, x, weights: LinearWeights, layout, batch, cell, inverse_frequencies, pairing: str) -> torch.Tensor | None:
-        """`linear(x, weights)` and `rotate_and_store` of its rows in one kernel, where it takes them and is ahead; else None, and nothing done."""
+        """`linear(x, weights)` and `rotate_and_store` of its rows in one kernel, where it takes them and is ahead; else None, and nothing done.
+        Neighbouring pairs alone: of half pairs a column's partner is dim / 2 away, in another tile."""
         rows, inner = x.shape
         dim, store = layout.head_dim, cell is not None and cell.writable
         if (
