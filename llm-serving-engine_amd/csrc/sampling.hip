@@ -236,11 +236,11 @@ extern "C" int llmserve_argmax_static(const float* logits, int* out, int rows, i
 // goes on with the block's part.  So one block never goes through all of a row but for the place of one among a thousand equal entries.
 // Us a call in a captured chain, 1 / 8 / 16 / 32 / 64 / 256 rows of 151,936: a launch a level, of many blocks a row | lists of any length,
 // searched by one block | this:
-//   spread 3, temperature 0.8, top-p 0.9   43 54 61 73 99 317   | 30 38 45 50 65 376     | 31 38 42 48 60 156
-//   spread 1, temperature 1.5 (20,000)     44 54 63 77 104      | 46 59 66 70 89         | 40 47 57 68 87
-//   spread 0.01 (nearly all)               49 62 76 104 155 523 | 162 195 218 263 324 977 | 43 57 69 93 137 394
+//   spread 3, temperature 0.8, top-p 0.9   43 54 61 73 99 317   | 30 38 45 50 65 376     | 31 37 42 47 60 156
+//   spread 1, temperature 1.5 (20,000)     44 54 63 77 104      | 46 59 66 70 89         | 40 48 55 67 87
+//   spread 0.01 (nearly all)               49 62 76 104 155 523 | 162 195 218 263 324 977 | 45 56 68 92 137 394
 //   equal entries                          62 86 130 215 383    | 129 141 144 160 221    | 61 66 81 111 170
-//   two values                             52 65 90 137 229     | 244 254 262 300 353    | 62 65 77 104 152
+//   two values                             52 65 90 137 229     | 244 254 262 300 353    | 62 64 76 102 152
 // What is left is four launches that wait for one another.
 //
 // The entries of a bin share their exponent (it lies in the ten bits that are fixed first), so their
@@ -327,6 +327,25 @@ __device__ __forceinline__ int lowest_bin(const double* above, double limit, boo
   if (met != 0ull && (int)threadIdx.x % WAVE == __ffsll((long long)met) - 1) atomicMin(lowest, mine);
   __syncthreads();
   return *lowest;
+}
+
+// The same for two bounds that are not strict, together; lowest: two of LDS.
+template <int THREADS>
+__device__ __forceinline__ void lowest_two_bins(const double* above, double limit0, double limit1, int* lowest) {
+  constexpr int EACH = SAMPLE_BINS / THREADS;
+  if (threadIdx.x < 2) lowest[threadIdx.x] = SAMPLE_BINS - 1;
+  __syncthreads();
+  int mine0 = SAMPLE_BINS, mine1 = SAMPLE_BINS;
+#pragma unroll
+  for (int j = EACH - 1; j >= 0; --j) {
+    const double m = above[threadIdx.x * EACH + j];
+    if (m <= limit0) mine0 = (int)threadIdx.x * EACH + j;
+    if (m <= limit1) mine1 = (int)threadIdx.x * EACH + j;
+  }
+  const unsigned long long met0 = __ballot(mine0 < SAMPLE_BINS), met1 = __ballot(mine1 < SAMPLE_BINS);
+  if (met0 != 0ull && (int)threadIdx.x % WAVE == __ffsll((long long)met0) - 1) atomicMin(lowest, mine0);
+  if (met1 != 0ull && (int)threadIdx.x % WAVE == __ffsll((long long)met1) - 1) atomicMin(lowest + 1, mine1);
+  __syncthreads();
 }
 
 // Which bins of the first histogram a row's choice is among, and the bound at which its kept set ends.
@@ -541,7 +560,7 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_list_kernel(const float* 
   __shared__ double above[SAMPLE_BINS], waves[SAMPLE_BLOCK / WAVE], sums_here[SAMPLE_PIECES_MAX];
   __shared__ unsigned long long fine_sums[SAMPLE_SLOTS * SAMPLE_BINS];
   __shared__ unsigned fine_counts[SAMPLE_SLOTS * SAMPLE_BINS];
-  __shared__ int lowest;
+  __shared__ int lowest, lowest_two[2];
   __shared__ unsigned candidates, found, place;
   constexpr unsigned STAGE = SAMPLE_SLOTS * SAMPLE_BINS;
   uint2* stage = (uint2*)fine_sums;  // (a row has a list or the second level)
@@ -569,10 +588,9 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_list_kernel(const float* 
   // the kept mass is at least the bound, and beyond it by less than a value of that bin (up to rounding, which the row's block sees to);
   // and what is chosen is not below the cut
   const double end_of_bin = (double)__uint_as_float((unsigned)(c.cut_bin + 1) << level_shift(0)), u = (double)uniforms[r];
-  __syncthreads();
-  c.first_bin = max(c.cut_bin, lowest_bin<SAMPLE_BLOCK>(above, u * (c.limit + end_of_bin), false, &lowest));
-  __syncthreads();
-  c.last_bin = max(c.cut_bin, lowest_bin<SAMPLE_BLOCK>(above, u * c.limit, false, &lowest));
+  lowest_two_bins<SAMPLE_BLOCK>(above, u * (c.limit + end_of_bin), u * c.limit, lowest_two);
+  c.first_bin = max(c.cut_bin, lowest_two[0]);
+  c.last_bin = max(c.cut_bin, lowest_two[1]);
 #pragma unroll
   for (int j = 0; j < SAMPLE_BINS / SAMPLE_BLOCK; ++j)
     if (c.has(t + j * SAMPLE_BLOCK) && in_bin[j] != 0u) atomicAdd(&candidates, in_bin[j]);
@@ -677,18 +695,17 @@ __device__ __forceinline__ void sample_top_p(const SampleBuffers& buffers, int r
     }
   };
   // one level of a search: the bin of a histogram at whose end the bound is met, inside the bucket that begins at `base`, `mass` above it
+  // (a barrier before the next)
   auto level_of = [&](const unsigned long long* of, unsigned& base, int level, double& mass, double bound, bool strict) __attribute__((always_inline)) {
     masses_above<T>(of, base, level, mass, above, waves);
     const int bin = lowest_bin<T>(above, bound, strict, &lowest);
     mass = above[bin];
     base += (unsigned)bin << level_shift(level);
-    __syncthreads();
   };
   // the levels from `level` on: the value's pattern to `base`, and the mass above it
   auto searched = [&](unsigned& base, int level, double& mass, double bound, bool strict) __attribute__((always_inline)) {
 #pragma unroll 1
     for (; level <= 2; ++level) {
-      __syncthreads();
       sums[t] = 0ull, counts[t] = 0u;
       __syncthreads();
       const int shift = level_shift(level);
@@ -698,6 +715,7 @@ __device__ __forceinline__ void sample_top_p(const SampleBuffers& buffers, int r
       });
       __syncthreads();
       level_of(sums, base, level, mass, bound, strict);
+      if (level < 2) __syncthreads();
     }
   };
   // of a row with many candidates: the run of 1,024 patterns of a bin at whose end the bound is met, and the mass above it
@@ -717,6 +735,7 @@ __device__ __forceinline__ void sample_top_p(const SampleBuffers& buffers, int r
     cut_run = (unsigned)c.cut_bin << level_shift(0);
     level_of(row.fine_sums[0], cut_run, 1, above_run, c.limit, true);
     cut_run >>= level_shift(1);
+    __syncthreads();
     auto run_of = [&](double bound, unsigned whole) __attribute__((always_inline)) -> unsigned {
       const int bin = lowest_bin<T>(first_above, bound, false, &lowest), slot = c.slot(bin);
       __syncthreads();
@@ -823,8 +842,7 @@ __device__ __forceinline__ void sample_top_p(const SampleBuffers& buffers, int r
       chosen = (unsigned)c.cut_bin << level_shift(0), above_chosen = c.above_cut;
       if (c.many) chosen = cut_run << level_shift(1), above_chosen = above_run, made = 0;
     } else {
-      const int bin = lowest_bin<T>(first_above, target, false, &lowest);
-      __syncthreads();
+      const int bin = lowest_bin<T>(first_above, target, false, &before_lowest);
       if (bin < c.cut_bin) break;
       chosen = (unsigned)bin << level_shift(0), above_chosen = first_above[bin];
       const int slot = c.many ? c.slot(bin) : -1;
@@ -837,6 +855,7 @@ __device__ __forceinline__ void sample_top_p(const SampleBuffers& buffers, int r
       const unsigned run = chosen >> level_shift(1);
       if (c.many ? made < 0 && (run < first_run || (slot >= 0 ? run : run | (SAMPLE_BINS - 1)) > last_run) : !c.has((unsigned)bin)) from_row = true;
     }
+    __syncthreads();
     if (made >= 0) level_of(sums + made, chosen, 2, above_chosen, search == 0 ? c.limit : target, search == 0);
     else searched(chosen, level, above_chosen, search == 0 ? c.limit : target, search == 0);
     equal = counts[max(made, 0) + (int)(chosen & (SAMPLE_BINS - 1))];
