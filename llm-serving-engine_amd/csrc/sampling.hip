@@ -410,10 +410,10 @@ __device__ __forceinline__ Batch load_batch(const float* __restrict__ p, int fir
   return batch;
 }
 
-__device__ __forceinline__ void add_entry(float value, unsigned bucket, int shift, unsigned long long* lds_sums, unsigned* lds_counts) {
-  const unsigned pattern = __float_as_uint(value);
-  if ((pattern >> (shift + SAMPLE_LEVEL_BITS)) == bucket) {
-    const unsigned bin = (pattern >> shift) & (SAMPLE_BINS - 1);
+// adds an entry to the first histogram (a pattern of more than 30 bits is that of no probability: of NaN)
+__device__ __forceinline__ void add_entry(float value, unsigned long long* lds_sums, unsigned* lds_counts) {
+  const unsigned pattern = __float_as_uint(value), bin = pattern >> level_shift(0);
+  if (bin < SAMPLE_BINS) {
     atomicAdd(lds_sums + bin, significand_of(pattern));
     atomicAdd(lds_counts + bin, 1u);
   }
@@ -509,7 +509,7 @@ __global__ __launch_bounds__(SAMPLE_BLOCK) void sample_exp_kernel(const float* _
       const float v = expf(batch.v[u] / temperature - top_logit);
       p[i] = v;
       partial += (double)v;
-      if (with_histogram) add_entry(v, 0u, level_shift(0), lds_sums, lds_counts);
+      if (with_histogram) add_entry(v, lds_sums, lds_counts);
     }
   }
   const double sum = block_sum_f64(partial, sd);  // (its barriers stand between the additions and what reads them)
