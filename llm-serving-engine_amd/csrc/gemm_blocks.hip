@@ -2,29 +2,31 @@
 // out[M, N] = x[M, K] . w[N, K]^T (+ bias), or silu(gate) * up of weight rows that alternate gate_j, up_j, or partial sums
 // over parts of K.
 //
-// A workgroup owns a tile of weight rows by rows of x; both operands of a stage of 64 k (32 where K is no multiple of 64)
-// go from global memory straight into LDS (global_load_lds_dwordx4: a wave's 64 lanes fill 1 KB in lane order, no
-// registers in between), two to six stages deep, and a wave multiplies TN x TM tiles of v_mfma_f32_32x32x16_bf16.  While
-// the products of sixteen k run, the operands of the next sixteen are read from LDS into a second set of registers.  One
-// barrier a stage, before its last products: by then every wave holds all it needs of the stage, so the stage is asked
-// for anew at once, as many stages ahead as there are, and the next one is known to have landed for everybody.
+// A workgroup owns a tile of weight rows by rows of x; both operands of a stage of 64 k go from global memory straight into LDS
+// (global_load_lds_dwordx4: a wave's 64 lanes fill 1 KB in lane order, no registers in between), two to five stages deep, and a wave
+// multiplies TN x TM tiles of v_mfma_f32_16x16x32_bf16, whose operands it reads from LDS some tiles ahead of their products (Reads).  One
+// barrier a stage, shortly before its last products: by then every wave has read all of the stage, and the next one is known to have landed for everybody;
+// the stage is asked for anew, as many stages ahead as there are, piece by piece between the products that follow.
 // A staged row of 64 k is 128 bytes, eight pieces of 16; piece p of row r lies in slot p ^ (r / 2 % 8), so that the
 // sixteen lanes that LDS serves together (the same piece of sixteen rows) hit all its banks (measured: no conflicts; with
 // p ^ (r % 8), half of the reads' time).
 //
-// What bounds it: at 8,192 rows of 8,192 x 8,192 the matrix cores (0.85 ms, 1.29 PFLOP/s; the library 0.73); at the sizes a
-// decoder has, how the tiles divide over 256 CUs, and what a tile costs besides its products: about 8 us for 256 x 256
-// (first loads, the way out), 4 for 128 x 128.  Hence the shapes below and `pick_shape`.  Us, a captured chain over different weights,
-// the library (with the kernel for silu(gate) * up behind it, 5 to 19 us) -> this: N 17,920 K 1,536 gated: 256 rows 35 -> 29, 384 rows 37 -> 30,
-// 2,048 rows 133 -> 111 (256 x 320 tiles: 490 of them make two rounds where 256 x 256 make 2.2); N 1,536 K 8,960 in parts: 96 rows
-// 18 -> 12, 256 rows 23 -> 15, 384 rows 25-33 -> 20, 1,024 rows 38 -> 36; K 1,536: 192 rows 8.1 -> 6.4, 384 rows 9.2 -> 7.8;
-// N 3,584 K 18,944 in parts: 128 rows 51 -> 34, 256 rows 61 -> 47, 512 rows 85 -> 80; N 37,888 K 3,584 gated: 2,048 rows 546 -> 474.
+// What bounds it: at 8,192 rows of 8,192 x 8,192 the power that the matrix cores draw (0.78 ms, 1.41 PFLOP/s; the library 0.73): products alone, of random
+// operands in registers, run at 2.0 PFLOP/s, of zeros at 2.4.  Tiles of 32 x 32 x 16, which move twice the sums in and out of the accumulators for a
+// product, reach 1.81 there, and 0.83 ms here.  At the sizes a decoder has, how the tiles divide over 256 CUs, what a tile costs besides its
+// products, and the way of the operands: a CU takes 64 bytes a clock from its caches, so what a stage brings (74 KB for 256 x 320) takes 1,150 clocks of the
+// 2,560 of its products, and asked for all at once it stops the wave that asks.  Spread over the products, us before (asked for in the stage's last quarter) -> after:
+// 2,048 rows of N 17,920 K 1,536 gated 110 -> 100, of N 2,048 K 1,536 20.4 -> 14.9, of N 1,536 K 1,536 16.9 -> 14.3, of N 1,536 K 8,960 in 128 x 128 77 -> 57;
+// 320 rows of N 17,920 27.5 -> 25.7, and 8,960 as K in parts 20.1 -> 18.6.  There what bounds it is the weights' way from memory: three stages of all tiles are 7 MB,
+// which take 2.4 us to come.  Bringing lines into L2 ahead of that gained nothing: what a wave asks for comes back in order, and waits for them.
+// Against the library (with the kernel for silu(gate) * up behind it, 5 to 19 us), us: N 17,920 K 1,536 gated: 384 rows 37 -> 30, 2,048 rows 133 -> 100;
+// N 1,536 K 8,960 in parts: 96 rows 18 -> 12, 384 rows 25-33 -> 19.
 #include "common.h"
 #include <type_traits>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 // Which tile a workgroup takes.  The chip hands workgroups to its eight chiplets (XCDs) in turn,
 // workgroup i to chiplet i % 8, and every chiplet has an L2 of its own: tiles dealt out in launch
@@ -44,6 +46,11 @@ __device__ __forceinline__ void tile_of_workgroup(int index, int tiles_n, int ti
   tile_n = within / rows;
 }
 
+// A result of more than so many bytes is stored past the caches: it does not fit the eight L2s (32 MB) beside the operands, and what lies there
+// at a kernel's end is written back before the next one starts.  Us, kept -> past: 2,048 rows of N 17,920 K 1,536 gated (37 MB) 110.8 -> 102.8; a prompt of
+// 2,048 tokens 7,138 -> 7,067.  Results that fit are read by the next kernel from there: a prompt of 77 1,798 -> 1,840.
+#define STREAMED_FROM (16u << 20)
+
 // What the way out does with the sums (and the bias).
 #define OUT_PLAIN 0
 #define OUT_GATED 1    // silu(gate) * up of columns that alternate gate_j, up_j
@@ -58,133 +65,182 @@ struct Rotated {
   int heads, kv_heads, dim, page_size;
 };
 
-// What a wave of OUT_ROTATED asks for before its products, as their way from memory would be waited for at the end: lane l
-// holds where row l % 32 of its row tile j goes (the place of a negative slot is not used), the bias of the columns that it will write, and,
-// where one tile leaves the registers, their angles.
+// Which of a wave's weight rows row r of its tile i is.  A lane's sums of a tile are four rows of the product's result, 4 q .. 4 q + 3 for lanes
+// 16 q .. 16 q + 15, all of one row of x.  So the rows are dealt to the tiles of a group (G of them) four at a time: over the group
+// a lane then holds 4 G neighbours, which leave as one piece of 16 bytes (four float32, eight bfloat16, sixteen gates and ups).  Tiles that
+// make no whole group hold their rows as they come.
+template <int TN, int G>
+__device__ __forceinline__ int weight_row(int i, int r) {
+  return (i / G + 1) * G <= TN ? i / G * G * 16 + r / 4 * (4 * G) + i % G * 4 + r % 4 : i * 16 + r;
+}
+template <typename TO, int OUT, int TN>
+constexpr int group_of() {
+  int tiles = sizeof(TO) == 4 ? 1 : OUT == OUT_GATED ? 4 : 2;
+  while (tiles > TN) tiles /= 2;
+  return tiles;
+}
+
+// What a wave of OUT_ROTATED asks for before its products, as their way from memory would be waited for at the end: where the rows of x that this
+// lane will write go (the place of a negative slot is not used), the bias of its columns as it lies in memory (eight bfloat16, or eight float32 in two
+// halves: nothing here may ask what it has brought, or it is waited for before the first stage is asked for), and their angles.
+typedef unsigned u32x4_anywhere __attribute__((ext_vector_type(4), aligned(2)));
 template <int TN, int TM>
 struct Early {
-  static constexpr int PASSES = TN * TM == 1 ? 32 / (64 / (4 * TN)) : 0;
-  int slot[TM], page[TM], offset[TM], value_row[TM];
-  float bias[8];
-  f32x4 angles[PASSES ? PASSES : 1][2];
+  int slot[TM];
+  u32x4 bias[TN / 2][2];
+  f32x4 angles[TN / 2][TM][2];
 };
+template <int TN, int TM>
+__device__ __forceinline__ float early_bias(const Early<TN, TM>& early, int i, int e, int bias_is_float) {
+  const unsigned half = early.bias[i][0][e / 2];
+  return __uint_as_float(bias_is_float ? early.bias[i][e / 4][e % 4] : e % 2 ? half & 0xffff0000u : half << 16);
+}
 
 __device__ __forceinline__ const f32x4* angles_of(const Rotated& to, int m, int d) { return (const f32x4*)(to.table + ((size_t)m * to.dim + d) / 2); }
 
 template <int TN, int TM>
 __device__ __forceinline__ void ask_early(Early<TN, TM>& early, const Rotated& to, const void* bias, int bias_is_float, int M, int N,
                                           int n_wave, int m_wave, int lane) {
-  constexpr int LANES_A_ROW = 4 * TN, ROWS_A_PASS = 64 / LANES_A_ROW;
-  const int n = min(n_wave + lane % LANES_A_ROW * 8, N - 8), width = value_piece_width(to.page_size);
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
-    const int m = m_wave + j * 32 + (lane & 31), slot = m < M ? to.slots[m] : -1;
-    early.slot[j] = slot;
-    early.page[j] = slot / to.page_size;
-    early.offset[j] = slot % to.page_size;
-    early.value_row[j] = early.offset[j] / width * width * to.dim + early.offset[j] % width;
+    const int m = m_wave + j * 16 + (lane & 15);
+    early.slot[j] = m < M ? to.slots[m] : -1;
   }
 #pragma unroll
-  for (int e = 0; e < 8; ++e) early.bias[e] = bias ? load_as_float(bias, bias_is_float, n + e) : 0.f;
+  for (int i = 0; i < TN / 2; ++i) {
+    const int n = min(n_wave + i * 32 + (lane >> 4) * 8, N - 8);
+    // (without a bias the same loads read the start of the angles, and nobody uses them)
+    const char* from = bias ? (const char*)bias + (size_t)n * (bias_is_float ? 4 : 2) : (const char*)to.table;
+    early.bias[i][0] = *(const u32x4_anywhere*)from;
+    early.bias[i][1] = *(const u32x4_anywhere*)(from + (bias && bias_is_float ? 16 : 0));
 #pragma unroll
-  for (int pass = 0; pass < Early<TN, TM>::PASSES; ++pass) {
-    const f32x4* angles = angles_of(to, min(m_wave + pass * ROWS_A_PASS + lane / LANES_A_ROW, M - 1), n % to.dim);
-    early.angles[pass][0] = angles[0], early.angles[pass][1] = angles[1];
+    for (int j = 0; j < TM; ++j) {
+      const f32x4* angles = angles_of(to, min(m_wave + j * 16 + (lane & 15), M - 1), n % to.dim);
+      early.angles[i][j][0] = angles[0], early.angles[i][j][1] = angles[1];
+    }
   }
 }
 
-// The values of 32 rows, which lie in `mine` with their bias (rows of `ROW` floats, a column each of the wave's 32 TN): a page keeps
+// The values of 16 rows, which lie in `mine` with their bias (rows of `ROW` floats, a column each of the wave's 16 TN): a page keeps
 // them transposed in pieces of eight keys, so a lane takes one column of eight rows, and where the rows are one piece (a prompt's
-// portion) 64 lanes store 1 KB in a row.
-template <int TN, int TM, int ROW>
-__device__ __forceinline__ void store_values(const Rotated& to, const float* mine, const Early<TN, TM>& early, int j, int N, int n_wave, int lane) {
+// portion) 64 lanes store 1 KB in a row.  `slot`: of row lane % 16.
+template <int TN, int ROW>
+__device__ __forceinline__ void store_values(const Rotated& to, const float* mine, int row_slot, int N, int n_wave, int lane) {
   const int v_first = (to.heads + to.kv_heads) * to.dim, width = value_piece_width(to.page_size);
-  if (n_wave + 32 * TN <= v_first) return;
+  const size_t a_page = (size_t)to.page_size * to.dim;
 #pragma unroll 1
-  for (int unit = 0; unit < 2 * TN; ++unit) {
-    const int column = (unit * 64 + lane) % (32 * TN), octet = (unit * 64 + lane) / (32 * TN);
+  for (int unit = 0; unit < TN / 2; ++unit) {
+    const int column = (unit * 64 + lane) % (16 * TN), octet = (unit * 64 + lane) / (16 * TN);
     const int n = n_wave + column;
     const bool mine_to_store = n >= v_first && n < N;
     const int head = (n - v_first) / to.dim, d = (n - v_first) % to.dim;
-    const size_t a_page = (size_t)to.page_size * to.dim;
     bf16x8 run;
 #pragma unroll
     for (int i = 0; i < 8; ++i) run[i] = (bf16_t)mine[(size_t)(octet * 8 + i) * ROW + column];
-    const int slot = __shfl(early.slot[j], octet * 8);
+    const int slot = __shfl(row_slot, octet * 8);
     bool together = width == 8 && slot >= 0 && slot % 8 == 0;
 #pragma unroll
     for (int i = 1; i < 8; ++i) {
-      const int place = __shfl(early.slot[j], octet * 8 + i);
+      const int place = __shfl(row_slot, octet * 8 + i);
       together = together & (place == slot + i);
     }
+    auto row_of = [&](int place) {
+      const int offset = place % to.page_size;
+      return ((size_t)(place / to.page_size) * to.kv_heads + head) * a_page + offset / width * width * to.dim + offset % width + d * width;
+    };
     if (__all(together)) {
-      const int page = __shfl(early.page[j], octet * 8), row = __shfl(early.value_row[j], octet * 8);
-      if (mine_to_store) *(bf16x8*)(to.values + ((size_t)page * to.kv_heads + head) * a_page + row + d * 8) = run;
+      if (mine_to_store) *(bf16x8*)(to.values + row_of(slot)) = run;
     } else {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        // (asked of other lanes by all lanes, before any is left out)
-        const int place = __shfl(early.slot[j], octet * 8 + i), page = __shfl(early.page[j], octet * 8 + i);
-        const int row = __shfl(early.value_row[j], octet * 8 + i);
-        if (mine_to_store && place >= 0) to.values[((size_t)page * to.kv_heads + head) * a_page + row + d * width] = run[i];
+        const int place = __shfl(row_slot, octet * 8 + i);  // (asked of other lanes by all lanes, before any is left out)
+        if (mine_to_store && place >= 0) to.values[row_of(place)] = run[i];
       }
     }
   }
 }
 
-// The way out.  D[n][m] of a 32 x 32 tile: a lane holds column m = lane % 32 and rows n = 8 * (e / 4) +
-// 4 * (lane / 32) + e % 4, so its values lie in 32 different rows of `out`.  They go through LDS (`mine`: 32 x
-// (32 TN + 4) floats of this wave's own), 32 rows of x at a time, and leave as whole rows: 4 TN lanes write the
-// 32 TN columns of a row, eight columns (16 bytes of bfloat16) a lane.  n_wave, m_wave: where the wave's tiles begin;
+// The way out.  D[n][m] of a 16 x 16 tile: a lane holds column m = lane % 16 and four rows n (weight_row), and stores its run of a group's
+// columns straight from its registers: four lanes write 64 bytes in a row, of sixteen rows.  n_wave, m_wave: where the wave's tiles begin;
 // `slice` the part of K (its own copy of `out`).  INSIDE: all of it lies inside the result, rows of which are a multiple of
-// eight long, so nothing is asked row by row (such questions kept the reads of one row from running beside the next).
+// eight long, so nothing is asked row by row.
 template <int TN, int TM, bool INSIDE, typename TO, int OUT>
-__device__ __forceinline__ void store_tiles(const f32x16 (&acc)[TN][TM], float* mine, TO* __restrict__ out,
+__device__ __forceinline__ void store_tiles(const f32x4 (&acc)[TN][TM], float* mine, TO* __restrict__ out,
                                             const void* __restrict__ bias, int bias_is_float, int slice, int M, int N,
-                                            int n_wave, int m_wave, int lane, const Rotated& rotated, const Early<TN, TM>& early) {
+                                            int n_wave, int m_wave, int lane, const Rotated& rotated, const Early<TN, TM>& early, bool streamed) {
   static_assert(OUT == OUT_PLAIN || sizeof(TO) == 2, "a gated or rotated result is bfloat16");
-  constexpr int ROW = 32 * TN + 4;  // floats of a transposed row, padded
-  constexpr int LANES_A_ROW = 4 * TN, ROWS_A_PASS = 64 / LANES_A_ROW;
-  const int r32 = lane & 31, half = lane >> 5;
-  const int piece = lane % LANES_A_ROW, row_in_pass = lane / LANES_A_ROW;
-  const int n_piece = n_wave + piece * 8;
+  constexpr int G = group_of<TO, OUT, TN>(), WHOLE = TN / G * G;
+  const int r16 = lane & 15, q = lane >> 4;
   const bool with_bias = bias && slice == 0;
-  float bias_here[8];
+  auto store_piece = [&](auto piece, TO* dst) {
+    if (streamed) __builtin_nontemporal_store(piece, (decltype(piece)*)dst);
+    else *(decltype(piece)*)dst = piece;
+  };
+  // a run of RUN neighbouring columns from n on, of row m: the sums of a group (or of one tile) and their bias
+  auto store_run = [&](auto run_of, int m, int n, const float* sums) {
+    constexpr int RUN = decltype(run_of)::value;
+    if constexpr (OUT == OUT_GATED) {
+      TO* dst = out + (size_t)m * (N / 2) + n / 2;
+      bf16_t gated[RUN / 2];
 #pragma unroll
-  for (int e = 0; e < 8; ++e)
-    bias_here[e] = OUT == OUT_ROTATED ? early.bias[e] : with_bias && (INSIDE || n_piece + e < N) ? load_as_float(bias, bias_is_float, n_piece + e) : 0.f;
-  const int head = OUT == OUT_ROTATED ? n_piece / rotated.dim : 0, d = OUT == OUT_ROTATED ? n_piece % rotated.dim : 0;
+      for (int e = 0; e < RUN / 2; ++e) {
+        // the hardware's 2^x and 1/x, as the result is bfloat16 (a tile has 80 of these a lane; the
+        // library routines are some forty instructions each and took most of a tile's way out)
+        const float gate = sums[2 * e], up = sums[2 * e + 1];
+        gated[e] = (bf16_t)(gate * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gate * -1.44269504088896f)) * up);
+      }
+      if (INSIDE ? N % 16 == 0 : n + RUN <= N && N % 16 == 0) {
+        if constexpr (RUN == 16) store_piece(*(const u32x4*)gated, dst);
+        else if constexpr (RUN == 8) *(uint2*)dst = *(const uint2*)gated;
+        else *(unsigned*)dst = *(const unsigned*)gated;
+      } else {
 #pragma unroll
-  for (int j = 0; j < TM; ++j) {
+        for (int e = 0; e < RUN / 2; ++e)
+          if (n + 2 * e + 1 < N) dst[e] = gated[e];
+      }
+    } else {
+      TO* dst = out + ((size_t)slice * M + m) * N + n;
+      if (INSIDE || (n + RUN <= N && N % 8 == 0)) {
+        if constexpr (sizeof(TO) == 4) {
+          store_piece((f32x4){sums[0], sums[1], sums[2], sums[3]}, dst);
+        } else {
+          bf16_t packed[RUN];
 #pragma unroll
-    for (int i = 0; i < TN; ++i)
+          for (int e = 0; e < RUN; ++e) packed[e] = (bf16_t)sums[e];
+          if constexpr (RUN == 8) store_piece(*(const u32x4*)packed, dst);
+          else *(uint2*)dst = *(const uint2*)packed;
+        }
+      } else {
 #pragma unroll
-      for (int quad = 0; quad < 4; ++quad)
-        *(f32x4*)(mine + (size_t)r32 * ROW + i * 32 + quad * 8 + half * 4) =
-            (f32x4){acc[i][j][quad * 4], acc[i][j][quad * 4 + 1], acc[i][j][quad * 4 + 2], acc[i][j][quad * 4 + 3]};
-    // (a wave reads only what it wrote itself: no barrier, the LDS operations of a wave complete in order)
+        for (int e = 0; e < RUN; ++e)
+          if (n + e < N) dst[e] = from_float<TO>(sums[e]);
+      }
+    }
+  };
+  if constexpr (OUT == OUT_ROTATED) {
+    static_assert(G == 2 && WHOLE == TN, "runs of eight columns");
+    constexpr int ROW = 16 * TN + 4;  // floats of a row of `mine`, padded
+    const int v_first = (rotated.heads + rotated.kv_heads) * rotated.dim;
+    const bool values_too = n_wave + 16 * TN > v_first;
 #pragma unroll
-    for (int pass = 0; pass < 32 / ROWS_A_PASS; ++pass) {
-      const int row = pass * ROWS_A_PASS + row_in_pass;
-      const int m = m_wave + j * 32 + row;
-      const f32x4 lo = *(const f32x4*)(mine + (size_t)row * ROW + piece * 8);
-      const f32x4 hi = *(const f32x4*)(mine + (size_t)row * ROW + piece * 8 + 4);
-      float value[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    for (int j = 0; j < TM; ++j) {
+      const int m = m_wave + j * 16 + r16;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) value[e] += bias_here[e];
-      int slot = 0, page = 0, offset = 0;
-      if constexpr (OUT == OUT_ROTATED) slot = __shfl(early.slot[j], row), page = __shfl(early.page[j], row), offset = __shfl(early.offset[j], row);
-      if (!INSIDE && m >= M) continue;
-      if constexpr (OUT == OUT_ROTATED) {
-        if (!INSIDE && n_piece >= N) continue;  // (N is a multiple of 16)
-        // rounded before they are rotated, as where a kernel of its own reads them from memory
+      for (int i = 0; i < TN / 2; ++i) {
+        const int n = n_wave + i * 32 + q * 8;
+        float value[8];
         bf16_t packed[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) packed[e] = (bf16_t)value[e];
-        if (head < rotated.heads + rotated.kv_heads) {
-          constexpr bool HERE = Early<TN, TM>::PASSES > 0;
-          const f32x4* angles = angles_of(rotated, m, d);
-          const f32x4 first = HERE ? early.angles[HERE ? pass : 0][0] : angles[0], second = HERE ? early.angles[HERE ? pass : 0][1] : angles[1];
+        for (int e = 0; e < 8; ++e) {
+          value[e] = acc[2 * i + e / 4][j][e % 4] + (with_bias ? early_bias(early, i, e, bias_is_float) : 0.f);
+          packed[e] = (bf16_t)value[e];  // rounded before they are rotated, as where a kernel of its own reads them from memory
+        }
+        const int head = n / rotated.dim, d = n % rotated.dim;
+        if (n >= v_first) {
+          *(f32x4*)(mine + (size_t)r16 * ROW + i * 32 + q * 8) = (f32x4){value[0], value[1], value[2], value[3]};  // (for store_values)
+          *(f32x4*)(mine + (size_t)r16 * ROW + i * 32 + q * 8 + 4) = (f32x4){value[4], value[5], value[6], value[7]};
+        } else {
+          const f32x4 first = early.angles[i][j][0], second = early.angles[i][j][1];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float c = e < 2 ? first[2 * e] : second[2 * e - 4], s = e < 2 ? first[2 * e + 1] : second[2 * e - 3];
@@ -193,57 +249,50 @@ __device__ __forceinline__ void store_tiles(const f32x16 (&acc)[TN][TM], float* 
             packed[2 * e] = (bf16_t)x, packed[2 * e + 1] = (bf16_t)y;
           }
         }
-        *(uint4*)(out + (size_t)m * N + n_piece) = *(const uint4*)packed;
-        if (head >= rotated.heads + rotated.kv_heads) {
-          *(f32x4*)(mine + (size_t)row * ROW + piece * 8) = (f32x4){value[0], value[1], value[2], value[3]};  // (for store_values)
-          *(f32x4*)(mine + (size_t)row * ROW + piece * 8 + 4) = (f32x4){value[4], value[5], value[6], value[7]};
-        } else if (head >= rotated.heads && slot >= 0) {
-          bf16_t* keys = rotated.keys + ((size_t)page * rotated.kv_heads + head - rotated.heads) * rotated.page_size * rotated.dim;
-          *(uint4*)(keys + ((size_t)(d / KEY_PIECE) * rotated.page_size + offset) * KEY_PIECE) = *(const uint4*)packed;
-        }
-      } else if constexpr (OUT == OUT_GATED) {
-        TO* dst = out + (size_t)m * (N / 2) + n_piece / 2;
-        float gated[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          // the hardware's 2^x and 1/x, as the result is bfloat16 (a tile has 128 of these a lane; the
-          // library routines are some forty instructions each and took most of a tile's way out)
-          const float gate = value[2 * e], up = value[2 * e + 1];
-          gated[e] = gate * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gate * -1.44269504088896f)) * up;
-        }
-        if (INSIDE || (n_piece + 8 <= N && (N / 2) % 4 == 0)) {
-          bf16_t packed[4] = {(bf16_t)gated[0], (bf16_t)gated[1], (bf16_t)gated[2], (bf16_t)gated[3]};
-          *(uint2*)dst = *(const uint2*)packed;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n_piece + 2 * e + 1 < N) dst[e] = from_float<TO>(gated[e]);
-        }
-      } else {
-        TO* dst = out + ((size_t)slice * M + m) * N + n_piece;
-        if (INSIDE || (n_piece + 8 <= N && N % 8 == 0)) {
-          if (sizeof(TO) == 2) {
-            bf16_t packed[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) packed[e] = (bf16_t)value[e];
-            *(uint4*)dst = *(const uint4*)packed;
-          } else {
-            *(f32x4*)dst = (f32x4){value[0], value[1], value[2], value[3]};
-            *(f32x4*)((float*)dst + 4) = (f32x4){value[4], value[5], value[6], value[7]};
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (n_piece + e < N) dst[e] = from_float<TO>(value[e]);
+        if (!INSIDE && (m >= M || n >= N)) continue;  // (N is a multiple of 16)
+        *(uint4*)(out + (size_t)m * N + n) = *(const uint4*)packed;
+        const int slot = early.slot[j];
+        if (n < v_first && head >= rotated.heads && slot >= 0) {
+          bf16_t* keys = rotated.keys + ((size_t)(slot / rotated.page_size) * rotated.kv_heads + head - rotated.heads) * rotated.page_size * rotated.dim;
+          *(uint4*)(keys + ((size_t)(d / KEY_PIECE) * rotated.page_size + slot % rotated.page_size) * KEY_PIECE) = *(const uint4*)packed;
         }
       }
+      if (values_too) store_values<TN, ROW>(rotated, mine, early.slot[j], N, n_wave, lane);  // (a wave reads only what it wrote itself: no barrier)
     }
-    if constexpr (OUT == OUT_ROTATED) store_values<TN, TM, ROW>(rotated, mine, early, j, N, n_wave, lane);
+  } else {
+    float bias_here[TN][4];
+    if (with_bias) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int n = n_wave + weight_row<TN, G>(i, q * 4 + e);
+          bias_here[i][e] = INSIDE || n < N ? load_as_float(bias, bias_is_float, n) : 0.f;
+        }
+    }
+    auto sum_at = [&](int i, int j, int e) { return with_bias ? acc[i][j][e] + bias_here[i][e] : acc[i][j][e]; };
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const int m = m_wave + j * 16 + r16;
+      if (!INSIDE && m >= M) continue;
+#pragma unroll
+      for (int i = 0; i < WHOLE; i += G) {
+        float sums[4 * G];
+#pragma unroll
+        for (int e = 0; e < 4 * G; ++e) sums[e] = sum_at(i + e / 4, j, e % 4);
+        store_run(std::integral_constant<int, 4 * G>{}, m, n_wave + i * 16 + q * 4 * G, sums);
+      }
+#pragma unroll
+      for (int i = WHOLE; i < TN; ++i) {
+        float sums[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sums[e] = sum_at(i, j, e);
+        store_run(std::integral_constant<int, 4>{}, m, n_wave + i * 16 + q * 4, sums);
+      }
+    }
   }
 }
 
-// The reads of LDS are written as instructions, with their waits: left to the compiler, every read of LDS waits for all
-// loads into LDS that are under way, whichever stage they fill.  What a read brings is used only after `arrived`.
 template <int N>
 __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -262,15 +311,41 @@ __device__ __forceinline__ void wait_stages(int younger) {
   }
 }
 
-// WN x WM waves of TN x TM tiles; stages of BK k; A_SIMD: the waves a SIMD is to hold.
-template <int WN, int WM, int TN, int TM, int BK, int STAGES, int A_SIMD, typename TO, int OUT>
+// The order in which a wave reads its operands of 32 k from LDS.  The products of such a step go x tile by x tile (group j: x tile j with all the
+// weight tiles), and the reads run AHEAD x tiles ahead of them, into SLOTS sets of registers in turn; the weight tiles have two sets, one a step.
+// Behind the first product of group j come: of this step x tile j + AHEAD, while there is one (groups before FIRST); in group TURN the weight tiles of
+// the next step and its x tiles that are due by then; later, one x tile of the next step a group.  At TURN nothing of this step is still to be read.
+template <int TN, int TM, int AHEAD>
+struct Reads {
+  static constexpr int SLOTS = AHEAD < TM ? AHEAD + 1 : 2 * TM, FIRST = TM - AHEAD, TURN = FIRST == 0 ? 0 : FIRST + 1 < TM ? FIRST + 1 : TM - 1;
+  static constexpr int AT_TURN = TURN - FIRST + 1;  // x tiles of the next step read in group TURN
+  static_assert(AHEAD >= 1 && AHEAD <= TM && 2 * TM % SLOTS == 0, "two steps take whole turns of the registers");
+  static constexpr int in_group(int j) { return j < FIRST ? 1 : j < TURN ? 0 : j == TURN ? TN + AT_TURN : 1; }
+  // how many reads are younger than x tile j's when group j begins (the weight tiles' are older than x tile 0's)
+  static constexpr int younger(int j) {
+    int count = 0;
+    if (j >= AHEAD) {
+      for (int g = j - AHEAD + 1; g < j; ++g) count += in_group(g);
+      return count;
+    }
+    for (int g = 0; g < j; ++g) count += in_group(g);
+    const int asked = FIRST + j;  // in the step before, in this group or, all at once, in TURN
+    for (int g = (asked > TURN ? asked : TURN) + 1; g < TM; ++g) count += in_group(g);
+    return count + (asked < TURN ? TURN - asked : 0);
+  }
+};
+
+// WN x WM waves of TN x TM tiles of 16 x 16; stages of 64 k, of which the last may be half full (HALF: K / splits % 64 == 32); A_SIMD: the waves a
+// SIMD is to hold; AHEAD: see Reads.
+template <int WN, int WM, int TN, int TM, int AHEAD, int STAGES, int A_SIMD, bool HALF, typename TO, int OUT>
 __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                           const void* __restrict__ bias, int bias_is_float,
                                                                           TO* __restrict__ out, int M, int N, int K, int k_split, Rotated rotated) {
-  constexpr int THREADS = WN * WM * 64, BN = WN * TN * 32, BM = WM * TM * 32, SLOTS = BK / 8, HALVES = BK / 16;
+  constexpr int BK = 64, THREADS = WN * WM * 64, BN = WN * TN * 16, BM = WM * TM * 16, SLOTS = BK / 8;
   constexpr int ROW_BYTES = BK * 2, W_BYTES = BN * ROW_BYTES, STAGE_BYTES = W_BYTES + BM * ROW_BYTES;
   constexpr int PER_W = BN * SLOTS / THREADS, PER = PER_W + BM * SLOTS / THREADS;  // 16-byte pieces of a stage a lane asks for
-  static_assert(BN * SLOTS % THREADS == 0 && BM * SLOTS % THREADS == 0 && HALVES % 2 == 0 && STAGES >= 2, "shape");
+  static_assert(BN * SLOTS % THREADS == 0 && BM * SLOTS % THREADS == 0 && STAGES >= 2, "shape");
+  using Order = Reads<TN, TM, AHEAD>;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wave_n = wave % WN, wave_m = wave / WN;
@@ -278,42 +353,44 @@ __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const 
   tile_of_workgroup(blockIdx.x, (N + BN - 1) / BN, (M + BM - 1) / BM, tile_n, tile_m);
   const int n0 = tile_n * BN, m0 = tile_m * BM;
   const int k_first = blockIdx.z * k_split;
-  const int r32 = lane & 31, half = lane >> 5;
-  auto swizzle = [](int row) { return BK == 64 ? (row >> 1) & 7 : ((((row >> 1) ^ (row >> 3)) & 1) | (((row >> 2) & 1) << 1)); };
+  const int r16 = lane & 15, q = lane >> 4;
+  auto swizzle = [](int row) { return (row >> 1) & 7; };
+  const int steps = (k_split + BK - 1) / BK, last = steps - 1;
 
   // where this lane's pieces of a stage come from: piece -> (row, slot), the slot holds part slot ^ swizzle(row)
-  // (rows beyond the operand are read as its last one: their results are dropped)
+  // (rows beyond the operand are read as its last one: their results are dropped; of a half stage the parts beyond it are read as the
+  // parts before: nothing multiplies them)
   const bf16_t* src[PER];
+  bool beyond[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int piece = (i < PER_W ? i : i - PER_W) * THREADS + threadIdx.x;
     const int row = piece / SLOTS, part = (piece % SLOTS) ^ swizzle(row);
-    src[i] = (i < PER_W ? w + (size_t)min(n0 + row, N - 1) * K : x + (size_t)min(m0 + row, M - 1) * K) + k_first + part * 8;
+    const int row_w = row / (TN * 16) * (TN * 16) + weight_row<TN, group_of<TO, OUT, TN>()>(row % (TN * 16) / 16, row % 16);
+    src[i] = (i < PER_W ? w + (size_t)min(n0 + row_w, N - 1) * K : x + (size_t)min(m0 + row, M - 1) * K) + k_first + part * 8;
+    beyond[i] = part >= SLOTS / 2;
   }
   auto load_piece = [&](int i, int step, unsigned stage) {
     unsigned char* to = lds + stage * STAGE_BYTES + (i < PER_W ? i * THREADS * 16 : W_BYTES + (i - PER_W) * THREADS * 16) + wave * 1024;
-    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(src[i] + step * BK),
-                                     (void __attribute__((address_space(3)))*)to, 16, 0, 0);
+    const bf16_t* from = src[i] + step * BK - (HALF && step == last && beyond[i] ? BK / 2 : 0);
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)from, (void __attribute__((address_space(3)))*)to, 16, 0, 0);
   };
-  // where it reads its operands: rows r32 + 32 t of the wave's, part 2 * sixteen + half
+  // where it reads its operands: rows r16 + 16 t of the wave's, part 4 * step of 32 k + q
   const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
-  const int turned = swizzle(r32);
-  const unsigned row_w = base + (unsigned)(wave_n * TN * 32 + r32) * ROW_BYTES;
-  const unsigned row_x = base + W_BYTES + (unsigned)(wave_m * TM * 32 + r32) * ROW_BYTES;
+  const int turned = swizzle(r16);
+  const unsigned row_w = base + (unsigned)(wave_n * TN * 16 + r16) * ROW_BYTES;
+  const unsigned row_x = base + W_BYTES + (unsigned)(wave_m * TM * 16 + r16) * ROW_BYTES;
 
   Early<TN, TM> early;
   if constexpr (OUT == OUT_ROTATED)
-    ask_early(early, rotated, bias, bias_is_float, M, N, n0 + wave_n * TN * 32, m0 + wave_m * TM * 32, lane);
+    ask_early(early, rotated, bias, bias_is_float, M, N, n0 + wave_n * TN * 16, m0 + wave_m * TM * 16, lane);
 
-  f32x16 acc[TN][TM];  // [tile of weight rows][tile of x rows]
+  f32x4 acc[TN][TM];  // [tile of weight rows][tile of x rows]
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
-    for (int j = 0; j < TM; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  const int steps = k_split / BK, last = steps - 1;
 #pragma unroll
   for (int s = 0; s < STAGES; ++s)
     if (s < steps) {
@@ -322,127 +399,163 @@ __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const 
     }
   wait_stages<PER, STAGES - 1>(min(last, STAGES - 1));  // stage 0 has landed
   __builtin_amdgcn_s_barrier();
-  bf16x8 a[2][TN], b[2][TM];  // two sets of operands
-  // operand o of a set (the weight tiles', then x's) from `at` behind the wave's rows
-#define READ_OPERAND(set, o, at)                                                                                            \
-  do {                                                                                                                      \
-    if ((o) < TN)                                                                                                           \
-      asm volatile("ds_read_b128 %0, %1 offset:%2"                                                                          \
-                   : "=v"(a[set][(o) < TN ? (o) : 0]) : "v"(row_w + (at)), "n"(((o) < TN ? (o) : 0) * 32 * ROW_BYTES) : "memory"); \
-    else                                                                                                                    \
-      asm volatile("ds_read_b128 %0, %1 offset:%2"                                                                          \
-                   : "=v"(b[set][(o) < TN ? 0 : (o) - TN]) : "v"(row_x + (at)), "n"(((o) < TN ? 0 : (o) - TN) * 32 * ROW_BYTES) : "memory"); \
-  } while (0)
-  // The operands pass through the statements so that nothing that uses them is moved in front of the wait.
-  auto arrived = [&](int set) {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  // The reads of LDS are written as instructions, with their waits: left to the compiler, every read of LDS waits for all
+  // loads into LDS that are under way, whichever stage they fill.  What a read brings is used only behind a wait that it passes through, so that
+  // nothing that uses it is moved in front of the wait.
+  bf16x8 a[2][TN], b[Order::SLOTS];
+#define READ_TILE(into, row, tile, at) \
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(into) : "v"((row) + (at)), "n"((tile) * 16 * ROW_BYTES) : "memory")
+  auto slot_of = [&](int chunk) { return (unsigned)(((chunk * 4 + q) ^ turned) * 16); };
 #pragma unroll
-    for (int i = 0; i < TN; ++i) asm volatile("" : "+v"(a[set][i]));
+  for (int i = 0; i < TN; ++i) READ_TILE(a[0][i], row_w, i, slot_of(0));
 #pragma unroll
-    for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(b[set][j]));
-  };
-  auto slot_of = [&](int sixteen) { return (unsigned)(((sixteen * 2 + half) ^ turned) * 16); };
-#pragma unroll
-  for (int o = 0; o < TN + TM; ++o) READ_OPERAND(0, o, slot_of(0));
+  for (int j = 0; j < AHEAD; ++j) READ_TILE(b[j], row_x, j, slot_of(0));
   unsigned stage = 0;
-  // A stage with the loads of the one STAGES ahead dealt out between its last products (LOADS), or, at the end of K,
-  // without: two bodies, so that neither has a branch inside.
-  auto one_step = [&](int step, auto with_loads) {
+  // Half a stage (chunk 0 or 1).  In the second one's group TURN this wave holds all it needs of the stage: behind a barrier the next stage is read, and
+  // this one is asked for anew (LOADS), a piece every PACE products, into the next stage's first half: a CU takes 64 bytes a clock from the caches, and
+  // what is asked for faster than that holds up the products behind it.
+  constexpr int LEFT = (TM - Order::TURN) * TN, PACE = LEFT + TM * TN < PER ? 1 : (LEFT + TM * TN) / PER;
+  auto multiply = [&](auto which, auto with_loads, int step) {
+    constexpr int CHUNK = decltype(which)::value;
     constexpr bool LOADS = decltype(with_loads)::value;
-    const unsigned now = stage * STAGE_BYTES;
-    const unsigned next_stage = stage + 1 == STAGES ? 0 : stage + 1;
-    const unsigned then = next_stage * STAGE_BYTES;
+    const unsigned next_stage = stage + 1 == STAGES ? 0 : stage + 1, stage_before = stage == 0 ? STAGES - 1 : stage - 1;
+    const unsigned here = stage * STAGE_BYTES + slot_of(CHUNK), then = CHUNK ? next_stage * STAGE_BYTES + slot_of(0) : stage * STAGE_BYTES + slot_of(1);
+    constexpr int SET = CHUNK, B0 = CHUNK * TM;
 #pragma unroll
-    for (int sixteen = 0; sixteen < HALVES; ++sixteen) {
-      constexpr int FINAL = HALVES - 1;
-      const int set = sixteen & 1;
-      arrived(set);
-      if (sixteen == FINAL) {
-        // this wave holds all it needs of the stage; the next one has to be there, for everybody
+    for (int j = 0; j < TM; ++j) {
+      if (CHUNK && j == Order::TURN) {
+        // (x tile j may still be on its way where TURN is the first group: the wait covers it)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (LOADS) wait_loads<PER * (STAGES - 2)>();
         else wait_stages<PER, STAGES - 2>(max(0, last - (step + 1)));
         __builtin_amdgcn_s_barrier();
+      } else {
+        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(Order::younger(j) < 15 ? Order::younger(j) : 15) : "memory");
       }
-      const unsigned slot = sixteen == FINAL ? then + slot_of(0) : now + slot_of(sixteen + 1);
+      if (j == 0) {
+#pragma unroll
+        for (int i = 0; i < TN; ++i) asm volatile("" : "+v"(a[SET][i]));
+      }
+      asm volatile("" : "+v"(b[(B0 + j) % Order::SLOTS]));
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int p = 0; p < TN * TM; ++p) {
-        const int i = p / TM, j = p % TM;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[set][i], b[set][j], acc[i][j], 0, 0, 0);
-        // two operands of the sixteen k to come behind each of the first products (after the last stage these read a
-        // stage that holds nothing new: they stay inside LDS and nobody uses them)
+      for (int i = 0; i < TN; ++i) {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[SET][i], b[(B0 + j) % Order::SLOTS], acc[i][j], 0, 0, 0);
+        if (j < Order::FIRST && i == 0) READ_TILE(b[(B0 + j + AHEAD) % Order::SLOTS], row_x, j + AHEAD, here);
+        if (j == Order::TURN) {
+          constexpr int COUNT = Order::in_group(Order::TURN), EACH = (COUNT + TN - 1) / TN;
 #pragma unroll
-        for (int o = 2 * p; o < (p + 1 == TN * TM ? TN + TM : min(2 * p + 2, TN + TM)); ++o) READ_OPERAND(set ^ 1, o, slot);
-        if (LOADS && sixteen == FINAL) {
+          for (int r = i * EACH; r < min((i + 1) * EACH, COUNT); ++r) {
+            if (r < TN) READ_TILE(a[SET ^ 1][r < TN ? r : 0], row_w, r < TN ? r : 0, then);
+            else READ_TILE(b[(B0 + TM + (r < TN ? 0 : r - TN)) % Order::SLOTS], row_x, r < TN ? 0 : r - TN, then);
+          }
+        }
+        if (j > Order::TURN && i == 0) READ_TILE(b[(B0 + j + AHEAD) % Order::SLOTS], row_x, j + AHEAD - TM, then);
+        if (LOADS) {
+          // (counted from TURN on; of the last product all that is left)
+          const int place = CHUNK ? (j - Order::TURN) * TN + i : LEFT + j * TN + i;
+          const bool end = CHUNK == 0 && j == TM - 1 && i == TN - 1;
+          if (place >= 0) {
 #pragma unroll
-          for (int q = p; q < PER; q += TN * TM) load_piece(q, step + STAGES, stage);
+            for (int l = (place + PACE - 1) / PACE; l < PER && (end || l * PACE < place + 1); ++l) load_piece(l, CHUNK ? step + STAGES : step - 1 + STAGES, CHUNK ? stage : stage_before);
+          }
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    stage = next_stage;
+    if (CHUNK) stage = next_stage;
   };
+  constexpr std::integral_constant<int, 0> first_half{};
+  constexpr std::integral_constant<int, 1> second_half{};
+  multiply(first_half, std::false_type{}, 0);
   int step = 0;
-  for (; step + STAGES < steps; ++step) one_step(step, std::true_type{});
-  for (; step < steps; ++step) one_step(step, std::false_type{});
-  arrived(0);
-  __syncthreads();  // every wave has read the last stage: LDS is free for the way out
-  const int n_wave = n0 + wave_n * TN * 32, m_wave = m0 + wave_m * TM * 32;
-  float* mine = (float*)lds + (size_t)wave * 32 * (32 * TN + 4);
+  for (; step + STAGES < steps; ++step) {
+    multiply(second_half, std::true_type{}, step);
+    multiply(first_half, std::true_type{}, step + 1);
+  }
+  for (; step < last; ++step) {
+    multiply(second_half, std::false_type{}, step);
+    multiply(first_half, std::false_type{}, step + 1);
+  }
+  if (!HALF) multiply(second_half, std::false_type{}, last);
+  // (what was read behind the last products stays inside LDS and nobody uses it, but its registers are not free before it has come)
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    asm volatile("" ::"v"(a[0][i]));
+    asm volatile("" ::"v"(a[1][i]));
+  }
+#pragma unroll
+  for (int j = 0; j < Order::SLOTS; ++j) asm volatile("" ::"v"(b[j]));
+#undef READ_TILE
+  const int n_wave = n0 + wave_n * TN * 16, m_wave = m0 + wave_m * TM * 16;
+  if constexpr (OUT == OUT_ROTATED) __syncthreads();  // every wave has read the last stage: LDS is free for the values
+  float* mine = (float*)lds + (size_t)wave * 16 * (16 * TN + 4);
+  const bool streamed = (size_t)gridDim.z * M * N * (OUT == OUT_GATED ? sizeof(TO) / 2 : sizeof(TO)) > STREAMED_FROM;
   if (m_wave >= M || n_wave >= N) return;
-  if (m_wave + 32 * TM <= M && n_wave + 32 * TN <= N && N % 8 == 0)
-    store_tiles<TN, TM, true, TO, OUT>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane, rotated, early);
+  if (m_wave + 16 * TM <= M && n_wave + 16 * TN <= N && N % 8 == 0)
+    store_tiles<TN, TM, true, TO, OUT>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane, rotated, early, streamed);
   else
-    store_tiles<TN, TM, false, TO, OUT>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane, rotated, early);
+    store_tiles<TN, TM, false, TO, OUT>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane, rotated, early, streamed);
 }
 
-template <int WN, int WM, int TN, int TM, int BK, int STAGES, int A_SIMD, typename TO, int OUT>
+template <int WN, int WM, int TN, int TM, int AHEAD, int STAGES, int A_SIMD, bool HALF, typename TO, int OUT>
 static int launch_block(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
                         int splits, hipStream_t stream, const Rotated& rotated) {
-  constexpr int BN = WN * TN * 32, BM = WM * TM * 32;
-  constexpr size_t stages = (size_t)STAGES * (BN + BM) * BK * 2, way_out = (size_t)WN * WM * 32 * (32 * TN + 4) * sizeof(float);
-  constexpr size_t bytes = stages > way_out ? stages : way_out;
+  constexpr int BN = WN * TN * 16, BM = WM * TM * 16;
+  constexpr size_t stages = (size_t)STAGES * (BN + BM) * 128, values = OUT == OUT_ROTATED ? (size_t)WN * WM * 16 * (16 * TN + 4) * sizeof(float) : 0;
+  constexpr size_t bytes = stages > values ? stages : values;
   static_assert(bytes <= 160 * 1024, "a CU's LDS");
   static bool asked = false;
   if (!asked) {
-    if (hipFuncSetAttribute((const void*)gemm_block_kernel<WN, WM, TN, TM, BK, STAGES, A_SIMD, TO, OUT>,
+    if (hipFuncSetAttribute((const void*)gemm_block_kernel<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
       return ERR_BAD_ARGUMENT;
     asked = true;
   }
-  hipLaunchKernelGGL((gemm_block_kernel<WN, WM, TN, TM, BK, STAGES, A_SIMD, TO, OUT>),
+  hipLaunchKernelGGL((gemm_block_kernel<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT>),
                      dim3(((N + BN - 1) / BN) * ((M + BM - 1) / BM), 1, splits), dim3(WN * WM * 64), bytes, stream, (const bf16_t*)x,
                      (const bf16_t*)w, bias, bias_is_float, (TO*)out, M, N, K, K / splits, rotated);
   return LAUNCH_STATUS();
 }
 
-// The shapes: a tile's weight rows and rows of x, how many a CU holds at a time, and what a launch, a tile, and a tile's
-// 64 k take, us (the last where few CUs are busy, and where all are: their clock is lower and they share L2).  Fitted to
-// 88 products of 96 to 2,048 rows with the weights of the 1.5B and 7B sizes, whole and in parts, each shape within 9 to 14
-// percent of what was measured; the shape picked by them is 4 percent slower than the best one on average.
+// The shapes: a tile's weight rows and rows of x, how many a CU holds at a time, and what a launch, a tile, a tile's
+// 64 k (where few CUs are busy, and where all are: their clock is lower and they share L2) and a million bytes of the result take, us.  Fitted to
+// 430 products of 96 to 2,048 rows with seventeen weights (K of 896 to 18,944), whole and in parts, x written by the kernel before and every weight
+// out of memory, each shape within 9 percent of what was measured; the shape picked by them is 2 to 3 percent slower than the best one on average.  Of
+// sixteen shapes measured these ten miss the least: without 160 x 160, 128 x 160, 192 x 128, 96 x 128 and 128 x 96 the best one left is 3 percent
+// slower on average.
 struct BlockShape {
   int n, m, a_cu;
-  float launch, tile, alone, busy;
+  float launch, tile, alone, busy, a_million;
 };
-static const BlockShape SHAPES[] = {{256, 256, 1, 0.95f, 7.25f, 1.195f, 2.156f}, {256, 320, 1, 1.99f, 8.13f, 1.347f, 2.404f},
-                                    {256, 128, 1, 1.75f, 4.71f, 0.699f, 1.156f}, {128, 128, 1, 1.51f, 3.95f, 0.443f, 0.645f},
-                                    {128, 64, 2, 3.98f, 0.74f, 0.336f, 0.866f},  {64, 64, 2, 3.68f, 1.08f, 0.235f, 0.492f}};
-#define SHAPE_COUNT 6
+static const BlockShape SHAPES[] = {{256, 256, 1, 7.30f, 0.89f, 1.337f, 1.426f, 0.243f}, {256, 320, 1, 10.40f, 0.00f, 1.429f, 1.799f, 0.238f},
+                                    {128, 256, 1, 5.74f, 0.00f, 0.668f, 0.884f, 0.348f}, {192, 128, 1, 3.33f, 2.10f, 0.673f, 0.673f, 0.278f},
+                                    {160, 160, 1, 5.35f, 0.53f, 0.616f, 0.737f, 0.297f}, {128, 160, 1, 3.89f, 0.80f, 0.554f, 0.616f, 0.336f},
+                                    {96, 128, 1, 2.90f, 1.31f, 0.460f, 0.443f, 0.290f}, {128, 96, 1, 3.01f, 0.72f, 0.448f, 0.397f, 0.372f},
+                                    {64, 128, 2, 3.90f, 0.00f, 0.389f, 0.777f, 0.238f}, {64, 64, 2, 4.78f, 0.00f, 0.225f, 0.484f, 0.171f}};
+#define SHAPE_COUNT 10
 
-static float shape_us(const BlockShape& t, int M, int N, int K, int splits) {
+static float shape_us(const BlockShape& t, int M, int N, int K, int splits, int bytes) {  // (`bytes` of a column of the product in the result)
   const long groups = (long)((N + t.n - 1) / t.n) * ((M + t.m - 1) / t.m) * splits;
   const long places = 256L * t.a_cu, full = groups / places, rest = groups % places;
   const float steps = (float)(K / splits) / 64.f;
-  float us = t.launch + (float)full * (t.tile + steps * t.busy);
+  float us = t.launch + t.a_million * 1e-6f * (float)bytes * splits * M * N + (float)full * (t.tile + steps * t.busy);
   if (rest) us += t.tile + steps * fmaxf(t.alone, t.busy * (float)rest / (float)places);
   return us;
 }
 
-static int pick_shape(int M, int N, int K, int splits) {
+static int pick_shape(int M, int N, int K, int splits, int bytes) {
   int best = 0;
   for (int s = 1; s < SHAPE_COUNT; ++s)
-    if (shape_us(SHAPES[s], M, N, K, splits) < shape_us(SHAPES[best], M, N, K, splits)) best = s;
+    if (shape_us(SHAPES[s], M, N, K, splits, bytes) < shape_us(SHAPES[best], M, N, K, splits, bytes)) best = s;
   return best;
+}
+
+// Which of the shapes a product takes (its place in SHAPES): `kind` 0 plain bfloat16, 1 float32, 2 gated.
+extern "C" int llmserve_gemm_blocks_shape(int M, int N, int K, int splits, int kind) {
+  if (M <= 0 || N <= 0 || K <= 0 || splits < 1 || kind < 0 || kind > 2) return -1;
+  return pick_shape(M, N, K, splits, kind == 0 ? 2 : kind == 1 ? 4 : 1);
 }
 
 // Into how many parts of K (at most 12, of whole stages) the product is best cut where its float32 result may stay partial
@@ -454,7 +567,7 @@ extern "C" int llmserve_gemm_blocks_parts(int M, int N, int K) {
   float best_us = 0.f;
   for (int splits = 1; splits <= 12; ++splits) {
     if (K % (splits * stage)) continue;
-    const float us = shape_us(SHAPES[pick_shape(M, N, K, splits)], M, N, K, splits) + (float)splits * M * N * 4e-6f / 4.5f;
+    const float us = shape_us(SHAPES[pick_shape(M, N, K, splits, 4)], M, N, K, splits, 4) + (float)splits * M * N * 4e-6f / 4.5f;
     if (splits == 1 || us < best_us) best = splits, best_us = us;
   }
   return best;
@@ -464,18 +577,22 @@ template <typename TO, int OUT>
 static int launch_shape(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
                         int splits, hipStream_t stream) {
 #define BLOCK(...) return launch_block<__VA_ARGS__, TO, OUT>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, {})
-  const int shape = pick_shape(M, N, K, splits);
-  if ((K / splits) % 64) {  // a K that ends in half a stage: stages of 32
-    if (shape < 3) BLOCK(2, 4, 4, 2, 32, 5, 2);
-    BLOCK(2, 2, 2, 2, 32, 4, 2);
+  const int shape = pick_shape(M, N, K, splits, OUT == OUT_GATED ? sizeof(TO) / 2 : sizeof(TO));
+  if ((K / splits) % 64) {  // a K that ends in half a stage
+    if (shape < 3) BLOCK(4, 2, 4, 8, 3, 2, 2, true);
+    BLOCK(2, 2, 4, 4, 4, 5, 2, true);
   }
   switch (shape) {
-    case 0: BLOCK(2, 4, 4, 2, 64, 2, 2);
-    case 1: BLOCK(4, 2, 2, 5, 64, 2, 2);
-    case 2: BLOCK(4, 2, 2, 2, 64, 3, 2);
-    case 3: BLOCK(2, 2, 2, 2, 64, 5, 1);
-    case 4: BLOCK(2, 2, 2, 1, 64, 3, 2);
-    default: BLOCK(2, 2, 1, 1, 64, 5, 2);
+    case 0: BLOCK(4, 2, 4, 8, 3, 2, 2, false);
+    case 1: BLOCK(4, 2, 4, 10, 4, 2, 2, false);
+    case 2: BLOCK(2, 4, 4, 4, 4, 3, 2, false);
+    case 3: BLOCK(2, 2, 6, 4, 4, 4, 2, false);
+    case 4: BLOCK(2, 2, 5, 5, 4, 4, 2, false);
+    case 5: BLOCK(2, 2, 4, 5, 4, 4, 2, false);
+    case 6: BLOCK(2, 2, 3, 4, 4, 5, 2, false);
+    case 7: BLOCK(2, 2, 4, 3, 3, 5, 2, false);
+    case 8: BLOCK(2, 2, 2, 4, 4, 3, 2, false);
+    default: BLOCK(2, 2, 2, 2, 2, 5, 2, false);
   }
 #undef BLOCK
 }
@@ -494,20 +611,19 @@ extern "C" int llmserve_gemm_blocks(const void* x, const void* w, const void* bi
 }
 
 // A product whose heads are rotated on the way out, in the smallest tile of which one round of 256 workgroups holds the result, as
-// more CUs then bring the operands.  Us at N 2,048 K 1,536, tiles of 64 x 32, 64 x 64, 128 x 64 and 128 x 128 (without the values' way to
-// their pages): 96 rows 10.4 10.9 16.1 21.1, 256 rows 10.6 11.4 16.4 22.8, 512 rows 13.7 11.7 16.4 22.4, 1,024 rows 26.8 16.6 16.9 23.8,
-// 2,048 rows 48.5 31.2 25.3 24.8; at N 4,608 K 3,584: 96 rows 19.2 19.9 30.0 37.6, 192 rows 26.6 21.3 30.7 36.0.  What it saves is a launch and
-// the rows' way to memory and back: with the kernel that rotates and stores behind the library's product 15.5 us at 96 rows of N 2,048 K 1,536, here
-// 11.6; 16.1 -> 11.7 at 256, 27.3 -> 26.0 at 2,048.  (Places, bias and angles asked for only on the way out: 13.4 at 96 rows.)
+// more CUs then bring the operands.  Us at N 2,048 K 1,536: 96 rows 8.2, 287 rows 9.9, 512 rows 9.0, 1,024 rows 13.4, 2,048 rows 21.6 (before the loads were
+// spread over the products, and with bias and places waited for before the first stage 10.6, 11.7, 11.9, 15.3, 22.5); in the smallest tile that does not
+// make one round, measured then: 512 rows of 64 x 32 13.7, of 64 x 64 11.7, 1,024 rows of 64 x 64 26.8, of 128 x 64 16.6.  What it saves is a launch and
+// the rows' way to memory and back: with the kernel that rotates and stores behind the library's product 15.5 us at 96 rows, 27.3 at 2,048.
 static int launch_rotated(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
                           hipStream_t stream, const Rotated& rotated) {
 #define BLOCK(...) return launch_block<__VA_ARGS__, bf16_t, OUT_ROTATED>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, rotated)
   auto one_round = [&](int n, int m) { return (long)((N + n - 1) / n) * ((M + m - 1) / m) <= 256; };
-  if (K % 64) BLOCK(2, 2, 2, 2, 32, 4, 2);  // (a K that ends in half a stage, which the entry point takes; `_rotated_ahead` leaves it to the two kernels)
-  if (one_round(64, 32)) BLOCK(2, 1, 1, 1, 64, 5, 2);
-  if (one_round(64, 64)) BLOCK(2, 2, 1, 1, 64, 5, 2);
-  if (one_round(128, 64)) BLOCK(2, 2, 2, 1, 64, 3, 2);
-  BLOCK(2, 2, 2, 2, 64, 5, 1);
+  if (K % 64) BLOCK(2, 2, 4, 4, 4, 5, 2, true);  // (a K that ends in half a stage, which the entry point takes; `_rotated_ahead` leaves it to the two kernels)
+  if (one_round(64, 32)) BLOCK(2, 1, 2, 2, 2, 5, 2, false);
+  if (one_round(64, 64)) BLOCK(2, 2, 2, 2, 2, 5, 2, false);
+  if (one_round(128, 64)) BLOCK(2, 2, 4, 2, 2, 3, 2, false);
+  BLOCK(2, 2, 4, 4, 4, 5, 2, false);
 #undef BLOCK
 }
 

@@ -80,6 +80,7 @@ _SIGNATURES = {
     "llmserve_gemm_rotated": "pppipiipiiipppip",
     "llmserve_gemm_blocks": "pppipiiiiiip",
     "llmserve_gemm_blocks_parts": "iii",
+    "llmserve_gemm_blocks_shape": "iiiii",
     "llmserve_attention_generic": "pipiipppippiiiiifipfpiiipip",
     "llmserve_attention_f32": "pipipppppippiiiiiifiipfpiiipip",
     "llmserve_attention_tiles": "pipipppppippiiiiiifiiipippfpiipiiifffpiiipiip",

@@ -151,6 +151,35 @@ def test_tiles_of_many_rows(own_kernels, rows, inner, outer):
         torch.testing.assert_close(parts.double().sum(0), expected, **bound)
 
 
+@pytest.mark.parametrize("shape,rows,plain,float32,gated,inner", [
+    (0, 700, 15681, 13070, None, 512), (0, 1300, None, None, 8964, 512), (1, 1025, 13057, 13059, None, 512), (1, 1300, None, None, 10892, 512),
+    (2, 700, 8200, None, 8212, 512), (2, 700, None, 8167, None, 576), (3, 321, 10881, 10888, 10890, 512), (4, 513, 9798, 9796, None, 512),
+    (4, 1025, None, None, 5378, 512), (5, 300, 10185, 11016, 9712, 512), (6, 2047, 1421, None, 1420, 512), (6, 161, None, 11523, None, 512),
+    (7, 161, 10113, 12297, 9542, 512), (8, 97, 9985, 10565, 9666, 512), (9, 97, 614, 603, 612, 512),
+])
+def test_every_shape_of_a_tile(kernels, shape, rows, plain, float32, gated, inner):
+    """Each shape of the LDS-tiled product where it is picked, at rows and weight rows that leave remainders, in each kind of result.  Bounds as in
+    `test_tiles_of_many_rows`; the hardware's 2^x and 1/x are within a few 2^-23."""
+    k = kernels[torch.bfloat16]
+    generator = torch.Generator(device="cuda").manual_seed(rows)
+    for kind, outer in enumerate((plain, float32, gated)):
+        if outer is None:
+            continue
+        assert k._gemm_blocks.llmserve_gemm_blocks_shape(rows, outer, inner, 1, kind) == shape
+        x = torch.randn(rows, inner, generator=generator, device="cuda").to(torch.bfloat16)
+        w = torch.randn(outer, inner, generator=generator, device="cuda").div_(math.sqrt(inner)).to(torch.bfloat16)
+        b = torch.randn(outer, generator=generator, device="cuda")
+        out = torch.full((rows, outer // 2 if kind == 2 else outer), float("nan"), device="cuda", dtype=torch.float32 if kind == 1 else torch.bfloat16)
+        status = k._gemm_blocks.llmserve_gemm_blocks(
+            x.data_ptr(), w.data_ptr(), b.data_ptr(), 1, out.data_ptr(), int(kind == 1), int(kind == 2), rows, outer, inner, 1, torch.cuda.current_stream().cuda_stream)
+        assert status == 0
+        expected = x.double() @ w.double().T + b.double()
+        if kind == 2:
+            expected = F.silu(expected[:, 0::2]) * expected[:, 1::2]
+        bound = dict(atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5) if kind == 1 else TOLERANCE[torch.bfloat16]
+        torch.testing.assert_close(out.double(), expected, **bound)
+
+
 @pytest.mark.parametrize("rows,inner,outer", [(512, 1536, 2048), (513, 1536, 2048), (2048, 1536, 2048), (2049, 1536, 2048), (513, 64, 1024), (777, 320, 1030), (600, 1536, 1536)])
 def test_small_weights_over_many_rows(kernels, rows, inner, outer):
     """Both sides of the line from which small plain products are the tiled kernel's, with and without leave to split: a route that takes
