@@ -30,6 +30,7 @@
 // model.py:188) to out[M, N / 2].  With `splits` > 1, K is cut over workgroups and `out` is
 // [splits, M, N] partial sums (bias in the first) that the reader adds in order.
 #include "common.h"
+#include <type_traits>
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -361,6 +362,169 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
   }
 }
 
+// gemm_f32_whole (more rows, K in parts of whole stages of 64): a tile of 16 NT weight rows by 16 MT rows of x a workgroup, of which each of its four
+// waves multiplies all with a quarter of every stage's k, in tiles of v_mfma_f32_16x16x4_f32, and whose sums meet through LDS at the end in the order of their
+// k.  So a tile may be any number of sixteens (129 rows make 144, not 160) and have what it takes for one round of 256 workgroups, which is what bounds the kernel
+// above.  Us before (that kernel) -> now, weights out of memory: N 17,920 K 1,536 gated: 65 rows 75 -> 54, 129 rows 105 -> 88, 160 rows 108 -> 96; N 2,048 K
+// 1,536: 65 rows 17 -> 11, 129 rows 24 -> 15, 512 rows 44 -> 35; N 1,536 K 8,960 in parts: 129 rows 60 -> 44, 384 rows 105 -> 103.  Both operands go from memory straight into LDS, as in gemm_blocks.hip: a stage is 64 k, 256 bytes a row, piece p of 16 of row r in slot
+// p ^ (r % 16), so that the sixteen rows that LDS serves together hit all its banks; element j of each lane's piece goes to instruction j, so that an instruction
+// takes k = 4 g + j of a wave's sixteen.  A wave holds all it needs of a stage when it begins to multiply it: behind one barrier the stage is asked for
+// anew, and the next one's operands are read, between the products.
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+constexpr int whole_stages(int rows) { return rows <= 64 ? 4 : rows < 208 ? 3 : 2; }
+constexpr int WHOLE_BATCH = 32;  // tiles whose sums meet at a time: a KB of each of four waves
+
+template <int NT, int MT, bool GATED>
+__global__ __launch_bounds__(256, 1) void gemm_f32_whole_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                const float* __restrict__ bias, float* __restrict__ out, int M, int N, int K,
+                                                                int k_split, int tiles_m, int tiles_n) {
+  constexpr int PER = NT + MT, ROWS = PER * 16, STAGES = whole_stages(ROWS), STAGE_BYTES = ROWS * 256;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r = lane & 15, g = lane >> 4;
+  const int tile = tile_of_workgroup(blockIdx.x, tiles_m * tiles_n);
+  const int n0 = tile / tiles_m * (NT * 16), m0 = tile % tiles_m * (MT * 16);
+  const int steps = k_split / 64, last = steps - 1;
+
+  // what this thread brings of a stage: of row threadIdx.x / 16 of every sixteen the piece that its slot holds (rows beyond the operand are read as
+  // its last one: their results are dropped)
+  const float* src[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int row = threadIdx.x >> 4, part = (threadIdx.x & 15) ^ row;
+    src[i] = (i < NT ? w + (size_t)min(n0 + i * 16 + row, N - 1) * K : x + (size_t)min(m0 + (i - NT) * 16 + row, M - 1) * K) +
+             (size_t)blockIdx.y * k_split + part * 4;
+  }
+  auto load_piece = [&](int i, int step, unsigned stage) {
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(src[i] + step * 64),
+                                     (void __attribute__((address_space(3)))*)(lds + stage * STAGE_BYTES + i * 4096 + wave * 1024), 16, 0, 0);
+  };
+  const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)lds + (unsigned)(r * 256 + ((wave * 4 + g) ^ r) * 16);
+
+  f32x4 acc[NT][MT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s)
+    if (s < steps) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i) load_piece(i, s, s);
+    }
+  // waits until the stage behind `step` has landed, of which `younger` are under way
+  auto landed = [&](int younger) {
+    if (STAGES > 3 && younger >= 3) wait_loads<(STAGES > 3 ? 3 : 0) * PER>();
+    else if (STAGES > 2 && younger == 2) wait_loads<(STAGES > 2 ? 2 : 0) * PER>();
+    else if (younger >= 1) wait_loads<PER>();
+    else wait_loads<0>();
+  };
+  landed(min(last, STAGES - 1));
+  __builtin_amdgcn_s_barrier();
+  // (the reads of LDS as instructions with their waits, as in gemm_blocks.hip; a set of operands is used behind the wait that it passes through)
+  f32x4 operand[2][PER];  // the weights' tiles, then x's
+#define READ_TILE(set, o, at) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(operand[set][o]) : "v"(base + (at)), "n"((o) * 4096) : "memory")
+#pragma unroll
+  for (int o = 0; o < PER; ++o) READ_TILE(0, o, 0u);
+  unsigned stage = 0;
+  auto multiply = [&](auto which, int step) {
+    constexpr int SET = decltype(which)::value;
+    const unsigned next_stage = stage + 1 == STAGES ? 0 : stage + 1;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int o = 0; o < PER; ++o) asm volatile("" : "+v"(operand[SET][o]));
+    landed(min(max(0, last - (step + 1)), STAGES - 2));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    const bool more = step + STAGES < steps;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(operand[SET][i][e], operand[SET][NT + j][e], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int o = j * PER / MT; o < (j + 1) * PER / MT; ++o) {  // (behind the last stage these read one that holds nothing new, and nobody uses them)
+        READ_TILE(SET ^ 1, o, next_stage * STAGE_BYTES);
+        if (more) load_piece(o, step + STAGES, stage);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    stage = next_stage;
+  };
+  int step = 0;
+  for (; step + 1 < steps; step += 2) {
+    multiply(std::integral_constant<int, 0>{}, step);
+    multiply(std::integral_constant<int, 1>{}, step + 1);
+  }
+  if (step < steps) multiply(std::integral_constant<int, 0>{}, step);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int o = 0; o < PER; ++o) {
+    asm volatile("" ::"v"(operand[0][o]));
+    asm volatile("" ::"v"(operand[1][o]));
+  }
+#undef READ_TILE
+
+  // D[n][m] of a tile: a lane holds column m = r and rows n = 4 g .. + 3
+  const bool with_bias = bias && blockIdx.y == 0;
+  f32x4* sums = (f32x4*)lds;
+#pragma unroll
+  for (int first = 0; first < NT * MT; first += WHOLE_BATCH) {
+    __syncthreads();
+#pragma unroll
+    for (int t = first; t < min(first + WHOLE_BATCH, NT * MT); ++t) sums[((t - first) * 4 + wave) * 64 + lane] = acc[t / MT][t % MT];
+    __syncthreads();
+    for (int t = first + wave; t < min(first + WHOLE_BATCH, NT * MT); t += 4) {
+      f32x4 total = sums[((t - first) * 4) * 64 + lane];
+#pragma unroll
+      for (int v = 1; v < 4; ++v) total += sums[((t - first) * 4 + v) * 64 + lane];
+      const int m = m0 + t % MT * 16 + r, n = n0 + t / MT * 16 + 4 * g;
+      if (m >= M || n >= N) continue;
+      if (with_bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) total[e] += bias[min(n + e, N - 1)];
+      }
+      if (GATED) {
+        float* dst = out + (size_t)m * (N / 2) + n / 2;
+        if (n + 1 < N) dst[0] = silu(total[0]) * total[1];
+        if (n + 3 < N) dst[1] = silu(total[2]) * total[3];
+      } else {
+        float* dst = out + ((size_t)blockIdx.y * M + m) * N + n;
+        if (n + 3 < N && (N & 3) == 0) {
+          *(f32x4*)dst = total;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) dst[e] = total[e];
+        }
+      }
+    }
+  }
+}
+
+template <int NT, int MT, bool GATED>
+static int launch_whole(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, int splits, hipStream_t stream) {
+  constexpr int ROWS = (NT + MT) * 16, staged = whole_stages(ROWS) * ROWS * 256, met = (NT * MT < WHOLE_BATCH ? NT * MT : WHOLE_BATCH) * 4096;
+  constexpr int bytes = staged > met ? staged : met;
+  static_assert(bytes <= 160 * 1024, "a CU's LDS");
+  static bool asked = false;
+  if (!asked) {
+    if (hipFuncSetAttribute((const void*)gemm_f32_whole_kernel<NT, MT, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)
+      return ERR_BAD_ARGUMENT;
+    asked = true;
+  }
+  const int tiles_m = (M + 16 * MT - 1) / (16 * MT), tiles_n = (N + 16 * NT - 1) / (16 * NT);
+  hipLaunchKernelGGL((gemm_f32_whole_kernel<NT, MT, GATED>), dim3(tiles_m * tiles_n, splits), dim3(256), bytes, stream, x, w, bias, out, M, N, K,
+                     K / splits, tiles_m, tiles_n);
+  return LAUNCH_STATUS();
+}
+
 template <int WN, int WM, int WK, int TN, int TM, int AHEAD, bool GATED>
 static int launch_tiles(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, int splits,
                         hipStream_t stream) {
@@ -392,11 +556,47 @@ static float tiled_us(const TileCost& t, int M, int N, int K, int splits) {
          (splits > 1 ? (float)splits * M * N * 8e-6f / 4.5f : 0.f);
 }
 
-static int pick_tile(int M, int N, int K, int splits) {
-  int best = 0;
-  for (int t = 1; t < 5; ++t)
+// The tiles of the kernel of whole tiles, in sixteens, and what a launch, a tile and a tile's 64 k (where few CUs are busy, and where all are) take, us; a
+// million bytes of the result 0.3.  Fitted to 90 products of 65 to 512 rows of five weights, in one to seven parts, every weight out of memory, each tile within
+// 2 to 7 percent of what was measured.  Of nineteen tiles measured these seven miss the best one by 0.2 percent on average.
+#define WHOLE_TILES(X) X(1, 3) X(1, 5) X(2, 2) X(2, 3) X(3, 3) X(3, 5) X(5, 5)
+struct WholeTile {
+  int n, m;
+  float launch, tile, alone, busy;
+};
+static const WholeTile WHOLES[] = {{1, 3, 4.04f, 0.10f, 0.247f, 0.287f}, {1, 5, 3.87f, 0.11f, 0.419f, 0.251f}, {2, 2, 3.45f, 0.25f, 0.328f, 0.018f},
+                                   {2, 3, 3.77f, 0.00f, 0.475f, 0.289f}, {3, 3, 3.53f, 0.00f, 0.720f, 0.515f}, {3, 5, 1.60f, 2.07f, 1.186f, 1.091f},
+                                   {5, 5, 1.92f, 3.12f, 1.861f, 1.561f}};
+constexpr int WHOLE_COUNT = sizeof(WHOLES) / sizeof(WHOLES[0]), TILE_COUNT = 5;
+
+static float whole_us(const WholeTile& t, int M, int N, int K, int splits) {
+  if (K % (64 * splits) || M > 512) return 1e30f;  // (this kernel takes whole stages; more rows have not been measured but for a few, of which half were behind)
+  const long groups = (long)((N + 16 * t.n - 1) / (16 * t.n)) * ((M + 16 * t.m - 1) / (16 * t.m)) * splits, full = groups / 256, rest = groups % 256;
+  const float steps = (float)(K / splits / 64), result = 4e-6f * (float)splits * M * N;  // (a gated one is half as large)
+  float us = t.launch + 0.3f * result + (float)full * (t.tile + steps * fmaxf(t.alone, t.busy));
+  if (rest) us += t.tile + steps * fmaxf(t.alone, t.busy * (float)rest / 256.f);
+  return us + (splits > 1 ? result / 4.5f : 0.f);
+}
+
+// How far the other kernel's tiles are from their own estimates beside these (the choice by both is 1 percent slower than the best of all tiles on average and 19
+// percent faster than that kernel alone; of 90 products one was 1 percent slower than that.  200 rows of N 17,920 K 1,536 126 -> 132 us, 300 rows of N 1,536 K 1,536 20.6 -> 18.9)
+static const float BESIDE_WHOLE[TILE_COUNT] = {0.95f, 0.95f, 1.f, 1.2f, 1.2f};
+// The tile that a product takes (first those of the kernel above, then the whole ones) and what it is estimated to take.
+static int pick_tile(int M, int N, int K, int splits, float* us = nullptr) {
+  int best = 0, whole = 0;
+  for (int t = 1; t < TILE_COUNT; ++t)
     if (tiled_us(TILE_COSTS[t], M, N, K, splits) < tiled_us(TILE_COSTS[best], M, N, K, splits)) best = t;
-  return best;
+  for (int t = 1; t < WHOLE_COUNT; ++t)
+    if (whole_us(WHOLES[t], M, N, K, splits) < whole_us(WHOLES[whole], M, N, K, splits)) whole = t;
+  const float apart = tiled_us(TILE_COSTS[best], M, N, K, splits), here = whole_us(WHOLES[whole], M, N, K, splits);
+  const bool ahead = here < BESIDE_WHOLE[best] * apart;
+  if (us) *us = ahead ? here : apart;
+  return ahead ? TILE_COUNT + whole : best;
+}
+
+// Which tile a product of more than 64 rows takes (its place, the whole ones from TILE_COUNT on).
+extern "C" int llmserve_gemm_f32_tile(int M, int N, int K, int splits) {
+  return M <= 64 || N <= 0 || K <= 0 || splits < 1 ? -1 : pick_tile(M, N, K, splits);
 }
 
 // Into how many parts of K (at most 8, each at least 256 long) the tiled product of these sizes is best cut where its
@@ -406,7 +606,8 @@ extern "C" int llmserve_gemm_f32_parts(int M, int N, int K) {
   float best_us = 0.f;
   for (int splits = 1; splits <= 8; ++splits) {
     if (splits > 1 && K / splits < 256) break;
-    const float us = tiled_us(TILE_COSTS[pick_tile(M, N, K, splits)], M, N, K, splits);
+    float us;
+    pick_tile(M, N, K, splits, &us);
     if (splits == 1 || us < best_us) best = splits, best_us = us;
   }
   return best;
@@ -415,7 +616,13 @@ extern "C" int llmserve_gemm_f32_parts(int M, int N, int K) {
 template <bool GATED>
 static int launch_tiled(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, int splits,
                         hipStream_t stream) {
-  switch (pick_tile(M, N, K, splits)) {
+  const int choice = pick_tile(M, N, K, splits);
+  int place = TILE_COUNT;
+#define LAUNCH_WHOLE(NT, MT) \
+  if (choice == place++) return launch_whole<NT, MT, GATED>(x, w, bias, out, M, N, K, splits, stream);
+  WHOLE_TILES(LAUNCH_WHOLE)
+#undef LAUNCH_WHOLE
+  switch (choice) {
     case 0: return launch_tiles<2, 2, 1, 2, 2, 4, GATED>(x, w, bias, out, M, N, K, splits, stream);
     case 1: return launch_tiles<4, 1, 1, 1, 2, 4, GATED>(x, w, bias, out, M, N, K, splits, stream);
     case 2: return launch_tiles<2, 2, 1, 1, 1, 4, GATED>(x, w, bias, out, M, N, K, splits, stream);

@@ -67,6 +67,7 @@ _SIGNATURES = {
     "llmserve_gemm_generic": "pipipipiiiip",
     "llmserve_gemm_f32": "ppppiiiiip",
     "llmserve_gemm_f32_parts": "iii",
+    "llmserve_gemm_f32_tile": "iiii",
     "llmserve_gemm_skinny": "pppipiiiiiip",
     "llmserve_gemm_skinny_tail": "pppipipiiiip",
     "llmserve_gemm_stream": "pppipiiiiiip",

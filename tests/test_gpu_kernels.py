@@ -511,6 +511,33 @@ def test_a_float32_row_has_the_same_bits_in_every_batch_of_few_rows(kernels, inn
     torch.testing.assert_close(k.linear(x, handle).double(), expected, atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5)
 
 
+@pytest.mark.parametrize("tile,rows,inner,outer,gated,splits", [
+    (0, 70, 512, 42, False, 1), (0, 70, 512, 42, True, 1), (0, 70, 1536, 42, False, 2), (1, 65, 320, 2723, False, 1),
+    (1, 65, 320, 2724, True, 1), (1, 65, 512, 6818, False, 2), (2, 97, 512, 1299, False, 1), (2, 97, 512, 1300, True, 1),
+    (2, 97, 1536, 690, False, 2), (3, 129, 256, 10887, False, 1), (3, 129, 256, 10888, True, 1), (3, 129, 256, 11469, False, 4),
+    (4, 129, 256, 11458, True, 1), (4, 65, 320, 5446, False, 1), (4, 129, 256, 13080, False, 4), (5, 65, 256, 10925, False, 1),
+    (5, 65, 256, 10926, True, 1), (5, 65, 512, 5452, False, 2), (6, 65, 256, 19128, True, 1), (6, 65, 320, 18435, False, 1),
+    (6, 65, 512, 9270, False, 2),
+])
+def test_float32_whole_tiles(kernels, tile, rows, inner, outer, gated, splits):
+    """The 32-bit product in whole tiles with each of its tiles, where it is picked, from one stage of K on (fewer stages than it has, as many, more), at rows and weight
+    rows that leave remainders: plain, gated and in parts (the bound as above; a gated result's error is that of its two sums)."""
+    k = kernels[torch.float32]
+    assert k._gemm_f32.llmserve_gemm_f32_tile(rows, outer, inner, splits) == 5 + tile
+    generator = torch.Generator(device="cuda").manual_seed(rows + outer)
+    x, w = torch.randn(rows, inner, generator=generator, device="cuda"), torch.randn(outer, inner, generator=generator, device="cuda") / math.sqrt(inner)
+    bias = torch.randn(outer, generator=generator, device="cuda")
+    out = torch.full((splits, rows, outer // 2 if gated else outer), float("nan"), device="cuda")
+    status = k._gemm_f32.llmserve_gemm_f32(x.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), int(gated), rows, outer, inner, splits,
+                                           torch.cuda.current_stream().cuda_stream)
+    assert status == 0
+    expected = x.double() @ w.double().T + bias.double()
+    if gated:
+        expected = F.silu(expected[:, 0::2]) * expected[:, 1::2]
+    bound = dict(atol=8 * math.sqrt(inner) * 2.0 ** -24 * (4 if gated else 1), rtol=1e-5)
+    torch.testing.assert_close(out.double().sum(0), expected, **bound)
+
+
 @pytest.mark.parametrize("rows,inner,outer", [(33, 1540, 96), (64, 260, 2050), (65, 1540, 98), (67, 260, 2050), (97, 516, 7003), (129, 1028, 9001), (230, 260, 37890),
                                               (509, 300, 16001), (1000, 300, 8197)])
 def test_float32_tiles(kernels, rows, inner, outer):
