@@ -458,7 +458,7 @@ class HipKernels:
     def _rotated_ahead(rows: int, out_features: int, in_features: int) -> bool:
         """Where `linear_rotated` is ahead of the product (the library's up to 512 rows) and the kernel that rotates and stores: while one
         round of 64 x 64 tiles holds the result, for K up to 2,048 one of 128 x 64, and where the product alone is the tiled kernel's too.
-        Us, both in a captured chain over different weights, before -> now: N 2,048 K 1,536: 96 rows 15.5 -> 11.6, 256 16.1 -> 11.7, 512 17.4
+        Us, both in a captured chain over different weights, before -> when it was made (the kernel alone has lost 1 to 2.5 us since): N 2,048 K 1,536: 96 rows 15.5 -> 11.6, 256 16.1 -> 11.7, 512 17.4
         -> 12.9, 1,024 23.9 -> 18.5, 2,048 27.3 -> 26.0; N 1,152 K 896: 96 rows 14.6 -> 8.9, 1,024 17.3 -> 13.1; N 2,560 K 2,048: 96 rows 17.5 -> 13.4,
         448 21.1 -> 21.5, 768 23.5 -> 21.5; N 4,608 K 3,584: 96 rows 26.0 -> 19.9, 192 36.2 -> 22.3, 320 30.3 -> 32.9, 1,024 52.2 -> 58.7; N 7,168 K
         5,120: 96 rows 35.6 -> 30.2, 320 54.2 -> 55.4, 2,048 142 -> 168."""
@@ -578,7 +578,9 @@ class HipKernels:
         the ring, else the library; a gated product there has the kernel for silu(gate) * up behind it).  Both sides measured in turn on the
         same buffers, a captured chain over different weights with what adds up the parts, at 62 weights (K of 768 to 27,648) and
         up to 29 numbers of rows each; below, the kernel's time over the other's.  The library's times jump by a third between
-        neighbouring sizes, so single points lie on the wrong side of every line: the lines follow the means.
+        neighbouring sizes, so single points lie on the wrong side of every line: the lines follow the means.  (The kernel has become
+        5 to 25 percent faster since, by spreading its loads and by more shapes; the lines have stayed, as what they leave to the library was not timed again
+        but for N 1,536 K 8,960 at 2,048 rows: the library 56 us, here 59 in two parts and what adds them up.)
 
         Gated, up to weights of 40 million: ahead while one round of 256 x 128 tiles holds the result (K 896 0.59-0.76, N 17,920 K 1,536
         0.79-0.90, K 2,048 0.70-0.97), behind where it takes a second one that is half empty (N 17,920 at 416-576 rows 1.00-1.14, N 16,384 K
