@@ -559,7 +559,27 @@ extern "C" int llmserve_gemm_blocks_shape(int M, int N, int K, int splits, int k
 }
 
 // Into how many parts of K (at most 12, of whole stages) the product is best cut where its float32 result may stay partial
-// sums: their way to the kernel that adds them up, at 4.5 TB/s, counts too.
+// sums: their way to the kernel that adds them up, at 4.5 TB/s, counts too.  The number of parts decides in which order a result's sums meet, so
+// it goes by an estimate of its own, over six tiles (weight rows, rows of x, how many a CU holds, what a launch, a tile and its 64 k take), which a shape added
+// above, or timed anew, does not move: the same product gives the same bits.  Parts counted by the shapes' own estimate differ at half of the sizes and were no gain
+// (us, those parts -> these: N 1,536 K 8,960 at 192 rows 22.8 -> 17.3, 960 rows 38.9 -> 38.7, 256 rows 18.5 -> 19.1; K 6,144 at 80 rows 9.8 -> 7.6).
+static const struct { int n, m, a_cu; float launch, tile, alone, busy; } PART_TILES[] = {
+    {256, 256, 1, 0.95f, 7.25f, 1.195f, 2.156f}, {256, 320, 1, 1.99f, 8.13f, 1.347f, 2.404f}, {256, 128, 1, 1.75f, 4.71f, 0.699f, 1.156f},
+    {128, 128, 1, 1.51f, 3.95f, 0.443f, 0.645f}, {128, 64, 2, 3.98f, 0.74f, 0.336f, 0.866f},  {64, 64, 2, 3.68f, 1.08f, 0.235f, 0.492f}};
+
+static float parts_us(int M, int N, int K, int splits) {
+  float best = 0.f;
+  for (const auto& t : PART_TILES) {
+    const long groups = (long)((N + t.n - 1) / t.n) * ((M + t.m - 1) / t.m) * splits;
+    const long places = 256L * t.a_cu, full = groups / places, rest = groups % places;
+    const float steps = (float)(K / splits) / 64.f;
+    float us = t.launch + (float)full * (t.tile + steps * t.busy);
+    if (rest) us += t.tile + steps * fmaxf(t.alone, t.busy * (float)rest / (float)places);
+    if (&t == PART_TILES || us < best) best = us;
+  }
+  return best + (float)splits * M * N * 4e-6f / 4.5f;
+}
+
 extern "C" int llmserve_gemm_blocks_parts(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 1;
   const int stage = K % 64 ? 32 : 64;
@@ -567,7 +587,7 @@ extern "C" int llmserve_gemm_blocks_parts(int M, int N, int K) {
   float best_us = 0.f;
   for (int splits = 1; splits <= 12; ++splits) {
     if (K % (splits * stage)) continue;
-    const float us = shape_us(SHAPES[pick_shape(M, N, K, splits, 4)], M, N, K, splits, 4) + (float)splits * M * N * 4e-6f / 4.5f;
+    const float us = parts_us(M, N, K, splits);
     if (splits == 1 || us < best_us) best = splits, best_us = us;
   }
   return best;

@@ -1,0 +1,23 @@
+"""What the host decides for products of many rows, asked of the built libraries (no GPU needed)."""
+
+from __future__ import annotations
+
+import pytest
+
+from llmserve_amd.kernels.build import load_module
+
+# (weight rows, K): parts of K by rows of x.  Sums of parts meet in another order, so a product whose number of parts changes gives other bits.
+PARTS = {
+    (1536, 8960): {65: 10, 96: 10, 128: 10, 160: 7, 192: 7, 224: 7, 256: 7, 320: 5, 384: 5, 448: 4, 512: 4, 640: 4, 960: 2, 1031: 4, 1536: 4, 2048: 2},
+    (1536, 1536): {65: 6, 96: 6, 128: 4, 160: 4, 192: 3, 224: 3, 256: 3, 320: 2, 384: 2, 448: 2, 512: 2, 640: 1, 960: 2, 1031: 1, 1536: 1, 2048: 1},
+    (3584, 18944): {65: 8, 96: 8, 128: 8, 160: 8, 192: 8, 224: 8, 256: 8, 320: 4, 384: 4, 448: 4, 512: 4, 640: 8, 960: 4, 1031: 4, 1536: 2, 2048: 2},
+    (3584, 3584): {65: 4, 96: 4, 128: 4, 160: 4, 192: 2, 224: 4, 256: 4, 320: 2, 384: 2, 448: 2, 512: 2, 640: 2, 960: 1, 1031: 1, 1536: 1, 2048: 1},
+    (1536, 6144): {65: 8, 96: 8, 128: 8, 160: 6, 192: 6, 224: 8, 256: 8, 320: 4, 384: 6, 448: 4, 512: 4, 640: 3, 960: 2, 1031: 3, 1536: 3, 2048: 2},
+    (1536, 480): {97: 3, 300: 3, 1000: 1}, (4096, 1568): {97: 7, 300: 1},
+}
+
+
+@pytest.mark.parametrize("weight", PARTS)
+def test_parts_of_a_product_stay_what_they_are(weight):
+    parts = load_module("gemm_blocks").llmserve_gemm_blocks_parts
+    assert {rows: parts(rows, *weight) for rows in PARTS[weight]} == PARTS[weight]
