@@ -581,33 +581,34 @@ static float whole_us(const WholeTile& t, int M, int N, int K, int splits) {
 // How far the other kernel's tiles are from their own estimates beside these (the choice by both is 1 percent slower than the best of all tiles on average and 19
 // percent faster than that kernel alone; of 90 products one was 1 percent slower than that.  200 rows of N 17,920 K 1,536 126 -> 132 us, 300 rows of N 1,536 K 1,536 20.6 -> 18.9)
 static const float BESIDE_WHOLE[TILE_COUNT] = {0.95f, 0.95f, 1.f, 1.2f, 1.2f};
-// The tile that a product takes (first those of the kernel above, then the whole ones) and what it is estimated to take.
-static int pick_tile(int M, int N, int K, int splits, float* us = nullptr) {
+// The tile that a product takes (first those of the kernel above, then the whole ones) and what it is estimated to take.  `in_pieces`: both operands
+// begin at a multiple of 16 bytes.  Whole tiles need that: their operands go into LDS by 16 bytes a lane without passing registers.
+static int pick_tile(int M, int N, int K, int splits, bool in_pieces, float* us = nullptr) {
   int best = 0, whole = 0;
   for (int t = 1; t < TILE_COUNT; ++t)
     if (tiled_us(TILE_COSTS[t], M, N, K, splits) < tiled_us(TILE_COSTS[best], M, N, K, splits)) best = t;
   for (int t = 1; t < WHOLE_COUNT; ++t)
     if (whole_us(WHOLES[t], M, N, K, splits) < whole_us(WHOLES[whole], M, N, K, splits)) whole = t;
   const float apart = tiled_us(TILE_COSTS[best], M, N, K, splits), here = whole_us(WHOLES[whole], M, N, K, splits);
-  const bool ahead = here < BESIDE_WHOLE[best] * apart;
+  const bool ahead = in_pieces && here < BESIDE_WHOLE[best] * apart;
   if (us) *us = ahead ? here : apart;
   return ahead ? TILE_COUNT + whole : best;
 }
 
-// Which tile a product of more than 64 rows takes (its place, the whole ones from TILE_COUNT on).
+// Which tile a product of more than 64 rows takes whose operands begin at a multiple of 16 bytes (its place, the whole ones from TILE_COUNT on).
 extern "C" int llmserve_gemm_f32_tile(int M, int N, int K, int splits) {
-  return M <= 64 || N <= 0 || K <= 0 || splits < 1 ? -1 : pick_tile(M, N, K, splits);
+  return M <= 64 || N <= 0 || K <= 0 || splits < 1 ? -1 : pick_tile(M, N, K, splits, true);
 }
 
 // Into how many parts of K (at most 8, each at least 256 long) the tiled product of these sizes is best cut where its
-// result may stay in parts.
-extern "C" int llmserve_gemm_f32_parts(int M, int N, int K) {
+// result may stay in parts.  `in_pieces`: whether both operands begin at a multiple of 16 bytes.
+extern "C" int llmserve_gemm_f32_parts(int M, int N, int K, int in_pieces) {
   int best = 1;
   float best_us = 0.f;
   for (int splits = 1; splits <= 8; ++splits) {
     if (splits > 1 && K / splits < 256) break;
     float us;
-    pick_tile(M, N, K, splits, &us);
+    pick_tile(M, N, K, splits, in_pieces, &us);
     if (splits == 1 || us < best_us) best = splits, best_us = us;
   }
   return best;
@@ -616,7 +617,7 @@ extern "C" int llmserve_gemm_f32_parts(int M, int N, int K) {
 template <bool GATED>
 static int launch_tiled(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, int splits,
                         hipStream_t stream) {
-  const int choice = pick_tile(M, N, K, splits);
+  const int choice = pick_tile(M, N, K, splits, ((size_t)x | (size_t)w) % 16 == 0);
   int place = TILE_COUNT;
 #define LAUNCH_WHOLE(NT, MT) \
   if (choice == place++) return launch_whole<NT, MT, GATED>(x, w, bias, out, M, N, K, splits, stream);

@@ -66,7 +66,7 @@ _SIGNATURES = {
     "llmserve_gather_rows": "ppiippiip",
     "llmserve_gemm_generic": "pipipipiiiip",
     "llmserve_gemm_f32": "ppppiiiiip",
-    "llmserve_gemm_f32_parts": "iii",
+    "llmserve_gemm_f32_parts": "iiii",
     "llmserve_gemm_f32_tile": "iiii",
     "llmserve_gemm_skinny": "pppipiiiiiip",
     "llmserve_gemm_skinny_tail": "pppipipiiiip",
@@ -800,7 +800,9 @@ class HipKernels:
             _check(status, "linear")
             return out
         if self._all_float32(x, weights) and (out_dtype or self.dtype) == torch.float32:
-            splits = self._float32_splits(rows, weights.out_features, inner) if partial and out_dtype == torch.float32 else 1
+            splits = 1
+            if partial and out_dtype == torch.float32:
+                splits = self._float32_splits(rows, weights.out_features, inner, _in_pieces(x, weights.weight))
             shape = (rows, weights.out_features) if splits == 1 else (splits, rows, weights.out_features)
             out = self._empty(shape, torch.float32)
             status = self._gemm_f32.llmserve_gemm_f32(
@@ -828,12 +830,13 @@ class HipKernels:
             and weights.in_features % 4 == 0
         )
 
-    def _float32_splits(self, rows: int, out_features: int, in_features: int) -> int:
+    def _float32_splits(self, rows: int, out_features: int, in_features: int, in_pieces: bool = True) -> int:
         """Into how many parts of K a float32 product is cut when its result may stay in parts: up to 64
         rows (the weight-streaming kernel, workgroups of 16 weight rows) until about a thousand workgroups
-        run, a part at least 512 long; more rows (the tiled kernel) as its own estimate has it."""
+        run, a part at least 512 long; more rows (tiles of rows of x) as their own estimate has it, which also asks whether
+        both operands begin at a multiple of 16 bytes."""
         if rows > 64:
-            return self._gemm_f32.llmserve_gemm_f32_parts(rows, out_features, in_features)
+            return self._gemm_f32.llmserve_gemm_f32_parts(rows, out_features, in_features, in_pieces)
         tiles, best = -(-out_features // 16), 1
         for splits in range(2, 9):
             if in_features // splits >= 512 and tiles * splits <= 1024:

@@ -538,6 +538,28 @@ def test_float32_whole_tiles(kernels, tile, rows, inner, outer, gated, splits):
     torch.testing.assert_close(out.double().sum(0), expected, **bound)
 
 
+@pytest.mark.parametrize("x_from,w_from", [(1, 0), (0, 2), (3, 1)])
+@pytest.mark.parametrize("rows,inner,outer", [(70, 512, 48), (129, 256, 10888), (200, 1536, 1536)])
+def test_float32_operands_that_begin_inside_a_piece(kernels, rows, inner, outer, x_from, w_from):
+    """Contiguous views that begin 4, 8 or 12 bytes into a piece of 16, at sizes of whole tiles, which need whole pieces: plain, gated and in the parts that the library
+    takes (the bound as above)."""
+    k = kernels[torch.float32]
+    generator = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows * inner + 4, generator=generator, device="cuda")[x_from : x_from + rows * inner].view(rows, inner)
+    w = torch.randn(outer * inner + 4, generator=generator, device="cuda").div_(math.sqrt(inner))[w_from : w_from + outer * inner].view(outer, inner)
+    assert (x.data_ptr() | w.data_ptr()) % 16 and k._gemm_f32.llmserve_gemm_f32_tile(rows, outer, inner, 1) >= 5
+    handle = k.prepare_linear([w], None)
+    assert handle.weight.data_ptr() == w.data_ptr()
+    expected = x.double() @ w.double().T
+    bound = dict(atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5)
+    torch.testing.assert_close(k.linear(x, handle).double(), expected, **bound)
+    parts = k.linear(x, handle, out_dtype=torch.float32, partial=True)
+    torch.testing.assert_close((parts if parts.ndim == 2 else parts.double().sum(0)), expected, check_dtype=False, **bound)
+    out = torch.full((rows, outer // 2), float("nan"), device="cuda")
+    assert k._gemm_f32.llmserve_gemm_f32(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), 1, rows, outer, inner, 1, torch.cuda.current_stream().cuda_stream) == 0
+    torch.testing.assert_close(out.double(), F.silu(expected[:, 0::2]) * expected[:, 1::2], atol=4 * bound["atol"], rtol=1e-5)
+
+
 @pytest.mark.parametrize("rows,inner,outer", [(33, 1540, 96), (64, 260, 2050), (65, 1540, 98), (67, 260, 2050), (97, 516, 7003), (129, 1028, 9001), (230, 260, 37890),
                                               (509, 300, 16001), (1000, 300, 8197)])
 def test_float32_tiles(kernels, rows, inner, outer):

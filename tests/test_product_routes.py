@@ -21,3 +21,17 @@ PARTS = {
 def test_parts_of_a_product_stay_what_they_are(weight):
     parts = load_module("gemm_blocks").llmserve_gemm_blocks_parts
     assert {rows: parts(rows, *weight) for rows in PARTS[weight]} == PARTS[weight]
+
+
+# the same in float32 where an operand begins inside a piece of 16 bytes: the kernel that brings its operands through registers, in the parts that are best for it
+FLOAT32_PARTS_ANYWHERE = {
+    (1536, 8960): {65: 7, 96: 7, 128: 8, 160: 8, 192: 7, 224: 6, 256: 8, 384: 7, 512: 8, 777: 8, 2048: 4},
+    (1536, 1536): {65: 5, 96: 5, 128: 5, 160: 6, 192: 5, 224: 6, 256: 5, 384: 5, 512: 4, 777: 4, 2048: 1},
+    (3584, 3584): {65: 6, 96: 6, 128: 8, 160: 8, 192: 6, 224: 5, 256: 8, 384: 3, 512: 4, 777: 4, 2048: 2},
+}
+
+
+@pytest.mark.parametrize("weight", FLOAT32_PARTS_ANYWHERE)
+def test_parts_of_a_float32_product_whose_operands_begin_anywhere(weight):
+    parts = load_module("gemm_f32").llmserve_gemm_f32_parts
+    assert {rows: parts(rows, *weight, 0) for rows in FLOAT32_PARTS_ANYWHERE[weight]} == FLOAT32_PARTS_ANYWHERE[weight]
