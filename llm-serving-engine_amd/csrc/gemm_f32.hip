@@ -600,16 +600,31 @@ extern "C" int llmserve_gemm_f32_tile(int M, int N, int K, int splits) {
   return M <= 64 || N <= 0 || K <= 0 || splits < 1 ? -1 : pick_tile(M, N, K, splits, true);
 }
 
-// Into how many parts of K (at most 8, each at least 256 long) the tiled product of these sizes is best cut where its
+// Into how many parts of K (at most 8, each at least 256 long) the product of these sizes is best cut where its
 // result may stay in parts.  `in_pieces`: whether both operands begin at a multiple of 16 bytes.
+// An error against 64 bits goes with the root of how many k one sum runs over (3.7e-8 of the result for 4 of them, in both kernels): a part of K over the
+// waves that share a tile, four of them here and TILE_WAVES there.  So whole tiles are taken in no fewer parts than keep their sums as short as the
+// other kernel's in its best number.  Relative errors, that kernel -> whole tiles in the parts that their time alone would have -> in
+// these: 160 rows of N 1,536 K 1,536 2.1e-7 -> 3.5e-7 -> 1.8e-7, 224 rows of N 1,536 K 8,960 4.9e-7 -> 8.5e-7 -> 4.3e-7, 65 rows of N 3,584 K 3,584
+// 3.2e-7 -> 5.4e-7 -> 2.0e-7.
+static const int TILE_WAVES[TILE_COUNT] = {1, 1, 1, 2, 4};
 extern "C" int llmserve_gemm_f32_parts(int M, int N, int K, int in_pieces) {
-  int best = 1;
+  int best = 1, tile = 0;
   float best_us = 0.f;
   for (int splits = 1; splits <= 8; ++splits) {
     if (splits > 1 && K / splits < 256) break;
     float us;
-    pick_tile(M, N, K, splits, in_pieces, &us);
-    if (splits == 1 || us < best_us) best = splits, best_us = us;
+    const int picked = pick_tile(M, N, K, splits, false, &us);
+    if (splits == 1 || us < best_us) best = splits, best_us = us, tile = picked;
+  }
+  if (!in_pieces) return best;
+  const int shortest = best * TILE_WAVES[tile];
+  best_us *= BESIDE_WHOLE[tile];
+  for (int splits = 1; splits <= 8; ++splits) {
+    if (splits > 1 && K / splits < 256) break;
+    float us;
+    if (4 * splits < shortest || pick_tile(M, N, K, splits, true, &us) < TILE_COUNT) continue;
+    if (us < best_us) best = splits, best_us = us;
   }
   return best;
 }

@@ -560,6 +560,29 @@ def test_float32_operands_that_begin_inside_a_piece(kernels, rows, inner, outer,
     torch.testing.assert_close(out.double(), F.silu(expected[:, 0::2]) * expected[:, 1::2], atol=4 * bound["atol"], rtol=1e-5)
 
 
+@pytest.mark.parametrize("inner,outer", [(1536, 1536), (8960, 1536), (3584, 3584), (4864, 896)])
+@pytest.mark.parametrize("rows", [65, 96, 160, 192, 224, 384, 512])
+def test_float32_parts_keep_their_sums_as_short(kernels, rows, inner, outer):
+    """A product left in parts is no further from 64 bits than from the kernel that views which begin inside a piece go to, in that one's own parts: an error
+    goes with the root of how many k one sum runs over, which parts of K have to keep as short.  (Over a result of 58,000 values and more the norm of the
+    error of one and the same order of sums varies by less than 1 percent from draw to draw.)"""
+    k = kernels[torch.float32]
+    generator = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, inner, generator=generator, device="cuda")
+    w = torch.randn(outer, inner, generator=generator, device="cuda") / math.sqrt(inner)
+    apart = torch.empty(rows * inner + 1, device="cuda")[1:].view(rows, inner).copy_(x)
+    handle, expected = k.prepare_linear([w], None), x.double() @ w.double().T
+
+    def error(rows_of_x):
+        parts = k.linear(rows_of_x, handle, out_dtype=torch.float32, partial=True)
+        total = parts if parts.ndim == 2 else parts[0].clone()
+        for part in parts[1:] if parts.ndim == 3 else ():
+            total += part
+        return ((total.double() - expected).norm() / expected.norm()).item()
+
+    assert error(x) <= 1.03 * error(apart)
+
+
 @pytest.mark.parametrize("rows,inner,outer", [(33, 1540, 96), (64, 260, 2050), (65, 1540, 98), (67, 260, 2050), (97, 516, 7003), (129, 1028, 9001), (230, 260, 37890),
                                               (509, 300, 16001), (1000, 300, 8197)])
 def test_float32_tiles(kernels, rows, inner, outer):
