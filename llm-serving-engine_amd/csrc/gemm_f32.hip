@@ -556,43 +556,59 @@ static float tiled_us(const TileCost& t, int M, int N, int K, int splits) {
          (splits > 1 ? (float)splits * M * N * 8e-6f / 4.5f : 0.f);
 }
 
-// The tiles of the kernel of whole tiles, in sixteens, and what a launch, a tile and a tile's 64 k (where few CUs are busy, and where all are) take, us; a
-// million bytes of the result 0.3.  Fitted to 90 products of 65 to 512 rows of five weights, in one to seven parts, every weight out of memory, each tile within
-// 2 to 7 percent of what was measured.  Of nineteen tiles measured these seven miss the best one by 0.2 percent on average.
+// The tiles of the kernel of whole tiles, in sixteens.
 #define WHOLE_TILES(X) X(1, 3) X(1, 5) X(2, 2) X(2, 3) X(3, 3) X(3, 5) X(5, 5)
-struct WholeTile {
-  int n, m;
-  float launch, tile, alone, busy;
-};
-static const WholeTile WHOLES[] = {{1, 3, 4.04f, 0.10f, 0.247f, 0.287f}, {1, 5, 3.87f, 0.11f, 0.419f, 0.251f}, {2, 2, 3.45f, 0.25f, 0.328f, 0.018f},
-                                   {2, 3, 3.77f, 0.00f, 0.475f, 0.289f}, {3, 3, 3.53f, 0.00f, 0.720f, 0.515f}, {3, 5, 1.60f, 2.07f, 1.186f, 1.091f},
-                                   {5, 5, 1.92f, 3.12f, 1.861f, 1.561f}};
-constexpr int WHOLE_COUNT = sizeof(WHOLES) / sizeof(WHOLES[0]), TILE_COUNT = 5;
+constexpr int TILE_COUNT = 5, WHOLE_COUNT = 7, ALL_TILES = TILE_COUNT + WHOLE_COUNT;
 
-static float whole_us(const WholeTile& t, int M, int N, int K, int splits) {
-  if (K % (64 * splits) || M > 512) return 1e30f;  // (this kernel takes whole stages; more rows have not been measured but for a few, of which half were behind)
-  const long groups = (long)((N + 16 * t.n - 1) / (16 * t.n)) * ((M + 16 * t.m - 1) / (16 * t.m)) * splits, full = groups / 256, rest = groups % 256;
-  const float steps = (float)(K / splits / 64), result = 4e-6f * (float)splits * M * N;  // (a gated one is half as large)
-  float us = t.launch + 0.3f * result + (float)full * (t.tile + steps * fmaxf(t.alone, t.busy));
-  if (rest) us += t.tile + steps * fmaxf(t.alone, t.busy * (float)rest / 256.f);
-  return us + (splits > 1 ? result / 4.5f : 0.f);
+// Which kernel takes a product of up to 512 rows goes by what their tiles take, us: a launch, a tile, and a tile's 64 k where it has its CU to itself, where two share
+// one, and where all CUs are as full as they get; a million bytes of the result.  (Once a CU has been full, what is left comes two to a CU, too.)  Fitted to
+// 5,700 products of 65 to 512 rows of twelve weights, in one to eight parts, every weight out of memory, each tile within 2 to 7 percent of what was measured on average.  Of 182
+// products the choice by them is 2 percent slower than the best of all tiles on average and 10 percent faster than the other kernel alone; of these and of 102 drawn
+// ones none is more than 1 percent slower than that kernel, which AHEAD_FROM is for (with 0.98 three of the drawn ones were 3 to 4 percent slower).  Us, that kernel ->
+// whole tiles wherever an estimate of theirs, beside that kernel's own, had them ahead -> now: N 17,920 K 1,536 gated 200 rows 124 -> 131 -> 124, 256 rows
+// 142 -> 151 -> 142; N 1,536 K 8,960 in parts 224 rows 68 -> 79 -> 68; N 4,608 K 3,584 384 rows 144 -> 152 -> 136.
+struct TileTimes {
+  int n, m, a_cu;
+  float launch, tile, alone, shared, busy, a_million;
+};
+static const TileTimes TIMES[ALL_TILES] = {
+    {128, 128, 1, 5.983f, 0.011f, 4.619f, 0.f, 3.662f, 0.259f}, {128, 64, 1, 5.231f, 0.116f, 2.649f, 0.f, 1.888f, 0.225f},
+    {64, 64, 1, 3.933f, 0.079f, 1.505f, 0.f, 0.988f, 0.253f},   {64, 32, 1, 3.292f, 0.244f, 0.970f, 0.f, 0.512f, 0.345f},
+    {32, 32, 1, 3.966f, 0.335f, 0.506f, 0.f, 0.314f, 0.511f},   {16, 48, 2, 3.100f, 0.000f, 0.328f, 0.531f, 0.505f, 0.724f},
+    {16, 80, 2, 3.422f, 0.000f, 0.455f, 0.765f, 0.774f, 0.550f}, {32, 32, 2, 2.859f, 0.052f, 0.355f, 0.635f, 0.597f, 0.667f},
+    {32, 48, 2, 3.355f, 0.028f, 0.516f, 0.930f, 0.856f, 0.376f}, {48, 48, 2, 2.818f, 0.021f, 0.773f, 1.348f, 1.209f, 0.472f},
+    {48, 80, 1, 2.043f, 1.903f, 1.173f, 0.f, 1.189f, 0.220f},   {80, 80, 1, 2.256f, 2.534f, 1.848f, 0.f, 1.872f, 0.313f}};
+constexpr float AHEAD_FROM = 0.94f;
+
+// Without what reads parts of K again.
+static float measured_us(const TileTimes& t, int M, int N, int K, int splits) {
+  const long groups = (long)((N + t.n - 1) / t.n) * ((M + t.m - 1) / t.m) * splits;
+  const long places = 256L * t.a_cu, full = groups / places, rest = groups % places;
+  const float steps = (float)K / (float)splits / 64.f;
+  float us = t.launch + t.a_million * 4e-6f * (float)splits * M * N + (float)full * (t.tile + steps * t.busy);  // (a gated result is half as large)
+  if (rest) us += t.tile + steps * fmaxf(t.a_cu == 2 && (full || rest > 256) ? t.shared : t.alone, t.busy * (float)rest / (float)places);
+  return us;
 }
 
-// How far the other kernel's tiles are from their own estimates beside these (the choice by both is 1 percent slower than the best of all tiles on average and 19
-// percent faster than that kernel alone; of 90 products one was 1 percent slower than that.  200 rows of N 17,920 K 1,536 126 -> 132 us, 300 rows of N 1,536 K 1,536 20.6 -> 18.9)
-static const float BESIDE_WHOLE[TILE_COUNT] = {0.95f, 0.95f, 1.f, 1.2f, 1.2f};
-// The tile that a product takes (first those of the kernel above, then the whole ones) and what it is estimated to take.  `in_pieces`: both operands
-// begin at a multiple of 16 bytes.  Whole tiles need that: their operands go into LDS by 16 bytes a lane without passing registers.
+// The tile that a product takes (first those of the kernel above, then the whole ones), and what it is estimated to take: that kernel's by its own estimate, the whole
+// ones by theirs.  `in_pieces`: both operands begin at a multiple of 16 bytes.  Whole tiles need that: their operands go into LDS by 16 bytes a lane without
+// passing registers.  They take whole stages of 64 k; more rows than 512 have not been measured but for a few, of which half were behind.
 static int pick_tile(int M, int N, int K, int splits, bool in_pieces, float* us = nullptr) {
-  int best = 0, whole = 0;
+  int best = 0;
   for (int t = 1; t < TILE_COUNT; ++t)
     if (tiled_us(TILE_COSTS[t], M, N, K, splits) < tiled_us(TILE_COSTS[best], M, N, K, splits)) best = t;
-  for (int t = 1; t < WHOLE_COUNT; ++t)
-    if (whole_us(WHOLES[t], M, N, K, splits) < whole_us(WHOLES[whole], M, N, K, splits)) whole = t;
-  const float apart = tiled_us(TILE_COSTS[best], M, N, K, splits), here = whole_us(WHOLES[whole], M, N, K, splits);
-  const bool ahead = in_pieces && here < BESIDE_WHOLE[best] * apart;
-  if (us) *us = ahead ? here : apart;
-  return ahead ? TILE_COUNT + whole : best;
+  if (in_pieces && M <= 512 && K % (64 * splits) == 0) {
+    int whole = TILE_COUNT;
+    for (int t = whole + 1; t < ALL_TILES; ++t)
+      if (measured_us(TIMES[t], M, N, K, splits) < measured_us(TIMES[whole], M, N, K, splits)) whole = t;
+    const float here = measured_us(TIMES[whole], M, N, K, splits);
+    if (here < AHEAD_FROM * measured_us(TIMES[best], M, N, K, splits)) {
+      if (us) *us = here;
+      return whole;
+    }
+  }
+  if (us) *us = tiled_us(TILE_COSTS[best], M, N, K, splits);
+  return best;
 }
 
 // Which tile a product of more than 64 rows takes whose operands begin at a multiple of 16 bytes (its place, the whole ones from TILE_COUNT on).
@@ -617,14 +633,15 @@ extern "C" int llmserve_gemm_f32_parts(int M, int N, int K, int in_pieces) {
     const int picked = pick_tile(M, N, K, splits, false, &us);
     if (splits == 1 || us < best_us) best = splits, best_us = us, tile = picked;
   }
-  if (!in_pieces) return best;
+  if (!in_pieces || M > 512) return best;
+  auto read_us = [&](int splits) { return splits > 1 ? (float)splits * M * N * 4e-6f / 4.5f : 0.f; };
   const int shortest = best * TILE_WAVES[tile];
-  best_us *= BESIDE_WHOLE[tile];
+  best_us = AHEAD_FROM * (measured_us(TIMES[tile], M, N, K, best) + read_us(best));
   for (int splits = 1; splits <= 8; ++splits) {
     if (splits > 1 && K / splits < 256) break;
     float us;
     if (4 * splits < shortest || pick_tile(M, N, K, splits, true, &us) < TILE_COUNT) continue;
-    if (us < best_us) best = splits, best_us = us;
+    if (us + read_us(splits) < best_us) best = splits, best_us = us + read_us(splits);
   }
   return best;
 }
