@@ -27,6 +27,7 @@
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 // Which tile a workgroup takes.  The chip hands workgroups to its eight chiplets (XCDs) in turn,
 // workgroup i to chiplet i % 8, and every chiplet has an L2 of its own: tiles dealt out in launch
@@ -189,9 +190,17 @@ __device__ __forceinline__ void store_tiles(const f32x4 (&acc)[TN][TM], float* m
         const float gate = sums[2 * e], up = sums[2 * e + 1];
         gated[e] = (bf16_t)(gate * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gate * -1.44269504088896f)) * up);
       }
-      if (INSIDE ? N % 16 == 0 : n + RUN <= N && N % 16 == 0) {
-        if constexpr (RUN == 16) store_piece(*(const u32x4*)gated, dst);
-        else if constexpr (RUN == 8) *(uint2*)dst = *(const uint2*)gated;
+      if (INSIDE || (n + RUN <= N && N % 8 == 0)) {
+        if constexpr (RUN == 16) {
+          // (of a width of 4 mod 8, N of 8 mod 16, every other row begins in the middle of 16 bytes: two halves.  Us by two bytes -> so: 2,048 rows of N 17,912
+          // K 1,536 127 -> 103, of N 9,720 K 896 62 -> 46)
+          if (N % 16 == 0) {
+            store_piece(*(const u32x4*)gated, dst);
+          } else {
+            store_piece(*(const u32x2*)gated, dst);
+            store_piece(*(const u32x2*)(gated + 4), dst + 4);
+          }
+        } else if constexpr (RUN == 8) *(uint2*)dst = *(const uint2*)gated;
         else *(unsigned*)dst = *(const unsigned*)gated;
       } else {
 #pragma unroll

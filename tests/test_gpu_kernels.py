@@ -180,6 +180,22 @@ def test_every_shape_of_a_tile(kernels, shape, rows, plain, float32, gated, inne
         torch.testing.assert_close(out.double(), expected, **bound)
 
 
+@pytest.mark.parametrize("rows,inner,width", [(130, 128, 44), (300, 192, 1092), (1000, 256, 4860), (700, 512, 4100), (2048, 128, 8956)])
+def test_gated_widths_of_four_mod_eight(own_kernels, rows, inner, width):
+    """A gated result whose rows begin in the middle of 16 bytes every other time: each value in its place and nothing outside (bound as in `test_tiles_of_many_rows`)."""
+    k, dtype = own_kernels, torch.bfloat16
+    generator = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, inner, generator=generator, device="cuda").to(dtype)
+    w = torch.randn(2 * width, inner, generator=generator, device="cuda").div_(math.sqrt(inner)).to(dtype)
+    around = torch.full((rows * width + 128,), float("nan"), device="cuda", dtype=dtype)
+    out = around[64 : 64 + rows * width].view(rows, width)
+    assert k._gemm_blocks.llmserve_gemm_blocks(x.data_ptr(), w.data_ptr(), None, 0, out.data_ptr(), 0, 1, rows, 2 * width, inner, 1,
+                                               torch.cuda.current_stream().cuda_stream) == 0
+    expected = x.double() @ w.double().T
+    torch.testing.assert_close(out.double(), F.silu(expected[:, 0::2]) * expected[:, 1::2], **TOLERANCE[dtype])
+    assert around[:64].isnan().all() and around[64 + rows * width :].isnan().all()
+
+
 @pytest.mark.parametrize("rows,inner,outer", [(512, 1536, 2048), (513, 1536, 2048), (2048, 1536, 2048), (2049, 1536, 2048), (513, 64, 1024), (777, 320, 1030), (600, 1536, 1536)])
 def test_small_weights_over_many_rows(kernels, rows, inner, outer):
     """Both sides of the line from which small plain products are the tiled kernel's, with and without leave to split: a route that takes
