@@ -384,11 +384,12 @@ __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const 
     const bf16_t* from = src[i] + step * BK - (HALF && step == last && beyond[i] ? BK / 2 : 0);
     __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)from, (void __attribute__((address_space(3)))*)to, 16, 0, 0);
   };
-  // where it reads its operands: rows r16 + 16 t of the wave's, part 4 * step of 32 k + q
+  // where it reads its operands: rows r16 + 16 t of the wave's, part 4 * step of 32 k + q.  Of that only `lane_at` differs by lane (a row is 128 bytes and
+  // the second step's part the first one's with bit 2 turned, so 64 of it are turned): one register, as 256 x 320 has none to spare: with rows and parts
+  // in four it kept two others in memory (READ_TILE says why none may lie there)
   const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
-  const int turned = swizzle(r16);
-  const unsigned row_w = base + (unsigned)(wave_n * TN * 16 + r16) * ROW_BYTES;
-  const unsigned row_x = base + W_BYTES + (unsigned)(wave_m * TM * 16 + r16) * ROW_BYTES;
+  const unsigned lane_at = (unsigned)(r16 * ROW_BYTES + (q ^ swizzle(r16)) * 16);
+  const unsigned row_w = base + (unsigned)(wave_n * TN * 16) * ROW_BYTES, row_x = base + W_BYTES + (unsigned)(wave_m * TM * 16) * ROW_BYTES;
 
   Early<TN, TM> early;
   if constexpr (OUT == OUT_ROTATED)
@@ -410,11 +411,12 @@ __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const 
   __builtin_amdgcn_s_barrier();
   // The reads of LDS are written as instructions, with their waits: left to the compiler, every read of LDS waits for all
   // loads into LDS that are under way, whichever stage they fill.  What a read brings is used only behind a wait that it passes through, so that
-  // nothing that uses it is moved in front of the wait.
+  // nothing that uses it is moved in front of the wait.  To the compiler a register is filled at its read: were it short of them, it could put one away that is
+  // still to be filled.  So no shape may spill (`test_kernels_that_read_ahead_keep_their_registers`).
   bf16x8 a[2][TN], b[Order::SLOTS];
 #define READ_TILE(into, row, tile, at) \
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(into) : "v"((row) + (at)), "n"((tile) * 16 * ROW_BYTES) : "memory")
-  auto slot_of = [&](int chunk) { return (unsigned)(((chunk * 4 + q) ^ turned) * 16); };
+  auto slot_of = [&](int chunk) { return lane_at ^ (unsigned)(chunk * 64); };
 #pragma unroll
   for (int i = 0; i < TN; ++i) READ_TILE(a[0][i], row_w, i, slot_of(0));
 #pragma unroll

@@ -2,9 +2,11 @@
 
 from __future__ import annotations
 
+import re
+
 import pytest
 
-from llmserve_amd.kernels.build import load_module
+from llmserve_amd.kernels.build import build_module, load_module
 
 # (weight rows, K): parts of K by rows of x.  Sums of parts meet in another order, so a product whose number of parts changes gives other bits.
 PARTS = {
@@ -41,3 +43,13 @@ def test_parts_of_a_float32_product_whose_operands_begin_anywhere(weight):
 def test_no_whole_tiles_where_the_other_float32_kernel_is_ahead(rows, outer, inner):
     """Sizes at which whole tiles were measured 3 to 6 percent behind."""
     assert 0 <= load_module("gemm_f32").llmserve_gemm_f32_tile(rows, outer, inner, 1) < 5
+
+
+@pytest.mark.parametrize("module,kernel", [("gemm_blocks", "gemm_block_kernel"), ("gemm_f32", "gemm_f32_whole_kernel"),
+                                           ("gemm_bf16", "gemm_stream_kernel"), ("gemm_bf16", "gemm_ring_kernel")])
+def test_kernels_that_read_ahead_keep_their_registers(module, kernel):
+    """Kernels whose reads of LDS are instructions with waits of their own have no memory of a lane's: a register put away there before its read has come
+    would come back with what it held before.  As the built library's own description of its kernels has it."""
+    described = re.findall(rb"\.private_segment_fixed_size(.).*?\.symbol.*?(_Z\w+)\.kd", build_module(module).read_bytes(), re.S)
+    sizes = {name.decode(): size for size, name in described if kernel.encode() in name}
+    assert sizes and {name: size for name, size in sizes.items() if size != b"\0"} == {}
