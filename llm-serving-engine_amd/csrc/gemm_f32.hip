@@ -374,8 +374,7 @@ template <int N>
 __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
-constexpr int whole_stages(int rows) { return rows <= 64 ? 4 : rows < 208 ? 3 : 2; }
-constexpr int WHOLE_BATCH = 32;  // tiles whose sums meet at a time: a KB of each of four waves
+constexpr int whole_stages(int rows) { return rows <= 64 ? 4 : 3; }
 
 template <int NT, int MT, bool GATED>
 __global__ __launch_bounds__(256, 1) void gemm_f32_whole_kernel(const float* __restrict__ x, const float* __restrict__ w,
@@ -474,35 +473,32 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_whole_kernel(const float* __r
   // D[n][m] of a tile: a lane holds column m = r and rows n = 4 g .. + 3
   const bool with_bias = bias && blockIdx.y == 0;
   f32x4* sums = (f32x4*)lds;
+  __syncthreads();
 #pragma unroll
-  for (int first = 0; first < NT * MT; first += WHOLE_BATCH) {
-    __syncthreads();
+  for (int t = 0; t < NT * MT; ++t) sums[(t * 4 + wave) * 64 + lane] = acc[t / MT][t % MT];
+  __syncthreads();
+  for (int t = wave; t < NT * MT; t += 4) {
+    f32x4 total = sums[t * 4 * 64 + lane];
 #pragma unroll
-    for (int t = first; t < min(first + WHOLE_BATCH, NT * MT); ++t) sums[((t - first) * 4 + wave) * 64 + lane] = acc[t / MT][t % MT];
-    __syncthreads();
-    for (int t = first + wave; t < min(first + WHOLE_BATCH, NT * MT); t += 4) {
-      f32x4 total = sums[((t - first) * 4) * 64 + lane];
+    for (int v = 1; v < 4; ++v) total += sums[(t * 4 + v) * 64 + lane];
+    const int m = m0 + t % MT * 16 + r, n = n0 + t / MT * 16 + 4 * g;
+    if (m >= M || n >= N) continue;
+    if (with_bias) {
 #pragma unroll
-      for (int v = 1; v < 4; ++v) total += sums[((t - first) * 4 + v) * 64 + lane];
-      const int m = m0 + t % MT * 16 + r, n = n0 + t / MT * 16 + 4 * g;
-      if (m >= M || n >= N) continue;
-      if (with_bias) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) total[e] += bias[min(n + e, N - 1)];
-      }
-      if (GATED) {
-        float* dst = out + (size_t)m * (N / 2) + n / 2;
-        if (n + 1 < N) dst[0] = silu(total[0]) * total[1];
-        if (n + 3 < N) dst[1] = silu(total[2]) * total[3];
+      for (int e = 0; e < 4; ++e) total[e] += bias[min(n + e, N - 1)];
+    }
+    if (GATED) {
+      float* dst = out + (size_t)m * (N / 2) + n / 2;
+      if (n + 1 < N) dst[0] = silu(total[0]) * total[1];
+      if (n + 3 < N) dst[1] = silu(total[2]) * total[3];
+    } else {
+      float* dst = out + ((size_t)blockIdx.y * M + m) * N + n;
+      if (n + 3 < N && (N & 3) == 0) {
+        *(f32x4*)dst = total;
       } else {
-        float* dst = out + ((size_t)blockIdx.y * M + m) * N + n;
-        if (n + 3 < N && (N & 3) == 0) {
-          *(f32x4*)dst = total;
-        } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < N) dst[e] = total[e];
-        }
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) dst[e] = total[e];
       }
     }
   }
@@ -510,9 +506,8 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_whole_kernel(const float* __r
 
 template <int NT, int MT, bool GATED>
 static int launch_whole(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, int splits, hipStream_t stream) {
-  constexpr int ROWS = (NT + MT) * 16, staged = whole_stages(ROWS) * ROWS * 256, met = (NT * MT < WHOLE_BATCH ? NT * MT : WHOLE_BATCH) * 4096;
-  constexpr int bytes = staged > met ? staged : met;
-  static_assert(bytes <= 160 * 1024, "a CU's LDS");
+  constexpr int ROWS = (NT + MT) * 16, bytes = whole_stages(ROWS) * ROWS * 256;
+  static_assert(bytes <= 160 * 1024 && NT * MT * 4096 <= bytes, "a CU's LDS, and in it the tiles' sums of four waves");
   static bool asked = false;
   if (!asked) {
     if (hipFuncSetAttribute((const void*)gemm_f32_whole_kernel<NT, MT, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)
