@@ -533,28 +533,34 @@ static int launch_block(const void* x, const void* w, const void* bias, int bias
 }
 
 // The shapes: a tile's weight rows and rows of x, how many a CU holds at a time, and what a launch, a tile, a tile's
-// 64 k (where few CUs are busy, and where all are: their clock is lower and they share L2) and a million bytes of the result take, us.  Fitted to
-// 430 products of 96 to 2,048 rows with seventeen weights (K of 896 to 18,944), whole and in parts, x written by the kernel before and every weight
-// out of memory, each shape within 9 percent of what was measured; the shape picked by them is 2 to 3 percent slower than the best one on average.  Of
-// sixteen shapes measured these ten miss the least: without 160 x 160, 128 x 160, 192 x 128, 96 x 128 and 128 x 96 the best one left is 3 percent
-// slower on average.
+// 64 k (where few CUs are busy, and where all are: their clock is lower and they share L2) and a million bytes of the result take, us; where a CU holds two,
+// also what 64 k take once a first CU holds two (`shared`) and once all do (`shared_all`): a workgroup that shares its CU takes up to twice as long, and the product ends
+// with it.  Fitted to 1,764 products of 65 to 3,000 rows with 36 weights (K of 448 to 18,944), whole and in parts, every weight out of memory; the shape
+// picked is 0.7 percent slower than the best one on average.  Two workgroups to a CU priced as one each as long as they were fewer than 512, and
+// without 128 x 128 and 256 x 128, it was 5 percent, and one product in eleven was more than 3 percent slower than with the shapes that this kernel had before
+// it spread its loads; of 936 others timed since it is one in eighty-five.  Us, those shapes -> ten under that estimate -> these: 400 rows of N 4,608 K 3,584 gated
+// 27.9 -> 37.0 -> 24.1, 640 rows of N 11,008 K 2,048 33.9 -> 47.3 -> 32.4; in parts 160 rows of N 1,536 K 8,960 14.4 -> 15.6 -> 13.8, 513 rows of N 896 K 4,864
+// 11.8 -> 15.1 -> 13.0.
 struct BlockShape {
   int n, m, a_cu;
-  float launch, tile, alone, busy, a_million;
+  float launch, tile, alone, busy, a_million, shared, shared_all;
 };
-static const BlockShape SHAPES[] = {{256, 256, 1, 7.30f, 0.89f, 1.337f, 1.426f, 0.243f}, {256, 320, 1, 10.40f, 0.00f, 1.429f, 1.799f, 0.238f},
-                                    {128, 256, 1, 5.74f, 0.00f, 0.668f, 0.884f, 0.348f}, {192, 128, 1, 3.33f, 2.10f, 0.673f, 0.673f, 0.278f},
-                                    {160, 160, 1, 5.35f, 0.53f, 0.616f, 0.737f, 0.297f}, {128, 160, 1, 3.89f, 0.80f, 0.554f, 0.616f, 0.336f},
-                                    {96, 128, 1, 2.90f, 1.31f, 0.460f, 0.443f, 0.290f}, {128, 96, 1, 3.01f, 0.72f, 0.448f, 0.397f, 0.372f},
-                                    {64, 128, 2, 3.90f, 0.00f, 0.389f, 0.777f, 0.238f}, {64, 64, 2, 4.78f, 0.00f, 0.225f, 0.484f, 0.171f}};
-#define SHAPE_COUNT 10
+static const BlockShape SHAPES[] = {
+    {256, 256, 1, 3.208f, 0.501f, 1.248f, 1.421f, 0.166f, 0.f, 0.f}, {256, 320, 1, 4.907f, 0.205f, 1.570f, 1.513f, 0.137f, 0.f, 0.f},
+    {128, 256, 1, 4.192f, 0.239f, 0.685f, 0.849f, 0.173f, 0.f, 0.f}, {192, 128, 1, 4.432f, 0.351f, 0.612f, 0.617f, 0.165f, 0.f, 0.f},
+    {160, 160, 1, 4.840f, 0.430f, 0.549f, 0.674f, 0.164f, 0.f, 0.f}, {128, 160, 1, 5.356f, 0.222f, 0.503f, 0.512f, 0.169f, 0.f, 0.f},
+    {96, 128, 1, 2.454f, 0.693f, 0.384f, 0.415f, 0.297f, 0.f, 0.f}, {128, 96, 1, 2.827f, 0.103f, 0.406f, 0.430f, 0.288f, 0.f, 0.f},
+    {64, 128, 2, 2.135f, 0.025f, 0.369f, 0.592f, 0.232f, 0.648f, 0.732f}, {64, 64, 2, 2.180f, 0.100f, 0.187f, 0.426f, 0.281f, 0.348f, 0.506f},
+    {128, 128, 1, 2.997f, 0.460f, 0.497f, 0.473f, 0.290f, 0.f, 0.f}, {256, 128, 1, 4.363f, 0.161f, 0.795f, 0.812f, 0.167f, 0.f, 0.f}};
+#define SHAPE_COUNT 12
 
 static float shape_us(const BlockShape& t, int M, int N, int K, int splits, int bytes) {  // (`bytes` of a column of the product in the result)
   const long groups = (long)((N + t.n - 1) / t.n) * ((M + t.m - 1) / t.m) * splits;
   const long places = 256L * t.a_cu, full = groups / places, rest = groups % places;
   const float steps = (float)(K / splits) / 64.f;
   float us = t.launch + t.a_million * 1e-6f * (float)bytes * splits * M * N + (float)full * (t.tile + steps * t.busy);
-  if (rest) us += t.tile + steps * fmaxf(t.alone, t.busy * (float)rest / (float)places);
+  if (full == 0 && rest > 256) us += t.tile + steps * (t.shared + (t.shared_all - t.shared) * (float)(rest - 256) / 256.f);
+  else if (rest) us += t.tile + steps * fmaxf(t.alone, t.busy * (float)rest / (float)places);
   return us;
 }
 
@@ -625,7 +631,9 @@ static int launch_shape(const void* x, const void* w, const void* bias, int bias
     case 6: BLOCK(2, 2, 3, 4, 4, 5, 2, false);
     case 7: BLOCK(2, 2, 4, 3, 3, 5, 2, false);
     case 8: BLOCK(2, 2, 2, 4, 4, 3, 2, false);
-    default: BLOCK(2, 2, 2, 2, 2, 5, 2, false);
+    case 9: BLOCK(2, 2, 2, 2, 2, 5, 2, false);
+    case 10: BLOCK(2, 2, 4, 4, 4, 5, 2, false);
+    default: BLOCK(4, 2, 4, 4, 4, 3, 2, false);
   }
 #undef BLOCK
 }

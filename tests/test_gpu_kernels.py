@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import contextlib
 import math
+import random
 import types
 
 import pytest
@@ -128,8 +129,8 @@ def test_products_without_the_library(own_kernels, rows, inner, outer):
 @pytest.mark.parametrize("rows,inner,outer", [(65, 64, 1536), (96, 1536, 17920), (129, 128, 2050), (200, 192, 40), (257, 1024, 4100), (384, 8960, 1536),
                                               (511, 640, 9000), (640, 320, 20000), (1100, 1536, 6400), (2048, 256, 17920)])
 def test_tiles_of_many_rows(own_kernels, rows, inner, outer):
-    """The LDS-tiled product with each of its tiles, from one stage of K on (fewer stages than it has, as many, more), at rows and weight
-    rows that leave remainders: plain, gated, and in every number of parts that K allows.  Partial sums are float32 sums of
+    """The LDS-tiled product, from one stage of K on, at rows and weight rows that leave remainders (each of its shapes and their stages:
+    `test_every_shape_of_a_tile`): plain, gated, and in every number of parts that K allows.  Partial sums are float32 sums of
     `inner` products of bfloat16 values: a few times sqrt(K) * 2^-24 of a result of size 1."""
     k, dtype = own_kernels, torch.bfloat16
     generator = torch.Generator(device="cuda").manual_seed(rows)
@@ -153,31 +154,76 @@ def test_tiles_of_many_rows(own_kernels, rows, inner, outer):
 
 @pytest.mark.parametrize("shape,rows,plain,float32,gated,inner", [
     (0, 700, 15681, 13070, None, 512), (0, 1300, None, None, 8964, 512), (1, 1025, 13057, 13059, None, 512), (1, 1300, None, None, 10892, 512),
-    (2, 700, 8200, None, 8212, 512), (2, 700, None, 8167, None, 576), (3, 321, 10881, 10888, 10890, 512), (4, 513, 9798, 9796, None, 512),
-    (4, 1025, None, None, 5378, 512), (5, 300, 10185, 11016, 9712, 512), (6, 2047, 1421, None, 1420, 512), (6, 161, None, 11523, None, 512),
-    (7, 161, 10113, 12297, 9542, 512), (8, 97, 9985, 10565, 9666, 512), (9, 97, 614, 603, 612, 512),
+    (2, 700, 8200, None, 8212, 512), (2, 700, None, 8167, None, 576), (3, 200, 16817, None, None, 512), (3, 161, None, 19309, None, 512), (3, 195, None, None, 16830, 512), (4, 513, 9798, 9796, None, 512),
+    (4, 194, None, None, 16590, 512), (5, 260, 12517, None, None, 512), (5, 265, None, 11301, None, 512), (5, 264, None, None, 13070, 512), (6, 2047, 1421, None, 1420, 512),
+    (6, 195, None, 10796, None, 512),
+    (7, 135, 10461, None, None, 512), (7, 130, None, 10525, None, 512), (7, 135, None, None, 10386, 512), (8, 97, 9985, 10565, 9666, 512), (9, 97, 614, 603, 612, 512),
+    (10, 193, 13273, None, None, 512), (10, 388, None, 8104, None, 512), (10, 205, None, None, 12482, 512), (11, 513, 11133, None, None, 512), (11, 324, None, 16577, None, 512),
+    (11, 514, None, None, 11510, 512),
 ])
 def test_every_shape_of_a_tile(kernels, shape, rows, plain, float32, gated, inner):
     """Each shape of the LDS-tiled product where it is picked, at rows and weight rows that leave remainders, in each kind of result.  Bounds as in
     `test_tiles_of_many_rows`; the hardware's 2^x and 1/x are within a few 2^-23."""
-    k = kernels[torch.bfloat16]
-    generator = torch.Generator(device="cuda").manual_seed(rows)
     for kind, outer in enumerate((plain, float32, gated)):
-        if outer is None:
+        if outer is not None:
+            check_shape(kernels[torch.bfloat16], shape, rows, outer, kind, inner)
+
+
+def check_shape(k, shape, rows, outer, kind, inner):
+    assert k._gemm_blocks.llmserve_gemm_blocks_shape(rows, outer, inner, 1, kind) == shape
+    generator = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, inner, generator=generator, device="cuda").to(torch.bfloat16)
+    w = torch.randn(outer, inner, generator=generator, device="cuda").div_(math.sqrt(inner)).to(torch.bfloat16)
+    b = torch.randn(outer, generator=generator, device="cuda")
+    out = torch.full((rows, outer // 2 if kind == 2 else outer), float("nan"), device="cuda", dtype=torch.float32 if kind == 1 else torch.bfloat16)
+    status = k._gemm_blocks.llmserve_gemm_blocks(
+        x.data_ptr(), w.data_ptr(), b.data_ptr(), 1, out.data_ptr(), int(kind == 1), int(kind == 2), rows, outer, inner, 1, torch.cuda.current_stream().cuda_stream)
+    assert status == 0
+    expected = x.double() @ w.double().T + b.double()
+    if kind == 2:
+        expected = F.silu(expected[:, 0::2]) * expected[:, 1::2]
+    bound = dict(atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5) if kind == 1 else TOLERANCE[torch.bfloat16]
+    torch.testing.assert_close(out.double(), expected, **bound)
+
+
+TILES = [(256, 256), (256, 320), (128, 256), (192, 128), (160, 160), (128, 160), (96, 128), (128, 96), (64, 128), (64, 64), (128, 128), (256, 128)]
+
+
+def sizes_of_a_shape(k, shape, kind, inner, multiple):
+    """The smallest of many products that a shape is picked for: more rows and weight rows than a tile has, a remainder of both, weight rows a multiple of `multiple`."""
+    n, m = TILES[shape]
+    draw, best = random.Random(inner + 10 * shape + kind), None
+    for _ in range(20000):
+        rows, outer = draw.randrange(65, 2100), multiple * draw.randrange(1, 20000 // multiple)
+        if rows < m or outer < n or rows % m == 0 or outer % n == 0 or (best and rows * outer >= best[0] * best[1]):
             continue
-        assert k._gemm_blocks.llmserve_gemm_blocks_shape(rows, outer, inner, 1, kind) == shape
-        x = torch.randn(rows, inner, generator=generator, device="cuda").to(torch.bfloat16)
-        w = torch.randn(outer, inner, generator=generator, device="cuda").div_(math.sqrt(inner)).to(torch.bfloat16)
-        b = torch.randn(outer, generator=generator, device="cuda")
-        out = torch.full((rows, outer // 2 if kind == 2 else outer), float("nan"), device="cuda", dtype=torch.float32 if kind == 1 else torch.bfloat16)
-        status = k._gemm_blocks.llmserve_gemm_blocks(
-            x.data_ptr(), w.data_ptr(), b.data_ptr(), 1, out.data_ptr(), int(kind == 1), int(kind == 2), rows, outer, inner, 1, torch.cuda.current_stream().cuda_stream)
-        assert status == 0
-        expected = x.double() @ w.double().T + b.double()
-        if kind == 2:
-            expected = F.silu(expected[:, 0::2]) * expected[:, 1::2]
-        bound = dict(atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5) if kind == 1 else TOLERANCE[torch.bfloat16]
-        torch.testing.assert_close(out.double(), expected, **bound)
+        if k._gemm_blocks.llmserve_gemm_blocks_shape(rows, outer, inner, 1, kind) == shape:
+            best = rows, outer
+    assert best
+    return best
+
+
+@pytest.mark.parametrize("kind", range(3))
+@pytest.mark.parametrize("shape", range(len(TILES)))
+def test_every_shape_of_a_tile_in_whole_pieces(kernels, shape, kind):
+    """Results whose rows are whole pieces of 16 bytes, which leave in such pieces, inside a tile and at both edges (bounds as above)."""
+    k = kernels[torch.bfloat16]
+    check_shape(k, shape, *sizes_of_a_shape(k, shape, kind, 512, 16), kind, 512)
+
+
+# (shape, kind): the K of as few stages of 64 as it is picked with, up to one more than it keeps in LDS
+FEW_STAGES = {(0, 0): (64, 128, 192), (0, 1): (64, 128, 192), (1, 2): (64, 128, 192), (2, 1): (128, 192, 256), (3, 0): (128, 192, 256, 320), (3, 2): (192, 256, 320),
+              (4, 2): (192, 256, 320), (4, 1): (192, 256, 320), (5, 0): (256, 320), (6, 2): (256, 320, 384), (7, 2): (192, 256, 320, 384), (7, 0): (256, 320, 384),
+              (8, 0): (64, 128, 192, 256), (8, 1): (64, 128, 192, 256), (9, 0): (64, 128, 192, 256, 320, 384), (9, 2): (64, 128, 192, 256, 320, 384),
+              (10, 2): (384,), (11, 1): (128, 192, 256), (11, 0): (192, 256)}
+
+
+@pytest.mark.parametrize("shape,kind", FEW_STAGES)
+def test_every_shape_of_a_tile_over_few_stages(kernels, shape, kind):
+    """A K of fewer stages than a shape keeps in LDS, of as many and of one more (bounds as above)."""
+    k = kernels[torch.bfloat16]
+    for inner in FEW_STAGES[shape, kind]:
+        check_shape(k, shape, *sizes_of_a_shape(k, shape, kind, inner, 2 if kind == 2 else 1), kind, inner)
 
 
 @pytest.mark.parametrize("rows,inner,width", [(130, 128, 44), (300, 192, 1092), (1000, 256, 4860), (700, 512, 4100), (2048, 128, 8956)])
@@ -536,8 +582,8 @@ def test_a_float32_row_has_the_same_bits_in_every_batch_of_few_rows(kernels, inn
     (6, 65, 512, 9270, False, 2),
 ])
 def test_float32_whole_tiles(kernels, tile, rows, inner, outer, gated, splits):
-    """The 32-bit product in whole tiles with each of its tiles, where it is picked, from one stage of K on (fewer stages than it has, as many, more), at rows and weight
-    rows that leave remainders: plain, gated and in parts (the bound as above; a gated result's error is that of its two sums)."""
+    """The 32-bit product in whole tiles with each of its tiles, where it is picked, over more stages of K than it keeps in LDS (fewer: `test_float32_whole_tiles_over_few_stages`),
+    at rows and weight rows that leave remainders: plain, gated and in parts (the bound as above; a gated result's error is that of its two sums)."""
     k = kernels[torch.float32]
     assert k._gemm_f32.llmserve_gemm_f32_tile(rows, outer, inner, splits) == 5 + tile
     generator = torch.Generator(device="cuda").manual_seed(rows + outer)
@@ -552,6 +598,27 @@ def test_float32_whole_tiles(kernels, tile, rows, inner, outer, gated, splits):
         expected = F.silu(expected[:, 0::2]) * expected[:, 1::2]
     bound = dict(atol=8 * math.sqrt(inner) * 2.0 ** -24 * (4 if gated else 1), rtol=1e-5)
     torch.testing.assert_close(out.double().sum(0), expected, **bound)
+
+
+@pytest.mark.parametrize("tile,shapes", [
+    (5, {192: (243, 1358), 256: (248, 1348), 320: (243, 1347)}), (6, {192: (65, 2791), 256: (66, 2728), 320: (65, 2764)}),
+    (7, {64: (70, 42), 128: (66, 340), 192: (70, 60), 256: (90, 200), 320: (120, 52)}), (8, {64: (65, 6228), 128: (67, 3002), 192: (97, 2056), 256: (97, 2076)}),
+    (9, {64: (65, 2727), 128: (97, 2721), 192: (68, 5468), 256: (66, 5494)}), (10, {64: (476, 1943), 128: (135, 5563), 192: (102, 5714), 256: (65, 8229)}),
+    (11, {128: (67, 16435), 192: (65, 16386), 256: (65, 16512)}),
+])
+def test_float32_whole_tiles_over_few_stages(kernels, tile, shapes):
+    """The whole tiles over as few stages of 64 k as each is picked with, up to one more than it keeps in LDS (bound as in `test_float32_whole_tiles`)."""
+    k = kernels[torch.float32]
+    for inner, (rows, outer) in shapes.items():
+        assert k._gemm_f32.llmserve_gemm_f32_tile(rows, outer, inner, 1) == tile
+        generator = torch.Generator(device="cuda").manual_seed(rows)
+        x = torch.randn(rows, inner, generator=generator, device="cuda")
+        w = torch.randn(outer, inner, generator=generator, device="cuda") / math.sqrt(inner)
+        b = torch.randn(outer, generator=generator, device="cuda")
+        out = torch.full((rows, outer), float("nan"), device="cuda")
+        status = k._gemm_f32.llmserve_gemm_f32(x.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), 0, rows, outer, inner, 1, torch.cuda.current_stream().cuda_stream)
+        assert status == 0
+        torch.testing.assert_close(out.double(), x.double() @ w.double().T + b.double(), atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5)
 
 
 @pytest.mark.parametrize("x_from,w_from", [(1, 0), (0, 2), (3, 1)])

@@ -39,6 +39,17 @@ def test_parts_of_a_float32_product_whose_operands_begin_anywhere(weight):
     assert {rows: parts(rows, *weight, 0) for rows in FLOAT32_PARTS_ANYWHERE[weight]} == FLOAT32_PARTS_ANYWHERE[weight]
 
 
+@pytest.mark.parametrize("rows,outer,inner,parts,kind", [
+    (400, 4608, 3584, 1, 0), (400, 4608, 3584, 1, 2), (448, 4608, 3584, 1, 2), (224, 4608, 3584, 2, 1), (640, 11008, 2048, 1, 1), (129, 9728, 896, 1, 1),
+    (160, 9728, 896, 1, 0), (513, 896, 4864, 4, 1), (366, 5712, 4608, 3, 1), (378, 5712, 4608, 3, 1),
+])
+def test_no_tiles_that_share_a_few_compute_units(rows, outer, inner, parts, kind):
+    """Tiles of 64 x 128 that come to a few more than 256 workgroups: those that share a CU take nearly twice as long, and the product with them (measured
+    20 to 40 percent behind the other shapes)."""
+    picked = load_module("gemm_blocks").llmserve_gemm_blocks_shape(rows, outer, inner, parts, kind)
+    assert picked >= 0 and not (picked == 8 and 256 < -(-outer // 64) * -(-rows // 128) * parts < 512)  # (8: 64 x 128)
+
+
 @pytest.mark.parametrize("rows,outer,inner", [(200, 17920, 1536), (256, 17920, 1536), (160, 37888, 3584), (200, 37888, 3584), (224, 37888, 3584)])
 def test_no_whole_tiles_where_the_other_float32_kernel_is_ahead(rows, outer, inner):
     """Sizes at which whole tiles were measured 3 to 6 percent behind."""
