@@ -557,17 +557,22 @@ static const BlockShape SHAPES[] = {
 static float shape_us(const BlockShape& t, int M, int N, int K, int splits, int bytes) {  // (`bytes` of a column of the product in the result)
   const long groups = (long)((N + t.n - 1) / t.n) * ((M + t.m - 1) / t.m) * splits;
   const long places = 256L * t.a_cu, full = groups / places, rest = groups % places;
-  const float steps = (float)(K / splits) / 64.f;
+  const float steps = (float)((K / splits + 63) / 64);
   float us = t.launch + t.a_million * 1e-6f * (float)bytes * splits * M * N + (float)full * (t.tile + steps * t.busy);
   if (full == 0 && rest > 256) us += t.tile + steps * (t.shared + (t.shared_all - t.shared) * (float)(rest - 256) / 256.f);
   else if (rest) us += t.tile + steps * fmaxf(t.alone, t.busy * (float)rest / (float)places);
   return us;
 }
 
+// The shapes that take a K which ends in half a stage: five, as each is a kernel of its own in every kind of result.  A half stage costs what a whole one does.
+// Us, in stages of 32 and tiles of 256 x 256 or 128 x 128 -> in those two tiles, picked by other shapes' estimates, and stages of 64 -> now: in three parts 160 rows
+// of N 1,536 K 480 5.4 -> 6.3 -> 3.6; 513 rows of N 512 K 96 4.3 -> 4.8 -> 2.9; 160 rows of N 4,096 K 1,568 18.2 -> 19.0 -> 10.3; 513 rows of it 16.3 -> 16.1 -> 17.6.
+static bool takes_half(int shape) { return shape == 0 || (shape >= 7 && shape <= 10); }
+
 static int pick_shape(int M, int N, int K, int splits, int bytes) {
   int best = 0;
   for (int s = 1; s < SHAPE_COUNT; ++s)
-    if (shape_us(SHAPES[s], M, N, K, splits, bytes) < shape_us(SHAPES[best], M, N, K, splits, bytes)) best = s;
+    if ((K / splits % 64 == 0 || takes_half(s)) && shape_us(SHAPES[s], M, N, K, splits, bytes) < shape_us(SHAPES[best], M, N, K, splits, bytes)) best = s;
   return best;
 }
 
@@ -618,8 +623,13 @@ static int launch_shape(const void* x, const void* w, const void* bias, int bias
 #define BLOCK(...) return launch_block<__VA_ARGS__, TO, OUT>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, {})
   const int shape = pick_shape(M, N, K, splits, OUT == OUT_GATED ? sizeof(TO) / 2 : sizeof(TO));
   if ((K / splits) % 64) {  // a K that ends in half a stage
-    if (shape < 3) BLOCK(4, 2, 4, 8, 3, 2, 2, true);
-    BLOCK(2, 2, 4, 4, 4, 5, 2, true);
+    switch (shape) {
+      case 0: BLOCK(4, 2, 4, 8, 3, 2, 2, true);
+      case 7: BLOCK(2, 2, 4, 3, 3, 5, 2, true);
+      case 8: BLOCK(2, 2, 2, 4, 4, 3, 2, true);
+      case 9: BLOCK(2, 2, 2, 2, 2, 5, 2, true);
+      default: BLOCK(2, 2, 4, 4, 4, 5, 2, true);
+    }
   }
   switch (shape) {
     case 0: BLOCK(4, 2, 4, 8, 3, 2, 2, false);

@@ -226,6 +226,14 @@ def test_every_shape_of_a_tile_over_few_stages(kernels, shape, kind):
         check_shape(k, shape, *sizes_of_a_shape(k, shape, kind, inner, 2 if kind == 2 else 1), kind, inner)
 
 
+@pytest.mark.parametrize("shape,inner", [(0, 96), (0, 160), (0, 480), (7, 288), (7, 352), (7, 544), (8, 32), (8, 96), (8, 224), (9, 32), (9, 96), (9, 352), (10, 544), (10, 800)])
+def test_every_shape_that_takes_half_a_stage(kernels, shape, inner):
+    """A K that ends in half a stage, one of half a stage alone among them: rows of the result in whole pieces and not (bounds as above)."""
+    k = kernels[torch.bfloat16]
+    for kind, multiple in ((0, 16), (1, 1), (2, 2)):
+        check_shape(k, shape, *sizes_of_a_shape(k, shape, kind, inner, multiple), kind, inner)
+
+
 @pytest.mark.parametrize("rows,inner,width", [(130, 128, 44), (300, 192, 1092), (1000, 256, 4860), (700, 512, 4100), (2048, 128, 8956)])
 def test_gated_widths_of_four_mod_eight(own_kernels, rows, inner, width):
     """A gated result whose rows begin in the middle of 16 bytes every other time: each value in its place and nothing outside (bound as in `test_tiles_of_many_rows`)."""
