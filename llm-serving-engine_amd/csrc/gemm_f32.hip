@@ -14,6 +14,8 @@
 // LDS in wave order, so a row's bits depend on the shape of the weight only, never on the batch (the tiled kernel's, for
 // larger ones, on the number of rows too).
 //
+// gemm_f32_whole (65 to 512 rows where its tiles are estimated ahead, see `pick_tile`) is described at its code.
+//
 // gemm_f32_tiled (more rows, prompt portions): a tile of weight rows by rows of x a workgroup of four waves, each
 // one to four tiles of v_mfma_f32_32x32x2_f32; K in steps of 16 (of 32 or 64 where two or four waves share a tile
 // and take 16 each) through two LDS buffers.  A staged row is padded by 4 floats, so that the 16-byte reads of an
@@ -362,11 +364,11 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const float* __rest
   }
 }
 
-// gemm_f32_whole (more rows, K in parts of whole stages of 64): a tile of 16 NT weight rows by 16 MT rows of x a workgroup, of which each of its four
+// gemm_f32_whole (65 to 512 rows, K in parts of whole stages of 64): a tile of 16 NT weight rows by 16 MT rows of x a workgroup, of which each of its four
 // waves multiplies all with a quarter of every stage's k, in tiles of v_mfma_f32_16x16x4_f32, and whose sums meet through LDS at the end in the order of their
 // k.  So a tile may be any number of sixteens (129 rows make 144, not 160) and have what it takes for one round of 256 workgroups, which is what bounds the kernel
-// above.  Us before (that kernel) -> now, weights out of memory: N 17,920 K 1,536 gated: 65 rows 75 -> 54, 129 rows 105 -> 88, 160 rows 108 -> 96; N 2,048 K
-// 1,536: 65 rows 17 -> 11, 129 rows 24 -> 15, 512 rows 44 -> 35; N 1,536 K 8,960 in parts: 129 rows 60 -> 44, 384 rows 105 -> 103.  Both operands go from memory straight into LDS, as in gemm_blocks.hip: a stage is 64 k, 256 bytes a row, piece p of 16 of row r in slot
+// above.  Us, that kernel -> this, weights out of memory: N 17,920 K 1,536 gated: 65 rows 75 -> 54, 129 rows 105 -> 88, 160 rows (which a replayed step of 129 tokens has)
+// 105 -> 99; N 2,048 K 1,536: 65 rows 17 -> 11, 129 rows 24 -> 15, 512 rows 43 -> 36; N 1,536 K 8,960 in parts: 129 rows 60 -> 44.  Both operands go from memory straight into LDS, as in gemm_blocks.hip: a stage is 64 k, 256 bytes a row, piece p of 16 of row r in slot
 // p ^ (r % 16), so that the sixteen rows that LDS serves together hit all its banks; element j of each lane's piece goes to instruction j, so that an instruction
 // takes k = 4 g + j of a wave's sixteen.  A wave holds all it needs of a stage when it begins to multiply it: behind one barrier the stage is asked for
 // anew, and the next one's operands are read, between the products.
@@ -555,33 +557,40 @@ static float tiled_us(const TileCost& t, int M, int N, int K, int splits) {
 #define WHOLE_TILES(X) X(1, 3) X(1, 5) X(2, 2) X(2, 3) X(3, 3) X(3, 5) X(5, 5)
 constexpr int TILE_COUNT = 5, WHOLE_COUNT = 7, ALL_TILES = TILE_COUNT + WHOLE_COUNT;
 
-// Which kernel takes a product of up to 512 rows goes by what their tiles take, us: a launch, a tile, and a tile's 64 k where it has its CU to itself, where two share
-// one, and where all CUs are as full as they get; a million bytes of the result.  (Once a CU has been full, what is left comes two to a CU, too.)  Fitted to
-// 5,700 products of 65 to 512 rows of twelve weights, in one to eight parts, every weight out of memory, each tile within 2 to 7 percent of what was measured on average.  Of 182
-// products the choice by them is 2 percent slower than the best of all tiles on average and 10 percent faster than the other kernel alone; of these and of 102 drawn
-// ones none is more than 1 percent slower than that kernel, which AHEAD_FROM is for (with 0.98 three of the drawn ones were 3 to 4 percent slower).  Us, that kernel ->
-// whole tiles wherever an estimate of theirs, beside that kernel's own, had them ahead -> now: N 17,920 K 1,536 gated 200 rows 124 -> 131 -> 124, 256 rows
-// 142 -> 151 -> 142; N 1,536 K 8,960 in parts 224 rows 68 -> 79 -> 68; N 4,608 K 3,584 384 rows 144 -> 152 -> 136.
+// Which kernel takes a product of up to 512 rows goes by what their tiles take, us: a launch, a tile, a million bytes of the result, and a tile's 64 k where few CUs are
+// busy, and where all are; of the whole ones of which a CU holds two also once a first CU holds two (`shared`) and once all do.  The other kernel's workgroups
+// come to a CU as many as are left, so theirs (`a_cu` 0) are the first one's 64 k and every further one's.  Fitted to 965 products of 65 to 512 rows
+// of 22 weights, in one to eight parts, every weight out of memory.  The choice by them is 18 percent faster than the other kernel alone and at none of 508 products in
+// one piece or 107 in parts more than 3 percent slower, which AHEAD_FROM is for (0.97: one 17 percent).  Priced as if a round of 256 of the other kernel's workgroups took what
+// one of many rounds does, that kernel kept products that were the whole tiles'.  Us, that kernel -> by that estimate -> by this: 128 rows of N 2,048 K 1,536
+// 18.3 -> 18.3 -> 13.4, 512 rows of it 43.0 -> 43.0 -> 36.2, 160 rows of N 17,920 K 1,536 gated 105 -> 106 -> 99; 200 rows of it 124 each way, as whole tiles 131.
 struct TileTimes {
   int n, m, a_cu;
-  float launch, tile, alone, shared, busy, a_million;
+  float launch, tile, alone, busy, a_million, shared, shared_all;
 };
 static const TileTimes TIMES[ALL_TILES] = {
-    {128, 128, 1, 5.983f, 0.011f, 4.619f, 0.f, 3.662f, 0.259f}, {128, 64, 1, 5.231f, 0.116f, 2.649f, 0.f, 1.888f, 0.225f},
-    {64, 64, 1, 3.933f, 0.079f, 1.505f, 0.f, 0.988f, 0.253f},   {64, 32, 1, 3.292f, 0.244f, 0.970f, 0.f, 0.512f, 0.345f},
-    {32, 32, 1, 3.966f, 0.335f, 0.506f, 0.f, 0.314f, 0.511f},   {16, 48, 2, 3.100f, 0.000f, 0.328f, 0.531f, 0.505f, 0.724f},
-    {16, 80, 2, 3.422f, 0.000f, 0.455f, 0.765f, 0.774f, 0.550f}, {32, 32, 2, 2.859f, 0.052f, 0.355f, 0.635f, 0.597f, 0.667f},
-    {32, 48, 2, 3.355f, 0.028f, 0.516f, 0.930f, 0.856f, 0.376f}, {48, 48, 2, 2.818f, 0.021f, 0.773f, 1.348f, 1.209f, 0.472f},
-    {48, 80, 1, 2.043f, 1.903f, 1.173f, 0.f, 1.189f, 0.220f},   {80, 80, 1, 2.256f, 2.534f, 1.848f, 0.f, 1.872f, 0.313f}};
-constexpr float AHEAD_FROM = 0.94f;
+    {128, 128, 0, 3.102f, 1.266f, 4.934f, 4.341f, 0.211f, 0.f, 0.f}, {128, 64, 0, 4.547f, 0.887f, 2.181f, 2.134f, 0.211f, 0.f, 0.f},
+    {64, 64, 0, 2.093f, 0.972f, 1.454f, 1.064f, 0.264f, 0.f, 0.f}, {64, 32, 0, 2.252f, 0.568f, 1.220f, 0.531f, 0.304f, 0.f, 0.f},
+    {32, 32, 0, 3.884f, 0.937f, 0.655f, 0.319f, 0.252f, 0.f, 0.f}, {16, 48, 2, 2.158f, 0.239f, 0.311f, 0.533f, 0.596f, 0.655f, 0.518f},
+    {16, 80, 2, 1.828f, 0.123f, 0.515f, 0.819f, 0.440f, 0.791f, 0.812f}, {32, 32, 2, 2.935f, 0.042f, 0.359f, 0.637f, 0.483f, 0.586f, 0.685f},
+    {32, 48, 2, 2.500f, 0.323f, 0.516f, 0.881f, 0.391f, 0.848f, 0.858f}, {48, 48, 2, 2.708f, 0.322f, 0.770f, 1.531f, 0.241f, 1.287f, 1.383f},
+    {48, 80, 1, 1.836f, 1.291f, 1.202f, 1.073f, 0.272f, 0.f, 0.f}, {80, 80, 1, 1.915f, 2.209f, 1.853f, 1.708f, 0.174f, 0.f, 0.f}};
+// (in parts, where two numbers of them are compared as well, from further ahead: with 0.95 224 rows of N 1,536 K 8,960 66 -> 71 us)
+constexpr float AHEAD_FROM = 0.95f, PARTS_AHEAD_FROM = 0.88f;
 
 // Without what reads parts of K again.
 static float measured_us(const TileTimes& t, int M, int N, int K, int splits) {
   const long groups = (long)((N + t.n - 1) / t.n) * ((M + t.m - 1) / t.m) * splits;
-  const long places = 256L * t.a_cu, full = groups / places, rest = groups % places;
   const float steps = (float)K / (float)splits / 64.f;
-  float us = t.launch + t.a_million * 4e-6f * (float)splits * M * N + (float)full * (t.tile + steps * t.busy);  // (a gated result is half as large)
-  if (rest) us += t.tile + steps * fmaxf(t.a_cu == 2 && (full || rest > 256) ? t.shared : t.alone, t.busy * (float)rest / (float)places);
+  float us = t.launch + t.a_million * 4e-6f * (float)splits * M * N;  // (a gated result is half as large)
+  if (t.a_cu == 0) {
+    const float rounds = (float)((groups + 255) / 256);
+    return us + rounds * t.tile + steps * (t.alone + (rounds - 1.f) * t.busy);
+  }
+  const long places = 256L * t.a_cu, full = groups / places, rest = groups % places;
+  us += (float)full * (t.tile + steps * t.busy);
+  if (rest > 256) us += t.tile + steps * (t.shared + (t.shared_all - t.shared) * (float)(rest - 256) / 256.f);
+  else if (rest) us += t.tile + steps * fmaxf(t.alone, t.busy * (float)rest / (float)places);
   return us;
 }
 
@@ -631,7 +640,7 @@ extern "C" int llmserve_gemm_f32_parts(int M, int N, int K, int in_pieces) {
   if (!in_pieces || M > 512) return best;
   auto read_us = [&](int splits) { return splits > 1 ? (float)splits * M * N * 4e-6f / 4.5f : 0.f; };
   const int shortest = best * TILE_WAVES[tile];
-  best_us = AHEAD_FROM * (measured_us(TIMES[tile], M, N, K, best) + read_us(best));
+  best_us = PARTS_AHEAD_FROM * (measured_us(TIMES[tile], M, N, K, best) + read_us(best));
   for (int splits = 1; splits <= 8; ++splits) {
     if (splits > 1 && K / splits < 256) break;
     float us;
@@ -661,7 +670,7 @@ static int launch_tiled(const float* x, const float* w, const float* bias, float
 
 // out [M, N] (or [splits, M, N] partial sums) = x [M, K] . w [N, K]^T (+ bias [N]); all float32, K a multiple
 // of 4.  gated: w's rows alternate gate and up (N even), out is [M, N / 2] = silu(gate) * up, no splits.
-// Up to 64 rows of x go to the weight-streaming kernel, more to the tiled one.  (Us at 33 / 48 / 64 rows, in parts with what adds them
+// Up to 64 rows of x go to the weight-streaming kernel, more to whole tiles or the tiled kernel (`pick_tile`).  (Us at 33 / 48 / 64 rows, in parts with what adds them
 // up, one tile of weights against the tiled kernel against this: N 17,920 K 1,536 gated 56 / 61 / 74, 53 / 54 / 54, 52 / 55 / 63; N 1,536 K 8,960
 // in parts 32 / 36 / 42, 30 / 30 / 31, 33 / 35 / 42; N 2,048 K 1,536 17 / 18 / 21, 18 / 18 / 18, 14 / 16 / 21; N 37,888 K 3,584 gated
 // 221 / 266 / 316, 202 / 206 / 205, 175 / 189 / 211; N 3,584 K 18,944 in parts 138 / 148 / 176, 109 / 110 / 110, 94 / 100 / 119.)

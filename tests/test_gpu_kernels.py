@@ -583,10 +583,10 @@ def test_a_float32_row_has_the_same_bits_in_every_batch_of_few_rows(kernels, inn
 
 @pytest.mark.parametrize("tile,rows,inner,outer,gated,splits", [
     (0, 70, 512, 42, False, 1), (0, 70, 512, 42, True, 1), (0, 70, 1536, 42, False, 2), (1, 65, 320, 2723, False, 1),
-    (1, 65, 320, 2724, True, 1), (1, 65, 512, 6818, False, 2), (2, 97, 512, 1299, False, 1), (2, 97, 512, 1300, True, 1),
-    (2, 97, 1536, 690, False, 2), (3, 129, 256, 10887, False, 1), (3, 129, 256, 10888, True, 1), (3, 129, 256, 11469, False, 4),
-    (4, 161, 256, 6108, True, 1), (4, 65, 320, 5446, False, 1), (4, 65, 256, 1367, False, 4), (5, 65, 256, 10925, False, 1),
-    (5, 65, 256, 10926, True, 1), (5, 65, 512, 5452, False, 2), (6, 65, 256, 19128, True, 1), (6, 65, 320, 18435, False, 1),
+    (1, 65, 320, 2724, True, 1), (1, 65, 512, 6818, False, 2), (2, 66, 512, 2078, False, 1), (2, 97, 512, 1368, True, 1),
+    (2, 97, 1536, 690, False, 2), (3, 129, 256, 10887, False, 1), (3, 129, 256, 10888, True, 1), (3, 81, 256, 1590, False, 4),
+    (4, 161, 256, 6108, True, 1), (4, 161, 320, 2740, False, 1), (4, 87, 256, 1418, False, 4), (5, 98, 256, 6134, False, 1),
+    (5, 98, 256, 6134, True, 1), (5, 97, 512, 3033, False, 2), (6, 65, 256, 19128, True, 1), (6, 65, 320, 18435, False, 1),
     (6, 65, 512, 9270, False, 2),
 ])
 def test_float32_whole_tiles(kernels, tile, rows, inner, outer, gated, splits):
@@ -608,17 +608,18 @@ def test_float32_whole_tiles(kernels, tile, rows, inner, outer, gated, splits):
     torch.testing.assert_close(out.double().sum(0), expected, **bound)
 
 
-@pytest.mark.parametrize("tile,shapes", [
-    (5, {192: (243, 1358), 256: (248, 1348), 320: (243, 1347)}), (6, {192: (65, 2791), 256: (66, 2728), 320: (65, 2764)}),
-    (7, {64: (70, 42), 128: (66, 340), 192: (70, 60), 256: (90, 200), 320: (120, 52)}), (8, {64: (65, 6228), 128: (67, 3002), 192: (97, 2056), 256: (97, 2076)}),
-    (9, {64: (65, 2727), 128: (97, 2721), 192: (68, 5468), 256: (66, 5494)}), (10, {64: (476, 1943), 128: (135, 5563), 192: (102, 5714), 256: (65, 8229)}),
-    (11, {128: (67, 16435), 192: (65, 16386), 256: (65, 16512)}),
-])
-def test_float32_whole_tiles_over_few_stages(kernels, tile, shapes):
-    """The whole tiles over as few stages of 64 k as each is picked with, up to one more than it keeps in LDS (bound as in `test_float32_whole_tiles`)."""
+WHOLE_TILES = [(16, 48), (16, 80), (32, 32), (32, 48), (48, 48), (48, 80), (80, 80)]
+FEW_FLOAT32_STAGES = [(0, 192), (0, 256), (0, 320), (1, 64), (1, 128), (1, 192), (1, 256), (2, 128), (2, 192), (2, 256), (2, 320),
+    (3, 64), (3, 128), (3, 192), (3, 256), (4, 64), (4, 128), (4, 192), (4, 256), (5, 128), (5, 192), (5, 256), (6, 64), (6, 128), (6, 192), (6, 256)]
+
+
+@pytest.mark.parametrize("tile,inner", FEW_FLOAT32_STAGES)
+def test_float32_whole_tiles_over_few_stages(kernels, tile, inner):
+    """The whole tiles over as few stages of 64 k as each is picked with, up to one more than it keeps in LDS: result rows that leave in pieces of 16 bytes and rows that
+    do not (bound as in `test_float32_whole_tiles`)."""
     k = kernels[torch.float32]
-    for inner, (rows, outer) in shapes.items():
-        assert k._gemm_f32.llmserve_gemm_f32_tile(rows, outer, inner, 1) == tile
+    for multiple in (1, 4):
+        rows, outer = sizes_of_a_whole_tile(k, tile, inner, multiple)
         generator = torch.Generator(device="cuda").manual_seed(rows)
         x = torch.randn(rows, inner, generator=generator, device="cuda")
         w = torch.randn(outer, inner, generator=generator, device="cuda") / math.sqrt(inner)
@@ -627,6 +628,20 @@ def test_float32_whole_tiles_over_few_stages(kernels, tile, shapes):
         status = k._gemm_f32.llmserve_gemm_f32(x.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), 0, rows, outer, inner, 1, torch.cuda.current_stream().cuda_stream)
         assert status == 0
         torch.testing.assert_close(out.double(), x.double() @ w.double().T + b.double(), atol=8 * math.sqrt(inner) * 2.0 ** -24, rtol=1e-5)
+
+
+def sizes_of_a_whole_tile(k, tile, inner, multiple):
+    """The smallest of many products that a whole tile is picked for, with a remainder of rows and of weight rows."""
+    n, m = WHOLE_TILES[tile]
+    draw, best = random.Random(inner + 10 * tile), None
+    for _ in range(20000):
+        rows, outer = draw.randrange(65, 513), multiple * draw.randrange(17, draw.choice((3000, 20000)) // multiple)
+        if rows % m == 0 or outer % n == 0 or (best and rows * outer >= best[0] * best[1]):
+            continue
+        if k._gemm_f32.llmserve_gemm_f32_tile(rows, outer, inner, 1) == 5 + tile:
+            best = rows, outer
+    assert best
+    return best
 
 
 @pytest.mark.parametrize("x_from,w_from", [(1, 0), (0, 2), (3, 1)])

@@ -56,6 +56,12 @@ def test_no_whole_tiles_where_the_other_float32_kernel_is_ahead(rows, outer, inn
     assert 0 <= load_module("gemm_f32").llmserve_gemm_f32_tile(rows, outer, inner, 1) < 5
 
 
+@pytest.mark.parametrize("rows,outer,inner", [(128, 2048, 1536), (512, 2048, 1536), (160, 17920, 1536), (96, 17920, 1536), (512, 3584, 3584)])
+def test_whole_tiles_where_they_are_ahead_of_the_other_float32_kernel(rows, outer, inner):
+    """Sizes of few rounds of workgroups, at which whole tiles were measured 5 to 30 percent ahead."""
+    assert load_module("gemm_f32").llmserve_gemm_f32_tile(rows, outer, inner, 1) >= 5
+
+
 @pytest.mark.parametrize("module,kernel", [("gemm_blocks", "gemm_block_kernel"), ("gemm_f32", "gemm_f32_whole_kernel"),
                                            ("gemm_bf16", "gemm_stream_kernel"), ("gemm_bf16", "gemm_ring_kernel")])
 def test_kernels_that_read_ahead_keep_their_registers(module, kernel):
