@@ -11,7 +11,7 @@
 // sixteen lanes that LDS serves together (the same piece of sixteen rows) hit all its banks (measured: no conflicts; with
 // p ^ (r % 8), half of the reads' time).
 //
-// What bounds it: at 8,192 rows of 8,192 x 8,192 the power that the matrix cores draw (0.78 ms, 1.41 PFLOP/s; the library 0.73): products alone, of random
+// What bounds it: at 8,192 rows of 8,192 x 8,192 the power that the matrix cores draw (shown for these sizes alone: gate/up of 2,048 rows is at 1.18 PFLOP/s; 0.78 ms, 1.41 PFLOP/s; the library 0.73): products alone, of random
 // operands in registers, run at 2.0 PFLOP/s, of zeros at 2.4.  Tiles of 32 x 32 x 16, which move twice the sums in and out of the accumulators for a
 // product, reach 1.81 there, and 0.83 ms here.  At the sizes a decoder has, how the tiles divide over 256 CUs, what a tile costs besides its
 // products, and the way of the operands: a CU takes 64 bytes a clock from its caches, so what a stage brings (74 KB for 256 x 320) takes 1,150 clocks of the
@@ -48,8 +48,8 @@ __device__ __forceinline__ void tile_of_workgroup(int index, int tiles_n, int ti
 }
 
 // A result of more than so many bytes is stored past the caches: it does not fit the eight L2s (32 MB) beside the operands, and what lies there
-// at a kernel's end is written back before the next one starts.  Us, kept -> past: 2,048 rows of N 17,920 K 1,536 gated (37 MB) 110.8 -> 102.8; a prompt of
-// 2,048 tokens 7,138 -> 7,067.  Results that fit are read by the next kernel from there: a prompt of 77 1,798 -> 1,840.
+// at a kernel's end is written back before the next one starts.  Us, kept -> past: 2,048 rows of N 17,920 K 1,536 gated (37 MB) 110.8 -> 102.8, a whole prompt of
+// 2,048 tokens with it by 1 percent (7,138 -> 7,067 in one run).  Results that fit are read by the next kernel from there: a prompt of 77 1,798 -> 1,840.
 #define STREAMED_FROM (16u << 20)
 
 // What the way out does with the sums (and the bias).

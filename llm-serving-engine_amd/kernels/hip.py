@@ -458,7 +458,7 @@ class HipKernels:
     def _rotated_ahead(rows: int, out_features: int, in_features: int) -> bool:
         """Where `linear_rotated` is ahead of the product (the library's up to 512 rows) and the kernel that rotates and stores: while one
         round of 64 x 64 tiles holds the result, for K up to 2,048 one of 128 x 64, and where the product alone is the tiled kernel's too.
-        Us, both in a captured chain over different weights, before -> when it was made (the kernel alone has lost 1 to 2.5 us since): N 2,048 K 1,536: 96 rows 15.5 -> 11.6, 256 16.1 -> 11.7, 512 17.4
+        Us, both in a captured chain over different weights, before -> when it was made (the kernel alone has become 1 to 2.5 us faster since): N 2,048 K 1,536: 96 rows 15.5 -> 11.6, 256 16.1 -> 11.7, 512 17.4
         -> 12.9, 1,024 23.9 -> 18.5, 2,048 27.3 -> 26.0; N 1,152 K 896: 96 rows 14.6 -> 8.9, 1,024 17.3 -> 13.1; N 2,560 K 2,048: 96 rows 17.5 -> 13.4,
         448 21.1 -> 21.5, 768 23.5 -> 21.5; N 4,608 K 3,584: 96 rows 26.0 -> 19.9, 192 36.2 -> 22.3, 320 30.3 -> 32.9, 1,024 52.2 -> 58.7; N 7,168 K
         5,120: 96 rows 35.6 -> 30.2, 320 54.2 -> 55.4, 2,048 142 -> 168."""
