@@ -575,7 +575,8 @@ static const TileTimes TIMES[ALL_TILES] = {
     {16, 80, 2, 1.828f, 0.123f, 0.515f, 0.819f, 0.440f, 0.791f, 0.812f}, {32, 32, 2, 2.935f, 0.042f, 0.359f, 0.637f, 0.483f, 0.586f, 0.685f},
     {32, 48, 2, 2.500f, 0.323f, 0.516f, 0.881f, 0.391f, 0.848f, 0.858f}, {48, 48, 2, 2.708f, 0.322f, 0.770f, 1.531f, 0.241f, 1.287f, 1.383f},
     {48, 80, 1, 1.836f, 1.291f, 1.202f, 1.073f, 0.272f, 0.f, 0.f}, {80, 80, 1, 1.915f, 2.209f, 1.853f, 1.708f, 0.174f, 0.f, 0.f}};
-// (in parts, where two numbers of them are compared as well, from further ahead: with 0.95 224 rows of N 1,536 K 8,960 66 -> 71 us)
+// (in parts, where two numbers of them are compared as well, from further ahead: with 0.95 224 rows of N 1,536 K 8,960 66 -> 71 us, 160 rows of N 3,584 K
+// 3,584 in eight 50 -> 55)
 constexpr float AHEAD_FROM = 0.95f, PARTS_AHEAD_FROM = 0.88f;
 
 // Without what reads parts of K again.
@@ -606,7 +607,7 @@ static int pick_tile(int M, int N, int K, int splits, bool in_pieces, float* us 
     for (int t = whole + 1; t < ALL_TILES; ++t)
       if (measured_us(TIMES[t], M, N, K, splits) < measured_us(TIMES[whole], M, N, K, splits)) whole = t;
     const float here = measured_us(TIMES[whole], M, N, K, splits);
-    if (here < AHEAD_FROM * measured_us(TIMES[best], M, N, K, splits)) {
+    if (here < (splits == 1 ? AHEAD_FROM : PARTS_AHEAD_FROM) * measured_us(TIMES[best], M, N, K, splits)) {
       if (us) *us = here;
       return whole;
     }

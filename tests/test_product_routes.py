@@ -56,6 +56,13 @@ def test_no_whole_tiles_where_the_other_float32_kernel_is_ahead(rows, outer, inn
     assert 0 <= load_module("gemm_f32").llmserve_gemm_f32_tile(rows, outer, inner, 1) < 5
 
 
+@pytest.mark.parametrize("rows,outer,inner", [(160, 3584, 3584), (224, 1536, 8960)])
+def test_no_whole_tiles_in_parts_where_the_other_float32_kernel_is_ahead(rows, outer, inner):
+    """Sizes at which whole tiles were measured 8 to 10 percent behind in the parts that the product has."""
+    library = load_module("gemm_f32")
+    assert 0 <= library.llmserve_gemm_f32_tile(rows, outer, inner, library.llmserve_gemm_f32_parts(rows, outer, inner, 1)) < 5
+
+
 @pytest.mark.parametrize("rows,outer,inner", [(128, 2048, 1536), (512, 2048, 1536), (160, 17920, 1536), (96, 17920, 1536), (512, 3584, 3584)])
 def test_whole_tiles_where_they_are_ahead_of_the_other_float32_kernel(rows, outer, inner):
     """Sizes of few rounds of workgroups, at which whole tiles were measured 5 to 30 percent ahead."""
