@@ -14,6 +14,7 @@
 // silu(gate) * up (reference model.py:188) to out[M, N / 2].
 #include "common.h"
 #include <type_traits>
+#include <utility>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -274,112 +275,8 @@ static int pick_waves(const void* x, const void* w, const void* bias, int bias_i
   return pick_tiles<16, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, tail);
 }
 
-// gemm_pair: gemm_skinny for up to 16 rows of x with NT tiles of 16 weight rows a wave, which share
-// the wave's x: every workgroup reads all of x for its K range, M / (16 NT) of what it reads of the
-// weights, and the chiplets' L2 delivers little more than HBM does, so at 16 rows and NT = 1 the
-// x doubles the traffic.  More tiles a wave also means more bytes under way a wave and fewer
-// workgroups: it pays for long K ranges and big weights (7B sizes at 8 rows: gate/up 57.7 -> 52.1 us
-// with two tiles, down 32.1 -> 26.3 us with four; 1.5B sizes at 16 rows: gate/up 18.0 -> 16.9 us).
-template <int WAVES, int NT, typename TO, int GATED>
-__global__ __launch_bounds__(WAVES * 64) void gemm_pair_kernel(const bf16_t* __restrict__ x,
-                                                               const bf16_t* __restrict__ w,
-                                                               const void* __restrict__ bias, int bias_is_float,
-                                                               TO* __restrict__ out, int M, int N, int K,
-                                                               int k_split, Tail tail) {
-  extern __shared__ float partial[];  // [WAVES][NT][64 lanes][4]
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int r = lane & 15, g = lane >> 4;
-  const int k_first = blockIdx.y * k_split;
-  const bf16_t* w_row[NT];
-#pragma unroll
-  for (int s = 0; s < NT; ++s)
-    w_row[s] = w + (size_t)min(((int)blockIdx.x * NT + s) * 16 + r, N - 1) * K + k_first + g * 8;
-  const bool x_live = r < M;
-  const bf16_t* x_row = x + (size_t)min(r, M - 1) * K + k_first + g * 8;
-  f32x4 acc[NT];
-#pragma unroll
-  for (int s = 0; s < NT; ++s) acc[s] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  // the bias of the four outputs this lane will finish (wave s finishes tile s) is asked for now
-  float bias_here[4] = {0.f, 0.f, 0.f, 0.f};
-  if (bias && blockIdx.y == 0 && wave < NT) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      bias_here[i] = load_as_float(bias, bias_is_float, min(((int)blockIdx.x * NT + wave) * 16 + g * 4 + i, N - 1));
-  }
-  const int groups = k_split / (STEP * GROUP);
-  bf16x8 a[NT][GROUP], a_next[NT][GROUP];
-  int group = wave;
-  if (group < groups) {
-#pragma unroll
-    for (int s = 0; s < NT; ++s)
-#pragma unroll
-      for (int u = 0; u < GROUP; ++u) a[s][u] = load8_stream(w_row[s] + (group * GROUP + u) * STEP);
-  }
-  while (group < groups) {
-    const int next = group + WAVES;
-    bf16x8 b[GROUP];
-#pragma unroll
-    for (int u = 0; u < GROUP; ++u) b[u] = x_live ? load8(x_row + (group * GROUP + u) * STEP) : zero;
-    asm volatile("" ::: "memory");
-    if (next < groups) {
-#pragma unroll
-      for (int s = 0; s < NT; ++s)
-#pragma unroll
-        for (int u = 0; u < GROUP; ++u) a_next[s][u] = load8_stream(w_row[s] + (next * GROUP + u) * STEP);
-    }
-#pragma unroll
-    for (int u = 0; u < GROUP; ++u)
-#pragma unroll
-      for (int s = 0; s < NT; ++s) acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s][u], b[u], acc[s], 0, 0, 0);
-#pragma unroll
-    for (int s = 0; s < NT; ++s)
-#pragma unroll
-      for (int u = 0; u < GROUP; ++u) a[s][u] = a_next[s][u];
-    group = next;
-  }
-#pragma unroll
-  for (int s = 0; s < NT; ++s) *(f32x4*)(partial + ((wave * NT + s) * 64 + lane) * 4) = acc[s];
-  __syncthreads();
-  if (wave >= NT) return;
-  const int s = wave;
-  f32x4 total = (f32x4){0.f, 0.f, 0.f, 0.f};
-  for (int v = 0; v < WAVES; ++v) total += *(const f32x4*)(partial + ((v * NT + s) * 64 + lane) * 4);
-  const int m = r;
-  const int n_first = ((int)blockIdx.x * NT + s) * 16 + g * 4;
-  if (m >= M) return;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) total[i] += bias_here[i];
-  if (GATED == 3) {
-    store_with_tail(out, tail, m, n_first, N, total);
-  } else if (GATED) {
-    TO* dst = out + (size_t)m * (N / 2) + n_first / 2;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      if (n_first + 2 * i + 1 < N) {
-        const float gate = total[2 * i], up = total[2 * i + 1];
-        dst[i] = from_float<TO>(gate_value<GATED>(gate) * up);
-      }
-    }
-  } else {
-    TO* dst = out + ((size_t)blockIdx.y * M + m) * N + n_first;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (n_first + i < N) dst[i] = from_float<TO>(total[i]);
-  }
-}
-
-template <int NT, typename TO, int GATED>
-static int launch_pair(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N,
-                       int K, int splits, hipStream_t stream, Tail tail = {}) {
-  const size_t lds = (size_t)4 * NT * 64 * 4 * sizeof(float);
-  hipLaunchKernelGGL((gemm_pair_kernel<4, NT, TO, GATED>), dim3((N + 16 * NT - 1) / (16 * NT), splits), dim3(256), lds,
-                     stream, (const bf16_t*)x, (const bf16_t*)w, bias, bias_is_float, (TO*)out, M, N, K, K / splits, tail);
-  return LAUNCH_STATUS();
-}
-
 // ---------------------------------------------------------------------------- the streams through LDS
-// gemm_stream: gemm_skinny / gemm_pair for up to 16 rows of x with both operands brought through LDS.
+// gemm_stream: 17 to 64 rows of x and a small weight, both operands brought through LDS.
 // The matrix cores take a weight row as a row of the A operand, lane (r, g) holding k = 8g .. 8g+7 of
 // row r, so the four lanes the address unit serves together (r .. r+3 at one g) would read 16 bytes
 // of four different rows, four cache lines, and a load of a wave costs that unit four times what
@@ -422,7 +319,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
                                                                  const bf16_t* __restrict__ w,
                                                                  const void* __restrict__ bias, int bias_is_float,
                                                                  TO* __restrict__ out, int M, int N, int K,
-                                                                 int k_split, Tail tail, Link link) {
+                                                                 int k_split, Link link) {
   extern __shared__ __attribute__((aligned(16))) unsigned char stream_lds[];
   constexpr int OPERANDS = (NT + MT) * G;                // of one group: the weight tiles' steps, then x's
   constexpr int STAGE_BYTES = OPERANDS * STREAM_CHUNK;
@@ -456,19 +353,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
           load_as_float(bias, bias_is_float, min(((int)blockIdx.x * NT + wave / MT) * 16 + g * 4 + i, N - 1));
   }
   static_assert(LINK != INTO_NORM || (TILES <= WAVES && sizeof(TO) == 4), "a wave finishes one tile of whole sums");
-  static_assert(LINK != SCALED || MT == 1, "up to 16 rows");
+  static_assert(LINK != SCALED, "gemm_flow and gemm_ring read such rows");
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // so that the counts below count the stream alone
   LinkedColumns columns;  // (ahead of the stream, whose first wait covers them)
   if (LINK == INTO_NORM) columns = linked_columns(link, (wave % MT) * 16 + r, ((int)blockIdx.x * NT + min(wave, TILES - 1) / MT) * 16 + g * 4, M, N);
-  // The sums of squares [tiles, 16 rows] go into LDS ahead of the stream, whose first wait covers them: a workgroup that waited
-  // for them by themselves lost a trip to memory, and there are several rounds of workgroups (gate/up 11.7 -> 15.6 us).
-  float* raw_sums = (float*)(stream_lds + (WAVES * WAVE_BYTES > WAVES * TILES * 1024 ? WAVES * WAVE_BYTES : WAVES * TILES * 1024));
-  float* shares = raw_sums + (size_t)(link.tiles + 15) / 16 * 256;  // [WAVES][16 rows]
-  if (LINK == SCALED)
-    for (int chunk = wave; chunk * 16 < link.tiles; chunk += WAVES)
-      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(link.sums + chunk * 256 + lane * 4),
-                                       (void __attribute__((address_space(3)))*)(raw_sums + chunk * 256), 16, 0, 0);
-
   auto request = [&](int group, int stage) {
     unsigned char* to = mine + (size_t)stage * STAGE_BYTES;
     const int k = group * G * STEP;
@@ -522,13 +410,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
   for (int s = 0; s < NT; ++s)
 #pragma unroll
     for (int t = 0; t < MT; ++t) *(f32x4*)(partial + ((wave * TILES + s * MT + t) * 64 + lane) * 4) = acc[s][t];
-  if (LINK == SCALED) {  // every wave adds up its share of the tiles' sums
-    float squares = 0.f;
-    for (int tile = wave * 4 + g; tile < link.tiles; tile += WAVES * 4) squares += raw_sums[tile * 16 + r];
-    squares += __shfl_xor(squares, 16, WAVE);
-    squares += __shfl_xor(squares, 32, WAVE);
-    if (g == 0) shares[wave * 16 + r] = squares;
-  }
   __syncthreads();
   for (int tile = wave; tile < TILES; tile += WAVES) {
     const int s = tile / MT;
@@ -544,15 +425,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
 #pragma unroll
       for (int i = 0; i < 4; ++i) total[i] += load_as_float(bias, bias_is_float, min(n_first + i, N - 1));
     }
-    if (LINK == SCALED) {
-      const float factor = row_factor<WAVES * 16, 16>(link, shares, m);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) total[i] *= factor;  // (such a product has no bias)
-    }
     if (LINK == INTO_NORM) {
       store_into_norm(link, columns, total, m, n_first, N);
-    } else if (GATED == 3) {
-      store_with_tail(out, tail, m, n_first, N, total);
     } else if (GATED) {
       TO* dst = out + (size_t)m * (N / 2) + n_first / 2;
 #pragma unroll
@@ -573,75 +447,366 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const bf16_t* _
 
 template <int WAVES, int NT, int MT, int G, typename TO, int GATED, int LINK = NO_LINK>
 static int launch_stream(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N,
-                         int K, int splits, hipStream_t stream, Tail tail = {}, Link link = {}) {
+                         int K, int splits, hipStream_t stream, Link link = {}) {
   const size_t stages = (size_t)WAVES * STREAM_STAGES * (NT + MT) * G * STREAM_CHUNK;
   const size_t sums = (size_t)WAVES * NT * MT * 64 * 4 * sizeof(float);
-  const size_t lds = (stages > sums ? stages : sums) + (LINK == SCALED ? ((size_t)(link.tiles + 15) / 16 * 256 + WAVES * 16) * sizeof(float) : 0);
+  const size_t lds = stages > sums ? stages : sums;
   if (lds > 64 * 1024) {
     static bool asked = false;
     if (!asked) {
       if (hipFuncSetAttribute((const void*)gemm_stream_kernel<WAVES, NT, MT, G, TO, GATED, LINK>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, LINK == SCALED ? 80 * 1024 : (int)lds) != hipSuccess)
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return ERR_BAD_ARGUMENT;
       asked = true;
     }
   }
   hipLaunchKernelGGL((gemm_stream_kernel<WAVES, NT, MT, G, TO, GATED, LINK>), dim3((N + 16 * NT - 1) / (16 * NT), splits),
                      dim3(WAVES * 64), lds, stream, (const bf16_t*)x, (const bf16_t*)w, bias, bias_is_float, (TO*)out, M,
-                     N, K, K / splits, tail, link);
+                     N, K, K / splits, link);
   return LAUNCH_STATUS();
 }
 
-// two tiles a wave for a middling number of weight rows over a K that is not cut (the qkv products of the
-// 7B and 32B sizes: 11.6 -> 10.6 and 20.0 -> 17.5 us); with K cut over workgroups one tile is as good or
-// better (the 32B sizes' o in two parts: 13.5 us against 16.9)
-static bool streams_by_two(long tiles, int K, int splits) {
-  return splits == 1 && tiles >= 256 && tiles < 1024 && tiles * K >= 1000000L;
-}
-
-// One tile a wave in groups of four steps, or two tiles in groups of two.  Measured at 8 rows against
-// gemm_skinny / gemm_pair, in a captured chain over different weights: 1.5B sizes qkv 4.9 -> 4.1 us,
-// gate/up 15.7 -> 13.0, down 9.5 -> 8.7, o 4.8 -> 3.4; 7B sizes qkv 13.8 -> 10.6 (two tiles), o 9.8 ->
-// 7.9, gate/up 54.7 -> 52.1; 32B sizes qkv 20.9 -> 16.3 (two tiles).  Where a wave walks a long K
-// for four tiles that share its x (the down projections and the 32B sizes' gate/up) gemm_pair's
-// registers stay ahead, and the caller keeps it there.
-// M <= 16, K / splits a multiple of 128.
+// 17 to 64 rows: two or four tiles of x.  nt, g: 0 = by the sizes, else as asked (measurements).  K / splits a multiple of 128.
 template <typename TO, int GATED>
 static int pick_stream(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
-                       int splits, hipStream_t stream, int nt = 0, int g = 0, Tail tail = {}) {
+                       int splits, hipStream_t stream, int nt = 0, int g = 0) {
   const long tiles = (N + 15) / 16;
-  if (M > 16) {
-    // 17 to 64 rows: two or four tiles of x.  nt, g: 0 = by the sizes, else as asked (measurements)
-    if (nt == 0) nt = tiles * splits >= 2048 ? 2 : 1;
-    if (g == 0) g = 1;
+  if (nt == 0) nt = tiles * splits >= 2048 ? 2 : 1;
+  if (g == 0) g = 1;
 #define ROWS_CASE(NT_, MT_, G_)                                                                              \
   if (nt == NT_ && g == G_ && M <= 16 * MT_)                                                                 \
-    return launch_stream<4, NT_, MT_, G_, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, tail);
-    ROWS_CASE(1, 2, 1)
-    ROWS_CASE(2, 2, 1)
-    ROWS_CASE(1, 2, 2)
-    ROWS_CASE(2, 2, 2)
-    ROWS_CASE(1, 4, 1)
-    ROWS_CASE(2, 4, 1)
-    ROWS_CASE(1, 4, 2)
-    ROWS_CASE(2, 4, 2)
-    ROWS_CASE(4, 2, 1)
-    ROWS_CASE(4, 4, 1)
+    return launch_stream<4, NT_, MT_, G_, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream);
+  ROWS_CASE(1, 2, 1)
+  ROWS_CASE(2, 2, 1)
+  ROWS_CASE(1, 2, 2)
+  ROWS_CASE(2, 2, 2)
+  ROWS_CASE(1, 4, 1)
+  ROWS_CASE(2, 4, 1)
+  ROWS_CASE(1, 4, 2)
+  ROWS_CASE(2, 4, 2)
+  ROWS_CASE(4, 2, 1)
+  ROWS_CASE(4, 4, 1)
 #undef ROWS_CASE
-    return ERR_BAD_ARGUMENT;
-  }
-  if (streams_by_two(tiles, K, splits))
-    return launch_stream<4, 2, 1, 2, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, tail);
-  return launch_stream<4, 1, 1, 4, TO, GATED>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, tail);
+  return ERR_BAD_ARGUMENT;
 }
 
-// The same product as llmserve_gemm_skinny, always through gemm_stream (tests and measurements); up to 64 rows.
+// ---------------------------------------------------------------------------- up to 16 rows
+// gemm_flow: up to 16 rows of x, the shape of decoding, which is a stream of the weight from memory and nothing else.  What the rate of that stream hangs on,
+// measured: whole cache lines (a load of a wave is 8 rows x 128 bytes; 16 rows x 64 bytes ask for every line twice), past the caches (non-temporal: a
+// line that is read once pushes nothing out, 8-20 % of a large weight's time), and the same number of rows for every CU.  So a workgroup takes
+// `rows_each` weight rows, any even number up to 8 NH, rather than a tile of sixteen (flow_shape), and its four waves take the units of 64 k in
+// turn.  Lane L asks for piece (L % 8) ^ (L / 8) of row L / 8 of every eight rows, straight into LDS, where lane (r, g) reads its operand of step s, piece
+// 4 s + g of row r, from slot 8 r + ((4 s + g) ^ (r % 8)): the eight lanes that LDS serves together hit all banks.  Every wave has STAGES units of its
+// own under way (XH eights of rows of x, then NH of weights), asks for a pair of eights anew as soon as it is read, and waits for its own loads alone, counted;
+// the waves' sums meet in LDS at the end, added up in wave order: a row's bits depend on sizes, not on what the other rows hold.
+// Rows past the last are asked for as the last one: their results are dropped.
+// Us in a captured chain over different weights at 1 / 8 / 16 rows, the kernels before (one and two tiles of sixteen rows through LDS, four through registers, the ring)
+// -> this one: 1.5B sizes gate/up 11.6 / 12.9 / 13.8 -> 10.5 / 10.5 / 11.3, down 6.8 / 7.4 / 7.9 -> 6.2 / 6.3 / 6.7, head 75 / 90 / 99 -> 72 / 73 / 79 (6.4 TB/s
+// at 8 rows); 7B sizes gate/up 46.6 / 49.1 / 49.0 -> 42.4 / 42.8 / 44.6, down 26.0 / 24.9 / 25.3 -> 21.7 / 21.9 / 23.1, qkv 9.9 / 10.4 / 11.3 -> 8.3 / 8.1 / 8.5.
+#define FLOW_UNIT 64    // k a unit
+#define FLOW_ROWS 40    // rows a workgroup at most
+#define FLOW_SCALED_K 8192  // a row's sums of 16 columns, which a workgroup's threads hold in registers
+
+template <typename F, int... I>
+__device__ __forceinline__ void flow_each(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+// Units that a wave has under way for so many eights of weight rows and of x, so that a workgroup has 32 KB of weights or more, and its LDS.
+constexpr int flow_stages(int eights, int x_eights) { return eights == 1 ? 6 : eights == 2 ? 4 : eights == 3 && x_eights == 1 ? 3 : 2; }
+constexpr size_t flow_lds_bytes(int eights, int x_eights) {
+  const size_t stages = (size_t)4 * flow_stages(eights, x_eights) * (eights + x_eights) * 1024 + eights % 2 * 1024;  // (what an odd number reads beyond its own)
+  const size_t sums = (size_t)4 * ((eights + 1) / 2) * 1024 + 4 * 16 * sizeof(float);
+  return stages > sums ? stages : sums;
+}
+
+// TEMPORAL: the weight is small, and may have been brought into the caches.  SUMS (SCALED): pieces of four sums a thread holds.
+template <int NH, int XH, bool TEMPORAL, typename TO, int GATED, int LINK, int SUMS>
+__global__ __launch_bounds__(256) void gemm_flow_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                        const void* __restrict__ bias, int bias_is_float, TO* __restrict__ out, int M, int N,
+                                                        int K, int k_split, int rows_each, Tail tail, Link link) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char flow_lds[];
+  constexpr int STAGES = flow_stages(NH, XH), WAVES = 4, NT = (NH + 1) / 2, LOADS = NH + XH, STAGE_BYTES = LOADS * 1024;
+  static_assert(STAGES * LOADS <= 63, "a wave's loads are counted in vmcnt");
+  static_assert(NT <= WAVES, "a wave finishes one tile");
+  static_assert(LINK != INTO_NORM || (NH == 2 && sizeof(TO) == 4), "whole tiles of sixteen columns");
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r = lane & 15, g = lane >> 4;
+  const int n_begin = (int)blockIdx.x * rows_each, n_end = min(N, n_begin + rows_each);
+  const int k_first = (int)blockIdx.y * k_split;
+  const int row8 = lane >> 3, piece = (lane & 7) ^ row8;
+  const bf16_t* w_src[NH];
+#pragma unroll
+  for (int h = 0; h < NH; ++h) w_src[h] = w + (size_t)min(n_begin + h * 8 + row8, n_end - 1) * K + k_first + piece * 8;
+  const bf16_t* x_src[XH];
+#pragma unroll
+  for (int h = 0; h < XH; ++h) x_src[h] = x + (size_t)min(h * 8 + row8, M - 1) * K + k_first + piece * 8;
+  unsigned char* mine = flow_lds + (size_t)wave * STAGES * STAGE_BYTES;
+  const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)mine;
+  // (an odd number of eights: the upper half of the last tile reads what lies behind, and its results are dropped)
+  const unsigned read_w = base + XH * 1024 + (unsigned)r * 128, read_x = base + (unsigned)(XH == 1 ? r & 7 : r) * 128;
+  const unsigned at[2] = {(unsigned)(g ^ (r & 7)) * 16, (unsigned)((g + 4) ^ (r & 7)) * 16};
+
+  const int n_first = n_begin + wave * 16 + g * 4;  // of the four columns that this lane finishes, where wave < NT
+  float bias_here[4] = {0.f, 0.f, 0.f, 0.f};
+  if (bias && blockIdx.y == 0 && wave < NT) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bias_here[i] = load_as_float(bias, bias_is_float, min(n_first + i, N - 1));
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // so that the counts below count the stream alone
+  LinkedColumns columns;  // (ahead of the stream, whose first wait covers them, as the sums of squares)
+  if (LINK == INTO_NORM) columns = linked_columns(link, r, n_begin + g * 4, M, N);
+  f32x4 sums[SUMS > 0 ? SUMS : 1];
+  if (LINK == SCALED) {
+#pragma unroll
+    for (int c = 0; c < SUMS; ++c) sums[c] = *(const f32x4*)(link.sums + min((int)threadIdx.x + c * 256, link.tiles * 4 - 1) * 4);
+    asm volatile("" ::: "memory");
+  }
+
+  auto ask = [&](const bf16_t* from, int unit, int stage, int slot) {
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(from + unit * FLOW_UNIT),
+                                     (void __attribute__((address_space(3)))*)(mine + stage * STAGE_BYTES + slot * 1024), 16, 0, 0);
+  };
+  auto ask_weight = [&](int h, int unit, int stage) {
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(w_src[h] + unit * FLOW_UNIT),
+                                     (void __attribute__((address_space(3)))*)(mine + stage * STAGE_BYTES + (XH + h) * 1024), 16, 0, TEMPORAL ? 0 : 2);
+  };
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const int units = k_split / FLOW_UNIT;
+  const int count = (units - wave + WAVES - 1) / WAVES;  // this wave's: wave, wave + 4, ...
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s)
+    if (s < count) {
+#pragma unroll
+      for (int h = 0; h < XH; ++h) ask(x_src[h], wave + s * WAVES, s, h);
+#pragma unroll
+      for (int h = 0; h < NH; ++h) ask_weight(h, wave + s * WAVES, s);
+    }
+  // This wave's unit i, in `stage`; AFTER units behind it are under way, and with AGAIN unit i + STAGES is asked for into the same places.
+  auto one_unit = [&](int i, int stage, auto after, auto again) {
+    constexpr int AFTER = decltype(after)::value;
+    constexpr bool AGAIN = decltype(again)::value;
+    const unsigned here = (unsigned)stage * STAGE_BYTES;
+    const int next = wave + (i + STAGES) * WAVES;
+    bf16x8 b[2];
+    flow_each([&](auto tile) {
+      constexpr int t = decltype(tile)::value, EIGHTS = 2 * t + 2 <= NH ? 2 : 1;
+      // asked for behind this tile's: the unit's other eights, the units behind, what has been asked for anew
+      stream_wait_loads<NH - 2 * t - EIGHTS + AFTER * LOADS + (AGAIN && t > 0 ? XH + 2 * t : 0)>();
+      bf16x8 a[2];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        if (t == 0) stream_read<0>(b[s], read_x + here + at[s]);
+        stream_read<2048 * t>(a[s], read_w + here + at[s]);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {  // used only after the wait
+        asm volatile("" : "+v"(a[s]));
+        if (t == 0) asm volatile("" : "+v"(b[s]));
+      }
+      if (AGAIN) {
+        if (t == 0) {
+#pragma unroll
+          for (int h = 0; h < XH; ++h) ask(x_src[h], next, stage, h);
+        }
+#pragma unroll
+        for (int h = 0; h < EIGHTS; ++h) ask_weight(2 * t + h, next, stage);
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], b[s], acc[t], 0, 0, 0);
+    }, std::make_integer_sequence<int, NT>{});
+  };
+  int i = 0, stage = 0;
+  for (; i + STAGES < count; ++i) {
+    one_unit(i, stage, std::integral_constant<int, STAGES - 1>{}, std::true_type{});
+    stage = stage + 1 == STAGES ? 0 : stage + 1;
+  }
+  flow_each([&](auto done) {  // the last STAGES units (or as many as there are)
+    constexpr int AFTER = STAGES - 1 - decltype(done)::value;
+    if (count - i != AFTER + 1) return;
+    one_unit(i, stage, std::integral_constant<int, AFTER>{}, std::false_type{});
+    ++i;
+    stage = stage + 1 == STAGES ? 0 : stage + 1;
+  }, std::make_integer_sequence<int, STAGES>{});
+
+  __syncthreads();  // every wave is done with its stages: LDS is free for the waves' sums
+  float* partial = (float*)flow_lds;  // [WAVES][NT][64 lanes][4]
+  float* shares = partial + WAVES * NT * 256;  // [WAVES][16 rows]
+#pragma unroll
+  for (int t = 0; t < NT; ++t) *(f32x4*)(partial + ((wave * NT + t) * 64 + lane) * 4) = acc[t];
+  if (LINK == SCALED) {  // piece threadIdx.x + 256 c holds rows 4 (threadIdx.x % 4) .. + 3 of a tile of columns
+    f32x4 squares = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < SUMS; ++c)
+      if ((int)threadIdx.x + c * 256 < link.tiles * 4) squares += sums[c];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int offset = 4; offset < WAVE; offset *= 2) squares[i] += __shfl_xor(squares[i], offset, WAVE);
+    }
+    if (lane < 4) *(f32x4*)(shares + wave * 16 + lane * 4) = squares;
+  }
+  __syncthreads();
+  if (wave >= NT) return;
+  f32x4 total = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int v = 0; v < WAVES; ++v) total += *(const f32x4*)(partial + ((v * NT + wave) * 64 + lane) * 4);
+  const int m = r;
+  if (m >= M) return;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) total[i] += bias_here[i];
+  if (LINK == SCALED) {
+    const float squares = ((shares[m] + shares[16 + m]) + shares[32 + m]) + shares[48 + m];
+    const float factor = rsqrtf(squares * link.inverse_width + link.eps);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) total[i] *= factor;  // (such a product has no bias)
+  }
+  if (LINK == INTO_NORM) {
+    store_into_norm(link, columns, total, m, n_first, N);
+  } else if (GATED == 3) {
+    store_with_tail(out, tail, m, n_first, n_end, total);
+  } else if (GATED) {
+    TO* dst = out + (size_t)m * (N / 2) + n_first / 2;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (n_first + 2 * i + 1 < n_end) {
+        const float gate = total[2 * i], up = total[2 * i + 1];
+        dst[i] = from_float<TO>(gate_value<GATED>(gate) * up);
+      }
+    }
+  } else {
+    TO* dst = out + ((size_t)blockIdx.y * M + m) * N + n_first;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (n_first + i < n_end) dst[i] = from_float<TO>(total[i]);
+  }
+}
+
+template <int NH, int XH, bool TEMPORAL, typename TO, int GATED, int LINK, int SUMS>
+static int launch_flow(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K, int splits, int rows_each,
+                       hipStream_t stream, Tail tail, Link link) {
+  constexpr size_t lds = flow_lds_bytes(NH, XH);
+  if (lds > 64 * 1024) {
+    static bool asked = false;
+    if (!asked) {
+      if (hipFuncSetAttribute((const void*)gemm_flow_kernel<NH, XH, TEMPORAL, TO, GATED, LINK, SUMS>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+        return ERR_BAD_ARGUMENT;
+      asked = true;
+    }
+  }
+  hipLaunchKernelGGL((gemm_flow_kernel<NH, XH, TEMPORAL, TO, GATED, LINK, SUMS>), dim3((N + rows_each - 1) / rows_each, splits), dim3(256), lds,
+                     stream, (const bf16_t*)x, (const bf16_t*)w, bias, bias_is_float, (TO*)out, M, N, K, K / splits, rows_each, tail, link);
+  return LAUNCH_STATUS();
+}
+
+// A weight of up to 8 MB is read as any other memory: the kernel before may have brought it into the caches, and a model of such weights may
+// live in them.  (Its rows give every CU a workgroup with no more than 16 rows.)
+static bool flow_temporal(int N, int K) { return (long)N * K <= (1L << 22); }
+
+// The rows a workgroup takes: what a CU has to bring, weight rows and rows of x, is least.  Workgroups that share a CU's LDS run
+// at once, so that CUs get whole numbers of them; of more, CUs take the next as they finish.  Gate/up of the 1.5B sizes (17,920 rows) at 8 rows of x: 18 rows each, four
+// a CU at most, 10.7 us; 24, three, 10.5; 32, three, 11.8; 40, two, 10.6.  The head (151,936 rows) at 8 and 16 rows of x: 24 rows
+// each 78.5 and 93.8 us, 32 72.6 and 79.0, 40 75.5 and 83.8 (hence the 1.06 and 1.12).
+struct FlowShape {
+  int rows_each;
+  double load;  // rows of K / splits that a CU brings
+};
+static FlowShape flow_shape(int M, int N, int K, int splits) {
+  FlowShape best = {0, 0.0};
+  const int most = flow_temporal(N, K) ? 16 : FLOW_ROWS;
+  for (int rows = 8; rows <= most; rows += 2) {
+    const int eights = (rows + 7) / 8;
+    const long workgroups = (long)((N + rows - 1) / rows) * splits;
+    const int held = (int)(160 * 1024 / flow_lds_bytes(eights, M <= 8 ? 1 : 2));
+    const double each = rows + 0.3 * (8 * eights - rows) + M + 2.0;
+    double load = workgroups <= 256L * held ? (double)((workgroups + 255) / 256) * each : (workgroups / 256.0 + 0.5) * each;
+    if (eights == 5) load *= M <= 8 ? 1.06 : 1.12;
+    if (best.rows_each == 0 || load < best.load) best = {rows, load};
+  }
+  return best;
+}
+
+template <typename TO, int GATED, int LINK, int SUMS>
+static int pick_flow(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K, int splits,
+                     hipStream_t stream, Tail tail = {}, Link link = {}) {
+  const int rows_each = flow_shape(M, N, K, splits).rows_each, eights = (rows_each + 7) / 8;
+#define FLOW_CASE(NH_, TEMPORAL_)                                                                                                             \
+  if (eights == NH_)                                                                                                                          \
+    return M <= 8 ? launch_flow<NH_, 1, TEMPORAL_, TO, GATED, LINK, SUMS>(x, w, bias, bias_is_float, out, M, N, K, splits,  \
+                                                                                            rows_each, stream, tail, link)                    \
+                  : launch_flow<NH_, 2, TEMPORAL_, TO, GATED, LINK, SUMS>(x, w, bias, bias_is_float, out, M, N, K, splits,  \
+                                                                                            rows_each, stream, tail, link);
+  if (flow_temporal(N, K)) {
+    FLOW_CASE(1, true)
+    FLOW_CASE(2, true)
+  } else {
+    FLOW_CASE(1, false)
+    FLOW_CASE(2, false)
+    FLOW_CASE(3, false)
+    FLOW_CASE(4, false)
+    FLOW_CASE(5, false)
+  }
+#undef FLOW_CASE
+  return ERR_BAD_ARGUMENT;
+}
+
+// K % 128 == 0, N % 16 == 0: tiles of sixteen columns, whose squares the reader adds up
+static int pick_flow_into_norm(const void* x, const void* w, const void* bias, int bias_is_float, int M, int N, int K, hipStream_t stream, Link link) {
+#define NORM_CASE(XH_, TEMPORAL_) \
+  launch_flow<2, XH_, TEMPORAL_, float, 0, INTO_NORM, 0>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, 16, stream, Tail{}, link)
+  if (flow_temporal(N, K)) return M <= 8 ? NORM_CASE(1, true) : NORM_CASE(2, true);
+  return M <= 8 ? NORM_CASE(1, false) : NORM_CASE(2, false);
+#undef NORM_CASE
+}
+
+static int pick_flow_scaled(const void* rows, const void* w, void* out, int M, int N, int K, hipStream_t stream, Link link) {
+  if (K <= 2048) return pick_flow<bf16_t, 1, SCALED, 2>(rows, w, nullptr, 0, out, M, N, K, 1, stream, {}, link);
+  if (K <= 4096) return pick_flow<bf16_t, 1, SCALED, 4>(rows, w, nullptr, 0, out, M, N, K, 1, stream, {}, link);
+  return pick_flow<bf16_t, 1, SCALED, 8>(rows, w, nullptr, 0, out, M, N, K, 1, stream, {}, link);
+}
+
+// Loads into LDS bring 16 bytes from a multiple of 16.
+static bool flow_takes(const void* x, const void* w, int out_is_float, int gated, int M, int N, int K, int splits) {
+  return M > 0 && M <= 16 && K % splits == 0 && (K / splits) % FLOW_UNIT == 0 && !(gated && out_is_float) && (((size_t)x | (size_t)w) & 15) == 0;
+}
+static int flow_entry(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int out_is_float, int gated, int M, int N, int K,
+                      int splits, hipStream_t stream, Tail tail) {
+  if (gated == 3) return pick_flow<bf16_t, 3, NO_LINK, 0>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, tail);
+  if (gated == 2) return pick_flow<bf16_t, 2, NO_LINK, 0>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
+  if (gated) return pick_flow<bf16_t, 1, NO_LINK, 0>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
+  return out_is_float ? pick_flow<float, 0, NO_LINK, 0>(x, w, bias, bias_is_float, out, M, N, K, splits, stream)
+                      : pick_flow<bf16_t, 0, NO_LINK, 0>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
+}
+
+// The weight rows that a workgroup of the product of M <= 16 rows takes (splits parts of K, a multiple of 64 each), for who brings them ahead.
+extern "C" int llmserve_gemm_flow_rows(int M, int N, int K, int splits) { return flow_shape(M, N, K, splits).rows_each; }
+
+// Into how many parts of K such a product is best cut when its float32 result may stay in parts, 1 to 8: by what a CU brings, and 0.12 us a part for
+// writing and adding it up (a CU brings 26 bytes a ns).  A part has two units a wave or more.
+extern "C" int llmserve_gemm_flow_parts(int M, int N, int K) {
+  const int units = K / FLOW_UNIT;
+  int best = 1;
+  double least = 0.0;
+  for (int splits = 1; splits <= 8; ++splits) {
+    if (K % FLOW_UNIT || units % splits || (splits > 1 && units / splits < 8)) continue;
+    const double us = flow_shape(M, N, K, splits).load * (K / splits) * 2.0 / 26e3 + 0.12 * splits;
+    if (splits == 1 || us < least) least = us, best = splits;
+  }
+  return best;
+}
+
+// The same product as llmserve_gemm_skinny, always through gemm_flow or, beyond 16 rows, gemm_stream (tests and measurements); up to 64 rows.
 static int stream_entry(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int out_is_float,
                         int gated, int M, int N, int K, int splits, hipStream_t stream, int nt, int g) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 64 || K <= 0 || splits < 1 || K % splits || (K / splits) % (STEP * GROUP) || (gated && N % 2) || gated > 1)
     return ERR_BAD_ARGUMENT;
   if (splits > 1 && (gated || !out_is_float)) return ERR_BAD_ARGUMENT;
+  if (M <= 16) return flow_takes(x, w, out_is_float, gated, M, N, K, splits) ? flow_entry(x, w, bias, bias_is_float, out, out_is_float, gated, M, N, K, splits, stream, Tail{}) : ERR_BAD_ARGUMENT;
   if (gated)
     return out_is_float ? pick_stream<float, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, nt, g)
                         : pick_stream<bf16_t, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, nt, g);
@@ -820,9 +985,9 @@ extern "C" int llmserve_gemm_into_norm(const void* x, const void* split_x, const
   const Ahead next = {(const unsigned char*)ahead, (unsigned)stripe, (unsigned)stripes};
   const Link link{hidden, weight, weight_is_float, (bf16_t*)rows, sums, sums_stride(M), N / 16, 0.f, 0.f};
   if (split_x) return pick_merged<INTO_NORM>(split_x, split_ml, splits, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, link, helpers, next);
-  if (M <= 16) return launch_stream<4, 1, 1, 4, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
-  if (M <= 32) return launch_stream<4, 1, 2, 2, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
-  return launch_stream<4, 1, 4, 1, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link);
+  if (M <= 16) return pick_flow_into_norm(x, w, bias, bias_is_float, M, N, K, stream, link);
+  if (M <= 32) return launch_stream<4, 1, 2, 2, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, link);
+  return launch_stream<4, 1, 4, 1, float, 0, INTO_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, link);
 }
 
 // ---------------------------------------------------------------------------- 16 < M <= 64
@@ -1308,34 +1473,16 @@ extern "C" int llmserve_gemm_ring(const void* x, const void* w, const void* bias
                       : pick_ring<bf16_t, false>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, nt);
 }
 
-// Weight tiles a wave of the kernels for up to 16 rows shares its x between: several where a wave has many groups of K to
-// walk (or x is all 16 rows) and enough workgroups are left (measured at the 1.5B and 7B sizes).
-static int skinny_share(int M, int N, int K, int splits) {
-  const int per_wave = K / splits / (STEP * GROUP) / 4;
-  const long tiles = (N + 15) / 16;
-  const long by_four = (tiles + 3) / 4 * splits, by_two = (tiles + 1) / 2 * splits;  // workgroups
-  return (per_wave >= 8 && by_four >= 128 && (M > 2 || tiles <= 1024)) || (tiles >= 4096 && M >= 4) ? 4
-         : (per_wave >= 4 || M > 8 || (tiles >= 4096 && M >= 4)) && by_two * 4 >= TARGET_WAVES ? 2
-                                                                                                 : 1;
-}
-// Whether such a product goes through LDS (gemm_stream): with one or two tiles, unless many rows of x meet a long walk over K.
-static bool skinny_streams(int M, int N, int K, int splits) {
-  const int share = skinny_share(M, N, K, splits);
-  return share != 4 && !(share == 2 && M > 8 && K / splits / (STEP * GROUP) / 4 >= 4);
-}
-
-#define SCALED_STREAM_K 3840  // the sums of so long a row leave room for two workgroups of gemm_stream in a CU's LDS
-
 // silu(gate) * up, bfloat16 [M, N / 2], of rows that a product into a norm has left (`rows` [M, K], `sums` as there, in a
 // buffer of whole KB): every result
-// times rsqrt(sum of the row's sums / K + eps).  tiles 0: through gemm_stream, M <= 16; else through gemm_ring with so many
-// weight tiles a workgroup.
+// times rsqrt(sum of the row's sums / K + eps).  Up to 16 rows and FLOW_SCALED_K through gemm_flow, whatever `tiles` is; else through
+// gemm_ring with so many weight tiles a workgroup.
 extern "C" int llmserve_gemm_scaled(const void* rows, float* sums, float eps, const void* w, void* out, int tiles, int M, int N, int K,
                                     hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 64 || K <= 0 || K % (STEP * GROUP) || N % 2 || (tiles == 0 && (M > 16 || K > SCALED_STREAM_K))) return ERR_BAD_ARGUMENT;
+  if (M > 64 || K <= 0 || K % (STEP * GROUP) || N % 2 || (tiles == 0 && (M > 16 || K > FLOW_SCALED_K))) return ERR_BAD_ARGUMENT;
   const Link link{nullptr, nullptr, 0, nullptr, sums, sums_stride(M), K / 16, 1.f / (float)K, eps};
-  if (tiles == 0) return launch_stream<4, 1, 1, 4, bf16_t, 1, SCALED>(rows, w, nullptr, 0, out, M, N, K, 1, stream, {}, link);
+  if (M <= 16 && K <= FLOW_SCALED_K) return pick_flow_scaled(rows, w, out, M, N, K, stream, link);
 #define SCALED_CASE(NT_, KSTEPS_)                                                                                      \
   if (tiles == NT_)                                                                                                    \
     return M <= 32 ? launch_ring<NT_, 2, KSTEPS_, 4, bf16_t, true, SCALED>(rows, w, nullptr, 0, out, M, N, K, 1, stream, link) \
@@ -1352,9 +1499,9 @@ extern "C" int llmserve_gemm_scaled(const void* rows, float* sums, float eps, co
   return ERR_BAD_ARGUMENT;
 }
 
-// Whether the kernel and shape of llmserve_gemm_scaled with tiles 0 is what a gated product of these sizes takes without the norm.
+// Whether llmserve_gemm_scaled takes these sizes with tiles 0.
 extern "C" int llmserve_gemm_scaled_streams(int M, int N, int K) {
-  return M > 0 && M <= 16 && K > 0 && K <= SCALED_STREAM_K && K % (STEP * GROUP) == 0 && skinny_streams(M, N, K, 1) && !streams_by_two((N + 15) / 16, K, 1);
+  return M > 0 && M <= 16 && K > 0 && K <= FLOW_SCALED_K && K % (STEP * GROUP) == 0;
 }
 
 // x, w bfloat16; out bfloat16 or float32.  Needs 1 <= M <= 64, K a multiple of 32, and with
@@ -1364,35 +1511,8 @@ extern "C" int llmserve_gemm_scaled_streams(int M, int N, int K) {
 static int skinny_entry(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int out_is_float, int gated,
                         int M, int N, int K, int splits, hipStream_t stream, Tail tail) {
   if (splits > 1 && (gated || !out_is_float || K % splits || (K / splits) % STEP)) return ERR_BAD_ARGUMENT;
-  if (M <= 16 && (K / splits) % (STEP * GROUP) == 0) {
-    const int share = skinny_share(M, N, K, splits);
-    if (skinny_streams(M, N, K, splits)) {
-      if (gated == 3) return pick_stream<bf16_t, 3>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, 0, 0, tail);
-      if (gated == 2)
-        return out_is_float ? pick_stream<float, 2>(x, w, bias, bias_is_float, out, M, N, K, 1, stream)
-                            : pick_stream<bf16_t, 2>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
-      if (gated)
-        return out_is_float ? pick_stream<float, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream)
-                            : pick_stream<bf16_t, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
-      return out_is_float ? pick_stream<float, false>(x, w, bias, bias_is_float, out, M, N, K, splits, stream)
-                          : pick_stream<bf16_t, false>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
-    }
-#define PAIR_CASE(NT)                                                                                              \
-  if (share == NT) {                                                                                               \
-    if (gated == 3) return launch_pair<NT, bf16_t, 3>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, tail);   \
-    if (gated == 2)                                                                                                \
-      return out_is_float ? launch_pair<NT, float, 2>(x, w, bias, bias_is_float, out, M, N, K, 1, stream)          \
-                          : launch_pair<NT, bf16_t, 2>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);        \
-    if (gated)                                                                                                     \
-      return out_is_float ? launch_pair<NT, float, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream)       \
-                          : launch_pair<NT, bf16_t, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);     \
-    return out_is_float ? launch_pair<NT, float, false>(x, w, bias, bias_is_float, out, M, N, K, splits, stream)   \
-                        : launch_pair<NT, bf16_t, false>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);      \
-  }
-    PAIR_CASE(2)
-    PAIR_CASE(4)
-#undef PAIR_CASE
-  }
+  if (flow_takes(x, w, out_is_float, gated, M, N, K, splits))
+    return flow_entry(x, w, bias, bias_is_float, out, out_is_float, gated, M, N, K, splits, stream, tail);
   if (M > 16 && !gated && K % splits == 0 && (K / splits) % (STEP * GROUP) == 0 && (long)N * K <= (1L << 22)) {
     // A small weight at 17 to 64 rows: two or four tiles of x beside one weight tile a workgroup, through
     // LDS.  In a captured chain over different weights, the 1.5B sizes' qkv and o: 4.8 and 4.0 us at 17

@@ -21,6 +21,7 @@ from .build import _say, load_module
 _PAIRINGS = {"none": 0, "adjacent": 1, "half": 2}
 # gate activations of a gated product (csrc/elementwise.hip: gate_activation); the products' fused epilogues know silu alone
 _ACTIVATIONS = {"silu": 0, "gelu": 1, "gelu_tanh": 2, "relu": 3, "limited_swish": 4, "squared_relu": 5}  # (limited_swish is a function of gate and up both, with a limit)
+_FLOW_SCALED = 8192  # columns of scaled rows that the gated product of up to 16 of them takes (csrc/gemm_bf16.hip: FLOW_SCALED_K)
 _GATED_RESULT = 16  # added to an activation's code: the experts' product gates its own result
 
 
@@ -78,6 +79,8 @@ _SIGNATURES = {
     "llmserve_gemm_into_norm": "pppippippippiiiipiip",
     "llmserve_gemm_scaled": "ppfppiiiip",
     "llmserve_gemm_scaled_streams": "iii",
+    "llmserve_gemm_flow_rows": "iiii",
+    "llmserve_gemm_flow_parts": "iii",
     "llmserve_gemm_rotated": "pppipiipiiipppip",
     "llmserve_gemm_blocks": "pppipiiiiiip",
     "llmserve_gemm_blocks_parts": "iii",
@@ -339,9 +342,9 @@ class HipKernels:
         index = self.device.index if self.device.index is not None else torch.cuda.current_device()
         return tensor.device.type == "cuda" and tensor.device.index == index
 
-    def _ahead(self, weights: Any, busy: int, up_to: int, tiles: int = 1) -> tuple:
+    def _ahead(self, weights: Any, busy: int, up_to: int, rows_each: int = 16) -> tuple:
         """What a kernel of `busy` workgroups is told of the weight that the next product reads (csrc/common.h: Ahead), which takes
-        `tiles` tiles of 16 weight rows a workgroup: (workgroups that bring it into the caches, its address, bytes a run, runs).  As
+        `rows_each` weight rows a workgroup: (workgroups that bring it into the caches, its address, bytes a run, runs).  As
         many workgroups as fill the CUs that the others leave idle; the weight's first `up_to` bytes, (0, ...) for nothing.  Nothing of what
         another library prepared, and of weights that lie elsewhere (a library derived from this one may bring them when it multiplies)."""
         if (
@@ -349,8 +352,8 @@ class HipKernels:
             or not _in_pieces(weights.weight) or weights.in_features % 8 or busy >= 256
         ):
             return 0, None, 0, 0
-        stripe = 32 * tiles * weights.in_features
-        stripes = min(weights.out_features // (16 * tiles), up_to // stripe)
+        stripe = 2 * rows_each * weights.in_features
+        stripes = min(weights.out_features // rows_each, up_to // stripe)
         return (256 - busy, _pointer(weights.weight), stripe, stripes) if stripes > 0 else (0, None, 0, 0)
 
     # The bytes of a weight that are brought ahead of a step of up to 64 single tokens: whole weights that a chiplet's L2 (4 MB) holds an eighth of beside
@@ -368,10 +371,14 @@ class HipKernels:
     # and 16 lose 3 %.
     _MERGING_AHEAD_EACH = 192 << 10
 
-    def _whole_ahead(self, weights: Any, rows: int, busy: int) -> tuple:
+    def _whole_ahead(self, weights: Any, rows: int, busy: int, plain: bool = False) -> tuple:
+        """`plain`: the next product is one by itself (its result whole, no norm or key splits about it)."""
         if not isinstance(weights, LinearWeights) or rows > 64 or weights.weight.numel() * weights.weight.element_size() > self._WHOLE_AHEAD:
             return 0, None, 0, 0
-        return self._ahead(weights, busy, self._WHOLE_AHEAD)
+        rows_each = 16
+        if plain and self._gemm_bf16 is not None and self._flows("skinny", rows, weights.in_features):
+            rows_each = self._gemm_bf16.llmserve_gemm_flow_rows(rows, weights.out_features, weights.in_features, 1)
+        return self._ahead(weights, busy, self._WHOLE_AHEAD, rows_each)
 
     def add_rms_norm(self, hidden, delta, weight, eps: float, ahead=None) -> torch.Tensor:
         rows, width = hidden.shape
@@ -381,7 +388,7 @@ class HipKernels:
         parts = 1 if delta is None or delta.ndim == 2 else delta.shape[0]  # [parts, rows, width]: partial sums
         status = self._elementwise.llmserve_add_rms_norm(
             _pointer(hidden), _pointer(delta), parts, _pointer(weight), _is_float(weight), _pointer(out),
-            _is_float(out), rows, width, eps, *self._whole_ahead(ahead, rows, rows), self._stream,
+            _is_float(out), rows, width, eps, *self._whole_ahead(ahead, rows, rows, plain=True), self._stream,
         )
         _check(status, "add_rms_norm")
         return out
@@ -511,7 +518,7 @@ class HipKernels:
         return GatedLinearWeights(LinearWeights(both, None), gate.shape[0], activation, float(limit or 0.0))
 
     def _streaming(self, x: torch.Tensor, weights: LinearWeights, gated: bool = False, may_split: bool = False) -> str | None:
-        """Which MFMA kernel takes this product: "skinny" (up to 16 rows of x, weights streamed),
+        """Which MFMA kernel takes this product: "skinny" (up to 16 rows of x, weights streamed; see `_flows`),
         "ring" (17 to 64 rows of a middling weight, both operands through a ring of stages in LDS),
         "medium" (up to 64, x shared through LDS), "tiled" (any number, both operands through LDS),
         or None (the BLAS library, or the generic kernel)."""
@@ -520,14 +527,8 @@ class HipKernels:
         rows, inner = x.shape[0], weights.in_features
         size = weights.out_features * inner
         if self.ring_products and rows <= 16 and inner % 128 == 0 and size > (1 << 22):
-            # A few rows of a large weight do as well or better on the kernel written for 17 to 64 rows where its
-            # workgroups make one round: from 4 rows on where the weight is very large or is large and its K may be
-            # cut over workgroups, from 12 rows on the middling ones.  Us at 4 / 8 / 16 rows in a captured chain over
-            # different weights: 7B sizes down 27.5 / 28.0 / 29.6 -> 26.2 / 26.3 / 26.5, gate/up 46.9 / 49.9 / 58.9 -> 47.6 /
-            # 47.7 / 47.9; 32B sizes gate/up 108.3 / 110.9 / 120.2 -> 100.8 / 101.1 / 101.3; the 1.5B sizes' down projection
-            # and gate/up at 16 rows 10.3 and 15.8 -> 8.2 and 14.0 (at 8 rows 8.8 -> 8.1 alone, but the step it is in 1.434 ->
-            # 1.441 ms); a single row, 7B qkv at 8 rows (11.8 -> 12.8) and what would take several rounds (the 1.5B sizes'
-            # head 89.6 / 94.2 -> 93.3 / 94.9, the 32B sizes' down projection 52.5 -> 54.2) stay.
+            # (Products of up to 16 rows with a K of whole units go to `_flows`' kernel, whichever name they get here; what the name still says is
+            # how rows that a norm has left scaled, longer than that kernel's, are read.)
             heavy = size > (1 << 26) or (may_split and size > (1 << 24))
             if rows >= (self.ring_rows_from if heavy else max(12, self.ring_rows_from)) and (heavy or may_split or size > (1 << 24)):
                 if self._ring_shape(rows, weights.out_features, inner, may_split)[2] == 1:
@@ -571,6 +572,12 @@ class HipKernels:
         if rows > 64 and inner % 32 == 0:
             return "tiled"
         return None
+
+    @staticmethod
+    def _flows(streaming: str | None, rows: int, in_features: int) -> bool:
+        """Whether a product of up to 16 rows goes to the kernel that streams whole cache lines (csrc/gemm_bf16.hip: gemm_flow), whichever of
+        the others `_streaming` names: those take a K that is no multiple of 64, and more rows."""
+        return streaming in ("skinny", "ring") and rows <= 16 and in_features % 64 == 0
 
     @staticmethod
     def _tiled_ahead(rows: int, out_features: int, in_features: int, gated: bool, may_split: bool) -> bool:
@@ -766,6 +773,10 @@ class HipKernels:
         bias_is_float = _is_float(bias) if bias is not None else 0
         if streaming is not None:
             splits = 1
+            if self._flows(streaming, rows, inner):
+                if partial and out_dtype == torch.float32:
+                    splits = self._gemm_bf16.llmserve_gemm_flow_parts(rows, weights.out_features, inner)
+                streaming = "flow"
             if streaming == "ring":
                 tiles, splits, _ = self._ring_shape(rows, weights.out_features, inner, partial and out_dtype == torch.float32)
                 out = self._empty((rows, weights.out_features) if splits == 1 else (splits, rows, weights.out_features), out_dtype or self.dtype)
@@ -775,7 +786,7 @@ class HipKernels:
                 )
                 _check(status, "linear")
                 return out
-            if partial and out_dtype == torch.float32:
+            if streaming != "flow" and partial and out_dtype == torch.float32:
                 if streaming == "tiled":
                     splits = self._gemm_blocks.llmserve_gemm_blocks_parts(rows, weights.out_features, inner)
                 elif streaming == "medium":
@@ -792,7 +803,7 @@ class HipKernels:
                     _is_float(out), 0, rows, weights.out_features, inner, splits, self._stream,
                 )
             else:
-                entry = self._gemm_bf16.llmserve_gemm_skinny if streaming == "skinny" else self._gemm_bf16.llmserve_gemm_medium
+                entry = self._gemm_bf16.llmserve_gemm_skinny if streaming in ("skinny", "flow") else self._gemm_bf16.llmserve_gemm_medium
                 status = entry(
                     _pointer(x), _pointer(weights.weight), _pointer(bias), bias_is_float, _pointer(out),
                     _is_float(out), 0, rows, weights.out_features, inner, splits, self._stream,
@@ -876,11 +887,14 @@ class HipKernels:
         sums = self._empty((-(-width // 256) * 16, stride), torch.float32)  # (whole KB: the reader brings them to LDS by the KB)
         split_x, split_ml, splits = split if split is not None else (None, None, 0)
         bias = project.bias
+        ahead = 0, None, 0, 0
+        if split is not None:
+            each = self._gemm_bf16.llmserve_gemm_flow_rows(rows, 2 * reader.width, width, 1) if width <= _FLOW_SCALED else 16 * tiles
+            ahead = self._ahead(reader.both, width // 16, self._MERGING_AHEAD_EACH * max(0, 256 - width // 16), each)
         status = self._gemm_bf16.llmserve_gemm_into_norm(
             _pointer(x) if split is None else None, _pointer(split_x), _pointer(split_ml), splits, _pointer(project.weight), _pointer(bias),
             _is_float(bias) if bias is not None else 0, _pointer(hidden), _pointer(into.weight), _is_float(into.weight), _pointer(scaled),
-            _pointer(sums), rows, width, project.in_features, *self._ahead(reader.both if split is not None else None, width // 16, self._MERGING_AHEAD_EACH * max(0, 256 - width // 16), max(1, tiles)),
-            self._stream,
+            _pointer(sums), rows, width, project.in_features, *ahead, self._stream,
         )
         _check(status, "linear into a norm")
         return ScaledRows(scaled, sums, into.eps, reader, tiles)
@@ -905,7 +919,7 @@ class HipKernels:
         if (
             weights.activation == "relu"
             and self.dtype == torch.bfloat16
-            and self._streaming(x, weights.both, gated=True) == "skinny"
+            and ((route := self._streaming(x, weights.both, gated=True)) == "skinny" or self._flows(route, *x.shape))
         ):
             # the kernels for a few rows (a decode step) apply relu in their epilogue too: one launch less a layer
             status = self._gemm_bf16.llmserve_gemm_skinny(
@@ -930,6 +944,8 @@ class HipKernels:
             _check(status, "gated_linear")
             return out
         streaming = self._streaming(x, weights.both, gated=True)
+        if self._flows(streaming, *x.shape):
+            streaming = "skinny"
         if streaming == "ring":
             tiles, _, _ = self._ring_shape(x.shape[0], 2 * weights.width, x.shape[1], False)
             status = self._gemm_bf16.llmserve_gemm_ring(
@@ -1631,9 +1647,8 @@ class HipKernels:
         if out.dtype != self.dtype or out.shape[0] != x.shape[0] or not 0 <= out_first <= out.shape[1] - width:
             raise KernelError("activated_linear: the rows to write are of the run dtype, one a token, and wide enough")
         streaming = self._streaming(x, weights)
-        if activation == "squared_relu" and (streaming == "skinny" or (streaming == "ring" and x.shape[0] <= 8)):
+        if activation == "squared_relu" and (streaming == "skinny" or self._flows(streaming, *x.shape)):
             # the kernels for a few rows (a decode step) apply it in their epilogue and store the two runs of columns apart
-            # (up to 8 rows the ring is not far enough ahead of them on a large weight to pay a launch more)
             rows = self._empty((x.shape[0], first), self.dtype) if first else None
             status = self._gemm_bf16.llmserve_gemm_skinny_tail(
                 _pointer(x), _pointer(weights.weight), _pointer(weights.bias), _is_float(weights.bias) if weights.bias is not None else 0,
