@@ -1164,20 +1164,39 @@ extern "C" int llmserve_gemm_medium(const void* x, const void* w, const void* bi
 // gemm_ring: the product for 17 to 128 rows of x (and few of a large weight), bound by how fast the weights come from memory.  A
 // workgroup of four waves owns NT tiles of 16 weight rows over its whole K range and MT tiles of x; both
 // go through a ring of DEPTH stages of KSTEPS * 32 k in LDS that the waves share, filled straight from
-// memory (global_load_lds_dwordx4, a chunk of 16 rows x 32 k in lane order, laid out and swizzled as in
-// gemm_stream) DEPTH - 1 stages ahead of the one being multiplied: what a CU has under way is then that
+// memory (global_load_lds_dwordx4, a chunk of eight rows x 64 k in lane order, laid out and swizzled as in
+// gemm_flow; the weights, which one workgroup alone reads, past the caches: with chunks of 16 rows x 32 k, half a cache line of
+// each, and through them, steps of 64 rows took 2 % longer, prompts of 77 tokens 1.8) DEPTH - 1 stages ahead of the one being multiplied: what a CU has under way is then that
 // many stages of weights whatever the compiler does with the registers, and a weight row is read from memory
 // once for all rows of x.  The waves divide a stage's chunks between them; one barrier a stage says that
 // everyone's loads have landed and that the stage before may be filled again.  A wave multiplies one tile of x
 // (two, with six or eight tiles of x: up to 96 and 128 rows) with its share of the weight tiles, so no sums meet at the end.
-__device__ __forceinline__ void ring_load(const bf16_t* from, unsigned to) {
+__device__ __forceinline__ void ring_load(const bf16_t* from, unsigned to, bool once) {
   // (M0 names the place in LDS; it is put back, the compiler keeps other things there)
   unsigned kept;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(kept)
-               : "s"(to), "v"(from)
-               : "memory");
+  if (once)
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off nt\n\ts_mov_b32 m0, %0"
+                 : "=&s"(kept)
+                 : "s"(to), "v"(from)
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(kept)
+                 : "s"(to), "v"(from)
+                 : "memory");
 }
+// What a lane reads of a tile of KSTEPS * 32 k, step by step: the tile's chunks are its upper and lower eight rows of 64 k, then of the next 64.
+template <int I, int COUNT>
+struct RingReads {
+  static __device__ __forceinline__ void run(bf16x8* operands, unsigned even, unsigned odd) {
+    stream_read<I / 2 * 2 * STREAM_CHUNK>(operands[I], I % 2 ? odd : even);
+    RingReads<I + 1, COUNT>::run(operands, even, odd);
+  }
+};
+template <int COUNT>
+struct RingReads<COUNT, COUNT> {
+  static __device__ __forceinline__ void run(bf16x8*, unsigned, unsigned) {}
+};
 
 // waits until at most `younger` stages' loads of this wave (PER_WAVE each) are under way; younger <= MOST
 template <int PER_WAVE, int MOST>
@@ -1205,15 +1224,16 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
   constexpr int APART = 4 / KSTEPS;             // tiles between two chunks of a wave
   static_assert(MT == 2 || MT == 4 || MT == 6 || MT == 8, "two, four, six or eight tiles of x");
   static_assert(KSTEPS == 2 || KSTEPS == 4, "stages of 64 or 128 k");
+  static_assert(NT % APART == 0, "a wave's chunks are weights up to one number of them, then x");
   static_assert(NT % WAYS == 0, "the waves divide the weight tiles evenly");
   static_assert(TILES * KSTEPS % 4 == 0, "the waves divide a stage's chunks evenly");
   static_assert((DEPTH - 2) * PER_WAVE <= 63, "the loads under way are counted in vmcnt");
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
   const int k_first = blockIdx.y * k_split;
-  const int load_row = lane >> 2, load_piece = (lane & 3) ^ ((load_row >> 1) & 3);
-  // chunk j of this wave: k-step wave % KSTEPS of tile j * APART + wave / KSTEPS (the weight tiles, then x's)
+  // chunk j of this wave: chunk wave % KSTEPS of tile j * APART + wave / KSTEPS (the weight tiles, then x's): eight rows of 64 k
   const int my_step = wave % KSTEPS, my_first = wave / KSTEPS;
+  const int load_row = my_step % 2 * 8 + (lane >> 3), load_piece = (lane & 7) ^ (lane >> 3);
   const bf16_t* src[PER_WAVE];  // this lane's piece of each, in the first stage
 #pragma unroll
   for (int j = 0; j < PER_WAVE; ++j) {
@@ -1221,14 +1241,14 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
     // rows of x beyond M are read as row M - 1: their columns of the result are dropped at the end
     const bf16_t* row = tile < NT ? w + (size_t)min(((int)blockIdx.x * NT + tile) * 16 + load_row, N - 1) * K
                                   : x + (size_t)min((tile - NT) * 16 + load_row, M - 1) * K;
-    src[j] = row + k_first + my_step * STEP + load_piece * 8;
+    src[j] = row + k_first + my_step / 2 * (2 * STEP) + load_piece * 8;
   }
   const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)ring;
   // the wave's first tile of x, of weights (of six tiles of x the fourth wave multiplies what the third does: the same sums to the same places)
   const int x_tile = min((wave % XGROUPS) * XPW, MT - XPW), first_tile = wave / XGROUPS;
-  const unsigned read_at = base + (unsigned)(4 * r + (g ^ ((r >> 1) & 3))) * 16;
-  const unsigned read_w = read_at + (unsigned)first_tile * KSTEPS * STREAM_CHUNK;
-  const unsigned read_x = read_at + (unsigned)(NT + x_tile) * KSTEPS * STREAM_CHUNK;
+  const unsigned even = base + (unsigned)(8 * r + (g ^ (r & 7))) * 16, to_odd = (unsigned)(((4 + g) ^ (r & 7)) - (g ^ (r & 7))) * 16;
+  const unsigned read_w = even + (unsigned)first_tile * KSTEPS * STREAM_CHUNK;
+  const unsigned read_x = even + (unsigned)(NT + x_tile) * KSTEPS * STREAM_CHUNK;
 
   // the bias of the outputs this lane will finish: all asked for at once, of either type
   float bias_here[MINE][4];
@@ -1256,7 +1276,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
     const unsigned to = base + (unsigned)(stage % DEPTH) * STAGE_BYTES + (unsigned)(my_first * KSTEPS + my_step) * STREAM_CHUNK;
 #pragma unroll
     for (int j = 0; j < PER_WAVE; ++j)
-      ring_load(src[j] + (size_t)stage * (KSTEPS * STEP), to + (unsigned)(j * APART * KSTEPS) * STREAM_CHUNK);
+      ring_load(src[j] + (size_t)stage * (KSTEPS * STEP), to + (unsigned)(j * APART * KSTEPS) * STREAM_CHUNK, j * APART < NT);
   };
   f32x4 acc[MINE][XPW];
 #pragma unroll
@@ -1275,9 +1295,15 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const bf16_t* __restrict
     const unsigned slot = (unsigned)(stage % DEPTH) * STAGE_BYTES;
     bf16x8 from_x[XPW][KSTEPS], from_w[MINE][KSTEPS];
 #pragma unroll
-    for (int j = 0; j < XPW; ++j) StreamReads<0, KSTEPS>::run(from_x[j], read_x + slot + (unsigned)(j * KSTEPS) * STREAM_CHUNK);
+    for (int j = 0; j < XPW; ++j) {
+      const unsigned at = read_x + slot + (unsigned)(j * KSTEPS) * STREAM_CHUNK;
+      RingReads<0, KSTEPS>::run(from_x[j], at, at + to_odd);
+    }
 #pragma unroll
-    for (int i = 0; i < MINE; ++i) StreamReads<0, KSTEPS>::run(from_w[i], read_w + slot + (unsigned)(WAYS * i * KSTEPS) * STREAM_CHUNK);
+    for (int i = 0; i < MINE; ++i) {
+      const unsigned at = read_w + slot + (unsigned)(WAYS * i * KSTEPS) * STREAM_CHUNK;
+      RingReads<0, KSTEPS>::run(from_w[i], at, at + to_odd);
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
     for (int j = 0; j < XPW; ++j)
