@@ -139,12 +139,9 @@ __device__ __forceinline__ void store_four(bf16_t* dst, float a, float b, float 
 }
 
 template <typename TO, int PIECES>
-__global__ __launch_bounds__(1024) void add_rms_norm_vector_kernel(float* __restrict__ hidden,
-                                                                   const float* __restrict__ delta, int parts,
-                                                                   size_t part_stride,
-                                                                   const void* __restrict__ weight,
-                                                                   int weight_is_float, TO* __restrict__ out,
-                                                                   int width, float eps, int rows, Ahead ahead) {
+__global__ __launch_bounds__(1024) void add_rms_norm_vector_kernel(float* __restrict__ hidden, const float* __restrict__ delta,
+                                                                   const void* __restrict__ weight, size_t part_stride, int parts, int width, int rows,
+                                                                   int weight_is_float, TO* __restrict__ out, float eps, Ahead ahead) {
   __shared__ float shared[17];
   if ((int)blockIdx.x >= rows) {  // (a few rows wait for their trips to memory; the path to it is free for the next product's weight)
     bring_ahead(ahead, blockIdx.x, rows, gridDim.x);
@@ -205,14 +202,14 @@ static void launch_add_rms_norm_vector(float* hidden, const float* delta, int pa
   const int pieces = quads <= 1024 ? 1 : quads <= 2048 ? 2 : 4;
   const int threads = ((quads + pieces - 1) / pieces + WAVE - 1) / WAVE * WAVE;
   if (pieces == 1)
-    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 1>), dim3(rows + helpers), dim3(threads), 0, stream, hidden, delta, parts,
-                       part_stride, weight, weight_is_float, out, width, eps, rows, ahead);
+    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 1>), dim3(rows + helpers), dim3(threads), 0, stream, hidden, delta, weight,
+                       part_stride, parts, width, rows, weight_is_float, out, eps, ahead);
   else if (pieces == 2)
-    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 2>), dim3(rows + helpers), dim3(threads), 0, stream, hidden, delta, parts,
-                       part_stride, weight, weight_is_float, out, width, eps, rows, ahead);
+    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 2>), dim3(rows + helpers), dim3(threads), 0, stream, hidden, delta, weight,
+                       part_stride, parts, width, rows, weight_is_float, out, eps, ahead);
   else
-    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 4>), dim3(rows + helpers), dim3(threads), 0, stream, hidden, delta, parts,
-                       part_stride, weight, weight_is_float, out, width, eps, rows, ahead);
+    hipLaunchKernelGGL((add_rms_norm_vector_kernel<TO, 4>), dim3(rows + helpers), dim3(threads), 0, stream, hidden, delta, weight,
+                       part_stride, parts, width, rows, weight_is_float, out, eps, ahead);
 }
 
 extern "C" int llmserve_add_rms_norm(float* hidden, const float* delta, int parts, const void* weight,

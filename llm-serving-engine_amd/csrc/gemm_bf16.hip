@@ -522,9 +522,9 @@ constexpr size_t flow_lds_bytes(int eights, int x_eights) {
 
 // TEMPORAL: the weight is small, and may have been brought into the caches.  SUMS (SCALED): pieces of four sums a thread holds.
 template <int NH, int XH, bool TEMPORAL, typename TO, int GATED, int LINK, int SUMS>
-__global__ __launch_bounds__(256) void gemm_flow_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-                                                        const void* __restrict__ bias, int bias_is_float, TO* __restrict__ out, int M, int N,
-                                                        int K, int k_split, int rows_each, Tail tail, Link link) {
+__global__ __launch_bounds__(256) void gemm_flow_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int M, int N, int K, int k_split,
+                                                        int rows_each, int bias_is_float, const void* __restrict__ bias, TO* __restrict__ out, Tail tail,
+                                                        Link link) {
   extern __shared__ __attribute__((aligned(16))) unsigned char flow_lds[];
   constexpr int STAGES = flow_stages(NH, XH), WAVES = 4, NT = (NH + 1) / 2, LOADS = NH + XH, STAGE_BYTES = LOADS * 1024;
   static_assert(STAGES * LOADS <= 63, "a wave's loads are counted in vmcnt");
@@ -547,22 +547,6 @@ __global__ __launch_bounds__(256) void gemm_flow_kernel(const bf16_t* __restrict
   const unsigned read_w = base + XH * 1024 + (unsigned)r * 128, read_x = base + (unsigned)(XH == 1 ? r & 7 : r) * 128;
   const unsigned at[2] = {(unsigned)(g ^ (r & 7)) * 16, (unsigned)((g + 4) ^ (r & 7)) * 16};
 
-  const int n_first = n_begin + wave * 16 + g * 4;  // of the four columns that this lane finishes, where wave < NT
-  float bias_here[4] = {0.f, 0.f, 0.f, 0.f};
-  if (bias && blockIdx.y == 0 && wave < NT) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) bias_here[i] = load_as_float(bias, bias_is_float, min(n_first + i, N - 1));
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // so that the counts below count the stream alone
-  LinkedColumns columns;  // (ahead of the stream, whose first wait covers them, as the sums of squares)
-  if (LINK == INTO_NORM) columns = linked_columns(link, r, n_begin + g * 4, M, N);
-  f32x4 sums[SUMS > 0 ? SUMS : 1];
-  if (LINK == SCALED) {
-#pragma unroll
-    for (int c = 0; c < SUMS; ++c) sums[c] = *(const f32x4*)(link.sums + min((int)threadIdx.x + c * 256, link.tiles * 4 - 1) * 4);
-    asm volatile("" ::: "memory");
-  }
-
   auto ask = [&](const bf16_t* from, int unit, int stage, int slot) {
     __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(from + unit * FLOW_UNIT),
                                      (void __attribute__((address_space(3)))*)(mine + stage * STAGE_BYTES + slot * 1024), 16, 0, 0);
@@ -584,6 +568,31 @@ __global__ __launch_bounds__(256) void gemm_flow_kernel(const bf16_t* __restrict
 #pragma unroll
       for (int h = 0; h < NH; ++h) ask_weight(h, wave + s * WAVES, s);
     }
+  // What the end needs is asked for behind the first units, which therefore wait for no argument beyond those that come with the wave.  (The counts
+  // below do not know of these loads, and so wait for as many of the stream's more, until they have come.)
+  const int n_first = n_begin + wave * 16 + g * 4;  // of the four columns that this lane finishes, where wave < NT
+  // (the bias without a branch, at whose end its loads would be waited for, and the stream with them: as 16-bit halves, a float32 two and a bfloat16 the
+  // upper one alone; where there is none the same loads read the weights' start)
+  unsigned short bias_low[4], bias_high[4];
+  const bool with_bias = LINK != SCALED && bias && blockIdx.y == 0;
+  if (LINK != SCALED) {
+    const unsigned short* source = with_bias ? (const unsigned short*)bias : (const unsigned short*)w;
+    const int halves = with_bias && bias_is_float ? 2 : 1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int at = min(n_first + i, N - 1) * halves;
+      bias_low[i] = source[at];
+      bias_high[i] = source[at + halves - 1];
+    }
+  }
+  LinkedColumns columns;
+  if (LINK == INTO_NORM) columns = linked_columns(link, r, n_begin + g * 4, M, N);
+  f32x4 sums[SUMS > 0 ? SUMS : 1];
+  if (LINK == SCALED) {
+#pragma unroll
+    for (int c = 0; c < SUMS; ++c) sums[c] = *(const f32x4*)(link.sums + min((int)threadIdx.x + c * 256, link.tiles * 4 - 1) * 4);
+  }
+  asm volatile("" ::: "memory");
   // This wave's unit i, in `stage`; AFTER units behind it are under way, and with AGAIN unit i + STAGES is asked for into the same places.
   auto one_unit = [&](int i, int stage, auto after, auto again) {
     constexpr int AFTER = decltype(after)::value;
@@ -656,8 +665,10 @@ __global__ __launch_bounds__(256) void gemm_flow_kernel(const bf16_t* __restrict
   for (int v = 0; v < WAVES; ++v) total += *(const f32x4*)(partial + ((v * NT + wave) * 64 + lane) * 4);
   const int m = r;
   if (m >= M) return;
+  if (with_bias) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) total[i] += bias_here[i];
+    for (int i = 0; i < 4; ++i) total[i] += __uint_as_float((unsigned)bias_high[i] << 16 | (bias_is_float ? (unsigned)bias_low[i] : 0u));
+  }
   if (LINK == SCALED) {
     const float squares = ((shares[m] + shares[16 + m]) + shares[32 + m]) + shares[48 + m];
     const float factor = rsqrtf(squares * link.inverse_width + link.eps);
@@ -699,7 +710,7 @@ static int launch_flow(const void* x, const void* w, const void* bias, int bias_
     }
   }
   hipLaunchKernelGGL((gemm_flow_kernel<NH, XH, TEMPORAL, TO, GATED, LINK, SUMS>), dim3((N + rows_each - 1) / rows_each, splits), dim3(256), lds,
-                     stream, (const bf16_t*)x, (const bf16_t*)w, bias, bias_is_float, (TO*)out, M, N, K, K / splits, rows_each, tail, link);
+                     stream, (const bf16_t*)x, (const bf16_t*)w, M, N, K, K / splits, rows_each, bias_is_float, bias, (TO*)out, tail, link);
   return LAUNCH_STATUS();
 }
 
@@ -838,12 +849,10 @@ extern "C" int llmserve_gemm_stream_shaped(const void* x, const void* w, const v
 // trips to memory); here the lanes that load x for the MFMA's B operand merge as they load.  Heads are
 // 128 wide, a group of K (128 k), so a wave's group is one head and its S coefficients are made once.
 template <int WAVES, int S, int LINK>
-__global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* __restrict__ split_x,
-                                                                 const float* __restrict__ split_ml,
-                                                                 const bf16_t* __restrict__ w,
-                                                                 const void* __restrict__ bias, int bias_is_float,
-                                                                 float* __restrict__ out, int M, int N, int K,
-                                                                 int k_split, Link link, int tiles, Ahead ahead) {
+__global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* __restrict__ split_x, const float* __restrict__ split_ml,
+                                                                 const bf16_t* __restrict__ w, int M, int N, int K, int k_split, int tiles,
+                                                                 int bias_is_float, const void* __restrict__ bias, float* __restrict__ out,
+                                                                 Link link, Ahead ahead) {
   extern __shared__ float partial[];  // [WAVES][64 lanes][4]
   if (LINK == INTO_NORM && (int)blockIdx.x >= tiles) {
     bring_ahead(ahead, blockIdx.x, tiles, gridDim.x);
@@ -865,18 +874,17 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* _
     for (int i = 0; i < 4; ++i)
       bias_here[i] = load_as_float(bias, bias_is_float, min((int)blockIdx.x * 16 + g * 4 + i, N - 1));
   }
-  LinkedColumns columns;  // (asked for now and used at the end, by the first wave)
-  if (LINK == INTO_NORM) columns = linked_columns(link, row, (int)blockIdx.x * 16 + g * 4, M, N);
+  LinkedColumns columns;  // (asked for behind the first head's loads, which wait for no argument beyond those that come with the wave, and used at the end, by the first wave)
   const int groups = k_split / (STEP * GROUP);
-  for (int group = wave; group < groups; group += WAVES) {
-    bf16x8 a[GROUP];
+  bf16x8 a[GROUP];
+  float2 ml[S];
+  bf16x8 piece[S][GROUP];
+  auto ask = [&](int group) {
 #pragma unroll
     for (int u = 0; u < GROUP; ++u) a[u] = load8_stream(w_row + (group * GROUP + u) * STEP);
     // split_x is [head][split][piece of 8][16 rows][8]: this lane's piece 4 u + g of row `row`, beside the
     // same piece of the next rows, which the next lanes ask for
     const size_t slot = (size_t)(head_first + group) * S;
-    float2 ml[S];
-    bf16x8 piece[S][GROUP];
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       ml[s] = *(const float2*)(split_ml + ((slot + s) * 16 + row) * 2);
@@ -884,6 +892,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* _
       for (int u = 0; u < GROUP; ++u)
         piece[s][u] = load8(split_x + (((slot + s) * (STEP * GROUP / 8) + u * 4 + g) * 16 + row) * 8);
     }
+    asm volatile("" ::: "memory");  // (asked for here)
+  };
+  ask(min(wave, groups - 1));
+  if (LINK == INTO_NORM) columns = linked_columns(link, row, (int)blockIdx.x * 16 + g * 4, M, N);
+  for (int group = wave; group < groups; group += WAVES) {
+    if (group > wave) ask(group);
     float best = -INFINITY;
 #pragma unroll
     for (int s = 0; s < S; ++s) best = fmaxf(best, ml[s].x);
@@ -936,13 +950,13 @@ static int launch_merged(const void* split_x, const float* split_ml, const void*
   const dim3 grid(tiles + helpers, k_splits);
   if (LINK == INTO_NORM && groups > 8)  // whole sums: a head a wave, or two
     hipLaunchKernelGGL((gemm_merged_kernel<12, S, LINK>), grid, dim3(768), 12 * 64 * 4 * sizeof(float), stream,
-                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link, tiles, ahead);
+                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, M, N, K, K / k_splits, tiles, bias_is_float, bias, out, link, ahead);
   else if (groups <= 4)
     hipLaunchKernelGGL((gemm_merged_kernel<4, S, LINK>), grid, dim3(256), 4 * 64 * 4 * sizeof(float), stream,
-                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link, tiles, ahead);
+                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, M, N, K, K / k_splits, tiles, bias_is_float, bias, out, link, ahead);
   else
     hipLaunchKernelGGL((gemm_merged_kernel<8, S, LINK>), grid, dim3(512), 8 * 64 * 4 * sizeof(float), stream,
-                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, bias, bias_is_float, out, M, N, K, K / k_splits, link, tiles, ahead);
+                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, M, N, K, K / k_splits, tiles, bias_is_float, bias, out, link, ahead);
   return LAUNCH_STATUS();
 }
 
