@@ -35,6 +35,7 @@
 // difference of the two results is normed before it is written.  In a step of single tokens whose maps fit one column tile (up to
 // eight query heads a kv head) both maps are columns of that tile (COLUMN_TILES 1: `heads` counts maps), each with zeros in the other half.
 #include "common.h"
+#include <type_traits>
 
 #ifndef HEAD_DIM
 #error "compile with -DHEAD_DIM=<multiple of 16>"
@@ -86,16 +87,16 @@ __device__ __forceinline__ f32x4 mfma_qk(const QkOperand& a, const QkOperand& b,
 
 // work[tile] = {request index in the step, first token row, first head, columns}: see ColumnMap
 // pairing: 0 none, 1 adjacent pairs (2j, 2j+1), 2 half pairs (j, j + D/2)
-__device__ __forceinline__ void rotate_pair(float& a, float& b, float2 cos_sin) {
-  const float x = a * cos_sin.x - b * cos_sin.y, y = b * cos_sin.x + a * cos_sin.y;
+// (pair j of a head; rounded where the kernels that rotate rows in memory round: common.h, turn_pair)
+__device__ __forceinline__ void rotate_pair(float& a, float& b, float2 cos_sin, bool first_of_eight) {
+  float x, y;
+  turn_pair(a, b, cos_sin.x, cos_sin.y, first_of_eight, &x, &y);
   a = x;
   b = y;
 }
 
-struct FusedDecode {          // what the kernel needs to rotate and store; unused unless FUSED
-  const float2* table;        // [rows][D / 2] (cos, sin) of each token's angles, or null
-  int pairing;
-  const int* slots;           // [rows] page * page_size + offset of each token, negative: store nothing
+struct FusedDecode {          // how the kernel rotates and stores; unused unless FUSED (where its `angle_table` is [rows][D / 2] (cos, sin) of each
+                              // token's angles, or null, and `slots` [rows] page * page_size + offset of each token, negative: store nothing)
   int unmerged;               // key splits are left for the reader to merge: each split's result is divided by its own
                               // sum of weights and stored as bfloat16 where partial_acc points, [rows][heads][splits][D]
   int by_item;                // the splits' partial results are kept by work item (item * tokens_per_tile + token)
@@ -321,25 +322,24 @@ __device__ __forceinline__ void weigh_and_add(Columns<COLUMN_TILES>& columns, St
 
 template <int COLUMN_TILES, bool FUSED, int WAVES, int CHANGED = CHANGED_NOT>
 __global__ __launch_bounds__(WAVES * 64, (COLUMN_TILES > 2 || HEAD_DIM > 192 || WAVES > 4) ? 1 : 2) void attention_tiles_kernel(
-    const bf16_t* __restrict__ qkv, int row_width, bf16_t* __restrict__ out, int out_stride, float* __restrict__ partial_acc,
-    float* __restrict__ partial_ml, bf16_t* __restrict__ keys,
-    bf16_t* __restrict__ values, const int* __restrict__ block_tables, int table_width,
-    const int* __restrict__ positions, const int* __restrict__ work, int heads, int kv_heads, int tokens_per_tile,
-    int page_size, int page_shift, float scale, int window, int splits, FusedDecode fused, ScoreChange change, Finish finish, Ahead ahead) {
+    // (a wave gets its first 56 bytes of arguments in registers, the others by a trip to memory: what the fused form's first loads need comes first)
+    const bf16_t* __restrict__ qkv, const int* __restrict__ positions, const int* __restrict__ block_tables, const float2* __restrict__ angle_table,
+    const int* __restrict__ slots, int row_width, int table_width, unsigned group_and_kv_heads, unsigned splits_and_pairing, bf16_t* __restrict__ keys,
+    bf16_t* __restrict__ values, int page_size, int page_shift, const int* __restrict__ work, bf16_t* __restrict__ out, int out_stride,
+    float* __restrict__ partial_acc, float* __restrict__ partial_ml, int tokens_per_tile, float scale, int window, FusedDecode fused, ScoreChange change,
+    Finish finish, Ahead ahead) {
   static_assert(!FUSED || CHANGED == CHANGED_NOT || CHANGED == CHANGED_EDGES, "the fused decode form leaves the scores as they are");
   constexpr bool PAIRED = CHANGED == CHANGED_MAPS && COLUMN_TILES == 1;  // a head's two maps are neighbouring columns
   constexpr bool TILE_A_MAP = CHANGED == CHANGED_MAPS && COLUMN_TILES == 2;
   extern __shared__ float lds[];  // [WAVES][16 columns][D + 4]
-  if (FUSED)  // a short kernel: fetch all arguments in one go rather than each before its first use
-    asm volatile("" ::"s"(row_width), "s"(table_width), "s"(heads), "s"(kv_heads), "s"(page_size), "s"(page_shift),
-                 "s"(scale), "s"(window), "s"(splits), "s"(fused.pairing));
+  const int splits = splits_and_pairing & 0xffff, pairing = splits_and_pairing >> 16;
   if (FUSED && (int)blockIdx.z >= splits) {  // (behind the workgroups that attend)
     const unsigned plane = gridDim.x * gridDim.y;
     bring_ahead(ahead, blockIdx.z * plane + blockIdx.y * gridDim.x + blockIdx.x, splits * plane, gridDim.z * plane);
     return;
   }
-  const int group = heads / kv_heads;
-  const int kv_head = blockIdx.y % kv_heads, head_tile = blockIdx.y / kv_heads;
+  const int group = group_and_kv_heads >> 16, kv_heads = group_and_kv_heads & 0xffff, heads = group * kv_heads;
+  const int kv_head = group <= 16 ? (int)blockIdx.y : (int)blockIdx.y % kv_heads, head_tile = group <= 16 ? 0 : (int)blockIdx.y / kv_heads;
   const int heads_here = min(group - head_tile * 16, 16);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the same in all lanes: kept in a scalar register
@@ -355,49 +355,31 @@ __global__ __launch_bounds__(WAVES * 64, (COLUMN_TILES > 2 || HEAD_DIM > 192 || 
   const int position0 = positions[row0];
   const int* table = block_tables + (size_t)request * table_width;
   // FUSED: a step of single tokens is short, and what it takes is mostly the time its loads need to come
-  // back.  So everything the start of the kernel needs is asked for here at once, before anything is
-  // used: the pieces of the token's key and value row (one wave will store them; which one depends on the
-  // position, so all ask), the angles, and the pages of this wave's first step, looked up as if that
-  // step lay wholly inside the context and the context's first key were in sight (if not, they are looked up again below:
+  // back.  So everything that no other load decides is asked for here at once: the request's row of the block table (a wave holds up to
+  // 64 TABLE_CHUNKS entries, one a lane and register, and looks its pages up there once it knows the position, where a load would be a trip
+  // to memory more), the queries and their angles, which are rotated while the keys are under way, and the pieces of the token's
+  // key and value row (one wave will store them; which one depends on the position, so all ask).  Of a longer row the registers hold the pages of this wave's
+  // first two steps, as if they lay wholly inside the context and the context's first key were in sight (if not, they are looked up again below:
   // a page behind a mask may have been given back, and its entry in the table is no page).
   constexpr int PAIR_PIECES = (D / 2 + WAVE - 1) / WAVE, VALUE_PIECES = (D + WAVE - 1) / WAVE;
   [[maybe_unused]] bf16_t new_a[PAIR_PIECES], new_b[PAIR_PIECES], new_v[VALUE_PIECES];
   [[maybe_unused]] float2 new_angle[PAIR_PIECES];
   [[maybe_unused]] int new_slot = -1;
-  [[maybe_unused]] int early_k = -1, early_k_hi = -1, early_v = -1;
-  const bool early_pages = FUSED && splits == 1 && (wave * KEYS + KEYS - 1) / page_size < table_width;
   // (heads up to 128 wide leave the registers for a wave's second step to be asked for together with its first)
   constexpr bool TWO_STEPS = (FUSED || (WAVES > 4 && COLUMN_TILES == 1 && CHANGED >= CHANGED_BIAS)) && HEAD_DIM <= 128;
-  [[maybe_unused]] int second_k = -1, second_k_hi = -1, second_v = -1;
-  const bool second_pages = TWO_STEPS && early_pages && ((wave + WAVES) * KEYS + KEYS - 1) / page_size < table_width;
+  constexpr int TABLE_CHUNKS = TWO_STEPS ? 6 : 4;
+  [[maybe_unused]] int table_chunk[TABLE_CHUNKS];
+  const bool whole_row = FUSED && table_width <= WAVE * TABLE_CHUNKS;  // the registers hold the whole of the row
   if (FUSED) {
-    const bf16_t* k_row = qkv + (size_t)row0 * row_width + (size_t)(heads + kv_head) * D;
-    const bf16_t* v_row = k_row + (size_t)kv_heads * D;
-    // (the slot is the same for all lanes; asked for as if it were not, or the compiler waits for it right
-    // here to move it into a scalar register)
-    int no_offset;
-    asm volatile("v_mov_b32 %0, 0" : "=v"(no_offset));
-    new_slot = fused.slots[row0 + no_offset];
+    const int early_key = wave * KEYS + 8 * (c >> 2) + (c & 3), second_key = early_key + WAVES * KEYS;
+    const int early_value = wave * KEYS + 8 * q, second_value = early_value + WAVES * KEYS;
+    if (whole_row) {
 #pragma unroll
-    for (int i = 0; i < PAIR_PIECES; ++i) {
-      const int j = min(lane + i * WAVE, D / 2 - 1);
-      new_a[i] = k_row[fused.pairing == 2 ? j : 2 * j];
-      new_b[i] = k_row[fused.pairing == 2 ? j + D / 2 : 2 * j + 1];
-      if (fused.pairing != 0) new_angle[i] = fused.table[(size_t)row0 * (D / 2) + j];
-    }
+      for (int j = 0; j < TABLE_CHUNKS; ++j) table_chunk[j] = table[min(lane + j * WAVE, table_width - 1)];
+    } else {
+      const int wanted[6] = {early_key, early_key + 4, early_value, second_key, second_key + 4, second_value};
 #pragma unroll
-    for (int i = 0; i < VALUE_PIECES; ++i) new_v[i] = v_row[min(lane + i * WAVE, D - 1)];
-    if (early_pages) {
-      const int key = wave * KEYS + 8 * (c >> 2) + (c & 3);
-      early_k = table[key / page_size];
-      early_k_hi = table[(key + 4) / page_size];
-      early_v = table[(wave * KEYS + 8 * q) / page_size];
-    }
-    if (second_pages) {
-      const int key = (wave + WAVES) * KEYS + 8 * (c >> 2) + (c & 3);
-      second_k = table[key / page_size];
-      second_k_hi = table[(key + 4) / page_size];
-      second_v = table[((wave + WAVES) * KEYS + 8 * q) / page_size];
+      for (int j = 0; j < TABLE_CHUNKS; ++j) table_chunk[j] = table[min(page_shift >= 0 ? wanted[j] >> page_shift : wanted[j] / page_size, table_width - 1)];
     }
   }
   const int last_key = position0 + tokens - 1;
@@ -445,43 +427,63 @@ __global__ __launch_bounds__(WAVES * 64, (COLUMN_TILES > 2 || HEAD_DIM > 192 || 
       if ((q >= 2) != (t == 1)) query[t][middle].v = (bf16x8){};
     }
 #endif
+  }
+  // The queries of a fused step come unrotated.  Their angles: adjacent pairs: lane q rotates pairs 4q .. 4q+3 of every 16; halves: elements
+  // 8q .. 8q+7 of every 32 with their partners D/2 on.  Two angles (16 bytes) a load, without a branch on the pairing.
+  [[maybe_unused]] f32x4 angle[QK_STEPS * 2];
 #if HEAD_DIM % 32 == 0
-    if (FUSED && fused.pairing != 0) {  // the queries come unrotated: rotate them here, in float32
-      const float2* angles = fused.table + (size_t)(row0 + safe) * (D / 2);
-      // All angles are asked for before the first is used, and without a branch on the pairing (the
-      // compiler would otherwise wait for the queries before it asks).  Adjacent pairs: lane q rotates
-      // pairs 4q .. 4q+3 of every 16; halves: elements 8q .. 8q+7 of every 32 with their partners D/2 on.
-      float2 angle[QK_STEPS * 4];
-      const bool adjacent = fused.pairing == 1;
+  if (FUSED) {  // (where nothing is rotated the same loads read the row itself, and their result is dropped)
+    const f32x4* angles = pairing != 0 ? (const f32x4*)(angle_table + (size_t)row0 * (D / 2)) : (const f32x4*)(qkv + (size_t)row0 * row_width);
+    const bool adjacent = pairing == 1;
 #pragma unroll
-      for (int n = 0; n < QK_STEPS * 4; ++n)
-        angle[n] = angles[adjacent ? (n / 4) * 16 + q * 4 + n % 4 : (n / 8) * 32 + q * 8 + n % 8];
-      // the position is wanted in a scalar register from here on: ask now, not at its first use
-      asm volatile("" ::"s"(position0));
-      if (adjacent) {
+    for (int n = 0; n < QK_STEPS * 2; ++n) angle[n] = angles[adjacent ? (n / 2) * 8 + q * 2 + n % 2 : (n / 4) * 16 + q * 4 + n % 4];
+  }
+#endif
+  if (FUSED) {
+    const bf16_t* k_row = qkv + (size_t)row0 * row_width + (size_t)(heads + kv_head) * D;
+    const bf16_t* v_row = k_row + (size_t)kv_heads * D;
+    // (the slot is the same for all lanes; asked for as if it were not, or the compiler waits for it right
+    // here to move it into a scalar register)
+    int no_offset;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(no_offset));
+    new_slot = slots[row0 + no_offset];
 #pragma unroll
-        for (int s = 0; s < QK_STEPS; ++s)
+    for (int i = 0; i < PAIR_PIECES; ++i) {
+      const int j = min(lane + i * WAVE, D / 2 - 1);
+      new_a[i] = k_row[pairing == 2 ? j : 2 * j];
+      new_b[i] = k_row[pairing == 2 ? j + D / 2 : 2 * j + 1];
+      new_angle[i] = pairing != 0 ? angle_table[(size_t)row0 * (D / 2) + j] : make_float2(1.f, 0.f);
+    }
 #pragma unroll
-          for (int pair = 0; pair < 4; ++pair) {
-            float a = (float)query[t][s].v[2 * pair], b = (float)query[t][s].v[2 * pair + 1];
-            rotate_pair(a, b, angle[s * 4 + pair]);
-            query[t][s].v[2 * pair] = (bf16_t)a;
-            query[t][s].v[2 * pair + 1] = (bf16_t)b;
-          }
-      } else {  // the partner of dim d is d + D/2: the same lane, QK_STEPS / 2 steps on (D % 64 == 0)
+    for (int i = 0; i < VALUE_PIECES; ++i) new_v[i] = v_row[min(lane + i * WAVE, D - 1)];
+    asm volatile("" ::: "memory");  // (asked for here)
+  }
+  // (float32, rounded to bfloat16 again; called where the first keys are under way)
+  [[maybe_unused]] auto rotate_queries = [&]() {
+#if HEAD_DIM % 32 == 0
+    if (pairing == 1) {
 #pragma unroll
-        for (int s = 0; s < QK_STEPS / 2; ++s)
+      for (int s = 0; s < QK_STEPS; ++s)
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            float a = (float)query[t][s].v[i], b = (float)query[t][s + QK_STEPS / 2].v[i];
-            rotate_pair(a, b, angle[s * 8 + i]);
-            query[t][s].v[i] = (bf16_t)a;
-            query[t][s + QK_STEPS / 2].v[i] = (bf16_t)b;
-          }
-      }
+        for (int pair = 0; pair < 4; ++pair) {
+          float a = (float)query[0][s].v[2 * pair], b = (float)query[0][s].v[2 * pair + 1];
+          rotate_pair(a, b, make_float2(angle[s * 2 + pair / 2][pair % 2 * 2], angle[s * 2 + pair / 2][pair % 2 * 2 + 1]), pair == 0 && q % 2 == 0);
+          query[0][s].v[2 * pair] = (bf16_t)a;
+          query[0][s].v[2 * pair + 1] = (bf16_t)b;
+        }
+    } else if (pairing == 2) {  // the partner of dim d is d + D/2: the same lane, QK_STEPS / 2 steps on (D % 64 == 0)
+#pragma unroll
+      for (int s = 0; s < QK_STEPS / 2; ++s)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          float a = (float)query[0][s].v[i], b = (float)query[0][s + QK_STEPS / 2].v[i];
+          rotate_pair(a, b, make_float2(angle[s * 4 + i / 2][i % 2 * 2], angle[s * 4 + i / 2][i % 2 * 2 + 1]), i == 0);
+          query[0][s].v[i] = (bf16_t)a;
+          query[0][s + QK_STEPS / 2].v[i] = (bf16_t)b;
+        }
     }
 #endif
-  }
+  };
 
 #pragma unroll
   for (int t = 0; t < COLUMN_TILES; ++t) {
@@ -524,9 +526,9 @@ __global__ __launch_bounds__(WAVES * 64, (COLUMN_TILES > 2 || HEAD_DIM > 192 || 
       const int j = lane + i * WAVE;
       if (j < D / 2) {
         float a = (float)new_a[i], b = (float)new_b[i];
-        if (fused.pairing != 0) rotate_pair(a, b, new_angle[i]);
-        k_at(fused.pairing == 2 ? j : 2 * j) = (bf16_t)a;
-        k_at(fused.pairing == 2 ? j + D / 2 : 2 * j + 1) = (bf16_t)b;
+        if (pairing != 0) rotate_pair(a, b, new_angle[i], j % 8 == 0);
+        k_at(pairing == 2 ? j : 2 * j) = (bf16_t)a;
+        k_at(pairing == 2 ? j + D / 2 : 2 * j + 1) = (bf16_t)b;
       }
     }
 #pragma unroll
@@ -586,7 +588,37 @@ __global__ __launch_bounds__(WAVES * 64, (COLUMN_TILES > 2 || HEAD_DIM > 192 || 
   auto page_index = [&](int key) { return page_shift >= 0 ? key >> page_shift : key / page_size; };
   auto pages_of = [&](int step) {
     const StepKeys at = keys_of(step);
+    if (FUSED && whole_row) {  // (a step's pages are neighbours in the row: of one register or of two that follow one another)
+      const int index[3] = {page_index(at.k), page_index(at.k_hi), page_index(at.v)};
+      const int key0 = step * KEYS;
+      const int low = __builtin_amdgcn_readfirstlane(page_index(min(max(key0, low_limit), last_key)) / WAVE);
+      int here = table_chunk[0], next = table_chunk[TABLE_CHUNKS - 1];
+      if (table_width > WAVE) {
+#pragma unroll
+        for (int j = 0; j < TABLE_CHUNKS; ++j) here = low == j ? table_chunk[j] : here;
+#pragma unroll
+        for (int j = 1; j < TABLE_CHUNKS; ++j) next = low + 1 == j ? table_chunk[j] : next;
+      }
+      int found[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        found[i] = __shfl(here, index[i] % WAVE, WAVE);
+        if (table_width > WAVE) {
+          const int beyond = __shfl(next, index[i] % WAVE, WAVE);
+          found[i] = index[i] / WAVE == low ? found[i] : beyond;
+        }
+      }
+      return StepPages{found[0], found[1], found[2]};
+    }
     return StepPages{table[page_index(at.k)], table[page_index(at.k_hi)], table[page_index(at.v)]};
+  };
+  // the pages of this wave's first or second step, where they have been asked for ahead of the position
+  [[maybe_unused]] auto early_pages_of = [&](int step, auto second) {
+    constexpr int FIRST = decltype(second)::value ? 3 : 0;
+    if constexpr (FUSED && FIRST + 3 <= TABLE_CHUNKS) {
+      if (!whole_row && splits == 1 && first_key == 0 && step < step_last) return StepPages{table_chunk[FIRST], table_chunk[FIRST + 1], table_chunk[FIRST + 2]};
+    }
+    return pages_of(step);
   };
   auto fetch_keys = [&](int step, const StepPages& P, StepLoads& L) {
     const StepKeys at = keys_of(step);
@@ -652,9 +684,13 @@ __global__ __launch_bounds__(WAVES * 64, (COLUMN_TILES > 2 || HEAD_DIM > 192 || 
   if (step_begin + wave < step_end) {
     const int step0 = step_begin + wave;
     StepLoads loads;
-    StepPages pages = early_pages && first_key == 0 && step0 < step_last ? StepPages{early_k, early_k_hi, early_v} : pages_of(step0);
+    StepPages pages = early_pages_of(step0, std::false_type{});
     fetch_keys(step0, pages, loads);
     fetch_values(step0, pages, loads);
+    if constexpr (FUSED && !TWO_STEPS) {
+      asm volatile("" ::: "memory");
+      rotate_queries();
+    }
     if constexpr (TWO_STEPS) {
       // A step of single tokens is a few trips to memory in a row, and a wave has two or three steps to
       // walk: its second step's K and V are asked for together with the first's, into registers of their
@@ -674,10 +710,13 @@ __global__ __launch_bounds__(WAVES * 64, (COLUMN_TILES > 2 || HEAD_DIM > 192 || 
       const int step1 = step0 + WAVES;
       if (step1 < step_end) {
         fetch_bias(step1 * KEYS, bias_odd);
-        const StepPages pages1 =
-            second_pages && first_key == 0 && step1 < step_last ? StepPages{second_k, second_k_hi, second_v} : pages_of(step1);
+        const StepPages pages1 = early_pages_of(step1, std::true_type{});
         fetch_keys(step1, pages1, ahead);
         fetch_values(step1, pages1, ahead);
+      }
+      if constexpr (FUSED) {
+        asm volatile("" ::: "memory");  // (the keys are asked for first)
+        rotate_queries();
       }
       StepPages pages_even = pages, pages_odd = pages;  // of the steps that will fill `loads` and `ahead` again
       if (step0 + 2 * WAVES < step_end) pages_even = pages_of(step0 + 2 * WAVES);
@@ -1284,8 +1323,8 @@ template <int COLUMN_TILES, bool FUSED, int WAVES, int CHANGED = CHANGED_NOT>
 static int launch_tiles(const void* qkv, int row_width, void* out, int out_stride, float* partial_acc, float* partial_ml,
                         void* keys, void* values, const int* block_tables, int table_width,
                         const int* positions, const int* work, int tiles, int heads, int kv_heads,
-                        int tokens_per_tile, int page_size, float scale, int window, int splits, FusedDecode fused,
-                        hipStream_t stream, ScoreChange change, Finish finish, int helpers, Ahead ahead) {
+                        int tokens_per_tile, int page_size, float scale, int window, int splits, const float2* angle_table, int pairing, const int* slots,
+                        FusedDecode fused, hipStream_t stream, ScoreChange change, Finish finish, int helpers, Ahead ahead) {
   const int group = heads / kv_heads;
   const int page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
   const int head_tiles = (group + 15) / 16;
@@ -1301,9 +1340,9 @@ static int launch_tiles(const void* qkv, int row_width, void* out, int out_strid
   }
   const int plane = tiles * kv_heads * head_tiles, planes = FUSED ? splits + (helpers + plane - 1) / plane : splits;
   hipLaunchKernelGGL((attention_tiles_kernel<COLUMN_TILES, FUSED, WAVES, CHANGED>), dim3(tiles, kv_heads * head_tiles, planes),
-                     dim3(WAVES * 64), shared, stream, (const bf16_t*)qkv, row_width, (bf16_t*)out, out_stride, partial_acc,
-                     partial_ml, (bf16_t*)keys, (bf16_t*)values, block_tables, table_width, positions, work,
-                     heads, kv_heads, tokens_per_tile, page_size, page_shift, scale, window, splits, fused, change, finish, ahead);
+                     dim3(WAVES * 64), shared, stream, (const bf16_t*)qkv, positions, block_tables, angle_table, slots, row_width, table_width,
+                     (unsigned)group << 16 | (unsigned)kv_heads, (unsigned)pairing << 16 | (unsigned)splits, (bf16_t*)keys, (bf16_t*)values, page_size, page_shift, work, (bf16_t*)out, out_stride,
+                     partial_acc, partial_ml, tokens_per_tile, scale, window, fused, change, finish, ahead);
   return LAUNCH_STATUS();
 }
 
@@ -1378,6 +1417,7 @@ extern "C" int llmserve_attention_tiles(const void* qkv, int row_width, void* ou
   if (heads % kv_heads || page_size % 8 || splits < 1 || splits > MERGE_SPLITS_MAX || (splits > 1 && (!partial_acc || !partial_ml)))
     return ERR_BAD_ARGUMENT;
   if ((long)kv_heads * page_size * D >= (1L << 31)) return ERR_BAD_ARGUMENT;  // a page's elements are counted in 32 bits
+  if (kv_heads >= 1 << 16 || 2 * heads / kv_heads >= 1 << 16) return ERR_BAD_ARGUMENT;  // (the two go in one argument)
   const int group = heads / kv_heads;
   const int tokens_per_tile = group >= 16 ? 1 : 16 / group;
   const bool unmerged = (fuse & 2) != 0 && splits > 1;  // the splits stay as they are: whoever reads them merges them
@@ -1385,7 +1425,7 @@ extern "C" int llmserve_attention_tiles(const void* qkv, int row_width, void* ou
   const bool by_item = (fuse & 4) != 0 && splits > 1;  // partial results by work item, merged for the items' rows only
   if (by_item && ((fuse & 3) != 0 || column_tiles != 1)) return ERR_BAD_ARGUMENT;
   fuse &= 1;
-  FusedDecode fused = {(const float2*)table, pairing, slots, unmerged ? 1 : 0, by_item ? 1 : 0};
+  FusedDecode fused = {unmerged ? 1 : 0, by_item ? 1 : 0};
   int status;
   if (fuse) {
     if (column_tiles != 1 || tiles != rows || !slots || !llmserve_attention_can_fuse(pairing) || (pairing != 0 && !table))
@@ -1393,7 +1433,7 @@ extern "C" int llmserve_attention_tiles(const void* qkv, int row_width, void* ou
 #define LAUNCH_TILES(COLUMN_TILES, FUSED, WAVES, CHANGED)                                                                 \
   launch_tiles<COLUMN_TILES, FUSED, WAVES, CHANGED>(qkv, row_width, out, out_stride, partial_acc, partial_ml, keys, values, \
                                                     block_tables, table_width, positions, work, tiles, heads, kv_heads,     \
-                                                    tokens_per_tile, page_size, scale, window, splits, fused, stream, change, finish, helpers, next)
+                                                    tokens_per_tile, page_size, scale, window, splits, fuse ? (const float2*)table : nullptr, fuse ? pairing : 0, slots, fused, stream, change, finish, helpers, next)
     status = edges ? LAUNCH_TILES(1, true, FUSED_WAVES, CHANGED_EDGES) : LAUNCH_TILES(1, true, FUSED_WAVES, CHANGED_NOT);
   } else if (finished) {
 #if HEAD_DIM % 32 == 0
