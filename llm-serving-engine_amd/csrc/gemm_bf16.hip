@@ -307,6 +307,19 @@ template <int COUNT>
 struct StreamReads<COUNT, COUNT> {
   static __device__ __forceinline__ void run(bf16x8*, unsigned) {}
 };
+// What a lane reads of a tile of sixteen rows, step by step: the tile's chunks are its upper and lower eight rows of 64 k, then of the next 64.
+template <int I, int COUNT>
+struct RingReads {
+  static __device__ __forceinline__ void run(bf16x8* operands, unsigned even, unsigned odd) {
+    stream_read<I / 2 * 2 * STREAM_CHUNK>(operands[I], I % 2 ? odd : even);
+    RingReads<I + 1, COUNT>::run(operands, even, odd);
+  }
+};
+template <int COUNT>
+struct RingReads<COUNT, COUNT> {
+  static __device__ __forceinline__ void run(bf16x8*, unsigned, unsigned) {}
+};
+
 template <int N>
 __device__ __forceinline__ void stream_wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -846,26 +859,34 @@ extern "C" int llmserve_gemm_stream_shaped(const void* x, const void* w, const v
 // of weights, with each split's maximum m_s (in units of log2) and sum of weights l_s.  The row's true
 // x[head] = sum_s c_s x_s[head] with c_s = l_s 2^(m_s - m) / sum_t l_t 2^(m_t - m), m the largest m_s.
 // A kernel of its own that merges costs a decode step as much as the attention itself (a launch and two
-// trips to memory); here the lanes that load x for the MFMA's B operand merge as they load.  Heads are
+// trips to memory); here every split's x is multiplied as it is, into sums of its own, and those of a head are added up times c_s: lane (r, g) of
+// the result holds row r, whose coefficients it has.  What bounds the kernel is what a CU can ask for: all of x, S times, comes to each of
+// the 96 workgroups (1.5B sizes), and the address unit takes four lanes a cycle, so lanes without a row ask for nothing and the weights come by whole
+// lines, as in gemm_flow (by operands, 16 bytes of four rows to four lanes, and with every lane asking, the first wave had its loads after 3.3 us
+// and the last after 5.5; merging x before the product cost 450 instructions a lane and head besides).  A pass of four steps with 20 MB of the next weight brought
+// beside it: 1 row 4,272 -> 4,141 us, 8 rows 4,525 -> 4,422.  Heads are
 // 128 wide, a group of K (128 k), so a wave's group is one head and its S coefficients are made once.
 template <int WAVES, int S, int LINK>
 __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* __restrict__ split_x, const float* __restrict__ split_ml,
                                                                  const bf16_t* __restrict__ w, int M, int N, int K, int k_split, int tiles,
                                                                  int bias_is_float, const void* __restrict__ bias, float* __restrict__ out,
                                                                  Link link, Ahead ahead) {
-  extern __shared__ float partial[];  // [WAVES][64 lanes][4]
+  extern __shared__ __attribute__((aligned(16))) unsigned char merged_lds[];  // [WAVES][4 KB]: the weights of a wave's head; then [WAVES][64 lanes][4] sums
   if (LINK == INTO_NORM && (int)blockIdx.x >= tiles) {
     bring_ahead(ahead, blockIdx.x, tiles, gridDim.x);
     return;
   }
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
-  const int n = min((int)blockIdx.x * 16 + r, N - 1);
-  const int heads = K / (STEP * GROUP);
   const int head_first = blockIdx.y * (k_split / (STEP * GROUP));
-  const bf16_t* w_row = w + (size_t)n * K + (size_t)head_first * (STEP * GROUP) + g * 8;
-  const bool x_live = r < M;
-  const int row = min(r, M - 1);
+  // (the weights as in gemm_flow: eight rows of 64 k a load, straight into LDS)
+  unsigned char* mine = merged_lds + (size_t)wave * 4096;
+  const bf16_t* w_src[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+    w_src[e] = w + (size_t)min((int)blockIdx.x * 16 + e * 8 + (lane >> 3), N - 1) * K + (size_t)head_first * (STEP * GROUP) + ((lane & 7) ^ (lane >> 3)) * 8;
+  const unsigned even = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)mine + (unsigned)(8 * r + (g ^ (r & 7))) * 16;
+  const unsigned odd = even + (unsigned)(((4 + g) ^ (r & 7)) - (g ^ (r & 7))) * 16;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   const bool with_bias = bias && blockIdx.y == 0;
   float bias_here[4] = {0.f, 0.f, 0.f, 0.f};
@@ -881,23 +902,33 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* _
   bf16x8 piece[S][GROUP];
   auto ask = [&](int group) {
 #pragma unroll
-    for (int u = 0; u < GROUP; ++u) a[u] = load8_stream(w_row + (group * GROUP + u) * STEP);
-    // split_x is [head][split][piece of 8][16 rows][8]: this lane's piece 4 u + g of row `row`, beside the
-    // same piece of the next rows, which the next lanes ask for
+    for (int chunk = 0; chunk < 4; ++chunk)
+      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(w_src[chunk % 2] + group * (STEP * GROUP) + chunk / 2 * 64),
+                                       (void __attribute__((address_space(3)))*)(mine + chunk * 1024), 16, 0, 0);
+    // split_x is [head][split][piece of 8][16 rows][8]: this lane's piece 4 u + g of row r, beside the
+    // same piece of the next rows, which the next lanes ask for.  (Lanes of rows that are not there ask for nothing: the CU's address unit takes a cycle
+    // for every four lanes, and all of x comes through it.)
     const size_t slot = (size_t)(head_first + group) * S;
+    if (r < M) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      ml[s] = *(const float2*)(split_ml + ((slot + s) * 16 + row) * 2);
+      for (int s = 0; s < S; ++s) {
+        ml[s] = *(const float2*)(split_ml + ((slot + s) * 16 + r) * 2);
 #pragma unroll
-      for (int u = 0; u < GROUP; ++u)
-        piece[s][u] = load8(split_x + (((slot + s) * (STEP * GROUP / 8) + u * 4 + g) * 16 + row) * 8);
+        for (int u = 0; u < GROUP; ++u)
+          piece[s][u] = load8(split_x + (((slot + s) * (STEP * GROUP / 8) + u * 4 + g) * 16 + r) * 8);
+      }
     }
     asm volatile("" ::: "memory");  // (asked for here)
   };
   ask(min(wave, groups - 1));
-  if (LINK == INTO_NORM) columns = linked_columns(link, row, (int)blockIdx.x * 16 + g * 4, M, N);
+  if (LINK == INTO_NORM) columns = linked_columns(link, r, (int)blockIdx.x * 16 + g * 4, M, N);
   for (int group = wave; group < groups; group += WAVES) {
     if (group > wave) ask(group);
+    stream_wait_loads<0>();
+    RingReads<0, GROUP>::run(a, even, odd);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int u = 0; u < GROUP; ++u) asm volatile("" : "+v"(a[u]));  // used only after the wait
     float best = -INFINITY;
 #pragma unroll
     for (int s = 0; s < S; ++s) best = fmaxf(best, ml[s].x);
@@ -908,21 +939,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* _
       total += share[s];
     }
     const float inverse = total > 0.f ? 1.f / total : 0.f;
+    f32x4 of_split[S];
 #pragma unroll
-    for (int u = 0; u < GROUP; ++u) {
-      float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < S; ++s) of_split[s] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
-        const float c = share[s] * inverse;
+    for (int u = 0; u < GROUP; ++u)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = fmaf(c, share[s] > 0.f ? (float)piece[s][u][i] : 0.f, x[i]);
-      }
-      bf16x8 b;
+      for (int s = 0; s < S; ++s) of_split[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], piece[s][u], of_split[s], 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) b[i] = x_live ? (bf16_t)x[i] : (bf16_t)0.f;
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b, acc, 0, 0, 0);
+    for (int s = 0; s < S; ++s) {  // (a split that saw no key holds whatever was there, in this row's column alone)
+      const float c = share[s] * inverse;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = share[s] > 0.f ? fmaf(c, of_split[s][i], acc[i]) : acc[i];
     }
   }
+  __syncthreads();  // (every wave has read its weights)
+  float* partial = (float*)merged_lds;
   *(f32x4*)(partial + (wave * 64 + lane) * 4) = acc;
   __syncthreads();
   if (wave > 0) return;
@@ -949,13 +981,13 @@ static int launch_merged(const void* split_x, const float* split_ml, const void*
   const int tiles = (N + 15) / 16;
   const dim3 grid(tiles + helpers, k_splits);
   if (LINK == INTO_NORM && groups > 8)  // whole sums: a head a wave, or two
-    hipLaunchKernelGGL((gemm_merged_kernel<12, S, LINK>), grid, dim3(768), 12 * 64 * 4 * sizeof(float), stream,
+    hipLaunchKernelGGL((gemm_merged_kernel<12, S, LINK>), grid, dim3(768), 12 * 4096, stream,
                        (const bf16_t*)split_x, split_ml, (const bf16_t*)w, M, N, K, K / k_splits, tiles, bias_is_float, bias, out, link, ahead);
   else if (groups <= 4)
-    hipLaunchKernelGGL((gemm_merged_kernel<4, S, LINK>), grid, dim3(256), 4 * 64 * 4 * sizeof(float), stream,
+    hipLaunchKernelGGL((gemm_merged_kernel<4, S, LINK>), grid, dim3(256), 4 * 4096, stream,
                        (const bf16_t*)split_x, split_ml, (const bf16_t*)w, M, N, K, K / k_splits, tiles, bias_is_float, bias, out, link, ahead);
   else
-    hipLaunchKernelGGL((gemm_merged_kernel<8, S, LINK>), grid, dim3(512), 8 * 64 * 4 * sizeof(float), stream,
+    hipLaunchKernelGGL((gemm_merged_kernel<8, S, LINK>), grid, dim3(512), 8 * 4096, stream,
                        (const bf16_t*)split_x, split_ml, (const bf16_t*)w, M, N, K, K / k_splits, tiles, bias_is_float, bias, out, link, ahead);
   return LAUNCH_STATUS();
 }
@@ -1199,19 +1231,6 @@ __device__ __forceinline__ void ring_load(const bf16_t* from, unsigned to, bool 
                  : "s"(to), "v"(from)
                  : "memory");
 }
-// What a lane reads of a tile of KSTEPS * 32 k, step by step: the tile's chunks are its upper and lower eight rows of 64 k, then of the next 64.
-template <int I, int COUNT>
-struct RingReads {
-  static __device__ __forceinline__ void run(bf16x8* operands, unsigned even, unsigned odd) {
-    stream_read<I / 2 * 2 * STREAM_CHUNK>(operands[I], I % 2 ? odd : even);
-    RingReads<I + 1, COUNT>::run(operands, even, odd);
-  }
-};
-template <int COUNT>
-struct RingReads<COUNT, COUNT> {
-  static __device__ __forceinline__ void run(bf16x8*, unsigned, unsigned) {}
-};
-
 // waits until at most `younger` stages' loads of this wave (PER_WAVE each) are under way; younger <= MOST
 template <int PER_WAVE, int MOST>
 __device__ __forceinline__ void ring_wait(int younger) {

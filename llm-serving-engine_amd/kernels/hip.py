@@ -363,13 +363,13 @@ class HipKernels:
     _WHOLE_AHEAD = 8 << 20
 
     # Of gate and up, beside an output projection that merges key splits, whose workgroups wait more than they read: as much as it leaves time for,
-    # for each workgroup that brings (they are what the projection's leave idle).  A layer of a step over 640 keys, us, with nothing and with 8, 16, 24,
-    # 30 and 38 MB, at 1 and 8 rows: width 1,536 of 12 heads, gate and up 52 MB (160 workgroups bring 30 MB) 43.6 42.9 42.7 42.7 42.1 44.2, 47.3 46.8 46.5 46.5 45.9
-    # 47.0; width 2,048 of 16, 66 MB (128: 24) 53.2 51.9 51.6 51.4 51.4 51.7, 58.0 56.6 56.8 56.2 56.3 56.2; width 2,560 of 12, 95 MB (96: 18) 58.5 57.6 57.2
-    # 57.8 58.7 60.5, 65.2 64.4 63.8 64.4 65.0 66.5; width 1,152 of 9, 30 MB (184: all) 36.5 36.1 35.1 35.1 34.7, 39.3 39.0 38.4 38.1 37.7; width 1,024 of 8, 22 MB
-    # 33.4 32.5 32.4 31.5, 34.9 34.8 34.7 33.9.  16 rows gain 0.3-1.5 us.  Beside the projection that has no splits to merge (4.8 us) 8 MB gain nothing
-    # and 16 lose 3 %.
-    _MERGING_AHEAD_EACH = 192 << 10
+    # for each workgroup that brings (they are what the projection's leave idle), and no more than the chiplets' L2 keep until it is read: what
+    # only the memory-side cache holds comes no faster than out of memory.  A pass of four steps over 640 keys, us, with nothing and with 10, 13, 15,
+    # 18, 20, 22, 25 and 30 MB (width 1,536 of 12 heads, gate and up 52 MB, 160 workgroups bring): 1 row 4,400 4,213 4,207 4,207 4,171 4,141 4,108 4,200 4,220, 4 rows
+    # 4,390 4,297 4,297 4,304 4,261 4,236 4,205 4,299 4,340, 8 rows 4,610 4,450 4,438 4,437 4,428 4,422 4,438 4,477 4,502, 16 rows 4,830 4,668 4,665 4,676 4,676
+    # 4,678 4,692 4,685 4,724.  The same brought beside attention too, ahead of this, made steps 1 to 4 % longer.  Beside the projection that has no
+    # splits to merge 8 MB gain nothing and 16 lose 3 %.
+    _MERGING_AHEAD_EACH = 128 << 10
 
     def _whole_ahead(self, weights: Any, rows: int, busy: int, plain: bool = False) -> tuple:
         """`plain`: the next product is one by itself (its result whole, no norm or key splits about it)."""
@@ -1538,6 +1538,7 @@ class HipKernels:
                 and rows <= 16
                 and project.weight.dtype == torch.bfloat16
                 and project.in_features == layout.num_heads * dim
+                and _in_pieces(project.weight)
                 # Every workgroup of the product reads all splits of its K range, rows * splits / 16 times the bytes
                 # of its weights more than a plain product, and the kernel that merges as it loads is built for a
                 # small weight (one tile a wave).  Ahead at the 1.5B sizes (4.7 MB of weights: attention and projection
