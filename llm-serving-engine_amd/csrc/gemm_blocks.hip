@@ -348,7 +348,11 @@ struct Reads {
 
 // WN x WM waves of TN x TM tiles of 16 x 16; stages of 64 k, of which the last may be half full (HALF: K / splits % 64 == 32); A_SIMD: the waves a
 // SIMD is to hold; AHEAD: see Reads.
-template <int WN, int WM, int TN, int TM, int AHEAD, int STAGES, int A_SIMD, bool HALF, typename TO, int OUT>
+// ONCE: no other workgroup reads these weights.  They then go past the caches: what a CU has under way of memory is limited (32 KB or so), a line that is kept
+// nowhere takes less of it (measured with nothing but the loads: 112 CUs take 44 bytes a ns each, past the caches 47 to 53), and x keeps its place in
+// L2.  Us, before -> after: 96 rows of N 17,920 K 1,536 18.3 -> 17.3, of N 1,536 K 8,960 in parts 11.6 -> 10.1, of N 37,888 K 3,584 60.1 -> 51.6; 160 rows 21.9 -> 21.2,
+// of N 37,888 59.5 -> 54.4.  With a second tile of rows the other workgroup would find them gone: 320 rows of N 1,536 K 8,960 18.1 -> 21.1.
+template <int WN, int WM, int TN, int TM, int AHEAD, int STAGES, int A_SIMD, bool HALF, typename TO, int OUT, bool ONCE>
 __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                           const void* __restrict__ bias, int bias_is_float,
                                                                           TO* __restrict__ out, int M, int N, int K, int k_split, Rotated rotated) {
@@ -384,7 +388,8 @@ __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const 
   auto load_piece = [&](int i, int step, unsigned stage) {
     unsigned char* to = lds + stage * STAGE_BYTES + (i < PER_W ? i * THREADS * 16 : W_BYTES + (i - PER_W) * THREADS * 16) + wave * 1024;
     const bf16_t* from = src[i] + step * BK - (HALF && step == last && beyond[i] ? BK / 2 : 0);
-    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)from, (void __attribute__((address_space(3)))*)to, 16, 0, 0);
+    if (ONCE && i < PER_W) __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)from, (void __attribute__((address_space(3)))*)to, 16, 0, 2);
+    else __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)from, (void __attribute__((address_space(3)))*)to, 16, 0, 0);
   };
   // where it reads its operands: rows r16 + 16 t of the wave's, part 4 * step of 32 k + q.  Of that only `lane_at` differs by lane (a row is 128 bytes and
   // the second step's part the first one's with bit 2 turned, so 64 of it are turned): one register, as 256 x 320 has none to spare: with rows and parts
@@ -512,24 +517,33 @@ __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const 
     store_tiles<TN, TM, false, TO, OUT>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane, rotated, early, streamed);
 }
 
-template <int WN, int WM, int TN, int TM, int AHEAD, int STAGES, int A_SIMD, bool HALF, typename TO, int OUT>
-static int launch_block(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
-                        int splits, hipStream_t stream, const Rotated& rotated) {
+template <int WN, int WM, int TN, int TM, int AHEAD, int STAGES, int A_SIMD, bool HALF, typename TO, int OUT, bool ONCE>
+static int launch_block_as(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
+                           int splits, hipStream_t stream, const Rotated& rotated) {
   constexpr int BN = WN * TN * 16, BM = WM * TM * 16;
   constexpr size_t stages = (size_t)STAGES * (BN + BM) * 128, values = OUT == OUT_ROTATED ? (size_t)WN * WM * 16 * (16 * TN + 4) * sizeof(float) : 0;
   constexpr size_t bytes = stages > values ? stages : values;
   static_assert(bytes <= 160 * 1024, "a CU's LDS");
   static bool asked = false;
   if (!asked) {
-    if (hipFuncSetAttribute((const void*)gemm_block_kernel<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT>,
+    if (hipFuncSetAttribute((const void*)gemm_block_kernel<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT, ONCE>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
       return ERR_BAD_ARGUMENT;
     asked = true;
   }
-  hipLaunchKernelGGL((gemm_block_kernel<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT>),
+  hipLaunchKernelGGL((gemm_block_kernel<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT, ONCE>),
                      dim3(((N + BN - 1) / BN) * ((M + BM - 1) / BM), 1, splits), dim3(WN * WM * 64), bytes, stream, (const bf16_t*)x,
                      (const bf16_t*)w, bias, bias_is_float, (TO*)out, M, N, K, K / splits, rotated);
   return LAUNCH_STATUS();
+}
+// (a weight of up to 8 MB may have been brought into the caches, or live there with the rest of a small model: it is kept)
+template <int WN, int WM, int TN, int TM, int AHEAD, int STAGES, int A_SIMD, bool HALF, typename TO, int OUT>
+static int launch_block(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
+                        int splits, hipStream_t stream, const Rotated& rotated) {
+  if constexpr (OUT != OUT_ROTATED && !HALF)
+    if (M <= WM * TM * 16 && (long)N * K > (1L << 22))
+      return launch_block_as<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT, true>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, rotated);
+  return launch_block_as<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT, false>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, rotated);
 }
 
 // The shapes: a tile's weight rows and rows of x, how many a CU holds at a time, and what a launch, a tile, a tile's

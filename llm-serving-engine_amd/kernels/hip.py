@@ -589,7 +589,12 @@ class HipKernels:
         5 to 25 percent faster since, by spreading its loads and by more shapes; the lines have stayed, as what they leave to the library was not timed again
         but for N 1,536 K 8,960 at 2,048 rows: the library 56 us, here 59 in two parts and what adds them up.)
 
-        Gated, up to weights of 40 million: ahead while one round of 256 x 128 tiles holds the result (K 896 0.59-0.76, N 17,920 K 1,536
+        Gated, 65 to 128 rows of weights of up to 150 million (beyond, the library was not timed against it): past the caches the weights come faster than
+        through the ring's stages.  Us at 65 / 96 / 128 rows, the ring -> here: N 17,920 K 1,536 18.7 / 17.7 / 20.9 -> 15.5 / 17.3 / 19.0, N 37,888 K 3,584 62.0 / 54.5 /
+        55.6 -> 53.2 / 52.0 / 53.5, N 9,728 K 896 9.9 / 10.0 / 11.9 -> 8.7 / 8.8 / 9.3, N 24,576 K 3,072 40.4 / 42.9 / 40.7 -> 34.6 / 34.7 / 34.9, N 13,824 K 2,304 18.6 /
+        19.0 / 23.1 -> 17.9 / 18.5 / 20.1, N 38,912 K 2,560 47.8 / 42.6 / 43.8 -> 44.4 / 42.7 / 44.2, N 7,168 K 1,024 7.9 / 8.1 / 8.9 -> 7.4 / 6.7 / 7.5.
+
+        Gated, more rows, up to weights of 40 million: ahead while one round of 256 x 128 tiles holds the result (K 896 0.59-0.76, N 17,920 K 1,536
         0.79-0.90, K 2,048 0.70-0.97), behind where it takes a second one that is half empty (N 17,920 at 416-576 rows 1.00-1.14, N 16,384 K
         2,048 at 520-600 1.28, N 11,264-16,384 K 2,048 at 700-900 1.05-1.30), ahead again for K up to 1,536 from about 160 tiles of 256 x 256
         on (N 17,920 at 640-896 0.79-0.98).  From 1,024 rows on the activation's own pass decides, which is a share of
@@ -611,7 +616,7 @@ class HipKernels:
         size, results = out_features * in_features, rows * out_features
         if gated:
             if rows <= 128:
-                return False
+                return (1 << 22) < size <= 150_000_000
             if rows < 1024:
                 one_round = -(-out_features // 256) * -(-rows // 128) <= 256
                 return size <= 40_000_000 and (one_round or (in_features <= 1536 and results >= 160 * 256 * 256))
