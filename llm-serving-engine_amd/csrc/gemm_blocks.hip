@@ -635,6 +635,14 @@ template <typename TO, int OUT>
 static int launch_shape(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
                         int splits, hipStream_t stream) {
 #define BLOCK(...) return launch_block<__VA_ARGS__, TO, OUT>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, {})
+  // Few rows of a weight that makes more than a round of such tiles (a head): a stream of the weight, for which what counts is 128 or 256 weight
+  // rows to a row of tiles that holds all of x, with 72 to 132 KB of LDS asked for at a time.  Us, the library -> the shape that the estimate would pick -> this one: N 151,936 K 1,536 at
+  // 17 rows 110 -> 81 -> 82, 32 rows 108 -> 93 -> 88, 48 rows 125 -> 104 -> 94, 64 rows 118 -> 113 -> 99 (5.1 TB/s, the result's way among it), 80 rows 133 -> 113 -> 105,
+  // 96 rows 128 -> 117 -> 108; N 152,064 K 3,584 at 32 rows 257 -> 201 -> 189, 64 rows 217 -> 241 -> 210, 96 rows 234 -> 239 -> 219.  128 x 32 at 32 rows 88 and 188, 256 x 64 at 64 rows 101 and 210.
+  if constexpr (OUT == OUT_PLAIN) {
+    if (K % 64 == 0 && splits == 1 && M <= 64 && N > 256 * 128) BLOCK(4, 1, 2, 4, 3, 3, 2, false);
+    if (K % 64 == 0 && splits == 1 && M > 64 && M <= 96 && N > 256 * 256) BLOCK(4, 1, 4, 6, 5, 3, 2, false);
+  }
   const int shape = pick_shape(M, N, K, splits, OUT == OUT_GATED ? sizeof(TO) / 2 : sizeof(TO));
   if ((K / splits) % 64) {  // a K that ends in half a stage
     switch (shape) {

@@ -557,7 +557,7 @@ class HipKernels:
             # On the device the library is ahead of "medium" as it stands, so a captured step (which
             # costs the host nothing per launch) takes the library; a step launched kernel by kernel
             # is bound by the host, where a torch call costs four times one of ours (but a weight beyond what the
-            # ring takes goes to the library either way: the 1.5B sizes' head at 64 rows 112 us against 174).
+            # ring takes goes to the library either way where `_one_row_of_tiles` leaves it here)
             # Except a small weight: there the library's fixed cost shows (qkv and o of the 1.5B sizes in a
             # captured chain: 7.1-7.7 us each, against 4.8 and 4.0 at 17 rows, 5.0 and 4.5 at 32, 6.7 and 6.2 at
             # 64 for the kernel that brings two or four tiles of x through LDS beside a weight tile; where K is
@@ -578,6 +578,18 @@ class HipKernels:
         """Whether a product of up to 16 rows goes to the kernel that streams whole cache lines (csrc/gemm_bf16.hip: gemm_flow), whichever of
         the others `_streaming` names: those take a K that is no multiple of 64, and more rows."""
         return streaming in ("skinny", "ring") and rows <= 16 and in_features % 64 == 0
+
+    @staticmethod
+    def _one_row_of_tiles(x: torch.Tensor, weights: LinearWeights, may_split: bool) -> bool:
+        """Whether a plain product that `_streaming` gives to the ring or to the library is the tiled kernel's, with x whole in one row of its tiles: 17 to 128 rows
+        of a weight of more rows than the ring takes in a round, and large (a head).  csrc/gemm_blocks.hip's launch_shape has the library's times against its; at 128 rows
+        N 151,936 K 1,536 takes 134 us at the library and 119 there, N 152,064 K 3,584 253 and 238.  Up to 150 million the other way is the ring up to 64 rows, us at 17 / 64
+        rows: N 151,936 K 896 57.5 / 72.6 -> 50.6 / 59.7, N 128,256 K 1,024 47.9 / 66.9 -> 47.4 / 55.9; in one round it is ahead (N 49,152 K 1,536 29.4 / 34.3, tiles 32.5 / 37.8)."""
+        rows, size = x.shape[0], weights.out_features * weights.in_features
+        return (
+            16 < rows <= 128 and not may_split and size > (100_000_000 if rows <= 64 else 150_000_000) and weights.out_features > 256 * 14 * 16
+            and weights.in_features % 64 == 0 and x.dtype == torch.bfloat16 and weights.weight.dtype == torch.bfloat16 and _in_pieces(x, weights.weight)
+        )
 
     @staticmethod
     def _tiled_ahead(rows: int, out_features: int, in_features: int, gated: bool, may_split: bool) -> bool:
@@ -741,6 +753,8 @@ class HipKernels:
             raise KernelError(f"linear: x has {inner} columns, the weight {weights.in_features}")
         bias = weights.bias
         streaming = self._streaming(x, weights, may_split=partial and out_dtype == torch.float32)
+        if self._one_row_of_tiles(x, weights, partial and out_dtype == torch.float32):
+            streaming = "tiled"
         if (
             streaming is None
             and not self.ring_products
