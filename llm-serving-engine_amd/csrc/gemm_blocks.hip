@@ -56,6 +56,26 @@ __device__ __forceinline__ void tile_of_workgroup(int index, int tiles_n, int ti
 #define OUT_PLAIN 0
 #define OUT_GATED 1    // silu(gate) * up of columns that alternate gate_j, up_j
 #define OUT_ROTATED 2  // rows of q, k and v heads: q and k rotated in neighbouring pairs, k and v stored in their pages too
+#define OUT_NORM 3     // added to the residual stream; what the product behind the norm reads, and the squares it divides by (Link)
+#define OUT_SCALED 4   // OUT_GATED of such rows: the sums are divided by the rows' root mean squares first
+constexpr bool is_gated(int out) { return out == OUT_GATED || out == OUT_SCALED; }
+
+// Two products with a norm between them, without a kernel for the norm (gemm_bf16.hip has the same for up to 64 rows).  The first (OUT_NORM) holds whole sums over
+// K, adds them to the residual stream, and writes x * weight in bfloat16, not yet divided by the row's root mean square, with the sum of squares of each tile's
+// columns a row.  The second (OUT_SCALED) adds those up and multiplies its float32 results by rsqrt(mean + eps): rounding
+// x * weight loses what rounding the normed row loses.  A norm's kernel takes 5 us of a step of 96 to 320 rows and 11 of 2,048; against that the first needs whole sums (us in a
+// step, before -> after: 96 rows of N 1,536 K 1,536 5.4 -> 6.9, 320 rows 6.5 -> 9.2, 2,048 rows 17.4 -> 21.2 with the stream's way) and the second the squares (17.9 -> 19.3,
+// 24.6 -> 25.7, 98 -> 98).  A pass: prompt 77 1,714 -> 1,699 us, mixed 31 + 256 9,914 -> 9,790, prompt 2,048 by 1.5 percent.
+struct Link {
+  float* hidden;             // OUT_NORM: [M, N], added to in place
+  const void* weight;        // OUT_NORM: the norm's [N]
+  int weight_is_float;
+  bf16_t* rows;              // OUT_NORM: [M, N]
+  float* sums;               // [pieces, stride]: of a tile's columns of x each, row by row; `stride` is M up to a multiple of four
+  float inverse_width, eps;  // OUT_SCALED
+};
+#define SUMS_MOST 48  // pieces of squares a row
+__host__ __device__ __forceinline__ int sums_stride(int M) { return (M + 3) / 4 * 4; }
 
 // What OUT_ROTATED needs: cos and sin of [token][dim / 2], the layer's pages and each token's place there (negative: none; the
 // layout of a page is common.h's).  `dim` is a multiple of 16.
@@ -76,7 +96,7 @@ __device__ __forceinline__ int weight_row(int i, int r) {
 }
 template <typename TO, int OUT, int TN>
 constexpr int group_of() {
-  int tiles = sizeof(TO) == 4 ? 1 : OUT == OUT_GATED ? 4 : 2;
+  int tiles = OUT == OUT_NORM ? 2 : sizeof(TO) == 4 ? 1 : is_gated(OUT) ? 4 : 2;
   while (tiles > TN) tiles /= 2;
   return tiles;
 }
@@ -170,11 +190,12 @@ __device__ __forceinline__ void store_values(const Rotated& to, const float* min
 template <int TN, int TM, bool INSIDE, typename TO, int OUT>
 __device__ __forceinline__ void store_tiles(const f32x4 (&acc)[TN][TM], float* mine, TO* __restrict__ out,
                                             const void* __restrict__ bias, int bias_is_float, int slice, int M, int N,
-                                            int n_wave, int m_wave, int lane, const Rotated& rotated, const Early<TN, TM>& early, bool streamed) {
-  static_assert(OUT == OUT_PLAIN || sizeof(TO) == 2, "a gated or rotated result is bfloat16");
+                                            int n_wave, int m_wave, int lane, const Rotated& rotated, const Early<TN, TM>& early, bool streamed,
+                                            const float* factor) {
+  static_assert(OUT == OUT_PLAIN || OUT == OUT_NORM || sizeof(TO) == 2, "a gated or rotated result is bfloat16");
   constexpr int G = group_of<TO, OUT, TN>(), WHOLE = TN / G * G;
   const int r16 = lane & 15, q = lane >> 4;
-  const bool with_bias = bias && slice == 0;
+  const bool with_bias = OUT != OUT_SCALED && bias && slice == 0;
   auto store_piece = [&](auto piece, TO* dst) {
     if (streamed) __builtin_nontemporal_store(piece, (decltype(piece)*)dst);
     else *(decltype(piece)*)dst = piece;
@@ -182,7 +203,7 @@ __device__ __forceinline__ void store_tiles(const f32x4 (&acc)[TN][TM], float* m
   // a run of RUN neighbouring columns from n on, of row m: the sums of a group (or of one tile) and their bias
   auto store_run = [&](auto run_of, int m, int n, const float* sums) {
     constexpr int RUN = decltype(run_of)::value;
-    if constexpr (OUT == OUT_GATED) {
+    if constexpr (is_gated(OUT)) {
       TO* dst = out + (size_t)m * (N / 2) + n / 2;
       bf16_t gated[RUN / 2];
 #pragma unroll
@@ -281,26 +302,99 @@ __device__ __forceinline__ void store_tiles(const f32x4 (&acc)[TN][TM], float* m
           bias_here[i][e] = INSIDE || n < N ? load_as_float(bias, bias_is_float, n) : 0.f;
         }
     }
-    auto sum_at = [&](int i, int j, int e) { return with_bias ? acc[i][j][e] + bias_here[i][e] : acc[i][j][e]; };
+    auto sum_at = [&](int i, int j, int e, float row_factor) { return OUT == OUT_SCALED ? acc[i][j][e] * row_factor : with_bias ? acc[i][j][e] + bias_here[i][e] : acc[i][j][e]; };
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
       const int m = m_wave + j * 16 + r16;
       if (!INSIDE && m >= M) continue;
+      const float row_factor = OUT == OUT_SCALED ? factor[j * 16 + r16] : 1.f;
 #pragma unroll
       for (int i = 0; i < WHOLE; i += G) {
         float sums[4 * G];
 #pragma unroll
-        for (int e = 0; e < 4 * G; ++e) sums[e] = sum_at(i + e / 4, j, e % 4);
+        for (int e = 0; e < 4 * G; ++e) sums[e] = sum_at(i + e / 4, j, e % 4, row_factor);
         store_run(std::integral_constant<int, 4 * G>{}, m, n_wave + i * 16 + q * 4 * G, sums);
       }
 #pragma unroll
       for (int i = WHOLE; i < TN; ++i) {
         float sums[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sums[e] = sum_at(i, j, e);
+        for (int e = 0; e < 4; ++e) sums[e] = sum_at(i, j, e, row_factor);
         store_run(std::integral_constant<int, 4>{}, m, n_wave + i * 16 + q * 4, sums);
       }
     }
+  }
+}
+
+// What OUT_NORM adds to, and its norm's weight: asked for behind the first stages, used at the end.  A lane's columns of tile i: n_wave + weight_row(i, 4 q) .. + 3.
+template <int TN, int TM>
+struct Stream {
+  f32x4 hidden[TN][TM];
+  uint2 low[TN], high[TN];  // of the weight: four bfloat16 (twice) or the halves of four float32
+};
+template <int TN, int TM, int G>
+__device__ __forceinline__ void ask_stream(Stream<TN, TM>& stream, const Link& link, int M, int N, int n_wave, int m_wave, int lane) {
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    const int n = min(n_wave + weight_row<TN, G>(i, (lane >> 4) * 4), N - 4);
+    const char* weight = (const char*)link.weight + (size_t)n * (link.weight_is_float ? 4 : 2);
+    stream.low[i] = *(const uint2*)weight;
+    stream.high[i] = *(const uint2*)(weight + (link.weight_is_float ? 8 : 0));
+#pragma unroll
+    for (int j = 0; j < TM; ++j) stream.hidden[i][j] = *(const f32x4*)(link.hidden + (size_t)min(m_wave + j * 16 + (lane & 15), M - 1) * N + n);
+  }
+}
+// The way out of OUT_NORM.  N is a multiple of eight: a run of four or eight columns lies inside it or beyond.
+// `shares`: in LDS, where the squares of this wave's rows and columns go.
+template <int TN, int TM, int G>
+__device__ __forceinline__ void store_norm(const f32x4 (&acc)[TN][TM], const Stream<TN, TM>& stream, const Link& link, const void* bias, int bias_is_float, int M,
+                                           int N, int n_wave, int m_wave, int lane, float* shares) {
+  constexpr int WHOLE = TN / G * G;
+  const int r16 = lane & 15, q = lane >> 4;
+  f32x4 bias_here[TN];
+  if (bias) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bias_here[i][e] = load_as_float(bias, bias_is_float, min(n_wave + weight_row<TN, G>(i, q * 4) + e, N - 1));
+  }
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    const int m = m_wave + j * 16 + r16;
+    float squares = 0.f;
+    uint2 packed[TN];
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      const int n = n_wave + weight_row<TN, G>(i, q * 4);
+      const bool inside = m < M && n < N;
+      f32x4 x = acc[i][j];
+      if (bias) x += bias_here[i];
+      x += stream.hidden[i][j];
+      const unsigned halves[4] = {stream.low[i].x << 16, stream.low[i].x & 0xffff0000u, stream.low[i].y << 16, stream.low[i].y & 0xffff0000u};
+      const unsigned words[4] = {stream.low[i].x, stream.low[i].y, stream.high[i].x, stream.high[i].y};
+      bf16_t row[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        row[e] = (bf16_t)(x[e] * __uint_as_float(link.weight_is_float ? words[e] : halves[e]));
+        squares = inside ? fmaf(x[e], x[e], squares) : squares;
+      }
+      packed[i] = *(const uint2*)row;
+      if (inside) *(f32x4*)(link.hidden + (size_t)m * N + n) = x;
+    }
+#pragma unroll
+    for (int i = 0; i < TN; i += G) {
+      const int n = n_wave + weight_row<TN, G>(i, q * 4);
+      if (m >= M || n >= N) continue;
+      bf16_t* to = link.rows + (size_t)m * N + n;
+      if (G == 2 && i < WHOLE) {
+        *(uint4*)to = make_uint4(packed[i].x, packed[i].y, packed[i + G - 1].x, packed[i + G - 1].y);
+      } else {
+        *(uint2*)to = packed[i];
+      }
+    }
+    squares += __shfl_xor(squares, 16, WAVE);
+    squares += __shfl_xor(squares, 32, WAVE);
+    if (q == 0) shares[j * 16 + r16] = squares;
   }
 }
 
@@ -355,7 +449,7 @@ struct Reads {
 template <int WN, int WM, int TN, int TM, int AHEAD, int STAGES, int A_SIMD, bool HALF, typename TO, int OUT, bool ONCE>
 __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                           const void* __restrict__ bias, int bias_is_float,
-                                                                          TO* __restrict__ out, int M, int N, int K, int k_split, Rotated rotated) {
+                                                                          TO* __restrict__ out, int M, int N, int K, int k_split, Rotated rotated, Link link) {
   constexpr int BK = 64, THREADS = WN * WM * 64, BN = WN * TN * 16, BM = WM * TM * 16, SLOTS = BK / 8;
   constexpr int ROW_BYTES = BK * 2, W_BYTES = BN * ROW_BYTES, STAGE_BYTES = W_BYTES + BM * ROW_BYTES;
   constexpr int PER_W = BN * SLOTS / THREADS, PER = PER_W + BM * SLOTS / THREADS;  // 16-byte pieces of a stage a lane asks for
@@ -414,6 +508,11 @@ __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const 
 #pragma unroll
       for (int i = 0; i < PER; ++i) load_piece(i, s, s);
     }
+  Stream<OUT == OUT_NORM ? TN : 1, OUT == OUT_NORM ? TM : 1> residual;
+  if constexpr (OUT == OUT_NORM) {  // (the counts below do not know of these loads, and wait for as many of the stages' more until they have come)
+    ask_stream<TN, TM, group_of<TO, OUT, TN>()>(residual, link, M, N, n0 + wave_n * TN * 16, m0 + wave_m * TM * 16, lane);
+    asm volatile("" ::: "memory");
+  }
   wait_stages<PER, STAGES - 1>(min(last, STAGES - 1));  // stage 0 has landed
   __builtin_amdgcn_s_barrier();
   // The reads of LDS are written as instructions, with their waits: left to the compiler, every read of LDS waits for all
@@ -491,8 +590,33 @@ __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const 
     multiply(second_half, std::true_type{}, step);
     multiply(first_half, std::true_type{}, step + 1);
   }
+  // OUT_SCALED: the squares of this tile's rows, [pieces][BM], are brought into the first stage that is not asked for anew, some stages before they are used.  (The
+  // waits below do not know of these loads, and wait for as many of the stages'.  The sums come as `bias`, their number, at most SUMS_MOST, as `bias_is_float`:
+  // arguments that come with the wave.  As loads into registers before the stages they were waited for with all the stages behind them: 320 rows of N 17,920 K 1,536
+  // 24.6 us without a norm, 26.1 so.)
+  // (Not the largest tile, which has no registers to spare for it: it asks behind its last products.)
+  constexpr bool SQUARES_EARLY = TN * TM <= 36;
+  unsigned char* squares_at = lds;
+  auto ask_squares = [&] {
+    constexpr int QUADS = BM / 4;
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));  // (nothing of this is to be made, and kept, before the products)
+    for (int chunk = wave; chunk * 64 < bias_is_float * QUADS; chunk += WN * WM) {
+      const int at = min(chunk * 64 + lane, bias_is_float * QUADS - 1), piece = at / QUADS, quad = at % QUADS;
+      const float* from = (const float*)bias + (size_t)piece * sums_stride(M) + min(m0 + quad * 4, sums_stride(M) - 4);
+      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)from, (void __attribute__((address_space(3)))*)(squares_at + chunk * 1024), 16, 0, 0);
+    }
+  };
+  [[maybe_unused]] const int first_free = step;
   for (; step < last; ++step) {
     multiply(second_half, std::false_type{}, step);
+    if constexpr (OUT == OUT_SCALED && SQUARES_EARLY) {
+      static_assert(SUMS_MOST * BM * 4 <= STAGE_BYTES, "in a stage's place");
+      if (step == first_free) {
+        squares_at = lds + (stage == 0 ? STAGES - 1 : stage - 1) * STAGE_BYTES;
+        ask_squares();
+      }
+    }
     multiply(first_half, std::false_type{}, step + 1);
   }
   if (!HALF) multiply(second_half, std::false_type{}, last);
@@ -508,18 +632,54 @@ __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const 
 #undef READ_TILE
   const int n_wave = n0 + wave_n * TN * 16, m_wave = m0 + wave_m * TM * 16;
   if constexpr (OUT == OUT_ROTATED) __syncthreads();  // every wave has read the last stage: LDS is free for the values
+  const float* factor = nullptr;  // of the wave's rows, in LDS
+  if constexpr (OUT == OUT_SCALED) {
+    if constexpr (!SQUARES_EARLY) {
+      __syncthreads();  // every wave has read the last stage
+      ask_squares();
+    }
+    wait_loads<0>();
+    __syncthreads();
+    float* shares = (float*)squares_at;
+    static_assert(BM <= THREADS, "a thread a row");
+    int row = threadIdx.x;
+    asm volatile("" : "+v"(row));
+    if (row < BM) {  // (a row's squares are read, and the factor written in the place of the first, by one thread)
+      float squares = 0.f;
+#pragma unroll 8
+      for (int c = 0; c < bias_is_float; ++c) squares += shares[c * BM + row];
+      shares[row] = rsqrtf(squares * link.inverse_width + link.eps);
+    }
+    __syncthreads();
+    factor = shares + wave_m * TM * 16;
+  }
   float* mine = (float*)lds + (size_t)wave * 16 * (16 * TN + 4);
-  const bool streamed = (size_t)gridDim.z * M * N * (OUT == OUT_GATED ? sizeof(TO) / 2 : sizeof(TO)) > STREAMED_FROM;
-  if (m_wave >= M || n_wave >= N) return;
+  const bool streamed = (size_t)gridDim.z * M * N * (is_gated(OUT) ? sizeof(TO) / 2 : sizeof(TO)) > STREAMED_FROM;
+  if constexpr (OUT == OUT_NORM) {
+    __syncthreads();  // every wave has read the last stage: LDS is free for the squares, [WN][BM]
+    float* shares = (float*)lds;
+    store_norm<TN, TM, group_of<TO, OUT, TN>()>(acc, residual, link, bias, bias_is_float, M, N, n_wave, m_wave, lane, shares + wave_n * BM + wave_m * TM * 16);
+    __syncthreads();
+    const int row = threadIdx.x;
+    static_assert(BM <= THREADS, "a thread a row");
+    if (row < BM && m0 + row < M) {
+      float squares = shares[row];
+#pragma unroll
+      for (int c = 1; c < WN; ++c) squares += shares[c * BM + row];
+      link.sums[(size_t)tile_n * sums_stride(M) + m0 + row] = squares;
+    }
+  } else {
+    if (m_wave >= M || n_wave >= N) return;
   if (m_wave + 16 * TM <= M && n_wave + 16 * TN <= N && N % 8 == 0)
-    store_tiles<TN, TM, true, TO, OUT>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane, rotated, early, streamed);
+    store_tiles<TN, TM, true, TO, OUT>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane, rotated, early, streamed, factor);
   else
-    store_tiles<TN, TM, false, TO, OUT>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane, rotated, early, streamed);
+    store_tiles<TN, TM, false, TO, OUT>(acc, mine, out, bias, bias_is_float, blockIdx.z, M, N, n_wave, m_wave, lane, rotated, early, streamed, factor);
+  }
 }
 
 template <int WN, int WM, int TN, int TM, int AHEAD, int STAGES, int A_SIMD, bool HALF, typename TO, int OUT, bool ONCE>
 static int launch_block_as(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
-                           int splits, hipStream_t stream, const Rotated& rotated) {
+                           int splits, hipStream_t stream, const Rotated& rotated, const Link& link) {
   constexpr int BN = WN * TN * 16, BM = WM * TM * 16;
   constexpr size_t stages = (size_t)STAGES * (BN + BM) * 128, values = OUT == OUT_ROTATED ? (size_t)WN * WM * 16 * (16 * TN + 4) * sizeof(float) : 0;
   constexpr size_t bytes = stages > values ? stages : values;
@@ -533,17 +693,17 @@ static int launch_block_as(const void* x, const void* w, const void* bias, int b
   }
   hipLaunchKernelGGL((gemm_block_kernel<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT, ONCE>),
                      dim3(((N + BN - 1) / BN) * ((M + BM - 1) / BM), 1, splits), dim3(WN * WM * 64), bytes, stream, (const bf16_t*)x,
-                     (const bf16_t*)w, bias, bias_is_float, (TO*)out, M, N, K, K / splits, rotated);
+                     (const bf16_t*)w, bias, bias_is_float, (TO*)out, M, N, K, K / splits, rotated, link);
   return LAUNCH_STATUS();
 }
 // (a weight of up to 8 MB may have been brought into the caches, or live there with the rest of a small model: it is kept)
 template <int WN, int WM, int TN, int TM, int AHEAD, int STAGES, int A_SIMD, bool HALF, typename TO, int OUT>
 static int launch_block(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
-                        int splits, hipStream_t stream, const Rotated& rotated) {
+                        int splits, hipStream_t stream, const Rotated& rotated, const Link& link = {}) {
   if constexpr (OUT != OUT_ROTATED && !HALF)
     if (M <= WM * TM * 16 && (long)N * K > (1L << 22))
-      return launch_block_as<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT, true>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, rotated);
-  return launch_block_as<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT, false>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, rotated);
+      return launch_block_as<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT, true>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, rotated, link);
+  return launch_block_as<WN, WM, TN, TM, AHEAD, STAGES, A_SIMD, HALF, TO, OUT, false>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, rotated, link);
 }
 
 // The shapes: a tile's weight rows and rows of x, how many a CU holds at a time, and what a launch, a tile, a tile's
@@ -633,8 +793,8 @@ extern "C" int llmserve_gemm_blocks_parts(int M, int N, int K) {
 
 template <typename TO, int OUT>
 static int launch_shape(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
-                        int splits, hipStream_t stream) {
-#define BLOCK(...) return launch_block<__VA_ARGS__, TO, OUT>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, {})
+                        int splits, hipStream_t stream, const Link& link = {}) {
+#define BLOCK(...) return launch_block<__VA_ARGS__, TO, OUT>(x, w, bias, bias_is_float, out, M, N, K, splits, stream, {}, link)
   // Few rows of a weight that makes more than a round of such tiles (a head): a stream of the weight, for which what counts is 128 or 256 weight
   // rows to a row of tiles that holds all of x, with 72 to 132 KB of LDS asked for at a time.  Us, the library -> the shape that the estimate would pick -> this one: N 151,936 K 1,536 at
   // 17 rows 110 -> 81 -> 82, 32 rows 108 -> 93 -> 88, 48 rows 125 -> 104 -> 94, 64 rows 118 -> 113 -> 99 (5.1 TB/s, the result's way among it), 80 rows 133 -> 113 -> 105,
@@ -643,8 +803,8 @@ static int launch_shape(const void* x, const void* w, const void* bias, int bias
     if (K % 64 == 0 && splits == 1 && M <= 64 && N > 256 * 128) BLOCK(4, 1, 2, 4, 3, 3, 2, false);
     if (K % 64 == 0 && splits == 1 && M > 64 && M <= 96 && N > 256 * 256) BLOCK(4, 1, 4, 6, 5, 3, 2, false);
   }
-  const int shape = pick_shape(M, N, K, splits, OUT == OUT_GATED ? sizeof(TO) / 2 : sizeof(TO));
-  if ((K / splits) % 64) {  // a K that ends in half a stage
+  const int shape = pick_shape(M, N, K, splits, is_gated(OUT) ? sizeof(TO) / 2 : sizeof(TO));
+  if constexpr (OUT != OUT_SCALED) if ((K / splits) % 64) {  // a K that ends in half a stage
     switch (shape) {
       case 0: BLOCK(4, 2, 4, 8, 3, 2, 2, true);
       case 7: BLOCK(2, 2, 4, 3, 3, 5, 2, true);
@@ -681,6 +841,63 @@ extern "C" int llmserve_gemm_blocks(const void* x, const void* w, const void* bi
   if (gated) return launch_shape<bf16_t, OUT_GATED>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
   return out_is_float ? launch_shape<float, OUT_PLAIN>(x, w, bias, bias_is_float, out, M, N, K, splits, stream)
                       : launch_shape<bf16_t, OUT_PLAIN>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
+}
+
+// The shape of OUT_NORM, which holds whole sums and a part of the stream beside them: tiles as small as one round of 256 workgroups allows, as more CUs then bring the
+// operands, and what a CU brings (44 bytes a ns) is what they take; beyond a round, the estimate's; no more than SUMS_MOST tiles a row.  0: 32 x 32, 1: 64 x 32, else of SHAPES.
+static int pick_norm_shape(int M, int N, int K) {
+  auto workgroups = [&](int n, int m) { return (long)((N + n - 1) / n) * ((M + m - 1) / m); };
+  if (workgroups(32, 32) <= 256 && N <= 32 * SUMS_MOST) return 0;
+  if (workgroups(64, 32) <= 256 && N <= 64 * SUMS_MOST) return 1;
+  int best = N <= 64 * SUMS_MOST ? 9 : 10;
+  for (int s : {8, 6, 10})
+    if (N <= SHAPES[s].n * SUMS_MOST && shape_us(SHAPES[s], M, N, K, 1, 10) < shape_us(SHAPES[best], M, N, K, 1, 10)) best = s;
+  return best;
+}
+
+// How many pieces of squares the product into a norm leaves a row.
+extern "C" int llmserve_gemm_blocks_norm_pieces(int M, int N, int K) {
+  const int shape = pick_norm_shape(M, N, K), columns = shape == 0 ? 32 : shape == 1 ? 64 : SHAPES[shape].n;
+  return (N + columns - 1) / columns;
+}
+
+// What the whole sums cost it, in thousandths of a us: its own time (of the two smallest tiles as measured in a step: K 1,536 of N 1,536 6.9 us at 96 rows, 9.2 at 320) over
+// that in as many parts as `llmserve_gemm_blocks_parts` says.
+extern "C" int llmserve_gemm_blocks_norm_cost(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 64 || N > 128 * SUMS_MOST) return 1 << 30;
+  const int splits = llmserve_gemm_blocks_parts(M, N, K);
+  const int shape = pick_norm_shape(M, N, K);
+  const float whole = shape < 2 ? 2.3f + (float)(K / 64) * (shape == 0 ? 0.19f : 0.28f) : shape_us(SHAPES[shape], M, N, K, 1, 4), parts = shape_us(SHAPES[pick_shape(M, N, K, splits, 4)], M, N, K, splits, 4);
+  return (int)(1000.f * (whole - parts));
+}
+
+// hidden [M, N] float32 += x . w^T (+ bias); rows [M, N] bfloat16 = hidden * weight; sums float32 [pieces, M up to a multiple of four], as above.  N a multiple
+// of 16 up to 6,144, K of 64; x, w, hidden, weight and rows begin at a multiple of 16 bytes.
+extern "C" int llmserve_gemm_blocks_into_norm(const void* x, const void* w, const void* bias, int bias_is_float, float* hidden, const void* weight,
+                                              int weight_is_float, void* rows, float* sums, int M, int N, int K, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K <= 0 || K % 64 || N % 16 || N > 128 * SUMS_MOST || (((size_t)x | (size_t)w | (size_t)hidden | (size_t)weight | (size_t)rows) & 15)) return ERR_BAD_ARGUMENT;
+  const Link link{hidden, weight, weight_is_float, (bf16_t*)rows, sums, 0.f, 0.f};
+#define BLOCK(...) return launch_block<__VA_ARGS__, float, OUT_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link)
+  switch (pick_norm_shape(M, N, K)) {
+    case 0: BLOCK(2, 1, 1, 2, 2, 8, 1, false);
+    case 1: BLOCK(2, 1, 2, 2, 2, 8, 1, false);
+    case 6: BLOCK(2, 2, 3, 4, 4, 5, 2, false);
+    case 8: BLOCK(2, 2, 2, 4, 4, 3, 2, false);
+    case 9: BLOCK(2, 2, 2, 2, 2, 5, 2, false);
+    default: BLOCK(2, 2, 4, 4, 4, 5, 2, false);
+  }
+#undef BLOCK
+}
+
+// silu(gate) * up of the rows that it leaves (K wide, a multiple of 64 from 128 on; w [N, K] alternates gate_j, up_j): out [M, N / 2] bfloat16.
+extern "C" int llmserve_gemm_blocks_scaled(const void* rows, const float* sums, int pieces, float eps, const void* w, void* out, int M, int N, int K,
+                                           hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K < 128 || K % 64 || N % 2 || pieces < 1 || pieces > SUMS_MOST || (((size_t)rows | (size_t)sums | (size_t)w) & 15)) return ERR_BAD_ARGUMENT;
+  Link link{};
+  link.inverse_width = 1.f / (float)K, link.eps = eps;
+  return launch_shape<bf16_t, OUT_SCALED>(rows, w, sums, pieces, out, M, N, K, 1, stream, link);
 }
 
 // A product whose heads are rotated on the way out, in the smallest tile of which one round of 256 workgroups holds the result, as

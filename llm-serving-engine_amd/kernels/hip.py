@@ -85,6 +85,10 @@ _SIGNATURES = {
     "llmserve_gemm_blocks": "pppipiiiiiip",
     "llmserve_gemm_blocks_parts": "iii",
     "llmserve_gemm_blocks_shape": "iiiii",
+    "llmserve_gemm_blocks_norm_pieces": "iii",
+    "llmserve_gemm_blocks_norm_cost": "iii",
+    "llmserve_gemm_blocks_into_norm": "pppippippiiip",
+    "llmserve_gemm_blocks_scaled": "ppifppiiip",
     "llmserve_attention_generic": "pipiipppippiiiiifipfpiiipip",
     "llmserve_attention_f32": "pipipppppippiiiiiifiipfpiiipip",
     "llmserve_attention_tiles": "pipipppppippiiiiiifiiipippfpiipiiifffpiiipiip",
@@ -208,7 +212,8 @@ class NormInto:
 @dataclass
 class ScaledRows:
     """Rows times a norm's weight that are not yet divided by their root mean square: `sums` [width / 16, rows] are the sums of
-    squares, of 16 columns each, that their `reader` divides by; `tiles`: how its kernel is shaped (`llmserve_gemm_scaled`)."""
+    squares, of 16 columns each, that their `reader` divides by; `tiles`: how its kernel is shaped (`llmserve_gemm_scaled`), -1: the tiled kernel, whose
+    squares are of a tile's columns each."""
 
     rows: torch.Tensor
     sums: torch.Tensor
@@ -876,14 +881,25 @@ class HipKernels:
     def norm_into(self, hidden: torch.Tensor, weight: torch.Tensor, eps: float, reader: GatedLinearWeights) -> NormInto:
         return NormInto(hidden, weight, eps, reader)
 
+    def _own_steps(self) -> bool:
+        """Whether the steps that a product into a norm stands for are this library's (one derived from it that has its own is asked for them)."""
+        return all(getattr(type(self), step) is getattr(HipKernels, step) for step in ("linear", "add_rms_norm", "gated_linear", "rotate_store_attend"))
+
+    def linear_into(self, x, project: LinearWeights, into: NormInto) -> ScaledRows | None:
+        """`linear(x, project)` added to the stream and left for the norm's reader, where both products take it; else None, and nothing done."""
+        return self._linear_into_norm(x, None, project, into) if self._own_steps() else None
+
     def _linear_into_norm(self, x, split: tuple | None, project: LinearWeights, into: NormInto) -> ScaledRows | None:
         """`into.hidden += linear(x, project)` (or of the merge of key splits: `split` is what the attention left) and the rows that
         `into.reader` reads, where both products are of the kernels that do a norm between them; else None, and nothing done.
         Up to 64 rows: those of the kernels for a few rows, the first with whole sums over K (the 1.5B sizes' output projection
-        costs 1.6 us more than in three parts, at 64 rows 2.7; the norm's kernel 4.4 and 4.7)."""
+        costs 1.6 us more than in three parts, at 64 rows 2.7; the norm's kernel 4.4 and 4.7).  In steps with portions too: the three in a captured chain 19.4 -> 18.2 us at 24 rows,
+        23.0 -> 21.5 at 64.  More rows: `_tiles_into_norm`."""
         hidden, reader = into.hidden, into.reader
         rows, width = hidden.shape
         weight = reader.both.weight
+        if rows > 64:
+            return self._tiles_into_norm(x, project, into) if split is None else None
         if (
             self.dtype != torch.bfloat16 or not 0 < rows <= 64 or width % 128 or project.out_features != width or project.in_features % 128
             or project.weight.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or reader.activation != "silu"
@@ -918,11 +934,51 @@ class HipKernels:
         _check(status, "linear into a norm")
         return ScaledRows(scaled, sums, into.eps, reader, tiles)
 
+    def _tiles_into_norm(self, x, project: LinearWeights, into: NormInto) -> ScaledRows | None:
+        """`_linear_into_norm` for more than 64 rows, where both products are the tiled kernel's."""
+        hidden, reader = into.hidden, into.reader
+        rows, width = hidden.shape
+        both = reader.both
+        if (
+            self.dtype != torch.bfloat16 or width % 128 or project.out_features != width or both.in_features != width or reader.activation != "silu"
+            or hidden.dtype != torch.float32 or x.dtype != torch.bfloat16 or x.shape != (rows, project.in_features)
+            or into.weight.dtype not in (torch.bfloat16, torch.float32) or into.weight.shape != (width,) or not _in_pieces(hidden, into.weight)
+            or self._streaming(x, project, may_split=True) != "tiled"
+        ):
+            return None
+        scaled = self._empty((rows, width), torch.bfloat16)
+        if (
+            self._streaming(scaled, both, gated=True) != "tiled"
+            or self._gemm_blocks.llmserve_gemm_blocks_norm_cost(rows, width, project.in_features) > self._TILES_INTO_NORM
+        ):
+            return None
+        pieces = self._gemm_blocks.llmserve_gemm_blocks_norm_pieces(rows, width, project.in_features)
+        sums = self._empty((pieces, -(-rows // 4) * 4), torch.float32)
+        bias = project.bias
+        status = self._gemm_blocks.llmserve_gemm_blocks_into_norm(
+            _pointer(x), _pointer(project.weight), _pointer(bias), _is_float(bias) if bias is not None else 0, _pointer(hidden), _pointer(into.weight),
+            _is_float(into.weight), _pointer(scaled), _pointer(sums), rows, width, project.in_features, self._stream,
+        )
+        _check(status, "linear into a norm")
+        return ScaledRows(scaled, sums, into.eps, reader, -1)
+
+    # What the first product's whole sums may cost, in thousandths of a us by its estimate, for the norm's kernel.  Us in a captured chain of the output projection, norm
+    # and gate/up, apart -> linked (cost): 1.5B sizes 80 rows 26.0 -> 25.0 (2.6), 128 rows 29.1 -> 27.9 (2.6), 160 rows 31.8 -> 30.3 (1.6), 192 rows 32.1 -> 32.9 (4.2), 256 rows 35.6 ->
+    # 34.0 (2.8), 320 rows 35.8 -> 35.3 (3.2), 384 rows 41.1 -> 39.3, 640 rows 56.5 -> 53.6, 1,536 rows 107.4 -> 104.2, 2,048 rows 126.8 -> 121.7; width 2,048 96 rows 32.6 -> 33.9 (6.7);
+    # 7B sizes 96 rows 75.6 -> 89.1.
+    _TILES_INTO_NORM = 3400
+
     def _scaled_gated_linear(self, x: ScaledRows, weights: GatedLinearWeights) -> torch.Tensor:
         if weights is not x.reader:
             raise KernelError("gated_linear: the rows were left for another product")
         rows, width = x.rows.shape
         out = self._empty((rows, weights.width), self.dtype)
+        if x.tiles < 0:
+            status = self._gemm_blocks.llmserve_gemm_blocks_scaled(
+                _pointer(x.rows), _pointer(x.sums), x.sums.shape[0], x.eps, _pointer(weights.both.weight), _pointer(out), rows, 2 * weights.width, width, self._stream,
+            )
+            _check(status, "gated_linear of scaled rows")
+            return out
         status = self._gemm_bf16.llmserve_gemm_scaled(
             _pointer(x.rows), _pointer(x.sums), x.eps, _pointer(weights.both.weight), _pointer(out), x.tiles, rows, 2 * weights.width, width,
             self._stream,
@@ -1519,7 +1575,7 @@ class HipKernels:
         out, projected = self._rotate_store_attend(qkv, layout, batch, cell, inverse_frequencies, pairing, scale, window, project, sinks, chunk, out, into)
         if project is None or projected:
             return out
-        if into is not None and batch.max_query_length == 1:
+        if into is not None and ((batch.max_query_length == 1 and out.shape[0] <= 64) or self._own_steps()):
             scaled = self._linear_into_norm(out, None, project, into)
             if scaled is not None:
                 return scaled

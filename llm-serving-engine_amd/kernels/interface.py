@@ -15,7 +15,7 @@ import torch
 
 
 class Kernels(Protocol):
-    """What every library has.  Two more the parts ask for where a library has them:
+    """What every library has.  Three more the parts ask for where a library has them:
 
     `linear_rotated(x, weights, layout, batch, cell, inverse_frequencies, pairing)`: the rows that `linear(x, weights)` and `rotate_and_store`
     leave, k and v stored, or None, and nothing done, where it doesn't take the sizes.  A library that derives from one with it and has
@@ -23,7 +23,9 @@ class Kernels(Protocol):
 
     `norm_into(hidden, weight, eps, reader)`: what `rotate_store_attend` may be handed as `into`: the stream, the norm behind the product
     `project`, and the gated product that reads the normed rows.  It may then add to the stream itself and return what that `reader` alone
-    takes, instead of rows to add."""
+    takes, instead of rows to add.
+
+    `linear_into(x, project, into)`: that for rows of attention that are there already, or None, and nothing done."""
 
     device: torch.device
     dtype: torch.dtype

@@ -117,7 +117,9 @@ class Attention(Mixer):
             qkv = self.position.project_and_store(x, self.qkv, self.layout, batch, cell)
             if qkv is not None:
                 mixed = self.kernels.paged_attention(qkv, self.layout, batch, cell, self.spec.scale, self.spec.window)
-                return self.kernels.linear(mixed, self.out, out_dtype=torch.float32, partial=True)
+                linked = getattr(self.kernels, "linear_into", None) if into else None
+                scaled = linked(mixed, self.out, **into) if linked is not None else None
+                return scaled if scaled is not None else self.kernels.linear(mixed, self.out, out_dtype=torch.float32, partial=True)
         qkv = self.kernels.linear(x, self.qkv)
         # the output projection goes with the attention: a kernel library may fuse the two (key splits of
         # a decode step merged by the product that reads them)
