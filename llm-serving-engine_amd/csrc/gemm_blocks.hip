@@ -867,7 +867,7 @@ extern "C" int llmserve_gemm_blocks_norm_cost(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64 || N > 128 * SUMS_MOST) return 1 << 30;
   const int splits = llmserve_gemm_blocks_parts(M, N, K);
   const int shape = pick_norm_shape(M, N, K);
-  const float whole = shape < 2 ? 2.3f + (float)(K / 64) * (shape == 0 ? 0.19f : 0.28f) : shape_us(SHAPES[shape], M, N, K, 1, 4), parts = shape_us(SHAPES[pick_shape(M, N, K, splits, 4)], M, N, K, splits, 4);
+  const float whole = shape < 2 ? 2.3f + (float)(K / 64) * (shape == 0 ? 0.18f : 0.27f) : shape_us(SHAPES[shape], M, N, K, 1, 4), parts = shape_us(SHAPES[pick_shape(M, N, K, splits, 4)], M, N, K, splits, 4);
   return (int)(1000.f * (whole - parts));
 }
 
@@ -880,8 +880,8 @@ extern "C" int llmserve_gemm_blocks_into_norm(const void* x, const void* w, cons
   const Link link{hidden, weight, weight_is_float, (bf16_t*)rows, sums, 0.f, 0.f};
 #define BLOCK(...) return launch_block<__VA_ARGS__, float, OUT_NORM>(x, w, bias, bias_is_float, nullptr, M, N, K, 1, stream, {}, link)
   switch (pick_norm_shape(M, N, K)) {
-    case 0: BLOCK(2, 1, 1, 2, 2, 8, 1, false);
-    case 1: BLOCK(2, 1, 2, 2, 2, 8, 1, false);
+    case 0: BLOCK(2, 2, 1, 1, 1, 8, 1, false);  // (in four waves: in two 6.6 us at 96 rows of N 1,536 K 1,536 for 6.4, the next 8.8 at 320 rows for 8.6)
+    case 1: BLOCK(2, 2, 2, 1, 1, 8, 1, false);
     case 6: BLOCK(2, 2, 3, 4, 4, 5, 2, false);
     case 8: BLOCK(2, 2, 2, 4, 4, 3, 2, false);
     case 9: BLOCK(2, 2, 2, 2, 2, 5, 2, false);
@@ -908,9 +908,15 @@ extern "C" int llmserve_gemm_blocks_scaled(const void* rows, const float* sums, 
 static int launch_rotated(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,
                           hipStream_t stream, const Rotated& rotated) {
 #define BLOCK(...) return launch_block<__VA_ARGS__, bf16_t, OUT_ROTATED>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, rotated)
-  auto one_round = [&](int n, int m) { return (long)((N + n - 1) / n) * ((M + m - 1) / m) <= 256; };
+  // Of the smallest, with as many waves as a tile has: 64 x 32 in four waves for two, us at N 2,048 K 1,536: 160 rows 8.9 -> 8.3, 256 rows 9.1 -> 8.4; 32 x 64 where that makes more
+  // workgroups: 160 rows 7.6 (256 rows 8.6, as many); 32 x 32: 65 to 128 rows 8.3 -> 6.8, N 1,152 K 896 65 to 224 rows 6.8 -> 5.6; 64 x 64 in eight waves for four gains nothing.  A
+  // prompt of 77 tokens with 32 x 32 1,699 -> 1,639.
+  auto workgroups = [&](int n, int m) { return (long)((N + n - 1) / n) * ((M + m - 1) / m); };
+  auto one_round = [&](int n, int m) { return workgroups(n, m) <= 256; };
   if (K % 64) BLOCK(2, 2, 4, 4, 4, 5, 2, true);  // (a K that ends in half a stage, which the entry point takes; `_rotated_ahead` leaves it to the two kernels)
-  if (one_round(64, 32)) BLOCK(2, 1, 2, 2, 2, 5, 2, false);
+  if (one_round(32, 32)) BLOCK(1, 2, 2, 1, 1, 8, 2, false);
+  if (one_round(32, 64) && workgroups(32, 64) > workgroups(64, 32)) BLOCK(1, 4, 2, 1, 1, 8, 2, false);
+  if (one_round(64, 32)) BLOCK(2, 2, 2, 1, 1, 6, 2, false);
   if (one_round(64, 64)) BLOCK(2, 2, 2, 2, 2, 5, 2, false);
   if (one_round(128, 64)) BLOCK(2, 2, 4, 2, 2, 3, 2, false);
   BLOCK(2, 2, 4, 4, 4, 5, 2, false);
