@@ -947,10 +947,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* _
 #pragma unroll
       for (int s = 0; s < S; ++s) of_split[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], piece[s][u], of_split[s], 0, 0, 0);
 #pragma unroll
-    for (int s = 0; s < S; ++s) {  // (a split that saw no key holds whatever was there, in this row's column alone)
+    for (int s = 0; s < S; ++s) {  // (a split that saw no key holds whatever was there, in this row's column alone; one whose share is NaN, from a key of
+                                   // NaN or a score of +inf, is none of those, and reaches the row)
       const float c = share[s] * inverse;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = share[s] > 0.f ? fmaf(c, of_split[s][i], acc[i]) : acc[i];
+      for (int i = 0; i < 4; ++i) acc[i] = share[s] != 0.f ? fmaf(c, of_split[s][i], acc[i]) : acc[i];
     }
   }
   __syncthreads();  // (every wave has read its weights)
