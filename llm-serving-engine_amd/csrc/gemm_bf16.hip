@@ -975,22 +975,30 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_merged_kernel(const bf16_t* _
     if (n_first + i < N) dst[i] = total_tile[i] + bias_here[i];
 }
 
+template <int WAVES, int S, int LINK>
+static int launch_merged_as(const void* split_x, const float* split_ml, const void* w, const void* bias, int bias_is_float,
+                            float* out, int M, int N, int K, int k_splits, hipStream_t stream, Link link, int helpers, Ahead ahead) {
+  const int tiles = (N + 15) / 16;
+  hipLaunchKernelGGL((gemm_merged_kernel<WAVES, S, LINK>), dim3(tiles + helpers, k_splits), dim3(WAVES * 64), WAVES * 4096, stream,
+                     (const bf16_t*)split_x, split_ml, (const bf16_t*)w, M, N, K, K / k_splits, tiles, bias_is_float, bias, out, link, ahead);
+  return LAUNCH_STATUS();
+}
+
+// Twelve waves for whole sums over more than eight heads, a head each or two, of which a wave has 168 registers.  Eight splits of a head take 128 for x and 32 for their
+// sums (six 96 and 24): in twelve waves that went to memory and came back, and a register put away before its read of LDS has come would come back with what
+// it held before.  Those have eight waves of 256.  A pass of four steps over contexts of about 1,500, which attention leaves in eight splits, us, in twelve waves ->
+// eight: 1 row 5,640 -> 4,386, 8 rows 5,935 -> 4,710, 16 rows 6,450 -> 5,290 (twelve waves that take eight splits as two runs of four: 4,385, 4,687 and 5,290,
+// and of more than twelve heads they would make four trips to memory for two or three).
 template <int S, int LINK>
 static int launch_merged(const void* split_x, const float* split_ml, const void* w, const void* bias, int bias_is_float,
                          float* out, int M, int N, int K, int k_splits, hipStream_t stream, Link link, int helpers, Ahead ahead) {
+#define MERGED(WAVES) launch_merged_as<WAVES, S, LINK>(split_x, split_ml, w, bias, bias_is_float, out, M, N, K, k_splits, stream, link, helpers, ahead)
   const int groups = K / k_splits / (STEP * GROUP);
-  const int tiles = (N + 15) / 16;
-  const dim3 grid(tiles + helpers, k_splits);
-  if (LINK == INTO_NORM && groups > 8)  // whole sums: a head a wave, or two
-    hipLaunchKernelGGL((gemm_merged_kernel<12, S, LINK>), grid, dim3(768), 12 * 4096, stream,
-                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, M, N, K, K / k_splits, tiles, bias_is_float, bias, out, link, ahead);
-  else if (groups <= 4)
-    hipLaunchKernelGGL((gemm_merged_kernel<4, S, LINK>), grid, dim3(256), 4 * 4096, stream,
-                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, M, N, K, K / k_splits, tiles, bias_is_float, bias, out, link, ahead);
-  else
-    hipLaunchKernelGGL((gemm_merged_kernel<8, S, LINK>), grid, dim3(512), 8 * 4096, stream,
-                       (const bf16_t*)split_x, split_ml, (const bf16_t*)w, M, N, K, K / k_splits, tiles, bias_is_float, bias, out, link, ahead);
-  return LAUNCH_STATUS();
+  if constexpr (LINK == INTO_NORM && S <= 4) {
+    if (groups > 8) return MERGED(12);
+  }
+  return groups <= 4 ? MERGED(4) : MERGED(8);
+#undef MERGED
 }
 
 // out [k_splits, M, N] float32 partial sums of x . w^T (+ bias in the first), x [M, K] being the merge of

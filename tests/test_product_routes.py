@@ -70,7 +70,7 @@ def test_whole_tiles_where_they_are_ahead_of_the_other_float32_kernel(rows, oute
 
 
 @pytest.mark.parametrize("module,kernel", [("gemm_blocks", "gemm_block_kernel"), ("gemm_f32", "gemm_f32_whole_kernel"),
-                                           ("gemm_bf16", "gemm_stream_kernel"), ("gemm_bf16", "gemm_ring_kernel")])
+                                           ("gemm_bf16", "gemm_stream_kernel"), ("gemm_bf16", "gemm_ring_kernel"), ("gemm_bf16", "gemm_merged_kernel")])
 def test_kernels_that_read_ahead_keep_their_registers(module, kernel):
     """Kernels whose reads of LDS are instructions with waits of their own have no memory of a lane's: a register put away there before its read has come
     would come back with what it held before.  As the built library's own description of its kernels has it."""
