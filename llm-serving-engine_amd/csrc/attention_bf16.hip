@@ -95,6 +95,10 @@ __device__ __forceinline__ void rotate_pair(float& a, float& b, float2 cos_sin, 
   b = y;
 }
 
+// The 16-byte piece (two angles' cos and sin) that lane quarter q of a fused step loads n-th of a token's angles, n < D / 16: its queries' pairs, which are
+// neighbours or (`halves`) D / 2 apart.
+__host__ __device__ constexpr int angle_piece(int n, int q, bool halves) { return halves ? (n / 4) * 16 + q * 4 + n % 4 : (n / 2) * 8 + q * 2 + n % 2; }
+
 struct FusedDecode {          // how the kernel rotates and stores; unused unless FUSED (where its `angle_table` is [rows][D / 2] (cos, sin) of each
                               // token's angles, or null, and `slots` [rows] page * page_size + offset of each token, negative: store nothing)
   int unmerged;               // key splits are left for the reader to merge: each split's result is divided by its own
@@ -432,11 +436,11 @@ __global__ __launch_bounds__(WAVES * 64, (COLUMN_TILES > 2 || HEAD_DIM > 192 || 
   // 8q .. 8q+7 of every 32 with their partners D/2 on.  Two angles (16 bytes) a load, without a branch on the pairing.
   [[maybe_unused]] f32x4 angle[QK_STEPS * 2];
 #if HEAD_DIM % 32 == 0
-  if (FUSED) {  // (where nothing is rotated the same loads read the row itself, and their result is dropped)
+  if (FUSED) {  // (where nothing is rotated the same loads read the row itself, 4 D bytes of 6 D or more, and their result is dropped)
     const f32x4* angles = pairing != 0 ? (const f32x4*)(angle_table + (size_t)row0 * (D / 2)) : (const f32x4*)(qkv + (size_t)row0 * row_width);
-    const bool adjacent = pairing == 1;
+    const bool halves = pairing == 2;
 #pragma unroll
-    for (int n = 0; n < QK_STEPS * 2; ++n) angle[n] = angles[adjacent ? (n / 2) * 8 + q * 2 + n % 2 : (n / 4) * 16 + q * 4 + n % 4];
+    for (int n = 0; n < QK_STEPS * 2; ++n) angle[n] = angles[angle_piece(n, q, halves)];
   }
 #endif
   if (FUSED) {
@@ -1354,6 +1358,14 @@ extern "C" int llmserve_attention_can_fuse(int pairing) {
   if (pairing == 0) return 1;
   if (D % 32 != 0) return 0;
   return pairing == 1 || (pairing == 2 && D % 64 == 0);
+}
+
+// How many bytes of a token's angles its loads reach, of its row of q, k and v where nothing is rotated.
+extern "C" int llmserve_attention_angle_bytes(int pairing) {
+  int pieces = 0;
+  for (int n = 0; D % 32 == 0 && n < D / 16; ++n)
+    for (int q = 0; q < 4; ++q) pieces = max(pieces, angle_piece(n, q, pairing == 2) + 1);
+  return pieces * 16;
 }
 
 // `work` holds `tiles` items of four ints {request index in the step, first token row, first head,
