@@ -19,6 +19,9 @@
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// Loads into LDS, and of vectors, bring 16 bytes from a multiple of 16.
+static bool in_pieces(const void* a, const void* b) { return (((size_t)a | (size_t)b) & 15) == 0; }
+
 #define STEP 32   // k per MFMA
 #define GROUP 4   // MFMA steps a wave loads at once: 128 k, 256 bytes of each weight row
 
@@ -793,9 +796,8 @@ static int pick_flow_scaled(const void* rows, const void* w, void* out, int M, i
   return pick_flow<bf16_t, 1, SCALED, 8>(rows, w, nullptr, 0, out, M, N, K, 1, stream, {}, link);
 }
 
-// Loads into LDS bring 16 bytes from a multiple of 16.
 static bool flow_takes(const void* x, const void* w, int out_is_float, int gated, int M, int N, int K, int splits) {
-  return M > 0 && M <= 16 && K % splits == 0 && (K / splits) % FLOW_UNIT == 0 && !(gated && out_is_float) && (((size_t)x | (size_t)w) & 15) == 0;
+  return M > 0 && M <= 16 && K % splits == 0 && (K / splits) % FLOW_UNIT == 0 && !(gated && out_is_float) && in_pieces(x, w);
 }
 static int flow_entry(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int out_is_float, int gated, int M, int N, int K,
                       int splits, hipStream_t stream, Tail tail) {
@@ -1021,7 +1023,7 @@ extern "C" int llmserve_gemm_merged(const void* split_x, const float* split_ml, 
                                     const void* bias, int bias_is_float, float* out, int M, int N, int K,
                                     int k_splits, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 16 || K <= 0 || k_splits < 1 || K % (STEP * GROUP * k_splits)) return ERR_BAD_ARGUMENT;
+  if (M > 16 || K <= 0 || k_splits < 1 || K % (STEP * GROUP * k_splits) || !in_pieces(split_x, w)) return ERR_BAD_ARGUMENT;
   return pick_merged<NO_LINK>(split_x, split_ml, splits, w, bias, bias_is_float, out, M, N, K, k_splits, stream, Link{});
 }
 
@@ -1029,13 +1031,14 @@ static int sums_stride(int M) { return M <= 16 ? 16 : M <= 32 ? 32 : 64; }
 
 // The product (split_x null: of x; else of the merge of its key splits, as above, M <= 16) into a norm: hidden [M, N] float32 +=
 // x . w^T (+ bias); rows [M, N] bfloat16 = hidden * weight; sums float32 [N / 16, 16 rows, or 32 or 64: as many as hold M].
-// M <= 64, N a multiple of 16, K of 128.  With split_x `helpers` further workgroups bring the runs of `ahead` into the caches (common.h: Ahead).
+// M <= 64, N a multiple of 16, K of 128; every operand begins at a multiple of 16 bytes.  With split_x `helpers` further workgroups bring the runs of `ahead` into the caches (common.h: Ahead).
 extern "C" int llmserve_gemm_into_norm(const void* x, const void* split_x, const float* split_ml, int splits, const void* w, const void* bias,
                                        int bias_is_float, float* hidden, const void* weight, int weight_is_float, void* rows, float* sums,
                                        int M, int N, int K, int helpers, const void* ahead, int stripe, int stripes,
                                        hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 64 || N % 16 || K <= 0 || K % (STEP * GROUP) || (split_x && M > 16) || (!x && !split_x)) return ERR_BAD_ARGUMENT;
+  if (!in_pieces(split_x ? split_x : x, w) || !in_pieces(hidden, weight) || !in_pieces(rows, sums)) return ERR_BAD_ARGUMENT;
   if (!ahead_fits(helpers, ahead, stripe, stripes) || (helpers && !split_x)) return ERR_BAD_ARGUMENT;
   const Ahead next = {(const unsigned char*)ahead, (unsigned)stripe, (unsigned)stripes};
   const Link link{hidden, weight, weight_is_float, (bf16_t*)rows, sums, sums_stride(M), N / 16, 0.f, 0.f};
@@ -1549,6 +1552,7 @@ extern "C" int llmserve_gemm_scaled(const void* rows, float* sums, float eps, co
                                     hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 64 || K <= 0 || K % (STEP * GROUP) || N % 2 || (tiles == 0 && (M > 16 || K > FLOW_SCALED_K))) return ERR_BAD_ARGUMENT;
+  if (!in_pieces(rows, w) || !in_pieces(sums, sums)) return ERR_BAD_ARGUMENT;
   const Link link{nullptr, nullptr, 0, nullptr, sums, sums_stride(M), K / 16, 1.f / (float)K, eps};
   if (M <= 16 && K <= FLOW_SCALED_K) return pick_flow_scaled(rows, w, out, M, N, K, stream, link);
 #define SCALED_CASE(NT_, KSTEPS_)                                                                                      \

@@ -910,6 +910,9 @@ class HipKernels:
         # (what `linear` and `add_rms_norm` refuse goes on to them)
         if hidden.dtype != torch.float32 or (split is None and (x.dtype != torch.bfloat16 or x.shape != (rows, project.in_features))):
             return None
+        # (the kernels bring pieces of 16 bytes, into LDS most of them)
+        if not _in_pieces(project.weight, weight, hidden, into.weight) or (split is None and not _in_pieces(x)):
+            return None
         scaled = self._empty((rows, width), torch.bfloat16)
         route = self._streaming(scaled, reader.both, gated=True)
         if route == "ring":
