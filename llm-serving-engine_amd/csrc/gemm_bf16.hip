@@ -831,7 +831,7 @@ static int stream_entry(const void* x, const void* w, const void* bias, int bias
   if (M <= 0 || N <= 0) return 0;
   if (M > 64 || K <= 0 || splits < 1 || K % splits || (K / splits) % (STEP * GROUP) || (gated && N % 2) || gated > 1)
     return ERR_BAD_ARGUMENT;
-  if (splits > 1 && (gated || !out_is_float)) return ERR_BAD_ARGUMENT;
+  if ((splits > 1 && (gated || !out_is_float)) || !in_pieces(x, w)) return ERR_BAD_ARGUMENT;
   if (M <= 16) return flow_takes(x, w, out_is_float, gated, M, N, K, splits) ? flow_entry(x, w, bias, bias_is_float, out, out_is_float, gated, M, N, K, splits, stream, Tail{}) : ERR_BAD_ARGUMENT;
   if (gated)
     return out_is_float ? pick_stream<float, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, nt, g)
@@ -1535,7 +1535,7 @@ extern "C" int llmserve_gemm_ring(const void* x, const void* w, const void* bias
                                   int out_is_float, int gated, int M, int N, int K, int splits, int nt,
                                   hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 128 || K <= 0 || splits < 1 || K % splits || (gated && N % 2) || gated > 1) return ERR_BAD_ARGUMENT;  // (these epilogues know silu alone)
+  if (M > 128 || K <= 0 || splits < 1 || K % splits || (gated && N % 2) || gated > 1 || !in_pieces(x, w)) return ERR_BAD_ARGUMENT;  // (these epilogues know silu alone)
   if (splits > 1 && (gated || !out_is_float)) return ERR_BAD_ARGUMENT;
   if (gated)
     return out_is_float ? pick_ring<float, true>(x, w, bias, bias_is_float, out, M, N, K, 1, stream, nt)
@@ -1585,7 +1585,7 @@ static int skinny_entry(const void* x, const void* w, const void* bias, int bias
   if (splits > 1 && (gated || !out_is_float || K % splits || (K / splits) % STEP)) return ERR_BAD_ARGUMENT;
   if (flow_takes(x, w, out_is_float, gated, M, N, K, splits))
     return flow_entry(x, w, bias, bias_is_float, out, out_is_float, gated, M, N, K, splits, stream, tail);
-  if (M > 16 && !gated && K % splits == 0 && (K / splits) % (STEP * GROUP) == 0 && (long)N * K <= (1L << 22)) {
+  if (M > 16 && !gated && K % splits == 0 && (K / splits) % (STEP * GROUP) == 0 && (long)N * K <= (1L << 22) && in_pieces(x, w)) {
     // A small weight at 17 to 64 rows: two or four tiles of x beside one weight tile a workgroup, through
     // LDS.  In a captured chain over different weights, the 1.5B sizes' qkv and o: 4.8 and 4.0 us at 17
     // rows, 5.0 and 4.5 at 32, 6.0 and 5.6 at 48, 6.7 and 6.2 at 64 (the library 7.1-7.7 throughout, the

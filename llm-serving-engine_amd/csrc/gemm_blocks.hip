@@ -830,7 +830,7 @@ static int launch_shape(const void* x, const void* w, const void* bias, int bias
 #undef BLOCK
 }
 
-// x, w bfloat16; out bfloat16 or float32; any M and N, K a multiple of 32, an even N and a bfloat16 result with `gated` (silu).
+// x, w bfloat16, both from a multiple of 16 bytes on; out bfloat16 or float32; any M and N, K a multiple of 32, an even N and a bfloat16 result with `gated` (silu).
 // With splits > 1 (float32 out, not gated, K / splits a multiple of 32) `out` is [splits, M, N]
 // partial sums, the bias in the first.
 extern "C" int llmserve_gemm_blocks(const void* x, const void* w, const void* bias, int bias_is_float, void* out,
@@ -838,6 +838,7 @@ extern "C" int llmserve_gemm_blocks(const void* x, const void* w, const void* bi
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || K % 32 || (gated && N % 2) || splits < 1 || gated > 1 || (gated && out_is_float)) return ERR_BAD_ARGUMENT;  // (this epilogue knows silu alone)
   if (splits > 1 && (gated || !out_is_float || K % splits || (K / splits) % 32)) return ERR_BAD_ARGUMENT;
+  if (((size_t)x | (size_t)w) & 15) return ERR_BAD_ARGUMENT;
   if (gated) return launch_shape<bf16_t, OUT_GATED>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);
   return out_is_float ? launch_shape<float, OUT_PLAIN>(x, w, bias, bias_is_float, out, M, N, K, splits, stream)
                       : launch_shape<bf16_t, OUT_PLAIN>(x, w, bias, bias_is_float, out, M, N, K, 1, stream);

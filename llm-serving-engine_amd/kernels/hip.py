@@ -579,6 +579,15 @@ class HipKernels:
         return None
 
     @staticmethod
+    def _for_operands(streaming: str | None, x: torch.Tensor, weights: LinearWeights) -> str | None:
+        """`streaming`, unless its kernel brings 16-byte pieces of operands of which one begins inside a piece: then the kernel for up to 64 rows that loads
+        through registers, and for more rows None.  (The kernels under "skinny" that bring pieces ask for themselves, and have others behind them; rows that are
+        views none of them takes, and a launch refuses.)"""
+        if streaming not in ("ring", "tiled") or HipKernels._flows(streaming, *x.shape) or not x.is_contiguous() or _in_pieces(x, weights.weight):
+            return streaming
+        return "medium" if x.shape[0] <= 64 and weights.in_features % 128 == 0 else None
+
+    @staticmethod
     def _flows(streaming: str | None, rows: int, in_features: int) -> bool:
         """Whether a product of up to 16 rows goes to the kernel that streams whole cache lines (csrc/gemm_bf16.hip: gemm_flow), whichever of
         the others `_streaming` names: those take a K that is no multiple of 64, and more rows."""
@@ -757,7 +766,7 @@ class HipKernels:
         if inner != weights.in_features:
             raise KernelError(f"linear: x has {inner} columns, the weight {weights.in_features}")
         bias = weights.bias
-        streaming = self._streaming(x, weights, may_split=partial and out_dtype == torch.float32)
+        streaming = self._for_operands(self._streaming(x, weights, may_split=partial and out_dtype == torch.float32), x, weights)
         if self._one_row_of_tiles(x, weights, partial and out_dtype == torch.float32):
             streaming = "tiled"
         if (
@@ -1021,7 +1030,7 @@ class HipKernels:
             )
             _check(status, "gated_linear")
             return out
-        streaming = self._streaming(x, weights.both, gated=True)
+        streaming = self._for_operands(self._streaming(x, weights.both, gated=True), x, weights.both)
         if self._flows(streaming, *x.shape):
             streaming = "skinny"
         if streaming == "ring":
