@@ -812,17 +812,22 @@ static int flow_entry(const void* x, const void* w, const void* bias, int bias_i
 extern "C" int llmserve_gemm_flow_rows(int M, int N, int K, int splits) { return flow_shape(M, N, K, splits).rows_each; }
 
 // Into how many parts of K such a product is best cut when its float32 result may stay in parts, 1 to 8: by what a CU brings, and 0.12 us a part for
-// writing and adding it up (a CU brings 26 bytes a ns).  A part has two units a wave or more.
-extern "C" int llmserve_gemm_flow_parts(int M, int N, int K) {
-  const int units = K / FLOW_UNIT;
-  int best = 1;
-  double least = 0.0;
+// writing and adding it up (a CU brings 26 bytes a ns).  A part has two units a wave or more.  The same at every M, as parts decide in which order a row's
+// sums meet: by what eight rows take, and the fewest that the estimate has within 7 percent of the best.  Us with the norm that adds them up, in the parts that M itself
+// would have -> these: 1 row of N 1,152 K 6,912 (three -> four) 7.1 -> 7.2, 8 rows (six -> four) 7.8 -> 7.6; 16 rows of N 1,536 K 8,960 (five -> four) 9.8 -> 9.8; 1 row
+// of N 1,024 K 3,072 (two -> four) 5.8 -> 5.9.  By what one row takes 16 rows of N 1,024 K 2,048 go from 5.6 to 5.9, of N 2,560 K 4,096 from 8.7 to 9.0.
+extern "C" int llmserve_gemm_flow_parts(int, int N, int K) {
+  const int rows = 8, units = K / FLOW_UNIT;
+  double us[9], least = 0.0;
   for (int splits = 1; splits <= 8; ++splits) {
-    if (K % FLOW_UNIT || units % splits || (splits > 1 && units / splits < 8)) continue;
-    const double us = flow_shape(M, N, K, splits).load * (K / splits) * 2.0 / 26e3 + 0.12 * splits;
-    if (splits == 1 || us < least) least = us, best = splits;
+    us[splits] = -1.0;
+    if (splits > 1 && (K % FLOW_UNIT || units % splits || units / splits < 8)) continue;
+    us[splits] = flow_shape(rows, N, K, splits).load * (K / splits) * 2.0 / 26e3 + 0.12 * splits;
+    if (splits == 1 || us[splits] < least) least = us[splits];
   }
-  return best;
+  int splits = 1;
+  while (us[splits] < 0.0 || us[splits] > 1.07 * least) ++splits;
+  return splits;
 }
 
 // The same product as llmserve_gemm_skinny, always through gemm_flow or, beyond 16 rows, gemm_stream (tests and measurements); up to 64 rows.

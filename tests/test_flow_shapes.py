@@ -23,6 +23,13 @@ def test_rows_and_parts_are_ones_that_the_kernel_takes():
     assert library.llmserve_gemm_flow_parts(1, 1536, 8960 + 32) == 1  # (not a K of whole units: another kernel's)
 
 
+def test_parts_are_the_same_for_every_number_of_rows():
+    """Parts decide in which order a row's sums meet: a row has the same bits whatever stands beside it."""
+    library, draw = load_module("gemm_bf16"), random.Random(12)
+    for outer, inner in [(1536, 8960), (1024, 3072), (1152, 6912)] + [(draw.randint(1, 8000), 64 * draw.randint(1, 400)) for _ in range(3000)]:
+        assert len({library.llmserve_gemm_flow_parts(rows, outer, inner) for rows in range(1, 17)}) == 1, (outer, inner)
+
+
 def test_sizes_that_were_measured():
     """Workgroups that come out even on 256 CUs, or within a few percent of the best of what was measured."""
     library = load_module("gemm_bf16")

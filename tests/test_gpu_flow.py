@@ -74,6 +74,15 @@ def test_a_row_has_the_same_bits_beside_others(kernels):
             assert torch.equal(kernels.linear(x[:rows].contiguous(), weights, out_dtype=torch.float32), whole[:rows]), rows
 
 
+@pytest.mark.parametrize("outer,inner", [(1536, 8960), (1024, 3072), (1152, 6912), (2560, 4096)])
+def test_a_row_has_the_same_bits_beside_others_in_parts(kernels, outer, inner):
+    x, weights = torch.randn(16, inner, device="cuda").bfloat16(), kernels.prepare_linear([torch.randn(outer, inner, device="cuda").bfloat16()], None)
+    whole = kernels.linear(x, weights, out_dtype=torch.float32, partial=True)
+    assert whole.ndim == 3 and whole.shape[0] > 1
+    for rows in range(1, 16):
+        assert torch.equal(kernels.linear(x[:rows].contiguous(), weights, out_dtype=torch.float32, partial=True), whole[:, :rows]), rows
+
+
 @pytest.mark.parametrize("width", [2048, 2176, 4096, 4224, 8192])
 def test_scaled_rows_at_the_edges_of_the_sums(kernels, width):
     """Widths at which a thread holds another number of pieces of the rows' sums."""
