@@ -738,6 +738,10 @@ static bool flow_temporal(int N, int K) { return (long)N * K <= (1L << 22); }
 // at once, so that CUs get whole numbers of them; of more, CUs take the next as they finish.  Gate/up of the 1.5B sizes (17,920 rows) at 8 rows of x: 18 rows each, four
 // a CU at most, 10.7 us; 24, three, 10.5; 32, three, 11.8; 40, two, 10.6.  The head (151,936 rows) at 8 and 16 rows of x: 24 rows
 // each 78.5 and 93.8 us, 32 72.6 and 79.0, 40 75.5 and 83.8 (hence the 1.06 and 1.12).
+// Of 128 or more workgroups side by side, those whose weights lie 256 or 512 KB apart walk them in step and ask the same few channels of memory at a time (1.3).  Us at one row,
+// the kernels before -> 32 rows each, which they are apart -> as it is picked now: gate/up of N 57,344 K 8,192 174 -> 193 -> 147, N 24,576 K 4,096 35.1 -> 38.8 -> 32.6, a head of
+// N 128,256 K 4,096 169 -> 186 -> 161; 16 rows each of K 8,192 cost a tenth too (N 57,344 160).  Three times 256 KB costs nothing (N 40,000 K 12,288 154 at 32 rows each, 154-160
+// about it), a million bytes little (N 32,768 K 16,384 193, 180 and at 16 rows of x 180, 193).
 struct FlowShape {
   int rows_each;
   double load;  // rows of K / splits that a CU brings
@@ -752,6 +756,8 @@ static FlowShape flow_shape(int M, int N, int K, int splits) {
     const double each = rows + 0.3 * (8 * eights - rows) + M + 2.0;
     double load = workgroups <= 256L * held ? (double)((workgroups + 255) / 256) * each : (workgroups / 256.0 + 0.5) * each;
     if (eights == 5) load *= M <= 8 ? 1.06 : 1.12;
+    const long apart = 2L * rows * K;
+    if ((apart == 256 << 10 || apart == 512 << 10) && (N + rows - 1) / rows >= 128) load *= 1.3;
     if (best.rows_each == 0 || load < best.load) best = {rows, load};
   }
   return best;
