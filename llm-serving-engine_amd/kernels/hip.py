@@ -367,14 +367,26 @@ class HipKernels:
     # 1.783 -> 1.737.  The 7B sizes' qkv and o (33 and 26 MB) gain nothing from their first 8 MB.
     _WHOLE_AHEAD = 8 << 20
 
-    # Of gate and up, beside an output projection that merges key splits, whose workgroups wait more than they read: as much as it leaves time for,
-    # for each workgroup that brings (they are what the projection's leave idle), and no more than the chiplets' L2 keep until it is read: what
-    # only the memory-side cache holds comes no faster than out of memory.  A pass of four steps over 640 keys, us, with nothing and with 10, 13, 15,
-    # 18, 20, 22, 25 and 30 MB (width 1,536 of 12 heads, gate and up 52 MB, 160 workgroups bring): 1 row 4,400 4,213 4,207 4,207 4,171 4,141 4,108 4,200 4,220, 4 rows
-    # 4,390 4,297 4,297 4,304 4,261 4,236 4,205 4,299 4,340, 8 rows 4,610 4,450 4,438 4,437 4,428 4,422 4,438 4,477 4,502, 16 rows 4,830 4,668 4,665 4,676 4,676
-    # 4,678 4,692 4,685 4,724.  The same brought beside attention too, ahead of this, made steps 1 to 4 % longer.  Beside the projection that has no
-    # splits to merge 8 MB gain nothing and 16 lose 3 %.
-    _MERGING_AHEAD_EACH = 128 << 10
+    @staticmethod
+    def _merging_ahead(busy: int, in_features: int, size: int) -> int:
+        """The bytes of gate and up, `size` in all, that are brought beside an output projection of `busy` workgroups which merges key splits, and whose workgroups wait more
+        than they read: as much as it leaves time for, a workgroup that brings (they are what the projection's leave idle) and head that it merges; and no more than the
+        chiplets' L2 (32 MB) keep until it is read: what only the memory-side cache holds comes no faster than out of memory.
+
+        A pass of four steps over 640 keys and over 1,500, us, at 8 rows, with nothing and with 96, 128, 160, 192 and 256 KB a workgroup.  Width 1,536 of 12 heads, gate and up 55 MB (160
+        workgroups bring) 4,264 4,169 4,154 4,207 4,237 4,369 and 4,540 4,451 4,472 4,460 4,417 4,529; width 2,048 of 16, 67 MB (128) 5,024 4,919 4,894 4,839 4,801 4,955 and
+        5,492 5,398 5,411 5,335 5,287 5,303; width 2,560 of 12, 94 MB (96) 5,352 5,305 5,299 5,370 5,430 5,537 and 5,643 5,556 5,530 5,527 5,541 5,608; width 1,280 of 10, 39 MB (176)
+        3,812 3,768 3,689 3,771 3,841 3,807 and 4,012 4,028 3,976 3,970 3,977 3,933.  Weights that L2 holds gain by all of them, where there is time for it, with nothing and with 96, 128, 176, 192
+        and 256 KB: width 1,536 of 12, 31 MB (160: 192 KB is all) 3,702 3,628 3,612 3,674 3,562 3,558 and 3,969 3,875 3,897 3,893 3,759 3,764; width 2,048 of 16, 31 MB (128: 240) 3,983 3,900 3,896
+        3,893 3,939 3,853 and 4,404 4,343 4,349 4,344 4,334 4,223; but not width 2,560 of 12, 31 MB (96: 320) 3,838 3,833 3,827 3,936 3,953 4,107, and for width 1,152 of 9, 30 MB (184: 160)
+        it depends: 3,591 3,582 3,544 3,568 3,567 3,568 and 3,856 3,837 3,844 3,765 3,765 3,758, one row over 640 keys 3,307 with 128 and 3,348 with all.  Widths 768 to 1,024, 13 to 22 MB, are within 2 % either way, but for one row
+        of width 1,024 and 8 heads (nothing 2,944, all 3,055).  The same brought beside attention too, ahead of this, made steps 1 to 4 % longer.  Beside the projection that has no splits
+        to merge 8 MB gain nothing and 16 lose 3 %."""
+        helpers, heads = max(0, 256 - busy), in_features // 128
+        each = max(128, 11 * heads) << 10
+        if size <= 32 << 20 and 2 * size <= helpers * (33 * heads << 10):
+            return size
+        return each * helpers
 
     def _whole_ahead(self, weights: Any, rows: int, busy: int, plain: bool = False) -> tuple:
         """`plain`: the next product is one by itself (its result whole, no norm or key splits about it)."""
@@ -937,7 +949,7 @@ class HipKernels:
         ahead = 0, None, 0, 0
         if split is not None:
             each = self._gemm_bf16.llmserve_gemm_flow_rows(rows, 2 * reader.width, width, 1) if width <= _FLOW_SCALED else 16 * tiles
-            ahead = self._ahead(reader.both, width // 16, self._MERGING_AHEAD_EACH * max(0, 256 - width // 16), each)
+            ahead = self._ahead(reader.both, width // 16, self._merging_ahead(width // 16, project.in_features, weight.numel() * weight.element_size()), each)
         status = self._gemm_bf16.llmserve_gemm_into_norm(
             _pointer(x) if split is None else None, _pointer(split_x), _pointer(split_ml), splits, _pointer(project.weight), _pointer(bias),
             _is_float(bias) if bias is not None else 0, _pointer(hidden), _pointer(into.weight), _is_float(into.weight), _pointer(scaled),
