@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 import types
 from dataclasses import dataclass
 from typing import Any
@@ -48,7 +49,10 @@ def _pointer(tensor: torch.Tensor | None) -> int | None:
 
 def _in_pieces(*tensors: torch.Tensor) -> bool:
     """Whether rows can be read in 16-byte pieces: contiguous tensors that begin at one (rows of a whole number of pieces)."""
-    return all(tensor.is_contiguous() and tensor.data_ptr() % 16 == 0 for tensor in tensors)
+    for tensor in tensors:  # (a loop: a generator costs the host as much again, twice a layer of a step that is launched kernel by kernel)
+        if tensor.data_ptr() % 16 or not tensor.is_contiguous():
+            return False
+    return True
 
 
 # Argument types of every entry point: p pointer, i int, f float.  Declared once, so that a call
@@ -220,6 +224,15 @@ class ScaledRows:
     eps: float
     reader: GatedLinearWeights
     tiles: int
+
+
+@functools.lru_cache(maxsize=4096)
+def _norm_pieces(blocks, rows: int, width: int, in_features: int, gated: int, most: int) -> int:
+    """How many pieces of squares a row the product of more than 64 rows into a norm leaves, where both products are the tiled kernel's (`HipKernels._tiled_ahead`) and the
+    first's whole sums cost no more than `most`; else 0."""
+    if width % 128 or not HipKernels._tiled_ahead(rows, width, in_features, False, True) or not HipKernels._tiled_ahead(rows, gated, width, True, False):
+        return 0
+    return blocks.llmserve_gemm_blocks_norm_pieces(rows, width, in_features) if blocks.llmserve_gemm_blocks_norm_cost(rows, width, in_features) <= most else 0
 
 
 class HipKernels:
@@ -539,27 +552,28 @@ class HipKernels:
         "ring" (17 to 64 rows of a middling weight, both operands through a ring of stages in LDS),
         "medium" (up to 64, x shared through LDS), "tiled" (any number, both operands through LDS),
         or None (the BLAS library, or the generic kernel)."""
-        if x.dtype != torch.bfloat16 or weights.weight.dtype != torch.bfloat16:
+        weight = weights.weight
+        if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
             return None
-        rows, inner = x.shape[0], weights.in_features
-        size = weights.out_features * inner
+        rows, (outer, inner) = x.shape[0], weight.shape
+        size = outer * inner
         if self.ring_products and rows <= 16 and inner % 128 == 0 and size > (1 << 22):
             # (Products of up to 16 rows with a K of whole units go to `_flows`' kernel, whichever name they get here; what the name still says is
             # how rows that a norm has left scaled, longer than that kernel's, are read.)
             heavy = size > (1 << 26) or (may_split and size > (1 << 24))
             if rows >= (self.ring_rows_from if heavy else max(12, self.ring_rows_from)) and (heavy or may_split or size > (1 << 24)):
-                if self._ring_shape(rows, weights.out_features, inner, may_split)[2] == 1:
+                if self._ring_shape(rows, outer, inner, may_split)[2] == 1:
                     return "ring"
         if 0 < rows <= 16 and inner % 32 == 0:
             return "skinny"
         if self.ring_products and 16 < rows <= 64 and inner % 128 == 0 and size > (1 << 22) and (
-            size <= 150_000_000 or weights.out_features <= 256 * 14 * 16
+            size <= 150_000_000 or outer <= 256 * 14 * 16
         ):
             # (a smaller weight: the kernels below; a larger one only while fourteen tiles a workgroup make one round of
             # workgroups: the 32B sizes' gate/up 100-110 us at the library, 98-106 here, 113-177 in several rounds; the 1.5B
             # sizes' head, 9,496 tiles, 108-120 against 101-165)
             return "ring"
-        if rows > 64 and HipKernels._tiled_ahead(rows, weights.out_features, inner, gated, may_split) and _in_pieces(x, weights.weight):
+        if rows > 64 and HipKernels._tiled_ahead(rows, outer, inner, gated, may_split) and _in_pieces(x, weight):
             return "tiled"
         if self.ring_products and 64 < rows <= 128 and inner % 128 == 0 and (
             (may_split and (1 << 20) < size <= 150_000_000) or (gated and (1 << 22) < size <= 150_000_000)
@@ -570,7 +584,7 @@ class HipKernels:
             # workgroups, 67.1 / 72.1 -> 60.2 / 60.4 (80-82 with five, which make 474); the library keeps qkv (7.5 against 10.2;
             # 19-23 against 21-23).
             return "ring"
-        if self.library_products and (rows > 64 or self._for_replay or weights.out_features * inner > 150_000_000):
+        if self.library_products and (rows > 64 or self._for_replay or size > 150_000_000):
             # On the device the library is ahead of "medium" as it stands, so a captured step (which
             # costs the host nothing per launch) takes the library; a step launched kernel by kernel
             # is bound by the host, where a torch call costs four times one of ours (but a weight beyond what the
@@ -579,25 +593,25 @@ class HipKernels:
             # captured chain: 7.1-7.7 us each, against 4.8 and 4.0 at 17 rows, 5.0 and 4.5 at 32, 6.7 and 6.2 at
             # 64 for the kernel that brings two or four tiles of x through LDS beside a weight tile; where K is
             # no multiple of 128 an older kernel takes up to 32 rows).
-            if not gated and inner % 32 == 0 and weights.out_features * inner <= (1 << 22) and (rows <= 32 or (rows <= 64 and inner % 128 == 0)):
+            if not gated and inner % 32 == 0 and size <= (1 << 22) and (rows <= 32 or (rows <= 64 and inner % 128 == 0)):
                 return "skinny"
             return None
         if 16 < rows <= 64 and inner % 128 == 0:
             return "medium"
         if 16 < rows <= 64 and inner % 32 == 0:
             return "skinny"
-        if rows > 64 and inner % 32 == 0:
+        if rows > 64 and inner % 32 == 0 and _in_pieces(x, weight):
             return "tiled"
         return None
 
     @staticmethod
-    def _for_operands(streaming: str | None, x: torch.Tensor, weights: LinearWeights) -> str | None:
-        """`streaming`, unless its kernel brings 16-byte pieces of operands of which one begins inside a piece: then the kernel for up to 64 rows that loads
-        through registers, and for more rows None.  (The kernels under "skinny" that bring pieces ask for themselves, and have others behind them; rows that are
-        views none of them takes, and a launch refuses.)"""
-        if streaming not in ("ring", "tiled") or HipKernels._flows(streaming, *x.shape) or not x.is_contiguous() or _in_pieces(x, weights.weight):
-            return streaming
-        return "medium" if x.shape[0] <= 64 and weights.in_features % 128 == 0 else None
+    def _instead_of_ring(x: torch.Tensor, weights: LinearWeights) -> str | None:
+        """The ring brings 16-byte pieces: "ring", or where an operand begins inside one the kernel for up to 64 rows that loads through registers, and for more rows
+        None.  (The kernels under "skinny" that bring pieces ask for themselves, and have others behind them; rows that are views none of them takes, and
+        a launch refuses.)"""
+        if HipKernels._flows("ring", *x.shape) or not x.is_contiguous() or _in_pieces(x, weights.weight):
+            return "ring"
+        return "medium" if x.shape[0] <= 64 else None
 
     @staticmethod
     def _flows(streaming: str | None, rows: int, in_features: int) -> bool:
@@ -775,11 +789,14 @@ class HipKernels:
         """`partial` allows a float32 result to come back as [parts, T, N] partial sums that
         the reader adds up in order (`add_rms_norm` and `gather_rows` do)."""
         rows, inner = x.shape
-        if inner != weights.in_features:
-            raise KernelError(f"linear: x has {inner} columns, the weight {weights.in_features}")
+        outer, depth = weights.weight.shape
+        if inner != depth:
+            raise KernelError(f"linear: x has {inner} columns, the weight {depth}")
         bias = weights.bias
-        streaming = self._for_operands(self._streaming(x, weights, may_split=partial and out_dtype == torch.float32), x, weights)
-        if self._one_row_of_tiles(x, weights, partial and out_dtype == torch.float32):
+        streaming = self._streaming(x, weights, may_split=partial and out_dtype == torch.float32)
+        if streaming == "ring":
+            streaming = self._instead_of_ring(x, weights)
+        if 16 < rows <= 128 and self._one_row_of_tiles(x, weights, partial and out_dtype == torch.float32):
             streaming = "tiled"
         if (
             streaming is None
@@ -790,14 +807,14 @@ class HipKernels:
             and weights.weight.dtype == torch.bfloat16
             and 16 < rows <= 64
             and inner % 128 == 0
-            and self._partial_splits(weights.out_features, inner) >= 4
+            and self._partial_splits(outer, inner) >= 4
         ):
             # a long K over few weight rows (the down projection): cut over K into partial sums, the
             # hand-written kernel is ahead of the library (16 against 25 us at 64 rows of the 1.5B sizes)
             streaming = "medium"
         if streaming is None and self._library(x, weights):
             if (out_dtype or self.dtype) == torch.float32:  # float32 straight from the accumulators
-                cuts = self._library_splits(rows, weights.out_features, inner) if partial else 1
+                cuts = self._library_splits(rows, outer, inner) if partial else 1
                 if cuts > 1:
                     # The library does not cut a long K over workgroups by itself (the down projection of the 7B
                     # sizes at 2,048 rows: 342 us in one piece, 217 in two; at 136 rows 103 and 43 in eight).  As a
@@ -805,7 +822,7 @@ class HipKernels:
                     # (Over the weight's transpose, which lies in such slices whatever `cuts` is: as fast as over views of
                     # the weight itself, 62.5 us against 61.8 at 2,048 rows of K 10,496 x N 1,536, where one piece takes 82.)
                     slices = x.view(rows, cuts, inner // cuts).transpose(0, 1)
-                    weight_slices = weights.transposed.view(cuts, inner // cuts, weights.out_features)
+                    weight_slices = weights.transposed.view(cuts, inner // cuts, outer)
                     parts = torch.bmm(slices, weight_slices, out_dtype=torch.float32)
                     if bias is not None:
                         parts[0].add_(weights.float_bias)
@@ -818,59 +835,59 @@ class HipKernels:
         bias_is_float = _is_float(bias) if bias is not None else 0
         if streaming is not None:
             splits = 1
-            if self._flows(streaming, rows, inner):
+            if rows <= 16 and self._flows(streaming, rows, inner):
                 if partial and out_dtype == torch.float32:
-                    splits = self._gemm_bf16.llmserve_gemm_flow_parts(rows, weights.out_features, inner)
+                    splits = self._gemm_bf16.llmserve_gemm_flow_parts(rows, outer, inner)
                 streaming = "flow"
             if streaming == "ring":
-                tiles, splits, _ = self._ring_shape(rows, weights.out_features, inner, partial and out_dtype == torch.float32)
-                out = self._empty((rows, weights.out_features) if splits == 1 else (splits, rows, weights.out_features), out_dtype or self.dtype)
+                tiles, splits, _ = self._ring_shape(rows, outer, inner, partial and out_dtype == torch.float32)
+                out = self._empty((rows, outer) if splits == 1 else (splits, rows, outer), out_dtype or self.dtype)
                 status = self._gemm_bf16.llmserve_gemm_ring(
                     _pointer(x), _pointer(weights.weight), _pointer(bias), bias_is_float, _pointer(out), _is_float(out), 0,
-                    rows, weights.out_features, inner, splits, tiles, self._stream,
+                    rows, outer, inner, splits, tiles, self._stream,
                 )
                 _check(status, "linear")
                 return out
             if streaming != "flow" and partial and out_dtype == torch.float32:
                 if streaming == "tiled":
-                    splits = self._gemm_blocks.llmserve_gemm_blocks_parts(rows, weights.out_features, inner)
+                    splits = self._gemm_blocks.llmserve_gemm_blocks_parts(rows, outer, inner)
                 elif streaming == "medium":
-                    splits = self._medium_splits(weights.out_features, inner)
-                elif rows > 16 and weights.out_features * inner <= (1 << 22) and inner % 256 == 0:
+                    splits = self._medium_splits(outer, inner)
+                elif rows > 16 and outer * inner <= (1 << 22) and inner % 256 == 0:
                     splits = 2  # what the kernel for a small weight at 17 to 64 rows does best with
                 else:
-                    splits = self._partial_splits(weights.out_features, inner)
-            shape = (rows, weights.out_features) if splits == 1 else (splits, rows, weights.out_features)
+                    splits = self._partial_splits(outer, inner)
+            shape = (rows, outer) if splits == 1 else (splits, rows, outer)
             out = self._empty(shape, out_dtype or self.dtype)
             if streaming == "tiled":
                 status = self._gemm_blocks.llmserve_gemm_blocks(
                     _pointer(x), _pointer(weights.weight), _pointer(bias), bias_is_float, _pointer(out),
-                    _is_float(out), 0, rows, weights.out_features, inner, splits, self._stream,
+                    _is_float(out), 0, rows, outer, inner, splits, self._stream,
                 )
             else:
                 entry = self._gemm_bf16.llmserve_gemm_skinny if streaming in ("skinny", "flow") else self._gemm_bf16.llmserve_gemm_medium
                 status = entry(
                     _pointer(x), _pointer(weights.weight), _pointer(bias), bias_is_float, _pointer(out),
-                    _is_float(out), 0, rows, weights.out_features, inner, splits, self._stream,
+                    _is_float(out), 0, rows, outer, inner, splits, self._stream,
                 )
             _check(status, "linear")
             return out
         if self._all_float32(x, weights) and (out_dtype or self.dtype) == torch.float32:
             splits = 1
             if partial and out_dtype == torch.float32:
-                splits = self._float32_splits(rows, weights.out_features, inner, _in_pieces(x, weights.weight))
-            shape = (rows, weights.out_features) if splits == 1 else (splits, rows, weights.out_features)
+                splits = self._float32_splits(rows, outer, inner, _in_pieces(x, weights.weight))
+            shape = (rows, outer) if splits == 1 else (splits, rows, outer)
             out = self._empty(shape, torch.float32)
             status = self._gemm_f32.llmserve_gemm_f32(
-                _pointer(x), _pointer(weights.weight), _pointer(bias), _pointer(out), 0, rows, weights.out_features,
+                _pointer(x), _pointer(weights.weight), _pointer(bias), _pointer(out), 0, rows, outer,
                 inner, splits, self._stream,
             )
             _check(status, "linear")
             return out
-        out = self._empty((rows, weights.out_features), out_dtype or self.dtype)
+        out = self._empty((rows, outer), out_dtype or self.dtype)
         status = self._gemm_generic.llmserve_gemm_generic(
             _pointer(x), _is_float(x), _pointer(weights.weight), _is_float(weights.weight), _pointer(bias),
-            bias_is_float, _pointer(out), _is_float(out), rows, weights.out_features, inner, self._stream,
+            bias_is_float, _pointer(out), _is_float(out), rows, outer, inner, self._stream,
         )
         _check(status, "linear")
         return out
@@ -908,7 +925,7 @@ class HipKernels:
 
     def linear_into(self, x, project: LinearWeights, into: NormInto) -> ScaledRows | None:
         """`linear(x, project)` added to the stream and left for the norm's reader, where both products take it; else None, and nothing done."""
-        return self._linear_into_norm(x, None, project, into) if self._own_steps() else None
+        return self._linear_into_norm(x, None, project, into) if x.shape[0] > 64 or self._own_steps() else None
 
     def _linear_into_norm(self, x, split: tuple | None, project: LinearWeights, into: NormInto) -> ScaledRows | None:
         """`into.hidden += linear(x, project)` (or of the merge of key splits: `split` is what the attention left) and the rows that
@@ -962,26 +979,24 @@ class HipKernels:
         """`_linear_into_norm` for more than 64 rows, where both products are the tiled kernel's."""
         hidden, reader = into.hidden, into.reader
         rows, width = hidden.shape
-        both = reader.both
+        inner = project.weight.shape[1]
+        # (the sizes first, and once for each: a step of more than 512 tokens is launched kernel by kernel, and what is asked in vain here is the host's
+        # time a layer: whole prompts of 513 tokens of a model of width 1,536 3,450 -> 3,740 us with 12 us of questions)
+        if self.dtype != torch.bfloat16 or not (pieces := _norm_pieces(self._gemm_blocks, rows, width, inner, 2 * reader.width, self._TILES_INTO_NORM)):
+            return None
         if (
-            self.dtype != torch.bfloat16 or width % 128 or project.out_features != width or both.in_features != width or reader.activation != "silu"
-            or hidden.dtype != torch.float32 or x.dtype != torch.bfloat16 or x.shape != (rows, project.in_features)
-            or into.weight.dtype not in (torch.bfloat16, torch.float32) or into.weight.shape != (width,) or not _in_pieces(hidden, into.weight)
-            or self._streaming(x, project, may_split=True) != "tiled"
+            not self._own_steps() or project.weight.shape[0] != width or (both := reader.both).weight.shape[1] != width or reader.activation != "silu" or project.weight.dtype != torch.bfloat16
+            or both.weight.dtype != torch.bfloat16 or hidden.dtype != torch.float32 or x.dtype != torch.bfloat16 or x.shape != (rows, inner)
+            or into.weight.dtype not in (torch.bfloat16, torch.float32) or into.weight.shape != (width,)
+            or not _in_pieces(x, project.weight, both.weight, hidden, into.weight)
         ):
             return None
         scaled = self._empty((rows, width), torch.bfloat16)
-        if (
-            self._streaming(scaled, both, gated=True) != "tiled"
-            or self._gemm_blocks.llmserve_gemm_blocks_norm_cost(rows, width, project.in_features) > self._TILES_INTO_NORM
-        ):
-            return None
-        pieces = self._gemm_blocks.llmserve_gemm_blocks_norm_pieces(rows, width, project.in_features)
         sums = self._empty((pieces, -(-rows // 4) * 4), torch.float32)
         bias = project.bias
         status = self._gemm_blocks.llmserve_gemm_blocks_into_norm(
             _pointer(x), _pointer(project.weight), _pointer(bias), _is_float(bias) if bias is not None else 0, _pointer(hidden), _pointer(into.weight),
-            _is_float(into.weight), _pointer(scaled), _pointer(sums), rows, width, project.in_features, self._stream,
+            _is_float(into.weight), _pointer(scaled), _pointer(sums), rows, width, inner, self._stream,
         )
         _check(status, "linear into a norm")
         return ScaledRows(scaled, sums, into.eps, reader, -1)
@@ -1042,9 +1057,9 @@ class HipKernels:
             )
             _check(status, "gated_linear")
             return out
-        streaming = self._for_operands(self._streaming(x, weights.both, gated=True), x, weights.both)
-        if self._flows(streaming, *x.shape):
-            streaming = "skinny"
+        streaming = self._streaming(x, weights.both, gated=True)
+        if streaming == "ring":
+            streaming = "skinny" if self._flows(streaming, *x.shape) else self._instead_of_ring(x, weights.both)
         if streaming == "ring":
             tiles, _, _ = self._ring_shape(x.shape[0], 2 * weights.width, x.shape[1], False)
             status = self._gemm_bf16.llmserve_gemm_ring(
@@ -1599,7 +1614,7 @@ class HipKernels:
         out, projected = self._rotate_store_attend(qkv, layout, batch, cell, inverse_frequencies, pairing, scale, window, project, sinks, chunk, out, into)
         if project is None or projected:
             return out
-        if into is not None and ((batch.max_query_length == 1 and out.shape[0] <= 64) or self._own_steps()):
+        if into is not None and (batch.max_query_length == 1 or out.shape[0] > 64 or self._own_steps()):
             scaled = self._linear_into_norm(out, None, project, into)
             if scaled is not None:
                 return scaled

@@ -1,4 +1,4 @@
-"""Operands that begin inside a piece of 16 bytes: kernels that bring pieces into LDS do not take them (`HipKernels._for_operands`)."""
+"""Operands that begin inside a piece of 16 bytes: kernels that bring pieces into LDS do not take them (`HipKernels._instead_of_ring`)."""
 
 from __future__ import annotations
 
