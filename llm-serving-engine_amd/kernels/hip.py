@@ -923,16 +923,21 @@ class HipKernels:
         """Whether the steps that a product into a norm stands for are this library's (one derived from it that has its own is asked for them)."""
         return all(getattr(type(self), step) is getattr(HipKernels, step) for step in ("linear", "add_rms_norm", "gated_linear", "rotate_store_attend"))
 
+    def _links_beside_portions(self, rows: int, project: LinearWeights) -> bool:
+        """Whether a step that is not of single tokens alone goes on to `_linear_into_norm`.  Of 33 to 64 rows its first product's sums are whole over a K of up to
+        1,536: a step more than that is longer linked than with parts and the norm's kernel (us a pass at 64 rows, apart -> linked: N 1,024 K 2,048 5,501 -> 5,621, N = K = 2,048 6,490 ->
+        6,582, N = K = 1,792 5,835 -> 5,937; N = K = 1,536 6,854 -> 6,865, N 2,560 K 1,536 6,589 -> 6,446; at 24 rows N 1,024 K 2,048 4,906 -> 4,795, N = K = 2,048 5,762 -> 5,705)."""
+        return rows > 64 or ((rows <= 32 or project.in_features <= 1536) and self._own_steps())
+
     def linear_into(self, x, project: LinearWeights, into: NormInto) -> ScaledRows | None:
         """`linear(x, project)` added to the stream and left for the norm's reader, where both products take it; else None, and nothing done."""
-        return self._linear_into_norm(x, None, project, into) if x.shape[0] > 64 or self._own_steps() else None
+        return self._linear_into_norm(x, None, project, into) if self._links_beside_portions(x.shape[0], project) else None
 
     def _linear_into_norm(self, x, split: tuple | None, project: LinearWeights, into: NormInto) -> ScaledRows | None:
         """`into.hidden += linear(x, project)` (or of the merge of key splits: `split` is what the attention left) and the rows that
         `into.reader` reads, where both products are of the kernels that do a norm between them; else None, and nothing done.
         Up to 64 rows: those of the kernels for a few rows, the first with whole sums over K (the 1.5B sizes' output projection
-        costs 1.6 us more than in three parts, at 64 rows 2.7; the norm's kernel 4.4 and 4.7).  In steps with portions too: the three in a captured chain 19.4 -> 18.2 us at 24 rows,
-        23.0 -> 21.5 at 64.  More rows: `_tiles_into_norm`."""
+        costs 1.6 us more than in three parts, at 64 rows 2.7; the norm's kernel 4.4 and 4.7).  In steps with portions too (`_links_beside_portions`).  More rows: `_tiles_into_norm`."""
         hidden, reader = into.hidden, into.reader
         rows, width = hidden.shape
         weight = reader.both.weight
@@ -1614,7 +1619,7 @@ class HipKernels:
         out, projected = self._rotate_store_attend(qkv, layout, batch, cell, inverse_frequencies, pairing, scale, window, project, sinks, chunk, out, into)
         if project is None or projected:
             return out
-        if into is not None and (batch.max_query_length == 1 or out.shape[0] > 64 or self._own_steps()):
+        if into is not None and (batch.max_query_length == 1 or self._links_beside_portions(out.shape[0], project)):
             scaled = self._linear_into_norm(out, None, project, into)
             if scaled is not None:
                 return scaled

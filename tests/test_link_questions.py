@@ -49,3 +49,16 @@ def test_answers_are_those_of_the_routes_apart():
                 pieces = _norm_pieces(library, rows, width, inner, gated, most)
                 assert bool(pieces) == (both and library.llmserve_gemm_blocks_norm_cost(rows, width, inner) <= most)
                 assert pieces in (0, library.llmserve_gemm_blocks_norm_pieces(rows, width, inner))
+
+
+@pytest.mark.parametrize("rows,inner,taken", [(24, 2048, True), (32, 2048, True), (33, 2048, False), (64, 1664, False), (64, 1536, True), (40, 1280, True), (96, 1536, True)])
+def test_steps_with_portions(rows, inner, taken):
+    """Both sides of the line that `_links_beside_portions` draws; a step of single tokens links at these sizes of up to 64 rows whatever K."""
+    kernels = on_the_host(_gemm_blocks=Blocks())
+    width, gated = 1536, 8960
+    project, weight = LinearWeights(torch.empty(width, inner, dtype=torch.bfloat16), None), torch.ones(width)
+    reader = kernels.prepare_gated_linear(*(torch.empty(gated, width, dtype=torch.bfloat16) for _ in range(2)))
+    into = kernels.norm_into(torch.empty(rows, width), weight, 1e-6, reader)
+    x = torch.empty(rows, inner, dtype=torch.bfloat16)
+    assert (kernels.linear_into(x, project, into) is not None) == taken
+    assert rows > 64 or kernels._linear_into_norm(x, None, project, into) is not None
