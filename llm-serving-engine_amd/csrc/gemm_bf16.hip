@@ -537,8 +537,10 @@ constexpr size_t flow_lds_bytes(int eights, int x_eights) {
 }
 
 // TEMPORAL: the weight is small, and may have been brought into the caches.  SUMS (SCALED): pieces of four sums a thread holds.
+// (On a page of its own: which kernels of a step share one, and which lie across two, otherwise hangs on all that the library holds before them.  With seven instances of
+// another kernel gone, which no step launches, a pass of 8 rows took 6,200 -> 6,250 us over 8,192 keys and 5,156 -> 5,199 over 3,000; on pages 6,213 and 5,155.)
 template <int NH, int XH, bool TEMPORAL, typename TO, int GATED, int LINK, int SUMS>
-__global__ __launch_bounds__(256) void gemm_flow_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int M, int N, int K, int k_split,
+__global__ __attribute__((aligned(4096))) __launch_bounds__(256) void gemm_flow_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int M, int N, int K, int k_split,
                                                         int rows_each, int bias_is_float, const void* __restrict__ bias, TO* __restrict__ out, Tail tail,
                                                         Link link) {
   extern __shared__ __attribute__((aligned(16))) unsigned char flow_lds[];
