@@ -1,8 +1,10 @@
 // bfloat16 products on the matrix cores (MFMA), float32 accumulation.
 //
-// gemm_skinny: out[M, N] = x[M, K] . w[N, K]^T (+ bias) for M <= 64, the shape of decoding.
-// Such a product is a stream of the weight matrix from HBM, so the kernel is built around
-// that stream: a workgroup owns 16 weight rows and its waves split K between them; every
+// Up to 16 rows of x, the shape of decoding, are gemm_flow's below, 17 to 128 gemm_stream's, gemm_medium's and gemm_ring's.
+//
+// gemm_skinny: out[M, N] = x[M, K] . w[N, K]^T (+ bias) for M <= 64 at the sizes and operands that those do not take: a K that is no multiple of 64 (up to 16
+// rows) or 128, and operands that begin inside a piece of 16 bytes.  Such a product is a stream of the weight matrix from HBM:
+// a workgroup owns 16 weight rows and its waves split K between them; every
 // lane keeps two groups of four 16-byte loads of its weight row in flight; the weights go
 // straight from global memory into the A operand of v_mfma_f32_16x16x32_bf16 (lane l holds
 // row l % 16, k = (l / 16) * 8 .. + 8 of a 32-wide step), the few activation rows into the B
@@ -26,7 +28,7 @@ static bool in_pieces(const void* a, const void* b) { return (((size_t)a | (size
 #define GROUP 4   // MFMA steps a wave loads at once: 128 k, 256 bytes of each weight row
 
 __device__ __forceinline__ bf16x8 load8(const bf16_t* p) { return *(const bf16x8*)p; }
-// The weight stream uses plain loads: non-temporal ones were measured 8-12 % slower here.
+// (Plain loads: a load here takes half a cache line of sixteen rows, the next the other half; past the caches they were 8-12 % slower.  gemm_flow takes whole lines, and past them.)
 __device__ __forceinline__ bf16x8 load8_stream(const bf16_t* p) { return *(const bf16x8*)p; }
 #ifndef TARGET_WAVES
 #define TARGET_WAVES 2048
@@ -59,15 +61,14 @@ __device__ __forceinline__ float gate_value(float gate) {
   return GATED == 2 ? fmaxf(gate, 0.f) : gate / (1.f + expf(-gate));
 }
 
-// Two products with a norm between them, without a kernel for the norm (steps of up to 64 single tokens).  The first one
+// Two products with a norm between them, without a kernel for the norm (up to 64 rows).  The first one
 // (INTO_NORM) holds whole sums over K, adds them to the residual stream in its epilogue, and writes what the second reads:
 // x * weight in bfloat16, not yet divided by the row's root mean square, and each tile's sum of squares of x a row.  The second
 // one (SCALED) multiplies its float32 results by rsqrt(mean of squares + eps), which is the same for all of a row's
 // products: rounding x * weight loses what rounding the normed row loses.  A norm's kernel is a launch, two trips to
-// memory and a sum over a workgroup: 4.4 us of a layer's 46 at the 1.5B sizes, whatever the rows.  Against that the first product
-// needs whole sums over K (with key splits to merge 6.6 -> 8.2 us: 96 workgroups read what 288 did; 7B sizes 7.3 -> 7.7) and the second one
-// brings the sums of squares (gate/up 11.7 -> 12.8 us at one row, 13.4 -> 13.9 at eight; 7B sizes 47.5 -> 48.7).  A decode step, ms, before -> after: 1.5B
-// sizes 1 row 1.320 -> 1.301, 8 rows 1.430 -> 1.409 (contexts of 8,192: 1.822 -> 1.765), 64 rows 2.045 -> 2.030; 7B sizes 8 rows 3.303 -> 3.206.
+// memory and a sum over a workgroup, 4 to 5 us whatever the rows.  Against that the first product needs whole sums over K, and the second one brings the sums of
+// squares.  A pass of four steps, us, the three apart -> linked: 1.5B sizes 1 row 4,130 -> 3,899, 8 rows 4,406 -> 4,160 (contexts of 4,000: 5,460 -> 5,166), 16 rows 4,666 -> 4,440, 64
+// rows 6,182 -> 6,059; 7B sizes 1 row 10,478 -> 10,187, 8 rows 10,773 -> 10,496, 16 rows 11,783 -> 11,597, 64 rows (no link there) 14,187.
 enum { NO_LINK = 0, INTO_NORM = 1, SCALED = 2 };
 struct Link {
   float* hidden;             // INTO_NORM: [M, N], added to in place

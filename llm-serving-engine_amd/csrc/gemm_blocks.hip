@@ -64,7 +64,7 @@ constexpr bool is_gated(int out) { return out == OUT_GATED || out == OUT_SCALED;
 // K, adds them to the residual stream, and writes x * weight in bfloat16, not yet divided by the row's root mean square, with the sum of squares of each tile's
 // columns a row.  The second (OUT_SCALED) adds those up and multiplies its float32 results by rsqrt(mean + eps): rounding
 // x * weight loses what rounding the normed row loses.  A norm's kernel takes 5 us of a step of 96 to 320 rows and 11 of 2,048; against that the first needs whole sums (us in a
-// step, before -> after: 96 rows of N 1,536 K 1,536 5.4 -> 6.9, 320 rows 6.5 -> 9.2, 2,048 rows 17.4 -> 21.2 with the stream's way) and the second the squares (17.9 -> 19.3,
+// step, before -> after: 96 rows of N 1,536 K 1,536 5.4 -> 6.4, 320 rows 6.5 -> 8.6, 2,048 rows 17.4 -> 21.2 with the stream's way) and the second the squares (17.9 -> 19.3,
 // 24.6 -> 25.7, 98 -> 98).  A pass: prompt 77 1,714 -> 1,699 us, mixed 31 + 256 9,914 -> 9,790, prompt 2,048 by 1.5 percent.
 struct Link {
   float* hidden;             // OUT_NORM: [M, N], added to in place
@@ -444,8 +444,9 @@ struct Reads {
 // SIMD is to hold; AHEAD: see Reads.
 // ONCE: no other workgroup reads these weights.  They then go past the caches: what a CU has under way of memory is limited (32 KB or so), a line that is kept
 // nowhere takes less of it (measured with nothing but the loads: 112 CUs take 44 bytes a ns each, past the caches 47 to 53), and x keeps its place in
-// L2.  Us, before -> after: 96 rows of N 17,920 K 1,536 18.3 -> 17.3, of N 1,536 K 8,960 in parts 11.6 -> 10.1, of N 37,888 K 3,584 60.1 -> 51.6; 160 rows 21.9 -> 21.2,
-// of N 37,888 59.5 -> 54.4.  With a second tile of rows the other workgroup would find them gone: 320 rows of N 1,536 K 8,960 18.1 -> 21.1.
+// L2.  Us, through them -> past them: 96 rows of N 17,920 K 1,536 17.7 -> 17.2, of N 37,888 K 3,584 56.8 -> 52.2; 160 rows 21.9 -> 21.2,
+// of N 5,120 K 27,648 in parts 96 rows 63 -> 58.  (In parts shorter than 24 stages the product gains 1 to 5 percent and the norm that adds them up, alone behind it, loses more; whole
+// prompts of 65 to 128 tokens are no longer for it, and at widths 1,536 to 2,560 up to 1 percent shorter.)  With a second tile of rows the other workgroup would find them gone: 320 rows of N 1,536 K 8,960 18.1 -> 21.1.
 template <int WN, int WM, int TN, int TM, int AHEAD, int STAGES, int A_SIMD, bool HALF, typename TO, int OUT, bool ONCE>
 __global__ __launch_bounds__(WN * WM * 64, A_SIMD) void gemm_block_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                           const void* __restrict__ bias, int bias_is_float,
@@ -862,8 +863,8 @@ extern "C" int llmserve_gemm_blocks_norm_pieces(int M, int N, int K) {
   return (N + columns - 1) / columns;
 }
 
-// What the whole sums cost it, in thousandths of a us: its own time (of the two smallest tiles as measured in a step: K 1,536 of N 1,536 6.9 us at 96 rows, 9.2 at 320) over
-// that in as many parts as `llmserve_gemm_blocks_parts` says.
+// What the whole sums cost it, in thousandths of a us: its own time (of the two smallest tiles by K alone: 6.6 and 8.8 us at K 1,536, where 96 and 320 rows of N 1,536 take 6.4 and 8.6)
+// over that in as many parts as `llmserve_gemm_blocks_parts` says.
 extern "C" int llmserve_gemm_blocks_norm_cost(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64 || N > 128 * SUMS_MOST) return 1 << 30;
   const int splits = llmserve_gemm_blocks_parts(M, N, K);
@@ -902,8 +903,8 @@ extern "C" int llmserve_gemm_blocks_scaled(const void* rows, const float* sums, 
 }
 
 // A product whose heads are rotated on the way out, in the smallest tile of which one round of 256 workgroups holds the result, as
-// more CUs then bring the operands.  Us at N 2,048 K 1,536: 96 rows 8.2, 287 rows 9.9, 512 rows 9.0, 1,024 rows 13.4, 2,048 rows 21.6 (before the loads were
-// spread over the products, and with bias and places waited for before the first stage 10.6, 11.7, 11.9, 15.3, 22.5); in the smallest tile that does not
+// more CUs then bring the operands.  Us at N 2,048 K 1,536: 96 rows 6.8, 287 rows 9.9, 512 rows 9.0, 1,024 rows 13.4, 2,048 rows 21.6 (before the loads were
+// spread over the products, the smallest tiles had as many waves as they have now, and with bias and places waited for before the first stage 10.6, 11.7, 11.9, 15.3, 22.5); in the smallest tile that does not
 // make one round, measured then: 512 rows of 64 x 32 13.7, of 64 x 64 11.7, 1,024 rows of 64 x 64 26.8, of 128 x 64 16.6.  What it saves is a launch and
 // the rows' way to memory and back: with the kernel that rotates and stores behind the library's product 15.5 us at 96 rows, 27.3 at 2,048.
 static int launch_rotated(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int N, int K,

@@ -548,8 +548,8 @@ class HipKernels:
         return GatedLinearWeights(LinearWeights(both, None), gate.shape[0], activation, float(limit or 0.0))
 
     def _streaming(self, x: torch.Tensor, weights: LinearWeights, gated: bool = False, may_split: bool = False) -> str | None:
-        """Which MFMA kernel takes this product: "skinny" (up to 16 rows of x, weights streamed; see `_flows`),
-        "ring" (17 to 64 rows of a middling weight, both operands through a ring of stages in LDS),
+        """Which MFMA kernel takes this product: "skinny" (weights streamed: up to 16 rows of x, where `_flows` says by which kernel, and 17 to 64 of a small weight),
+        "ring" (17 to 128 rows of a middling weight, both operands through a ring of stages in LDS; up to 16 rows see below),
         "medium" (up to 64, x shared through LDS), "tiled" (any number, both operands through LDS),
         or None (the BLAS library, or the generic kernel)."""
         weight = weights.weight
@@ -558,8 +558,8 @@ class HipKernels:
         rows, (outer, inner) = x.shape[0], weight.shape
         size = outer * inner
         if self.ring_products and rows <= 16 and inner % 128 == 0 and size > (1 << 22):
-            # (Products of up to 16 rows with a K of whole units go to `_flows`' kernel, whichever name they get here; what the name still says is
-            # how rows that a norm has left scaled, longer than that kernel's, are read.)
+            # (The name decides one thing alone: rows that a norm has left scaled and that are wider than _FLOW_SCALED are read through the ring, in the shape that `_linear_into_norm`
+            # asks for by it.  Every other product of up to 16 rows that gets it goes to `_flows`' kernel, as those named "skinny" with a K of whole units do.)
             heavy = size > (1 << 26) or (may_split and size > (1 << 24))
             if rows >= (self.ring_rows_from if heavy else max(12, self.ring_rows_from)) and (heavy or may_split or size > (1 << 24)):
                 if self._ring_shape(rows, outer, inner, may_split)[2] == 1:
@@ -1006,10 +1006,10 @@ class HipKernels:
         _check(status, "linear into a norm")
         return ScaledRows(scaled, sums, into.eps, reader, -1)
 
-    # What the first product's whole sums may cost, in thousandths of a us by its estimate, for the norm's kernel.  Us in a captured chain of the output projection, norm
-    # and gate/up, apart -> linked (cost): 1.5B sizes 80 rows 26.0 -> 25.0 (2.6), 128 rows 29.1 -> 27.9 (2.6), 160 rows 31.8 -> 30.3 (1.6), 192 rows 32.1 -> 32.9 (4.2), 256 rows 35.6 ->
-    # 34.0 (2.8), 320 rows 35.8 -> 35.3 (3.2), 384 rows 41.1 -> 39.3, 640 rows 56.5 -> 53.6, 1,536 rows 107.4 -> 104.2, 2,048 rows 126.8 -> 121.7; width 2,048 96 rows 32.6 -> 33.9 (6.7);
-    # 7B sizes 96 rows 75.6 -> 89.1.
+    # What the first product's whole sums may cost, in thousandths of a us by its estimate, for the norm's kernel.  Whole prompts, us, apart -> linked (cost): width 1,536 80 tokens
+    # 1,622 -> 1,588 (2.3), 128 1,683 -> 1,667 (2.3), 160 1,997 -> 1,936 (1.3), 256 2,170 -> 2,110 (2.6), 320 2,414 -> 2,375 (3.0), 384 2,513 -> 2,461, 768 4,040 -> 3,960, 2,048 7,666 ->
+    # 7,530, but 192 2,069 -> 2,077 (4.0); width 2,048 320 tokens 2,337 -> 2,307, 512 2,940 -> 2,870, but 96 1,510 -> 1,564 (6.1); width 1,024 with 16 heads 256 tokens 1,310 -> 1,291 (2.9), but
+    # 96 1,047 -> 1,058 (4.0); 7B sizes 96 tokens 1,618 -> 1,805 (16); widths 896, 1,152 and 2,560 the same either way.
     _TILES_INTO_NORM = 3400
 
     def _scaled_gated_linear(self, x: ScaledRows, weights: GatedLinearWeights) -> torch.Tensor:
