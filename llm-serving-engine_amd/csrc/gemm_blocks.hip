@@ -926,13 +926,14 @@ static int launch_rotated(const void* x, const void* w, const void* bias, int bi
 }
 
 // Rows of q, k and v heads: out [M, (heads + 2 kv_heads) dim] bfloat16 = x . w^T (+ bias), of which the q and k heads are rotated in
-// neighbouring pairs by `table` (cos, sin of [M][dim / 2]), and k and v also stored in the pages.  `dim` a multiple of 16, K of 32.
+// neighbouring pairs by `table` (cos, sin of [M][dim / 2]), and k and v also stored in the pages.  `dim` a multiple of 16, K of 32; x,
+// w, the table and the pages begin at a multiple of 16 bytes.
 extern "C" int llmserve_gemm_rotated(const void* x, const void* w, const void* bias, int bias_is_float, void* out, int M, int K,
                                      const float* table, int heads, int kv_heads, int dim, void* keys, void* values, const int* slots,
                                      int page_size, hipStream_t stream) {
   if (M <= 0) return 0;
   if (K <= 0 || K % 32 || heads < 1 || kv_heads < 1 || dim < 16 || dim % 16 || page_size < 1 || !table || !keys || !values || !slots) return ERR_BAD_ARGUMENT;
-  if ((size_t)table % 16 || (size_t)keys % 16 || (size_t)values % 16) return ERR_BAD_ARGUMENT;
+  if (((size_t)x | (size_t)w | (size_t)table | (size_t)keys | (size_t)values) & 15) return ERR_BAD_ARGUMENT;
   return launch_rotated(x, w, bias, bias_is_float, out, M, (heads + 2 * kv_heads) * dim, K, stream,
                         {(const float2*)table, (bf16_t*)keys, (bf16_t*)values, slots, heads, kv_heads, dim, page_size});
 }

@@ -91,3 +91,16 @@ def test_entry_points_refuse_them():
         assert kernels._gemm_bf16.llmserve_gemm_ring(a.data_ptr(), b.data_ptr(), None, 0, out.data_ptr(), 0, 0, 24, 8192, 1024, 1, 4, kernels._stream) == 1001
         assert kernels._gemm_bf16.llmserve_gemm_stream(a.data_ptr(), b.data_ptr(), None, 0, out.data_ptr(), 0, 0, 24, 512, 1024, 1, kernels._stream) == 1001
         assert kernels._gemm_blocks.llmserve_gemm_blocks(a.data_ptr(), b.data_ptr(), None, 0, out.data_ptr(), 0, 0, 128, 8192, 1024, 1, kernels._stream) == 1001
+
+
+@pytest.mark.gpu
+def test_the_rotated_product_refuses_them():
+    from llmserve_amd.kernels import HipKernels
+
+    kernels, rows, inner, heads, kv_heads, dim, page = HipKernels(torch.bfloat16), 96, 1536, 12, 2, 128, 16
+    x, w, out, keys, values = (torch.zeros(n + 8, device="cuda", dtype=torch.bfloat16) for n in (rows * inner, 2048 * inner, rows * 2048, 8 * page * kv_heads * dim, 8 * page * kv_heads * dim))
+    table, slots = torch.zeros(rows * dim, device="cuda"), torch.full((rows,), -1, device="cuda", dtype=torch.int32)
+    for a, b, status in ((x, w, 0), (x[1:], w, 1001), (x, w[4:], 1001)):
+        assert kernels._gemm_blocks.llmserve_gemm_rotated(a.data_ptr(), b.data_ptr(), None, 0, out.data_ptr(), rows, inner, table.data_ptr(), heads, kv_heads, dim, keys.data_ptr(),
+                                                          values.data_ptr(), slots.data_ptr(), page, kernels._stream) == status
+    torch.cuda.synchronize()
